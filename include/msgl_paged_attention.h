@@ -223,6 +223,22 @@ MSGL_API int msgl_build_attention_metadata(const int32_t* page_table, int64_t ta
                                   int32_t max_kv_splits, void* stream);
 
 /*
+ * The same for a caller whose per-request integers are in host memory (a scheduler's are):
+ * table_rows, kv_lens and extend_lens are HOST pointers, read before the call returns, and reach
+ * the kernel as its arguments, so nothing is uploaded and nothing waits.
+ * batch <= MSGL_METADATA_HOST_BATCH.
+ */
+#define MSGL_METADATA_HOST_BATCH 128
+MSGL_API int msgl_build_attention_metadata_host(const int32_t* page_table, int64_t table_stride0,
+                                  int64_t n_table_rows, int64_t max_seq_len,
+                                  const int32_t* table_rows, const int32_t* kv_lens,
+                                  const int32_t* extend_lens, int64_t batch,
+                                  int32_t* kv_indptr, int32_t* kv_indices, int64_t kv_capacity,
+                                  int32_t* qo_indptr, int32_t* prefix_lens, int32_t* positions,
+                                  int64_t q_capacity, int32_t* num_kv_splits,
+                                  int32_t max_kv_splits, void* stream);
+
+/*
  * qk_norm_rope_store -- replaces the chain in front of the attention call in the reference's
  * Qwen3 attention layer (mini_sglang_mlx/models/qwen3.py:60-68) together with the store that
  * AttnBackend.forward does first (mini_sglang_mlx/attention/backend.py:139):

@@ -4,7 +4,9 @@ Usage: ``python build.py [--force]``.  hipcc cross-compiles, so this runs withou
 Each ``.hip`` file is compiled to an object on its own (in parallel) and the objects are
 linked into one shared library whose only exported symbols are the ``msgl_*`` C ABI of
 ``include/msgl_paged_attention.h``, ``include/msgl_radix_cache.h`` and
-``include/msgl_state_pool.h``.
+``include/msgl_state_pool.h``.  ``csrc/torch_binding.cpp`` (host code: the operators' Python call
+path) is compiled by g++ against torch's headers into ``mini_sglang_amd_kernel/_native.so``, which
+loads that library from its place beside it.
 """
 from __future__ import annotations
 
@@ -21,6 +23,9 @@ LIB_PATH = os.path.join(LIB_DIR, "libmsgl_paged_attention.so")
 SOURCES = ["api.hip", "store_kv_cache.hip", "paged_splitkv.hip", "paged_prefill.hip", "paged_prefill_d256.hip",
            "build_metadata.hip", "qk_norm_rope_store.hip",
            "gdn_state.hip", "radix_cache.hip", "state_slots.hip"]
+
+NATIVE_SRC = os.path.join(CSRC, "torch_binding.cpp")
+NATIVE_PATH = os.path.join(HERE, "mini_sglang_amd_kernel", "_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Packed fp32 VALU forms are switched off for every device compile on this target.
@@ -53,6 +58,25 @@ def _compile(src: str, save_temps: bool) -> str:
     return obj
 
 
+def _build_native() -> None:
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    libs = library_paths()
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-sign-compare",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-I" + sysconfig.get_paths()["include"],
+           *("-isystem" + p for p in (*include_paths(), "/opt/rocm/include")), NATIVE_SRC,
+           "-L" + LIB_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN/../lib",
+           *("-L" + p for p in libs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
+           "-ltorch_python", "-o", NATIVE_PATH]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_binding.cpp:\n{proc.stderr}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr)
+
+
 def build(force: bool = False, save_temps: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -73,6 +97,8 @@ def build(force: bool = False, save_temps: bool = False) -> str:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
+    if force or _newer([NATIVE_SRC, headers[-3]], NATIVE_PATH):
+        _build_native()
     return LIB_PATH
 
 

@@ -452,14 +452,15 @@ int msgl_copy_state_slots(void* slab, int64_t layer_stride_bytes, int64_t slot_s
                                   num_slots, src, dst, n_pairs, static_cast<hipStream_t>(stream));
 }
 
-int msgl_build_attention_metadata(const int32_t* page_table, int64_t table_stride0,
-                                  int64_t n_table_rows, int64_t max_seq_len,
-                                  const int32_t* table_rows, const int32_t* kv_lens,
-                                  const int32_t* extend_lens, int64_t batch, int32_t* kv_indptr,
-                                  int32_t* kv_indices, int64_t kv_capacity, int32_t* qo_indptr,
-                                  int32_t* prefix_lens, int32_t* positions, int64_t q_capacity,
-                                  int32_t* num_kv_splits, int32_t max_kv_splits, void* stream) {
-  if (batch < 0 || batch > msgl::kMetadataMaxBatch || n_table_rows <= 0 || max_seq_len < 0 ||
+static int build_metadata(bool lens_on_host, const int32_t* page_table, int64_t table_stride0,
+                          int64_t n_table_rows, int64_t max_seq_len,
+                          const int32_t* table_rows, const int32_t* kv_lens,
+                          const int32_t* extend_lens, int64_t batch, int32_t* kv_indptr,
+                          int32_t* kv_indices, int64_t kv_capacity, int32_t* qo_indptr,
+                          int32_t* prefix_lens, int32_t* positions, int64_t q_capacity,
+                          int32_t* num_kv_splits, int32_t max_kv_splits, void* stream) {
+  const int64_t max_batch = lens_on_host ? MSGL_METADATA_HOST_BATCH : msgl::kMetadataMaxBatch;
+  if (batch < 0 || batch > max_batch || n_table_rows <= 0 || max_seq_len < 0 ||
       table_stride0 < max_seq_len || kv_capacity < 0 || q_capacity < 0 ||
       kv_capacity > 0x7fffffffLL || q_capacity > 0x7fffffffLL || max_seq_len > 0x7fffffffLL ||
       n_table_rows > 0x7fffffffLL)
@@ -485,7 +486,30 @@ int msgl_build_attention_metadata(const int32_t* page_table, int64_t table_strid
   a.kv_capacity = kv_capacity;
   a.q_capacity = positions ? q_capacity : 0;
   a.max_kv_splits = max_kv_splits;
+  a.lens_on_host = lens_on_host ? 1 : 0;
   return msgl::launch_build_metadata(a, static_cast<hipStream_t>(stream));
+}
+
+int msgl_build_attention_metadata(const int32_t* page_table, int64_t table_stride0,
+                                  int64_t n_table_rows, int64_t max_seq_len, const int32_t* table_rows,
+                                  const int32_t* kv_lens, const int32_t* extend_lens, int64_t batch,
+                                  int32_t* kv_indptr, int32_t* kv_indices, int64_t kv_capacity, int32_t* qo_indptr,
+                                  int32_t* prefix_lens, int32_t* positions, int64_t q_capacity,
+                                  int32_t* num_kv_splits, int32_t max_kv_splits, void* stream) {
+  return build_metadata(false, page_table, table_stride0, n_table_rows, max_seq_len, table_rows, kv_lens, extend_lens,
+                        batch, kv_indptr, kv_indices, kv_capacity, qo_indptr, prefix_lens, positions, q_capacity,
+                        num_kv_splits, max_kv_splits, stream);
+}
+
+int msgl_build_attention_metadata_host(const int32_t* page_table, int64_t table_stride0,
+                                       int64_t n_table_rows, int64_t max_seq_len, const int32_t* table_rows,
+                                       const int32_t* kv_lens, const int32_t* extend_lens, int64_t batch,
+                                       int32_t* kv_indptr, int32_t* kv_indices, int64_t kv_capacity, int32_t* qo_indptr,
+                                       int32_t* prefix_lens, int32_t* positions, int64_t q_capacity,
+                                       int32_t* num_kv_splits, int32_t max_kv_splits, void* stream) {
+  return build_metadata(true, page_table, table_stride0, n_table_rows, max_seq_len, table_rows, kv_lens, extend_lens,
+                        batch, kv_indptr, kv_indices, kv_capacity, qo_indptr, prefix_lens, positions, q_capacity,
+                        num_kv_splits, max_kv_splits, stream);
 }
 
 int msgl_qk_norm_rope_store(const void* q, const void* k, const void* v, int64_t q_stride0,

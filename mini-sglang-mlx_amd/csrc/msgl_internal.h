@@ -110,8 +110,9 @@ struct MetadataArgs {
   int32_t* num_kv_splits;
   int64_t table_stride0, batch, n_table_rows, max_seq_len, kv_capacity, q_capacity;
   int32_t max_kv_splits;
+  int32_t lens_on_host;  // table_rows, kv_lens, extend_lens are host pointers
 };
-// largest batch one launch handles (two scanned offset arrays live in LDS)
+// largest batch one launch handles (two scanned offset arrays and the table rows live in LDS)
 constexpr int64_t kMetadataMaxBatch = 8000;
 int launch_build_metadata(const MetadataArgs& a, hipStream_t stream);
 

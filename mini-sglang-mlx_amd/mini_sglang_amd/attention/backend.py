@@ -15,7 +15,7 @@ from typing import List, Optional, Sequence
 
 import torch
 
-from mini_sglang_amd_kernel import (build_attention_metadata, paged_decode_attention,
+from mini_sglang_amd_kernel import (build_metadata_from_host, paged_decode_attention,
                                     paged_prefill_attention, qk_norm_rope_store)
 
 MAX_KV_SPLITS = 32
@@ -143,18 +143,10 @@ class AttnBackend:
 
     def _device_metadata(self, reqs, kv_lens: Sequence[int],
                          extend_lens: Optional[Sequence[int]]) -> dict:
-        """One upload of the per-request integers, one kernel for every array (slot table on
-        the GPU).  The host lists are the reference's own inputs (backend.py:228-238)."""
-        device = self.page_table.device
-        host = [[req.table_idx for req in reqs], list(kv_lens)]
-        if extend_lens is not None:
-            host.append(list(extend_lens))
-        packed = torch.tensor(host, dtype=torch.int32).to(device, non_blocking=True)
-        return build_attention_metadata(
-            self.page_table, packed[0], packed[1], packed[2] if extend_lens is not None else None,
-            total_kv=int(sum(kv_lens)),
-            total_q=int(sum(extend_lens)) if extend_lens is not None else len(reqs),
-            max_kv_splits=MAX_KV_SPLITS)
+        """One kernel for every array (slot table on the GPU).  The host lists are the
+        reference's own inputs (backend.py:228-238)."""
+        return build_metadata_from_host(self.page_table, [req.table_idx for req in reqs], kv_lens,
+                                        extend_lens, max_kv_splits=MAX_KV_SPLITS)
 
     def build_prefill_metadata(self, reqs: List, *, extend_lens: Optional[List[int]] = None,
                                kv_lens: Optional[List[int]] = None,
@@ -191,14 +183,22 @@ class AttnBackend:
         device = self.page_table.device
         if kv_lens is None:
             kv_lens = [req.device_len for req in reqs]
-        if positions is None:
-            positions = torch.tensor([req.cached_len for req in reqs], dtype=torch.int32,
-                                     device=device)
         if device.type == "cuda":
             m = self._device_metadata(reqs, kv_lens, None)
+            if positions is None:
+                cached = [req.cached_len for req in reqs]
+                # the new token's position is the last one, as a rule: the kernel has written it
+                if (cached and min(cached) >= 0 and cached == [n - 1 for n in kv_lens]
+                        and max(kv_lens) <= self.page_table.shape[1]):
+                    positions = m["positions"]
+                else:
+                    positions = torch.tensor(cached, dtype=torch.int32, device=device)
             return DecodeMetadata(positions=positions, kv_indptr=m["kv_indptr"],
                                   kv_indices=m["kv_indices"], num_kv_splits=m["num_kv_splits"],
                                   max_kv_splits=MAX_KV_SPLITS)
+        if positions is None:
+            positions = torch.tensor([req.cached_len for req in reqs], dtype=torch.int32,
+                                     device=device)
         return DecodeMetadata(
             positions=positions,
             kv_indptr=_build_indptr(kv_lens, device),

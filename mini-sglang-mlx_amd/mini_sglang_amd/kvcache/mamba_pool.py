@@ -100,6 +100,10 @@ class MambaStatePool:
             slab.allocate()
         # copies and zero fills move the slot state, not the verify windows (mamba_pool.py:170-189)
         self._state_slabs = [s for (kind, _, _), s in slabs.items() if kind != "window"]
+        # the accessors are called for every layer of every step: their views are made once
+        self._temporal_views = [slab.data[at] for slab, at in self._temporal]
+        self._conv_views = [[slab.data[at] for slab, at in groups] for groups in self._conv]
+        self._window_views = [[slab.data[at] for slab, at in groups] for groups in self._windows]
         self._free_slots: List[int] = list(range(1, config.num_slots + 1))
 
     # ---- slot lifecycle (host) -------------------------------------------------------------
@@ -200,18 +204,15 @@ class MambaStatePool:
 
     # ---- accessors -------------------------------------------------------------------------
     def temporal_state(self, layer_idx: int) -> torch.Tensor:
-        slab, at = self._temporal[layer_idx]
-        return slab.data[at]
+        return self._temporal_views[layer_idx]
 
     def conv_state(self, layer_idx: int, group: int = 0) -> torch.Tensor:
-        slab, at = self._conv[layer_idx][group]
-        return slab.data[at]
+        return self._conv_views[layer_idx][group]
 
     def conv_window(self, layer_idx: int, group: int = 0) -> torch.Tensor:
         """Row ``[slot, j]``: the conv window after ``j + 1`` verify tokens (mamba_pool.py:194-203)."""
         assert self.verify_width > 0, "conv windows not allocated"
-        slab, at = self._windows[layer_idx][group]
-        return slab.data[at]
+        return self._window_views[layer_idx][group]
 
     def mem_usage_bytes(self) -> int:
         return sum(s.data.numel() * s.data.element_size() for s in self._slabs)

@@ -31,13 +31,17 @@ class MHAKVCache(BaseKVCache):
         slab = (num_layers, num_pages, num_kv_heads, head_dim)
         self._k_slab = torch.zeros(slab, dtype=dtype, device=device)
         self._v_slab = torch.zeros(slab, dtype=dtype, device=device)
+        # a layer's views are asked for several times per layer and step: made once (indexing the
+        # slab costs 1-2 us of host time each time)
+        self._k_layers = self._k_slab.unbind(0)
+        self._v_layers = self._v_slab.unbind(0)
 
     # ---- the reference's surface -----------------------------------------------------------
     def k_cache(self, index: int) -> torch.Tensor:
-        return self._k_slab[index]
+        return self._k_layers[index]
 
     def v_cache(self, index: int) -> torch.Tensor:
-        return self._v_slab[index]
+        return self._v_layers[index]
 
     def store_kv(self, k: torch.Tensor, v: torch.Tensor, out_loc: torch.Tensor,
                  layer_id: int) -> None:
@@ -47,7 +51,7 @@ class MHAKVCache(BaseKVCache):
         if k.shape[0] != rows or v.shape[0] != rows:
             raise ValueError(f"store_kv: {rows} slot ids for k of shape {tuple(k.shape)} and v of "
                              f"shape {tuple(v.shape)}")
-        store_kv_cache(self._k_slab[layer_id], self._v_slab[layer_id], out_loc, k, v)
+        store_kv_cache(self._k_layers[layer_id], self._v_layers[layer_id], out_loc, k, v)
 
     @property
     def dtype(self) -> torch.dtype:

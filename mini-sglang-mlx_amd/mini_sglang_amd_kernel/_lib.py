@@ -46,6 +46,10 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp,
          _i32, _vp]),
+    "msgl_build_attention_metadata_host": (
+        ctypes.c_int,
+        [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp,
+         _i32, _vp]),
     "msgl_qk_norm_rope_store": (
         ctypes.c_int,
         [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64,
@@ -96,6 +100,22 @@ _lib = None
 
 class KernelLibraryMissing(ImportError):
     pass
+
+
+class MissingNative:
+    """Stands in for the extension module ``_native`` where it has not been built: any use raises."""
+
+    def __init__(self, cause: ImportError) -> None:
+        self._cause = cause
+
+    def set_checks(self, fn) -> None:
+        pass
+
+    def __getattr__(self, name: str):
+        raise KernelLibraryMissing(
+            f"mini_sglang_amd_kernel/_native.so cannot be loaded ({self._cause}): build it with "
+            "`python mini-sglang-mlx_amd/build.py` (or __graft_entry__.build()); there is no "
+            "fallback implementation")
 
 
 def load() -> ctypes.CDLL:
