@@ -21,7 +21,11 @@
 namespace msgl {
 namespace {
 
-constexpr int kHeadsPerGroup = 8;
+// Heads a group of lanes walks.  Many tokens: 8, so that the sines and cosines are computed once per
+// 8 heads (HBM-bound, 21 us for 4096 tokens of 32 + 16 heads, 4.8 TB/s).  Few tokens: 1, because
+// then the launch is the chain of one group's loads and not bytes: with 8 heads one after the other
+// a decode step of 4 requests (16 + 16 heads) took 11.1 us on a single workgroup.
+constexpr int kHeadsPerGroupMany = 8;
 constexpr int kGroupLanes = 16;
 constexpr int kThreads = 256;
 
@@ -37,7 +41,7 @@ struct NormRopeParams {
   uint16_t* k_cache;
   uint16_t* v_cache;
   int64_t q_stride0, k_stride0, v_stride0, kc_stride0, vc_stride0, num_slots;
-  int32_t n_tokens, n_q, n_kv, chunks;  // chunks of kHeadsPerGroup heads per token
+  int32_t n_tokens, n_q, n_kv, chunks;  // chunks of heads per token
   float eps, log2_base;
 };
 
@@ -53,23 +57,46 @@ struct Vec<4> { typedef u32x2_t type; };
 template <>
 struct Vec<8> { typedef u32x4_t type; };
 
-template <int D>
+template <int D, int kHeadsPerGroup>
 __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopeParams p) {
   constexpr int E = D / 32;  // elements per lane and half
   using V = typename Vec<E>::type;
   const int j = threadIdx.x & (kGroupLanes - 1);
   const int64_t item = (int64_t)blockIdx.x * (kThreads / kGroupLanes) + (threadIdx.x / kGroupLanes);
   if (item >= (int64_t)p.n_tokens * p.chunks) return;  // whole groups leave together
-  const int t = (int)(item / p.chunks);
+  // few tokens: the item number fits 32 bits (a 64-bit division is 40 instructions of the chain)
+  const int t = kHeadsPerGroup == 1 ? (int)((uint32_t)item / (uint32_t)p.chunks) : (int)(item / p.chunks);
   const int chunk = (int)(item - (int64_t)t * p.chunks);
   const int n_heads = p.n_q + 2 * p.n_kv;
   const int h_begin = chunk * kHeadsPerGroup;
   const int h_end = min(h_begin + kHeadsPerGroup, n_heads);
 
+  const int off = j * E;
+  // a head's row and, for q and k, its norm weights; asked for one head ahead, the first ones before
+  // the sines and cosines
+  struct Head {
+    V lo, hi, wl, wh;
+  };
+  auto fetch = [&](int h) {
+    Head x{};
+    const uint16_t* src = h < p.n_q ? p.q + (int64_t)t * p.q_stride0 + (int64_t)h * D
+                          : h < p.n_q + p.n_kv ? p.k + (int64_t)t * p.k_stride0 + (int64_t)(h - p.n_q) * D
+                                               : p.v + (int64_t)t * p.v_stride0 + (int64_t)(h - p.n_q - p.n_kv) * D;
+    const uint16_t* w = h < p.n_q ? p.q_weight : p.k_weight;  // of no use to a v head
+    x.lo = *reinterpret_cast<const V*>(src + off);
+    x.hi = *reinterpret_cast<const V*>(src + D / 2 + off);
+    x.wl = *reinterpret_cast<const V*>(w + off);
+    x.wh = *reinterpret_cast<const V*>(w + D / 2 + off);
+    return x;
+  };
+  const int32_t position = p.positions[t];
+  const int64_t slot = p.out_loc[t];
+  Head next = fetch(h_begin);
+
   // sines and cosines of this lane's pairs (only if the chunk holds a q or k head)
   float cs[E], sn[E];
   if (h_begin < p.n_q + p.n_kv) {
-    const float pos = (float)p.positions[t];
+    const float pos = (float)position;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const float d = (float)(j * E + e) / (float)(D / 2);
@@ -77,33 +104,18 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopePa
       sincosf(pos * inv_freq, &sn[e], &cs[e]);
     }
   }
-  const int64_t slot = p.out_loc[t];
   // a slot id outside the pools stores no k / v row (q_out is still produced): a wild store
   // would be a GPU memory fault
   const bool slot_ok = (uint64_t)slot < (uint64_t)p.num_slots;
-  const int off = j * E;
 
   for (int h = h_begin; h < h_end; ++h) {
-    const uint16_t* src;
-    uint16_t* dst;
-    const uint16_t* w = nullptr;
-    if (h < p.n_q) {
-      src = p.q + (int64_t)t * p.q_stride0 + (int64_t)h * D;
-      dst = p.q_out + ((int64_t)t * p.n_q + h) * D;
-      w = p.q_weight;
-    } else if (h < p.n_q + p.n_kv) {
-      src = p.k + (int64_t)t * p.k_stride0 + (int64_t)(h - p.n_q) * D;
-      dst = p.k_cache + slot * p.kc_stride0 + (int64_t)(h - p.n_q) * D;
-      w = p.k_weight;
-    } else {
-      src = p.v + (int64_t)t * p.v_stride0 + (int64_t)(h - p.n_q - p.n_kv) * D;
-      dst = p.v_cache + slot * p.vc_stride0 + (int64_t)(h - p.n_q - p.n_kv) * D;
-    }
-    V lo = *reinterpret_cast<const V*>(src + off);
-    V hi = *reinterpret_cast<const V*>(src + D / 2 + off);
-    if (w != nullptr) {
-      const V wl = *reinterpret_cast<const V*>(w + off);
-      const V wh = *reinterpret_cast<const V*>(w + D / 2 + off);
+    uint16_t* dst = h < p.n_q ? p.q_out + ((int64_t)t * p.n_q + h) * D
+                    : h < p.n_q + p.n_kv ? p.k_cache + slot * p.kc_stride0 + (int64_t)(h - p.n_q) * D
+                                         : p.v_cache + slot * p.vc_stride0 + (int64_t)(h - p.n_q - p.n_kv) * D;
+    V lo = next.lo, hi = next.hi;
+    const V wl = next.wl, wh = next.wh;
+    if (h + 1 < h_end) next = fetch(h + 1);
+    if (h < p.n_q + p.n_kv) {
       float xl[E], xh[E];
       float ss = 0.f;
 #pragma unroll
@@ -165,7 +177,10 @@ int launch_qk_norm_rope_store(const NormRopeArgs& a, hipStream_t stream) {
   p.n_q = (int32_t)a.n_q;
   p.n_kv = (int32_t)a.n_kv;
   const int64_t n_heads = a.n_q + 2 * a.n_kv;
-  p.chunks = (int32_t)((n_heads + kHeadsPerGroup - 1) / kHeadsPerGroup);
+  // one head per group until its workgroups fill the chip twice over
+  const bool few = a.n_tokens * n_heads <= 512 * (kThreads / kGroupLanes);
+  const int per_group = few ? 1 : kHeadsPerGroupMany;
+  p.chunks = (int32_t)((n_heads + per_group - 1) / per_group);
   p.eps = a.eps;
   p.log2_base = log2f(a.rope_base);
   const int64_t items = a.n_tokens * p.chunks;
@@ -173,12 +188,10 @@ int launch_qk_norm_rope_store(const NormRopeArgs& a, hipStream_t stream) {
   const int64_t blocks = (items + per_block - 1) / per_block;
   if (blocks <= 0) return MSGL_OK;
   if (blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  if (a.head_dim == 128)
-    hipLaunchKernelGGL(qk_norm_rope_store_kernel<128>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, p);
-  else if (a.head_dim == 256)
-    hipLaunchKernelGGL(qk_norm_rope_store_kernel<256>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, p);
-  else
-    return MSGL_ERR_HEAD_DIM;
+  if (a.head_dim != 128 && a.head_dim != 256) return MSGL_ERR_HEAD_DIM;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, p); };
+  if (a.head_dim == 128) few ? launch(qk_norm_rope_store_kernel<128, 1>) : launch(qk_norm_rope_store_kernel<128, kHeadsPerGroupMany>);
+  else few ? launch(qk_norm_rope_store_kernel<256, 1>) : launch(qk_norm_rope_store_kernel<256, kHeadsPerGroupMany>);
   return check_launch();
 }
 
