@@ -319,6 +319,9 @@ MSGL_API int msgl_gdn_state_inplace(const void* q, const void* k, const void* v,
  *                            Workgroup 0 of every attention kernel launched by this thread then
  *                            leaves there the shader cycles and the 100 MHz wall ticks it lived
  *                            for: cycles / ticks x 0.1 = the shader clock in GHz under that kernel
+ *   MSGL_TUNE_SHARES         decode and verify on one launch of per-request key shares instead of
+ *                            equal segments and a merge: negative: never; 0: chosen from the sizes;
+ *                            positive: always, with share_len | kv heads per workgroup << 20
  */
 #define MSGL_TUNE_SEGMENTS 0
 #define MSGL_TUNE_MIN_SEGMENT 1
@@ -330,6 +333,7 @@ MSGL_API int msgl_gdn_state_inplace(const void* q, const void* k, const void* v,
 #define MSGL_TUNE_SPLITKV_BOUNDARY 7
 #define MSGL_TUNE_PREFILL_GANGS 8
 #define MSGL_TUNE_CLOCK_PROBE 9
+#define MSGL_TUNE_SHARES 10
 MSGL_API int msgl_set_tuning(int32_t knob, int64_t value);
 /* The value the calling thread last set for `knob` (0 if it never did): what its launches and
  * workspace queries use.  Makes the per-thread scope observable: a value set on another thread

@@ -20,7 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(LIB_DIR, "libmsgl_paged_attention.so")
-SOURCES = ["api.hip", "store_kv_cache.hip", "paged_splitkv.hip", "paged_prefill.hip", "paged_prefill_d256.hip",
+SOURCES = ["api.hip", "store_kv_cache.hip", "paged_splitkv.hip", "paged_shares.hip", "paged_prefill.hip", "paged_prefill_d256.hip",
            "build_metadata.hip", "qk_norm_rope_store.hip",
            "gdn_state.hip", "radix_cache.hip", "state_slots.hip"]
 

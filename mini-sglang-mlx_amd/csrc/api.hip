@@ -17,7 +17,7 @@ thread_local int64_t t_tune[3] = {0, 0, 0};
 thread_local int64_t t_key_splits = 0;
 thread_local int64_t t_gangs = 0;  // negative: never use gang ranges
 thread_local long long* t_clock_probe = nullptr;
-constexpr int kTuneKnobs = 10;
+constexpr int kTuneKnobs = 11;
 thread_local int64_t t_last_set[kTuneKnobs] = {};  // what this thread last passed to msgl_set_tuning
 // launch numbers for the count words of gang ranges (see prefill_gangs()); never 0
 std::atomic<unsigned long long> g_gang_nonce{1};
@@ -54,6 +54,13 @@ int32_t segments(int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols)
   const int64_t t = t_tune[MSGL_TUNE_SEGMENTS];
   if (t >= 1) return (int32_t)(t < (1 << 20) ? t : (1 << 20));
   return msgl::splitkv_default_segments(total_kv, n_kv, head_dim, cols, min_segment(head_dim));
+}
+// Shares instead of segments (paged_shares.hip); a knob that shapes the segments asks for segments.
+msgl::SharePlan shares_for(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols) {
+  if (t_tune[MSGL_TUNE_SEGMENTS] != 0 || t_tune[MSGL_TUNE_MIN_SEGMENT] != 0 || t_last_set[MSGL_TUNE_SPLITKV_WAVES] != 0 ||
+      t_last_set[MSGL_TUNE_SPLITKV_BOUNDARY] != 0)
+    return msgl::SharePlan{};
+  return msgl::share_plan(batch, total_kv, n_kv, head_dim, cols);
 }
 // Largest q_len * group that takes the split-K route whatever the launch: at head_dim 128 48 (up
 // to three column tiles in one wave; 49-64 columns would run on two waves per kv head that each
@@ -135,6 +142,10 @@ int msgl_set_tuning(int32_t knob, int64_t value) {
     t_clock_probe = reinterpret_cast<long long*>(static_cast<intptr_t>(value));
     return MSGL_OK;
   }
+  if (knob == MSGL_TUNE_SHARES) {
+    msgl::shares_force(value);
+    return MSGL_OK;
+  }
   if (knob < 0 || knob > 2) return MSGL_ERR_SHAPE;
   t_tune[knob] = value;
   return MSGL_OK;
@@ -164,6 +175,9 @@ size_t msgl_paged_decode_workspace_bytes(int64_t batch, int64_t total_kv, int64_
       num_q_heads % num_kv_heads != 0)
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
+  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, group);
+  if (msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group, 0, 1))
+    return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
   return msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1,
                                        segments(total_kv, num_kv_heads, head_dim, group));
 }
@@ -188,8 +202,11 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
   if (!kv_indptr || !num_kv_splits || (total_kv > 0 && !kv_indices)) return MSGL_ERR_NULL_POINTER;
   (void)max_kv_splits;  // split hints do not steer the cut (result is split-invariant)
   const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, group);
-  const size_t need =
-      msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1, n_seg);
+  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, group);
+  const bool shares = msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group, 0, 1);
+  const size_t need = shares
+                          ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group)
+                          : msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1, n_seg);
   if (builtin_scratch) {
     rc = msgl::splitkv_scratch(&workspace, &workspace_bytes);
     if (rc != MSGL_OK) return rc;
@@ -221,6 +238,7 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
   a.window = 0;
   a.n_seg = n_seg;
   a.min_seg = min_segment(head_dim);
+  if (shares) return msgl::launch_shares(a, plan, static_cast<hipStream_t>(stream));
   return msgl::launch_splitkv(a, static_cast<hipStream_t>(stream));
 }
 
@@ -312,9 +330,13 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
       return std::max(split_need, msgl::prefill_gang_workspace_bytes(batch, num_kv_heads, group, max_len_extend, gangs));
     return split_need;
   }
-  const size_t split_need = msgl::splitkv_workspace_bytes(
-      batch, num_q_heads, num_kv_heads, head_dim, max_len_extend,
-      segments(total_kv, num_kv_heads, head_dim, group * max_len_extend));
+  const int64_t cols = group * max_len_extend;
+  size_t split_need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend,
+                                                    segments(total_kv, num_kv_heads, head_dim, cols));
+  // a window, unknown here too, may make the launch one for shares
+  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, cols);
+  if (plan.share_len > 0)
+    split_need = std::max(split_need, msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols));
   // a sliding window (unknown here) may send the launch to the tile kernel instead
   const int ragged = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
   const size_t tile_need = ragged > 0 ? msgl::prefill_ragged_workspace_bytes(batch, total_kv, num_kv_heads, group,
@@ -351,8 +373,14 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
                                             sliding_window_size);
   if (direct) {
     const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, group * max_len_extend);
-    const size_t need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim,
-                                                      max_len_extend, n_seg);
+    const int64_t cols = group * max_len_extend;
+    const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, cols);
+    const bool shares = msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, cols,
+                                               sliding_window_size, max_len_extend);
+    const size_t need = shares
+                            ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group * max_len_extend)
+                            : msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim,
+                                                            max_len_extend, n_seg);
     if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;
     msgl::SplitKvArgs a{};
     a.q = q;
@@ -380,6 +408,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     a.n_seg = n_seg;
     a.min_seg = min_segment(head_dim);
     a.q_begin = 0;
+    if (shares) return msgl::launch_shares(a, plan, s);
     return msgl::launch_splitkv(a, s);
   }
   msgl::PrefillArgs a{};

@@ -57,6 +57,24 @@ int splitkv_scratch(void** ptr, size_t* bytes);
 // benchmarking switch: most waves (adjacent kv heads) a split-K workgroup may hold
 void splitkv_set_max_waves(int v);
 
+// ---- paged_shares.hip --------------------------------------------------------------
+// How a small launch is cut into shares of its requests' keys; share_len == 0: it is not
+struct SharePlan {
+  int32_t share_len;    // most keys of a share
+  int32_t share_waves;  // waves per share and kv head
+  int32_t heads_wg;     // adjacent kv heads of a workgroup
+  int64_t max_shares;   // most shares these sizes can give
+};
+SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols);
+// whether the launch is small enough for its shares to beat the segment kernel
+bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim,
+                      int64_t cols, int64_t window, int64_t max_len_extend);
+int device_cus();  // paged_splitkv.hip
+size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);
+int launch_shares(const SplitKvArgs& a, const SharePlan& plan, hipStream_t stream);
+// benchmarking switch: 0 default, negative never, else share_len | heads_wg << 20
+void shares_force(int64_t v);
+
 // ---- paged_prefill.hip -------------------------------------------------------------
 struct PrefillArgs {
   const void* q;

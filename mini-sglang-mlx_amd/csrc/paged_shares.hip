@@ -1,0 +1,382 @@
+// Paged attention for short query blocks (decode, verify) when the launch is small for the chip:
+// one workgroup per share of a request's keys, no second launch.
+//
+// The segment kernel (paged_splitkv.hip) is made for launches that the memory system bounds: one
+// round of equal segments, a merge launch behind it.  On a small launch what counts is the chain of
+// round trips and the second launch: a decode step of 4 requests with 1.7 K tokens in all took
+// 14 us of attention and 4 us of merge, one after the other, for 0.9 MB per layer and head group.
+//
+// Work decomposition
+//   A request's visible keys are cut into ceil(keys / share_len) equal shares.  A workgroup takes one
+//   share of `heads_wg` adjacent kv heads; `share_waves` waves cut the share of each head into
+//   adjacent ranges, so a share is read with every load of its first tiles in flight at once.  The
+//   waves of a head meet in LDS.  The grid holds the largest number of shares the sizes allow; a
+//   workgroup finds its (request, share) with one wave-wide prefix sum over kv_indptr and takes the
+//   request's geometry from the same registers; a workgroup past the last share ends.
+//   A request with one share is written at once.  Otherwise the share's normalised fp32 partial and
+//   its log-sum-exp go to the workspace, the workgroup counts itself in the request's count word, and
+//   the one that counts last reads the others and writes the result: nobody waits for anybody.
+//   Partials and counts travel at agent scope (they cross XCDs).  A count word is
+//   launch number << 16 | shares done; a word of any other launch counts as zero, so the workspace
+//   needs no clearing, and the last share puts the word back to zero, so a captured launch replays.
+#include <algorithm>
+#include <atomic>
+
+#include "splitkv_tiles.h"
+
+namespace msgl {
+namespace {
+
+struct ShareParams {
+  SplitKvParams s;
+  unsigned long long* counts;  // [batch][head_groups]
+  unsigned long long nonce;
+  int32_t share_len, share_waves, heads_wg, head_groups;
+};
+
+__device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
+  return (unsigned long long)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo);
+}
+__device__ __forceinline__ void st_agent(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_agent(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Share number `item` of the launch: its request, which of the request's shares it is, of how many.
+// All lanes must call; false past the last share.
+__device__ __forceinline__ bool find_share(const SplitKvParams& p, int share_len, int item, ReqInfo* r, int* b,
+                                           int* share, int* n_shares) {
+  const int lane = lane_id();
+  int base = 0;
+  for (int b0 = 0; b0 < p.batch; b0 += kWave) {
+    ReqInfo mine{};
+    int n = 0;
+    if (b0 + lane < p.batch) {
+      mine = request_info(p, b0 + lane);
+      // a request without visible keys has one empty share: its rows are zero
+      n = max((mine.hi - mine.lo + share_len - 1) / share_len, 1);
+    }
+    const int incl = wave_inclusive_scan(n);
+    const int sum = __builtin_amdgcn_readlane(incl, kWave - 1);
+    if (item < base + sum) {
+      const int first = base + incl - n;
+      const unsigned long long hit = __ballot(item >= first && item < first + n);
+      const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+      r->kv_start = __builtin_amdgcn_readlane(mine.kv_start, src);
+      r->kv_len = __builtin_amdgcn_readlane(mine.kv_len, src);
+      r->q_start = __builtin_amdgcn_readlane(mine.q_start, src);
+      r->q_len = __builtin_amdgcn_readlane(mine.q_len, src);
+      r->prefix = __builtin_amdgcn_readlane(mine.prefix, src);
+      r->lo = __builtin_amdgcn_readlane(mine.lo, src);
+      r->hi = __builtin_amdgcn_readlane(mine.hi, src);
+      *b = b0 + src;
+      *share = item - __builtin_amdgcn_readlane(first, src);
+      *n_shares = __builtin_amdgcn_readlane(n, src);
+      return true;
+    }
+    base += sum;
+  }
+  return false;
+}
+
+template <int D, int NCT, int NW, bool WIDE, bool F16>
+__global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(ShareParams sp) {
+  const SplitKvParams& p = sp.s;
+  constexpr int VH = D / 128;
+  constexpr int kCols = 16 * NCT;
+  constexpr int kBlock = kCols * 8 + 8;  // floats of one block of 8 dims: [col][8], padded
+  __shared__ __attribute__((aligned(16))) float part[NW][D / 8][kBlock];
+  __shared__ float2 state[NW][kCols];  // (maximum, sum) of a wave's columns
+  __shared__ int is_last;
+  const ClockProbe clock_probe_(p.clock_probe);
+  const int lane = lane_id();
+  const int t16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = blockIdx.x / sp.head_groups;
+  const int hg = blockIdx.x - item * sp.head_groups;
+  const int sub = wave / sp.share_waves;  // which of the workgroup's kv heads
+  const int sw = wave - sub * sp.share_waves;
+  const int kvh = hg * sp.heads_wg + sub;
+
+  ReqInfo r;
+  int b, share, n_shares;
+  if (!find_share(p, sp.share_len, item, &r, &b, &share, &n_shares)) return;  // the whole workgroup
+  const int ncols = r.q_len * p.group;
+  if (ncols == 0) return;
+  const int vis = r.hi - r.lo;
+  const int per = ((vis + n_shares - 1) / n_shares + 31) & ~31;
+  const int s_begin = min(r.lo + share * per, r.hi), s_end = min(s_begin + per, r.hi);
+  const int per_wave = ((per + sp.share_waves - 1) / sp.share_waves + 31) & ~31;
+  const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
+
+  unsigned long long* const cnt = sp.counts + (int64_t)b * sp.head_groups + hg;
+  const unsigned long long fresh = sp.nonce << 16;
+  // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
+  // for it: whoever finds the word not made yet makes it (below).
+  if (n_shares > 1 && share == 0 && threadIdx.x == 0) {
+    unsigned long long seen = ld_agent(cnt);
+    if ((seen >> 16) != sp.nonce)
+      (void)__hip_atomic_compare_exchange_strong(cnt, &seen, fresh, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+  }
+
+  Columns<D, NCT> c;
+  start_columns(p, r, kvh, 0, t_end, c);
+  if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16>(p, r, kvh, t_begin, t_end, c);
+
+  // ---- the waves of a kv head meet in LDS ---------------------------------------------------
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    float l = c.l[ct];
+    l += __shfl_xor(l, 16, kWave);
+    l += __shfl_xor(l, 32, kWave);
+    const int col = ct * 16 + t16;
+    if (col >= ncols) continue;
+    if (g == 0) state[wave][col] = float2{c.m[ct], l};
+#pragma unroll
+    for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f32x4_t w0, w1;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          w0[n] = c.o[ct][hf][n][i];
+          w1[n] = c.o[ct][hf][4 + n][i];
+        }
+        float* dst = &part[wave][hf * 16 + 4 * g + i][col * 8];
+        *reinterpret_cast<f32x4_t*>(dst) = w0;
+        *reinterpret_cast<f32x4_t*>(dst + 4) = w1;
+      }
+  }
+  __syncthreads();
+
+  constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column
+  const int threads = 64 * sp.share_waves;
+  const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols;
+  for (int it = threadIdx.x - sub * threads; it < ncols * kQuads; it += threads) {
+    const int col = it / kQuads, d4 = (it - col * kQuads) * 4;
+    float m = kNegInf;
+    for (int w = 0; w < sp.share_waves; ++w) m = fmaxf(m, state[sub * sp.share_waves + w][col].x);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    const float m_safe = (m == kNegInf) ? 0.f : m;
+    for (int w = 0; w < sp.share_waves; ++w) {
+      const float2 ml = state[sub * sp.share_waves + w][col];
+      const float e = fast_exp2(ml.x - m_safe);  // 0 for a wave without visible keys
+      acc += e * *reinterpret_cast<const f32x4_t*>(&part[sub * sp.share_waves + w][d4 >> 3][col * 8 + (d4 & 7)]);
+      l += e * ml.y;
+    }
+    acc *= (l > 0.f) ? 1.0f / l : 0.f;
+    if (n_shares == 1) {
+      const int qi = col / p.group;
+      uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4;
+      *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(acc[0], acc[1]), pack_16x2<F16>(acc[2], acc[3])};
+    } else {
+      unsigned long long* dst = reinterpret_cast<unsigned long long*>(p.part_o + (row0 + col) * D + d4);
+      st_agent(dst, pair_bits(acc[0], acc[1]));
+      st_agent(dst + 1, pair_bits(acc[2], acc[3]));
+      if (d4 == 0)
+        __hip_atomic_store(p.part_lse + row0 + col, (l > 0.f) ? m + __log2f(l) : kNegInf, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (n_shares == 1) return;
+
+  // ---- the share that counts last puts the request together ------------------------------------
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are where every CU sees them
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    // one addition where the word is this launch's already; an addition to a word that was not did
+    // not count, and the loop counts this share whatever the others do meanwhile
+    unsigned long long seen = __hip_atomic_fetch_add(cnt, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long want = seen + 1;
+    if ((seen >> 16) != sp.nonce) {
+      seen = ld_agent(cnt);
+      do {
+        want = ((seen >> 16) == sp.nonce ? seen : fresh) + 1;
+      } while (!__hip_atomic_compare_exchange_strong(cnt, &seen, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT));
+    }
+    const bool last = (int)(want & 0xffff) == n_shares;
+    if (last) st_agent(cnt, 0ull);
+    is_last = last;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  constexpr int U = 8;                  // shares whose loads are in flight together ...
+  constexpr int I = NW == 4 ? 2 : 1;    // ... for this many of a thread's quads
+  const int64_t step = (int64_t)p.n_kv * p.cols;  // rows from one share to the next
+  const int64_t first = ((int64_t)(item - share) * p.n_kv + kvh) * p.cols;
+  const int quads = ncols * kQuads;
+  for (int it0 = threadIdx.x - sub * threads; it0 < quads; it0 += I * threads) {
+    float m[I], l[I];
+    f32x4_t acc[I];
+    int64_t row[I];
+    int d4[I];
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int it = min(it0 + i * threads, quads - 1);  // past the end: the last quad again, not written
+      row[i] = first + it / kQuads;
+      d4[i] = (it % kQuads) * 4;
+      m[i] = kNegInf;
+      l[i] = 0.f;
+      acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int s0 = 0; s0 < n_shares; s0 += U) {
+      float lse[I][U];
+      unsigned long long lo[I][U], hi[I][U];
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {  // shares past the last one: the last again, with weight 0
+          const int64_t at = row[i] + min(s0 + u, n_shares - 1) * step;
+          const unsigned long long* src = reinterpret_cast<const unsigned long long*>(p.part_o + at * D + d4[i]);
+          lse[i][u] = __hip_atomic_load(p.part_lse + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          lo[i][u] = ld_agent(src);
+          hi[i][u] = ld_agent(src + 1);
+          if (s0 + u >= n_shares) lse[i][u] = kNegInf;
+        }
+#pragma unroll
+      for (int i = 0; i < I; ++i) {
+        float m_new = m[i];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m_new = fmaxf(m_new, lse[i][u]);
+        const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
+        const float old = fast_exp2(m[i] - m_safe);
+        acc[i] *= old;
+        l[i] *= old;
+        m[i] = m_new;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float e = fast_exp2(lse[i][u] - m_safe);
+          acc[i][0] += e * __builtin_bit_cast(float, (uint32_t)lo[i][u]);
+          acc[i][1] += e * __builtin_bit_cast(float, (uint32_t)(lo[i][u] >> 32));
+          acc[i][2] += e * __builtin_bit_cast(float, (uint32_t)hi[i][u]);
+          acc[i][3] += e * __builtin_bit_cast(float, (uint32_t)(hi[i][u] >> 32));
+          l[i] += e;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      if (it0 + i * threads >= quads) break;
+      const int col = (int)(row[i] - first), qi = col / p.group;
+      const f32x4_t o = acc[i] * ((l[i] > 0.f) ? 1.0f / l[i] : 0.f);
+      uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4[i];
+      *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(o[0], o[1]), pack_16x2<F16>(o[2], o[3])};
+    }
+  }
+}
+
+int nct_of(int64_t cols) { return (int)((cols + 15) / 16); }
+// waves of a workgroup: two per SIMD where a wave fits 256 registers
+int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
+
+template <int D, int NCT, int NW>
+int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
+  const dim3 grid(blocks), block(64 * NW);
+  if constexpr (NCT == 1) {  // IEEE half exists for decode only (one column tile)
+    if (sp.s.f16) {
+      if (sp.s.wide) hipLaunchKernelGGL((share_attention_kernel<D, NCT, NW, true, true>), grid, block, 0, stream, sp);
+      else hipLaunchKernelGGL((share_attention_kernel<D, NCT, NW, false, true>), grid, block, 0, stream, sp);
+      return check_launch();
+    }
+  }
+  if (sp.s.f16) return MSGL_ERR_DTYPE;
+  if (sp.s.wide) hipLaunchKernelGGL((share_attention_kernel<D, NCT, NW, true, false>), grid, block, 0, stream, sp);
+  else hipLaunchKernelGGL((share_attention_kernel<D, NCT, NW, false, false>), grid, block, 0, stream, sp);
+  return check_launch();
+}
+
+thread_local int64_t t_force = 0;  // benchmarking switch, see shares_force()
+std::atomic<unsigned long long> g_nonce{1};
+
+}  // namespace
+
+void shares_force(int64_t v) { t_force = v; }
+
+SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols) {
+  SharePlan plan{};
+  const int nct = nct_of(cols);
+  if (t_force < 0 || batch < 1 || cols < 1 || nct > (head_dim == 128 ? 3 : 1)) return plan;
+  const int nw = waves_of(head_dim, nct);
+  const int64_t slots = device_cus();  // a workgroup takes a CU
+  int64_t heads = 1, len;
+  if (t_force > 0) {
+    len = t_force & 0xfffff;
+    heads = t_force >> 20;
+    if (heads < 1 || heads > nw || n_kv % heads != 0 || nw % heads != 0) heads = 1;
+  } else {
+    // as many waves on one kv head as possible while the requests alone do not fill the chip
+    while (batch * n_kv > slots * heads && 2 * heads <= nw && n_kv % (2 * heads) == 0) heads *= 2;
+    // the shortest shares that fit the chip in one round (half a share of rounding per request), and
+    // at most 16 of an average request: the last of them reads the others' partials
+    len = nct == 3 ? 512 : (nw == 4 && heads == 1) ? 256 : 128;
+    auto fits = [&](int64_t c) {
+      return std::max(batch, total_kv / c + batch / 2) * (n_kv / heads) <= slots && total_kv <= 16 * c * batch;
+    };
+    while (!fits(len) && len < (1 << 19)) len *= 2;
+  }
+  plan.share_len = (int32_t)len;
+  plan.heads_wg = (int32_t)heads;
+  plan.share_waves = nw / plan.heads_wg;
+  plan.max_shares = total_kv / plan.share_len + batch;
+  return plan;
+}
+
+// Measured against the segment kernel and its merge on 140 random shapes (1-256 requests of 1-60 K
+// keys, 1-16 queries, both head sizes; us, segments -> shares): 46 x 4-18 keys 42.1 -> 7.3, 64 x 20-200
+// 18.9 -> 11.3, 200 x 6-99 28.5 -> 18.0, 4 x 37-1023 15.7 -> 9.1, one of 2 K 13.5 -> 10.3, 24 x 127-4095
+// at head_dim 256 35.9 -> 28.1.  Short requests gain most (a segment pays 8 us for each request
+// boundary it crosses) and up to the largest launches; where requests are long the segments' fixed
+// costs are the same for any number of bytes, while a share's last workgroup has ever more partials
+// to read and the shares' lengths vary: one request of 12 K keys 16.6 -> 19.2, 12 of 3-8 K 59 -> 71.
+// The lines lie where the two meet.
+bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim,
+                      int64_t cols, int64_t window, int64_t max_len_extend) {
+  if (plan.share_len == 0) return false;
+  if (t_force > 0) return true;
+  int64_t keys = total_kv;
+  if (window > 0) keys = std::min(keys, batch * (window + max_len_extend + 15));
+  const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch;
+  if (mean <= 512) return mb <= 160;
+  // few units: most of the time is the last share's, which reads all the others of a wide head group
+  if (head_dim == 256 && batch * n_kv < 12) return false;
+  if (mean <= 4096) return mb <= (head_dim == 256 ? 128 : 56);
+  return mb <= (mean <= 8192 ? 36 : 20);
+}
+
+size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {
+  const size_t counts = (size_t)(batch * (n_kv / plan.heads_wg)) * sizeof(unsigned long long);
+  const size_t rows = (size_t)plan.max_shares * (size_t)(n_kv * cols);
+  return ((counts + 255) / 256 + (rows * (size_t)(head_dim + 1) * sizeof(float) + 255) / 256) * 256;
+}
+
+int launch_shares(const SplitKvArgs& a, const SharePlan& plan, hipStream_t stream) {
+  const int64_t group = a.n_q / a.n_kv, cols = group * a.max_len_extend;
+  const int64_t head_groups = a.n_kv / plan.heads_wg;
+  const int64_t blocks = plan.max_shares * head_groups;
+  if (blocks > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
+  ShareParams sp{};
+  fill_splitkv_params(a, sp.s);
+  char* ws = static_cast<char*>(a.workspace);
+  sp.counts = reinterpret_cast<unsigned long long*>(ws);
+  ws += ((size_t)(a.batch * head_groups) * sizeof(unsigned long long) + 255) / 256 * 256;
+  sp.s.part_o = reinterpret_cast<float*>(ws);
+  sp.s.part_lse = sp.s.part_o + (size_t)plan.max_shares * (size_t)(a.n_kv * cols * a.head_dim);
+  sp.nonce = g_nonce.fetch_add(1, std::memory_order_relaxed) & ((1ull << 47) - 1);
+  if (sp.nonce == 0) sp.nonce = g_nonce.fetch_add(1, std::memory_order_relaxed);
+  sp.share_len = plan.share_len;
+  sp.share_waves = plan.share_waves;
+  sp.heads_wg = plan.heads_wg;
+  sp.head_groups = (int32_t)head_groups;
+  const int nct = nct_of(cols);
+  if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
+  if (nct == 1) return launch_shape<128, 1, 8>(sp, (unsigned)blocks, stream);
+  if (nct == 2) return launch_shape<128, 2, 4>(sp, (unsigned)blocks, stream);
+  return nct == 3 ? launch_shape<128, 3, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
+}
+
+}  // namespace msgl

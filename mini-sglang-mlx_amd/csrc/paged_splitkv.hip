@@ -41,74 +41,10 @@
 #include <atomic>
 #include <type_traits>
 
-#include "msgl_device.h"
-#include "msgl_internal.h"
+#include "splitkv_tiles.h"
 
 namespace msgl {
 namespace {
-
-struct SplitKvParams {
-  const uint16_t* q;
-  const uint16_t* k_cache;
-  const uint16_t* v_cache;
-  const int32_t* kv_indptr;
-  const int32_t* kv_indices;
-  const int32_t* qo_indptr;
-  const int32_t* prefix_lens;
-  uint16_t* out;
-  float* part_o;        // [n_seg + batch][n_kv][D / 8][cols][8], fp32 or IEEE half: see partial_offset()
-  float* part_lse;      // [n_seg + batch][n_kv][cols]
-  int32_t* req_items;   // [batch][2] first segment holding the request, number of segments sharing it
-  int64_t k_stride0, v_stride0;
-  int32_t batch, n_q, n_kv, group;
-  int32_t nwh;          // kv heads per workgroup
-  int32_t head_groups;  // n_kv / nwh
-  int32_t n_seg, min_seg, cols, max_len_extend;
-  int32_t boundary;  // stream positions a request boundary is charged with (see stream_length)
-  int32_t q_begin, q_cap;  // first query of every request in this launch; cap on a request's queries
-  int32_t f16;             // elements are IEEE half instead of bf16
-  int32_t is_cross, window;
-  int32_t wide;  // pool byte offsets need 64 bits
-  uint32_t max_slot;  // num_slots - 1: slot ids are clamped to it before they become addresses
-  float scale_log2e;
-  long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
-};
-
-// Visible key range and query geometry of one request.
-struct ReqInfo {
-  int32_t kv_start, kv_len;  // CSR segment
-  int32_t q_start, q_len;    // rows of q / out
-  int32_t prefix;            // position of query 0
-  int32_t lo, hi;            // keys [lo, hi) can be visible to some query of the request
-};
-
-__device__ __forceinline__ ReqInfo request_info(const SplitKvParams& p, int b) {
-  ReqInfo r;
-  r.kv_start = p.kv_indptr[b];
-  r.kv_len = p.kv_indptr[b + 1] - r.kv_start;
-  if (r.kv_len < 0) r.kv_len = 0;
-  if (p.qo_indptr == nullptr) {
-    r.q_start = b;
-    r.q_len = 1;
-    r.prefix = r.kv_len - 1;
-  } else {
-    // this launch covers queries q_begin .. q_begin + max_len_extend - 1 of every request
-    const int q0 = p.qo_indptr[b];
-    const int q_all = min(p.qo_indptr[b + 1] - q0, p.q_cap);
-    r.q_start = q0 + p.q_begin;
-    r.q_len = max(min(q_all - p.q_begin, p.max_len_extend), 0);
-    r.prefix = p.prefix_lens[b] + p.q_begin;
-  }
-  // first query has the lowest window floor, last query the highest causal limit
-  r.lo = (p.window > 0) ? max(0, r.prefix - p.window + 1) : 0;
-  r.lo &= ~15;
-  r.hi = p.is_cross ? r.kv_len : min(r.kv_len, r.prefix + r.q_len);
-  if (r.q_len <= 0 || r.hi <= r.lo) {
-    r.lo = 0;
-    r.hi = 0;
-  }
-  return r;
-}
 
 // Element type of the partials.  bf16 launches keep them as IEEE half: a normalised partial row is
 // a weighted mean of V rows, every bf16 value of ordinary size is a half value exactly (a share
@@ -207,19 +143,12 @@ __device__ __forceinline__ bool locate_segment(const SplitKvParams& p, int seg, 
   return false;
 }
 
-template <int D>
-struct KvTile {
-  u32x4_t k[2][D / 32];   // [16-token sub-tile][32-wide slice of D]: MFMA A operand of S^T
-  u32x4_t v[D / 128][8];  // [128-wide half of D][token j of the lane group]: raw V segments
-};
-
 // NCT = tiles of 16 columns per wave, NW = waves per workgroup (launch bound only).  One
 // column tile at head dim 128 fits 256 VGPRs, so two such waves per SIMD can be resident.
 // WIDE: pool byte offsets need 64 bits (a pool of 4 GiB or more); otherwise a row's offset is
 // one 32-bit multiply instead of a 64-bit multiply-add per load.
 template <int D, int NCT, int NW, bool WIDE, bool F16>
 __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void splitkv_attention_kernel(SplitKvParams p) {
-  constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const ClockProbe clock_probe_(p.clock_probe);
   const int lane = lane_id();
@@ -237,17 +166,6 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
   vs = __builtin_amdgcn_readfirstlane(vs);
   int vpos = seg * seg_len;
   const int seg_end = min(vpos + seg_len, total);
-
-  const unsigned char* kbase =
-      reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * D + g * 8);
-  const unsigned char* vbase =
-      reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * D + t16 * 8);
-  const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
-  const uint32_t v_row_bytes = (uint32_t)p.v_stride0 * 2u;
-  auto row_offset = [](int slot_id, uint32_t row_bytes) -> uint64_t {
-    if constexpr (WIDE) return (uint64_t)(uint32_t)slot_id * row_bytes;
-    else return (uint64_t)((uint32_t)slot_id * row_bytes);
-  };
 
   while (vpos < seg_end && cur_b < p.batch) {
     const ReqInfo r = request_info(p, cur_b);
@@ -269,189 +187,14 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     }
     const int ncols = r.q_len * p.group;
 
-    // ---- Q operand and per-column visibility bounds --------------------------------
-    u32x4_t qreg[NCT][KS];
-    int col_lo[NCT], col_hi[NCT];
-    int all_lo = 0, all_hi = 0x7fffffff;  // tile is mask-free iff inside [all_lo, all_hi]
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-      const int col = (ct0 + ct) * 16 + t16;
-      const bool valid = col < ncols;
-      const int qi = valid ? col / p.group : 0;
-      const int hh = valid ? col - qi * p.group : 0;
-      const uint16_t* qrow =
-          p.q + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + hh) * D + g * 8;
-#pragma unroll
-      for (int c = 0; c < KS; ++c) {
-        u32x4_t raw = {0u, 0u, 0u, 0u};
-        if (valid) raw = ld_global_b128(qrow + c * 32);
-        qreg[ct][c] = raw;
-      }
-      const int qpos = r.prefix + qi;
-      int lo = (p.window > 0) ? qpos - p.window + 1 : 0;
-      int hi = p.is_cross ? r.kv_len - 1 : min(qpos, r.kv_len - 1);
-      hi = min(hi, t_end - 1);
-      if (valid) {
-        all_lo = max(all_lo, lo);
-        all_hi = min(all_hi, hi);
-      } else {
-        lo = 1;
-        hi = 0;
-      }
-      col_lo[ct] = lo;
-      col_hi[ct] = hi;
-    }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-      all_lo = max(all_lo, __shfl_xor(all_lo, off, kWave));
-      all_hi = min(all_hi, __shfl_xor(all_hi, off, kWave));
-    }
-    all_lo = __builtin_amdgcn_readfirstlane(all_lo);
-    all_hi = __builtin_amdgcn_readfirstlane(all_hi);
-
-    // ---- accumulators ----------------------------------------------------------------
-    f32x4_t oacc[NCT][VH][8];
-    float m_run[NCT], l_run[NCT];
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-      m_run[ct] = kNegInf;
-      l_run[ct] = 0.f;
-#pragma unroll
-      for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-        for (int n = 0; n < 8; ++n) oacc[ct][hf][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-
-    const int32_t* idx_base = p.kv_indices + r.kv_start;
-    const int last_tok = t_end - 1;
-
-    // slot ids of the two K rows this lane loads in a 32-token tile starting at tb
-    auto load_idx = [&](int tb, int& s0, int& s1) {
-      s0 = (int)min((uint32_t)idx_base[min(tb + t16, last_tok)], p.max_slot);
-      s1 = (int)min((uint32_t)idx_base[min(tb + 16 + t16, last_tok)], p.max_slot);
-    };
-    auto load_tile = [&](KvTile<D>& t, int s0, int s1) {
-#pragma unroll
-      for (int c = 0; c < KS; ++c) {
-        t.k[0][c] = ld_global_b128(kbase + row_offset(s0, k_row_bytes) + c * 64);
-        t.k[1][c] = ld_global_b128(kbase + row_offset(s1, k_row_bytes) + c * 64);
-      }
-      // V rows of this lane group: tokens 4g+j (j<4) of sub-tile 0, then of sub-tile 1;
-      // their slot ids sit in lanes 4g+j of the K index registers.
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int src = 4 * g + (j & 3);
-        const int slot = __shfl(j < 4 ? s0 : s1, src, kWave);
-        const unsigned char* vrow = vbase + row_offset(slot, v_row_bytes);
-#pragma unroll
-        for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = ld_global_b128(vrow + hf * 256);
-      }
-    };
-
-    auto compute_tile = [&](const KvTile<D>& t, int tb) {
-      // S^T[token][col] for the two 16-token sub-tiles
-      f32x4_t s[2][NCT];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-          f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int c = 0; c < KS; ++c)
-            acc = mfma_16x16x32_raw<F16>(t.k[sub][c], qreg[ct][c], acc);
-          s[sub][ct] = acc;
-        }
-      const bool need_mask = (tb < all_lo) || (tb + 31 > all_hi);
-      uint32_t pb[NCT][4];
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        float x[2][4];
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) x[sub][i] = s[sub][ct][i] * p.scale_log2e;
-        if (need_mask) {
-#pragma unroll
-          for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int tok = tb + sub * 16 + 4 * g + i;
-              if (tok < col_lo[ct] || tok > col_hi[ct]) x[sub][i] = kNegInf;
-            }
-        }
-        float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
-                         fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
-        mx = wave_max_xor(mx, 16);
-        mx = wave_max_xor(mx, 32);
-        const float m_new = fmaxf(m_run[ct], mx);
-        const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
-        const float alpha = fast_exp2(m_run[ct] - m_safe);
-        m_run[ct] = m_new;
-        float psum = 0.f;
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            x[sub][i] = fast_exp2(x[sub][i] - m_safe);
-            psum += x[sub][i];
-          }
-        l_run[ct] = l_run[ct] * alpha + psum;
-        pb[ct][0] = pack_16x2<F16>(x[0][0], x[0][1]);
-        pb[ct][1] = pack_16x2<F16>(x[0][2], x[0][3]);
-        pb[ct][2] = pack_16x2<F16>(x[1][0], x[1][1]);
-        pb[ct][3] = pack_16x2<F16>(x[1][2], x[1][3]);
-        if (__any(alpha != 1.0f)) {
-#pragma unroll
-          for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-            for (int n = 0; n < 8; ++n) oacc[ct][hf][n] *= alpha;
-        }
-      }
-      // O^T += V^T P^T.  MFMA n of half hf produces d = hf*128 + 8*row + n on row = l%16.
-#pragma unroll
-      for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-          u32x4_t vt;
-#pragma unroll
-          for (int qd = 0; qd < 4; ++qd) {
-            const uint32_t a = t.v[hf][2 * qd][n >> 1];
-            const uint32_t c = t.v[hf][2 * qd + 1][n >> 1];
-            vt[qd] = (n & 1) ? pack_hi16(a, c) : pack_lo16(a, c);
-          }
-#pragma unroll
-          for (int ct = 0; ct < NCT; ++ct) {
-            const u32x4_t pv = {pb[ct][0], pb[ct][1], pb[ct][2], pb[ct][3]};
-            oacc[ct][hf][n] = mfma_16x16x32_raw<F16>(vt, pv, oacc[ct][hf][n]);
-          }
-        }
-    };
-
-    // ---- tile loop: two register tiles, slot ids fetched two tiles ahead.  Every load in
-    // the loop body is unconditional (tokens past the range clamp to its last token and
-    // are masked), so the number of loads in flight at each wait is a compile-time
-    // constant and the next tile stays in flight while the current one is computed. ----
-    const int n_pairs = (t_end - t_begin + 63) / 64;
-    KvTile<D> ta, tb_;
-    int i0a, i0b, i1a, i1b;
-    load_idx(t_begin, i0a, i0b);
-    load_idx(t_begin + 32, i1a, i1b);
-    load_tile(ta, i0a, i0b);
-    load_idx(t_begin + 64, i0a, i0b);
-    for (int pr = 0; pr < n_pairs; ++pr) {
-      const int tok = t_begin + pr * 64;
-      load_tile(tb_, i1a, i1b);
-      load_idx(tok + 96, i1a, i1b);
-      compute_tile(ta, tok);
-      load_tile(ta, i0a, i0b);
-      load_idx(tok + 128, i0a, i0b);
-      compute_tile(tb_, tok + 32);
-    }
+    Columns<D, NCT> c_;
+    start_columns(p, r, kvh, ct0, t_end, c_);
+    attend_keys<D, NCT, WIDE, F16>(p, r, kvh, t_begin, t_end, c_);
 
     // ---- this request's share is done: write output or partial -------------------------
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
-      float l = l_run[ct];
+      float l = c_.l[ct];
       l += __shfl_xor(l, 16, kWave);
       l += __shfl_xor(l, 32, kWave);
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
@@ -468,7 +211,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
             u32x4_t w;
 #pragma unroll
             for (int n = 0; n < 4; ++n)
-              w[n] = pack_16x2<F16>(oacc[ct][hf][2 * n][i] * inv, oacc[ct][hf][2 * n + 1][i] * inv);
+              w[n] = pack_16x2<F16>(c_.o[ct][hf][2 * n][i] * inv, c_.o[ct][hf][2 * n + 1][i] * inv);
             st_global_b128(orow + hf * 128 + (4 * g + i) * 8, w);
           }
       } else {
@@ -481,8 +224,8 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
               f32x4_t w0, w1;
 #pragma unroll
               for (int n = 0; n < 4; ++n) {
-                w0[n] = oacc[ct][hf][n][i] * inv;
-                w1[n] = oacc[ct][hf][4 + n][i] * inv;
+                w0[n] = c_.o[ct][hf][n][i] * inv;
+                w1[n] = c_.o[ct][hf][4 + n][i] * inv;
               }
               float* dst = p.part_o + partial_offset(block, p.cols, col, hf * 128 + (4 * g + i) * 8, D);
               *reinterpret_cast<f32x4_t*>(dst) = w0;
@@ -496,13 +239,13 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
               u32x4_t w;
 #pragma unroll
               for (int n = 0; n < 4; ++n)
-                w[n] = pack_half2_clamped(oacc[ct][hf][2 * n][i] * inv, oacc[ct][hf][2 * n + 1][i] * inv);
+                w[n] = pack_half2_clamped(c_.o[ct][hf][2 * n][i] * inv, c_.o[ct][hf][2 * n + 1][i] * inv);
               _Float16* dst = reinterpret_cast<_Float16*>(p.part_o) +
                               partial_offset(block, p.cols, col, hf * 128 + (4 * g + i) * 8, D);
               *reinterpret_cast<u32x4_t*>(dst) = w;
             }
         }
-        if (g == 0) p.part_lse[block * p.cols + col] = (l > 0.f) ? m_run[ct] + __log2f(l) : kNegInf;
+        if (g == 0) p.part_lse[block * p.cols + col] = (l > 0.f) ? c_.m[ct] + __log2f(l) : kNegInf;
       }
     }
 
@@ -705,21 +448,6 @@ int heads_per_group(int64_t n_kv) {
   return (cap >= 2 && n_kv % 2 == 0) ? 2 : 1;
 }
 
-int device_cus() {
-  static std::atomic<int> cache{0};
-  int v = cache.load();
-  if (v > 0) return v;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0) {
-    (void)hipGetLastError();
-    return 256;  // MI355X
-  }
-  cache.store(cus);
-  return cus;
-}
-
 template <int D, int NCT, int NW>
 void launch_attn(const SplitKvParams& p, hipStream_t stream) {
   const dim3 grid((unsigned)(p.n_seg * p.head_groups)), block(64 * NW);
@@ -818,6 +546,21 @@ int splitkv_scratch(void** ptr, size_t* bytes) {
   return MSGL_OK;
 }
 
+int device_cus() {
+  static std::atomic<int> cache{0};
+  int v = cache.load();
+  if (v > 0) return v;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus <= 0) {
+    (void)hipGetLastError();
+    return 256;  // MI355X
+  }
+  cache.store(cus);
+  return cus;
+}
+
 void splitkv_set_max_waves(int v) { t_max_waves = v > 0 ? v : 4; }  // 0 restores the default
 
 // benchmarking switch, one value per host thread: stream positions charged per request boundary
@@ -878,17 +621,7 @@ size_t splitkv_workspace_bytes(int64_t batch, int64_t n_q, int64_t n_kv, int64_t
   return (bytes + 255) / 256 * 256 + 256;
 }
 
-int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
-  const int64_t group = a.n_q / a.n_kv;
-  const int64_t cols = group * a.max_len_extend;
-  if (cols < 1 || cols > kSplitKvMaxCols || a.n_seg < 1 || a.min_seg < 64 || a.min_seg % 64 != 0)
-    return MSGL_ERR_SHAPE;
-  if (a.batch * a.max_len_extend > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  if (a.batch == 0) return MSGL_OK;
-  const int nct = nct_for(cols);
-  const int nwh = nwh_for(a.n_kv, nct, a.head_dim);
-
-  SplitKvParams p;
+void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   p.q = static_cast<const uint16_t*>(a.q);
   p.k_cache = static_cast<const uint16_t*>(a.k_cache);
   p.v_cache = static_cast<const uint16_t*>(a.v_cache);
@@ -897,24 +630,14 @@ int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
   p.qo_indptr = a.qo_indptr;
   p.prefix_lens = a.prefix_lens;
   p.out = static_cast<uint16_t*>(a.out);
-  p.cols = (int32_t)cols;
-  const int64_t rows = ((int64_t)a.n_seg + a.batch) * a.n_kv * cols;
-  char* ws = static_cast<char*>(a.workspace);
-  p.part_o = reinterpret_cast<float*>(ws);
-  p.part_lse = reinterpret_cast<float*>(ws + (size_t)rows * a.head_dim * sizeof(float));
-  p.req_items = reinterpret_cast<int32_t*>(ws + (size_t)rows * (a.head_dim + 1) * sizeof(float));
+  p.group = (int32_t)(a.n_q / a.n_kv);
+  p.cols = p.group * a.max_len_extend;
   p.k_stride0 = a.k_stride0;
   p.v_stride0 = a.v_stride0;
   p.batch = (int32_t)a.batch;
   p.n_q = (int32_t)a.n_q;
   p.n_kv = (int32_t)a.n_kv;
-  p.group = (int32_t)group;
   p.max_slot = (uint32_t)(a.num_slots > 0 ? a.num_slots - 1 : 0);
-  p.nwh = nwh;
-  p.head_groups = (int32_t)(a.n_kv / nwh);
-  p.n_seg = a.n_seg;
-  p.boundary = boundary_tokens((int64_t)a.n_seg * (a.n_kv / nwh), nwh, a.head_dim);
-  p.min_seg = a.min_seg;
   p.max_len_extend = a.max_len_extend;
   p.f16 = a.f16;
   p.q_begin = a.q_begin;
@@ -925,6 +648,29 @@ int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
   p.clock_probe = clock_probe();
   p.wide = ((uint64_t)a.num_slots * (uint64_t)a.k_stride0 * 2u >= (1ull << 32) ||
             (uint64_t)a.num_slots * (uint64_t)a.v_stride0 * 2u >= (1ull << 32)) ? 1 : 0;
+}
+
+int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
+  const int64_t cols = a.n_q / a.n_kv * a.max_len_extend;
+  if (cols < 1 || cols > kSplitKvMaxCols || a.n_seg < 1 || a.min_seg < 64 || a.min_seg % 64 != 0)
+    return MSGL_ERR_SHAPE;
+  if (a.batch * a.max_len_extend > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
+  if (a.batch == 0) return MSGL_OK;
+  const int nct = nct_for(cols);
+  const int nwh = nwh_for(a.n_kv, nct, a.head_dim);
+
+  SplitKvParams p{};
+  fill_splitkv_params(a, p);
+  const int64_t rows = ((int64_t)a.n_seg + a.batch) * a.n_kv * cols;
+  char* ws = static_cast<char*>(a.workspace);
+  p.part_o = reinterpret_cast<float*>(ws);
+  p.part_lse = reinterpret_cast<float*>(ws + (size_t)rows * a.head_dim * sizeof(float));
+  p.req_items = reinterpret_cast<int32_t*>(ws + (size_t)rows * (a.head_dim + 1) * sizeof(float));
+  p.nwh = nwh;
+  p.head_groups = (int32_t)(a.n_kv / nwh);
+  p.n_seg = a.n_seg;
+  p.boundary = boundary_tokens((int64_t)a.n_seg * (a.n_kv / nwh), nwh, a.head_dim);
+  p.min_seg = a.min_seg;
   if ((int64_t)p.n_seg * p.head_groups > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   if (a.head_dim == 128) return launch_d<128>(p, nct, stream);
   if (a.head_dim == 256) return launch_d<256>(p, nct, stream);

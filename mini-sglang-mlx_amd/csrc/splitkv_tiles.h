@@ -1,0 +1,293 @@
+// What the kernels for short query blocks share (paged_splitkv.hip: equal segments of the token
+// stream; paged_shares.hip: shares of one request): launch parameters, a request's geometry, and
+// one wave's walk over a range of keys with its columns' softmax state in registers.
+#pragma once
+#include "msgl_device.h"
+#include "msgl_internal.h"
+
+namespace msgl {
+
+struct SplitKvParams {
+  const uint16_t* q;
+  const uint16_t* k_cache;
+  const uint16_t* v_cache;
+  const int32_t* kv_indptr;
+  const int32_t* kv_indices;
+  const int32_t* qo_indptr;
+  const int32_t* prefix_lens;
+  uint16_t* out;
+  float* part_o;        // [n_seg + batch][n_kv][D / 8][cols][8], fp32 or IEEE half: see partial_offset()
+  float* part_lse;      // [n_seg + batch][n_kv][cols]
+  int32_t* req_items;   // [batch][2] first segment holding the request, number of segments sharing it
+  int64_t k_stride0, v_stride0;
+  int32_t batch, n_q, n_kv, group;
+  int32_t nwh;          // kv heads per workgroup
+  int32_t head_groups;  // n_kv / nwh
+  int32_t n_seg, min_seg, cols, max_len_extend;
+  int32_t boundary;  // stream positions a request boundary is charged with (see stream_length)
+  int32_t q_begin, q_cap;  // first query of every request in this launch; cap on a request's queries
+  int32_t f16;             // elements are IEEE half instead of bf16
+  int32_t is_cross, window;
+  int32_t wide;  // pool byte offsets need 64 bits
+  uint32_t max_slot;  // num_slots - 1: slot ids are clamped to it before they become addresses
+  float scale_log2e;
+  long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
+};
+
+// Everything but the workspace pointers and the cut (paged_splitkv.hip).
+void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p);
+
+// Visible key range and query geometry of one request.
+struct ReqInfo {
+  int32_t kv_start, kv_len;  // CSR segment
+  int32_t q_start, q_len;    // rows of q / out
+  int32_t prefix;            // position of query 0
+  int32_t lo, hi;            // keys [lo, hi) can be visible to some query of the request
+};
+
+__device__ __forceinline__ ReqInfo request_info(const SplitKvParams& p, int b) {
+  ReqInfo r;
+  r.kv_start = p.kv_indptr[b];
+  r.kv_len = p.kv_indptr[b + 1] - r.kv_start;
+  if (r.kv_len < 0) r.kv_len = 0;
+  if (p.qo_indptr == nullptr) {
+    r.q_start = b;
+    r.q_len = 1;
+    r.prefix = r.kv_len - 1;
+  } else {
+    // this launch covers queries q_begin .. q_begin + max_len_extend - 1 of every request
+    const int q0 = p.qo_indptr[b];
+    const int q_all = min(p.qo_indptr[b + 1] - q0, p.q_cap);
+    r.q_start = q0 + p.q_begin;
+    r.q_len = max(min(q_all - p.q_begin, p.max_len_extend), 0);
+    r.prefix = p.prefix_lens[b] + p.q_begin;
+  }
+  // first query has the lowest window floor, last query the highest causal limit
+  r.lo = (p.window > 0) ? max(0, r.prefix - p.window + 1) : 0;
+  r.lo &= ~15;
+  r.hi = p.is_cross ? r.kv_len : min(r.kv_len, r.prefix + r.q_len);
+  if (r.q_len <= 0 || r.hi <= r.lo) {
+    r.lo = 0;
+    r.hi = 0;
+  }
+  return r;
+}
+
+template <int D>
+struct KvTile {
+  u32x4_t k[2][D / 32];   // [16-token sub-tile][32-wide slice of D]: MFMA A operand of S^T
+  u32x4_t v[D / 128][8];  // [128-wide half of D][token j of the lane group]: raw V segments
+};
+
+// One wave's columns (NCT tiles of 16) against one range of keys: the Q operand, what each column
+// may see, and the running softmax state with the unnormalised output O^T.
+template <int D, int NCT>
+struct Columns {
+  u32x4_t q[NCT][D / 32];
+  int lo[NCT], hi[NCT];        // first and last visible key of this lane's column in each tile
+  int all_lo, all_hi;          // a tile of keys is mask-free iff inside [all_lo, all_hi]
+  float m[NCT], l[NCT];        // running maximum (base 2); this lane's part of the sum
+  f32x4_t o[NCT][D / 128][8];  // o[ct][hf][n][i]: dim hf * 128 + 8 * (4 * (lane / 16) + i) + n
+};
+
+// Columns ct0 * 16 .. of kv head `kvh` of request `r`, for the keys before `t_end`.
+template <int D, int NCT>
+__device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqInfo& r, int kvh, int ct0,
+                                              int t_end, Columns<D, NCT>& c_) {
+  constexpr int KS = D / 32, VH = D / 128;
+  const int t16 = lane_id() & 15, g = lane_id() >> 4;
+  const int ncols = r.q_len * p.group;
+  int all_lo = 0, all_hi = 0x7fffffff;
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    const int col = (ct0 + ct) * 16 + t16;
+    const bool valid = col < ncols;
+    const int qi = valid ? col / p.group : 0;
+    const int hh = valid ? col - qi * p.group : 0;
+    const uint16_t* qrow =
+        p.q + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + hh) * D + g * 8;
+#pragma unroll
+    for (int c = 0; c < KS; ++c) {
+      u32x4_t raw = {0u, 0u, 0u, 0u};
+      if (valid) raw = ld_global_b128(qrow + c * 32);
+      c_.q[ct][c] = raw;
+    }
+    const int qpos = r.prefix + qi;
+    int lo = (p.window > 0) ? qpos - p.window + 1 : 0;
+    int hi = p.is_cross ? r.kv_len - 1 : min(qpos, r.kv_len - 1);
+    hi = min(hi, t_end - 1);
+    if (valid) {
+      all_lo = max(all_lo, lo);
+      all_hi = min(all_hi, hi);
+    } else {
+      lo = 1;
+      hi = 0;
+    }
+    c_.lo[ct] = lo;
+    c_.hi[ct] = hi;
+  }
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) {
+    all_lo = max(all_lo, __shfl_xor(all_lo, off, kWave));
+    all_hi = min(all_hi, __shfl_xor(all_hi, off, kWave));
+  }
+  c_.all_lo = __builtin_amdgcn_readfirstlane(all_lo);
+  c_.all_hi = __builtin_amdgcn_readfirstlane(all_hi);
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    c_.m[ct] = kNegInf;
+    c_.l[ct] = 0.f;
+#pragma unroll
+    for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+      for (int n = 0; n < 8; ++n) c_.o[ct][hf][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+// Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`.
+template <int D, int NCT, bool WIDE, bool F16>
+__device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInfo& r, int kvh, int t_begin,
+                                            int t_end, Columns<D, NCT>& c_) {
+  constexpr int KS = D / 32;   // k-steps of the QK product
+  constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
+  const int lane = lane_id();
+  const int t16 = lane & 15;
+  const int g = lane >> 4;
+  const unsigned char* kbase =
+      reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * D + g * 8);
+  const unsigned char* vbase =
+      reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * D + t16 * 8);
+  const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
+  const uint32_t v_row_bytes = (uint32_t)p.v_stride0 * 2u;
+  auto row_offset = [](int slot_id, uint32_t row_bytes) -> uint64_t {
+    if constexpr (WIDE) return (uint64_t)(uint32_t)slot_id * row_bytes;
+    else return (uint64_t)((uint32_t)slot_id * row_bytes);
+  };
+  const int32_t* idx_base = p.kv_indices + r.kv_start;
+  const int last_tok = t_end - 1;
+
+  // slot ids of the two K rows this lane loads in a 32-token tile starting at tb
+  auto load_idx = [&](int tb, int& s0, int& s1) {
+    s0 = (int)min((uint32_t)idx_base[min(tb + t16, last_tok)], p.max_slot);
+    s1 = (int)min((uint32_t)idx_base[min(tb + 16 + t16, last_tok)], p.max_slot);
+  };
+  auto load_tile = [&](KvTile<D>& t, int s0, int s1) {
+#pragma unroll
+    for (int c = 0; c < KS; ++c) {
+      t.k[0][c] = ld_global_b128(kbase + row_offset(s0, k_row_bytes) + c * 64);
+      t.k[1][c] = ld_global_b128(kbase + row_offset(s1, k_row_bytes) + c * 64);
+    }
+    // V rows of this lane group: tokens 4g+j (j<4) of sub-tile 0, then of sub-tile 1;
+    // their slot ids sit in lanes 4g+j of the K index registers.
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int src = 4 * g + (j & 3);
+      const int slot = __shfl(j < 4 ? s0 : s1, src, kWave);
+      const unsigned char* vrow = vbase + row_offset(slot, v_row_bytes);
+#pragma unroll
+      for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = ld_global_b128(vrow + hf * 256);
+    }
+  };
+
+  auto compute_tile = [&](const KvTile<D>& t, int tb) {
+    // S^T[token][col] for the two 16-token sub-tiles
+    f32x4_t s[2][NCT];
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) {
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KS; ++c)
+          acc = mfma_16x16x32_raw<F16>(t.k[sub][c], c_.q[ct][c], acc);
+        s[sub][ct] = acc;
+      }
+    const bool need_mask = (tb < c_.all_lo) || (tb + 31 > c_.all_hi);
+    uint32_t pb[NCT][4];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      float x[2][4];
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[sub][i] = s[sub][ct][i] * p.scale_log2e;
+      if (need_mask) {
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int tok = tb + sub * 16 + 4 * g + i;
+            if (tok < c_.lo[ct] || tok > c_.hi[ct]) x[sub][i] = kNegInf;
+          }
+      }
+      float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
+                       fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
+      mx = wave_max_xor(mx, 16);
+      mx = wave_max_xor(mx, 32);
+      const float m_new = fmaxf(c_.m[ct], mx);
+      const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
+      const float alpha = fast_exp2(c_.m[ct] - m_safe);
+      c_.m[ct] = m_new;
+      float psum = 0.f;
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[sub][i] = fast_exp2(x[sub][i] - m_safe);
+          psum += x[sub][i];
+        }
+      c_.l[ct] = c_.l[ct] * alpha + psum;
+      pb[ct][0] = pack_16x2<F16>(x[0][0], x[0][1]);
+      pb[ct][1] = pack_16x2<F16>(x[0][2], x[0][3]);
+      pb[ct][2] = pack_16x2<F16>(x[1][0], x[1][1]);
+      pb[ct][3] = pack_16x2<F16>(x[1][2], x[1][3]);
+      if (__any(alpha != 1.0f)) {
+#pragma unroll
+        for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+          for (int n = 0; n < 8; ++n) c_.o[ct][hf][n] *= alpha;
+      }
+    }
+    // O^T += V^T P^T.  MFMA n of half hf produces d = hf*128 + 8*row + n on row = l%16.
+#pragma unroll
+    for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        u32x4_t vt;
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+          const uint32_t a = t.v[hf][2 * qd][n >> 1];
+          const uint32_t c = t.v[hf][2 * qd + 1][n >> 1];
+          vt[qd] = (n & 1) ? pack_hi16(a, c) : pack_lo16(a, c);
+        }
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+          const u32x4_t pv = {pb[ct][0], pb[ct][1], pb[ct][2], pb[ct][3]};
+          c_.o[ct][hf][n] = mfma_16x16x32_raw<F16>(vt, pv, c_.o[ct][hf][n]);
+        }
+      }
+  };
+
+  // ---- tile loop: two register tiles, slot ids fetched two tiles ahead.  Every load in
+  // the loop body is unconditional (tokens past the range clamp to its last token and
+  // are masked), so the number of loads in flight at each wait is a compile-time
+  // constant and the next tile stays in flight while the current one is computed. ----
+  const int n_pairs = (t_end - t_begin + 63) / 64;
+  KvTile<D> ta, tb_;
+  int i0a, i0b, i1a, i1b;
+  load_idx(t_begin, i0a, i0b);
+  load_idx(t_begin + 32, i1a, i1b);
+  load_tile(ta, i0a, i0b);
+  load_idx(t_begin + 64, i0a, i0b);
+  for (int pr = 0; pr < n_pairs; ++pr) {
+    const int tok = t_begin + pr * 64;
+    load_tile(tb_, i1a, i1b);
+    load_idx(tok + 96, i1a, i1b);
+    compute_tile(ta, tok);
+    load_tile(ta, i0a, i0b);
+    load_idx(tok + 128, i0a, i0b);
+    compute_tile(tb_, tok + 32);
+  }
+}
+
+}  // namespace msgl

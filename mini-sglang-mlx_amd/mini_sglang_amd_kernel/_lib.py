@@ -94,6 +94,7 @@ TUNE_PREFILL_KEY_SPLITS = 6
 TUNE_SPLITKV_BOUNDARY = 7
 TUNE_PREFILL_GANGS = 8
 TUNE_CLOCK_PROBE = 9
+TUNE_SHARES = 10
 
 _lib = None
 
