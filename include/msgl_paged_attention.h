@@ -304,8 +304,8 @@ MSGL_API int msgl_gdn_state_inplace(const void* q, const void* k, const void* v,
  *   MSGL_TUNE_SPLITKV_BOUNDARY tokens' worth of time a split-K workgroup is charged for starting
  *                            on another request inside its segment (0: default from the shape,
  *                            negative: none)
- *   MSGL_TUNE_GDN_ROWS       state rows per 16-lane group of the gdn_state kernel: 1, 2, 4
- *                            (0: chosen from the problem size)
+ *   MSGL_TUNE_GDN_ROWS       the gdn_state kernel that goes token by token, with 1, 2 or 4 state rows
+ *                            per 16-lane group (0: kernel and rows chosen from the problem size)
  *   MSGL_TUNE_PREFILL_KEY_SPLITS  workgroups that share the keys of one query block of the MFMA
  *                            tile kernels (1: never split, up to 32; 0: chosen from the sizes,
  *                            and launches with one query block per request and kv head give each

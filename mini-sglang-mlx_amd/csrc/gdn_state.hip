@@ -14,34 +14,18 @@
 // one load of k and q serves R independent recurrences whose latencies overlap; the inputs of
 // the next kDepth tokens are always in flight.  Decode (one token) is
 // HBM-bound: 2 * dv * dk * 4 bytes of state per (request, hv head) read and written once.
-// Prefill is a serial chain per row (as in the reference); parallelism is batch * hv * dv rows.
+// Prefill is a serial chain per row (as in the reference); parallelism is batch * hv * dv rows.  It takes
+// requests of a few tokens here; longer ones go in chunks (gdn_chunk.hip, prefer_chunks() below).
+#include <algorithm>
 #include <atomic>
 
-#include "msgl_device.h"
-#include "msgl_internal.h"
+#include "gdn_params.h"
 
 namespace msgl {
 namespace {
 
-constexpr int kDK = 128, kDV = 128;
 constexpr int kLanesPerRow = 16;
 constexpr int kPerLane = kDK / kLanesPerRow;  // 8 state values per lane and row
-
-struct GdnParams {
-  float* state;
-  uint16_t* y;
-  const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
-  const uint16_t* g;
-  const uint16_t* beta;
-  const int32_t* slot_ids;
-  const int32_t* qo_indptr;
-  int64_t state_stride0, q_stride0, k_stride0, v_stride0;
-  int32_t batch, hv, hv_per_hk, tokens, single_token;
-};
-
-__device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __builtin_bit_cast(float, b << 16); }
 
 template <int N>
 __device__ __forceinline__ float row_rotate(float x) {  // lane i of a 16-lane row reads lane (i + N) % 16
@@ -174,6 +158,18 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 
 }  // namespace
 
+// Whether the chunk kernel (gdn_chunk.hip) is the faster one.  Its time for up to 64 tokens per request
+// does not depend on their number: 12.8 us for each round of workgroups (two per value head, one per
+// compute unit).  The token kernel's grows with the mean length, by 0.315 us per token while the requests
+// run side by side and by 0.095 us per token and request of 32 heads beyond.  Both fitted to 1, 4, 16 and 64
+// requests of 8, 16, 32 and 64 tokens; they meet between 15 and 30 tokens.
+static bool prefer_chunks(const GdnArgs& a) {
+  if (a.v_stride0 >= (1 << 24) || a.k_stride0 >= (1 << 24) || a.q_stride0 >= (1 << 24) || a.hv >= (1 << 17))
+    return false;  // its offsets inside a chunk are 32 bits wide
+  const double units = (double)(a.batch * a.hv) / 32, mean = (double)a.tokens / (double)a.batch;
+  const double rounds = (double)((a.batch * a.hv * 2 + device_cus() - 1) / device_cus());
+  return 12.8 * rounds < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
+}
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 void gdn_set_rows(int v) { t_force_rows = (v == 1 || v == 2 || v == 4) ? v : 0; }
 
@@ -199,6 +195,7 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   p.single_token = a.single_token_mode ? 1 : 0;
   const int64_t heads = a.batch * a.hv;
   if (heads <= 0) return MSGL_OK;
+  if (!p.single_token && t_force_rows == 0 && prefer_chunks(a)) return launch_gdn_chunks(p, stream);
   // more rows per lane group (more overlap inside a wave) once there are enough workgroups
   // to fill the chip without it
   const int64_t blocks_r1 = heads * (kDV / 16);
