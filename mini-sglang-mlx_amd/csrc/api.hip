@@ -434,6 +434,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   a.is_cross = is_cross_attention ? 1 : 0;
   a.window = sliding_window_size;
   a.key_splits = 1;
+  a.by_length = 1;
   a.ragged_tiles = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
   if (a.ragged_tiles > 0) {
     // ragged shares need room for their partials; without it the keys go in one pass

@@ -102,6 +102,7 @@ struct PrefillArgs {
   // number no earlier launch on this workspace has used
   int32_t gangs;
   unsigned long long gang_nonce;
+  int32_t by_length;  // query blocks may go in order of length (the fused kernel does not know that order)
 };
 int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream);     // head_dim 128
 // ---- paged_prefill_d256.hip ----------------------------------------------------------

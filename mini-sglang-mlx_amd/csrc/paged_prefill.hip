@@ -671,7 +671,12 @@ static_assert(kHandoff >= 0 && kHandoff <= 2, "the sends of a phase must have le
 constexpr int kOperandBuffers = kAhead + 1;
 }  // namespace pp
 
-template <bool WIDE>
+// How a workgroup comes by its work: kBatch, (request, kv head, key split, query block) or ragged share;
+// kGang, the parts of a gang's range; kLength, query blocks in order of length.  A kernel each: with all of
+// them in one, their registers spill inside the loop.
+enum class Order { kBatch, kGang, kLength };
+
+template <bool WIDE, Order ORDER>
 __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) {
   constexpr int D = 128, NW = 8, UPW = kUnits / NW, KSTEPS = D / 16, DT = D / 32;
   constexpr int kRows = NW * 32;
@@ -691,7 +696,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   // fall into its gang's range, one after the other (see gang_plan) -----------------------------
   __shared__ GangLds gang_lds;
   __shared__ int gang_last;
-  const bool ganged = p.gangs > 0;
+  constexpr bool ganged = ORDER == Order::kGang;
   const int gang_xcd = (int)(blockIdx.x & 7);
   const int gang_id = ganged ? (int)(blockIdx.x >> 3) / p.n_qblk : 0;
   const int gang_member = ganged ? (int)(blockIdx.x >> 3) % p.n_qblk : 0;
@@ -706,6 +711,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   int64_t part_at = 0;               // partial row of the block's row 0 (ragged shares)
   int piece_a = 0, piece_b = 0x7fffff, unit_start = 0, unit_tiles = 0;  // gang ranges: tiles [a, b) of the unit
   bool piece_whole = true;
+  LengthBlock by_length{};
   if (ganged) {
     if (piece > plan.last_unit) break;
     // the stages double as the staging area of the previous part's output: read out by now
@@ -723,6 +729,12 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     to_partial = false;
   } else if (piece > 0) {
     break;
+  } else if (ORDER == Order::kLength) {
+    by_length = block_by_length<kRows>(p);
+    if (!by_length.ok) return;
+    b = by_length.b;
+    kvh = by_length.kvh;
+    qblk = by_length.qblk;
   } else if (p.ragged_tiles > 0) {
     kvh = (int)(blockIdx.x % (unsigned)p.n_kv);
     const int u = (int)(blockIdx.x / (unsigned)p.n_kv);
@@ -749,13 +761,30 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     b = request_of_rank<NW * 64>(p.kv_indptr, p.batch, want_rank, tid);
   }
 
-  // (gang ranges keep every request's geometry in LDS: a part starts without a memory round trip)
+  // the request's geometry: gang ranges keep it in LDS, blocks in order of length come with it (a part or
+  // block starts without another memory round trip)
   auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
-  const int q_start = ganged ? uniform(gang_lds.q_start[b]) : p.qo_indptr[b];
-  const int q_len = ganged ? uniform(gang_lds.q_len[b]) : min(p.qo_indptr[b + 1] - q_start, p.max_len_extend);
-  const int kv_start = ganged ? uniform(gang_lds.kv_start[b]) : p.kv_indptr[b];
-  const int kn = ganged ? uniform(gang_lds.kv_len[b]) : max(p.kv_indptr[b + 1] - kv_start, 0);
-  const int prefix = ganged ? uniform(gang_lds.prefix[b]) : p.prefix_lens[b];
+  int q_start, q_len, kv_start, kn, prefix;
+  if (ganged) {
+    q_start = uniform(gang_lds.q_start[b]);
+    q_len = uniform(gang_lds.q_len[b]);
+    kv_start = uniform(gang_lds.kv_start[b]);
+    kn = uniform(gang_lds.kv_len[b]);
+    prefix = uniform(gang_lds.prefix[b]);
+  } else if (ORDER == Order::kLength) {
+    q_start = by_length.q_start;
+    q_len = by_length.q_len;
+    kv_start = by_length.kv_start;
+    kn = by_length.kv_len;
+    prefix = by_length.prefix;
+  } else {
+    b = uniform(b);
+    q_start = p.qo_indptr[b];
+    q_len = min(p.qo_indptr[b + 1] - q_start, p.max_len_extend);
+    kv_start = p.kv_indptr[b];
+    kn = max(p.kv_indptr[b + 1] - kv_start, 0);
+    prefix = p.prefix_lens[b];
+  }
   const int rows_total = q_len * p.group;
   const int row0 = qblk * kRows;
   if (row0 >= rows_total) {
@@ -1432,6 +1461,7 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
   if (tile_variant() != 0) {  // the fused kernel knows uniform key splits only
     args.ragged_tiles = 0;
     args.gangs = 0;
+    args.by_length = 0;
   }
   const int rc = make_prefill_params(args, p, n_blocks, wide);
   if (rc != MSGL_OK || n_blocks == 0) return rc;
@@ -1440,8 +1470,10 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
     if (wide) hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, true>), grid, dim3(512), 0, stream, p);
     else hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, false>), grid, dim3(512), 0, stream, p);
   } else {
-    if (wide) hipLaunchKernelGGL((prefill_pingpong_kernel<true>), grid, dim3(512), 0, stream, p);
-    else hipLaunchKernelGGL((prefill_pingpong_kernel<false>), grid, dim3(512), 0, stream, p);
+    auto* const kernel = p.gangs > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kGang> : prefill_pingpong_kernel<false, Order::kGang>)
+                         : p.length_heads > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kLength> : prefill_pingpong_kernel<false, Order::kLength>)
+                                              : (wide ? prefill_pingpong_kernel<true, Order::kBatch> : prefill_pingpong_kernel<false, Order::kBatch>);
+    hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, p);
   }
   const int launched = check_launch();
   if (launched != MSGL_OK || (p.n_ksplit == 1 && p.ragged_tiles == 0)) return launched;

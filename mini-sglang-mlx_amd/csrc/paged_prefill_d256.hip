@@ -73,9 +73,10 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // run heaviest first, requests in order of decreasing kv length (each block ranks the requests
   // itself from kv_indptr)
   // With ragged shares: block -> (unit = (request, share), kv head), see prefill_ragged_tiles().
-  int b, kvh, split, qblk, n_shares = 1;
+  int b, kvh, split = 0, qblk, n_shares = 1;
   bool to_partial = p.n_ksplit > 1;  // leave a partial for the merge kernel, not the result
   int64_t part_at = 0;               // partial row of the block's row 0 (ragged shares)
+  LengthBlock by_length{};
   if (p.ragged_tiles > 0) {
     kvh = (int)(blockIdx.x % (unsigned)p.n_kv);
     const int u = (int)(blockIdx.x / (unsigned)p.n_kv);
@@ -91,6 +92,12 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       p.req_units[2 * b] = ru.first;  // tells the merge kernel where the request's partials are
       p.req_units[2 * b + 1] = ru.count;
     }
+  } else if (p.length_heads > 0) {
+    by_length = block_by_length<kRows>(p);
+    if (!by_length.ok) return;
+    b = by_length.b;
+    kvh = by_length.kvh;
+    qblk = by_length.qblk;
   } else {
     const BlockWork work = prefill_block_work(p);
     if (!work.ok) return;
@@ -102,11 +109,20 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     b = __builtin_amdgcn_readfirstlane(request_of_rank<kNW * 64>(p.kv_indptr, p.batch, want_rank, tid));
   }
 
-  const int q_start = __builtin_amdgcn_readfirstlane(p.qo_indptr[b]);
-  const int q_len = min(__builtin_amdgcn_readfirstlane(p.qo_indptr[b + 1]) - q_start, p.max_len_extend);
-  const int kv_start = __builtin_amdgcn_readfirstlane(p.kv_indptr[b]);
-  const int kn = max(__builtin_amdgcn_readfirstlane(p.kv_indptr[b + 1]) - kv_start, 0);
-  const int prefix = __builtin_amdgcn_readfirstlane(p.prefix_lens[b]);
+  int q_start, q_len, kv_start, kn, prefix;
+  if (by_length.ok) {  // they came with the block
+    q_start = by_length.q_start;
+    q_len = by_length.q_len;
+    kv_start = by_length.kv_start;
+    kn = by_length.kv_len;
+    prefix = by_length.prefix;
+  } else {
+    q_start = __builtin_amdgcn_readfirstlane(p.qo_indptr[b]);
+    q_len = min(__builtin_amdgcn_readfirstlane(p.qo_indptr[b + 1]) - q_start, p.max_len_extend);
+    kv_start = __builtin_amdgcn_readfirstlane(p.kv_indptr[b]);
+    kn = max(__builtin_amdgcn_readfirstlane(p.kv_indptr[b + 1]) - kv_start, 0);
+    prefix = __builtin_amdgcn_readfirstlane(p.prefix_lens[b]);
+  }
   const int rows_total = q_len * p.group;
   const int row0 = qblk * kRows;
   if (row0 >= rows_total) return;

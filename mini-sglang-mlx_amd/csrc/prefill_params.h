@@ -38,6 +38,9 @@ struct PrefillParams {
   float* gang_slots;
   unsigned long long* gang_counts;
   unsigned long long gang_nonce;
+  // query blocks in order of length (see prefill_by_length()): kv heads per XCD, 0 = off, and the
+  // logarithm of the number of XCDs that share a kv head's blocks
+  int32_t length_heads, length_log2_xcds;
   long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
 };
 
@@ -156,6 +159,27 @@ inline size_t prefill_ragged_workspace_bytes(int64_t batch, int64_t total_kv, in
   return rows * (size_t)(head_dim + 1) * sizeof(float) + (size_t)batch * 2 * sizeof(int32_t);
 }
 
+// Query blocks in order of length, for launches in one pass over the keys (no splits, shares or gang
+// ranges).  Every XCD takes one kv head in eight of every request (fewer kv heads than XCDs: an equal part
+// of one kv head's blocks, taken in turn), so the XCDs have the same work whatever the requests' lengths,
+// and issues its blocks longest first, whatever request they belong to: the dispatcher then fills the
+// compute units with ever shorter blocks and the last ones end together.  (With whole requests dealt to
+// the XCDs one request after the other, an XCD with the two longest of four requests ran 1.5 times as long
+// as the average: 4 requests of 512-1972 tokens on prefixes up to 8 K, 24 / 4 heads of 256: 1173 -> 837 us;
+// 6 prompts of 771-2710 tokens, 32 / 8 heads of 128: 262 -> 247 us.)  The blocks of a
+// request no longer run side by side on one XCD; what its L2 then misses, the memory-side cache has.
+//
+// The kernel's wave holds one request per lane: at most 64.  The kv heads have to go into the XCDs evenly.
+// A launch of fewer blocks than compute units has no order.  Whole prompts of one length in many blocks
+// each are even as they are, and gain more from a request's blocks side by side (5 x 1722 tokens, 32 / 8
+// heads: 166 us against 172; below 16 blocks a request the order is the better one or equal: 11 x 463
+// tokens, 16 / 8 heads, 4 blocks: 48.7 against 42.5).
+inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
+  const bool even_prompts = !a.is_cross && a.total_kv == a.total_q && a.total_q == a.batch * a.max_len_extend;
+  return a.by_length && a.batch <= 64 && (a.n_kv == 1 || a.n_kv == 2 || a.n_kv == 4 || a.n_kv % 8 == 0) &&
+         a.batch * a.n_kv * n_qblk > kComputeUnits && !(even_prompts && n_qblk >= 16);
+}
+
 // Gang ranges, for launches with several query blocks per (request, kv head) (chunked extends on
 // long prefixes: their cost is the MFMA work, and it differs from unit to unit with the prefix).
 // One workgroup per compute unit stays for the whole launch.  The 32 workgroups on an XCD form
@@ -243,6 +267,8 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
   p.gang_slots = nullptr;
   p.gang_counts = nullptr;
   p.gang_nonce = 0;
+  p.length_heads = 0;
+  p.length_log2_xcds = 0;
   p.clock_probe = clock_probe();
   if (a.ragged_tiles > 0 && n_qblk == 1) {
     const int64_t units = prefill_ragged_units(a.batch, a.total_kv, a.ragged_tiles);
@@ -288,6 +314,13 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     p.gang_counts = reinterpret_cast<unsigned long long*>(static_cast<char*>(a.workspace) + slots * kGangSlotBytes);
     p.gang_nonce = a.gang_nonce;
     n_blocks = kComputeUnits;  // one workgroup per compute unit, 32 per XCD
+  }
+  if (p.gangs == 0 && p.n_ksplit == 1 && prefill_by_length(a, n_qblk)) {
+    p.length_heads = a.n_kv >= 8 ? (int32_t)(a.n_kv / 8) : 1;
+    p.length_log2_xcds = a.n_kv == 1 ? 3 : a.n_kv == 2 ? 2 : a.n_kv == 4 ? 1 : 0;
+    const int64_t xcds = 1 << p.length_log2_xcds;
+    n_blocks = 8 * a.batch * p.length_heads * ((n_qblk + xcds - 1) / xcds);
+    if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   }
   // narrow offsets: slot * row_bytes fits 32 bits and both factors fit 24 bits (one
   // full-rate 24-bit multiply per row)

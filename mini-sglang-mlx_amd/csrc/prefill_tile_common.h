@@ -1,5 +1,7 @@
 // LDS-direct loads, counted waits and transposing LDS reads shared by the prefill tile kernels.
 #pragma once
+#include <type_traits>
+
 #include "msgl_device.h"
 #include "prefill_params.h"
 
@@ -82,6 +84,111 @@ __device__ __forceinline__ BlockWork prefill_block_work(const PrefillParams& p) 
     w.qblk = p.n_qblk - 1 - j;
     w.ok = w.unit < n_units && j < p.n_qblk;
   }
+  return w;
+}
+
+// Wave-wide sum (the same in every lane) and inclusive prefix sum without LDS: a prefix sum inside each row
+// of 16 lanes, the rows' totals through scalar registers.
+__device__ __forceinline__ int row_scan(int v) {
+  auto shifted = [](int x, auto n) { return __builtin_amdgcn_update_dpp(0, x, 0x110 + decltype(n)::value, 0xf, 0xf, true); };
+  v += shifted(v, std::integral_constant<int, 1>{});  // row_shr
+  v += shifted(v, std::integral_constant<int, 2>{});
+  v += shifted(v, std::integral_constant<int, 4>{});
+  v += shifted(v, std::integral_constant<int, 8>{});
+  return v;
+}
+__device__ __forceinline__ int wave_sum(int v) {
+  v = row_scan(v);
+  return __builtin_amdgcn_readlane(v, 15) + __builtin_amdgcn_readlane(v, 31) + __builtin_amdgcn_readlane(v, 47) +
+         __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_scan(int v) {
+  v = row_scan(v);
+  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31), r2 = __builtin_amdgcn_readlane(v, 47);
+  const int row = lane_id() >> 4;
+  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
+
+// Workgroup id -> query block and its request's geometry, in order of length (see prefill_by_length()).
+// Lengths count in steps of an eighth to a quarter of the longest: within a step a request's blocks stay
+// together, because those that run at the same time then read the same keys (strictly by length, 11 prompts
+// of 3637 tokens took 1415 us instead of 1345).  The length of block i of a request does not fall with i, so
+// the number of its blocks of at least T steps is a division; a wave holds a request per lane, finds the T at
+// which its XCD's blocks of at least T steps pass its own number by bisection, and its place among those of
+// T steps by a prefix sum.  Every wave does this for itself: one memory round trip,
+// no LDS, no barrier.
+// (The length is the causal one; under a window it is cut off, so that the order stays the same for all
+// masks.  It decides the order only: any order is correct.)
+struct LengthBlock {
+  int b, kvh, qblk;
+  int q_start, q_len, kv_start, kv_len, prefix;
+  bool ok;
+};
+template <int ROWS>
+__device__ __forceinline__ LengthBlock block_by_length(const PrefillParams& p) {
+  const int lane = lane_id();
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int heads_across = min(p.n_kv, 8);
+  const int part = xcd / heads_across, mask = (1 << p.length_log2_xcds) - 1;
+  // the lane's request
+  int q_start = 0, q_len = 0, kv_start = 0, kv_len = 0, prefix = 0;
+  if (lane < p.batch) {
+    q_start = p.qo_indptr[lane];
+    q_len = p.qo_indptr[lane + 1];
+    kv_start = p.kv_indptr[lane];
+    kv_len = p.kv_indptr[lane + 1];
+    prefix = p.prefix_lens[lane];
+  }
+  q_len = min(q_len - q_start, p.max_len_extend);
+  kv_len = max(kv_len - kv_start, 0);
+  const int rows = q_len * p.group;
+  const int kn = min(kv_len, p.window > 0 ? p.window + ROWS / p.group + 1 : 0x7fffffff);
+  const int first_of = (part + lane) & mask;  // this XCD's blocks: first_of, first_of + XCDs per head, ...
+  const int blocks = rows > 0 ? (rows + ROWS - 1) / ROWS : 0;
+  auto in_class = [&](int below) {  // this XCD's blocks among the first `below`
+    return below > first_of ? ((below - first_of - 1) >> p.length_log2_xcds) + 1 : 0;
+  };
+  const int in_all = in_class(blocks);
+  int longest = kn;
+  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x128, 0xf, 0xf, true));  // row_ror: 8, 4, 2, 1
+  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x124, 0xf, 0xf, true));
+  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x122, 0xf, 0xf, true));
+  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x121, 0xf, 0xf, true));
+  longest = max(max(__builtin_amdgcn_readlane(longest, 0), __builtin_amdgcn_readlane(longest, 16)),
+                max(__builtin_amdgcn_readlane(longest, 32), __builtin_amdgcn_readlane(longest, 48)));
+  const int shift = max(31 - __builtin_clz(max(longest, 1)) - 2, 6);  // 4 to 8 steps, whole key tiles
+  // this XCD's blocks of the request of at least `steps` steps
+  auto at_least = [&](int steps) {
+    if (steps <= 0) return in_all;
+    const int keys = ((steps - 1) << shift) + 1;
+    const int row = p.is_cross ? 0 : max(keys - 1 - prefix, 0) * p.group;  // first row that sees so many
+    return in_all - in_class(kn >= keys && row < rows ? row / ROWS : blocks);
+  };
+  auto count = [&](int steps) { return wave_sum(at_least(steps)) * p.length_heads; };
+  LengthBlock w{};
+  // count(lo) > seq >= count(hi)
+  int lo = 0, hi = (longest >> shift) + 2;
+  if (seq >= count(0)) return w;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (count(mid) > seq) lo = mid;
+    else hi = mid;
+  }
+  const int longer = at_least(lo + 1), equal = (at_least(lo) - longer) * p.length_heads;
+  const int left = seq - wave_sum(longer) * p.length_heads;  // its number among the blocks of exactly `lo` steps
+  const int incl = wave_scan(equal), before = incl - equal;
+  const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(left >= before && left < incl)) - 1);
+  const int mine = left - __builtin_amdgcn_readlane(before, src);
+  const int from_top = __builtin_amdgcn_readlane(longer, src) + mine / p.length_heads;
+  w.b = src;
+  w.kvh = xcd % heads_across + 8 * (mine % p.length_heads);
+  w.qblk = __builtin_amdgcn_readlane(first_of, src) + ((__builtin_amdgcn_readlane(in_all, src) - 1 - from_top) << p.length_log2_xcds);
+  w.q_start = __builtin_amdgcn_readlane(q_start, src);
+  w.q_len = __builtin_amdgcn_readlane(q_len, src);
+  w.kv_start = __builtin_amdgcn_readlane(kv_start, src);
+  w.kv_len = __builtin_amdgcn_readlane(kv_len, src);
+  w.prefix = __builtin_amdgcn_readlane(prefix, src);
+  w.ok = true;
   return w;
 }
 
