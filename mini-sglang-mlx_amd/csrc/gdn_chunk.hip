@@ -12,21 +12,25 @@
 // the state, so the serial part of a chunk is five products.
 //
 // Token after token a request costs 0.33 us per token whatever the chip has free; here a chunk of 64 costs
-// 5.2 us.  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32: 1353 -> 330 us; one of 1024: 298 -> 90.
+// 4.4 us.  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32: 1353 -> 282 us; one of 1024: 298 -> 77.
 //
 // Work: one workgroup per (request, value head, half of its 128 rows).  Waves 0-3 ("state" waves, 16
 // rows each, S^T in 32 accumulator registers) run the serial part of chunk j; waves 4-7 ("chunk" waves,
 // 16 tokens each) make T and P of chunk j + 1 beside them, one of each on a SIMD.  Three slots per
 // chunk, a workgroup barrier behind each:
 //     slot   state waves, chunk j                 chunk waves
-//      1     X = K S^T, Z = Q S^T                  P of chunk j and K, Q of chunk j + 1 to LDS
-//      2     R = beta (V - G X), U = T R           A, P and the diagonal blocks of T of chunk j + 1
-//      3     Y = G Z + P U, S = G_64 S + K^T U     the blocks of T below the diagonal; T of chunk j + 1 to LDS;
+//      1     X = K S^T, Z = Q S^T                  T and P of chunk j and K, Q of chunk j + 1 to LDS
+//      2     R = beta (V - G X), U = T R           A, the decay ratios of P, the diagonal blocks of T of chunk j + 1
+//      3     Y = G Z + P U, S = G_64 S + K^T U     P, the blocks of T below the diagonal, V of chunk j + 1;
 //                                                  decay products of chunk j + 2
-// What bounds it: a chunk takes 12.5 K cycles (slots of 3.1, 3.9 and 5.0 K), of which the matrix pipe is busy
-// 4.4 K, LDS 5.2 K and the vector ALU about 5 K: three chains that depend on each other, on one wave each per
-// SIMD.  Operands are asked for a step, and across the barriers a slot, before they are used, and the splits
-// stand between the matrix instructions.
+// What bounds it: a chunk takes 10.7 K cycles (slots of 3.2, 2.9 and 4.6 K), in which a SIMD has 5 K cycles of
+// matrix instructions and as many of vector instructions in two chains that wait for their own results, and a
+// wave that has the SIMD for itself still pays about 5 cycles per instruction of any kind.  Hence: fp32 values
+// are split by the matrix pipe (see Split: 16 instructions instead of 44), Z and Y are made transposed (4 stores
+// of 8 bytes a chunk instead of 16 of 2), V comes by transposing LDS reads, and the chunk waves share the blocks
+// out evenly (12.5 -> 10.7 K).  T and P of all chunks in a launch of their own, in parallel, measured the same
+// for the longest request of a launch and less for many short ones: their 20 KB per chunk and head cost 40 us
+// of writing for the requests above, and LDS and issue time in the serial part.
 //
 // Precision: fp32 throughout, as in the token kernel.  q, k, v are bf16 and enter the bf16 matrix
 // instructions as they are; fp32 operands (S, R, U, T, P) are split into three bf16 parts of 8
@@ -49,16 +53,17 @@ namespace {
 
 constexpr int kChunk = 64;        // tokens per chunk
 constexpr int kRowsPerWg = 64;    // dv rows of a workgroup
-// Rows of 304 bytes: 16 rows at one column lie in 16 different groups of four banks, and so do, all but
-// three, the 4 rows x 4 columns of a transposing read (rows of 272 bytes: 4 of those in one group).
-constexpr int kRowPad = 152;
 constexpr int kRanked = 512;      // requests ranked by length (one per thread)
 
+// T and P as operands: fragment f of row block m and contraction step c (32 columns), those that are not
+// zero; lane x16 + 16 g of a fragment holds row x16, columns 32 c + 4 g .. and 32 c + 16 + 4 g ..
+constexpr int kFragments = 6;
+__device__ constexpr int fragment(int m, int c) { return c == 0 ? m : m + 2; }
+
 struct ChunkLds {
-  uint16_t k[2][kChunk][kRowPad];
-  uint16_t q[2][kChunk][kRowPad];
-  uint16_t t[3][kChunk][72];      // T and P in three bf16 parts, columns in contraction order
-  uint16_t p[3][kChunk][72];
+  uint16_t k[2][kChunk][kDK], q[2][kChunk][kDK];  // 16-byte pieces of a row in swizzled order (see piece())
+  uint16_t v[kChunk][kRowsPerWg];
+  u32x4_t t[3][kFragments][64], p[3][kFragments][64];  // T and P in three bf16 parts
   float a[kChunk][68];            // A of the chunk being prepared (blocks on and below the diagonal)
   float diag[4][16][20];          // inverses of the diagonal blocks of I + A
   // per token, chunks j .. j + 2: beta, G, and tail_i = G_64 / G_i
@@ -70,42 +75,65 @@ struct ChunkLds {
   int request;
 };
 
-// Eight fp32 values as three operands of bf16 parts: x = hi + mid + lo (each cut, so exact).
+// Piece `c` of 16 bytes of row `row` lies at this place.  LDS serves 8 lanes of a 16-byte read and 16 of an
+// 8-byte one at a time: the rows 0-7 and 8-15 of an operand at one column go to 8 different places modulo 8,
+// the 4 rows x 4 columns of a transposing read to 16 different ones.
+__device__ __forceinline__ int swizzle(int row) {
+  const int r0 = row & 1, r1 = (row >> 1) & 1, r2 = (row >> 2) & 1, r3 = (row >> 3) & 1;
+  return (r1 ^ r3) << 3 | r0 << 2 | r1 << 1 | r2;
+}
+__device__ __forceinline__ int piece(int row, int c) { return c ^ swizzle(row); }
+
+// Eight fp32 values as three operands of bf16 parts: x = hi + mid + lo, each the nearest to what is left, so
+// exact.  The matrix pipe takes the parts off: x - hi is x plus the product of a matrix that picks, negated,
+// the result tile's rows out of the 32 contraction rows, and hi as it stands (12 conversions and 4 matrix
+// instructions; by vector instructions 44, and their issue is what a wave waits for).
 struct Split {
   bf16x8_t hi, mid, lo;
 };
-__device__ __forceinline__ float upper(float x) {
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
-}
-__device__ __forceinline__ Split split(f32x4_t a, f32x4_t b) {
-  u32x4_t hi, mid, lo;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float x0 = j < 2 ? a[2 * j] : b[2 * j - 4], x1 = j < 2 ? a[2 * j + 1] : b[2 * j - 3];
-    const float y0 = x0 - upper(x0), y1 = x1 - upper(x1);
-    const float z0 = y0 - upper(y0), z1 = y1 - upper(y1);
-    hi[j] = pack_hi16(__builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, x1));
-    mid[j] = pack_hi16(__builtin_bit_cast(uint32_t, y0), __builtin_bit_cast(uint32_t, y1));
-    lo[j] = pack_hi16(__builtin_bit_cast(uint32_t, z0), __builtin_bit_cast(uint32_t, z1));
+struct Picker {
+  bf16x8_t first, second;
+  __device__ __forceinline__ Picker() {  // row 4 a + i of the first tile: contraction row 8 a + i; second: 8 a + 4 + i
+    const int x16 = lane_id() & 15, g = lane_id() >> 4;
+    u32x4_t f = {0u, 0u, 0u, 0u};
+    const uint32_t minus_one = g == (x16 >> 2) ? 0xbf80u << (16 * (x16 & 1)) : 0u;
+    const uint32_t even = (x16 & 2) ? 0u : minus_one, odd = (x16 & 2) ? minus_one : 0u;
+    f[0] = even;
+    f[1] = odd;
+    first = as_bf16x8(f);
+    second = as_bf16x8(u32x4_t{0u, 0u, even, odd});
   }
-  return Split{as_bf16x8(hi), as_bf16x8(mid), as_bf16x8(lo)};
+};
+__device__ __forceinline__ bf16x8_t nearest(f32x4_t a, f32x4_t b) {
+  return bf16x8_t{(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3], (__bf16)b[0], (__bf16)b[1], (__bf16)b[2], (__bf16)b[3]};
 }
-// Four neighbouring values of a row of T or P, in three parts.
-__device__ __forceinline__ void split_store(f32x4_t x, uint16_t (*m)[kChunk][72], int row, int col) {
-  f32x4_t y, z;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float f = x[i], rest = f - upper(f);
-    y[i] = rest;
-    z[i] = rest - upper(rest);
-  }
-  auto cut = [](f32x4_t f) {
-    const u32x4_t u = __builtin_bit_cast(u32x4_t, f);
-    return u32x2_t{pack_hi16(u[0], u[1]), pack_hi16(u[2], u[3])};
+__device__ __forceinline__ Split split(const Picker& pick, f32x4_t a, f32x4_t b) {
+  Split s;
+  s.hi = nearest(a, b);
+  a = mfma_16x16x32(pick.first, s.hi, a);
+  b = mfma_16x16x32(pick.second, s.hi, b);
+  s.mid = nearest(a, b);
+  a = mfma_16x16x32(pick.first, s.mid, a);
+  b = mfma_16x16x32(pick.second, s.mid, b);
+  s.lo = nearest(a, b);
+  return s;
+}
+
+// Four neighbouring values of a row of T or P, a lane's part of block (r, c), to LDS.
+__device__ __forceinline__ void split_store(const Picker& pick, f32x4_t x, u32x4_t (*m)[kFragments][64], int r, int c) {
+  auto half = [&](f32x4_t f) { return u32x2_t{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])}; };
+  auto rest = [&](f32x4_t f, u32x2_t part) {
+    return mfma_16x16x32(pick.first, as_bf16x8(u32x4_t{part[0], part[1], 0u, 0u}), f);
   };
-  *reinterpret_cast<u32x2_t*>(&m[0][row][col]) = cut(x);
-  *reinterpret_cast<u32x2_t*>(&m[1][row][col]) = cut(y);
-  *reinterpret_cast<u32x2_t*>(&m[2][row][col]) = cut(z);
+  const u32x2_t hi = half(x);
+  const f32x4_t y = rest(x, hi);
+  const u32x2_t mid = half(y);
+  const u32x2_t lo = half(rest(y, mid));
+  u32x2_t* to = reinterpret_cast<u32x2_t*>(&m[0][fragment(r, c >> 1)][lane_id()]) + (c & 1);
+  constexpr int kPart = kFragments * 64 * 2;
+  to[0] = hi;
+  to[kPart] = mid;
+  to[2 * kPart] = lo;
 }
 
 // LDS traffic of every wave done, then the workgroup barrier; loads from memory stay in flight.
@@ -119,29 +147,31 @@ __device__ __forceinline__ bf16x8_t operand(const uint16_t* p) {
   return as_bf16x8(*reinterpret_cast<const u32x4_t*>(p));
 }
 
-// Column of tokens 16 c + 4 q .. + 3 of a chunk in the rows of T and P (see Layouts).
-__device__ __forceinline__ int token_column(int c, int q) { return 32 * (c >> 1) + 8 * q + 4 * (c & 1); }
-
-// Operands of the row blocks of T or P that reach contraction step c (m = 2 c .. 3), in three parts.
 struct Triangle {
-  bf16x8_t hi[4], mid[4], lo[4];
+  bf16x8_t hi[kFragments], mid[kFragments], lo[kFragments];
 };
-__device__ __forceinline__ void load_triangle(const uint16_t (*m0)[kChunk][72], int c, Triangle& t) {
-  const int x16 = lane_id() & 15, g = lane_id() >> 4;
+template <int FROM, int TO>
+__device__ __forceinline__ void load_triangle(const u32x4_t (*m)[kFragments][64], Triangle& t) {
+  const int lane = lane_id();
 #pragma unroll
-  for (int m = 2 * c; m < 4; ++m) {
-    t.hi[m] = operand(&m0[0][16 * m + x16][32 * c + 8 * g]);
-    t.mid[m] = operand(&m0[1][16 * m + x16][32 * c + 8 * g]);
-    t.lo[m] = operand(&m0[2][16 * m + x16][32 * c + 8 * g]);
+  for (int f = FROM; f < TO; ++f) {
+    t.lo[f] = as_bf16x8(m[2][f][lane]);
+    t.mid[f] = as_bf16x8(m[1][f][lane]);
+    t.hi[f] = as_bf16x8(m[0][f][lane]);
   }
 }
-// acc += M B for contraction step C of M (row blocks m = 2 C .. 3), B split: the six products above 2^-24,
-// smallest first, the row blocks side by side.
-template <int C>
-__device__ __forceinline__ void triangle_product(const Triangle& t, const Split& b, f32x4_t (&acc)[4]) {
-  auto step = [&](const bf16x8_t (&part)[4], const bf16x8_t& b0) {
+// a b, or its transpose: operands of both kinds have the same layout
+template <bool TRANSPOSED>
+__device__ __forceinline__ f32x4_t product(bf16x8_t a, bf16x8_t b, f32x4_t acc) {
+  return TRANSPOSED ? mfma_16x16x32(b, a, acc) : mfma_16x16x32(a, b, acc);
+}
+// acc += M B for contraction step 0 of M, B split: the six products above 2^-24, smallest first, four rows
+// of blocks side by side.
+template <bool TRANSPOSED>
+__device__ __forceinline__ void triangle_first(const Triangle& t, const Split& b, f32x4_t (&acc)[4]) {
+  auto step = [&](const bf16x8_t (&part)[kFragments], const bf16x8_t& b0) {
 #pragma unroll
-    for (int m = 2 * C; m < 4; ++m) acc[m] = mfma_16x16x32(part[m], b0, acc[m]);
+    for (int m = 0; m < 4; ++m) acc[m] = product<TRANSPOSED>(part[fragment(m, 0)], b0, acc[m]);
   };
   step(t.lo, b.hi);
   step(t.mid, b.mid);
@@ -150,21 +180,27 @@ __device__ __forceinline__ void triangle_product(const Triangle& t, const Split&
   step(t.hi, b.mid);
   step(t.hi, b.hi);
 }
-// Scheduling of what stands between two fences: N times one matrix instruction and V vector instructions
-// behind it.  A wave alone issues a vector instruction every 5 cycles and a matrix instruction every 16, so
-// two or three of the former run in the shadow of each of the latter, if they stand there.
-template <int N, int V>
-__device__ __forceinline__ void interleave() {
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
-  }
+// The same for step 1, which two rows of blocks reach: three products of each in a sum of their own.
+template <bool TRANSPOSED>
+__device__ __forceinline__ void triangle_second(const Triangle& t, const Split& b, f32x4_t (&acc)[4]) {
+  f32x4_t x2 = {0.f, 0.f, 0.f, 0.f}, x3 = x2;
+  auto step = [&](const bf16x8_t (&pa)[kFragments], const bf16x8_t& ba, const bf16x8_t (&pb)[kFragments], const bf16x8_t& bb) {
+    x2 = product<TRANSPOSED>(pa[fragment(2, 1)], ba, x2);
+    x3 = product<TRANSPOSED>(pa[fragment(3, 1)], ba, x3);
+    acc[2] = product<TRANSPOSED>(pb[fragment(2, 1)], bb, acc[2]);
+    acc[3] = product<TRANSPOSED>(pb[fragment(3, 1)], bb, acc[3]);
+  };
+  step(t.lo, b.hi, t.mid, b.hi);
+  step(t.mid, b.mid, t.hi, b.mid);
+  step(t.hi, b.lo, t.hi, b.hi);
+  acc[2] += x2;
+  acc[3] += x3;
 }
+
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 
 __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int slot, int hv,
-                                            int row) {
+                                            int row, int column) {
   const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
   const int n_chunks = (end - start + kChunk - 1) / kChunk;
   float* srow = p.state + (int64_t)slot * p.state_stride0 + ((int64_t)hv * kDV + row + x16) * kDK + 8 * g;
@@ -172,61 +208,42 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
 #pragma unroll
   for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
 
-  // V and Y of tokens 16 m + 4 g + i of a chunk: one scalar base per chunk, 32-bit offsets of the rows
-  const uint16_t* vrow = p.v + (int64_t)start * p.v_stride0 + hv * kDV + row;
-  const int64_t y_stride = (int64_t)p.hv * kDV;
-  uint16_t* yrow = p.y + (int64_t)start * y_stride + (int64_t)hv * kDV + row;
-  const uint32_t v_step = (uint32_t)p.v_stride0 * 2u, y_step = (uint32_t)y_stride * 2u;
-  uint32_t v_lane = 4 * g * v_step + 2 * x16, y_lane = 4 * g * y_step + 2 * x16;
-  uint32_t v[16];
-  auto load_v = [&](int j) {
-    const int last = end - 1 - start - j * kChunk;
-    const char* base = reinterpret_cast<const char*>(vrow + (int64_t)j * kChunk * p.v_stride0);
-    uint32_t off[16];
-    asm volatile("" : "+v"(v_lane));  // the offsets are made here and now, not kept in 16 registers
-    if (last >= kChunk - 1) {
+  // a lane's part of Y: of token 16 m + x16 the rows 4 g ..
+  const uint32_t y_step = (uint32_t)p.hv * kDV * 2u, y_lane = x16 * y_step + 8 * g;
+  char* ybase = reinterpret_cast<char*>(p.y + ((int64_t)start * p.hv + hv) * kDV + row);
+  const Picker pick;
+  // places of K's and Q's pieces in LDS: as operands, row x16, and transposed, row `trow`, per 32 dims
+  const int trow = 4 * g + (x16 >> 2);
+  uint32_t at[4], kt_at[4];
 #pragma unroll
-      for (int n = 0; n < 16; ++n) off[n] = v_lane + (16 * (n >> 2) + (n & 3)) * v_step;
-    } else {  // rows past the request's end: its last row (counted as zero where it is used)
-#pragma unroll
-      for (int n = 0; n < 16; ++n) off[n] = min(16 * (n >> 2) + 4 * g + (n & 3), last) * v_step + 2 * x16;
-    }
-    // in assembly: loads the compiler knows it packs in pairs, and waits for, where they are issued
-#pragma unroll
-    for (int n = 0; n < 16; ++n) asm volatile("global_load_ushort %0, %1, %2" : "=v"(v[n]) : "v"(off[n]), "s"(base));
-  };
-  auto wait_v = [&]() {
-    asm volatile("s_waitcnt vmcnt(0)"
-                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]),
-                   "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
-  };
-  slot_barrier();  // K, Q of chunk 0
-  slot_barrier();  // A, P of chunk 0
-  slot_barrier();  // T of chunk 0
-
-  // transposing reads of K: token 4 g + x16 / 4 of a tile, dims 8 (x16 % 4) .. of a block of 32
-  const int kt_lane = (4 * g + (x16 >> 2)) * kRowPad + 8 * (x16 & 3);
+  for (int c = 0; c < 4; ++c) {
+    at[c] = x16 * kDK + 8 * piece(x16, 4 * c + g);
+    kt_at[c] = trow * kDK + 8 * piece(trow, 4 * c + (x16 & 3));
+  }
   struct Rows {
     bf16x8_t k[4], q[4];
   };
   auto load_rows = [&](int par, int c, Rows& r) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      r.k[m] = operand(&lds.k[par][16 * m + x16][32 * c + 8 * g]);
-      r.q[m] = operand(&lds.q[par][16 * m + x16][32 * c + 8 * g]);
+      r.k[m] = operand(&lds.k[par][16 * m][0] + at[c]);
+      r.q[m] = operand(&lds.q[par][16 * m][0] + at[c]);
     }
   };
+  __builtin_amdgcn_s_setprio(1);  // before the chunk waves, but in slot 2, where those have the longer way
+  slot_barrier();  // K, Q of chunk 0
+  slot_barrier();  // A of chunk 0
+  slot_barrier();  // what T of chunk 0 is made of
+
   Rows rows[2];
   load_rows(0, 0, rows[0]);
+  Split sp = split(pick, s[0], s[1]);
   for (int j = 0, tri = 0; j < n_chunks; ++j, tri = tri == 2 ? 0 : tri + 1) {
-    const int first = start + j * kChunk, par = j & 1;
-    Triangle tp[2];
+    const int par = j & 1;
     // ---- slot 1 ----------------------------------------------------------------------------
-    load_v(j);
-    f32x4_t x[4], z[4];
+    f32x4_t x[4], z[4];  // X, and Z transposed: a lane's four values are neighbours in a row of Y
 #pragma unroll
     for (int m = 0; m < 4; ++m) x[m] = z[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    Split sp = split(s[0], s[1]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       if (c < 3) load_rows(par, c + 1, rows[(c + 1) & 1]);
@@ -235,27 +252,21 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
       auto step = [&](bf16x8_t part) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-          x[m] = mfma_16x16x32(r.k[m], part, x[m]);
-          z[m] = mfma_16x16x32(r.q[m], part, z[m]);
+          x[m] = product<false>(r.k[m], part, x[m]);
+          z[m] = product<true>(r.q[m], part, z[m]);
         }
       };
-      step(sp.lo);
-      step(sp.mid);
-      step(sp.hi);
-      if (c < 3) {
-        sp = split(s[2 * c + 2], s[2 * c + 3]);
-        interleave<24, 2>();
-      }
+      const Split now = sp;
+      step(now.lo);
+      if (c < 3) sp = split(pick, s[2 * c + 2], s[2 * c + 3]);
+      step(now.mid);
+      step(now.hi);
       fence();
     }
     slot_barrier();
     // ---- slot 2 ----------------------------------------------------------------------------
-    load_triangle(lds.t, 0, tp[0]);
-    wait_v();
-    if (first + kChunk > end) {
-#pragma unroll
-      for (int n = 0; n < 16; ++n) v[n] = first + 16 * (n >> 2) + 4 * g + (n & 3) < end ? v[n] : 0u;
-    }
+    Triangle tp;
+    load_triangle<0, 4>(lds.t, tp);
     f32x4_t u[4];
     {
       f32x4_t r[4];
@@ -263,93 +274,98 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
       for (int m = 0; m < 4; ++m) {
         const f32x4_t bet = *reinterpret_cast<const f32x4_t*>(&lds.beta[tri][16 * m + 4 * g]);
         const f32x4_t gam = *reinterpret_cast<const f32x4_t*>(&lds.gamma[tri][16 * m + 4 * g]);
+        const u32x2_t v = lds_read_tr16(reinterpret_cast<const unsigned char*>(&lds.v[16 * m + trow][column + 4 * (x16 & 3)]));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[m][i] = (bf16_bits_to_f32(v[4 * m + i]) - gam[i] * x[m][i]) * bet[i];
-        z[m] *= gam;
+        for (int i = 0; i < 4; ++i)
+          r[m][i] = (bf16_bits_to_f32(i & 1 ? v[i >> 1] >> 16 : v[i >> 1] & 0xffffu) - gam[i] * x[m][i]) * bet[i];
         u[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
-      load_triangle(lds.t, 1, tp[1]);
-      const Split rs0 = split(r[0], r[1]);
-      fence();
-      triangle_product<0>(tp[0], rs0, u);
-      const Split rs1 = split(r[2], r[3]);
-      interleave<24, 2>();
-      fence();
-      load_triangle(lds.p, 0, tp[0]);
-      triangle_product<1>(tp[1], rs1, u);
+      load_triangle<4, 6>(lds.t, tp);
+      const Split rs0 = split(pick, r[0], r[1]);
+      const Split rs1 = split(pick, r[2], r[3]);
+      triangle_first<false>(tp, rs0, u);
+      triangle_second<false>(tp, rs1, u);
     }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) z[m] *= lds.gamma[tri][16 * m + x16];
+    fence();
+    load_triangle<0, 4>(lds.p, tp);
     slot_barrier();
     // ---- slot 3 ----------------------------------------------------------------------------
-    const uint16_t* kt = &lds.k[par][0][0] + kt_lane;
-    auto load_kt = [&](int n, bf16x8_t (&ka)[4]) {  // contraction step n / 2, dims 64 (n % 2) ..
+    const uint16_t* k = &lds.k[par][0][0];
+    auto load_kt = [&](int n, bf16x8_t (&ka)[4]) {  // K transposed: tokens 32 (n % 2) .., dims 64 (n / 2) ..
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int c = 4 * (n & 1) + i;
-        const uint16_t* at = kt + 32 * (c >> 1) + 4 * (c & 1) + 32 * (n >> 1) * kRowPad;
-        const u32x2_t a0 = lds_read_tr16(reinterpret_cast<const unsigned char*>(at));
-        const u32x2_t a1 = lds_read_tr16(reinterpret_cast<const unsigned char*>(at + 16 * kRowPad));
+        const int c = 4 * (n >> 1) + i;
+        const uint16_t* a = k + kt_at[c >> 1] + 4 * (c & 1) + 32 * (n & 1) * kDK;
+        const u32x2_t a0 = lds_read_tr16(reinterpret_cast<const unsigned char*>(a));
+        const u32x2_t a1 = lds_read_tr16(reinterpret_cast<const unsigned char*>(a + 16 * kDK));
         ka[i] = as_bf16x8(u32x4_t{a0[0], a0[1], a1[0], a1[1]});
       }
     };
-    load_triangle(lds.p, 1, tp[1]);
-    {
-      const Split us0 = split(u[0], u[1]);
-      fence();
-      triangle_product<0>(tp[0], us0, z);
-      const Split us1 = split(u[2], u[3]);
-      interleave<24, 2>();
-      fence();
-      bf16x8_t ka[2][4];
-      load_kt(0, ka[0]);
-      f32x4_t tail[4];
+    bf16x8_t ka[2][4];
+    f32x4_t tail[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) tail[m] = *reinterpret_cast<const f32x4_t*>(&lds.tail[tri][16 * m + 4 * g]);
-      const float total = lds.total[tri];
-      triangle_product<1>(tp[1], us1, z);
+    for (int m = 0; m < 4; ++m) tail[m] = *reinterpret_cast<const f32x4_t*>(&lds.tail[tri][16 * m + 4 * g]);
+    const float total = lds.total[tri];
+    load_triangle<4, 6>(lds.p, tp);
+    load_kt(0, ka[0]);
+    load_kt(1, ka[1]);
+    const Split us0 = split(pick, u[0], u[1]);
+    const Split us1 = split(pick, u[2], u[3]);
+    fence();
+    triangle_first<true>(tp, us0, z);
+    const Split ut0 = split(pick, u[0] * tail[0], u[1] * tail[1]);
+    const Split ut1 = split(pick, u[2] * tail[2], u[3] * tail[3]);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) s[c] *= total;
-      const Split ut0 = split(u[0] * tail[0], u[1] * tail[1]);
-      interleave<12, 5>();
-      fence();
-      auto step = [&](int n, bf16x8_t part) {
+    for (int c = 0; c < 8; ++c) s[c] *= total;
+    fence();
+    triangle_second<true>(tp, us1, z);
+    auto steps = [&](int n, const Split& b) {
+      auto step = [&](bf16x8_t part) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[4 * (n & 1) + i] = mfma_16x16x32(ka[n & 1][i], part, s[4 * (n & 1) + i]);
+        for (int i = 0; i < 4; ++i) s[4 * (n >> 1) + i] = mfma_16x16x32(ka[n & 1][i], part, s[4 * (n >> 1) + i]);
       };
-      auto steps = [&](int n, const Split& b) {
-        step(n, b.lo);
-        step(n, b.mid);
-        step(n, b.hi);
-      };
-      load_kt(1, ka[1]);
-      steps(0, ut0);
-      const Split ut1 = split(u[2] * tail[2], u[3] * tail[3]);
-      interleave<12, 4>();
-      fence();
-      load_kt(2, ka[0]);
-      steps(1, ut0);
-      fence();
-      load_kt(3, ka[1]);
-      steps(2, ut1);
-      fence();
-      load_rows(par ^ 1, 0, rows[0]);  // of chunk j + 1 (of no use behind the last chunk)
-      steps(3, ut1);
-      char* base = reinterpret_cast<char*>(yrow + (int64_t)j * kChunk * y_stride);
-      asm volatile("" : "+v"(y_lane));
-      const bool whole = first + kChunk <= end;
+      step(b.lo);
+      step(b.mid);
+      step(b.hi);
+    };
+    steps(0, ut0);
+    fence();
+    load_kt(2, ka[0]);
+    steps(1, ut1);
+    fence();
+    load_kt(3, ka[1]);
+    steps(2, ut0);
+    char* to = ybase + (int64_t)j * kChunk * y_step;
+    const int left = end - start - j * kChunk;
+    auto store = [&](int m) {
+      *reinterpret_cast<u32x2_t*>(to + (y_lane + 16 * m * y_step)) = u32x2_t{pack_bf16x2(z[m][0], z[m][1]), pack_bf16x2(z[m][2], z[m][3])};
+    };
+    if (left >= kChunk) {
 #pragma unroll
-      for (int n = 0; n < 16; ++n) {
-        const uint16_t bits = __builtin_bit_cast(uint16_t, (__bf16)z[n >> 2][n & 3]);
-        uint16_t* to = reinterpret_cast<uint16_t*>(base + (y_lane + (16 * (n >> 2) + (n & 3)) * y_step));
-        if (whole) *to = bits;
-        else if (first + 16 * (n >> 2) + 4 * g + (n & 3) < end) *to = bits;
-      }
+      for (int m = 0; m < 4; ++m) store(m);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (16 * m + x16 < left) store(m);
     }
+    fence();
+    load_rows(par ^ 1, 0, rows[0]);  // of chunk j + 1 (of no use behind the last chunk)
+    steps(3, ut1);
+    sp = split(pick, s[0], s[1]);
     slot_barrier();
   }
 #pragma unroll
   for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
 }
 
+// A value from another lane of the row of 16, 1 where there is none.  DPP control C: 0x110 + n the lane n below,
+// 0x100 + n the lane n above.
+template <int C>
+__device__ __forceinline__ float row_shift(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), C, 0xf, 0xf, false));
+}
 // Lane t of every row of 16 lanes, in all of them.
 template <int T>
 __device__ __forceinline__ float row_broadcast(float x) {
@@ -372,39 +388,27 @@ __device__ __forceinline__ f32x4_t mfma_f32_block(f32x4_t a, f32x4_t b, f32x4_t 
   return c;
 }
 
-// Column block W of T below the diagonal: T_rW = -T_rr X_r, X_r = sum over W <= k < r of A_rk T_kW.  T_rW is
-// made twice, as the operand of the rows below it and transposed, four neighbours of a row to a lane, for
-// LDS.  Everything the chain needs from LDS is asked for before it starts.
-template <int W>
-__device__ __forceinline__ void column_block(ChunkLds& lds) {
-  const int x16 = lane_id() & 15, g = lane_id() >> 4;
-  f32x4_t a[4][4], d[4], tk[4];
+// Blocks (R, C) of T below the diagonal from those of A and the inverses on the diagonal:
+// T_RC = -T_RR X_R, X_R = sum over C <= k < R of A_Rk T_kC.  A block is made as the operand of the rows below it
+// and transposed, four neighbours of a row to a lane, for LDS (T_RC^T = -X_R^T T_RR^T).  Operands of that:
+struct Inverse {
+  const ChunkLds& lds;
+  int x16, g;
+  __device__ __forceinline__ explicit Inverse(const ChunkLds& l) : lds(l), x16(lane_id() & 15), g(lane_id() >> 4) {}
+  __device__ __forceinline__ f32x4_t a(int r, int k) const { return *reinterpret_cast<const f32x4_t*>(&lds.a[16 * r + x16][16 * k + 4 * g]); }
+  __device__ __forceinline__ f32x4_t minus_diag(int r) const { return -*reinterpret_cast<const f32x4_t*>(&lds.diag[r][x16][4 * g]); }
+  __device__ __forceinline__ f32x4_t diag_plain(int r) const {
+    f32x4_t d;
 #pragma unroll
-  for (int n = 0; n < 4; ++n) tk[W][n] = lds.diag[W][4 * g + n][x16];
-#pragma unroll
-  for (int r = W + 1; r < 4; ++r) {
-#pragma unroll
-    for (int k = W; k < r; ++k) a[r][k] = *reinterpret_cast<const f32x4_t*>(&lds.a[16 * r + x16][16 * k + 4 * g]);
-    d[r] = *reinterpret_cast<const f32x4_t*>(&lds.diag[r][x16][4 * g]);
+    for (int n = 0; n < 4; ++n) d[n] = lds.diag[r][4 * g + n][x16];
+    return d;
   }
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4_t x[4];
-#pragma unroll
-  for (int r = W + 1; r < 4; ++r) x[r] = mfma_f32_block(a[r][W], tk[W], zero);
-#pragma unroll
-  for (int r = W + 1; r < 4; ++r) {
-    const f32x4_t minus = -d[r];
-    if (r < 3) {
-      tk[r] = mfma_f32_block(minus, x[r], zero);
-#pragma unroll
-      for (int n = r + 1; n < 4; ++n) x[n] = mfma_f32_block(a[n][r], tk[r], x[n]);
-    }
-    split_store(mfma_f32_block(x[r], minus, zero), lds.t, 16 * r + x16, token_column(W, g));
-  }
-}
+};
 
-__device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int hv, int w) {
+__device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int hv,
+                                            int wg_row, int w) {
   const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
+  const Picker pick;
   const int n_chunks = (end - start + kChunk - 1) / kChunk;
   const int hk = hv / p.hv_per_hk;
   // this wave's 16 tokens of K and Q, four rows per load, and every token's gates: scalar bases at the
@@ -414,6 +418,17 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
   const char* gbase = reinterpret_cast<const char*>(p.g + (int64_t)start * p.hv + hv);
   const char* bbase = reinterpret_cast<const char*>(p.beta + (int64_t)start * p.hv + hv);
   const uint32_t k_step = (uint32_t)p.k_stride0 * 2u, q_step = (uint32_t)p.q_stride0 * 2u, g_step = (uint32_t)p.hv * 2u;
+  // V of the workgroup's rows, 8 tokens a load, straight to LDS; rows past the request's end: the last row
+  // (beta is zero there)
+  const char* vbase = reinterpret_cast<const char*>(p.v + (int64_t)start * p.v_stride0 + hv * kDV + wg_row);
+  const uint32_t v_step = (uint32_t)p.v_stride0 * 2u, v_lds = (uint32_t)(uintptr_t)MSGL_LDS_PTR(uint16_t, &lds.v[16 * w][0]);
+  auto fetch_v = [&](int first) {
+    const char* base = vbase + (int64_t)(first - start) * v_step;
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      lds_direct_b128(__builtin_amdgcn_readfirstlane(v_lds + 1024 * n), base,
+                      min((uint32_t)(16 * w + 8 * n + (lane >> 3)), (uint32_t)(end - 1 - first)) * v_step + 16 * (lane & 7));
+  };
   u32x4_t kr[4], qr[4];
   uint32_t graw, braw;
   auto fetch = [&](int first) {
@@ -436,8 +451,8 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
       const int t = 16 * w + 4 * n + g;
       const u32x4_t zero = {0u, 0u, 0u, 0u};
       const bool in = first + t < end;
-      *reinterpret_cast<u32x4_t*>(&lds.k[par][t][8 * x16]) = in ? kr[n] : zero;
-      *reinterpret_cast<u32x4_t*>(&lds.q[par][t][8 * x16]) = in ? qr[n] : zero;
+      *reinterpret_cast<u32x4_t*>(&lds.k[par][t][8 * piece(t, x16)]) = in ? kr[n] : zero;
+      *reinterpret_cast<u32x4_t*>(&lds.q[par][t][8 * piece(t, x16)]) = in ? qr[n] : zero;
     }
   };
   // decay products of a chunk from the gates fetched with it: the last wave's work, it has the least to do
@@ -445,19 +460,18 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
   auto decays = [&](int first, int tri) {
     const bool in = first + lane < end;
     const float gv = in ? bf16_bits_to_f32(graw) : 1.0f, bv = in ? bf16_bits_to_f32(braw) : 0.0f;
-    float pre = gv, suf = gv, quad_pre = gv;
-#pragma unroll
-    for (int n = 1; n < 16; n <<= 1) {
-      const float a = __shfl_up(pre, n, 16), b = __shfl_down(suf, n, 16);
-      if (n < 4) {
-        const float q = __shfl_up(quad_pre, n, 4);
-        if ((x16 & 3) >= n) quad_pre *= q;
-      }
-      if (x16 >= n) pre *= a;
-      if (x16 + n < 16) suf *= b;
-    }
-    const float after = __shfl_down(suf, 1, 16);
-    suf = x16 == 15 ? 1.0f : after;
+    // products over a row of 16 lanes, or over quads (every lane shifts, then takes what is in its quad)
+    const float before1 = row_shift<0x111>(gv);
+    float pre = gv * before1, suf = gv * row_shift<0x101>(gv), quad_pre = gv * ((x16 & 3) >= 1 ? before1 : 1.0f);
+    const float quad2 = row_shift<0x112>(quad_pre);
+    quad_pre *= (x16 & 3) >= 2 ? quad2 : 1.0f;
+    pre *= row_shift<0x112>(pre);
+    suf *= row_shift<0x102>(suf);
+    pre *= row_shift<0x114>(pre);
+    suf *= row_shift<0x104>(suf);
+    pre *= row_shift<0x118>(pre);
+    suf *= row_shift<0x108>(suf);
+    suf = row_shift<0x101>(suf);  // behind the token
     auto lane_value = [](float f, int l) {
       return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), l));
     };
@@ -475,54 +489,50 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
     if ((lane & 3) == 3) lds.quad[lane >> 2] = quad_pre;
     if (lane == 0) lds.total[tri] = b0 * b1 * b2 * b3;
   };
-  // The ten blocks (r, c) of A and P on and below the diagonal: every wave its diagonal block, waves 0-2
-  // two more.  Results are transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n), so that a
+  // The ten blocks (r, c) of A and P on and below the diagonal: every wave its diagonal block and one
+  // more, waves 1 and 2 two.  Results are transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n), so that a
   // lane's four values are neighbours in a row of A and of P.
-  const int n_blocks = w == 3 ? 1 : 3;
+  const int n_blocks = w == 0 || w == 3 ? 2 : 3;
   auto block_row = [&](int n) { return n == 0 ? w : n == 1 ? (w == 0 ? 3 : w) : (w == 2 ? 2 : 3); };
-  auto block_col = [&](int n) { return n == 0 ? w : n == 1 ? 0 : (w == 1 ? 2 : 1); };
-  f32x4_t pp[3];  // P of these blocks
+  auto block_col = [&](int n) { return n == 0 ? w : n == 1 ? (w == 3 ? 1 : 0) : (w == 1 ? 2 : 1); };
+  f32x4_t pp[3];  // the ratios of P of these blocks, then P
   f32x4_t inv;    // the inverse of the diagonal block: row x16, columns 4 g ..
   auto products = [&](int par, int tri) {
     struct Block {
-      bf16x8_t kc[4], kr[4], qr[4];
+      bf16x8_t kc[4], kr[4];
       f32x4_t col;
       float row, beta;
     };
     auto load = [&](int r, int c, Block& x) {
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        x.kc[d] = operand(&lds.k[par][16 * c + x16][32 * d + 8 * g]);
-        x.kr[d] = operand(&lds.k[par][16 * r + x16][32 * d + 8 * g]);
-        x.qr[d] = operand(&lds.q[par][16 * r + x16][32 * d + 8 * g]);
+        x.kc[d] = operand(&lds.k[par][16 * c + x16][8 * piece(x16, 4 * d + g)]);
+        x.kr[d] = operand(&lds.k[par][16 * r + x16][8 * piece(x16, 4 * d + g)]);
       }
       x.beta = lds.beta[tri][16 * r + x16];
       x.row = r == c ? lds.quad_pre[16 * r + x16] : lds.pre[16 * r + x16];
       x.col = *reinterpret_cast<const f32x4_t*>(r == c ? &lds.g[16 * r + 4 * g] : &lds.suf[16 * c + 4 * g]);
     };
-    auto dots = [&](const Block& x, f32x4_t& kk, f32x4_t& qk) {
-      kk = qk = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto dots = [&](const Block& x) {
+      f32x4_t kk = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        kk = mfma_16x16x32(x.kc[d], x.kr[d], kk);
-        qk = mfma_16x16x32(x.kc[d], x.qr[d], qk);
-      }
+      for (int d = 0; d < 4; ++d) kk = mfma_16x16x32(x.kc[d], x.kr[d], kk);
+      return kk;
     };
     // G_t / G_i of a block below the diagonal: token t's block up to it, whole blocks, token i's block behind it
-    auto below = [&](int n, int r, int c, const Block& x, const f32x4_t& kk, const f32x4_t& qk) {
+    auto below_block = [&](int n, int r, int c, const Block& x, const f32x4_t& kk) {
       float row = x.row;
       if (c < 1 && r > 1) row *= lds.block[1];
       if (c < 2 && r > 2) row *= lds.block[2];
       const f32x4_t ratio = row * x.col;
-      pp[n] = ratio * qk;
+      pp[n] = ratio;
       *reinterpret_cast<f32x4_t*>(&lds.a[16 * r + x16][16 * c + 4 * g]) = x.beta * ratio * kk;
     };
     Block b0, b1, b2;
-    f32x4_t kk0, qk0, kk1, qk1, kk2, qk2;
     const int r1 = block_row(1), c1 = block_col(1), r2 = block_row(2), c2 = block_col(2);
     load(w, w, b0);
-    if (n_blocks > 1) load(r1, c1, b1);
-    dots(b0, kk0, qk0);
+    load(r1, c1, b1);
+    const f32x4_t kk0 = dots(b0);
     {
       // on the diagonal: token t's quad up to it and the quads between, then token by token down the columns
       float far = b0.row;
@@ -535,7 +545,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         a[i] = 4 * g + i < x16 ? b0.beta * ratio[i] * kk0[i] : 0.f;
-        pp[0][i] = 4 * g + i <= x16 ? ratio[i] * qk0[i] : 0.f;
+        pp[0][i] = 4 * g + i <= x16 ? ratio[i] : 0.f;
       }
       *reinterpret_cast<f32x4_t*>(&lds.a[16 * w + x16][16 * w + 4 * g]) = a;
     }
@@ -548,55 +558,117 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n) inv[n] = x16 == 4 * g + n ? 1.0f : 0.0f;
-    if (n_blocks > 1) {
+    if (n_blocks > 2) {
       load(r2, c2, b2);
-      dots(b1, kk1, qk1);
-      dots(b2, kk2, qk2);
+      const f32x4_t kk1 = dots(b1), kk2 = dots(b2);
       eliminate<0>(arow, inv);
-      below(1, r1, c1, b1, kk1, qk1);
-      below(2, r2, c2, b2, kk2, qk2);
+      below_block(1, r1, c1, b1, kk1);
+      below_block(2, r2, c2, b2, kk2);
     } else {
+      const f32x4_t kk1 = dots(b1);
       eliminate<0>(arow, inv);
+      below_block(1, r1, c1, b1, kk1);
     }
     *reinterpret_cast<f32x4_t*>(&lds.diag[w][x16][4 * g]) = inv;
   };
+  auto finish_p = [&](int par) {  // P = ratios times <k, q>
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      if (n >= n_blocks) break;
+      f32x4_t qk = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        qk = mfma_16x16x32(operand(&lds.k[par][16 * block_col(n) + x16][8 * piece(x16, 4 * d + g)]),
+                           operand(&lds.q[par][16 * block_row(n) + x16][8 * piece(x16, 4 * d + g)]), qk);
+      pp[n] *= qk;
+    }
+  };
+  // Blocks of T below the diagonal, two waves with the first column: (1, 0) and (2, 0); (2, 1) and (3, 1); (3, 2);
+  // (3, 0).  Everything a chain needs from LDS is asked for before it starts.
+  f32x4_t below[2];
   auto inverse = [&]() {
-    split_store(inv, lds.t, 16 * w + x16, token_column(w, g));
-    if (w == 0) column_block<0>(lds);
-    else if (w == 1) column_block<1>(lds);
-    else if (w == 2) column_block<2>(lds);
+    const Inverse of(lds);
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    if (w == 2) {
+      const f32x4_t a32 = of.a(3, 2), t2 = of.diag_plain(2), d3 = of.minus_diag(3);
+      below[0] = mfma_f32_block(mfma_f32_block(a32, t2, zero), d3, zero);
+    } else if (w == 1) {
+      const f32x4_t a21 = of.a(2, 1), a31 = of.a(3, 1), a32 = of.a(3, 2), t1 = of.diag_plain(1), d2 = of.minus_diag(2), d3 = of.minus_diag(3);
+      const f32x4_t x2 = mfma_f32_block(a21, t1, zero);
+      f32x4_t x3 = mfma_f32_block(a31, t1, zero);
+      const f32x4_t t21 = mfma_f32_block(d2, x2, zero);
+      below[0] = mfma_f32_block(x2, d2, zero);
+      x3 = mfma_f32_block(a32, t21, x3);
+      below[1] = mfma_f32_block(x3, d3, zero);
+    } else {
+      const f32x4_t a10 = of.a(1, 0), a20 = of.a(2, 0), a21 = of.a(2, 1), t0 = of.diag_plain(0), d1 = of.minus_diag(1), d2 = of.minus_diag(2);
+      if (w == 0) {
+        const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
+        f32x4_t x2 = mfma_f32_block(a20, t0, zero);
+        const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
+        below[0] = mfma_f32_block(x1, d1, zero);
+        x2 = mfma_f32_block(a21, t10, x2);
+        below[1] = mfma_f32_block(x2, d2, zero);
+      } else {
+        const f32x4_t a30 = of.a(3, 0), a31 = of.a(3, 1), a32 = of.a(3, 2), d3 = of.minus_diag(3);
+        const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
+        f32x4_t x2 = mfma_f32_block(a20, t0, zero), x3 = mfma_f32_block(a30, t0, zero);
+        const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
+        x2 = mfma_f32_block(a21, t10, x2);
+        x3 = mfma_f32_block(a31, t10, x3);
+        const f32x4_t t20 = mfma_f32_block(d2, x2, zero);
+        x3 = mfma_f32_block(a32, t20, x3);
+        below[0] = mfma_f32_block(x3, d3, zero);
+      }
+    }
+  };
+  auto store_t = [&]() {
+    split_store(pick, inv, lds.t, w, w);
+    const int r = w == 0 ? 1 : w == 1 ? 2 : 3, c = w == 1 ? 1 : w == 2 ? 2 : 0;
+    split_store(pick, below[0], lds.t, r, c);
+    if (w < 2) split_store(pick, below[1], lds.t, r + 1, c);
   };
   auto store_p = [&]() {
 #pragma unroll
     for (int n = 0; n < 3; ++n) {
       if (n >= n_blocks) break;
-      split_store(pp[n], lds.p, 16 * block_row(n) + x16, token_column(block_col(n), g));
+      split_store(pick, pp[n], lds.p, block_row(n), block_col(n));
     }
   };
 
   fetch(start);
   stage(start, 0);
-  if (w == 3) decays(start, 0);
+  if (w == 2) decays(start, 0);
   slot_barrier();
+  fetch_v(start);
   if (n_chunks > 1) fetch(start + kChunk);
   products(0, 0);
   slot_barrier();
+  finish_p(0);
   inverse();
-  if (w == 3 && n_chunks > 1) decays(start + kChunk, 1);
+  if (w == 2 && n_chunks > 1) decays(start + kChunk, 1);
   slot_barrier();
   int tri = 1;  // of chunk j + 1, modulo 3
   for (int j = 0; j < n_chunks; ++j) {
     const int next = start + (j + 1) * kChunk, par = (j + 1) & 1;
     const bool more = j + 1 < n_chunks, two = j + 2 < n_chunks;
+    store_t();
     store_p();
+    wait_all_vm();  // V of chunk j is in LDS
     if (more) stage(next, par);
     if (two) fetch(next + kChunk);
     slot_barrier();
+    __builtin_amdgcn_s_setprio(2);
     if (more) products(par, tri);
+    __builtin_amdgcn_s_setprio(0);
     slot_barrier();
     tri = tri == 2 ? 0 : tri + 1;
-    if (more) inverse();
-    if (w == 3 && two) decays(next + kChunk, tri);
+    if (more) {
+      fetch_v(next);
+      finish_p(par);
+      inverse();
+    }
+    if (w == 2 && two) decays(next + kChunk, tri);
     slot_barrier();
   }
 }
@@ -643,8 +715,8 @@ __global__ __launch_bounds__(512) void gdn_chunk_kernel(GdnParams p, int ranked)
   // the blocks of T and P above the diagonal that are read are never written: zero from here on
   for (int i = threadIdx.x; i < (int)(sizeof(lds.t) + sizeof(lds.p)) / 16; i += 512)
     reinterpret_cast<u32x4_t*>(&lds.t[0][0][0])[i] = u32x4_t{0u, 0u, 0u, 0u};
-  if (wave < 4) state_waves(p, lds, start, end, p.slot_ids[b], hv, row + 16 * wave);
-  else chunk_waves(p, lds, start, end, hv, wave - 4);
+  if (wave < 4) state_waves(p, lds, start, end, p.slot_ids[b], hv, row + 16 * wave, 16 * wave);
+  else chunk_waves(p, lds, start, end, hv, row, wave - 4);
 }
 
 }  // namespace

@@ -166,6 +166,7 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 static bool prefer_chunks(const GdnArgs& a) {
   if (a.v_stride0 >= (1 << 24) || a.k_stride0 >= (1 << 24) || a.q_stride0 >= (1 << 24) || a.hv >= (1 << 17))
     return false;  // its offsets inside a chunk are 32 bits wide
+  if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return false;  // loads of 16 bytes, stores of 8
   const double units = (double)(a.batch * a.hv) / 32, mean = (double)a.tokens / (double)a.batch;
   const double rounds = (double)((a.batch * a.hv * 2 + device_cus() - 1) / device_cus());
   return 12.8 * rounds < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
