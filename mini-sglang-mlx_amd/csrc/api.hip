@@ -56,11 +56,29 @@ int32_t segments(int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols)
   return msgl::splitkv_default_segments(total_kv, n_kv, head_dim, cols, min_segment(head_dim));
 }
 // Shares instead of segments (paged_shares.hip); a knob that shapes the segments asks for segments.
-msgl::SharePlan shares_for(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols) {
+msgl::SharePlan shares_for(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (t_tune[MSGL_TUNE_SEGMENTS] != 0 || t_tune[MSGL_TUNE_MIN_SEGMENT] != 0 || t_last_set[MSGL_TUNE_SPLITKV_WAVES] != 0 ||
       t_last_set[MSGL_TUNE_SPLITKV_BOUNDARY] != 0)
     return msgl::SharePlan{};
-  return msgl::share_plan(batch, total_kv, n_kv, head_dim, cols);
+  return msgl::share_plan(batch, keys, each, n_kv, head_dim, cols);
+}
+// The keys that the rows of a launch see, at most.
+int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t max_len_extend, bool is_cross) {
+  if (window <= 0 || is_cross) return total_kv;
+  return std::min(total_kv, batch * (window + max_len_extend + 15));  // a window starts at a multiple of 16
+}
+// Under a sliding window that most requests exceed every request shows about `window` keys: one workgroup per
+// (request, kv head) is balanced as it is, whatever the requests' lengths, and needs no second launch.  Up to three
+// column tiles and windows of some thousand keys the share kernel is that workgroup: 32 requests of 8 tokens,
+// 32 / 8 heads, window 1024: 42.8 us in the tile kernel with its merge launch, 38 in shares; 64 of 4 tokens, 64 / 8
+// heads: 76 and 61; 64 of 16, 16 / 8 heads: 76 and 63; 16 of 4, 32 / 8: 23.6 both.
+// Beyond 32 columns a workgroup of several kv heads has a wave, and most of a window's time, for each (66 requests
+// of 6 tokens, 64 / 8 heads: 83 us in the tile kernel, 89 in shares).
+bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv, int64_t keys, int64_t n_kv,
+                   int64_t head_dim, int64_t cols) {
+  if (plan.share_len == 0 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
+  if (head_dim == 256 && batch * n_kv < 12) return false;  // see shares_preferred()
+  return cols <= 32 || plan.heads_wg == 1;
 }
 // Largest q_len * group that takes the split-K route whatever the launch: at head_dim 128 48 (up
 // to three column tiles in one wave; 49-64 columns would run on two waves per kv head that each
@@ -175,8 +193,8 @@ size_t msgl_paged_decode_workspace_bytes(int64_t batch, int64_t total_kv, int64_
       num_q_heads % num_kv_heads != 0)
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
-  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, group);
-  if (msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group, 0, 1))
+  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  if (msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group))
     return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
   return msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1,
                                        segments(total_kv, num_kv_heads, head_dim, group));
@@ -202,8 +220,8 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
   if (!kv_indptr || !num_kv_splits || (total_kv > 0 && !kv_indices)) return MSGL_ERR_NULL_POINTER;
   (void)max_kv_splits;  // split hints do not steer the cut (result is split-invariant)
   const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, group);
-  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, group);
-  const bool shares = msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group, 0, 1);
+  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  const bool shares = msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group);
   const size_t need = shares
                           ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group)
                           : msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1, n_seg);
@@ -315,28 +333,29 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
       num_q_heads % num_kv_heads != 0)
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
+  const int64_t cols = group * max_len_extend;
+  // a window, unknown here, may make the launch one for shares
+  size_t share_need = 0;
+  if (const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, cols); plan.share_len > 0)
+    share_need = msgl::share_workspace_bytes(msgl::with_any_window(plan, batch, num_kv_heads), batch, num_kv_heads, head_dim, cols);
   if (!use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads)) {
     // tile kernels: partials of a key split, if this launch would use one (a sliding window,
     // unknown here, can only lower the count)
     const int ragged = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
     if (ragged > 0)
-      return msgl::prefill_ragged_workspace_bytes(batch, total_kv, num_kv_heads, group,
-                                                  max_len_extend, head_dim, ragged);
+      return std::max(share_need, msgl::prefill_ragged_workspace_bytes(batch, total_kv, num_kv_heads, group,
+                                                                       max_len_extend, head_dim, ragged));
     const int k = msgl::prefill_key_splits(batch, total_kv, num_kv_heads, group, max_len_extend, 0,
                                            msgl::prefill_block_rows(head_dim), t_key_splits);
     const int gangs = gangs_for(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim, 0, k);
-    const size_t split_need = msgl::prefill_split_workspace_bytes(total_q, num_q_heads, head_dim, k);
+    const size_t split_need = std::max(share_need, msgl::prefill_split_workspace_bytes(total_q, num_q_heads, head_dim, k));
     if (gangs > 0)
       return std::max(split_need, msgl::prefill_gang_workspace_bytes(batch, num_kv_heads, group, max_len_extend, gangs));
     return split_need;
   }
-  const int64_t cols = group * max_len_extend;
-  size_t split_need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend,
-                                                    segments(total_kv, num_kv_heads, head_dim, cols));
-  // a window, unknown here too, may make the launch one for shares
-  const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, cols);
-  if (plan.share_len > 0)
-    split_need = std::max(split_need, msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols));
+  const size_t split_need =
+      std::max(share_need, msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend,
+                                                         segments(total_kv, num_kv_heads, head_dim, cols)));
   // a sliding window (unknown here) may send the launch to the tile kernel instead
   const int ragged = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
   const size_t tile_need = ragged > 0 ? msgl::prefill_ragged_workspace_bytes(batch, total_kv, num_kv_heads, group,
@@ -368,17 +387,19 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     return MSGL_ERR_NULL_POINTER;
   const int64_t group = num_q_heads / num_kv_heads;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool direct = use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
-                      !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
-                                            sliding_window_size);
+  const int64_t cols = group * max_len_extend;
+  const int64_t keys = visible_keys(batch, total_kv, sliding_window_size, max_len_extend, is_cross_attention != 0);
+  const msgl::SharePlan plan = shares_for(batch, keys, keys < total_kv ? keys / batch : 0, num_kv_heads, head_dim, cols);
+  const bool window_share = window_shares(plan, batch, total_kv, keys, num_kv_heads, head_dim, cols);
+  const bool direct = window_share ||
+                      (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
+                       !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
+                                             sliding_window_size));
   if (direct) {
-    const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, group * max_len_extend);
-    const int64_t cols = group * max_len_extend;
-    const msgl::SharePlan plan = shares_for(batch, total_kv, num_kv_heads, head_dim, cols);
-    const bool shares = msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, cols,
-                                               sliding_window_size, max_len_extend);
+    const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, cols);
+    const bool shares = window_share || msgl::shares_preferred(plan, batch, keys, num_kv_heads, head_dim, cols);
     const size_t need = shares
-                            ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group * max_len_extend)
+                            ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols)
                             : msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim,
                                                             max_len_extend, n_seg);
     if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;

@@ -65,10 +65,12 @@ struct SharePlan {
   int32_t heads_wg;     // adjacent kv heads of a workgroup
   int64_t max_shares;   // most shares these sizes can give
 };
-SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols);
+// for `keys` visible keys in all; each > 0: about so many in every request
+SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols);
+// the same plan with as many shares as under any sliding window: for the size of a workspace
+SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv);
 // whether the launch is small enough for its shares to beat the segment kernel
-bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim,
-                      int64_t cols, int64_t window, int64_t max_len_extend);
+bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols);
 int device_cus();  // paged_splitkv.hip
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);
 int launch_shares(const SplitKvArgs& a, const SharePlan& plan, hipStream_t stream);

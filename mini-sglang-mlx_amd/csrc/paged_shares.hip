@@ -297,7 +297,7 @@ std::atomic<unsigned long long> g_nonce{1};
 
 void shares_force(int64_t v) { t_force = v; }
 
-SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols) {
+SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols) {
   SharePlan plan{};
   const int nct = nct_of(cols);
   if (t_force < 0 || batch < 1 || cols < 1 || nct > (head_dim == 128 ? 3 : 1)) return plan;
@@ -315,14 +315,26 @@ SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head
     // at most 16 of an average request: the last of them reads the others' partials
     len = nct == 3 ? 512 : (nw == 4 && heads == 1) ? 256 : 128;
     auto fits = [&](int64_t c) {
-      return std::max(batch, total_kv / c + batch / 2) * (n_kv / heads) <= slots && total_kv <= 16 * c * batch;
+      return std::max(batch, keys / c + batch / 2) * (n_kv / heads) <= slots && keys <= 16 * c * batch;
     };
-    while (!fits(len) && len < (1 << 19)) len *= 2;
+    if (each > 0) {  // one length for all: as many equal shares as fit
+      const int64_t n = std::min<int64_t>(std::max<int64_t>(slots * heads / (batch * n_kv), 1), 16);
+      len = std::max(len, ((each + n - 1) / n + 31) & ~(int64_t)31);
+    } else {
+      while (!fits(len) && len < (1 << 19)) len *= 2;
+    }
   }
   plan.share_len = (int32_t)len;
   plan.heads_wg = (int32_t)heads;
   plan.share_waves = nw / plan.heads_wg;
-  plan.max_shares = total_kv / plan.share_len + batch;
+  plan.max_shares = keys / plan.share_len + batch;
+  return plan;
+}
+
+// Fewer visible keys make shorter shares, but never more of them than fit the chip in one round.
+SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
+  const int64_t one_round = device_cus() * plan.heads_wg / n_kv;
+  plan.max_shares = std::max(plan.max_shares, one_round + batch);
   return plan;
 }
 
@@ -334,12 +346,9 @@ SharePlan share_plan(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head
 // costs are the same for any number of bytes, while a share's last workgroup has ever more partials
 // to read and the shares' lengths vary: one request of 12 K keys 16.6 -> 19.2, 12 of 3-8 K 59 -> 71.
 // The lines lie where the two meet.
-bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t total_kv, int64_t n_kv, int64_t head_dim,
-                      int64_t cols, int64_t window, int64_t max_len_extend) {
+bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
-  int64_t keys = total_kv;
-  if (window > 0) keys = std::min(keys, batch * (window + max_len_extend + 15));
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch;
   if (mean <= 512) return mb <= 160;
   // few units: most of the time is the last share's, which reads all the others of a wide head group
