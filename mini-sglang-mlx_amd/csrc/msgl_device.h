@@ -92,11 +92,85 @@ __device__ __forceinline__ uint32_t pack_16x2(float lo, float hi) {
   }
 }
 
-__device__ __forceinline__ float wave_max_xor(float v, int mask) {
-  return fmaxf(v, __shfl_xor(v, mask, kWave));
-}
-
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
+
+// ---- values of other lanes, without LDS (a shuffle through LDS costs about 100 cycles, these 5 to 10) -------------
+// All lanes of the wave have to be active.
+// DPP control C, 0 where there is no such lane: 0xB1 lane ^ 1, 0x4E lane ^ 2, 0x141 mirror in 8, 0x140 mirror in 16,
+// 0x110 + n the lane n below and 0x120 + n the lane n below with rotation, in 16.
+template <int C>
+__device__ __forceinline__ int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, C, 0xf, 0xf, true);
+}
+template <int C>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, dpp<C>(__builtin_bit_cast(int, v)));
+}
+// For M = 16 and 32: the swap leaves a row's (half's) value and its partner's in the two results.
+template <int M>
+__device__ __forceinline__ float max_across(float v) {  // of lanes l and l ^ M
+  const uint32_t x = __builtin_bit_cast(uint32_t, v);
+  if constexpr (M == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)s[0]), __builtin_bit_cast(float, (uint32_t)s[1]));
+  } else {
+    const auto s = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)s[0]), __builtin_bit_cast(float, (uint32_t)s[1]));
+  }
+}
+template <int M>
+__device__ __forceinline__ float sum_across(float v) {  // of lanes l and l ^ M
+  const uint32_t x = __builtin_bit_cast(uint32_t, v);
+  if constexpr (M == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return __builtin_bit_cast(float, (uint32_t)s[0]) + __builtin_bit_cast(float, (uint32_t)s[1]);
+  } else {
+    const auto s = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return __builtin_bit_cast(float, (uint32_t)s[0]) + __builtin_bit_cast(float, (uint32_t)s[1]);
+  }
+}
+// Sum over a row of 16 lanes, in the order of a butterfly: once the lanes of a group of 4 (of 8) agree, the mirrors
+// in 8 (in 16) are as good as lane ^ 4 (lane ^ 8).
+__device__ __forceinline__ float row_sum16(float v) {
+  v += dpp<0xB1>(v);
+  v += dpp<0x4E>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  return v;
+}
+__device__ __forceinline__ int row_max16(int v) {
+  v = max(v, dpp<0x128>(v));
+  v = max(v, dpp<0x124>(v));
+  v = max(v, dpp<0x122>(v));
+  return max(v, dpp<0x121>(v));
+}
+// The largest and the smallest value of a wave, in a scalar register.
+__device__ __forceinline__ int wave_max(int v) {
+  v = row_max16(v);
+  return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+__device__ __forceinline__ int wave_min(int v) { return ~wave_max(~v); }
+// Wave-wide sum (a scalar) and inclusive prefix sum: a prefix sum inside each row of 16 lanes, the rows' totals
+// through scalar registers.
+__device__ __forceinline__ int row_scan(int v) {
+  v += dpp<0x111>(v);
+  v += dpp<0x112>(v);
+  v += dpp<0x114>(v);
+  v += dpp<0x118>(v);
+  return v;
+}
+__device__ __forceinline__ int wave_sum(int v) {
+  v = row_scan(v);
+  return __builtin_amdgcn_readlane(v, 15) + __builtin_amdgcn_readlane(v, 31) + __builtin_amdgcn_readlane(v, 47) +
+         __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v = row_scan(v);
+  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31), r2 = __builtin_amdgcn_readlane(v, 47);
+  const int row = lane_id() >> 4;
+  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
 
 // Measurement aid: when `dst` is given, thread 0 of workgroup 0 leaves the shader cycles and the
 // 100 MHz wall ticks between its construction and its destruction (every way out of the kernel) in
@@ -119,16 +193,5 @@ struct ClockProbe {
     }
   }
 };
-
-// Inclusive prefix sum over the 64 lanes of a wave.
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const int n = __shfl_up(v, off, kWave);
-    if (lane >= off) v += n;
-  }
-  return v;
-}
 
 }  // namespace msgl

@@ -144,13 +144,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_tile_kernel(PrefillParams p) 
     row_lo[rt] = lo;
     row_hi[rt] = hi;
   }
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    w_lo_max = max(w_lo_max, __shfl_xor(w_lo_max, off, kWave));
-    w_hi_min = min(w_hi_min, __shfl_xor(w_hi_min, off, kWave));
-  }
-  w_lo_max = __builtin_amdgcn_readfirstlane(w_lo_max);
-  w_hi_min = __builtin_amdgcn_readfirstlane(w_hi_min);
+  w_lo_max = wave_max(w_lo_max);
+  w_hi_min = wave_min(w_hi_min);
 
   f32x16_t oacc[DT][RT];
 #pragma unroll
@@ -315,7 +310,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_tile_kernel(PrefillParams p) 
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      const float m = wave_max_xor(mx[rt] * st.mul, 32);
+      const float m = max_across<32>(mx[rt] * st.mul);
       const float m_old = m_run[rt];
       const float m_new = fmaxf(m_old, m);
       const float m_use = (m_new - m_old > kLazy) ? m_new : m_old;
@@ -554,7 +549,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_tile_kernel(PrefillParams p) 
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float l = l_run[rt];
-      l += __shfl_xor(l, 32, kWave);
+      l = sum_across<32>(l);
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
       const int row = row0 + (w * RT + rt) * 32 + c32;
       if (row < rows_total) {
@@ -580,7 +575,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_tile_kernel(PrefillParams p) 
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     float l = l_run[rt];
-    l += __shfl_xor(l, 32, kWave);
+    l = sum_across<32>(l);
     const float inv = (l > 0.f) ? 1.0f / l : 0.f;
     const int lrow = (w * RT + rt) * 32 + c32;
 #pragma unroll
@@ -844,13 +839,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     row_lo = lo;
     row_hi = hi;
   }
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    w_lo_max = max(w_lo_max, __shfl_xor(w_lo_max, off, kWave));
-    w_hi_min = min(w_hi_min, __shfl_xor(w_hi_min, off, kWave));
-  }
-  w_lo_max = __builtin_amdgcn_readfirstlane(w_lo_max);
-  w_hi_min = __builtin_amdgcn_readfirstlane(w_hi_min);
+  w_lo_max = wave_max(w_lo_max);
+  w_hi_min = wave_min(w_hi_min);
 
   f32x16_t oacc[DT];
 #pragma unroll
@@ -1110,7 +1100,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       // reference moves (both halves of a row sit in this wave).  Otherwise the cross-lane
       // exchange, the new state and, where a reference did move, the rescaling of O.
       if (__any(mx * mul > m_run + kLazy)) {
-        const float m = wave_max_xor(mx * mul, 32);
+        const float m = max_across<32>(mx * mul);
         const float m_old = m_run;
         const float m_new = fmaxf(m_old, m);
         const float m_use = (m_new - m_old > kLazy) ? m_new : m_old;
@@ -1278,7 +1268,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
 
   // accumulator i of O^T tile dt is dim 32dt + 8(i/4) + 4h + i%4 of query row c32
   float l = l_run;
-  l += __shfl_xor(l, 32, kWave);
+  l = sum_across<32>(l);
   const float inv = (l > 0.f) ? 1.0f / l : 0.f;
   if (to_partial) {
     const int row = row0 + w * 32 + c32;

@@ -180,13 +180,8 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       row_hi = 0;
     }
   }
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    w_lo_max = max(w_lo_max, __shfl_xor(w_lo_max, off, kWave));
-    w_hi_min = min(w_hi_min, __shfl_xor(w_hi_min, off, kWave));
-  }
-  w_lo_max = __builtin_amdgcn_readfirstlane(w_lo_max);
-  w_hi_min = __builtin_amdgcn_readfirstlane(w_hi_min);
+  w_lo_max = wave_max(w_lo_max);
+  w_hi_min = wave_min(w_hi_min);
 
   f32x16_t oacc[kDT];
 #pragma unroll
@@ -298,7 +293,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     float mx = fmaxf(s[0], s[1]);
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    m_own = wave_max_xor(mx * mul, 32);
+    m_own = max_across<32>(mx * mul);
     *my_max = m_own;
   };
   float m_safe = 0.f, alpha = 1.0f;
@@ -484,7 +479,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   }
   // both halves of the row sum
   float l = l_run;
-  l += __shfl_xor(l, 32, kWave);
+  l = sum_across<32>(l);
   __syncthreads();
   *my_max = l;
   __syncthreads();

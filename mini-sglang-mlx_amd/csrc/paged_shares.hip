@@ -123,15 +123,17 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   }
 
   Columns<D, NCT> c;
+  FirstIds ids{};
+  if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
   start_columns(p, r, kvh, 0, t_end, c);
-  if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16>(p, r, kvh, t_begin, t_end, c);
+  if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c);
 
   // ---- the waves of a kv head meet in LDS ---------------------------------------------------
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
     float l = c.l[ct];
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
+    l = sum_across<16>(l);
+    l = sum_across<32>(l);
     const int col = ct * 16 + t16;
     if (col >= ncols) continue;
     if (g == 0) state[wave][col] = float2{c.m[ct], l};

@@ -188,15 +188,16 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     const int ncols = r.q_len * p.group;
 
     Columns<D, NCT> c_;
+    const FirstIds ids = first_ids(p, r, t_begin, t_end);
     start_columns(p, r, kvh, ct0, t_end, c_);
-    attend_keys<D, NCT, WIDE, F16>(p, r, kvh, t_begin, t_end, c_);
+    attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_);
 
     // ---- this request's share is done: write output or partial -------------------------
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
       float l = c_.l[ct];
-      l += __shfl_xor(l, 16, kWave);
-      l += __shfl_xor(l, 32, kWave);
+      l = sum_across<16>(l);
+      l = sum_across<32>(l);
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
       const int col = (ct0 + ct) * 16 + t16;
       if (col >= ncols) continue;

@@ -87,28 +87,6 @@ __device__ __forceinline__ BlockWork prefill_block_work(const PrefillParams& p) 
   return w;
 }
 
-// Wave-wide sum (the same in every lane) and inclusive prefix sum without LDS: a prefix sum inside each row
-// of 16 lanes, the rows' totals through scalar registers.
-__device__ __forceinline__ int row_scan(int v) {
-  auto shifted = [](int x, auto n) { return __builtin_amdgcn_update_dpp(0, x, 0x110 + decltype(n)::value, 0xf, 0xf, true); };
-  v += shifted(v, std::integral_constant<int, 1>{});  // row_shr
-  v += shifted(v, std::integral_constant<int, 2>{});
-  v += shifted(v, std::integral_constant<int, 4>{});
-  v += shifted(v, std::integral_constant<int, 8>{});
-  return v;
-}
-__device__ __forceinline__ int wave_sum(int v) {
-  v = row_scan(v);
-  return __builtin_amdgcn_readlane(v, 15) + __builtin_amdgcn_readlane(v, 31) + __builtin_amdgcn_readlane(v, 47) +
-         __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_scan(int v) {
-  v = row_scan(v);
-  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31), r2 = __builtin_amdgcn_readlane(v, 47);
-  const int row = lane_id() >> 4;
-  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
-}
-
 // Workgroup id -> query block and its request's geometry, in order of length (see prefill_by_length()).
 // Lengths count in steps of an eighth to a quarter of the longest: within a step a request's blocks stay
 // together, because those that run at the same time then read the same keys (strictly by length, 11 prompts
@@ -149,13 +127,7 @@ __device__ __forceinline__ LengthBlock block_by_length(const PrefillParams& p) {
     return below > first_of ? ((below - first_of - 1) >> p.length_log2_xcds) + 1 : 0;
   };
   const int in_all = in_class(blocks);
-  int longest = kn;
-  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x128, 0xf, 0xf, true));  // row_ror: 8, 4, 2, 1
-  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x124, 0xf, 0xf, true));
-  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x122, 0xf, 0xf, true));
-  longest = max(longest, __builtin_amdgcn_update_dpp(0, longest, 0x121, 0xf, 0xf, true));
-  longest = max(max(__builtin_amdgcn_readlane(longest, 0), __builtin_amdgcn_readlane(longest, 16)),
-                max(__builtin_amdgcn_readlane(longest, 32), __builtin_amdgcn_readlane(longest, 48)));
+  const int longest = wave_max(kn);
   const int shift = max(31 - __builtin_clz(max(longest, 1)) - 2, 6);  // 4 to 8 steps, whole key tiles
   // this XCD's blocks of the request of at least `steps` steps
   auto at_least = [&](int steps) {
@@ -176,7 +148,7 @@ __device__ __forceinline__ LengthBlock block_by_length(const PrefillParams& p) {
   }
   const int longer = at_least(lo + 1), equal = (at_least(lo) - longer) * p.length_heads;
   const int left = seq - wave_sum(longer) * p.length_heads;  // its number among the blocks of exactly `lo` steps
-  const int incl = wave_scan(equal), before = incl - equal;
+  const int incl = wave_inclusive_scan(equal), before = incl - equal;
   const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(left >= before && left < incl)) - 1);
   const int mine = left - __builtin_amdgcn_readlane(before, src);
   const int from_top = __builtin_amdgcn_readlane(longer, src) + mine / p.length_heads;
@@ -233,8 +205,7 @@ __device__ __forceinline__ RaggedUnit ragged_unit(const PrefillParams& p, int u,
   for (int c = wave; c < n_chunks; c += THREADS / kWave) {
     const int i = c * kWave + lane;
     int v = i < p.batch ? count[i] : 0;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) v += __shfl_xor(v, off, kWave);
+    v = wave_sum(v);
     if (lane == 0) chunk_sum[c] = v;
   }
   __syncthreads();

@@ -125,8 +125,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopePa
         xh[e] = bf16_to_f32((uint16_t)((e & 1) ? b >> 16 : b & 0xffffu));
         ss += xl[e] * xl[e] + xh[e] * xh[e];
       }
-#pragma unroll
-      for (int m = 1; m < kGroupLanes; m <<= 1) ss += __shfl_xor(ss, m, kWave);
+      ss = row_sum16(ss);
       const float norm = rsqrtf(ss * (1.0f / D) + p.eps);
       uint16_t ol[E], oh[E];
 #pragma unroll

@@ -126,13 +126,8 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
     c_.lo[ct] = lo;
     c_.hi[ct] = hi;
   }
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) {
-    all_lo = max(all_lo, __shfl_xor(all_lo, off, kWave));
-    all_hi = min(all_hi, __shfl_xor(all_hi, off, kWave));
-  }
-  c_.all_lo = __builtin_amdgcn_readfirstlane(all_lo);
-  c_.all_hi = __builtin_amdgcn_readfirstlane(all_hi);
+  c_.all_lo = __builtin_amdgcn_readfirstlane(row_max16(all_lo));
+  c_.all_hi = __builtin_amdgcn_readfirstlane(~row_max16(~all_hi));
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct) {
     c_.m[ct] = kNegInf;
@@ -144,10 +139,22 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
   }
 }
 
-// Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`.
-template <int D, int NCT, bool WIDE, bool F16>
+// Slot ids of a wave's first two tiles: lane l those of tokens l % 16 and 16 + l % 16 of each.
+struct FirstIds {
+  int a[2], b[2];
+};
+__device__ __forceinline__ FirstIds first_ids(const SplitKvParams& p, const ReqInfo& r, int t_begin, int t_end) {
+  const int32_t* idx = p.kv_indices + r.kv_start;
+  const int at = t_begin + (lane_id() & 15), last = t_end - 1;
+  return FirstIds{{idx[min(at, last)], idx[min(at + 16, last)]}, {idx[min(at + 32, last)], idx[min(at + 48, last)]}};
+}
+
+// Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`; `first`: its first_ids(), asked for before
+// the columns were made.
+// SHORT: ranges of one tile are common, end behind it (in a long walk the test costs more than it saves).
+template <int D, int NCT, bool WIDE, bool F16, bool SHORT>
 __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInfo& r, int kvh, int t_begin,
-                                            int t_end, Columns<D, NCT>& c_) {
+                                            int t_end, const FirstIds& first, Columns<D, NCT>& c_) {
   constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const int lane = lane_id();
@@ -222,8 +229,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
       }
       float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
                        fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
-      mx = wave_max_xor(mx, 16);
-      mx = wave_max_xor(mx, 32);
+      mx = max_across<32>(max_across<16>(mx));
       const float m_new = fmaxf(c_.m[ct], mx);
       const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
       const float alpha = fast_exp2(c_.m[ct] - m_safe);
@@ -274,9 +280,8 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
   // constant and the next tile stays in flight while the current one is computed. ----
   const int n_pairs = (t_end - t_begin + 63) / 64;
   KvTile<D> ta, tb_;
-  int i0a, i0b, i1a, i1b;
-  load_idx(t_begin, i0a, i0b);
-  load_idx(t_begin + 32, i1a, i1b);
+  int i0a = (int)min((uint32_t)first.a[0], p.max_slot), i0b = (int)min((uint32_t)first.a[1], p.max_slot);
+  int i1a = (int)min((uint32_t)first.b[0], p.max_slot), i1b = (int)min((uint32_t)first.b[1], p.max_slot);
   load_tile(ta, i0a, i0b);
   load_idx(t_begin + 64, i0a, i0b);
   for (int pr = 0; pr < n_pairs; ++pr) {
@@ -284,6 +289,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     load_tile(tb_, i1a, i1b);
     load_idx(tok + 96, i1a, i1b);
     compute_tile(ta, tok);
+    if (SHORT && tok + 32 >= t_end) break;
     load_tile(ta, i0a, i0b);
     load_idx(tok + 128, i0a, i0b);
     compute_tile(tb_, tok + 32);
