@@ -815,7 +815,6 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   // (the Q rows themselves are requested in the prologue, after the first tiles' slot ids: the
   // ids gate the first tile moves, and a wait for them would otherwise wait for the Q rows too)
   bf16x8_t qreg[KSTEPS];
-  bool q_valid;
   int64_t q_off;
   int row_lo, row_hi;
   int w_lo_max = -0x7fffffff, w_hi_min = 0x7fffffff;
@@ -824,7 +823,6 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     const bool valid = row < rows_total;
     const int qi = valid ? row / p.group : 0;
     const int hh = valid ? row - qi * p.group : 0;
-    q_valid = valid;
     q_off = ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * D;
     const int qpos = prefix + qi;
     int lo = (p.window > 0) ? qpos - p.window + 1 : 0;
@@ -1120,39 +1118,65 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   };
 
   if (n_tiles > 0) {
-    // ---- prologue: K(0..2) and V(0) leave and are waited for; the ring holds tiles 3, 4 ------
+    // ---- prologue: K(0..2) and V(0) leave, the ring gets tiles 3, 4.  Only the Q rows, the ring and K(0) are
+    // waited for: the first M phase needs no more, its own wait (or, in the group that runs a slot
+    // behind, the one before its first barrier) covers the rest.  The slot ids, which the moves hang on, and
+    // the Q rows are asked for together, hidden from the compiler, whose waits for them
+    // would be waits for everything in flight.
     {
       uint32_t first[3][UPW];
 #pragma unroll
       for (int t = 0; t < 3; ++t)
 #pragma unroll
         for (int i = 0; i < UPW; ++i)
-          first[t][i] = min((uint32_t)idx_base[min(k_lo + t * kBN + unit_key + i, kn - 1)], p.max_slot);
+          asm volatile("global_load_dword %0, %1, %2"
+                       : "=v"(first[t][i])
+                       : "v"((uint32_t)min(k_lo + t * kBN + unit_key + i, kn - 1) * 4u), "s"(idx_base)
+                       : "memory");
+      u32x4_t raw[KSTEPS];
+      const uint16_t* qrow = p.q + q_off + h * 8;  // rows past the request's last: its first, never stored
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        u32x4_t raw = {0u, 0u, 0u, 0u};
-        if (q_valid) raw = ld_global_b128(p.q + q_off + ks * 16 + h * 8);
-        qreg[ks] = as_bf16x8(raw);
-      }
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(raw[ks]) : "v"(qrow), "n"(ks * 32) : "memory");
       ring_fetch(3);
       ring_fetch(4);
+      static_assert(UPW == 2 && KSTEPS == 8, "the slot ids and the Q rows are named one by one");
+      asm volatile("s_waitcnt vmcnt(%6)"
+                   : "+v"(first[0][0]), "+v"(first[0][1]), "+v"(first[1][0]), "+v"(first[1][1]), "+v"(first[2][0]), "+v"(first[2][1])
+                   : "n"(KSTEPS + 2)
+                   : "memory");
+      OffT v_first[UPW];
+#pragma unroll
+      for (int i = 0; i < UPW; ++i) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) first[t][i] = min(first[t][i], p.max_slot);
+        v_first[i] = row_offset(first[0][i], v_row_bytes);
+        v_off[i] = row_offset(first[1][i], v_row_bytes);       // leaves in M phase -1
+        v_off_then[i] = row_offset(first[2][i], v_row_bytes);  // leaves in M phase 0
+      }
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
 #pragma unroll
-        for (int i = 0; i < UPW; ++i) {
-          const OffT vo = row_offset(first[t][i], v_row_bytes);
+        for (int i = 0; i < UPW; ++i)
           lds_direct_b128(lds0 + k_stage_of(t) + (uint32_t)(w * UPW + i) * kKUnit, k_src,
                           row_offset(first[t][i], k_row_bytes));
-          if (t == 0) lds_direct_b128(lds0 + v_stage_of(t) + (uint32_t)(w * UPW + i) * kVUnit, v_src, vo);
-          if (t == 1) v_off[i] = vo;       // leaves in M phase -1
-          if (t == 2) v_off_then[i] = vo;  // leaves in M phase 0
+        if (t == 0) {
+#pragma unroll
+          for (int i = 0; i < UPW; ++i)
+            lds_direct_b128(lds0 + v_stage_of(0) + (uint32_t)(w * UPW + i) * kVUnit, v_src, v_first[i]);
         }
       }
+      asm volatile("s_waitcnt vmcnt(%8)"
+                   : "+v"(raw[0]), "+v"(raw[1]), "+v"(raw[2]), "+v"(raw[3]), "+v"(raw[4]), "+v"(raw[5]), "+v"(raw[6]), "+v"(raw[7])
+                   : "n"(3 * UPW)
+                   : "memory");
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) qreg[ks] = as_bf16x8(raw[ks]);
     }
-    wait_all_vm();
     ring_read(3, ids);
     __syncthreads();
     const bool second = w >= 4;  // the group that runs one slot behind
+    if (second) wait_all_vm();
     if (idle) {
       // the moves, waits and barriers of a computing wave of the same group, nothing else
       if (second) slot_barrier();
