@@ -74,10 +74,17 @@ int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t ma
 // heads: 76 and 61; 64 of 16, 16 / 8 heads: 76 and 63; 16 of 4, 32 / 8: 23.6 both.
 // Beyond 32 columns a workgroup of several kv heads has a wave, and most of a window's time, for each (66 requests
 // of 6 tokens, 64 / 8 heads: 83 us in the tile kernel, 89 in shares).
+// Requests beyond one round of workgroups take whole rounds of a share's time, and a last round that leaves most of
+// the chip idle costs more than the tile kernel's second launch.  Windows of 256 and 1024, 32 / 8 heads, tile or
+// segment kernel against shares, us: rounds 51 % full (261 requests of 4 tokens) 65 and 78, 222 and 280; 55 % (140 of 8)
+// 67 and 52, 148 and 156; 68 % (261 of 8) 126 and 87, 261 and 257; 78 % (400 of 4) 116 and 99, 332 and 308; 91 % (700
+// of 4) 202 and 164, 571 and 513.
 bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv, int64_t keys, int64_t n_kv,
                    int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
   if (head_dim == 256 && batch * n_kv < 12) return false;  // see shares_preferred()
+  const int64_t blocks = batch * (n_kv / plan.heads_wg), cus = msgl::device_cus();
+  if (blocks > cus && 3 * blocks < 2 * cus * ((blocks + cus - 1) / cus)) return false;
   return cols <= 32 || plan.heads_wg == 1;
 }
 // Largest q_len * group that takes the split-K route whatever the launch: at head_dim 128 48 (up

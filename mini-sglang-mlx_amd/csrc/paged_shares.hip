@@ -337,10 +337,12 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
   return plan;
 }
 
-// Fewer visible keys make shorter shares, but never more of them than fit the chip in one round.
+// Fewer visible keys make shorter shares, but never more of them than fit the chip in one round, or than requests
+// where those alone are more: with n = one_round / batch, at least 1, share_plan() makes them of keys / (n batch) keys
+// or more, so keys / share_len is at most n batch.
 SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
   const int64_t one_round = device_cus() * plan.heads_wg / n_kv;
-  plan.max_shares = std::max(plan.max_shares, one_round + batch);
+  plan.max_shares = std::max(plan.max_shares, std::max(one_round, batch) + batch);
   return plan;
 }
 

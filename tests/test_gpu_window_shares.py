@@ -17,6 +17,9 @@ CASES = [
     (32, 8, 128, 12, [2600] * 5 + [12, 13, 700], 513),                  # three column tiles
     (16, 4, 256, 3, [700, 900, 1500, 3, 65], 129),
     (64, 8, 128, 5, [1300, 2200], 100),                                 # three column tiles, few requests
+    (32, 8, 128, 8, [450 + 7 * (i % 50) for i in range(200)], 200),     # more requests than the chip has room for
+    (64, 8, 128, 2, [9 + 5 * (i % 90) for i in range(400)], 128),       # as many, some shorter than the window
+    (16, 2, 256, 2, [420 + i for i in range(430)], 100),
 ]
 
 

@@ -1,0 +1,53 @@
+"""The sizes that the ``*_workspace_bytes`` queries give are enough for the call they are asked for, whatever mask the
+call then has.  Host code only: the pointers are made up, so this runs
+where no GPU is visible, and a call that passes every check ends with MSGL_ERR_LAUNCH for want of a device."""
+import ctypes
+import random
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="made-up pointers: only where nothing can be launched")
+
+ERR_LAUNCH = -11
+FAKE = ctypes.c_void_p(0x1000)
+HEADS = [(16, 8, 128), (32, 8, 128), (64, 8, 128), (8, 1, 128), (128, 16, 128), (16, 2, 256), (24, 4, 256), (32, 2, 256)]
+
+
+def _prefill(batch, heads, ext, kv, window=0, cross=0):
+    from mini_sglang_amd_kernel import _lib
+
+    lib, (n_q, n_kv, d) = _lib.load(), heads
+    total_q, total_kv = batch * ext, kv
+    need = lib.msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, n_q, n_kv, d, ext)
+    return lib.msgl_paged_prefill_attention(FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, need,
+                                            batch, total_q, total_kv, n_q, n_kv, d, 1 << 20, n_kv * d, n_kv * d, 0.1,
+                                            ext, cross, window, 0, None)
+
+
+def _decode(batch, heads, kv):
+    from mini_sglang_amd_kernel import _lib
+
+    lib, (n_q, n_kv, d) = _lib.load(), heads
+    need = lib.msgl_paged_decode_workspace_bytes(batch, kv, n_q, n_kv, d)
+    return lib.msgl_paged_decode_attention(FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, need, batch, kv, n_q, n_kv, d,
+                                           1 << 20, n_kv * d, n_kv * d, 0.1, 32, 0, None)
+
+
+@pytest.mark.parametrize("heads,ext", [((32, 8, 128), 8), ((64, 8, 128), 4), ((32, 8, 128), 4), ((16, 8, 128), 8),
+                                       ((24, 4, 256), 2), ((16, 2, 256), 2)])
+def test_windowed_short_blocks_of_any_batch(heads, ext):
+    """Around and beyond the batch that fills the chip with one share per request."""
+    for batch in (*range(1, 700, 5), 131, 256, 257, 260, 261, 512, 513, 3000):
+        assert _prefill(batch, heads, ext, 4096 * batch, window=1024) == ERR_LAUNCH, batch
+
+
+def test_the_size_asked_for_is_enough():
+    rng = random.Random(7)
+    log = lambda lo, hi: int(lo * (hi / lo) ** rng.random())  # noqa: E731
+    for _ in range(20000):
+        batch, heads, ext = log(1, 2000), rng.choice(HEADS), log(1, 64)
+        kv = batch * (log(1, 20000) + ext) + rng.randrange(64)
+        mask = dict(window=rng.choice((0, 1, 100, 128, 500, 1024, 4096, log(1, 8192))), cross=rng.random() < 0.2)
+        assert _prefill(batch, heads, ext, kv, **mask) == ERR_LAUNCH, (batch, heads, ext, kv, mask)
+        assert _decode(batch, heads, kv) == ERR_LAUNCH, (batch, heads, kv)
