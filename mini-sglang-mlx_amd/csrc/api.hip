@@ -397,19 +397,19 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   const int64_t cols = group * max_len_extend;
   const int64_t keys = visible_keys(batch, total_kv, sliding_window_size, max_len_extend, is_cross_attention != 0);
   const msgl::SharePlan plan = shares_for(batch, keys, keys < total_kv ? keys / batch : 0, num_kv_heads, head_dim, cols);
-  const bool window_share = window_shares(plan, batch, total_kv, keys, num_kv_heads, head_dim, cols);
+  // without room for their partials a launch goes the way it goes without shares
+  const bool share_room = plan.share_len > 0 && workspace && aligned16(workspace) &&
+                          workspace_bytes >= msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols);
+  const bool window_share = share_room && window_shares(plan, batch, total_kv, keys, num_kv_heads, head_dim, cols);
   const bool direct = window_share ||
                       (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
                        !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
                                              sliding_window_size));
   if (direct) {
     const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, cols);
-    const bool shares = window_share || msgl::shares_preferred(plan, batch, keys, num_kv_heads, head_dim, cols);
-    const size_t need = shares
-                            ? msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols)
-                            : msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim,
-                                                            max_len_extend, n_seg);
-    if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;
+    const bool shares = window_share || (share_room && msgl::shares_preferred(plan, batch, keys, num_kv_heads, head_dim, cols));
+    const size_t need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend, n_seg);
+    if (!shares && (!workspace || workspace_bytes < need || !aligned16(workspace))) return MSGL_ERR_WORKSPACE;
     msgl::SplitKvArgs a{};
     a.q = q;
     a.k_cache = k_cache;

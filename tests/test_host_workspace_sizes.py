@@ -1,5 +1,5 @@
 """The sizes that the ``*_workspace_bytes`` queries give are enough for the call they are asked for, whatever mask the
-call then has.  Host code only: the pointers are made up, so this runs
+call then has, and launches that can do without a workspace do.  Host code only: the pointers are made up, so this runs
 where no GPU is visible, and a call that passes every check ends with MSGL_ERR_LAUNCH for want of a device."""
 import ctypes
 import random
@@ -9,18 +9,18 @@ import torch
 
 pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="made-up pointers: only where nothing can be launched")
 
-ERR_LAUNCH = -11
+ERR_WORKSPACE, ERR_LAUNCH = -8, -11
 FAKE = ctypes.c_void_p(0x1000)
 HEADS = [(16, 8, 128), (32, 8, 128), (64, 8, 128), (8, 1, 128), (128, 16, 128), (16, 2, 256), (24, 4, 256), (32, 2, 256)]
 
 
-def _prefill(batch, heads, ext, kv, window=0, cross=0):
+def _prefill(batch, heads, ext, kv, window=0, cross=0, workspace=True):
     from mini_sglang_amd_kernel import _lib
 
     lib, (n_q, n_kv, d) = _lib.load(), heads
     total_q, total_kv = batch * ext, kv
-    need = lib.msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, n_q, n_kv, d, ext)
-    return lib.msgl_paged_prefill_attention(FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, need,
+    need = lib.msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, n_q, n_kv, d, ext) if workspace else 0
+    return lib.msgl_paged_prefill_attention(FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE if need else None, need,
                                             batch, total_q, total_kv, n_q, n_kv, d, 1 << 20, n_kv * d, n_kv * d, 0.1,
                                             ext, cross, window, 0, None)
 
@@ -51,3 +51,14 @@ def test_the_size_asked_for_is_enough():
         mask = dict(window=rng.choice((0, 1, 100, 128, 500, 1024, 4096, log(1, 8192))), cross=rng.random() < 0.2)
         assert _prefill(batch, heads, ext, kv, **mask) == ERR_LAUNCH, (batch, heads, ext, kv, mask)
         assert _decode(batch, heads, kv) == ERR_LAUNCH, (batch, heads, kv)
+
+
+def test_launches_that_can_do_without_a_workspace_do():
+    """17-48 columns under a window that most requests exceed, and longer query blocks, fall back to one pass of the tile
+    kernel; short blocks of the split-K route cannot."""
+    for batch in (1, 4, 32, 100, 200, 600):
+        for heads, ext in (((32, 8, 128), 8), ((32, 8, 128), 5), ((64, 8, 128), 3), ((16, 8, 128), 24)):
+            assert _prefill(batch, heads, ext, 4096 * batch, window=1024, workspace=False) == ERR_LAUNCH, (batch, heads, ext)
+        assert _prefill(batch, (32, 8, 128), 100, 4096 * batch, workspace=False) == ERR_LAUNCH
+        assert _prefill(batch, (32, 8, 128), 4, 4096 * batch, window=1024, workspace=False) == ERR_WORKSPACE
+        assert _prefill(batch, (32, 8, 128), 8, 4096 * batch, workspace=False) == ERR_WORKSPACE
