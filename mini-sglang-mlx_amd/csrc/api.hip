@@ -3,8 +3,8 @@
 // paged_prefill_attention.cpp:31-76, store_kv_cache.cpp:22-63) as far as raw pointers
 // and sizes can express them; rank and dtype-equality checks live in the Python shim.
 #include <algorithm>
-#include <atomic>
 
+#include "launch_number.h"
 #include "msgl_internal.h"
 #include "prefill_params.h"
 
@@ -19,8 +19,6 @@ thread_local int64_t t_gangs = 0;  // negative: never use gang ranges
 thread_local long long* t_clock_probe = nullptr;
 constexpr int kTuneKnobs = 11;
 thread_local int64_t t_last_set[kTuneKnobs] = {};  // what this thread last passed to msgl_set_tuning
-// launch numbers for the count words of gang ranges (see prefill_gangs()); never 0
-std::atomic<unsigned long long> g_gang_nonce{1};
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -491,8 +489,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
         workspace_bytes >= msgl::prefill_gang_workspace_bytes(batch, num_kv_heads, group, max_len_extend, gangs)) {
       a.gangs = gangs;
       a.workspace = workspace;
-      a.gang_nonce = g_gang_nonce.fetch_add(1, std::memory_order_relaxed) & ((1ull << 47) - 1);
-      if (a.gang_nonce == 0) a.gang_nonce = g_gang_nonce.fetch_add(1, std::memory_order_relaxed);
+      a.gang_nonce = msgl::next_launch_number();
     }
   }
   return head_dim == 256 ? msgl::launch_prefill_tile256(a, s) : msgl::launch_prefill_tile(a, s);

@@ -100,8 +100,8 @@ struct PrefillArgs {
   // 0 = off; `workspace` then holds prefill_ragged_workspace_bytes()
   int32_t ragged_tiles;
   // gang ranges instead (several query blocks per (request, kv head), head_dim 128 only): gangs
-  // per XCD, 0 = off; `workspace` then holds prefill_gang_workspace_bytes(); `gang_nonce` is a
-  // number no earlier launch on this workspace has used
+  // per XCD, 0 = off; `workspace` then holds prefill_gang_workspace_bytes(); `gang_nonce` is the
+  // launch's number (launch_number.h)
   int32_t gangs;
   unsigned long long gang_nonce;
   int32_t by_length;  // query blocks may go in order of length (the fused kernel does not know that order)

@@ -1236,8 +1236,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       __hip_atomic_store(mine + 8 * 32 * kWave + w * kWave + lane, pair_bits(m_run, l_run), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
     }
-    // count word = launch number << 16 | parts done; a word from another launch counts as zero.
-    // It is read while the slot's stores drain (the update below then usually succeeds at once).
+    // count word = launch number << 16 | parts done; any other word counts as zero
+    // (launch_number.h).  It is read while the slot's stores drain (the update below then usually succeeds at once).
     unsigned long long* cnt = p.gang_counts + ((int64_t)(piece * 8 + gang_xcd) * p.n_qblk + gang_member);
     unsigned long long seen = 0;
     if (tid == 0) seen = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

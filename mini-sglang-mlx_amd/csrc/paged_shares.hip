@@ -17,12 +17,12 @@
 //   its log-sum-exp go to the workspace, the workgroup counts itself in the request's count word, and
 //   the one that counts last reads the others and writes the result: nobody waits for anybody.
 //   Partials and counts travel at agent scope (they cross XCDs).  A count word is
-//   launch number << 16 | shares done; a word of any other launch counts as zero, so the workspace
-//   needs no clearing, and the last share puts the word back to zero, so a captured launch replays.
+//   launch number << 16 | shares done; any other word counts as zero, so the workspace
+//   needs no clearing (launch_number.h: why no data is taken for one), and the last share puts the word back to zero, so a captured launch replays.
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 
+#include "launch_number.h"
 #include "splitkv_tiles.h"
 
 namespace msgl {
@@ -294,7 +294,6 @@ int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
 }
 
 thread_local int64_t t_force = 0;  // benchmarking switch, see shares_force()
-std::atomic<unsigned long long> g_nonce{1};
 
 }  // namespace
 
@@ -383,8 +382,7 @@ int launch_shares(const SplitKvArgs& a, const SharePlan& plan, hipStream_t strea
   ws += ((size_t)(a.batch * head_groups) * sizeof(unsigned long long) + 255) / 256 * 256;
   sp.s.part_o = reinterpret_cast<float*>(ws);
   sp.s.part_lse = sp.s.part_o + (size_t)plan.max_shares * (size_t)(a.n_kv * cols * a.head_dim);
-  sp.nonce = g_nonce.fetch_add(1, std::memory_order_relaxed) & ((1ull << 47) - 1);
-  if (sp.nonce == 0) sp.nonce = g_nonce.fetch_add(1, std::memory_order_relaxed);
+  sp.nonce = next_launch_number();
   sp.share_len = plan.share_len;
   sp.share_waves = plan.share_waves;
   sp.heads_wg = plan.heads_wg;
