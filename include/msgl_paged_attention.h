@@ -129,13 +129,15 @@ MSGL_API int msgl_paged_decode_attention(const void* q, const void* k_cache, con
  * the library's code object (every GPU the library runs on holds it until the process ends).
  * The call makes no hipMalloc / hipFree and no allocating library call; the first call on a
  * device looks the array's address up (hipGetSymbolAddress) and keeps it, so make that first
- * call outside a capture.  Sizes whose split-K partials need more than the array
- * ((segments + batch) * num_q_heads * (head_dim + 1) floats; 3.2 MB at batch 64, 32 / 8 heads
- * of 128) return MSGL_ERR_SCRATCH_LIMIT and launch nothing.  Every call on one GPU uses the
+ * call outside a capture.  Sizes that need more than the array, by
+ * msgl_paged_decode_workspace_bytes, return MSGL_ERR_SCRATCH_LIMIT and launch nothing.  That is
+ * (segments or shares + batch) * num_q_heads * (head_dim + 1) floats and some words (3.2 MB at
+ * batch 64, 32 / 8 heads of 128); shares can need 1.38 times what segments do, which is why the
+ * array is 12 MiB: all sizes whose segments take up to 8 MiB run.  Every call on one GPU uses the
  * same array, whatever the stream: calls that overlap in time on one GPU race.  Nothing in the
- * array has to start at zero (the attention kernel writes every entry the merge reads).
+ * array has to start at zero.
  */
-#define MSGL_DECODE_SCRATCH_BYTES (8 * 1024 * 1024)
+#define MSGL_DECODE_SCRATCH_BYTES (12 * 1024 * 1024)
 MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_cache,
                                 const void* v_cache,
                                 const int32_t* kv_indptr, const int32_t* kv_indices,

@@ -122,7 +122,7 @@ const char* msgl_strerror(int code) {
     case MSGL_ERR_HEAD_DIM_MULT4: return "head_dim must be a multiple of 4";
     case MSGL_ERR_GDN_DIMS: return "this specialized kernel requires dk=dv=128";
     case MSGL_ERR_SCRATCH_LIMIT:
-      return "sizes need more split-K scratch than the library's built-in 8 MiB; use the entry "
+      return "sizes need more split-K scratch than the library's built-in 12 MiB; use the entry "
              "point that takes a workspace";
     default: return "unknown error code";
   }

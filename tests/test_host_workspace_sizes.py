@@ -2,7 +2,10 @@
 call then has, and launches that can do without a workspace do.  Host code only: the pointers are made up, so this runs
 where no GPU is visible, and a call that passes every check ends with MSGL_ERR_LAUNCH for want of a device."""
 import ctypes
+import math
+import os
 import random
+import re
 
 import pytest
 import torch
@@ -62,3 +65,28 @@ def test_launches_that_can_do_without_a_workspace_do():
         assert _prefill(batch, (32, 8, 128), 100, 4096 * batch, workspace=False) == ERR_LAUNCH
         assert _prefill(batch, (32, 8, 128), 4, 4096 * batch, window=1024, workspace=False) == ERR_WORKSPACE
         assert _prefill(batch, (32, 8, 128), 8, 4096 * batch, workspace=False) == ERR_WORKSPACE
+
+
+def test_the_builtin_scratch_holds_every_size_whose_segments_fit_8_mib():
+    """Whatever route the call takes: it is refused for its size only where segments would need more."""
+    from mini_sglang_amd_kernel import _lib
+
+    lib, rng = _lib.load(), random.Random(11)
+    header = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "msgl_paged_attention.h")
+    scratch = math.prod(map(int, re.search(r"#define MSGL_DECODE_SCRATCH_BYTES \(([\d* ]+)\)", open(header).read()).group(1).split("*")))
+    log = lambda lo, hi: int(lo * (hi / lo) ** rng.random())  # noqa: E731
+    sizes = [(136, 28074, 64, 8, 128), (70, 11110, 128, 16, 128)]
+    while len(sizes) < 40000:
+        n_kv, batch = rng.choice((1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 64, 128)), log(1, 2000)
+        sizes.append((batch, batch * log(1, 4000) + rng.randrange(100), n_kv * rng.randint(1, 16), n_kv, rng.choice((128, 256))))
+    beyond = 0
+    for size in sizes:
+        need = lib.msgl_paged_decode_workspace_bytes(*size)
+        if need <= 8 << 20:
+            continue
+        _lib.set_tuning(_lib.TUNE_SHARES, -1)
+        segments = lib.msgl_paged_decode_workspace_bytes(*size)
+        _lib.set_tuning(_lib.TUNE_SHARES, 0)
+        beyond += segments <= 8 << 20
+        assert segments > 8 << 20 or need <= scratch, (size, segments, need)
+    assert beyond > 2

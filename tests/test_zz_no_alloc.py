@@ -64,6 +64,18 @@ def test_noalloc_decode_other_head_shapes(gpu):
         _both(lib, wl, gpu, f"heads {n_q}/{n_kv} head_dim {d}")
 
 
+def test_noalloc_decode_where_shares_need_more_than_segments(gpu):
+    """Many short requests: the partials of shares take more than 8 MiB, those of segments would not."""
+    from mini_sglang_amd_kernel import _lib
+
+    lib = _lib.load()
+    for batch, keys, n_q, n_kv in ((136, 28074, 64, 8), (70, 11110, 128, 16)):
+        lens = [keys // batch + (i < keys % batch) for i in range(batch)]
+        assert lib.msgl_paged_decode_workspace_bytes(batch, keys, n_q, n_kv, 128) > 8 << 20
+        wl = build_workload("t", "decode", seed=31, n_q=n_q, n_kv=n_kv, kv_lens=lens, pool_factor=1.0)
+        _both(lib, wl, gpu, f"shares, {n_q}/{n_kv} heads")
+
+
 def test_noalloc_decode_refuses_sizes_beyond_its_scratch(gpu):
     from mini_sglang_amd_kernel import _lib
 
