@@ -38,6 +38,13 @@
 // two split operands the six products above 2^-24 of the result).  The inverse is built from fp32
 // matrix instructions.  Decay ratios are products of the decays (no logarithms: a decay may be 0).
 //
+// Infinities and NaN: the products above run over a whole chunk, zeros of a triangle included, and would carry
+// 0 * infinity from a token to the ones before it and from a dim to the others.  So every wave keeps the largest
+// magnitude of its U (not finite if v, k, a gate or the state is not, or if T overflowed) and of P on the diagonal
+// (not finite if a query is not), and if that is not finite in the end, goes through the request again from the
+// state it started with, token by token: what the token kernel gives.  Keeping it costs 0.7 % (286 -> 288 us for the
+// requests above); the second pass takes 0.6 us a token (one request of 4005: 0.29 -> 2.8 ms).
+//
 // Layouts (v_mfma 16x16x32: lane l holds row / column l % 16 and the 8 contraction values of lane group
 // g = l / 16; results: column l % 16, rows 4 g + i).  A result used as an operand of the next product
 // keeps its registers: the contraction order is permuted to match instead, i.e. lane group g
@@ -73,6 +80,7 @@ struct ChunkLds {
   float g[kChunk], pre[kChunk], suf[kChunk], quad_pre[kChunk], block[4], quad[16];
   float total[3];                 // G_64, chunks j .. j + 2 (last: the arrays above are read 16 bytes at a time)
   int request;
+  alignas(16) float p_largest[4 * 64];  // per lane of the chunk waves: largest() of P's diagonal blocks, all chunks
 };
 
 // Piece `c` of 16 bytes of row `row` lies at this place.  LDS serves 8 lanes of a 16-byte read and 16 of an
@@ -199,12 +207,110 @@ __device__ __forceinline__ void triangle_second(const Triangle& t, const Split& 
 
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 
+// The larger of m and the magnitudes of x, NaN if there is one (two instructions).
+__device__ __forceinline__ float largest(f32x4_t x, float m) {
+  auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
+  m = larger(larger(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])), m);
+  return larger(larger(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])), m);
+}
+// Finite, and so is the nearest bf16.
+__device__ __forceinline__ bool splits(float largest) { return largest < 0x1p127f; }
+
+// A parameter of the launch (they are the kernel's first argument), read where it stands: what is only needed behind
+// the chunks would push others out of the scalar registers meanwhile (2 % of a launch's time).
+template <typename T>
+__device__ __forceinline__ T parameter(T GdnParams::* member) {
+  auto args = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return ((const GdnParams*)args)->*member;
+}
+// Address of a lane's part of state row `row + lane % 16`: its four pieces of 8 dims lie 32 apart.
+__device__ __forceinline__ float* state_row(int slot, int hv, int row) {
+  uint32_t lane = lane_id();
+  pin(lane);
+  return parameter(&GdnParams::state) + (int64_t)slot * parameter(&GdnParams::state_stride0) +
+         ((int64_t)hv * kDV + row + (lane & 15)) * kDK + 8 * (lane >> 4);
+}
+
+// A request token after token, as in gdn_state.hip, for a wave's 16 rows from `row` on.
+__device__ __forceinline__ void token_by_token(int start, int end, int slot, int hv, int row) {
+  GdnParams p;
+  p.y = parameter(&GdnParams::y);
+  p.q = parameter(&GdnParams::q);
+  p.k = parameter(&GdnParams::k);
+  p.v = parameter(&GdnParams::v);
+  p.g = parameter(&GdnParams::g);
+  p.beta = parameter(&GdnParams::beta);
+  p.q_stride0 = parameter(&GdnParams::q_stride0);
+  p.k_stride0 = parameter(&GdnParams::k_stride0);
+  p.v_stride0 = parameter(&GdnParams::v_stride0);
+  p.hv = parameter(&GdnParams::hv);
+  p.hv_per_hk = parameter(&GdnParams::hv_per_hk);
+  uint32_t lane = lane_id();
+  pin(lane);
+  const int g = lane >> 4, hk = hv / p.hv_per_hk;
+  float* const srow = state_row(slot, hv, row);
+  row += lane & 15;
+  f32x4_t s[8];  // s[2 c + h][i]: dim 32 c + 8 g + 4 h + i
+#pragma unroll
+  for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
+  struct TokenIn {
+    u32x4_t k[4], q[4];
+    uint32_t g, beta, v;
+  };
+  auto load = [&](int64_t t, TokenIn& in) {
+    const uint16_t* k = p.k + t * p.k_stride0 + hk * kDK + 8 * g;
+    const uint16_t* q = p.q + t * p.q_stride0 + hk * kDK + 8 * g;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      in.k[c] = ld_global_b128(k + 32 * c);
+      in.q[c] = ld_global_b128(q + 32 * c);
+    }
+    in.g = p.g[t * p.hv + hv];
+    in.beta = p.beta[t * p.hv + hv];
+    in.v = p.v[t * p.v_stride0 + hv * kDV + row];
+  };
+  auto four = [](u32x4_t raw, int h) {
+    return f32x4_t{bf16_bits_to_f32(raw[2 * h] & 0xffffu), bf16_bits_to_f32(raw[2 * h] >> 16),
+                   bf16_bits_to_f32(raw[2 * h + 1] & 0xffffu), bf16_bits_to_f32(raw[2 * h + 1] >> 16)};
+  };
+  TokenIn next;
+  load(start, next);
+  for (int t = start; t < end; ++t) {
+    const TokenIn in = next;
+    load(min(t + 1, end - 1), next);
+    const float decay = bf16_bits_to_f32(in.g);
+    float dot = 0.f, y = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const f32x4_t k = four(in.k[c >> 1], c & 1);
+      s[c] *= decay;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(s[c][i], k[i], dot);
+    }
+    const float delta = (bf16_bits_to_f32(in.v) - sum_across<32>(sum_across<16>(dot))) * bf16_bits_to_f32(in.beta);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const f32x4_t k = four(in.k[c >> 1], c & 1), q = four(in.q[c >> 1], c & 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[c][i] = __builtin_fmaf(k[i], delta, s[c][i]);
+        y = __builtin_fmaf(s[c][i], q[i], y);
+      }
+    }
+    y = sum_across<32>(sum_across<16>(y));
+    if (g == 0) p.y[((int64_t)t * p.hv + hv) * kDV + row] = __builtin_bit_cast(uint16_t, (__bf16)y);
+  }
+#pragma unroll
+  for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
+}
+
 __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int slot, int hv,
                                             int row, int column) {
   const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
   const int n_chunks = (end - start + kChunk - 1) / kChunk;
-  float* srow = p.state + (int64_t)slot * p.state_stride0 + ((int64_t)hv * kDV + row + x16) * kDK + 8 * g;
   f32x4_t s[8];  // s[2 c + h][i]: dim 32 c + 8 g + 4 h + i of row `row + x16`
+  float* srow = state_row(slot, hv, row);
 #pragma unroll
   for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
 
@@ -238,6 +344,7 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
   Rows rows[2];
   load_rows(0, 0, rows[0]);
   Split sp = split(pick, s[0], s[1]);
+  float most = 0.f;  // largest() of every U
   for (int j = 0, tri = 0; j < n_chunks; ++j, tri = tri == 2 ? 0 : tri + 1) {
     const int par = j & 1;
     // ---- slot 1 ----------------------------------------------------------------------------
@@ -319,6 +426,8 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
     const Split ut1 = split(pick, u[2] * tail[2], u[3] * tail[3]);
 #pragma unroll
     for (int c = 0; c < 8; ++c) s[c] *= total;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) most = largest(u[m], most);
     fence();
     triangle_second<true>(tp, us1, z);
     auto steps = [&](int n, const Split& b) {
@@ -356,6 +465,13 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
     sp = split(pick, s[0], s[1]);
     slot_barrier();
   }
+  most = largest(*reinterpret_cast<const f32x4_t*>(&lds.p_largest[4 * lane]), most);
+  if (__builtin_expect(!__all(splits(most)), 0)) {
+    wait_all_vm();  // the stores of Y: the same places are written again
+    token_by_token(start, end, slot, hv, row);
+    return;
+  }
+  srow = state_row(slot, hv, row);
 #pragma unroll
   for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
 }
@@ -496,6 +612,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
   auto block_row = [&](int n) { return n == 0 ? w : n == 1 ? (w == 0 ? 3 : w) : (w == 2 ? 2 : 3); };
   auto block_col = [&](int n) { return n == 0 ? w : n == 1 ? (w == 3 ? 1 : 0) : (w == 1 ? 2 : 1); };
   f32x4_t pp[3];  // the ratios of P of these blocks, then P
+  float most = 0.f;  // largest() of P's diagonal block, every chunk
   f32x4_t inv;    // the inverse of the diagonal block: row x16, columns 4 g ..
   auto products = [&](int par, int tri) {
     struct Block {
@@ -582,6 +699,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
                            operand(&lds.q[par][16 * block_row(n) + x16][8 * piece(x16, 4 * d + g)]), qk);
       pp[n] *= qk;
     }
+    most = largest(pp[0], most);
   };
   // Blocks of T below the diagonal, two waves with the first column: (1, 0) and (2, 0); (2, 1) and (3, 1); (3, 2);
   // (3, 0).  Everything a chain needs from LDS is asked for before it starts.
@@ -669,6 +787,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
       inverse();
     }
     if (w == 2 && two) decays(next + kChunk, tri);
+    if (!more) lds.p_largest[64 * w + lane] = most;
     slot_barrier();
   }
 }
@@ -715,7 +834,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_kernel(GdnParams p, int ranked)
   // the blocks of T and P above the diagonal that are read are never written: zero from here on
   for (int i = threadIdx.x; i < (int)(sizeof(lds.t) + sizeof(lds.p)) / 16; i += 512)
     reinterpret_cast<u32x4_t*>(&lds.t[0][0][0])[i] = u32x4_t{0u, 0u, 0u, 0u};
-  if (wave < 4) state_waves(p, lds, start, end, p.slot_ids[b], hv, row + 16 * wave, 16 * wave);
+  if (wave < 4) state_waves(p, lds, start, end, __builtin_amdgcn_readfirstlane(p.slot_ids[b]), hv, row + 16 * wave, 16 * wave);
   else chunk_waves(p, lds, start, end, hv, row, wave - 4);
 }
 
