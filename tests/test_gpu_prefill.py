@@ -82,6 +82,21 @@ def test_tile_route_masks(gpu, tile_variant, is_cross, window):
     _check(wl, gpu, f"tile route variant={tile_variant} cross={is_cross} W={window}")
 
 
+@pytest.mark.parametrize("is_cross,window", MASKS)
+def test_tile_route_row_maxima_that_grow(gpu, tile_variant, is_cross, window):
+    """Keys that get longer along every request: the row maximum grows by more than the margin in tile after tile, under
+    a window with part of a row's lanes masked, so the two halves of a row exchange it all the time.  A weight is cut to
+    bf16 (2^-7 of it) and the result rounded (2^-9), of values up to 4.5: 4.4e-2."""
+    wl = build_workload("t", "prefill", seed=205, n_q=8, n_kv=2, kv_lens=[70, 300, 64 + 130, 1500], extend_lens=[70, 100, 130, 65],
+                        pool_factor=1.3, is_cross_attention=is_cross, sliding_window_size=window)
+    ip = wl.kv_indptr.tolist()
+    for b in range(4):
+        ids = wl.kv_indices[ip[b]:ip[b + 1]].long()
+        wl.k_cache[ids] = (wl.k_cache[ids].float() * (1 + torch.arange(ids.numel()) / 40)[:, None, None]).bfloat16()
+    print(f"tile route, growing maxima, variant={tile_variant} cross={is_cross} W={window}", flush=True)
+    assert_close_bf16(run_gpu(wl, gpu)[0], run_oracle(wl)[0], "growing maxima", max_tol=4.5e-2, mean_tol=4e-3)
+
+
 @pytest.mark.parametrize("n_q,n_kv", [(8, 8), (32, 8), (12, 4), (16, 1)])
 def test_tile_route_group_sizes(gpu, tile_variant, n_q, n_kv):
     wl = build_workload("t", "prefill", seed=210 + n_q, n_q=n_q, n_kv=n_kv,
