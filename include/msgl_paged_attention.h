@@ -101,7 +101,8 @@ MSGL_API size_t msgl_paged_decode_workspace_bytes(int64_t batch, int64_t total_k
  *   kv_indptr (batch+1)   kv_indices (total_kv)   num_kv_splits (batch)
  * Request b attends to all kv_indptr[b+1]-kv_indptr[b] tokens listed for it.
  * The concatenated KV stream of the batch is cut into equal segments, one resident round of
- * workgroups on MI355X; partial results are merged by log-sum-exp.  The result does not
+ * workgroups on MI355X, or (small launches) every request's keys into equal shares; partial
+ * results are merged by log-sum-exp.  The result does not
  * depend on the split, so `num_kv_splits` / `max_kv_splits` (the reference's
  * split hints, backend.py:304-307) are accepted and validated but do not steer
  * the cut.  A request with no tokens gets zeros (the reference leaves its rows
@@ -157,10 +158,11 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
  * slots and count words of gang ranges, with which one workgroup per compute unit stays for the
  * launch and the (request, kv head) units are shared out by length; 0 otherwise.  The split-K
  * route needs its workspace (MSGL_ERR_WORKSPACE without it); the tile kernels fall back to one
- * pass over the keys per query block when the workspace is missing or too small.  total_kv must
+ * pass over the keys per query block when the workspace is missing or too small, and a launch that
+ * would go in shares of its requests' keys goes the way it goes without them.  total_kv must
  * be at least kv_indptr[batch], here and in msgl_paged_prefill_attention: key shares, grids and
  * this size are derived from it (a smaller value leaves requests' rows unwritten).  Nothing in
- * the workspace has to be initialised.
+ * the workspace has to be initialised, whatever it held before.
  */
 MSGL_API size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv,
                                           int64_t num_q_heads, int64_t num_kv_heads,

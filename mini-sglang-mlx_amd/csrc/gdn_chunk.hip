@@ -12,7 +12,7 @@
 // the state, so the serial part of a chunk is five products.
 //
 // Token after token a request costs 0.33 us per token whatever the chip has free; here a chunk of 64 costs
-// 4.4 us.  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32: 1353 -> 282 us; one of 1024: 298 -> 77.
+// 4.4 us.  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32: 1353 -> 287 us; one of 1024: 298 -> 78.
 //
 // Work: one workgroup per (request, value head, half of its 128 rows).  Waves 0-3 ("state" waves, 16
 // rows each, S^T in 32 accumulator registers) run the serial part of chunk j; waves 4-7 ("chunk" waves,
@@ -23,9 +23,10 @@
 //      2     R = beta (V - G X), U = T R           A, the decay ratios of P, the diagonal blocks of T of chunk j + 1
 //      3     Y = G Z + P U, S = G_64 S + K^T U     P, the blocks of T below the diagonal, V of chunk j + 1;
 //                                                  decay products of chunk j + 2
-// What bounds it: a chunk takes 10.7 K cycles (slots of 3.2, 2.9 and 4.6 K), in which a SIMD has 5 K cycles of
+// What bounds it: a chunk takes 10.6 K cycles (slots of 3.3, 2.9 and 4.4 K), in which a SIMD has 5.3 K cycles of
 // matrix instructions and as many of vector instructions in two chains that wait for their own results, and a
-// wave that has the SIMD for itself still pays about 5 cycles per instruction of any kind.  Hence: fp32 values
+// wave that has the SIMD for itself still pays about 5 cycles per instruction of any kind.  The last wave of a slot is
+// a chunk wave in all three, 0.6 K, 0.4 K and 0.5 K cycles behind the slowest state wave.  Hence: fp32 values
 // are split by the matrix pipe (see Split: 16 instructions instead of 44), Z and Y are made transposed (4 stores
 // of 8 bytes a chunk instead of 16 of 2), V comes by transposing LDS reads, and the chunk waves share the blocks
 // out evenly (12.5 -> 10.7 K).  T and P of all chunks in a launch of their own, in parallel, measured the same

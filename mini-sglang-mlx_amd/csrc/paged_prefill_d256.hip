@@ -21,8 +21,9 @@
 //   slot ids   = fetched a step ahead by loads issued before the step's moves and hidden from
 //                the compiler's wait bookkeeping, so that the wait at the end of the step covers them and
 //                nothing else waits.
-// What bounds it: 32 keys take 1750 cycles, of which the matrix pipe is busy 1024, at the 1.64 GHz that the
-// power leaves (1.13 PFLOP/s; the kernel for head_dim 128 reaches 1.23).  Whole rows to a wave, for comparison:
+// What bounds it: 32 keys take 1690-1770 cycles, of which the matrix pipe is busy 1024, at the 1.9 GHz that the
+// power leaves (1.04 PFLOP/s on the requests below; 1.16 on one long request, where the kernel for head_dim 128
+// reaches 1.23).  Whole rows to a wave, for comparison:
 // one wave of 32 rows per SIMD issued 400 instructions per 32 keys at 5 cycles each (2380 cycles), two of 16 rows
 // read K and V twice as often from LDS (2050).  4 requests of 512-1972 tokens on prefixes up to 8 K, 24 / 4
 // heads: 837 us with the first, 775 with the second, 717 so.
