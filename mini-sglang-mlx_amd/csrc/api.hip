@@ -215,6 +215,7 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
                             int64_t head_dim, int64_t num_slots, int64_t k_cache_stride0,
                             int64_t v_cache_stride0, float sm_scale, int32_t max_kv_splits,
                             int32_t dtype, void* stream) {
+  const msgl::NewTokens tokens{};  // every row is in the pool
   if (batch < 0 || total_kv < 0 || num_slots < 0) return MSGL_ERR_SHAPE;
   if (batch == 0) return MSGL_OK;
   int rc = check_common(q, k_cache, v_cache, out, num_q_heads, num_kv_heads, head_dim,
@@ -261,7 +262,7 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
   a.window = 0;
   a.n_seg = n_seg;
   a.min_seg = min_segment(head_dim);
-  if (shares) return msgl::launch_shares(a, plan, static_cast<hipStream_t>(stream));
+  if (shares) return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
   return msgl::launch_splitkv(a, static_cast<hipStream_t>(stream));
 }
 
@@ -290,6 +291,77 @@ int msgl_paged_decode_attention_noalloc(const void* q, const void* k_cache, cons
   return decode_attention(q, k_cache, v_cache, kv_indptr, kv_indices, num_kv_splits, out, nullptr,
                           0, true, batch, total_kv, num_q_heads, num_kv_heads, head_dim, num_slots,
                           k_cache_stride0, v_cache_stride0, sm_scale, max_kv_splits, dtype, stream);
+}
+
+size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads, int64_t num_kv_heads,
+                                        int64_t head_dim) {
+  if (batch <= 0 || total_kv < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      num_q_heads / num_kv_heads > 16 || (head_dim != 128 && head_dim != 256))
+    return 0;
+  const int64_t group = num_q_heads / num_kv_heads;
+  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  if (!msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) return 0;
+  return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
+}
+
+int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stride0, int64_t k_stride0, int64_t v_stride0,
+                     const void* q_weight, const void* k_weight, const int32_t* positions, const int32_t* out_loc,
+                     void* k_cache, void* v_cache, const int32_t* kv_indptr, const int32_t* kv_indices, void* out,
+                     void* workspace, size_t workspace_bytes, int64_t batch, int64_t total_kv, int64_t num_q_heads,
+                     int64_t num_kv_heads, int64_t head_dim, int64_t num_slots, int64_t k_cache_stride0,
+                     int64_t v_cache_stride0, float sm_scale, float rms_norm_eps, float rope_base, int32_t dtype,
+                     void* stream) {
+  if (batch < 0 || total_kv < 0 || num_slots <= 0) return MSGL_ERR_SHAPE;
+  if (batch == 0) return MSGL_OK;
+  const int rc = check_common(q, k_cache, v_cache, out, num_q_heads, num_kv_heads, head_dim, k_cache_stride0,
+                              v_cache_stride0, dtype, /*f16_ok=*/q_weight == nullptr);
+  if (rc != MSGL_OK) return rc;
+  const int64_t group = num_q_heads / num_kv_heads;
+  if (group > 16) return MSGL_ERR_GROUP_TOO_LARGE;
+  if (!k || !v || !out_loc || !kv_indptr || (total_kv > 0 && !kv_indices)) return MSGL_ERR_NULL_POINTER;
+  if ((q_weight == nullptr) != (k_weight == nullptr) || (q_weight && !positions)) return MSGL_ERR_NULL_POINTER;
+  if (q_stride0 < num_q_heads * head_dim || k_stride0 < num_kv_heads * head_dim || v_stride0 < num_kv_heads * head_dim)
+    return MSGL_ERR_SHAPE;
+  if (q_weight && (!(rope_base > 1.0f) || !(rms_norm_eps >= 0.0f))) return MSGL_ERR_SHAPE;
+  if (!aligned16(k) || !aligned16(v) || q_stride0 % 8 || k_stride0 % 8 || v_stride0 % 8 || !aligned16(q_weight) ||
+      !aligned16(k_weight))
+    return MSGL_ERR_ALIGNMENT;
+  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  if (!msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) return MSGL_ERR_SHAPE;
+  const size_t need = msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
+  if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;
+  msgl::SplitKvArgs a{};
+  a.q = q;
+  a.k_cache = k_cache;
+  a.v_cache = v_cache;
+  a.kv_indptr = kv_indptr;
+  a.kv_indices = kv_indices;
+  a.out = out;
+  a.workspace = workspace;
+  a.batch = batch;
+  a.total_kv = total_kv;
+  a.n_q = num_q_heads;
+  a.n_kv = num_kv_heads;
+  a.head_dim = head_dim;
+  a.num_slots = num_slots;
+  a.k_stride0 = k_cache_stride0;
+  a.v_stride0 = v_cache_stride0;
+  a.q_stride0 = q_stride0;
+  a.sm_scale = sm_scale;
+  a.max_len_extend = 1;
+  a.f16 = (dtype == MSGL_DTYPE_F16) ? 1 : 0;
+  msgl::NewTokens tokens{};
+  tokens.k = k;
+  tokens.v = v;
+  tokens.q_weight = q_weight;
+  tokens.k_weight = k_weight;
+  tokens.positions = positions;
+  tokens.out_loc = out_loc;
+  tokens.k_stride0 = k_stride0;
+  tokens.v_stride0 = v_stride0;
+  tokens.eps = rms_norm_eps;
+  tokens.rope_base = rope_base;
+  return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
 }
 
 // Ragged key shares for the tile kernels (one query block per (request, kv head)): the ping-pong
@@ -434,7 +506,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     a.n_seg = n_seg;
     a.min_seg = min_segment(head_dim);
     a.q_begin = 0;
-    if (shares) return msgl::launch_shares(a, plan, s);
+    if (shares) return msgl::launch_shares(a, msgl::NewTokens{}, plan, s);
     return msgl::launch_splitkv(a, s);
   }
   msgl::PrefillArgs a{};

@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     Columns<D, NCT> c_;
     const FirstIds ids = first_ids(p, r, t_begin, t_end);
     start_columns(p, r, kvh, ct0, t_end, c_);
-    attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_);
+    attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
 
     // ---- this request's share is done: write output or partial -------------------------
 #pragma unroll
@@ -635,6 +635,7 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   p.cols = p.group * a.max_len_extend;
   p.k_stride0 = a.k_stride0;
   p.v_stride0 = a.v_stride0;
+  p.q_stride0 = a.q_stride0 > 0 ? a.q_stride0 : a.n_q * a.head_dim;
   p.batch = (int32_t)a.batch;
   p.n_q = (int32_t)a.n_q;
   p.n_kv = (int32_t)a.n_kv;

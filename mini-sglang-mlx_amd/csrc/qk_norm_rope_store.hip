@@ -17,6 +17,7 @@
 // positions reach 10^5 radians) are computed once per chunk, not once per head.
 #include "msgl_device.h"
 #include "msgl_internal.h"
+#include "norm_rope.h"
 
 namespace msgl {
 namespace {
@@ -45,22 +46,10 @@ struct NormRopeParams {
   float eps, log2_base;
 };
 
-__device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  return __builtin_bit_cast(uint16_t, (__bf16)f);
-}
-
-template <int E>
-struct Vec;  // E bf16 values as one load
-template <>
-struct Vec<4> { typedef u32x2_t type; };
-template <>
-struct Vec<8> { typedef u32x4_t type; };
-
 template <int D, int kHeadsPerGroup>
 __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopeParams p) {
   constexpr int E = D / 32;  // elements per lane and half
-  using V = typename Vec<E>::type;
+  using V = typename HalfRow<E>::type;
   const int j = threadIdx.x & (kGroupLanes - 1);
   const int64_t item = (int64_t)blockIdx.x * (kThreads / kGroupLanes) + (threadIdx.x / kGroupLanes);
   if (item >= (int64_t)p.n_tokens * p.chunks) return;  // whole groups leave together
@@ -99,9 +88,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopePa
     const float pos = (float)position;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const float d = (float)(j * E + e) / (float)(D / 2);
-      const float inv_freq = exp2f(-d * p.log2_base);
-      sincosf(pos * inv_freq, &sn[e], &cs[e]);
+      sincosf(rope_angle<D>(pos, j * E + e, p.log2_base), &sn[e], &cs[e]);
     }
   }
   // a slot id outside the pools stores no k / v row (q_out is still produced): a wild store
@@ -115,37 +102,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_store_kernel(NormRopePa
     V lo = next.lo, hi = next.hi;
     const V wl = next.wl, wh = next.wh;
     if (h + 1 < h_end) next = fetch(h + 1);
-    if (h < p.n_q + p.n_kv) {
-      float xl[E], xh[E];
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const uint32_t a = lo[e >> 1], b = hi[e >> 1];
-        xl[e] = bf16_to_f32((uint16_t)((e & 1) ? a >> 16 : a & 0xffffu));
-        xh[e] = bf16_to_f32((uint16_t)((e & 1) ? b >> 16 : b & 0xffffu));
-        ss += xl[e] * xl[e] + xh[e] * xh[e];
-      }
-      ss = row_sum16(ss);
-      const float norm = rsqrtf(ss * (1.0f / D) + p.eps);
-      uint16_t ol[E], oh[E];
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const uint32_t a = wl[e >> 1], b = wh[e >> 1];
-        const float wlo = bf16_to_f32((uint16_t)((e & 1) ? a >> 16 : a & 0xffffu));
-        const float whi = bf16_to_f32((uint16_t)((e & 1) ? b >> 16 : b & 0xffffu));
-        // normalised value and weighted value each pass through bf16, as they do when the
-        // norm is a kernel of its own with a bf16 result
-        const float yl = bf16_to_f32(f32_to_bf16(wlo * bf16_to_f32(f32_to_bf16(xl[e] * norm))));
-        const float yh = bf16_to_f32(f32_to_bf16(whi * bf16_to_f32(f32_to_bf16(xh[e] * norm))));
-        ol[e] = f32_to_bf16(yl * cs[e] - yh * sn[e]);
-        oh[e] = f32_to_bf16(yl * sn[e] + yh * cs[e]);
-      }
-#pragma unroll
-      for (int e = 0; e < E; e += 2) {
-        lo[e >> 1] = (uint32_t)ol[e] | ((uint32_t)ol[e + 1] << 16);
-        hi[e >> 1] = (uint32_t)oh[e] | ((uint32_t)oh[e + 1] << 16);
-      }
-    }
+    if (h < p.n_q + p.n_kv) norm_rope_head<D>(lo, hi, wl, wh, cs, sn, p.eps);
     if (h >= p.n_q && !slot_ok) continue;
     *reinterpret_cast<V*>(dst + off) = lo;
     *reinterpret_cast<V*>(dst + D / 2 + off) = hi;

@@ -20,6 +20,7 @@ struct SplitKvParams {
   float* part_lse;      // [n_seg + batch][n_kv][cols]
   int32_t* req_items;   // [batch][2] first segment holding the request, number of segments sharing it
   int64_t k_stride0, v_stride0;
+  int64_t q_stride0;    // elements from one row of q to the next
   int32_t batch, n_q, n_kv, group;
   int32_t nwh;          // kv heads per workgroup
   int32_t head_groups;  // n_kv / nwh
@@ -90,8 +91,9 @@ struct Columns {
   f32x4_t o[NCT][D / 128][8];  // o[ct][hf][n][i]: dim hf * 128 + 8 * (4 * (lane / 16) + i) + n
 };
 
-// Columns ct0 * 16 .. of kv head `kvh` of request `r`, for the keys before `t_end`.
-template <int D, int NCT>
+// Columns ct0 * 16 .. of kv head `kvh` of request `r`, for the keys before `t_end`.  LOAD_Q: the Q operand from memory
+// (else it is left to the caller).
+template <int D, int NCT, bool LOAD_Q = true>
 __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqInfo& r, int kvh, int ct0,
                                               int t_end, Columns<D, NCT>& c_) {
   constexpr int KS = D / 32, VH = D / 128;
@@ -105,11 +107,11 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
     const int qi = valid ? col / p.group : 0;
     const int hh = valid ? col - qi * p.group : 0;
     const uint16_t* qrow =
-        p.q + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + hh) * D + g * 8;
+        p.q + (int64_t)(r.q_start + qi) * p.q_stride0 + (kvh * p.group + hh) * D + g * 8;
 #pragma unroll
     for (int c = 0; c < KS; ++c) {
       u32x4_t raw = {0u, 0u, 0u, 0u};
-      if (valid) raw = ld_global_b128(qrow + c * 32);
+      if (LOAD_Q && valid) raw = ld_global_b128(qrow + c * 32);
       c_.q[ct][c] = raw;
     }
     const int qpos = r.prefix + qi;
@@ -152,9 +154,11 @@ __device__ __forceinline__ FirstIds first_ids(const SplitKvParams& p, const ReqI
 // Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`; `first`: its first_ids(), asked for before
 // the columns were made.
 // SHORT: ranges of one tile are common, end behind it (in a long walk the test costs more than it saves).
-template <int D, int NCT, bool WIDE, bool F16, bool SHORT>
+// meanwhile(): called once the first tile has been asked for; may finish the columns' Q operand and put keys of its own
+// into their state.
+template <int D, int NCT, bool WIDE, bool F16, bool SHORT, typename Meanwhile>
 __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInfo& r, int kvh, int t_begin,
-                                            int t_end, const FirstIds& first, Columns<D, NCT>& c_) {
+                                            int t_end, const FirstIds& first, Columns<D, NCT>& c_, Meanwhile&& meanwhile) {
   constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const int lane = lane_id();
@@ -284,6 +288,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
   int i1a = (int)min((uint32_t)first.b[0], p.max_slot), i1b = (int)min((uint32_t)first.b[1], p.max_slot);
   load_tile(ta, i0a, i0b);
   load_idx(t_begin + 64, i0a, i0b);
+  meanwhile();
   for (int pr = 0; pr < n_pairs; ++pr) {
     const int tok = t_begin + pr * 64;
     load_tile(tb_, i1a, i1b);

@@ -516,6 +516,74 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* args, Py_ssize_t n_args
   });
 }
 
+// ---- decode_step(q, k, v, q_weight | None, k_weight | None, positions | None, out_loc, k_cache, v_cache, kv_indptr,
+//                  kv_indices, num_kv_splits, sm_scale, eps, rope_base) -> out or None ------------------
+// Store (or norm, rotary embedding and store) and decode attention as one launch, None where that is not the way: the
+// caller then makes the two calls, which check what is refused here and say why, and take every form.
+PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  return guarded(args, n_args, 15, [](PyObject* const* a) -> PyObject* {
+    static const char op[] = "decode_step";
+    const bool norm = a[3] != Py_None;
+    for (int i = 0; i < 12; ++i)
+      if (!THPVariable_Check(a[i]) && (norm || i < 3 || i > 5)) return none();
+    if (const char* env = std::getenv("MSGL_DEBUG_CHECKS"); env && *env && std::strcmp(env, "0") != 0) return none();
+    auto t = [&](int i) -> const Tensor& { return THPVariable_Unpack(a[i]); };
+    const Tensor &q = t(0), &k = t(1), &v = t(2), &loc = t(6), &kc = t(7), &vc = t(8), &ip = t(9), &ix = t(10), &ns = t(11);
+    if (q.dim() != 3 || k.dim() != 3 || kc.dim() != 3 || vc.dim() != 3) return none();
+    const int64_t batch = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = k.size(1), slots = kc.size(0);
+    const auto dt = q.scalar_type();
+    if (batch == 0 || slots == 0 || n_kv == 0 || n_q == 0 || (dt != at::kBFloat16 && (norm || dt != at::kHalf))) return none();
+    const c10::Device dev = q.device();
+    if (!dev.is_cuda()) return none();
+    auto same = [&](const Tensor& x) { return x.scalar_type() == dt && x.device() == dev; };
+    auto ints_of = [&](const Tensor& x, int64_t n) {
+      return x.dim() == 1 && x.size(0) == n && x.scalar_type() == at::kInt && x.device() == dev && x.is_contiguous();
+    };
+    auto rows = [&](const Tensor& x) {
+      return x.stride(2) == 1 && x.stride(1) == d && (batch == 1 || (x.stride(0) >= x.size(1) * d && x.stride(0) % 8 == 0)) &&
+             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    };
+    auto pool = [&](const Tensor& x) {
+      return x.stride(2) == 1 && x.stride(1) == d && (slots == 1 || (x.stride(0) >= n_kv * d && x.stride(0) % 8 == 0)) &&
+             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    };
+    const c10::IntArrayRef pool_size = kc.sizes();
+    if (!same(k) || !same(v) || !same(kc) || !same(vc) || k.size(0) != batch || k.size(2) != d || v.sizes() != k.sizes() ||
+        pool_size[1] != n_kv || pool_size[2] != d || vc.sizes() != pool_size || !rows(q) || !rows(k) || !rows(v) || !pool(kc) ||
+        !pool(vc) || !ints_of(loc, batch) || !ints_of(ip, batch + 1) || !ints_of(ix, ix.numel()) || !ints_of(ns, batch))
+      return none();
+    float eps = 0.f, base = 0.f;
+    if (norm) {
+      auto weight = [&](const Tensor& x) {
+        return same(x) && x.dim() == 1 && x.size(0) == d && x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+      };
+      if (!weight(t(3)) || !weight(t(4)) || !ints_of(t(5), batch)) return none();
+      eps = static_cast<float>(real(a[13]));
+      base = static_cast<float>(real(a[14]));
+      if (!(base > 1.0f) || !(eps >= 0.0f)) return none();
+    }
+    const size_t bytes = msgl_decode_step_workspace_bytes(batch, ix.size(0), n_q, n_kv, d);
+    if (bytes == 0) return none();
+    const float scale = static_cast<float>(real(a[12]));
+    auto stride0 = [](const Tensor& x) { return x.size(0) > 1 ? x.stride(0) : x.size(1) * x.size(2); };
+    Tensor out;
+    int rc;
+    {
+      NoGil nogil;
+      OnDevice on(dev);
+      out = empty({batch, n_q, d}, dt, dev);
+      const Tensor ws = scratch(bytes, dev);
+      rc = msgl_decode_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), stride0(q), stride0(k), stride0(v),
+                            norm ? t(3).data_ptr() : nullptr, norm ? t(4).data_ptr() : nullptr, norm ? ints(t(5)) : nullptr,
+                            ints(loc), kc.data_ptr(), vc.data_ptr(), ints(ip), ints(ix), out.data_ptr(), ws.data_ptr(), bytes,
+                            batch, ix.size(0), n_q, n_kv, d, slots, stride0(kc), stride0(vc), scale, eps, base,
+                            dt == at::kHalf ? MSGL_DTYPE_F16 : MSGL_DTYPE_BF16, on.ptr());
+    }
+    check_rc(op, rc);
+    return THPVariable_Wrap(std::move(out));
+  });
+}
+
 // ---- gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr, single_token_mode) -> y -------
 PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 9, [](PyObject* const* a) -> PyObject* {
@@ -582,6 +650,7 @@ PyMethodDef g_methods[] = {MSGL_FAST(store_kv_cache),
                            MSGL_FAST(build_attention_metadata),
                            MSGL_FAST(build_metadata_from_host),
                            MSGL_FAST(qk_norm_rope_store),
+                           MSGL_FAST(decode_step),
                            MSGL_FAST(gdn_state_inplace),
                            {"set_checks", set_checks, METH_O, nullptr},
                            {nullptr, nullptr, 0, nullptr}};

@@ -15,7 +15,8 @@ from typing import List, Optional, Sequence
 
 import torch
 
-from mini_sglang_amd_kernel import (build_metadata_from_host, paged_decode_attention,
+from mini_sglang_amd.kvcache.mha_pool import MHAKVCache
+from mini_sglang_amd_kernel import (_native, build_metadata_from_host, paged_decode_attention,
                                     paged_prefill_attention, qk_norm_rope_store)
 
 MAX_KV_SPLITS = 32
@@ -83,10 +84,26 @@ class AttnBackend:
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
         metadata = batch.attn_metadata
+        if not is_cross_attention and sliding_window_size == 0:
+            out = self._decode_step(q, k, v, layer_id, batch)
+            if out is not None:
+                return out
         self.kvcache.store_kv(k, v, batch.out_loc, layer_id)
         k_cache = self.kvcache.k_cache(layer_id)
         v_cache = self.kvcache.v_cache(layer_id)
         return self._attend(q, k_cache, v_cache, metadata, is_cross_attention, sliding_window_size)
+
+    def _decode_step(self, q, k, v, layer_id: int, batch, q_weight=None, k_weight=None,
+                     positions=None, eps: float = 0.0, rope_base: float = 0.0) -> Optional[torch.Tensor]:
+        """``mini_sglang_amd_kernel.decode_step`` on the step's pool, where this package writes that
+        itself; ``None``: the step takes its two calls."""
+        metadata, cache = batch.attn_metadata, self.kvcache
+        if type(metadata) is not DecodeMetadata or type(cache) is not MHAKVCache:
+            return None
+        return _native.decode_step(q, k, v, q_weight, k_weight, positions, batch.out_loc,
+                                   cache.k_cache(layer_id), cache.v_cache(layer_id),
+                                   metadata.kv_indptr, metadata.kv_indices, metadata.num_kv_splits,
+                                   self.sm_scale, eps, rope_base)
 
     def _attend(self, q, k_cache, v_cache, metadata, is_cross_attention: bool,
                 sliding_window_size: int) -> torch.Tensor:
@@ -118,6 +135,11 @@ class AttnBackend:
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
         metadata = batch.attn_metadata
+        if not is_cross_attention and sliding_window_size == 0:
+            out = self._decode_step(q, k, v, layer_id, batch, q_norm_weight, k_norm_weight,
+                                    metadata.positions, rms_norm_eps, rope_base)
+            if out is not None:
+                return out
         k_cache = self.kvcache.k_cache(layer_id)
         v_cache = self.kvcache.v_cache(layer_id)
         q = qk_norm_rope_store(q, k, v, q_norm_weight, k_norm_weight, metadata.positions,

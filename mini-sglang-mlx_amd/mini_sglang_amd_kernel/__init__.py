@@ -28,7 +28,8 @@ except ImportError as _exc:  # not built: the first call says so
     _native = _lib.MissingNative(_exc)
 
 __all__ = ["store_kv_cache", "paged_decode_attention", "paged_prefill_attention",
-           "build_attention_metadata", "build_metadata_from_host", "qk_norm_rope_store", "gdn_state_inplace",
+           "build_attention_metadata", "build_metadata_from_host", "qk_norm_rope_store", "decode_step",
+           "gdn_state_inplace",
            "fast_compare_key"]
 
 
@@ -255,6 +256,24 @@ def qk_norm_rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_weig
     with _on_stream(stream, q):
         return _native.qk_norm_rope_store(q, k, v, q_weight, k_weight, positions, out_loc, k_cache,
                                           v_cache, eps, rope_base, validate)
+
+
+def decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torch.Tensor,
+                k_cache: torch.Tensor, v_cache: torch.Tensor, kv_indptr: torch.Tensor,
+                kv_indices: torch.Tensor, num_kv_splits: torch.Tensor, *, sm_scale: float,
+                q_weight: Optional[torch.Tensor] = None, k_weight: Optional[torch.Tensor] = None,
+                positions: Optional[torch.Tensor] = None, eps: float = 0.0,
+                rope_base: float = 0.0) -> Optional[torch.Tensor]:
+    """``store_kv_cache`` and ``paged_decode_attention`` of a decode step as one launch or, with norm
+    weights, ``qk_norm_rope_store`` and ``paged_decode_attention``: the attention output, or ``None``
+    (nothing done) where the two calls are the way: large launches, forms that need a copy, arguments
+    that they refuse, index validation on.
+
+    One new token per request, row ``b`` at slot ``out_loc[b]``.  A slot of ``out_loc`` must not be
+    listed for any other key that the step sees: the launch that reads it writes it.
+    """
+    return _native.decode_step(q, k, v, q_weight, k_weight, positions, out_loc, k_cache, v_cache,
+                               kv_indptr, kv_indices, num_kv_splits, sm_scale, eps, rope_base)
 
 
 def gdn_state_inplace(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,

@@ -1,0 +1,96 @@
+"""A decode step's store (or norm, rotary embedding and store) inside its attention launch, against the same
+step as two launches, which the oracle tests pin: at the edges of a wave's 32 keys and of a share, for requests
+without keys, for a new token that is not its request's last key, for a slot outside the pool, on strided rows,
+and from a pool whose new slots hold NaN before the step."""
+import pytest
+import torch
+
+from mini_sglang_amd.workloads import build_workload
+from mini_sglang_amd_kernel import _lib, decode_step, paged_decode_attention, qk_norm_rope_store, store_kv_cache
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # kv lengths, q heads, kv heads, head_dim, share_len, kv heads per workgroup (0: the default cut)
+    ([1], 16, 8, 128, 0, 0),
+    ([37, 128, 500, 1023], 16, 8, 128, 0, 0),
+    ([31, 32, 33, 64, 65, 0, 127, 128, 129, 257], 32, 8, 128, 128, 1),
+    ([2100, 5, 64], 64, 4, 128, 64, 4),
+    ([1 + i % 90 for i in range(150)], 16, 8, 128, 0, 0),
+    ([600, 0, 1, 255, 256, 257], 16, 2, 256, 0, 0),
+    ([1500, 40, 32], 24, 4, 256, 64, 4),
+]
+
+
+def _step(gpu, lens, n_q, n_kv, d, dtype, seed):
+    """The step's tensors: q, k, v as views of one projection, and a pool with NaN in the new slots."""
+    wl = build_workload("step", "decode", seed=seed, n_q=n_q, n_kv=n_kv, head_dim=d, kv_lens=lens).to(gpu)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(seed)
+    b = len(lens)
+    qkv = torch.randn((b, n_q + 2 * n_kv, d), generator=g, device=gpu).to(dtype)
+    slots = wl.k_cache.shape[0]
+    kc, vc = (torch.cat([c.to(dtype), c.to(dtype)]) for c in (wl.k_cache, wl.v_cache))  # the upper half is nobody's
+    loc = torch.arange(b, dtype=torch.int32, device=gpu) + slots
+    for i, n in enumerate(lens):  # as a rule a request's last slot is the new token's
+        if n > 0 and i % 5 != 4:
+            loc[i] = wl.kv_indices[int(wl.kv_indptr[i + 1]) - 1]
+    for c in (kc, vc):
+        c[loc.long()] = float("nan")
+    for i, n in enumerate(lens):  # a last slot that is not the new token's holds a row
+        if n > 0 and i % 5 == 4:
+            for c in (kc, vc):
+                c[wl.kv_indices[int(wl.kv_indptr[i + 1]) - 1].long()] = 0.5
+    if b > 2:
+        loc[2] = kc.shape[0] + 7  # outside the pool: nothing is stored
+        at = wl.kv_indices[int(wl.kv_indptr[3]) - 1].long()
+        if lens[2] > 0:
+            kc[at] = vc[at] = 0.25
+    parts = (qkv[:, :n_q], qkv[:, n_q:n_q + n_kv], qkv[:, n_q + n_kv:])
+    return wl, parts, loc, kc, vc
+
+
+@pytest.mark.parametrize("lens,n_q,n_kv,d,share,heads", CASES)
+@pytest.mark.parametrize("mode", ["bf16", "f16", "norm"])
+def test_one_launch_is_two(gpu, tuning, lens, n_q, n_kv, d, share, heads, mode):
+    dtype = torch.float16 if mode == "f16" else torch.bfloat16
+    wl, (q, k, v), loc, kc, vc = _step(gpu, lens, n_q, n_kv, d, dtype, len(lens) + d)
+    norm = {}
+    if mode == "norm":
+        g = torch.Generator(device=gpu)
+        g.manual_seed(1)
+        w = (1 + 0.2 * torch.randn((2, d), generator=g, device=gpu)).to(dtype)
+        pos = torch.tensor([max(n - 1, 0) + 40000 * (i % 3 == 1) for i, n in enumerate(lens)], dtype=torch.int32, device=gpu)
+        norm = dict(q_weight=w[0], k_weight=w[1], positions=pos, eps=1e-6, rope_base=1e6)
+    tuning(_lib.TUNE_SHARES, share | heads << 20)
+    kc2, vc2 = kc.clone(), vc.clone()
+    print(f"decode step {lens[:4]} {n_q}/{n_kv} d{d} {mode} cut {share} x {heads}", flush=True)
+    got = decode_step(q, k, v, loc, kc, vc, wl.kv_indptr, wl.kv_indices, wl.num_kv_splits, sm_scale=wl.sm_scale, **norm)
+    assert got is not None
+    if mode == "norm":
+        q = qk_norm_rope_store(q, k, v, w[0], w[1], pos, loc, kc2, vc2, eps=1e-6, rope_base=1e6)
+    else:
+        store_kv_cache(kc2, vc2, loc, k, v)
+    want = paged_decode_attention(q, kc2, vc2, wl.kv_indptr, wl.kv_indices, wl.num_kv_splits, wl.sm_scale, 32)
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))  # noqa: E731
+    assert bool(torch.isfinite(got).all())
+    assert same(vc, vc2)
+    assert same(kc, kc2)
+    # the new key's weight and its products are fp32 where the other launch has them in 16 bits: a step of the result's
+    # type, and where few keys share the weight half a 16-bit step of the new key's own
+    diff = (got.float() - want.float()).abs()
+    assert float(diff.max()) <= 2e-2 and float(diff.mean()) <= 1e-3, (float(diff.max()), float(diff.mean()))
+
+
+def test_what_is_left_to_the_two_calls(gpu, monkeypatch):
+    """None, and nothing done: rows that need a copy, a large launch, index validation on."""
+    wl, (q, k, v), loc, kc, vc = _step(gpu, [40, 70], 16, 8, 128, torch.bfloat16, 3)
+    before = kc.clone()
+    args = lambda k=k: (q, k, v, loc, kc, vc, wl.kv_indptr, wl.kv_indices, wl.num_kv_splits)  # noqa: E731
+    turned = k.transpose(1, 2).contiguous().transpose(1, 2)
+    assert decode_step(*args(turned), sm_scale=0.1) is None
+    monkeypatch.setenv("MSGL_DEBUG_CHECKS", "1")
+    assert decode_step(*args(), sm_scale=0.1) is None
+    monkeypatch.setenv("MSGL_DEBUG_CHECKS", "0")
+    assert torch.equal(before.view(torch.int16), kc.view(torch.int16))
+    assert decode_step(*args(), sm_scale=0.1) is not None
+    assert _lib.load().msgl_decode_step_workspace_bytes(64, 64 * 4096, 32, 8, 128) == 0
