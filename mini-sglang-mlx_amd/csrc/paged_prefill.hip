@@ -635,6 +635,10 @@ __global__ __launch_bounds__(NW * 64) void prefill_tile_kernel(PrefillParams p) 
 // M phase before the one that uses them), which keeps every vector-memory operation of the loop
 // out of the compiler's wait bookkeeping: the only vector-memory wait in the loop is the counted
 // one before an M phase's barrier.  Order of issue inside an M phase: [ring fetch, 4 moves].
+//
+// A workgroup that stays for several query blocks (kStay) runs all of this as one stream of tiles: tile numbers,
+// stages and the ring go on from block to block, so the moves of the next block's tiles take the places of
+// moves past a block's end, and nothing drains in between.
 #ifndef MSGL_PP_PRIO_M
 #define MSGL_PP_PRIO_M 3
 #endif
@@ -667,9 +671,59 @@ constexpr int kOperandBuffers = kAhead + 1;
 }  // namespace pp
 
 // How a workgroup comes by its work: kBatch, (request, kv head, key split, query block) or ragged share;
-// kGang, the parts of a gang's range; kLength, query blocks in order of length.  A kernel each: with all of
-// them in one, their registers spill inside the loop.
-enum class Order { kBatch, kGang, kLength };
+// kGang, the parts of a gang's range; kLength, a query block in order of length; kStay, several of those.  A
+// kernel each: with all of them in one, their registers spill inside the loop.
+enum class Order { kBatch, kGang, kLength, kStay };
+
+// Scores of keys beyond `bound` (AFTER: above it, else below) become -infinity: of a lane's 32 scores of a tile, number
+// i of half kt is key 32 kt + 8 (i / 4) + i % 4.  Four at a time, so that no result of a compare is wanted by the
+// next two instructions (which would have to wait for it); left to the compiler, all compares come first and their
+// results push the kernel's scalars out of their registers.
+template <bool AFTER>
+__device__ __forceinline__ void mask_keys(f32x16_t (&s)[2], int bound) {
+  const float low = kNegInf;
+#define MSGL_MASK4(op)                                                                                        \
+  asm volatile(op " vcc, %[k0], %[bound]\n\t" op " %[a], %[k1], %[bound]\n\t" op " %[b], %[k2], %[bound]\n\t"  \
+               op " %[c], %[k3], %[bound]\n\tv_cndmask_b32 %[x0], %[x0], %[low], vcc\n\t"                     \
+               "v_cndmask_b32 %[x1], %[x1], %[low], %[a]\n\tv_cndmask_b32 %[x2], %[x2], %[low], %[b]\n\t"      \
+               "v_cndmask_b32 %[x3], %[x3], %[low], %[c]"                                                     \
+               : [x0] "+v"(x[0]), [x1] "+v"(x[1]), [x2] "+v"(x[2]), [x3] "+v"(x[3]), [a] "=&s"(a), [b] "=&s"(b), [c] "=&s"(c) \
+               : [k0] "n"(key), [k1] "n"(key + 1), [k2] "n"(key + 2), [k3] "n"(key + 3), [bound] "v"(bound), [low] "v"(low)   \
+               : "vcc")
+  auto quad = [&](auto number) {
+    constexpr int q = decltype(number)::value, key = 8 * q;
+    float x[4];
+    uint64_t a, b, c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = s[q >> 2][4 * (q & 3) + e];
+    if constexpr (AFTER) MSGL_MASK4("v_cmp_gt_i32");
+    else MSGL_MASK4("v_cmp_lt_i32");
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[q >> 2][4 * (q & 3) + e] = x[e];
+  };
+#undef MSGL_MASK4
+  // the scores may have left the matrix pipe just now; the compiler, which knows how long a result takes, does not look
+  // into the statements above
+  asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+  quad(std::integral_constant<int, 0>{});
+  quad(std::integral_constant<int, 1>{});
+  quad(std::integral_constant<int, 2>{});
+  quad(std::integral_constant<int, 3>{});
+  quad(std::integral_constant<int, 4>{});
+  quad(std::integral_constant<int, 5>{});
+  quad(std::integral_constant<int, 6>{});
+  quad(std::integral_constant<int, 7>{});
+}
+
+// A workgroup's blocks of a launch in order of length
+struct ListedBlock {
+  int kvh, qblk, q_start, q_len, kv_start, kv_len, prefix;
+  int k_lo, k_hi, n_tiles;  // keys that some row of the block sees, from a whole tile on
+};
+struct BlockList {
+  ListedBlock block[kMaxRounds];
+  int count, blank;  // blocks; whether one has no keys
+};
 
 template <bool WIDE, Order ORDER>
 __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) {
@@ -691,10 +745,71 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   // fall into its gang's range, one after the other (see gang_plan) -----------------------------
   __shared__ GangLds gang_lds;
   __shared__ int gang_last;
+  __shared__ BlockList list;
   constexpr bool ganged = ORDER == Order::kGang;
   const int gang_xcd = (int)(blockIdx.x & 7);
   const int gang_id = ganged ? (int)(blockIdx.x >> 3) / p.n_qblk : 0;
   const int gang_member = ganged ? (int)(blockIdx.x >> 3) % p.n_qblk : 0;
+  // keys that some row of a block sees
+  auto visible = [&](int prefix, int kn, int row0, int rows_total, int* lo, int* hi) {
+    const int qi_lo = row0 / p.group;
+    const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;
+    *hi = p.is_cross ? kn : min(kn, prefix + qi_hi + 1);
+    *lo = (p.window > 0) ? max(0, prefix + qi_lo - p.window + 1) : 0;
+    *lo &= ~(kBN - 1);
+    if (*hi < *lo) *hi = *lo;
+  };
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
+  auto row_of = [&](int start, int head, int row, int total) {  // rows past the request's last: its first, never stored
+    const int qi = row < total ? row_to_query(p, row) : 0;
+    return (start + qi) * p.n_q + head * p.group + (row < total ? row - qi * p.group : 0);
+  };
+  // ---- order of length: the workgroup's blocks, found by its waves side by side -----------------
+  constexpr bool listed = ORDER == Order::kStay;
+  int n_listed = 0;
+  if constexpr (listed) {
+    if (tid == 0) list.count = list.blank = 0;
+    const LengthOrder<kRows> order(p);
+    const int r = (int)(blockIdx.x >> 3), rounds = p.length_rounds;
+    __syncthreads();
+    for (int i = w; i < rounds; i += NW) {
+      constexpr int kPerXcd = kComputeUnits / 8;
+      const int seq = i * kPerXcd + ((i & 1) ? kPerXcd - 1 - r : r);
+      const LengthBlock x = order.find(seq);
+      if (!x.ok) break;
+      ListedBlock l{x.kvh, x.qblk, x.q_start, x.q_len, x.kv_start, x.kv_len, x.prefix, 0, 0, 0};
+      visible(l.prefix, l.kv_len, l.qblk * kRows, l.q_len * p.group, &l.k_lo, &l.k_hi);
+      l.n_tiles = (l.k_hi - l.k_lo + kBN - 1) / kBN;
+      if (lane == 0) {
+        list.block[i] = l;
+        atomicMax(&list.count, i + 1);
+        if (l.n_tiles == 0) list.blank = 1;
+      }
+    }
+    __syncthreads();
+    n_listed = uniform(list.count);
+    if (uniform(list.blank) != 0) {  // rows without keys are zero; the list goes on without their blocks
+      for (int i = 0; i < n_listed; ++i) {
+        const ListedBlock& l = list.block[i];
+        const int row = l.qblk * kRows + tid / 2, total = l.q_len * p.group;
+        if (l.n_tiles == 0 && row < total) {
+          uint16_t* dst = p.out + (int64_t)row_of(l.q_start, l.kvh, row, total) * D + 64 * (tid & 1);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) st_global_b128(dst + 8 * e, u32x4_t{0u, 0u, 0u, 0u});
+        }
+      }
+      __syncthreads();
+      if (tid == 0) {
+        int n = 0;
+        for (int i = 0; i < n_listed; ++i)
+          if (list.block[i].n_tiles > 0) list.block[n++] = list.block[i];
+        list.count = n;
+      }
+      __syncthreads();
+      n_listed = uniform(list.count);
+    }
+    if (n_listed == 0) return;
+  }
   GangPlan plan{0, 0, 0, 0};
   if (ganged) plan = gang_plan<NW * 64>(p, gang_lds, gang_xcd, gang_id, gang_member, kRows, tid);
   for (int piece = plan.first_unit;; ++piece) {
@@ -724,8 +839,10 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     to_partial = false;
   } else if (piece > 0) {
     break;
+  } else if (listed) {
+    b = kvh = qblk = 0;  // the list has them
   } else if (ORDER == Order::kLength) {
-    by_length = block_by_length<kRows>(p);
+    by_length = LengthOrder<kRows>(p).find((int)(blockIdx.x >> 3));
     if (!by_length.ok) return;
     b = by_length.b;
     kvh = by_length.kvh;
@@ -756,16 +873,31 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     b = request_of_rank<NW * 64>(p.kv_indptr, p.batch, want_rank, tid);
   }
 
-  // the request's geometry: gang ranges keep it in LDS, blocks in order of length come with it (a part or
+  // the request's geometry: gang ranges keep it in LDS, blocks in order of length have it in their list (a part or
   // block starts without another memory round trip)
-  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
   int q_start, q_len, kv_start, kn, prefix;
+  int k_lo, k_hi, n_tiles;
+  auto take = [&](int i) {
+    const ListedBlock& l = list.block[i];
+    kvh = uniform(l.kvh);
+    qblk = uniform(l.qblk);
+    q_start = uniform(l.q_start);
+    q_len = uniform(l.q_len);
+    kv_start = uniform(l.kv_start);
+    kn = uniform(l.kv_len);
+    prefix = uniform(l.prefix);
+    k_lo = uniform(l.k_lo);
+    k_hi = uniform(l.k_hi);
+    n_tiles = uniform(l.n_tiles);
+  };
   if (ganged) {
     q_start = uniform(gang_lds.q_start[b]);
     q_len = uniform(gang_lds.q_len[b]);
     kv_start = uniform(gang_lds.kv_start[b]);
     kn = uniform(gang_lds.kv_len[b]);
     prefix = uniform(gang_lds.prefix[b]);
+  } else if (listed) {
+    take(0);
   } else if (ORDER == Order::kLength) {
     q_start = by_length.q_start;
     q_len = by_length.q_len;
@@ -780,72 +912,69 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     kn = max(p.kv_indptr[b + 1] - kv_start, 0);
     prefix = p.prefix_lens[b];
   }
-  const int rows_total = q_len * p.group;
-  const int row0 = qblk * kRows;
+  int rows_total = q_len * p.group;
+  int row0 = qblk * kRows;
   if (row0 >= rows_total) {
     if (ganged) continue;  // this request has no such query block
     return;
   }
 
-  const bool idle = __builtin_amdgcn_readfirstlane(row0 + w * 32 >= rows_total ? 1 : 0) != 0;
-  const int qi_lo = row0 / p.group;
-  const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;
-  int k_hi = p.is_cross ? kn : min(kn, prefix + qi_hi + 1);
-  int k_lo = (p.window > 0) ? max(0, prefix + qi_lo - p.window + 1) : 0;
-  k_lo &= ~(kBN - 1);
-  if (k_hi < k_lo) k_hi = k_lo;
-  if (ganged) {  // tiles [piece_a, piece_b) of the unit, as far as this query block sees them
-    k_lo = min(k_lo + piece_a * kBN, k_hi);
-    k_hi = min(k_hi, piece_b * kBN);
-    if (k_hi < k_lo) k_hi = k_lo;
-  } else if (p.ragged_tiles > 0) {  // the request's shares are equal: none longer than ragged_tiles
-    const int all_tiles = (k_hi - k_lo + kBN - 1) / kBN;
-    const int share = (all_tiles + n_shares - 1) / n_shares * kBN;
-    k_lo = min(k_lo + split * share, k_hi);
-    k_hi = min(k_hi, k_lo + share);
-  } else if (p.n_ksplit > 1) {
-    const int all_tiles = (k_hi - k_lo + kBN - 1) / kBN;
-    const int share = (all_tiles + p.n_ksplit - 1) / p.n_ksplit * kBN;
-    k_lo = min(k_lo + split * share, k_hi);
-    k_hi = min(k_hi, k_lo + share);
+  bool idle = __builtin_amdgcn_readfirstlane(row0 + w * 32 >= rows_total ? 1 : 0) != 0;
+  if constexpr (!listed) {
+    visible(prefix, kn, row0, rows_total, &k_lo, &k_hi);
+    if (ganged) {  // tiles [piece_a, piece_b) of the unit, as far as this query block sees them
+      k_lo = min(k_lo + piece_a * kBN, k_hi);
+      k_hi = min(k_hi, piece_b * kBN);
+      if (k_hi < k_lo) k_hi = k_lo;
+    } else if (p.ragged_tiles > 0) {  // the request's shares are equal: none longer than ragged_tiles
+      const int all_tiles = (k_hi - k_lo + kBN - 1) / kBN;
+      const int share = (all_tiles + n_shares - 1) / n_shares * kBN;
+      k_lo = min(k_lo + split * share, k_hi);
+      k_hi = min(k_hi, k_lo + share);
+    } else if (p.n_ksplit > 1) {
+      const int all_tiles = (k_hi - k_lo + kBN - 1) / kBN;
+      const int share = (all_tiles + p.n_ksplit - 1) / p.n_ksplit * kBN;
+      k_lo = min(k_lo + split * share, k_hi);
+      k_hi = min(k_hi, k_lo + share);
+    }
+    n_tiles = (k_hi - k_lo + kBN - 1) / kBN;
   }
-  const int n_tiles = (k_hi - k_lo + kBN - 1) / kBN;
 
   // ---- this lane's row: Q operand, visibility bounds ---------------------------------------
   // (the Q rows themselves are requested in the prologue, after the first tiles' slot ids: the
   // ids gate the first tile moves, and a wait for them would otherwise wait for the Q rows too)
   bf16x8_t qreg[KSTEPS];
-  int64_t q_off;
+  int q_row;  // row of q and of out
   int row_lo, row_hi;
-  int w_lo_max = -0x7fffffff, w_hi_min = 0x7fffffff;
-  {
-    const int row = row0 + w * 32 + c32;
+  int w_lo_max, w_hi_min;
+  auto row_bounds = [&]() {
+    const int first = row0 + w * 32, row = first + c32, end = min(rows_total, first + 32);
+    auto low = [&](int qpos) { return (p.window > 0) ? qpos - p.window + 1 : 0; };
+    auto high = [&](int qpos) { return min(p.is_cross ? kn - 1 : min(qpos, kn - 1), k_hi - 1); };
+    // the wave's rows in order of position: its last row has the highest lower bound, its first the lowest upper one
+    const bool some = first < rows_total;
+    w_lo_max = some ? low(prefix + uniform(row_to_query(p, end - 1))) : -0x7fffffff;
+    w_hi_min = some ? high(prefix + uniform(row_to_query(p, first))) : 0x7fffffff;
     const bool valid = row < rows_total;
-    const int qi = valid ? row / p.group : 0;
-    const int hh = valid ? row - qi * p.group : 0;
-    q_off = ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * D;
-    const int qpos = prefix + qi;
-    int lo = (p.window > 0) ? qpos - p.window + 1 : 0;
-    int hi = min(p.is_cross ? kn - 1 : min(qpos, kn - 1), k_hi - 1);
-    if (valid) {
-      w_lo_max = lo;
-      w_hi_min = hi;
-    } else {
-      lo = 1;
-      hi = 0;
-    }
-    row_lo = lo;
-    row_hi = hi;
-  }
-  w_lo_max = wave_max(w_lo_max);
-  w_hi_min = wave_min(w_hi_min);
+    const int qpos = prefix + row_to_query(p, valid ? row : 0);
+    row_lo = valid ? low(qpos) : 1;
+    row_hi = valid ? high(qpos) : 0;
+  };
+  q_row = row_of(q_start, kvh, row0 + w * 32 + c32, rows_total);
+  row_bounds();
 
   f32x16_t oacc[DT];
+  float m_run, l_run, m_safe_run;
+  auto zero_output = [&]() {
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
-  float m_run = kNegInf, l_run = 0.f, m_safe_run = 0.f;
+      for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+    m_run = kNegInf;
+    l_run = 0.f;
+    m_safe_run = 0.f;
+  };
+  zero_output();
 
   // ---- moving tiles -------------------------------------------------------------------------
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSGL_LDS_PTR(unsigned char, smem);
@@ -864,9 +993,31 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   // e = 0 .. 4 UPW - 1; lanes past that repeat the entries
   const uint32_t ring0 = (uint32_t)pp::kRingBase + (uint32_t)w * pp::kRingWave;
   const int ring_key = w * UPW + (lane % UPW) + 16 * ((lane / UPW) & 3);
-  auto ring_fetch = [&](int t) {  // tile t of this block
-    const uint32_t off = (uint32_t)min(k_lo + t * kBN + ring_key, kn - 1) * 4u;
-    lds_direct_b32(lds0 + ring0 + (uint32_t)(t & (pp::kRingStages - 1)) * pp::kRingStage, idx_base, off);
+  // Order of length: the next tile whose slot ids are wanted, through all blocks of the list (behind the last tile:
+  // that again, for moves that nobody reads)
+  struct Cursor {
+    const int32_t* idx;
+    int block, tile, tiles, first, last;  // the block's: place, next tile, tiles, first key, last listed key
+  } ahead{idx_base, 0, 0, n_tiles, k_lo, kn - 1};
+  auto next_tile = [&]() {
+    if (++ahead.tile < ahead.tiles) return;
+    if (ahead.block + 1 == n_listed) {
+      --ahead.tile;
+      return;
+    }
+    const ListedBlock& l = list.block[ahead.block + 1];
+    ahead = Cursor{p.kv_indices + uniform(l.kv_start), ahead.block + 1, 0, uniform(l.n_tiles), uniform(l.k_lo), uniform(l.kv_len) - 1};
+  };
+  auto ring_fetch = [&](int t) {  // tile t of this block, or of the list
+    int key = k_lo + t * kBN, last = kn - 1;
+    const int32_t* idx = idx_base;
+    if constexpr (listed) {
+      key = ahead.first + ahead.tile * kBN;
+      last = ahead.last;
+      idx = ahead.idx;
+    }
+    lds_direct_b32(lds0 + ring0 + (uint32_t)(t & (pp::kRingStages - 1)) * pp::kRingStage, idx,
+                   (uint32_t)min(key + ring_key, last) * 4u);
   };
   auto ring_read = [&](int t, uint32_t (&ids)[UPW]) {
     // read through an LDS pointer: a volatile read through a generic one would be a flat load,
@@ -995,6 +1146,9 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       constexpr int t = i % 4;
       if constexpr (QK && pp::kHandoff > 0 && i == NS - pp::kHandoff) {
         end_of_sends(j);
+        // a phase of scores only ends with a slice of scores behind the barrier, and K's stage is refilled in the
+        // next phase: its operands are there before the barrier
+        if constexpr (!PV) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         slot_barrier();
       }
       request(std::integral_constant<int, i + pp::kAhead>{});
@@ -1067,31 +1221,34 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     return (psum[0] + psum[1]) + (psum[2] + psum[3]);
   };
   // V phase j: P(j+1) from S(j+1), then the first operands of M phase j+1
-  auto v_phase = [&](int j, bf16x8_t (&o)[pp::kOperandBuffers][4]) {
+  // (t: its number in the stream of tiles, which decides the stages; as j where the stream is one block's)
+  auto v_phase = [&](int j, int t, bf16x8_t (&o)[pp::kOperandBuffers][4]) {
     // First of all the operands of the first slice of M phase j+1 (its scores', if it computes
     // any) are requested: they arrive while the VALU works, and that phase's first MFMA finds
     // them there.  (The last phase, P V only, asks for its operands itself: the V tile it reads
     // may only have been published by the barrier that precedes it.)
-    if (j + 2 < n_tiles) k_ops(smem + k_stage_of(j + 2) + k_lane, 0, 0, o[0]);
+    // (and before that the next tile wanted is found: a branch behind the exponentials would let the compiler move
+    // them behind it, into the M phase)
+    if constexpr (listed) next_tile();
+    if (j + 2 < n_tiles) k_ops(smem + k_stage_of(t + 2) + k_lane, 0, 0, o[0]);
     __builtin_amdgcn_sched_barrier(0);
     const int base = k_lo + (j + 1) * kBN;
-    const bool boundary = general_scale || base < w_lo_max || base + kBN - 1 > w_hi_min;
     {
       float mul = p.scale_log2e;
-      if (boundary) {
-        // boundary tile: scale and mask in place.  The empty volatile statement keeps this a
-        // branch: as selects it would put 100 more VALU instructions into every tile.
+      // Boundary tiles: masked in place, one side at a time (the causal diagonal has no other; both sides and the
+      // scale at once were 160 instructions a tile, one side is 64).  Keys count from the lane's first, so their
+      // numbers are constants.
+      if (general_scale) {  // a negative scale would turn the marks round
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = base + 32 * kt + 8 * (i >> 2) + 4 * h + (i & 3);
-            const float x = s[kt][i] * p.scale_log2e;
-            s[kt][i] = (key < row_lo || key > row_hi) ? kNegInf : x;
-          }
+          for (int i = 0; i < 16; ++i) s[kt][i] *= p.scale_log2e;
         mul = 1.0f;
       }
+      const int lane_base = base + 4 * h;
+      if (base + kBN - 1 > w_hi_min) mask_keys<true>(s, row_hi - lane_base);
+      if (base < w_lo_max) mask_keys<false>(s, row_lo - lane_base);
       const float mx = fmaxf(half_max(0), half_max(1));
       float m_safe = m_safe_run, alpha = 1.0f;
       // Has some lane seen a score more than kLazy above its row's reference?  If not, no row's
@@ -1104,7 +1261,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
         const float m_use = (m_new - m_old > kLazy) ? m_new : m_old;
         m_safe = (m_use == kNegInf) ? 0.f : m_use;
         m_safe_run = m_safe;
-        alpha = fast_exp2(m_old - m_safe);
+        alpha = m_old == kNegInf ? 1.0f : fast_exp2(m_old - m_safe);  // the first keys of a row: nothing to rescale
         m_run = m_use;
         if (__any(alpha != 1.0f)) {
 #pragma unroll
@@ -1117,6 +1274,43 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     }
   };
 
+  // ---- order of length: from block to block ---------------------------------------------------
+  // Rows straight from the accumulators: the lanes of a row (c32, both h) swap four dims for four, so that each has 8
+  // neighbours of every 16.  (Through LDS, as below, they would need stages that hold the next block's tiles.)
+  // (pin: what a lane adds to a row's address is made anew, not kept through the tile loop)
+  auto row_at = [&](const uint16_t* base, int row, uint32_t lane_off) {
+    pin(lane_off);
+    return base + (int64_t)row * D + lane_off;
+  };
+  auto write_rows = [&](int row) {  // -1: none
+    const float l = sum_across<32>(l_run);
+    const float inv = (l > 0.f) ? 1.0f / l : 0.f;
+    u32x4_t out[DT][2];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int i = 8 * a + 2 * e;
+          const auto swapped = __builtin_amdgcn_permlane32_swap(pack_bf16x2(oacc[dt][i] * inv, oacc[dt][i + 1] * inv),
+                                                                pack_bf16x2(oacc[dt][i + 4] * inv, oacc[dt][i + 5] * inv), false, false);
+          out[dt][a][e] = swapped[0];
+          out[dt][a][2 + e] = swapped[1];
+        }
+    if (row < 0) return;
+    uint16_t* dst = const_cast<uint16_t*>(row_at(p.out, row, 8 * h));
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) st_global_b128(dst + 32 * dt + 16 * a, out[dt][a]);
+  };
+  // The list's block `i`, but for the lane's bounds: row_bounds() when the block before it is done with its own.
+  auto enter = [&](int i) {
+    take(i);
+    rows_total = q_len * p.group;
+    row0 = qblk * kRows;
+  };
   if (n_tiles > 0) {
     // ---- prologue: K(0..2) and V(0) leave, the ring gets tiles 3, 4.  Only the Q rows, the ring and K(0) are
     // waited for: the first M phase needs no more, its own wait (or, in the group that runs a slot
@@ -1125,21 +1319,55 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     // would be waits for everything in flight.
     {
       uint32_t first[3][UPW];
+      int key[3], last[3];
+      const int32_t* idx[3];
+      // (all five tiles wanted here are the first block's, as a rule)
+      const bool stepwise = listed && n_tiles < 6;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        key[t] = k_lo + t * kBN;
+        last[t] = kn - 1;
+        idx[t] = idx_base;
+      }
+      if (stepwise) {
+#pragma unroll 1
+        for (int t = 0; t < 3; ++t) {
+          const int k = ahead.first + ahead.tile * kBN;
+          key[0] = t == 0 ? k : key[0];
+          key[1] = t == 1 ? k : key[1];
+          key[2] = t == 2 ? k : key[2];
+          last[1] = t == 1 ? ahead.last : last[1];
+          last[2] = t == 2 ? ahead.last : last[2];
+          idx[1] = t == 1 ? ahead.idx : idx[1];
+          idx[2] = t == 2 ? ahead.idx : idx[2];
+          next_tile();
+        }
+      } else if (listed) {
+        ahead.tile = 3;
+      }
 #pragma unroll
       for (int t = 0; t < 3; ++t)
 #pragma unroll
         for (int i = 0; i < UPW; ++i)
           asm volatile("global_load_dword %0, %1, %2"
                        : "=v"(first[t][i])
-                       : "v"((uint32_t)min(k_lo + t * kBN + unit_key + i, kn - 1) * 4u), "s"(idx_base)
+                       : "v"((uint32_t)min(key[t] + unit_key + i, last[t]) * 4u), "s"(idx[t])
                        : "memory");
       u32x4_t raw[KSTEPS];
-      const uint16_t* qrow = p.q + q_off + h * 8;  // rows past the request's last: its first, never stored
+      const uint16_t* qrow = p.q + (int64_t)q_row * D + h * 8;  // rows past the request's last: its first, never stored
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ++ks)
         asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(raw[ks]) : "v"(qrow), "n"(ks * 32) : "memory");
       ring_fetch(3);
+      if constexpr (listed) {
+        if (stepwise) next_tile();
+        else ahead.tile = 4;
+      }
       ring_fetch(4);
+      if constexpr (listed) {
+        if (stepwise) next_tile();
+        else ahead.tile = 5;
+      }
       static_assert(UPW == 2 && KSTEPS == 8, "the slot ids and the Q rows are named one by one");
       asm volatile("s_waitcnt vmcnt(%6)"
                    : "+v"(first[0][0]), "+v"(first[0][1]), "+v"(first[1][0]), "+v"(first[1][1]), "+v"(first[2][0]), "+v"(first[2][1])
@@ -1177,6 +1405,54 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     __syncthreads();
     const bool second = w >= 4;  // the group that runs one slot behind
     if (second) wait_all_vm();
+    if constexpr (listed) {
+      // One stream of tiles through all blocks: t is a tile's number in it (and its M phase's), j its number in its
+      // block.  Where a block ends, its last P V and the scores of the next one's first tile share an M phase, and its
+      // rows leave in the V phase behind that; the Q rows of the next block are asked for when the last
+      // scores of this one are done, a V phase and four slices ahead of their use.
+      bf16x8_t oa[pp::kOperandBuffers][4];
+      int t = -1, at_block = 0;
+      int out_row = -1;  // row of the block before this one, still in the accumulators
+      if (second) slot_barrier();
+      for (;;) {
+        t = uniform(t);
+        int then_row = 0;
+        auto next_rows = [&]() {
+          if (at_block + 1 >= n_listed) return;
+          const ListedBlock& l = list.block[at_block + 1];
+          then_row = row_of(uniform(l.q_start), uniform(l.kvh), uniform(l.qblk) * kRows + w * 32 + c32, uniform(l.q_len) * p.group);
+          const uint16_t* src = row_at(p.q, then_row, 8 * h);
+#pragma unroll
+          for (int ks = 0; ks < KSTEPS; ++ks) qreg[ks] = as_bf16x8(ld_global_b128(src + ks * 16));
+        };
+        // the Q rows are there before the phase's moves leave: a wait behind those would be one for them
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(qreg[ks]));
+        m_phase(t, oa, No{}, Yes{});  // with its barrier
+        write_rows(out_row);
+        row_bounds();
+        zero_output();
+        int j = -1;
+        for (; j + 2 < n_tiles; ++j) {
+          v_phase(j, t, oa);
+          slot_barrier();
+          m_phase(++t, oa, Yes{}, Yes{});  // with its barrier
+        }
+        next_rows();
+        v_phase(j, t, oa);
+        slot_barrier();
+        m_phase(++t, oa, Yes{}, No{});
+        out_row = row0 + w * 32 + c32 < rows_total ? q_row : -1;
+        if (++at_block == n_listed) break;
+        enter(at_block);
+        q_row = then_row;
+      }
+      wait_all_vm();
+      slot_barrier();
+      if (!second) slot_barrier();
+      write_rows(out_row);
+      return;
+    }
     if (idle) {
       // the moves, waits and barriers of a computing wave of the same group, nothing else
       if (second) slot_barrier();
@@ -1194,11 +1470,11 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       bf16x8_t oa[pp::kOperandBuffers][4];
       if (second) slot_barrier();
       m_phase(-1, oa, No{}, Yes{});  // with its barrier
-      v_phase(-1, oa);
+      v_phase(-1, -1, oa);
       slot_barrier();
       for (int j = 0; j < n_tiles - 1; ++j) {
         m_phase(j, oa, Yes{}, Yes{});  // with its barrier
-        v_phase(j, oa);
+        v_phase(j, j, oa);
         slot_barrier();
       }
       m_phase(n_tiles - 1, oa, Yes{}, No{});
@@ -1485,6 +1761,7 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
     else hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, false>), grid, dim3(512), 0, stream, p);
   } else {
     auto* const kernel = p.gangs > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kGang> : prefill_pingpong_kernel<false, Order::kGang>)
+                         : p.length_rounds > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kStay> : prefill_pingpong_kernel<false, Order::kStay>)
                          : p.length_heads > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kLength> : prefill_pingpong_kernel<false, Order::kLength>)
                                               : (wide ? prefill_pingpong_kernel<true, Order::kBatch> : prefill_pingpong_kernel<false, Order::kBatch>);
     hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, p);

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       p.req_units[2 * b + 1] = ru.count;
     }
   } else if (p.length_heads > 0) {
-    by_length = block_by_length<kRows>(p);
+    by_length = LengthOrder<kRows>(p).find((int)(blockIdx.x >> 3));
     if (!by_length.ok) return;
     b = by_length.b;
     kvh = by_length.kvh;

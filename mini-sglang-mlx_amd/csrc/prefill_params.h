@@ -41,6 +41,10 @@ struct PrefillParams {
   // query blocks in order of length (see prefill_by_length()): kv heads per XCD, 0 = off, and the
   // logarithm of the number of XCDs that share a kv head's blocks
   int32_t length_heads, length_log2_xcds;
+  // head_dim 128: above 0, one workgroup per compute unit stays for the launch and takes one block in each of
+  // this many rounds (see kMaxRounds)
+  int32_t length_rounds;
+  uint32_t group_magic, group_shift;  // row / group of a row below 2^31: see row_to_query()
   long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
 };
 
@@ -180,6 +184,20 @@ inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
          a.batch * a.n_kv * n_qblk > kComputeUnits && !(even_prompts && n_qblk >= 16);
 }
 
+// Rounds of blocks that a workgroup may stay for.  A workgroup of the head_dim 128 kernel that ends pays for the next
+// one's start: some 13 us outside the tile loop (finding the block, three dependent memory round trips, the epilogue)
+// with the compute unit idle.  Instead workgroup r of an XCD's 32 takes the blocks 32 i + r of the order above, or
+// 32 i + 31 - r in odd rounds i, as one stream of key tiles: the moves of a block's first tiles and its Q rows are
+// under way while the block before it is computed, and a change of blocks costs 6.5 K cycles (both wave groups'
+// rows and masks, in turn) beside 2.9 K a tile.  us, 32 / 8 heads unless said: prompts of 771-2710 tokens (11574 in
+// all) 249.8 -> 235.3, 30 x 100-300 on up to 500 cached 83.9 -> 74.9, 16 x 50-2000 at 64 / 8 heads 408 -> 370, three
+// of 1000-3000 under a window of 1024 166 -> 149.  A wave without rows computes all the same here (a loop of its own
+// costs 260 bytes of spills), and of few rounds the last ones are short: with 2 rounds (4 x 200-900) 33.1 -> 34.8,
+// with 3 (12 x 100-1000, 16 / 8 heads) 39.3 -> 40.9, with 4 (20 x 33-257 on 8 K, both sides) 281 -> 279: from 4 on.
+// The list of a workgroup's blocks is in LDS, hence the other limit; an XCD's workgroups work on one kv head (the
+// bases of the moves stay the same).
+constexpr int kMinRounds = 4, kMaxRounds = 64;
+
 // Gang ranges, for launches with several query blocks per (request, kv head) (chunked extends on
 // long prefixes: their cost is the MFMA work, and it differs from unit to unit with the prefix).
 // One workgroup per compute unit stays for the whole launch.  The 32 workgroups on an XCD form
@@ -269,6 +287,10 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
   p.gang_nonce = 0;
   p.length_heads = 0;
   p.length_log2_xcds = 0;
+  p.length_rounds = 0;
+  p.group_shift = 0;
+  while ((1u << p.group_shift) < (uint32_t)p.group) ++p.group_shift;
+  p.group_magic = (uint32_t)(((1ull << (31 + p.group_shift)) + p.group - 1) / p.group);
   p.clock_probe = clock_probe();
   if (a.ragged_tiles > 0 && n_qblk == 1) {
     const int64_t units = prefill_ragged_units(a.batch, a.total_kv, a.ragged_tiles);
@@ -321,6 +343,11 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     const int64_t xcds = 1 << p.length_log2_xcds;
     n_blocks = 8 * a.batch * p.length_heads * ((n_qblk + xcds - 1) / xcds);
     if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
+    const int64_t rounds = (n_blocks + kComputeUnits - 1) / kComputeUnits;
+    if (block_rows == kPrefillBlockRows && p.length_heads == 1 && rounds >= kMinRounds && rounds <= kMaxRounds) {
+      p.length_rounds = (int32_t)rounds;
+      n_blocks = kComputeUnits;
+    }
   }
   // narrow offsets: slot * row_bytes fits 32 bits and both factors fit 24 bits (one
   // full-rate 24-bit multiply per row)

@@ -59,6 +59,12 @@ __device__ __forceinline__ u32x2_t lds_read_tr16(const unsigned char* p) {
   return __builtin_bit_cast(u32x2_t, v);
 }
 
+// row / group, a multiplication: with 2^shift the power of two that holds the group, magic = ceil(2^(31 + shift) / group)
+// has 32 bits and the quotient is exact for rows below 2^31 (a division is 35 instructions).
+__device__ __forceinline__ int row_to_query(const PrefillParams& p, int row) {
+  return (int)(__umulhi((uint32_t)row << 1, p.group_magic) >> p.group_shift);
+}
+
 // Workgroup id -> (unit = (request rank, kv head, key split), query block), heaviest query block
 // (latest rows) first; `ok` is false for the ids that pad the grid.  Consecutive ids go to
 // different XCDs.
@@ -103,66 +109,73 @@ struct LengthBlock {
   bool ok;
 };
 template <int ROWS>
-__device__ __forceinline__ LengthBlock block_by_length(const PrefillParams& p) {
-  const int lane = lane_id();
-  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-  const int heads_across = min(p.n_kv, 8);
-  const int part = xcd / heads_across, mask = (1 << p.length_log2_xcds) - 1;
-  // the lane's request
-  int q_start = 0, q_len = 0, kv_start = 0, kv_len = 0, prefix = 0;
-  if (lane < p.batch) {
-    q_start = p.qo_indptr[lane];
-    q_len = p.qo_indptr[lane + 1];
-    kv_start = p.kv_indptr[lane];
-    kv_len = p.kv_indptr[lane + 1];
-    prefix = p.prefix_lens[lane];
+struct LengthOrder {
+  const PrefillParams& p;
+  int xcd, q_start, q_len, kv_start, kv_len, prefix;  // the lane's request
+  int rows, kn, first_of, blocks, in_all, longest, shift;
+  __device__ __forceinline__ explicit LengthOrder(const PrefillParams& params) : p(params) {
+    const int lane = lane_id();
+    xcd = blockIdx.x & 7;
+    const int heads_across = min(p.n_kv, 8);
+    const int part = xcd / heads_across, mask = (1 << p.length_log2_xcds) - 1;
+    q_start = q_len = kv_start = kv_len = prefix = 0;
+    if (lane < p.batch) {
+      q_start = p.qo_indptr[lane];
+      q_len = p.qo_indptr[lane + 1];
+      kv_start = p.kv_indptr[lane];
+      kv_len = p.kv_indptr[lane + 1];
+      prefix = p.prefix_lens[lane];
+    }
+    q_len = min(q_len - q_start, p.max_len_extend);
+    kv_len = max(kv_len - kv_start, 0);
+    rows = q_len * p.group;
+    kn = min(kv_len, p.window > 0 ? p.window + ROWS / p.group + 1 : 0x7fffffff);
+    first_of = (part + lane) & mask;  // this XCD's blocks: first_of, first_of + XCDs per head, ...
+    blocks = rows > 0 ? (rows + ROWS - 1) / ROWS : 0;
+    in_all = in_class(blocks);
+    longest = wave_max(kn);
+    // 4 to 8 steps, whole key tiles; two tiles where a workgroup's blocks are laid down (see kMaxRounds)
+    shift = p.length_rounds > 0 ? 7 : max(31 - __builtin_clz(max(longest, 1)) - 2, 6);
   }
-  q_len = min(q_len - q_start, p.max_len_extend);
-  kv_len = max(kv_len - kv_start, 0);
-  const int rows = q_len * p.group;
-  const int kn = min(kv_len, p.window > 0 ? p.window + ROWS / p.group + 1 : 0x7fffffff);
-  const int first_of = (part + lane) & mask;  // this XCD's blocks: first_of, first_of + XCDs per head, ...
-  const int blocks = rows > 0 ? (rows + ROWS - 1) / ROWS : 0;
-  auto in_class = [&](int below) {  // this XCD's blocks among the first `below`
+  __device__ __forceinline__ int in_class(int below) const {  // this XCD's blocks among the first `below`
     return below > first_of ? ((below - first_of - 1) >> p.length_log2_xcds) + 1 : 0;
-  };
-  const int in_all = in_class(blocks);
-  const int longest = wave_max(kn);
-  const int shift = max(31 - __builtin_clz(max(longest, 1)) - 2, 6);  // 4 to 8 steps, whole key tiles
-  // this XCD's blocks of the request of at least `steps` steps
-  auto at_least = [&](int steps) {
+  }
+  __device__ __forceinline__ int at_least(int steps) const {  // this XCD's blocks of the request of at least `steps` steps
     if (steps <= 0) return in_all;
     const int keys = ((steps - 1) << shift) + 1;
     const int row = p.is_cross ? 0 : max(keys - 1 - prefix, 0) * p.group;  // first row that sees so many
     return in_all - in_class(kn >= keys && row < rows ? row / ROWS : blocks);
-  };
-  auto count = [&](int steps) { return wave_sum(at_least(steps)) * p.length_heads; };
-  LengthBlock w{};
-  // count(lo) > seq >= count(hi)
-  int lo = 0, hi = (longest >> shift) + 2;
-  if (seq >= count(0)) return w;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (count(mid) > seq) lo = mid;
-    else hi = mid;
   }
-  const int longer = at_least(lo + 1), equal = (at_least(lo) - longer) * p.length_heads;
-  const int left = seq - wave_sum(longer) * p.length_heads;  // its number among the blocks of exactly `lo` steps
-  const int incl = wave_inclusive_scan(equal), before = incl - equal;
-  const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(left >= before && left < incl)) - 1);
-  const int mine = left - __builtin_amdgcn_readlane(before, src);
-  const int from_top = __builtin_amdgcn_readlane(longer, src) + mine / p.length_heads;
-  w.b = src;
-  w.kvh = xcd % heads_across + 8 * (mine % p.length_heads);
-  w.qblk = __builtin_amdgcn_readlane(first_of, src) + ((__builtin_amdgcn_readlane(in_all, src) - 1 - from_top) << p.length_log2_xcds);
-  w.q_start = __builtin_amdgcn_readlane(q_start, src);
-  w.q_len = __builtin_amdgcn_readlane(q_len, src);
-  w.kv_start = __builtin_amdgcn_readlane(kv_start, src);
-  w.kv_len = __builtin_amdgcn_readlane(kv_len, src);
-  w.prefix = __builtin_amdgcn_readlane(prefix, src);
-  w.ok = true;
-  return w;
-}
+  __device__ __forceinline__ int count(int steps) const { return wave_sum(at_least(steps)) * p.length_heads; }
+  // Block number `seq` of the XCD.
+  __device__ __forceinline__ LengthBlock find(int seq) const {
+    LengthBlock w{};
+    // count(lo) > seq >= count(hi)
+    int lo = 0, hi = (longest >> shift) + 2;
+    if (seq >= count(0)) return w;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (count(mid) > seq) lo = mid;
+      else hi = mid;
+    }
+    const int longer = at_least(lo + 1), equal = (at_least(lo) - longer) * p.length_heads;
+    const int left = seq - wave_sum(longer) * p.length_heads;  // its number among the blocks of exactly `lo` steps
+    const int incl = wave_inclusive_scan(equal), before = incl - equal;
+    const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(left >= before && left < incl)) - 1);
+    const int mine = left - __builtin_amdgcn_readlane(before, src);
+    const int from_top = __builtin_amdgcn_readlane(longer, src) + mine / p.length_heads;
+    w.b = src;
+    w.kvh = xcd % min(p.n_kv, 8) + 8 * (mine % p.length_heads);
+    w.qblk = __builtin_amdgcn_readlane(first_of, src) + ((__builtin_amdgcn_readlane(in_all, src) - 1 - from_top) << p.length_log2_xcds);
+    w.q_start = __builtin_amdgcn_readlane(q_start, src);
+    w.q_len = __builtin_amdgcn_readlane(q_len, src);
+    w.kv_start = __builtin_amdgcn_readlane(kv_start, src);
+    w.kv_len = __builtin_amdgcn_readlane(kv_len, src);
+    w.prefix = __builtin_amdgcn_readlane(prefix, src);
+    w.ok = true;
+    return w;
+  }
+};
 
 // ---- ragged shares: which (request, share) is unit `u`? ------------------------------------------
 // Visible key range of a request's only query block (rows 0 .. q_len * group - 1), the floor
