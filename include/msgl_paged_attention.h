@@ -151,12 +151,13 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
                                 int32_t dtype, void* stream);
 
 /*
- * A decode step's store and attention in one launch -- AttnBackend.forward for decode metadata
+ * A decode step's store inside its attention -- AttnBackend.forward for decode metadata
  * (mini_sglang_mlx/attention/backend.py:129-172): what msgl_store_kv_cache on (k, v, out_loc) and
  * msgl_paged_decode_attention behind it do or, with norm weights (bf16 only),
  * msgl_qk_norm_rope_store and msgl_paged_decode_attention (models/qwen3.py:60-68 in front of them).
- * For small launches: msgl_decode_step_workspace_bytes is 0 where two launches are the better way,
- * and msgl_decode_step refuses those sizes (MSGL_ERR_SHAPE).
+ * msgl_decode_step_workspace_bytes is 0 where the calls one by one are the better way (norm weights on
+ * large launches: `norm_rope` says whether there are weights), and msgl_decode_step refuses those sizes
+ * (MSGL_ERR_SHAPE).
  *   q (batch, num_q_heads, head_dim); k, v (batch, num_kv_heads, head_dim); leading strides free
  *   q_weight, k_weight (head_dim) or both NULL; positions (batch), of no use without weights
  *   out_loc (batch): the slot of request b's row, which as a rule is the last one listed for it in
@@ -167,7 +168,8 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
  * the row is there: such a step takes the two calls.
  */
 MSGL_API size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads,
-                                                 int64_t num_kv_heads, int64_t head_dim);
+                                                 int64_t num_kv_heads, int64_t head_dim,
+                                                 int32_t norm_rope);
 MSGL_API int msgl_decode_step(const void* q, const void* k, const void* v,
                               int64_t q_stride0, int64_t k_stride0, int64_t v_stride0,
                               const void* q_weight, const void* k_weight,

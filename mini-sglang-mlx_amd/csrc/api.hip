@@ -263,7 +263,7 @@ static int decode_attention(const void* q, const void* k_cache, const void* v_ca
   a.n_seg = n_seg;
   a.min_seg = min_segment(head_dim);
   if (shares) return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
-  return msgl::launch_splitkv(a, static_cast<hipStream_t>(stream));
+  return msgl::launch_splitkv(a, tokens, static_cast<hipStream_t>(stream));
 }
 
 int msgl_paged_decode_attention(const void* q, const void* k_cache, const void* v_cache,
@@ -294,14 +294,16 @@ int msgl_paged_decode_attention_noalloc(const void* q, const void* k_cache, cons
 }
 
 size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads, int64_t num_kv_heads,
-                                        int64_t head_dim) {
+                                        int64_t head_dim, int32_t norm_rope) {
   if (batch <= 0 || total_kv < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
       num_q_heads / num_kv_heads > 16 || (head_dim != 128 && head_dim != 256))
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
   const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
-  if (!msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) return 0;
-  return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
+  // norm and rotary embedding would be made anew by every segment of a request: 3.5 us of a launch of their own is
+  // less on the launches that go in segments
+  if (norm_rope && !msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) return 0;
+  return msgl_paged_decode_workspace_bytes(batch, total_kv, num_q_heads, num_kv_heads, head_dim);
 }
 
 int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stride0, int64_t k_stride0, int64_t v_stride0,
@@ -326,9 +328,8 @@ int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stri
   if (!aligned16(k) || !aligned16(v) || q_stride0 % 8 || k_stride0 % 8 || v_stride0 % 8 || !aligned16(q_weight) ||
       !aligned16(k_weight))
     return MSGL_ERR_ALIGNMENT;
-  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
-  if (!msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) return MSGL_ERR_SHAPE;
-  const size_t need = msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, group);
+  const size_t need = msgl_decode_step_workspace_bytes(batch, total_kv, num_q_heads, num_kv_heads, head_dim, q_weight != nullptr);
+  if (need == 0) return MSGL_ERR_SHAPE;
   if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;
   msgl::SplitKvArgs a{};
   a.q = q;
@@ -361,7 +362,12 @@ int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stri
   tokens.v_stride0 = v_stride0;
   tokens.eps = rms_norm_eps;
   tokens.rope_base = rope_base;
-  return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
+  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  if (msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group))
+    return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
+  a.n_seg = segments(total_kv, num_kv_heads, head_dim, group);
+  a.min_seg = min_segment(head_dim);
+  return msgl::launch_splitkv(a, tokens, static_cast<hipStream_t>(stream));
 }
 
 // Ragged key shares for the tile kernels (one query block per (request, kv head)): the ping-pong
@@ -507,7 +513,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     a.min_seg = min_segment(head_dim);
     a.q_begin = 0;
     if (shares) return msgl::launch_shares(a, msgl::NewTokens{}, plan, s);
-    return msgl::launch_splitkv(a, s);
+    return msgl::launch_splitkv(a, msgl::NewTokens{}, s);
   }
   msgl::PrefillArgs a{};
   a.q = q;

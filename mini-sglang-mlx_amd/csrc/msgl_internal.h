@@ -41,6 +41,19 @@ struct SplitKvArgs {
   int32_t min_seg;  // smallest segment length in tokens, multiple of 64
   int64_t q_stride0;  // elements from one row of q to the next (0: n_q * head_dim)
 };
+// What a decode step's own tokens bring: request b's new row of k and v, stored at slot out_loc[b] and taken from
+// here instead of the pool where the request's last slot is that one.  With norm weights (bf16 only) q and k are
+// normalised and rotated first.
+struct NewTokens {
+  const void* k;  // nullptr: the pool holds every row already
+  const void* v;
+  const void* q_weight;  // nullptr: q and k as they are
+  const void* k_weight;
+  const int32_t* positions;
+  const int32_t* out_loc;
+  int64_t k_stride0, v_stride0;  // elements
+  float eps, rope_base;
+};
 // largest q_len * group the split-K kernel is instantiated for
 constexpr int kSplitKvMaxCols = 64;
 constexpr int kSplitKvMinSegment = 128;
@@ -51,7 +64,7 @@ int splitkv_default_segments(int64_t total_kv, int64_t n_kv, int64_t head_dim, i
 void splitkv_set_boundary(int v);
 size_t splitkv_workspace_bytes(int64_t batch, int64_t n_q, int64_t n_kv, int64_t head_dim,
                                int64_t max_len_extend, int32_t n_seg);
-int launch_splitkv(const SplitKvArgs& a, hipStream_t stream);
+int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream);  // n without norm weights
 // Address (on the current device) and size of the library's built-in split-K scratch, for the
 // entry point that takes no workspace.  The first call on a device resolves the address.
 int splitkv_scratch(void** ptr, size_t* bytes);
@@ -74,19 +87,6 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv);
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols);
 int device_cus();  // paged_splitkv.hip
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);
-// What a decode step's own tokens bring: request b's new row of k and v, stored at slot out_loc[b] and taken from
-// here instead of the pool where the request's last slot is that one.  With norm weights (bf16 only) q and k are
-// normalised and rotated first.
-struct NewTokens {
-  const void* k;  // nullptr: the pool holds every row already
-  const void* v;
-  const void* q_weight;  // nullptr: q and k as they are
-  const void* k_weight;
-  const int32_t* positions;
-  const int32_t* out_loc;
-  int64_t k_stride0, v_stride0;  // elements
-  float eps, rope_base;
-};
 int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& plan, hipStream_t stream);
 // benchmarking switch: 0 default, negative never, else share_len | heads_wg << 20
 void shares_force(int64_t v);

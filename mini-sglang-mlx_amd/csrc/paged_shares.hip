@@ -20,23 +20,15 @@
 //   launch number << 16 | shares done; any other word counts as zero, so the workspace
 //   needs no clearing (launch_number.h: why no data is taken for one), and the last share puts the word back to zero, so a captured launch replays.
 //
-// The new tokens of a decode step (NEW)
-//   A step's own row of k and v goes into the pool in this launch too, by the wave whose range holds its request's
-//   last key.  That wave takes the row from its source and not from the pool, so nobody waits for the
-//   store: while its first tile is under way the new key makes the first state of the columns, and the walk
-//   ends in front of it.  (Put into the tile that the walk computes last, it cost registers: 124 bytes of
-//   spills and 6 us at head_dim 256.)  With norm weights every wave normalises and rotates its own q heads (and that
-//   one the new key) at that time, four heads at once: a lane finds sine and cosine of one or two of the head's
-//   angles and the wave exchanges them through LDS.  (At head_dim 256 all that goes in front of the first tile: there
-//   are no registers for both.)  Norm, rotary embedding, store and attention of 4 requests of 36-1022 tokens, 16 / 8
-//   heads: 3.5 + 8.9 us in two launches, 9.8 in one, and one launch's host time less (28 layers 359 -> 281 us); store and
-//   attention of 24 requests of 127-4095, 16 / 2 heads of 256: 4.5 + 25.0 us, 26.0 in one.
+// A decode step's new tokens (NEW) are stored here, normalised and rotated before where the step asks for that
+//   (new_token.h), instead of by a launch in front.  Norm, rotary embedding, store and attention of 4 requests of
+//   36-1022 tokens, 16 / 8 heads: 3.5 + 8.9 us in two launches, 9.8 in one, and one launch's host time less (28 layers
+//   359 -> 281 us); store and attention of 24 requests of 127-4095, 16 / 2 heads of 256: 4.5 + 25.0 us, 26.0 in one.
 #include <algorithm>
 #include <cmath>
 
 #include "launch_number.h"
-#include "norm_rope.h"
-#include "splitkv_tiles.h"
+#include "new_token.h"
 
 namespace msgl {
 namespace {
@@ -46,22 +38,7 @@ struct ShareParams {
   unsigned long long* counts;  // [batch][head_groups]
   unsigned long long nonce;
   int32_t share_len, share_waves, heads_wg, head_groups;
-  // the step's new tokens (NEW kernels only)
-  const uint16_t* new_k;
-  const uint16_t* new_v;
-  const uint16_t* q_weight;
-  const uint16_t* k_weight;
-  const int32_t* positions;
-  const int32_t* out_loc;
-  uint16_t* k_pool;
-  uint16_t* v_pool;
-  int64_t new_k_stride0, new_v_stride0;
-  float eps, log2_base;
 };
-
-// What a decode launch does with its requests' new tokens: they are in the pool already; they are stored; q and k
-// are normalised and rotated, k and v stored.
-enum NewMode { kStored = 0, kStore = 1, kNormRopeStore = 2 };
 
 __device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
   return (unsigned long long)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo);
@@ -109,163 +86,6 @@ __device__ __forceinline__ bool find_share(const SplitKvParams& p, int share_len
   }
   return false;
 }
-
-// A decode step's new token for a wave.
-template <int D>
-struct HeadLds {  // NORM: of one wave
-  uint16_t row[17][D];  // the new key, the heads of the columns
-  float cosines[D / 2], sines[D / 2];
-};
-template <int D, bool NORM, bool F16>
-struct NewToken {
-  static constexpr int E = D / 32, KS = D / 32, VH = D / 128;
-  // the rows of k and v are asked for in front of the first tile where they fit the registers beside it
-  static constexpr bool kRowsAhead = true;
-  static constexpr int kEarly = 2;  // trips of four heads whose rows are asked for before the first tile
-  using Half = typename HalfRow<E>::type;
-  const ShareParams& sp;
-  Columns<D, 1>& columns;
-  HeadLds<D>& lds;
-  const uint16_t* q;  // the first of the columns' heads
-  const uint16_t *k, *v;
-  bool owner;         // the request's last key is this wave's (in a request without keys: the wave stores the rows)
-  bool seen;          // and that key is the new token
-  int kvh;
-  int before;         // slot id of the key in front of the last
-  uint32_t slot;
-  float position;
-  u32x4_t krow[KS], vrow[VH][4];  // lane group g: dims 32 c + 8 g .. (as operand), hf 128 + 32 g + 8 i .. (as output)
-  Half lo[kEarly], hi[kEarly], qwl, qwh, kwl, kwh;
-
-  __device__ __forceinline__ NewToken(const ShareParams& s, const ReqInfo& r, Columns<D, 1>& c, HeadLds<D>& l, int b, int head, bool own)
-      : sp(s), columns(c), lds(l), owner(own), kvh(head) {
-    const int lane = lane_id();
-    // one round trip for all three, beside that of the first tile's slot ids
-    const int32_t *loc = sp.out_loc + b, *last = r.kv_len > 0 ? sp.s.kv_indices + r.kv_start + r.kv_len - 1 : loc;
-    const int32_t* second = r.kv_len > 1 ? last - 1 : last;
-    slot = (uint32_t)*loc;
-    const uint32_t last_id = (uint32_t)*last;
-    before = *second;
-    seen = owner & (r.kv_len > 0) & (slot <= sp.s.max_slot) & (last_id == slot);
-    q = sp.s.q + (int64_t)b * sp.s.q_stride0 + kvh * sp.s.group * D;
-    k = sp.new_k + (int64_t)b * sp.new_k_stride0 + kvh * D;
-    if constexpr (NORM) {
-      position = (float)sp.positions[b];
-#pragma unroll
-      for (int i = 0; i < kEarly; ++i) head_of(i, lo[i], hi[i]);
-      const int off = E * (lane & 15);
-      qwl = *reinterpret_cast<const Half*>(sp.q_weight + off);
-      qwh = *reinterpret_cast<const Half*>(sp.q_weight + D / 2 + off);
-      kwl = *reinterpret_cast<const Half*>(sp.k_weight + off);
-      kwh = *reinterpret_cast<const Half*>(sp.k_weight + D / 2 + off);
-    }
-    v = sp.new_v + (int64_t)b * sp.new_v_stride0 + kvh * D;
-    if (kRowsAhead && owner) rows();
-  }
-  __device__ __forceinline__ void rows() {
-    const int g = lane_id() >> 4;
-#pragma unroll
-    for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) vrow[hf][i] = ld_global_b128(v + hf * 128 + g * 32 + i * 8);
-    if constexpr (!NORM) {
-#pragma unroll
-      for (int c = 0; c < KS; ++c) krow[c] = ld_global_b128(k + c * 32 + g * 8);
-    }
-  }
-
-  // Row 0 is the new key, row n the head of column n - 1; four rows a trip, 16 lanes each (past the last: the last).
-  __device__ __forceinline__ int row_of(int trip) const { return min(4 * trip + (lane_id() >> 4), sp.s.group); }
-  __device__ __forceinline__ void head_of(int trip, Half& l, Half& h) const {
-    const int row = row_of(trip);
-    const uint16_t* src = (row == 0 ? k : q + (row - 1) * D) + E * (lane_id() & 15);
-    l = *reinterpret_cast<const Half*>(src);
-    h = *reinterpret_cast<const Half*>(src + D / 2);
-  }
-  // The wave's own writes to LDS before its reads: no barrier
-  __device__ __forceinline__ static void own_writes() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-  __device__ __forceinline__ void normalise() {
-    const int lane = lane_id(), t16 = lane & 15, g = lane >> 4, off = E * t16;
-#pragma unroll
-    for (int i = lane; i < D / 2; i += kWave) {
-      float sn, cs;
-      sincosf(rope_angle<D>(position, i, sp.log2_base), &sn, &cs);
-      lds.cosines[i] = cs;
-      lds.sines[i] = sn;
-    }
-    own_writes();
-    float cs[E], sn[E];
-#pragma unroll
-    for (int e = 0; e < E; e += 4) {
-      *reinterpret_cast<f32x4_t*>(cs + e) = *reinterpret_cast<const f32x4_t*>(&lds.cosines[off + e]);
-      *reinterpret_cast<f32x4_t*>(sn + e) = *reinterpret_cast<const f32x4_t*>(&lds.sines[off + e]);
-    }
-    auto trip = [&](int i, Half l, Half h) {
-      const int row = row_of(i);
-      norm_rope_head<D>(l, h, row == 0 ? kwl : qwl, row == 0 ? kwh : qwh, cs, sn, sp.eps);
-      *reinterpret_cast<Half*>(&lds.row[row][off]) = l;
-      *reinterpret_cast<Half*>(&lds.row[row][off + D / 2]) = h;
-    };
-    trip(0, lo[0], hi[0]);
-    if (sp.s.group >= 4) trip(1, lo[1], hi[1]);
-    for (int i = kEarly; 4 * i <= sp.s.group; ++i) {
-      Half l, h;
-      head_of(i, l, h);
-      trip(i, l, h);
-    }
-    own_writes();
-#pragma unroll
-    for (int c = 0; c < KS; ++c) {
-      krow[c] = *reinterpret_cast<const u32x4_t*>(&lds.row[0][c * 32 + g * 8]);
-      if (t16 < sp.s.group) columns.q[0][c] = *reinterpret_cast<const u32x4_t*>(&lds.row[t16 + 1][c * 32 + g * 8]);
-    }
-  }
-
-  static __device__ __forceinline__ float value(uint32_t pair, int e) {
-    if constexpr (F16) return (float)__builtin_bit_cast(f16x2_t, pair)[e];
-    else return __builtin_bit_cast(float, e ? pair & 0xffff0000u : pair << 16);
-  }
-
-  __device__ __forceinline__ void operator()() {
-    __builtin_amdgcn_sched_barrier(0);
-    run();
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  __device__ __forceinline__ void run() {
-    if (!kRowsAhead && owner) rows();
-    if constexpr (NORM) normalise();
-    if (!owner) return;
-    const int lane = lane_id(), t16 = lane & 15, g = lane >> 4;
-    if (seen) {  // the columns' first key: its score the maximum, its weight 1
-      float score = 0.f;
-#pragma unroll
-      for (int c = 0; c < KS; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          score = __builtin_fmaf(value(columns.q[0][c][e >> 1], e & 1), value(krow[c][e >> 1], e & 1), score);
-      columns.m[0] = sum_across<32>(sum_across<16>(score)) * sp.s.scale_log2e;
-      columns.l[0] = g == 0 ? 1.f : 0.f;
-#pragma unroll
-      for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int n = 0; n < 8; ++n) columns.o[0][hf][n][i] = value(vrow[hf][i][n >> 1], n & 1);
-    }
-    if (slot > sp.s.max_slot) return;  // a slot id outside the pool stores nothing
-    if (t16 == 0) {
-      uint16_t* to_k = sp.k_pool + (int64_t)slot * sp.s.k_stride0 + kvh * D + g * 8;
-      uint16_t* to_v = sp.v_pool + (int64_t)slot * sp.s.v_stride0 + kvh * D + g * 32;
-#pragma unroll
-      for (int c = 0; c < KS; ++c) st_global_b128(to_k + c * 32, krow[c]);
-#pragma unroll
-      for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) st_global_b128(to_v + hf * 128 + i * 8, vrow[hf][i]);
-    }
-  }
-};
 
 template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
 __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(ShareParams sp) {
@@ -318,17 +138,11 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     static_assert(sizeof(HeadLds<D>) <= sizeof(part[0]), "a wave's heads have their place in its part of the partials");
     const int tail = r.kv_len - 1;
     const bool owner = r.kv_len > 0 ? t_begin <= tail && tail < t_end : share == 0 && sw == 0;
-    NewToken<D, NEW == kNormRopeStore, F16> token(sp, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), b, kvh, owner);
+    NewToken<D, NEW == kNormRopeStore, F16> token(p, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), b, kvh, owner);
     int walk_end = t_end;
     if (token.seen) {
-      // the walk ends in front of the new token, whose place in the pool is read by nobody (the last tile's rows
-      // repeat the last key walked; what has weight 0 still has to be a number)
       walk_end = tail;
-      const int at = t_begin + t16;
-      if (at >= tail) ids.a[0] = token.before;
-      if (at + 16 >= tail) ids.a[1] = token.before;
-      if (at + 32 >= tail) ids.b[0] = token.before;
-      if (at + 48 >= tail) ids.b[1] = token.before;
+      end_ids(ids, t_begin, tail, token.before);
     }
     start_columns<D, NCT, NEW != kNormRopeStore>(p, r, kvh, 0, walk_end, c);
     if constexpr (D == 256) {
@@ -495,7 +309,7 @@ int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
     return check_launch();
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
-    const int mode = sp.new_k == nullptr ? kStored : sp.q_weight == nullptr ? kStore : kNormRopeStore;
+    const int mode = sp.s.nt.k == nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
     if (sp.s.f16) {
       if (mode == kStored)
         return launch(share_attention_kernel<D, NCT, NW, false, true, kStored>, share_attention_kernel<D, NCT, NW, true, true, kStored>);
@@ -509,7 +323,7 @@ int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
       return launch(share_attention_kernel<D, NCT, NW, false, false, kNormRopeStore>,
                     share_attention_kernel<D, NCT, NW, true, false, kNormRopeStore>);
   }
-  if (sp.s.f16 || sp.new_k != nullptr) return MSGL_ERR_DTYPE;
+  if (sp.s.f16 || sp.s.nt.k != nullptr) return MSGL_ERR_DTYPE;
   return launch(share_attention_kernel<D, NCT, NW, false, false, kStored>, share_attention_kernel<D, NCT, NW, true, false, kStored>);
 }
 
@@ -607,20 +421,7 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   sp.share_waves = plan.share_waves;
   sp.heads_wg = plan.heads_wg;
   sp.head_groups = (int32_t)head_groups;
-  if (n.k != nullptr) {
-    sp.new_k = static_cast<const uint16_t*>(n.k);
-    sp.new_v = static_cast<const uint16_t*>(n.v);
-    sp.q_weight = static_cast<const uint16_t*>(n.q_weight);
-    sp.k_weight = static_cast<const uint16_t*>(n.k_weight);
-    sp.positions = n.positions;
-    sp.out_loc = n.out_loc;
-    sp.k_pool = const_cast<uint16_t*>(sp.s.k_cache);
-    sp.v_pool = const_cast<uint16_t*>(sp.s.v_cache);
-    sp.new_k_stride0 = n.k_stride0;
-    sp.new_v_stride0 = n.v_stride0;
-    sp.eps = n.eps;
-    sp.log2_base = n.q_weight ? log2f(n.rope_base) : 0.f;
-  }
+  fill_new_tokens(n, sp.s);
   const int nct = nct_of(cols);
   if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
   if (nct == 1) return launch_shape<128, 1, 8>(sp, (unsigned)blocks, stream);

@@ -41,7 +41,7 @@
 #include <atomic>
 #include <type_traits>
 
-#include "splitkv_tiles.h"
+#include "new_token.h"
 
 namespace msgl {
 namespace {
@@ -147,7 +147,8 @@ __device__ __forceinline__ bool locate_segment(const SplitKvParams& p, int seg, 
 // column tile at head dim 128 fits 256 VGPRs, so two such waves per SIMD can be resident.
 // WIDE: pool byte offsets need 64 bits (a pool of 4 GiB or more); otherwise a row's offset is
 // one 32-bit multiply instead of a 64-bit multiply-add per load.
-template <int D, int NCT, int NW, bool WIDE, bool F16>
+// NEW: a decode step's rows are stored here (kStore), or are in the pool already (kStored).
+template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
 __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void splitkv_attention_kernel(SplitKvParams p) {
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const ClockProbe clock_probe_(p.clock_probe);
@@ -161,6 +162,15 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
   const int ct0 = cw * NCT;     // first of its tiles of 16 columns
   const int kvh = (blockIdx.x - seg * p.head_groups) * p.nwh + (wave - cw * p.nwh);
   int seg_len, total, cur_b, vs;
+  __shared__ __attribute__((aligned(16))) NewRowsLds<D> rows[NW];
+  if (NEW != kStored && seg == 0) {  // requests without keys come up in no segment
+    for (int b0 = 0; b0 < p.batch; b0 += kWave) {
+      const int b = min(b0 + lane, p.batch - 1);
+      unsigned long long empty = __ballot(b0 + lane < p.batch && p.kv_indptr[b + 1] <= p.kv_indptr[b]);
+      for (; empty != 0; empty &= empty - 1)
+        store_new_rows<D>(p, __builtin_amdgcn_readfirstlane(b0 + __ffsll((long long)empty) - 1), kvh);
+    }
+  }
   if (!locate_segment(p, seg, &seg_len, &total, &cur_b, &vs)) return;
   cur_b = __builtin_amdgcn_readfirstlane(cur_b);
   vs = __builtin_amdgcn_readfirstlane(vs);
@@ -188,9 +198,18 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     const int ncols = r.q_len * p.group;
 
     Columns<D, NCT> c_;
-    const FirstIds ids = first_ids(p, r, t_begin, t_end);
-    start_columns(p, r, kvh, ct0, t_end, c_);
-    attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
+    FirstIds ids = first_ids(p, r, t_begin, t_end);
+    if constexpr (NEW == kStored) {
+      start_columns(p, r, kvh, ct0, t_end, c_);
+      attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
+    } else {
+      LateToken<D, F16> token(p, r, rows[wave], cur_b, kvh, t_end == r.hi);
+      const int walk_end = token.seen ? t_end - 1 : t_end;
+      if (token.seen) end_ids(ids, t_begin, walk_end, token.before);
+      start_columns(p, r, kvh, ct0, walk_end, c_);
+      if (t_begin < walk_end) attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, walk_end, ids, c_, [] {});
+      token.finish(c_, kvh, t_begin < walk_end);
+    }
 
     // ---- this request's share is done: write output or partial -------------------------
 #pragma unroll
@@ -451,21 +470,23 @@ int heads_per_group(int64_t n_kv) {
 
 template <int D, int NCT, int NW>
 void launch_attn(const SplitKvParams& p, hipStream_t stream) {
-  const dim3 grid((unsigned)(p.n_seg * p.head_groups)), block(64 * NW);
-  if constexpr (NCT == 1) {  // IEEE half exists for decode only (one column tile)
-    if (p.f16) {
-      if (p.wide) hipLaunchKernelGGL((splitkv_attention_kernel<D, NCT, NW, true, true>), grid, block, 0, stream, p);
-      else hipLaunchKernelGGL((splitkv_attention_kernel<D, NCT, NW, false, true>), grid, block, 0, stream, p);
-      return;
-    }
+  auto launch = [&](auto narrow, auto wide) {
+    hipLaunchKernelGGL(p.wide ? wide : narrow, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), 0, stream, p);
+  };
+  if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
+    if (p.nt.k != nullptr && p.f16)
+      return launch(splitkv_attention_kernel<D, NCT, NW, false, true, kStore>, splitkv_attention_kernel<D, NCT, NW, true, true, kStore>);
+    if (p.nt.k != nullptr)
+      return launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStore>, splitkv_attention_kernel<D, NCT, NW, true, false, kStore>);
+    if (p.f16)
+      return launch(splitkv_attention_kernel<D, NCT, NW, false, true, kStored>, splitkv_attention_kernel<D, NCT, NW, true, true, kStored>);
   }
-  if (p.wide) hipLaunchKernelGGL((splitkv_attention_kernel<D, NCT, NW, true, false>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((splitkv_attention_kernel<D, NCT, NW, false, false>), grid, block, 0, stream, p);
+  launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStored>, splitkv_attention_kernel<D, NCT, NW, true, false, kStored>);
 }
 
 template <int D, int NCT>
 int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
-  if (p.f16 && NCT != 1) return MSGL_ERR_DTYPE;
+  if ((p.f16 || p.nt.k != nullptr) && NCT != 1) return MSGL_ERR_DTYPE;
   switch (waves) {
     case 1: launch_attn<D, NCT, 1>(p, stream); break;
     case 2: launch_attn<D, NCT, 2>(p, stream); break;
@@ -652,7 +673,7 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
             (uint64_t)a.num_slots * (uint64_t)a.v_stride0 * 2u >= (1ull << 32)) ? 1 : 0;
 }
 
-int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
+int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream) {
   const int64_t cols = a.n_q / a.n_kv * a.max_len_extend;
   if (cols < 1 || cols > kSplitKvMaxCols || a.n_seg < 1 || a.min_seg < 64 || a.min_seg % 64 != 0)
     return MSGL_ERR_SHAPE;
@@ -663,6 +684,8 @@ int launch_splitkv(const SplitKvArgs& a, hipStream_t stream) {
 
   SplitKvParams p{};
   fill_splitkv_params(a, p);
+  fill_new_tokens(n, p);
+  if (p.nt.q_weight != nullptr) return MSGL_ERR_SHAPE;  // norm and rotary embedding are the shares' alone
   const int64_t rows = ((int64_t)a.n_seg + a.batch) * a.n_kv * cols;
   char* ws = static_cast<char*>(a.workspace);
   p.part_o = reinterpret_cast<float*>(ws);

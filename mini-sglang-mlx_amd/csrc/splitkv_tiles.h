@@ -33,6 +33,13 @@ struct SplitKvParams {
   uint32_t max_slot;  // num_slots - 1: slot ids are clamped to it before they become addresses
   float scale_log2e;
   long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
+  struct {  // a decode step's new tokens (new_token.h); k == nullptr: none
+    const uint16_t *k, *v, *q_weight, *k_weight;
+    const int32_t *positions, *out_loc;
+    uint16_t *k_pool, *v_pool;
+    int64_t k_stride0, v_stride0;
+    float eps, log2_base;
+  } nt;
 };
 
 // Everything but the workspace pointers and the cut (paged_splitkv.hip).

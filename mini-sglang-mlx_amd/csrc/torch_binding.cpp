@@ -518,7 +518,7 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* args, Py_ssize_t n_args
 
 // ---- decode_step(q, k, v, q_weight | None, k_weight | None, positions | None, out_loc, k_cache, v_cache, kv_indptr,
 //                  kv_indices, num_kv_splits, sm_scale, eps, rope_base) -> out or None ------------------
-// Store (or norm, rotary embedding and store) and decode attention as one launch, None where that is not the way: the
+// Decode attention with the store (or norm, rotary embedding and store) inside, None where that is not the way: the
 // caller then makes the two calls, which check what is refused here and say why, and take every form.
 PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 15, [](PyObject* const* a) -> PyObject* {
@@ -562,7 +562,7 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       base = static_cast<float>(real(a[14]));
       if (!(base > 1.0f) || !(eps >= 0.0f)) return none();
     }
-    const size_t bytes = msgl_decode_step_workspace_bytes(batch, ix.size(0), n_q, n_kv, d);
+    const size_t bytes = msgl_decode_step_workspace_bytes(batch, ix.size(0), n_q, n_kv, d, norm ? 1 : 0);
     if (bytes == 0) return none();
     const float scale = static_cast<float>(real(a[12]));
     auto stride0 = [](const Tensor& x) { return x.size(0) > 1 ? x.stride(0) : x.size(1) * x.size(2); };

@@ -54,7 +54,7 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64,
          _i64, _i64, _i64, _i64, _f32, _f32, _i32, _vp]),
-    "msgl_decode_step_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "msgl_decode_step_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i32]),
     "msgl_decode_step": (
         ctypes.c_int,
         [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz,

@@ -10,7 +10,7 @@ from mini_sglang_amd_kernel import _lib, decode_step, paged_decode_attention, qk
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # kv lengths, q heads, kv heads, head_dim, share_len, kv heads per workgroup (0: the default cut)
+CASES = [  # kv lengths, q heads, kv heads, head_dim, share_len, kv heads per workgroup (0: the default cut; -1: segments)
     ([1], 16, 8, 128, 0, 0),
     ([37, 128, 500, 1023], 16, 8, 128, 0, 0),
     ([31, 32, 33, 64, 65, 0, 127, 128, 129, 257], 32, 8, 128, 128, 1),
@@ -18,6 +18,11 @@ CASES = [  # kv lengths, q heads, kv heads, head_dim, share_len, kv heads per wo
     ([1 + i % 90 for i in range(150)], 16, 8, 128, 0, 0),
     ([600, 0, 1, 255, 256, 257], 16, 2, 256, 0, 0),
     ([1500, 40, 32], 24, 4, 256, 64, 4),
+    ([0, 31, 32, 33, 64, 65, 0, 127, 128, 129, 257, 0], 32, 8, 128, -1, 9),
+    ([1, 1, 1], 16, 8, 128, -1, 1),
+    ([0, 0], 16, 8, 128, -1, 3),
+    ([1 + i % 90 for i in range(150)], 24, 3, 128, -1, 60),
+    ([2100, 5, 0, 193], 16, 2, 256, -1, 20),
 ]
 
 
@@ -61,7 +66,14 @@ def test_one_launch_is_two(gpu, tuning, lens, n_q, n_kv, d, share, heads, mode):
         w = (1 + 0.2 * torch.randn((2, d), generator=g, device=gpu)).to(dtype)
         pos = torch.tensor([max(n - 1, 0) + 40000 * (i % 3 == 1) for i, n in enumerate(lens)], dtype=torch.int32, device=gpu)
         norm = dict(q_weight=w[0], k_weight=w[1], positions=pos, eps=1e-6, rope_base=1e6)
-    tuning(_lib.TUNE_SHARES, share | heads << 20)
+    if share >= 0:
+        tuning(_lib.TUNE_SHARES, share | heads << 20)
+    elif mode == "norm":
+        pytest.skip("norm weights: shares only")
+    else:  # segments of at least 64 keys
+        tuning(_lib.TUNE_SHARES, -1)
+        tuning(_lib.TUNE_SEGMENTS, heads)
+        tuning(_lib.TUNE_MIN_SEGMENT, 64)
     kc2, vc2 = kc.clone(), vc.clone()
     print(f"decode step {lens[:4]} {n_q}/{n_kv} d{d} {mode} cut {share} x {heads}", flush=True)
     got = decode_step(q, k, v, loc, kc, vc, wl.kv_indptr, wl.kv_indices, wl.num_kv_splits, sm_scale=wl.sm_scale, **norm)
@@ -93,4 +105,5 @@ def test_what_is_left_to_the_two_calls(gpu, monkeypatch):
     monkeypatch.setenv("MSGL_DEBUG_CHECKS", "0")
     assert torch.equal(before.view(torch.int16), kc.view(torch.int16))
     assert decode_step(*args(), sm_scale=0.1) is not None
-    assert _lib.load().msgl_decode_step_workspace_bytes(64, 64 * 4096, 32, 8, 128) == 0
+    need = _lib.load().msgl_decode_step_workspace_bytes
+    assert need(64, 64 * 4096, 32, 8, 128, 0) > 0 and need(64, 64 * 4096, 32, 8, 128, 1) == 0
