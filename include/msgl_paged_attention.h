@@ -155,9 +155,9 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
  * (mini_sglang_mlx/attention/backend.py:129-172): what msgl_store_kv_cache on (k, v, out_loc) and
  * msgl_paged_decode_attention behind it do or, with norm weights (bf16 only),
  * msgl_qk_norm_rope_store and msgl_paged_decode_attention (models/qwen3.py:60-68 in front of them).
- * msgl_decode_step_workspace_bytes is 0 where the calls one by one are the better way (norm weights on
- * large launches: `norm_rope` says whether there are weights), and msgl_decode_step refuses those sizes
- * (MSGL_ERR_SHAPE).
+ * msgl_decode_step_workspace_bytes is 0 where the calls one by one are the better way (large launches, with norm
+ * weights earlier than without: `norm_rope` says whether there are any), and msgl_decode_step refuses those
+ * sizes (MSGL_ERR_SHAPE).
  *   q (batch, num_q_heads, head_dim); k, v (batch, num_kv_heads, head_dim); leading strides free
  *   q_weight, k_weight (head_dim) or both NULL; positions (batch), of no use without weights
  *   out_loc (batch): the slot of request b's row, which as a rule is the last one listed for it in

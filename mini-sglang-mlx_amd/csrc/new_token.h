@@ -205,8 +205,8 @@ struct NewToken {
 // The same without norm weights for the long walks of paged_splitkv.hip, whose two tiles leave no registers for a state
 // in front of them (140 bytes of spills at head_dim 128, 196 at 256): the rows go to LDS by themselves when the walk starts
 // and the new key comes into the state behind it.  Against a store launch in front, us: one request of 29 K keys, 32 / 8
-// heads, 24.2 -> 22.4; two of 408-2260, 24 / 4 heads of 256, 23.3 -> 20.9; 68 of 325-1056, 16 / 8, 38.2 -> 37.0; 64 of
-// 1-8 K, 32 / 8, 225 both.
+// heads, 24.2 -> 22.4; two of 408-2260, 24 / 4 heads of 256, 23.3 -> 20.9; 68 of 325-1056, 16 / 8, 38.2 -> 37.0
+// (larger launches lose: msgl_decode_step_workspace_bytes has the line).
 template <int D>
 struct NewRowsLds {
   uint16_t k[D], v[D];

@@ -769,7 +769,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   int n_listed = 0;
   if constexpr (listed) {
     if (tid == 0) list.count = list.blank = 0;
-    const LengthOrder<kRows> order(p);
+    const LengthOrder<kRows, true> order(p);
     const int r = (int)(blockIdx.x >> 3), rounds = p.length_rounds;
     __syncthreads();
     for (int i = w; i < rounds; i += NW) {

@@ -41,11 +41,11 @@ struct PrefillParams {
   // query blocks in order of length (see prefill_by_length()): kv heads per XCD, 0 = off, and the
   // logarithm of the number of XCDs that share a kv head's blocks
   int32_t length_heads, length_log2_xcds;
+  long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
   // head_dim 128: above 0, one workgroup per compute unit stays for the launch and takes one block in each of
   // this many rounds (see kMaxRounds)
   int32_t length_rounds;
   uint32_t group_magic, group_shift;  // row / group of a row below 2^31: see row_to_query()
-  long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
 };
 
 constexpr int kBN = 64;  // keys per tile

@@ -108,7 +108,8 @@ struct LengthBlock {
   int q_start, q_len, kv_start, kv_len, prefix;
   bool ok;
 };
-template <int ROWS>
+// STAY: see kMaxRounds
+template <int ROWS, bool STAY = false>
 struct LengthOrder {
   const PrefillParams& p;
   int xcd, q_start, q_len, kv_start, kv_len, prefix;  // the lane's request
@@ -116,8 +117,8 @@ struct LengthOrder {
   __device__ __forceinline__ explicit LengthOrder(const PrefillParams& params) : p(params) {
     const int lane = lane_id();
     xcd = blockIdx.x & 7;
-    const int heads_across = min(p.n_kv, 8);
-    const int part = xcd / heads_across, mask = (1 << p.length_log2_xcds) - 1;
+    // the XCDs take 8 >> length_log2_xcds kv heads side by side
+    const int part = xcd >> (3 - p.length_log2_xcds), mask = (1 << p.length_log2_xcds) - 1;
     q_start = q_len = kv_start = kv_len = prefix = 0;
     if (lane < p.batch) {
       q_start = p.qo_indptr[lane];
@@ -134,8 +135,8 @@ struct LengthOrder {
     blocks = rows > 0 ? (rows + ROWS - 1) / ROWS : 0;
     in_all = in_class(blocks);
     longest = wave_max(kn);
-    // 4 to 8 steps, whole key tiles; two tiles where a workgroup's blocks are laid down (see kMaxRounds)
-    shift = p.length_rounds > 0 ? 7 : max(31 - __builtin_clz(max(longest, 1)) - 2, 6);
+    // 4 to 8 steps, whole key tiles; two tiles where a workgroup's blocks are laid down
+    shift = STAY ? 7 : max(31 - __builtin_clz(max(longest, 1)) - 2, 6);
   }
   __device__ __forceinline__ int in_class(int below) const {  // this XCD's blocks among the first `below`
     return below > first_of ? ((below - first_of - 1) >> p.length_log2_xcds) + 1 : 0;
@@ -165,7 +166,7 @@ struct LengthOrder {
     const int mine = left - __builtin_amdgcn_readlane(before, src);
     const int from_top = __builtin_amdgcn_readlane(longer, src) + mine / p.length_heads;
     w.b = src;
-    w.kvh = xcd % min(p.n_kv, 8) + 8 * (mine % p.length_heads);
+    w.kvh = (xcd & ((8 >> p.length_log2_xcds) - 1)) + 8 * (mine % p.length_heads);
     w.qblk = __builtin_amdgcn_readlane(first_of, src) + ((__builtin_amdgcn_readlane(in_all, src) - 1 - from_top) << p.length_log2_xcds);
     w.q_start = __builtin_amdgcn_readlane(q_start, src);
     w.q_len = __builtin_amdgcn_readlane(q_len, src);

@@ -266,7 +266,7 @@ def decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
                 rope_base: float = 0.0) -> Optional[torch.Tensor]:
     """``paged_decode_attention`` of a decode step with ``store_kv_cache`` inside or, with norm weights,
     ``qk_norm_rope_store``: the attention output, or ``None`` (nothing done) where the two calls are
-    the way: norm weights on large launches, forms that need a copy, arguments that they refuse, index
+    the way: large launches, forms that need a copy, arguments that they refuse, index
     validation on.
 
     One new token per request, row ``b`` at slot ``out_loc[b]``.  A slot of ``out_loc`` must not be

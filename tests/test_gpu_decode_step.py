@@ -106,4 +106,5 @@ def test_what_is_left_to_the_two_calls(gpu, monkeypatch):
     assert torch.equal(before.view(torch.int16), kc.view(torch.int16))
     assert decode_step(*args(), sm_scale=0.1) is not None
     need = _lib.load().msgl_decode_step_workspace_bytes
-    assert need(64, 64 * 4096, 32, 8, 128, 0) > 0 and need(64, 64 * 4096, 32, 8, 128, 1) == 0
+    assert need(64, 64 * 4096, 32, 8, 128, 0) == 0  # a large launch
+    assert need(1, 20000, 32, 8, 128, 0) > 0 and need(1, 20000, 32, 8, 128, 1) == 0  # segments: without norm weights
