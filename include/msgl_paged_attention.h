@@ -161,11 +161,10 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
  *   q (batch, num_q_heads, head_dim); k, v (batch, num_kv_heads, head_dim); leading strides free
  *   q_weight, k_weight (head_dim) or both NULL; positions (batch), of no use without weights
  *   out_loc (batch): the slot of request b's row, which as a rule is the last one listed for it in
- *   kv_indices; the request then sees the row itself and not the pool.  A slot outside the pool
- *   stores nothing.
- * The rows are stored by the launch that attends, so a slot of out_loc that is listed anywhere but
- * as its own request's last one (among another request's keys, say) may be read before or after
- * the row is there: such a step takes the two calls.
+ *   kv_indices; the request then sees the row itself and not the pool.  Otherwise the row is in the
+ *   pool before that is read for the request.  A slot outside the pool stores nothing.
+ * The rows are stored by the launch that attends, so a slot of out_loc that is listed for another
+ * request may be read before or after the row is there: such a step takes the two calls.
  */
 MSGL_API size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads,
                                                  int64_t num_kv_heads, int64_t head_dim,
@@ -231,6 +230,38 @@ MSGL_API int msgl_paged_prefill_attention(const void* q, const void* k_cache, co
                                  float sm_scale, int32_t max_len_extend,
                                  int32_t is_cross_attention, int32_t sliding_window_size,
                                  int32_t dtype, void* stream);
+
+/*
+ * A prefill call's store inside its attention launch -- AttnBackend.forward for prefill metadata
+ * (mini_sglang_mlx/attention/backend.py:129-172): what msgl_store_kv_cache on (k, v, out_loc) and
+ * msgl_paged_prefill_attention behind it do.  For short query blocks of small launches (speculative verify,
+ * drafts): msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
+ * msgl_extend_step refuses them (MSGL_ERR_SHAPE).
+ *   q, k, v, out_loc: total_q rows each, in the order of qo_indptr; leading strides of k and v free, q
+ *   contiguous; bf16
+ * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; the request then sees
+ * the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
+ * request.  As with msgl_decode_step a slot of out_loc that is listed for another request may be read
+ * before or after the row is there: such a batch takes the two calls.
+ */
+MSGL_API size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv,
+                                                 int64_t num_q_heads, int64_t num_kv_heads,
+                                                 int64_t head_dim, int64_t max_len_extend,
+                                                 int32_t is_cross_attention,
+                                                 int32_t sliding_window_size);
+MSGL_API int msgl_extend_step(const void* q, const void* k, const void* v,
+                              int64_t k_stride0, int64_t v_stride0, const int32_t* out_loc,
+                              void* k_cache, void* v_cache,
+                              const int32_t* qo_indptr, const int32_t* kv_indptr,
+                              const int32_t* kv_indices, const int32_t* prefix_lens, void* out,
+                              void* workspace, size_t workspace_bytes,
+                              int64_t batch, int64_t total_q, int64_t total_kv,
+                              int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
+                              int64_t num_slots,
+                              int64_t k_cache_stride0, int64_t v_cache_stride0,
+                              float sm_scale, int32_t max_len_extend,
+                              int32_t is_cross_attention, int32_t sliding_window_size,
+                              int32_t dtype, void* stream);
 
 /*
  * build_attention_metadata -- replaces AttnBackend.build_prefill_metadata /

@@ -414,6 +414,17 @@ static bool window_prefers_tiles(int64_t batch, int64_t total_kv, int64_t n_kv, 
   return ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim) > 0;
 }
 
+// Whether a prefill call goes in shares, given room for their partials: `window_share` for its window's sake, else where
+// it is a short query block's call and small.
+static bool shares_route(const msgl::SharePlan& plan, bool window_share, int64_t batch, int64_t total_kv, int64_t keys,
+                         int64_t n_kv, int64_t group, int64_t max_len_extend, int64_t head_dim, int64_t window) {
+  if (plan.share_len == 0) return false;
+  if (window_share) return true;
+  return use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) &&
+         !window_prefers_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim, window) &&
+         msgl::shares_preferred(plan, batch, keys, n_kv, head_dim, group * max_len_extend);
+}
+
 size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv,
                                           int64_t num_q_heads, int64_t num_kv_heads,
                                           int64_t head_dim, int64_t max_len_extend) {
@@ -482,13 +493,13 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   const bool share_room = plan.share_len > 0 && workspace && aligned16(workspace) &&
                           workspace_bytes >= msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols);
   const bool window_share = share_room && window_shares(plan, batch, total_kv, keys, num_kv_heads, head_dim, cols);
-  const bool direct = window_share ||
-                      (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
-                       !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
-                                             sliding_window_size));
+  const bool shares = share_room && shares_route(plan, window_share, batch, total_kv, keys, num_kv_heads, group, max_len_extend,
+                                                 head_dim, sliding_window_size);
+  const bool direct = shares || (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
+                                 !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
+                                                       sliding_window_size));
   if (direct) {
     const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, cols);
-    const bool shares = window_share || (share_room && msgl::shares_preferred(plan, batch, keys, num_kv_heads, head_dim, cols));
     const size_t need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend, n_seg);
     if (!shares && (!workspace || workspace_bytes < need || !aligned16(workspace))) return MSGL_ERR_WORKSPACE;
     msgl::SplitKvArgs a{};
@@ -576,6 +587,81 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     }
   }
   return head_dim == 256 ? msgl::launch_prefill_tile256(a, s) : msgl::launch_prefill_tile(a, s);
+}
+
+// The plan of a prefill call whose store goes into its attention launch; share_len == 0: none
+static msgl::SharePlan extend_step_plan(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_q, int64_t n_kv,
+                                        int64_t head_dim, int64_t max_len_extend, bool is_cross, int64_t window) {
+  const msgl::SharePlan none{};
+  if (batch <= 0 || total_q <= 0 || total_kv <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv != 0 || max_len_extend <= 0 ||
+      window < 0 || (head_dim != 128 && head_dim != 256))
+    return none;
+  const int64_t group = n_q / n_kv, cols = group * max_len_extend;
+  const int64_t keys = visible_keys(batch, total_kv, window, max_len_extend, is_cross);
+  const msgl::SharePlan plan = shares_for(batch, keys, keys < total_kv ? keys / batch : 0, n_kv, head_dim, cols);
+  const bool window_share = window_shares(plan, batch, total_kv, keys, n_kv, head_dim, cols);
+  return shares_route(plan, window_share, batch, total_kv, keys, n_kv, group, max_len_extend, head_dim, window) ? plan : none;
+}
+
+size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv, int64_t num_q_heads,
+                                        int64_t num_kv_heads, int64_t head_dim, int64_t max_len_extend,
+                                        int32_t is_cross_attention, int32_t sliding_window_size) {
+  const msgl::SharePlan plan = extend_step_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
+                                                is_cross_attention != 0, sliding_window_size);
+  if (plan.share_len == 0) return 0;
+  return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, num_q_heads / num_kv_heads * max_len_extend);
+}
+
+int msgl_extend_step(const void* q, const void* k, const void* v, int64_t k_stride0, int64_t v_stride0, const int32_t* out_loc,
+                     void* k_cache, void* v_cache, const int32_t* qo_indptr, const int32_t* kv_indptr,
+                     const int32_t* kv_indices, const int32_t* prefix_lens, void* out, void* workspace,
+                     size_t workspace_bytes, int64_t batch, int64_t total_q, int64_t total_kv, int64_t num_q_heads,
+                     int64_t num_kv_heads, int64_t head_dim, int64_t num_slots, int64_t k_cache_stride0,
+                     int64_t v_cache_stride0, float sm_scale, int32_t max_len_extend, int32_t is_cross_attention,
+                     int32_t sliding_window_size, int32_t dtype, void* stream) {
+  if (num_slots <= 0) return MSGL_ERR_SHAPE;
+  const int rc = check_common(q, k_cache, v_cache, out, num_q_heads, num_kv_heads, head_dim, k_cache_stride0,
+                              v_cache_stride0, dtype, /*f16_ok=*/false);
+  if (rc != MSGL_OK) return rc;
+  if (!k || !v || !out_loc || !qo_indptr || !kv_indptr || !kv_indices || !prefix_lens) return MSGL_ERR_NULL_POINTER;
+  if (k_stride0 < num_kv_heads * head_dim || v_stride0 < num_kv_heads * head_dim) return MSGL_ERR_SHAPE;
+  if (!aligned16(k) || !aligned16(v) || k_stride0 % 8 || v_stride0 % 8) return MSGL_ERR_ALIGNMENT;
+  const msgl::SharePlan plan = extend_step_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
+                                                is_cross_attention != 0, sliding_window_size);
+  if (plan.share_len == 0) return MSGL_ERR_SHAPE;
+  const int64_t cols = num_q_heads / num_kv_heads * max_len_extend;
+  if (!workspace || !aligned16(workspace) || workspace_bytes < msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols))
+    return MSGL_ERR_WORKSPACE;
+  msgl::SplitKvArgs a{};
+  a.q = q;
+  a.k_cache = k_cache;
+  a.v_cache = v_cache;
+  a.kv_indptr = kv_indptr;
+  a.kv_indices = kv_indices;
+  a.qo_indptr = qo_indptr;
+  a.prefix_lens = prefix_lens;
+  a.out = out;
+  a.workspace = workspace;
+  a.batch = batch;
+  a.total_kv = total_kv;
+  a.n_q = num_q_heads;
+  a.n_kv = num_kv_heads;
+  a.head_dim = head_dim;
+  a.num_slots = num_slots;
+  a.k_stride0 = k_cache_stride0;
+  a.v_stride0 = v_cache_stride0;
+  a.sm_scale = sm_scale;
+  a.max_len_extend = max_len_extend;
+  a.q_cap = max_len_extend;
+  a.is_cross = is_cross_attention ? 1 : 0;
+  a.window = sliding_window_size;
+  msgl::NewTokens tokens{};
+  tokens.k = k;
+  tokens.v = v;
+  tokens.out_loc = out_loc;
+  tokens.k_stride0 = k_stride0;
+  tokens.v_stride0 = v_stride0;
+  return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
 }
 
 int msgl_copy_state_slots(void* slab, int64_t layer_stride_bytes, int64_t slot_stride_bytes,

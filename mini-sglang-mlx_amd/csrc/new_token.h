@@ -3,7 +3,8 @@
 // A step's own row of k and v goes into the pool in the launch that attends, by the wave whose range holds its
 // request's last key.  That wave takes the row from its source and not from the pool, so nobody waits for the
 // store: while its first tile is under way the new key makes the first state of the columns, and the walk
-// ends in front of it.  (Put into the tile that the walk computes last, it cost registers: 124 bytes of
+// ends in front of it.  (Where the request's last key is another slot, every wave of the request stores the row and
+// waits for that before it reads the pool.)  (Put into the tile that the walk computes last, it cost registers: 124 bytes of
 // spills and 6 us at head_dim 256.)  With norm weights every wave normalises and rotates its own q heads (and that
 // one the new key) at that time, four heads at once: a lane finds sine and cosine of one or two of the head's
 // angles and the wave exchanges them through LDS.  (At head_dim 256 all that goes in front of the first tile: there
@@ -17,7 +18,8 @@ namespace msgl {
 
 // What a decode launch does with its requests' new tokens: they are in the pool already; they are stored; q and k
 // are normalised and rotated, k and v stored.
-enum NewMode { kStored = 0, kStore = 1, kNormRopeStore = 2 };
+// (kStoreRows: kStore for several new tokens per request, a prefill call's.)
+enum NewMode { kStored = 0, kStore = 1, kNormRopeStore = 2, kStoreRows = 3 };
 
 inline void fill_new_tokens(const NewTokens& n, SplitKvParams& p) {
   if (n.k == nullptr) return;
@@ -70,6 +72,7 @@ struct NewToken {
   const uint16_t *k, *v;
   bool owner;         // the request's last key is this wave's (in a request without keys: the wave stores the rows)
   bool seen;          // and that key is the new token
+  bool elsewhere;     // the request's last key is not the new token, which may be any other of its keys
   int kvh;
   int before;         // slot id of the key in front of the last
   uint32_t slot;
@@ -86,6 +89,7 @@ struct NewToken {
     slot = (uint32_t)*loc;
     const uint32_t last_id = (uint32_t)*last;
     before = *second;
+    elsewhere = (r.kv_len > 0) & (slot <= sp.max_slot) & (last_id != slot);
     seen = owner & (r.kv_len > 0) & (slot <= sp.max_slot) & (last_id == slot);
     q = sp.q + (int64_t)b * sp.q_stride0 + kvh * sp.group * D;
     k = sp.nt.k + (int64_t)b * sp.nt.k_stride0 + kvh * D;
@@ -162,6 +166,15 @@ struct NewToken {
     }
   }
 
+  // Once, before the wave reads a row of the pool: a new token that may be any key of its request is in the pool then,
+  // stored by every wave of the request.
+  __device__ __forceinline__ void check() {
+    if (!elsewhere) return;
+    if (!owner) rows();
+    if constexpr (NORM) normalise();
+    store();
+    wait_all_vm();
+  }
   __device__ __forceinline__ void operator()() {
     __builtin_amdgcn_sched_barrier(0);
     run();
@@ -171,7 +184,7 @@ struct NewToken {
     if (!kRowsAhead && owner) rows();
     if constexpr (NORM) normalise();
     if (!owner) return;
-    const int lane = lane_id(), t16 = lane & 15, g = lane >> 4;
+    const int g = lane_id() >> 4;
     if (seen) {  // the columns' first key: its score the maximum, its weight 1
       float score = 0.f;
 #pragma unroll
@@ -188,6 +201,10 @@ struct NewToken {
 #pragma unroll
           for (int n = 0; n < 8; ++n) columns.o[0][hf][n][i] = value_of<F16>(vrow[hf][i][n >> 1], n & 1);
     }
+    store();
+  }
+  __device__ __forceinline__ void store() const {
+    const int t16 = lane_id() & 15, g = lane_id() >> 4;
     if (slot > sp.max_slot) return;  // a slot id outside the pool stores nothing
     if (t16 == 0) {
       uint16_t* to_k = sp.nt.k_pool + (int64_t)slot * sp.k_stride0 + kvh * D + g * 8;
@@ -201,6 +218,18 @@ struct NewToken {
     }
   }
 };
+
+// The new rows of a request, from their source to the pool.
+template <int D>
+__device__ __forceinline__ void store_new_rows(const SplitKvParams& p, int b, int kvh) {
+  const int lane = lane_id();
+  const uint32_t slot = (uint32_t)p.nt.out_loc[b];
+  if (slot > p.max_slot || lane >= D / 8) return;
+  st_global_b128(p.nt.k_pool + (int64_t)slot * p.k_stride0 + kvh * D + 8 * lane,
+                 ld_global_b128(p.nt.k + (int64_t)b * p.nt.k_stride0 + kvh * D + 8 * lane));
+  st_global_b128(p.nt.v_pool + (int64_t)slot * p.v_stride0 + kvh * D + 8 * lane,
+                 ld_global_b128(p.nt.v + (int64_t)b * p.nt.v_stride0 + kvh * D + 8 * lane));
+}
 
 // The same without norm weights for the long walks of paged_splitkv.hip, whose two tiles leave no registers for a state
 // in front of them (140 bytes of spills at head_dim 128, 196 at 256): the rows go to LDS by themselves when the walk starts
@@ -227,6 +256,10 @@ struct LateToken {
     const uint32_t last_id = (uint32_t)*last;
     before = *(r.kv_len > 1 ? last - 1 : last);
     seen = owner & (slot <= p.max_slot) & (last_id == slot);
+    if ((slot <= p.max_slot) & (last_id != slot)) {  // any key of its request, maybe: see NewToken::check()
+      store_new_rows<D>(p, b, kvh);
+      wait_all_vm();
+    }
     if (owner) {
       const int lane = lane_id(), at = lane & (2 * D / 8 - 1);
       const uint16_t* src = at < D / 8 ? p.nt.k + (int64_t)b * p.nt.k_stride0 + kvh * D + 8 * at
@@ -271,16 +304,102 @@ struct LateToken {
     st_global_b128(p.nt.v_pool + (int64_t)slot * p.v_stride0 + kvh * D + 8 * lane, *reinterpret_cast<const u32x4_t*>(&lds.v[8 * lane]));
   }
 };
-// The rows of a request without keys.
-template <int D>
-__device__ __forceinline__ void store_new_rows(const SplitKvParams& p, int b, int kvh) {
-  const int lane = lane_id();
-  const uint32_t slot = (uint32_t)p.nt.out_loc[b];
-  if (slot > p.max_slot || lane >= D / 8) return;
-  st_global_b128(p.nt.k_pool + (int64_t)slot * p.k_stride0 + kvh * D + 8 * lane,
-                 ld_global_b128(p.nt.k + (int64_t)b * p.nt.k_stride0 + kvh * D + 8 * lane));
-  st_global_b128(p.nt.v_pool + (int64_t)slot * p.v_stride0 + kvh * D + 8 * lane,
-                 ld_global_b128(p.nt.v + (int64_t)b * p.nt.v_stride0 + kvh * D + 8 * lane));
-}
+// The new tokens of a prefill call's request (kStoreRows, paged_shares.hip): rows q0 .. q0 + n - 1 of k and v.  As a rule
+// they are the request's last n keys and their slots stand there in kv_indices; then the waves walk the keys in front of
+// them, and one of them (the last wave of the last share) takes the new ones from their source, a tile of 32 at a time
+// while its first tile is under way, and stores them.  Against a store launch in front, us: 32 requests of 8 tokens on
+// 2-8 K, window 1024, 32 / 8 heads, 31.5 -> 30.0; 52 of 16, the same window, 69.3 -> 67.4; three of 3 tokens on some
+// hundred 11.2 -> 9.6; one of 5 tokens 16.0 -> 14.7.  Where the slots listed are others, or the tokens are not the
+// last keys, every wave of the request stores its head's rows and waits for that before it reads the pool.
+template <int D, int NCT>
+struct NewRows {
+  static constexpr int KS = D / 32, VH = D / 128;
+  const SplitKvParams& p;
+  const ReqInfo& r;
+  Columns<D, NCT>& columns;
+  int kvh, q0, n;
+  int end;                // of the keys that are walked
+  bool last_keys, owner;  // the new tokens are the request's last keys; this wave takes them
+  bool listed;            // their slots are the ones listed
+  uint32_t slot, id;      // lane i: slot of row i; slot id listed for its place
+
+  __device__ __forceinline__ NewRows(const SplitKvParams& params, const ReqInfo& req, Columns<D, NCT>& c, int b, int head)
+      : p(params), r(req), columns(c), kvh(head), owner(false) {
+    const int lane = lane_id();
+    q0 = p.qo_indptr[b];
+    n = p.qo_indptr[b + 1] - q0;
+    last_keys = n > 0 && n <= kWave && r.prefix >= 0 && r.prefix + n == r.kv_len && r.hi > r.lo;
+    end = last_keys ? max(min(r.hi, r.prefix), r.lo) : r.hi;
+    slot = lane < n ? (uint32_t)p.nt.out_loc[q0 + lane] : 0u;
+    id = last_keys && lane < n ? (uint32_t)p.kv_indices[r.kv_start + r.prefix + lane] : slot;
+  }
+  // Once, before the wave reads a row of the pool.
+  __device__ __forceinline__ void check() {
+    listed = last_keys && __all(lane_id() >= n || (slot == id && slot <= p.max_slot));
+    if (listed) return;
+    for (int i = 0; i < n; ++i) store_row(i);
+    wait_all_vm();
+  }
+  __device__ __forceinline__ void store_row(int i) const {
+    const int at = 8 * lane_id();
+    const uint32_t to = (uint32_t)p.nt.out_loc[q0 + i];
+    if (to > p.max_slot || at >= D) return;  // a slot id outside the pool stores nothing
+    st_global_b128(p.nt.k_pool + (int64_t)to * p.k_stride0 + kvh * D + at, ld_global_b128(p.nt.k + (int64_t)(q0 + i) * p.nt.k_stride0 + kvh * D + at));
+    st_global_b128(p.nt.v_pool + (int64_t)to * p.v_stride0 + kvh * D + at, ld_global_b128(p.nt.v + (int64_t)(q0 + i) * p.nt.v_stride0 + kvh * D + at));
+  }
+  __device__ __forceinline__ void operator()() {
+    if (!owner) return;
+    const int t16 = lane_id() & 15, g = lane_id() >> 4;
+    for (int i0 = 0; i0 < n; i0 += 32) {
+      KvTile<D> t;
+      // a row's place: in the source, or in the pool
+      auto k_row = [&](int i) {
+        const int64_t from = (int64_t)(q0 + i) * p.nt.k_stride0, in = (int64_t)min(__shfl(id, i, kWave), p.max_slot) * p.k_stride0;
+        return (listed ? p.nt.k + from : p.k_cache + in) + kvh * D;
+      };
+      auto v_row = [&](int i) {
+        const int64_t from = (int64_t)(q0 + i) * p.nt.v_stride0, in = (int64_t)min(__shfl(id, i, kWave), p.max_slot) * p.v_stride0;
+        return (listed ? p.nt.v + from : p.v_cache + in) + kvh * D;
+      };
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) {
+        const uint16_t* row = k_row(min(i0 + 16 * sub + t16, n - 1));
+#pragma unroll
+        for (int c = 0; c < KS; ++c) t.k[sub][c] = ld_global_b128(row + c * 32 + g * 8);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint16_t* row = v_row(min(i0 + (j < 4 ? 0 : 16) + 4 * g + (j & 3), n - 1));
+#pragma unroll
+        for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = ld_global_b128(row + hf * 128 + t16 * 8);
+      }
+      if (listed) {
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+          const int i = i0 + 16 * sub + t16;
+          uint16_t* to = p.nt.k_pool + (int64_t)(uint32_t)__shfl(slot, min(i, n - 1), kWave) * p.k_stride0 + kvh * D + g * 8;
+          if (i < n) {
+#pragma unroll
+            for (int c = 0; c < KS; ++c) st_global_b128(to + c * 32, t.k[sub][c]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int i = i0 + (j < 4 ? 0 : 16) + 4 * g + (j & 3);
+          uint16_t* to = p.nt.v_pool + (int64_t)(uint32_t)__shfl(slot, min(i, n - 1), kWave) * p.v_stride0 + kvh * D + t16 * 8;
+          if (i < n) {
+#pragma unroll
+            for (int hf = 0; hf < VH; ++hf) st_global_b128(to + hf * 128, t.v[hf][j]);
+          }
+        }
+      }
+      compute_tile<D, NCT, false>(p, t, r.prefix + i0, columns);
+    }
+    // what the walk's last tile holds past the walk's end is not visible in it
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) columns.hi[ct] = min(columns.hi[ct], end - 1);
+    columns.all_hi = min(columns.all_hi, end - 1);
+  }
+};
 
 }  // namespace msgl

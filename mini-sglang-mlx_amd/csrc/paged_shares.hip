@@ -87,6 +87,11 @@ __device__ __forceinline__ bool find_share(const SplitKvParams& p, int share_len
   return false;
 }
 
+struct Nothing {
+  template <typename... Args>
+  __device__ __forceinline__ explicit Nothing(const Args&...) {}
+};
+
 template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
 __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(ShareParams sp) {
   const SplitKvParams& p = sp.s;
@@ -111,9 +116,14 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   if (!find_share(p, sp.share_len, item, &r, &b, &share, &n_shares)) return;  // the whole workgroup
   const int ncols = r.q_len * p.group;
   if (ncols == 0) return;
-  const int vis = r.hi - r.lo;
+  Columns<D, NCT> c;
+  // the keys that are walked: all, but for a prefill call's own new ones
+  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, b, kvh);
+  int hi = r.hi;
+  if constexpr (NEW == kStoreRows) hi = new_rows.end;
+  const int vis = hi - r.lo;
   const int per = ((vis + n_shares - 1) / n_shares + 31) & ~31;
-  const int s_begin = min(r.lo + share * per, r.hi), s_end = min(s_begin + per, r.hi);
+  const int s_begin = min(r.lo + share * per, hi), s_end = min(s_begin + per, hi);
   const int per_wave = ((per + sp.share_waves - 1) / sp.share_waves + 31) & ~31;
   const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
 
@@ -128,12 +138,17 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
                                                  __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  Columns<D, NCT> c;
   FirstIds ids{};
   if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
   if constexpr (NEW == kStored) {
     start_columns(p, r, kvh, 0, t_end, c);
     if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
+  } else if constexpr (NEW == kStoreRows) {
+    new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == sp.share_waves - 1;
+    start_columns(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
+    new_rows.check();
+    if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
+    else new_rows();
   } else {
     static_assert(sizeof(HeadLds<D>) <= sizeof(part[0]), "a wave's heads have their place in its part of the partials");
     const int tail = r.kv_len - 1;
@@ -144,6 +159,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
       walk_end = tail;
       end_ids(ids, t_begin, tail, token.before);
     }
+    token.check();
     start_columns<D, NCT, NEW != kNormRopeStore>(p, r, kvh, 0, walk_end, c);
     if constexpr (D == 256) {
       token();
@@ -309,9 +325,9 @@ int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
     return check_launch();
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
-    const int mode = sp.s.nt.k == nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
+    const int mode = sp.s.nt.k == nullptr || sp.s.qo_indptr != nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
     if (sp.s.f16) {
-      if (mode == kStored)
+      if (mode == kStored && sp.s.nt.k == nullptr)
         return launch(share_attention_kernel<D, NCT, NW, false, true, kStored>, share_attention_kernel<D, NCT, NW, true, true, kStored>);
       if (mode == kStore)
         return launch(share_attention_kernel<D, NCT, NW, false, true, kStore>, share_attention_kernel<D, NCT, NW, true, true, kStore>);
@@ -323,7 +339,9 @@ int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
       return launch(share_attention_kernel<D, NCT, NW, false, false, kNormRopeStore>,
                     share_attention_kernel<D, NCT, NW, true, false, kNormRopeStore>);
   }
-  if (sp.s.f16 || sp.s.nt.k != nullptr) return MSGL_ERR_DTYPE;
+  if (sp.s.f16) return MSGL_ERR_DTYPE;
+  if (sp.s.nt.k != nullptr)  // a prefill call's
+    return launch(share_attention_kernel<D, NCT, NW, false, false, kStoreRows>, share_attention_kernel<D, NCT, NW, true, false, kStoreRows>);
   return launch(share_attention_kernel<D, NCT, NW, false, false, kStored>, share_attention_kernel<D, NCT, NW, true, false, kStored>);
 }
 

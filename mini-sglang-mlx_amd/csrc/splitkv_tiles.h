@@ -158,6 +158,89 @@ __device__ __forceinline__ FirstIds first_ids(const SplitKvParams& p, const ReqI
   return FirstIds{{idx[min(at, last)], idx[min(at + 16, last)]}, {idx[min(at + 32, last)], idx[min(at + 48, last)]}};
 }
 
+// Keys tb .. tb + 31, in registers, for the columns in `c_`.
+template <int D, int NCT, bool F16>
+__device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTile<D>& t, int tb, Columns<D, NCT>& c_) {
+  constexpr int KS = D / 32;   // k-steps of the QK product
+  constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
+  const int g = lane_id() >> 4;
+  // S^T[token][col] for the two 16-token sub-tiles
+  f32x4_t s[2][NCT];
+#pragma unroll
+  for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < KS; ++c)
+        acc = mfma_16x16x32_raw<F16>(t.k[sub][c], c_.q[ct][c], acc);
+      s[sub][ct] = acc;
+    }
+  const bool need_mask = (tb < c_.all_lo) || (tb + 31 > c_.all_hi);
+  uint32_t pb[NCT][4];
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    float x[2][4];
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[sub][i] = s[sub][ct][i] * p.scale_log2e;
+    if (need_mask) {
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int tok = tb + sub * 16 + 4 * g + i;
+          if (tok < c_.lo[ct] || tok > c_.hi[ct]) x[sub][i] = kNegInf;
+        }
+    }
+    float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
+                     fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
+    mx = max_across<32>(max_across<16>(mx));
+    const float m_new = fmaxf(c_.m[ct], mx);
+    const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
+    const float alpha = fast_exp2(c_.m[ct] - m_safe);
+    c_.m[ct] = m_new;
+    float psum = 0.f;
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[sub][i] = fast_exp2(x[sub][i] - m_safe);
+        psum += x[sub][i];
+      }
+    c_.l[ct] = c_.l[ct] * alpha + psum;
+    pb[ct][0] = pack_16x2<F16>(x[0][0], x[0][1]);
+    pb[ct][1] = pack_16x2<F16>(x[0][2], x[0][3]);
+    pb[ct][2] = pack_16x2<F16>(x[1][0], x[1][1]);
+    pb[ct][3] = pack_16x2<F16>(x[1][2], x[1][3]);
+    if (__any(alpha != 1.0f)) {
+#pragma unroll
+      for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+        for (int n = 0; n < 8; ++n) c_.o[ct][hf][n] *= alpha;
+    }
+  }
+  // O^T += V^T P^T.  MFMA n of half hf produces d = hf*128 + 8*row + n on row = l%16.
+#pragma unroll
+  for (int hf = 0; hf < VH; ++hf)
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      u32x4_t vt;
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        const uint32_t a = t.v[hf][2 * qd][n >> 1];
+        const uint32_t c = t.v[hf][2 * qd + 1][n >> 1];
+        vt[qd] = (n & 1) ? pack_hi16(a, c) : pack_lo16(a, c);
+      }
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) {
+        const u32x4_t pv = {pb[ct][0], pb[ct][1], pb[ct][2], pb[ct][3]};
+        c_.o[ct][hf][n] = mfma_16x16x32_raw<F16>(vt, pv, c_.o[ct][hf][n]);
+      }
+    }
+}
+
 // Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`; `first`: its first_ids(), asked for before
 // the columns were made.
 // SHORT: ranges of one tile are common, end behind it (in a long walk the test costs more than it saves).
@@ -207,84 +290,6 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     }
   };
 
-  auto compute_tile = [&](const KvTile<D>& t, int tb) {
-    // S^T[token][col] for the two 16-token sub-tiles
-    f32x4_t s[2][NCT];
-#pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < KS; ++c)
-          acc = mfma_16x16x32_raw<F16>(t.k[sub][c], c_.q[ct][c], acc);
-        s[sub][ct] = acc;
-      }
-    const bool need_mask = (tb < c_.all_lo) || (tb + 31 > c_.all_hi);
-    uint32_t pb[NCT][4];
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-      float x[2][4];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[sub][i] = s[sub][ct][i] * p.scale_log2e;
-      if (need_mask) {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int tok = tb + sub * 16 + 4 * g + i;
-            if (tok < c_.lo[ct] || tok > c_.hi[ct]) x[sub][i] = kNegInf;
-          }
-      }
-      float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
-                       fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
-      mx = max_across<32>(max_across<16>(mx));
-      const float m_new = fmaxf(c_.m[ct], mx);
-      const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
-      const float alpha = fast_exp2(c_.m[ct] - m_safe);
-      c_.m[ct] = m_new;
-      float psum = 0.f;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          x[sub][i] = fast_exp2(x[sub][i] - m_safe);
-          psum += x[sub][i];
-        }
-      c_.l[ct] = c_.l[ct] * alpha + psum;
-      pb[ct][0] = pack_16x2<F16>(x[0][0], x[0][1]);
-      pb[ct][1] = pack_16x2<F16>(x[0][2], x[0][3]);
-      pb[ct][2] = pack_16x2<F16>(x[1][0], x[1][1]);
-      pb[ct][3] = pack_16x2<F16>(x[1][2], x[1][3]);
-      if (__any(alpha != 1.0f)) {
-#pragma unroll
-        for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-          for (int n = 0; n < 8; ++n) c_.o[ct][hf][n] *= alpha;
-      }
-    }
-    // O^T += V^T P^T.  MFMA n of half hf produces d = hf*128 + 8*row + n on row = l%16.
-#pragma unroll
-    for (int hf = 0; hf < VH; ++hf)
-#pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        u32x4_t vt;
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const uint32_t a = t.v[hf][2 * qd][n >> 1];
-          const uint32_t c = t.v[hf][2 * qd + 1][n >> 1];
-          vt[qd] = (n & 1) ? pack_hi16(a, c) : pack_lo16(a, c);
-        }
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-          const u32x4_t pv = {pb[ct][0], pb[ct][1], pb[ct][2], pb[ct][3]};
-          c_.o[ct][hf][n] = mfma_16x16x32_raw<F16>(vt, pv, c_.o[ct][hf][n]);
-        }
-      }
-  };
-
   // ---- tile loop: two register tiles, slot ids fetched two tiles ahead.  Every load in
   // the loop body is unconditional (tokens past the range clamp to its last token and
   // are masked), so the number of loads in flight at each wait is a compile-time
@@ -300,11 +305,11 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     const int tok = t_begin + pr * 64;
     load_tile(tb_, i1a, i1b);
     load_idx(tok + 96, i1a, i1b);
-    compute_tile(ta, tok);
+    compute_tile<D, NCT, F16>(p, ta, tok, c_);
     if (SHORT && tok + 32 >= t_end) break;
     load_tile(ta, i0a, i0b);
     load_idx(tok + 128, i0a, i0b);
-    compute_tile(tb_, tok + 32);
+    compute_tile<D, NCT, F16>(p, tb_, tok + 32, c_);
   }
 }
 

@@ -584,6 +584,59 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   });
 }
 
+// ---- extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, sm_scale,
+//                  max_len_extend, is_cross_attention, sliding_window_size) -> out or None ---------------
+// As decode_step, for prefill metadata.
+PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  return guarded(args, n_args, 14, [](PyObject* const* a) -> PyObject* {
+    static const char op[] = "extend_step";
+    for (int i = 0; i < 10; ++i)
+      if (!THPVariable_Check(a[i])) return none();
+    auto t = [&](int i) -> const Tensor& { return THPVariable_Unpack(a[i]); };
+    const Tensor &q = t(0), &k = t(1), &v = t(2), &loc = t(3), &kc = t(4), &vc = t(5), &qp = t(6), &ip = t(7), &ix = t(8), &pl = t(9);
+    if (q.dim() != 3 || k.dim() != 3 || kc.dim() != 3 || vc.dim() != 3 || qp.dim() != 1 || ix.dim() != 1) return none();
+    const int64_t total = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = k.size(1), slots = kc.size(0), batch = qp.size(0) - 1;
+    const c10::Device dev = q.device();
+    if (total == 0 || batch <= 0 || slots == 0 || q.scalar_type() != at::kBFloat16 || !dev.is_cuda()) return none();
+    const int64_t max_extend = integer(a[11]), window = integer(a[13]);
+    const bool cross = truth(a[12]);
+    if (window < 0 || window > 0x7fffffff || max_extend > 0x7fffffff) return none();
+    const size_t bytes = msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross, static_cast<int32_t>(window));
+    if (bytes == 0) return none();
+    if (const char* env = std::getenv("MSGL_DEBUG_CHECKS"); env && *env && std::strcmp(env, "0") != 0) return none();
+    auto same = [&](const Tensor& x) { return x.scalar_type() == at::kBFloat16 && x.device() == dev; };
+    auto ints_of = [&](const Tensor& x, int64_t n) {
+      return x.dim() == 1 && x.size(0) == n && x.scalar_type() == at::kInt && x.device() == dev && x.is_contiguous();
+    };
+    auto rows = [&](const Tensor& x) {
+      return x.stride(2) == 1 && x.stride(1) == d && (x.size(0) == 1 || (x.stride(0) >= x.size(1) * d && x.stride(0) % 8 == 0)) &&
+             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    };
+    const c10::IntArrayRef pool_size = kc.sizes();
+    if (!same(k) || !same(v) || !same(kc) || !same(vc) || k.size(0) != total || k.size(2) != d || v.sizes() != k.sizes() ||
+        pool_size[1] != n_kv || pool_size[2] != d || vc.sizes() != pool_size || !q.is_contiguous() || !rows(q) || !rows(k) ||
+        !rows(v) || !rows(kc) || !rows(vc) || !ints_of(loc, total) || !ints_of(qp, batch + 1) || !ints_of(ip, batch + 1) ||
+        !ints_of(ix, ix.numel()) || !ints_of(pl, batch))
+      return none();
+    const float scale = static_cast<float>(real(a[10]));
+    auto stride0 = [](const Tensor& x) { return x.size(0) > 1 ? x.stride(0) : x.size(1) * x.size(2); };
+    Tensor out;
+    int rc;
+    {
+      NoGil nogil;
+      OnDevice on(dev);
+      out = empty({total, n_q, d}, at::kBFloat16, dev);
+      const Tensor ws = scratch(bytes, dev);
+      rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), stride0(k), stride0(v), ints(loc), kc.data_ptr(),
+                            vc.data_ptr(), ints(qp), ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.data_ptr(), bytes, batch,
+                            total, ix.size(0), n_q, n_kv, d, slots, stride0(kc), stride0(vc), scale,
+                            static_cast<int32_t>(max_extend), cross ? 1 : 0, static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+    }
+    check_rc(op, rc);
+    return THPVariable_Wrap(std::move(out));
+  });
+}
+
 // ---- gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr, single_token_mode) -> y -------
 PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 9, [](PyObject* const* a) -> PyObject* {
@@ -651,6 +704,7 @@ PyMethodDef g_methods[] = {MSGL_FAST(store_kv_cache),
                            MSGL_FAST(build_metadata_from_host),
                            MSGL_FAST(qk_norm_rope_store),
                            MSGL_FAST(decode_step),
+                           MSGL_FAST(extend_step),
                            MSGL_FAST(gdn_state_inplace),
                            {"set_checks", set_checks, METH_O, nullptr},
                            {nullptr, nullptr, 0, nullptr}};

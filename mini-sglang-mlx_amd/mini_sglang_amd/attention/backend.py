@@ -84,10 +84,13 @@ class AttnBackend:
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
         metadata = batch.attn_metadata
-        if not is_cross_attention and sliding_window_size == 0:
+        out = None
+        if type(metadata) is PrefillMetadata:
+            out = self._extend_step(q, k, v, layer_id, batch, is_cross_attention, sliding_window_size)
+        elif not is_cross_attention and sliding_window_size == 0:
             out = self._decode_step(q, k, v, layer_id, batch)
-            if out is not None:
-                return out
+        if out is not None:
+            return out
         self.kvcache.store_kv(k, v, batch.out_loc, layer_id)
         k_cache = self.kvcache.k_cache(layer_id)
         v_cache = self.kvcache.v_cache(layer_id)
@@ -104,6 +107,17 @@ class AttnBackend:
                                    cache.k_cache(layer_id), cache.v_cache(layer_id),
                                    metadata.kv_indptr, metadata.kv_indices, metadata.num_kv_splits,
                                    self.sm_scale, eps, rope_base)
+
+    def _extend_step(self, q, k, v, layer_id: int, batch, is_cross_attention: bool,
+                     sliding_window_size: int) -> Optional[torch.Tensor]:
+        """The same for ``mini_sglang_amd_kernel.extend_step``."""
+        metadata, cache = batch.attn_metadata, self.kvcache
+        if type(cache) is not MHAKVCache:
+            return None
+        return _native.extend_step(q, k, v, batch.out_loc, cache.k_cache(layer_id),
+                                   cache.v_cache(layer_id), metadata.qo_indptr, metadata.kv_indptr,
+                                   metadata.kv_indices, metadata.prefix_lens, self.sm_scale,
+                                   metadata.max_len_extend, is_cross_attention, sliding_window_size)
 
     def _attend(self, q, k_cache, v_cache, metadata, is_cross_attention: bool,
                 sliding_window_size: int) -> torch.Tensor:

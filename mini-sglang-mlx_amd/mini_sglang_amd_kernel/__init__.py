@@ -28,7 +28,7 @@ except ImportError as _exc:  # not built: the first call says so
     _native = _lib.MissingNative(_exc)
 
 __all__ = ["store_kv_cache", "paged_decode_attention", "paged_prefill_attention",
-           "build_attention_metadata", "build_metadata_from_host", "qk_norm_rope_store", "decode_step",
+           "build_attention_metadata", "build_metadata_from_host", "qk_norm_rope_store", "decode_step", "extend_step",
            "gdn_state_inplace",
            "fast_compare_key"]
 
@@ -270,10 +270,25 @@ def decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
     validation on.
 
     One new token per request, row ``b`` at slot ``out_loc[b]``.  A slot of ``out_loc`` must not be
-    listed for any other key that the step sees: the launch that reads it writes it.
+    listed for another request: the launch that reads it writes it.
     """
     return _native.decode_step(q, k, v, q_weight, k_weight, positions, out_loc, k_cache, v_cache,
                                kv_indptr, kv_indices, num_kv_splits, sm_scale, eps, rope_base)
+
+
+def extend_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torch.Tensor,
+                k_cache: torch.Tensor, v_cache: torch.Tensor, qo_indptr: torch.Tensor,
+                kv_indptr: torch.Tensor, kv_indices: torch.Tensor, prefix_lens: torch.Tensor, *,
+                sm_scale: float, max_len_extend: int, is_cross_attention: bool = False,
+                sliding_window_size: int = 0) -> Optional[torch.Tensor]:
+    """``paged_prefill_attention`` with ``store_kv_cache`` of the queries' own rows of k and v inside: the
+    attention output, or ``None`` (nothing done) where the two calls are the way: longer query blocks,
+    large launches, forms that need a copy, arguments that they refuse, index validation on.  As with
+    ``decode_step`` a slot of ``out_loc`` must not be listed for another request.
+    """
+    return _native.extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices,
+                               prefix_lens, sm_scale, max_len_extend, is_cross_attention,
+                               sliding_window_size)
 
 
 def gdn_state_inplace(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,

@@ -1,12 +1,13 @@
-"""A decode step's store (or norm, rotary embedding and store) inside its attention launch, against the same
-step as two launches, which the oracle tests pin: at the edges of a wave's 32 keys and of a share, for requests
-without keys, for a new token that is not its request's last key, for a slot outside the pool, on strided rows,
+"""The store of a step (for decode also norm, rotary embedding and store) inside its attention launch, against the
+same step as two launches, which the oracle tests pin: at the edges of a wave's 32 keys and of a share, for requests
+without keys, for new tokens that are not their request's last keys, for a slot outside the pool, on strided rows,
 and from a pool whose new slots hold NaN before the step."""
 import pytest
 import torch
 
 from mini_sglang_amd.workloads import build_workload
-from mini_sglang_amd_kernel import _lib, decode_step, paged_decode_attention, qk_norm_rope_store, store_kv_cache
+from mini_sglang_amd_kernel import (_lib, decode_step, extend_step, paged_decode_attention, paged_prefill_attention,
+                                    qk_norm_rope_store, store_kv_cache)
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +40,8 @@ def _step(gpu, lens, n_q, n_kv, d, dtype, seed):
     for i, n in enumerate(lens):  # as a rule a request's last slot is the new token's
         if n > 0 and i % 5 != 4:
             loc[i] = wl.kv_indices[int(wl.kv_indptr[i + 1]) - 1]
+        if n > 2 and i % 5 == 3:  # ... or stands in the middle
+            loc[i] = wl.kv_indices[int(wl.kv_indptr[i]) + n // 2]
     for c in (kc, vc):
         c[loc.long()] = float("nan")
     for i, n in enumerate(lens):  # a last slot that is not the new token's holds a row
@@ -108,3 +111,64 @@ def test_what_is_left_to_the_two_calls(gpu, monkeypatch):
     need = _lib.load().msgl_decode_step_workspace_bytes
     assert need(64, 64 * 4096, 32, 8, 128, 0) == 0  # a large launch
     assert need(1, 20000, 32, 8, 128, 0) > 0 and need(1, 20000, 32, 8, 128, 1) == 0  # segments: without norm weights
+
+
+# kv lengths before the step, new tokens, q heads, kv heads, head_dim, share_len, max_len_extend below the longest
+ROWS = [
+    ([0, 31, 32, 33, 257, 700], [8] * 6, 32, 8, 128, 0, 0),
+    ([5, 64, 1000, 130, 0, 40, 300], [3, 1, 7, 0, 4, 2, 5], 16, 8, 128, 64, 0),
+    ([90, 500], [48, 33], 8, 8, 128, 128, 0),
+    ([90, 500, 2100], [11, 12, 5], 32, 8, 128, 512, 0),
+    ([0, 1500, 77], [3, 4, 2], 16, 4, 256, 128, 0),
+    ([100, 600], [9, 4], 16, 8, 128, 128, 6),
+]
+
+
+@pytest.mark.parametrize("cached,ext,n_q,n_kv,d,share,cap", ROWS)
+@pytest.mark.parametrize("cross,window", [(False, 0), (True, 0), (False, 100), (True, 70)])
+@pytest.mark.parametrize("places", ["last", "mixed"])
+def test_extend_one_launch_is_two(gpu, tuning, cached, ext, n_q, n_kv, d, share, cap, cross, window, places):
+    kv = [c + e for c, e in zip(cached, ext)]
+    wl = build_workload("step", "prefill", seed=sum(kv), n_q=n_q, n_kv=n_kv, head_dim=d, kv_lens=kv, extend_lens=ext,
+                        is_cross_attention=cross, sliding_window_size=window).to(gpu)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(sum(kv))
+    total = sum(ext)
+    kvr = torch.randn((total, 2 * n_kv, d), generator=g, device=gpu).bfloat16()
+    k, v = kvr[:, :n_kv], kvr[:, n_kv:]
+    kc, vc = (torch.cat([c, c]) for c in (wl.k_cache, wl.v_cache))  # the upper half is nobody's
+    loc, at = torch.empty(total, dtype=torch.int32, device=gpu), 0
+    for b, (c, e) in enumerate(zip(cached, ext)):
+        first = int(wl.kv_indptr[b])
+        loc[at:at + e] = wl.kv_indices[first + c:first + c + e]
+        if places == "mixed" and b % 3 == 0 and e > 1:  # one token elsewhere, its place an old key
+            loc[at + 1] = wl.k_cache.shape[0] + b
+        if places == "mixed" and b % 3 == 1 and c > e:  # the tokens stand in front of the last keys
+            loc[at:at + e] = wl.kv_indices[first + c - e:first + c]
+        at += e
+    for c in (kc, vc):
+        c[loc.long()] = float("nan")
+    if places == "mixed" and total > 2:
+        loc[total - 1] = kc.shape[0] + 3  # outside the pool: nothing is stored
+        kc.nan_to_num_(0.5)
+        vc.nan_to_num_(0.5)
+    limit = cap or max(ext)
+    tuning(_lib.TUNE_SHARES, (share or 96) | 1 << 20)
+    tuning(_lib.TUNE_SMALLQ_MAXCOLS, 48)  # whatever the window
+    kc2, vc2 = kc.clone(), vc.clone()
+    print(f"extend step {cached[:4]} + {ext[:4]} {n_q}/{n_kv} d{d} cross={cross} window={window} {places}", flush=True)
+    got = extend_step(wl.q, k, v, loc, kc, vc, wl.qo_indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, sm_scale=wl.sm_scale,
+                      max_len_extend=limit, is_cross_attention=cross, sliding_window_size=window)
+    assert got is not None
+    store_kv_cache(kc2, vc2, loc, k, v)
+    want = paged_prefill_attention(wl.q, kc2, vc2, wl.qo_indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, wl.sm_scale,
+                                   limit, is_cross_attention=cross, sliding_window_size=window)
+    for a, b in ((kc, kc2), (vc, vc2)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    at = 0
+    for e in ext:  # rows past the cap are not computed
+        x, y = got[at:at + min(e, limit)].float(), want[at:at + min(e, limit)].float()
+        assert bool(torch.isfinite(x).all())
+        diff = (x - y).abs()
+        assert e == 0 or (float(diff.max()) <= 2e-2 and float(diff.mean()) <= 1e-3), (float(diff.max()), float(diff.mean()))
+        at += e
