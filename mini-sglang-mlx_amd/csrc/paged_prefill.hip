@@ -1621,6 +1621,55 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
 }
 
 
+// One row from `count` partials that lie `step` rows apart: a lane's dims of it, of 32 lanes.  Eight partials are asked
+// for together, sums and rows, and go into a running maximum: a partial at a time, each behind its sum, is a
+// chain of round trips (30 partials of 1440 rows of 128 25.6 -> 6.8 us, 28 of 832 rows of 256 22.2 -> 6.6).
+template <int D>
+__device__ __forceinline__ void merge_row(const float* part, const float* lse, int64_t step, int count, uint16_t* dst) {
+  constexpr int V = D / 32;  // dims per lane
+  constexpr int U = 8;
+  float top = kNegInf, total = 0.f;
+  float acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = 0.f;
+  for (int s0 = 0; s0 < count; s0 += U) {
+    float sum[U];
+    f32x4_t x[U][V / 4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // past the last partial: that again, with weight 0
+      const int64_t at = (int64_t)min(s0 + u, count - 1) * step;
+      sum[u] = lse[at];
+#pragma unroll
+      for (int i = 0; i < V / 4; ++i) x[u][i] = *reinterpret_cast<const f32x4_t*>(part + at * D + 4 * i);
+    }
+    float next = top;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u >= count) sum[u] = kNegInf;
+      next = fmaxf(next, sum[u]);
+    }
+    const float ref = next == kNegInf ? 0.f : next;
+    const float old = exp2f(top - ref);
+    top = next;
+    total *= old;
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] *= old;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool seen = sum[u] != kNegInf;  // a share that saw no key of this row counts for nothing, whatever it holds
+      const float wgt = seen ? exp2f(sum[u] - ref) : 0.f;
+      total += wgt;
+#pragma unroll
+      for (int i = 0; i < V; ++i) acc[i] += seen ? wgt * x[u][i >> 2][i & 3] : 0.f;
+    }
+  }
+  const float inv = (total > 0.f) ? 1.0f / total : 0.f;
+#pragma unroll
+  for (int i = 0; i < V; i += 4)
+    *reinterpret_cast<u32x2_t*>(dst + i) = u32x2_t{pack_bf16x2(acc[i] * inv, acc[i + 1] * inv), pack_bf16x2(acc[i + 2] * inv, acc[i + 3] * inv)};
+}
+
+
 // ---- merge of a key-split launch: one 32-lane group per (token, q head) row -----------------
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restrict__ part_o,
@@ -1628,7 +1677,6 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
                                                             const int32_t* __restrict__ qo_indptr,
                                                             uint16_t* __restrict__ out, int64_t part_rows,
                                                             int n_q, int n_ksplit, int max_len_extend) {
-  constexpr int V = D / 32;  // dims per lane
   const int b = blockIdx.y;
   const int q_start = qo_indptr[b];
   const int q_len = min(qo_indptr[b + 1] - q_start, max_len_extend);
@@ -1636,41 +1684,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
   if (r >= (int64_t)q_len * n_q) return;
   const int64_t row = (int64_t)q_start * n_q + r;
   const int c = threadIdx.x & 31;
-  float top = kNegInf;
-  for (int s = 0; s < n_ksplit; ++s) top = fmaxf(top, part_lse[s * part_rows + row]);
-  float acc[V];
-#pragma unroll
-  for (int i = 0; i < V; ++i) acc[i] = 0.f;
-  float total = 0.f;
-  for (int s = 0; s < n_ksplit; ++s) {
-    const float lse = part_lse[s * part_rows + row];
-    if (lse == kNegInf) continue;  // that share saw no key of this row
-    const float wgt = exp2f(lse - top);
-    total += wgt;
-    const float* src = part_o + (s * part_rows + row) * D + c * V;
-#pragma unroll
-    for (int i = 0; i < V; i += 4) {
-      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + i);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i + e] += wgt * x[e];
-    }
-  }
-  const float inv = (total > 0.f) ? 1.0f / total : 0.f;
-  uint16_t* dst = out + row * D + c * V;
-#pragma unroll
-  for (int i = 0; i < V; i += 4) {
-    u32x2_t wv;
-    wv[0] = pack_bf16x2(acc[i] * inv, acc[i + 1] * inv);
-    wv[1] = pack_bf16x2(acc[i + 2] * inv, acc[i + 3] * inv);
-    *reinterpret_cast<u32x2_t*>(dst + i) = wv;
-  }
+  merge_row<D>(part_o + row * D + c * (D / 32), part_lse + row, part_rows, n_ksplit, out + row * D + c * (D / 32));
 }
 
 // The same for ragged shares: request b's partials are units req_units[2 b] .. + req_units[2 b + 1],
 // each [kv head][row of the block]; a request with one share was written by the attention kernel.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_ragged_merge_kernel(PrefillParams p) {
-  constexpr int V = D / 32;  // dims per lane
   const int b = blockIdx.y;
   const int q_start = p.qo_indptr[b];
   const int q_len = min(p.qo_indptr[b + 1] - q_start, p.max_len_extend);
@@ -1686,34 +1706,7 @@ __global__ __launch_bounds__(256) void prefill_ragged_merge_kernel(PrefillParams
   const int64_t step = (int64_t)p.n_kv * p.ragged_rows;  // partial rows from one unit to the next
   const int64_t at0 = ((int64_t)first * p.n_kv + kvh) * p.ragged_rows + local;
   const int c = threadIdx.x & 31;
-  float top = kNegInf;
-  for (int s = 0; s < count; ++s) top = fmaxf(top, p.part_lse[at0 + s * step]);
-  float acc[V];
-#pragma unroll
-  for (int i = 0; i < V; ++i) acc[i] = 0.f;
-  float total = 0.f;
-  for (int s = 0; s < count; ++s) {
-    const float lse = p.part_lse[at0 + s * step];
-    if (lse == kNegInf) continue;  // that share saw no key of this row
-    const float wgt = exp2f(lse - top);
-    total += wgt;
-    const float* src = p.part_o + (at0 + s * step) * D + c * V;
-#pragma unroll
-    for (int i = 0; i < V; i += 4) {
-      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + i);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i + e] += wgt * x[e];
-    }
-  }
-  const float inv = (total > 0.f) ? 1.0f / total : 0.f;
-  uint16_t* dst = p.out + ((int64_t)q_start * p.n_q + r) * D + c * V;
-#pragma unroll
-  for (int i = 0; i < V; i += 4) {
-    u32x2_t wv;
-    wv[0] = pack_bf16x2(acc[i] * inv, acc[i + 1] * inv);
-    wv[1] = pack_bf16x2(acc[i + 2] * inv, acc[i + 3] * inv);
-    *reinterpret_cast<u32x2_t*>(dst + i) = wv;
-  }
+  merge_row<D>(p.part_o + at0 * D + c * (D / 32), p.part_lse + at0, step, count, p.out + ((int64_t)q_start * p.n_q + r) * D + c * (D / 32));
 }
 
 }  // namespace
