@@ -385,10 +385,10 @@ static int ragged_tiles(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t g
 }
 
 // Gang ranges for the head_dim 128 ping-pong kernel (several query blocks per (request, kv head)).
-static int gangs_for(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t group, int64_t max_len_extend,
+static int gangs_for(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_kv, int64_t group, int64_t max_len_extend,
                      int64_t head_dim, int64_t window, int key_splits) {
   if (head_dim != 128 || msgl::tile_variant() != 0 || t_gangs < 0) return 0;
-  return msgl::prefill_gangs(batch, total_kv, n_kv, group, max_len_extend, window, msgl::kPrefillBlockRows,
+  return msgl::prefill_gangs(batch, total_q, total_kv, n_kv, group, max_len_extend, window, msgl::kPrefillBlockRows,
                              t_gangs > 0 ? 1 : key_splits, t_key_splits, /*whatever_the_size=*/t_gangs > 0);
 }
 
@@ -444,9 +444,10 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
     if (ragged > 0)
       return std::max(share_need, msgl::prefill_ragged_workspace_bytes(batch, total_kv, num_kv_heads, group,
                                                                        max_len_extend, head_dim, ragged));
-    const int k = msgl::prefill_key_splits(batch, total_kv, num_kv_heads, group, max_len_extend, 0,
-                                           msgl::prefill_block_rows(head_dim), t_key_splits);
-    const int gangs = gangs_for(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim, 0, k);
+    const int k = msgl::prefill_key_splits(batch, total_q, total_kv, num_kv_heads, group, max_len_extend, 0, head_dim,
+                                           t_key_splits);
+    // (the slots of gang ranges are the same however many queries there are)
+    const int gangs = gangs_for(batch, batch * max_len_extend, total_kv, num_kv_heads, group, max_len_extend, head_dim, 0, k);
     const size_t split_need = std::max(share_need, msgl::prefill_split_workspace_bytes(total_q, num_q_heads, head_dim, k));
     if (gangs > 0)
       return std::max(split_need, msgl::prefill_gang_workspace_bytes(batch, num_kv_heads, group, max_len_extend, gangs));
@@ -563,9 +564,8 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) a.ragged_tiles = 0;
     else a.workspace = workspace;
   } else {
-    a.key_splits = msgl::prefill_key_splits(batch, total_kv, num_kv_heads, group, max_len_extend,
-                                            sliding_window_size, msgl::prefill_block_rows(head_dim),
-                                            t_key_splits);
+    a.key_splits = msgl::prefill_key_splits(batch, total_q, total_kv, num_kv_heads, group, max_len_extend,
+                                            sliding_window_size, head_dim, t_key_splits);
   }
   if (a.key_splits > 1) {
     // the split is an optimisation: without room for its partials the keys go in one pass
@@ -576,7 +576,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   a.gangs = 0;
   if (t_gangs > 0 && a.ragged_tiles == 0) a.key_splits = 1;  // forced for a test: gang ranges instead
   if (a.ragged_tiles == 0 && a.key_splits == 1) {
-    const int gangs = gangs_for(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
+    const int gangs = gangs_for(batch, total_q, total_kv, num_kv_heads, group, max_len_extend, head_dim,
                                 sliding_window_size, a.key_splits);
     // so are gang ranges: without room for their slots every unit goes to one workgroup per query block
     if (gangs > 0 && workspace && aligned16(workspace) &&

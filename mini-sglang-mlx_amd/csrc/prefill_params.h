@@ -1,5 +1,7 @@
 // Kernel parameter block and launch geometry shared by the prefill tile kernels.
 #pragma once
+#include <algorithm>
+
 #include "msgl_internal.h"
 
 namespace msgl {
@@ -62,7 +64,7 @@ constexpr int kPrefillBlockRows256 = 128;   // head_dim 256
 // query block are shared out over several workgroups.
 constexpr int kComputeUnits = 256;
 constexpr int kMaxKeySplits = 32;
-constexpr int kMinKeysPerSplit = 1024;
+constexpr int kMinTilesPerSplit = 2;
 
 inline int prefill_block_rows(int64_t head_dim) {
   return head_dim == 256 ? kPrefillBlockRows256 : kPrefillBlockRows;
@@ -86,34 +88,50 @@ inline int64_t prefill_blocks_per_xcd(int64_t n_units, int64_t n_qblk) {
 }
 
 // Number of key splits for a launch, from sizes the host knows (the per-request lengths stay on
-// the device: the average visible length stands for all of them).  Cost model: the (request, kv
-// head, split) units are dealt round-robin to the 8 XCDs, a unit brings its query blocks, and an
-// XCD runs its workgroups in rounds of one per compute unit; a split costs a few percent (its
-// partial, the merge).  The count minimises rounds(k) / k * (1 + 0.03 (k - 1)); launches of more
-// than four rounds are left alone.  `forced` > 0 overrides (clamped to kMaxKeySplits).
-inline int prefill_key_splits(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t group,
-                              int64_t max_len_extend, int64_t window, int block_rows,
-                              int64_t forced) {
+// the device: the average visible length stands for all of them).  The (request, kv head, split)
+// units are dealt round-robin to the 8 XCDs, a unit brings its query blocks, and an XCD runs its
+// workgroups in rounds of one per compute unit.  A launch then takes about
+//   rounds x (10 us + 1.2 us x tiles / k)  +  for k > 1: 8 us + k partials written and read at 12 TB/s
+// (a block's beginning and end; a tile; the merge launch and the wait in front of it).  On 500 launches of 1-10
+// requests of 5-2500 tokens on prefixes up to 30 K, of even and uneven lengths, with and without a window or a causal
+// mask, at 7 head configurations of both head sizes, each timed with 1-16 splits, the count that this chooses is
+// 1.6 % from the best on average (one pass always: 28 %; rounds / k with 3 % a split and 1024 keys or more in one:
+// 9.4 %).  The best is mostly the largest that stays in one round, however short the splits (16 / 8 heads, 152 tokens on
+// 1000: 32.4 us in one pass, 23.9 in 6 splits; on 4000: 38.4 in 4, 28.9 in 16), unless the partials cost
+// more than it saves (32 / 8, 1000 tokens on 1000: 51 us in 1 and in 2), and a second round is rarely worth
+// it (24 / 4 heads of 256, 1000 tokens on 6000: 181 us in one pass, 203 in 4 splits).
+// Fewer visible keys never mean more splits: both the cost apart from the tiles and the bound grow with k.
+// `forced` > 0 overrides (clamped to kMaxKeySplits).
+inline int prefill_key_splits(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_kv, int64_t group,
+                              int64_t max_len_extend, int64_t window, int64_t head_dim, int64_t forced) {
   if (forced > 0) return (int)(forced < kMaxKeySplits ? forced : kMaxKeySplits);
-  if (batch <= 0) return 1;
+  if (batch <= 0 || max_len_extend <= 0) return 1;
   constexpr int64_t kXcds = 8, kUnitsPerXcd = kComputeUnits / kXcds;
+  constexpr double kRoundUs = 10.0, kTileUs = 1.2, kMergeUs = 8.0, kPartialBytesPerUs = 12e6;
+  const int block_rows = prefill_block_rows(head_dim);
   const int64_t n_qblk = (max_len_extend * group + block_rows - 1) / block_rows;
-  const int64_t pairs = batch * n_kv;
+  // Requests shorter than the longest leave some of the grid's blocks empty, which end at once.  In one pass the
+  // others go in order of length (see prefill_by_length()) and fill the rounds; splits of them do not, and the XCD
+  // that has the longest requests' counts: a fifth on top of the average.
+  const int64_t grid_blocks = batch * n_qblk, filled = (total_q * group + block_rows - 1) / block_rows + batch / 2;
   auto rounds = [&](int64_t k) {
-    const int64_t blocks = prefill_blocks_per_xcd(pairs * k, n_qblk);  // on the busiest XCD
-    return (blocks + kUnitsPerXcd - 1) / kUnitsPerXcd;
+    const int64_t grid = prefill_blocks_per_xcd(batch * n_kv * k, n_qblk);  // on the busiest XCD
+    const int64_t uneven = (6 * grid * filled + 5 * grid_blocks - 1) / (5 * grid_blocks);
+    if (k == 1 && filled < grid_blocks) return std::max(1.0, (double)(grid * filled) / (double)(grid_blocks * kUnitsPerXcd));
+    return (double)((std::min(grid, uneven) + kUnitsPerXcd - 1) / kUnitsPerXcd);
   };
-  if (n_qblk <= 0 || rounds(1) > 4) return 1;
+  if (rounds(1) > 4) return 1;  // what splits could even out is then little
   int64_t keys = total_kv / batch;
-  if (window > 0 && keys > window + max_len_extend) keys = window + max_len_extend;
-  int64_t most = keys / kMinKeysPerSplit;
-  if (most > kMaxKeySplits) most = kMaxKeySplits;
+  if (window > 0 && keys > window + block_rows / group) keys = window + block_rows / group;  // a block sees that many
+  const double tiles = (double)keys / kBN;
+  const double partial_us = (double)total_q * (double)(n_kv * group) * (double)head_dim * 2 * sizeof(float) / kPartialBytesPerUs;
+  const int64_t most = keys / (kMinTilesPerSplit * kBN) < kMaxKeySplits ? keys / (kMinTilesPerSplit * kBN) : kMaxKeySplits;
   int best = 1;
-  double best_cost = (double)rounds(1);
+  double best_us = rounds(1) * (kRoundUs + kTileUs * tiles);
   for (int64_t k = 2; k <= most; ++k) {
-    const double cost = (double)rounds(k) / (double)k * (1.0 + 0.03 * (double)(k - 1));
-    if (cost < best_cost) {
-      best_cost = cost;
+    const double us = rounds(k) * (kRoundUs + kTileUs * tiles / (double)k) + kMergeUs + (double)k * partial_us;
+    if (us < best_us) {
+      best_us = us;
       best = (int)k;
     }
   }
@@ -209,9 +227,17 @@ constexpr int kMinRounds = 4, kMaxRounds = 64;
 // rows, row maxima and row sums in its slot and counts itself; the part that counts last adds the
 // others to its registers and writes the result.  Returns gangs per XCD, 0 when the launch does
 // not qualify (the host knows sizes, not lengths).
+//
+// A gang stops at every unit's end and waits there for its longest workgroup, and a unit with fewer blocks than the
+// gang has workgroups leaves some idle; blocks in order of length have neither, but pack whole blocks.  Beyond one
+// round, then, gangs are for extends of about one length on long prefixes (time of gangs / of the order; 32 / 8,
+// 16 / 8 and 64 / 8 heads, 2-6 rounds): on 6000 cached 0.93-1.0, 0-16 K 0.92-1.0, 0-32 K 0.91-0.99, but on 0-12 K
+// 1.0-1.04, 1000-6000 1.03-1.17, 0-2000 1.1-1.2; extends of 0.3-1 of the longest 1.06-1.24 whatever the prefixes,
+// of 0.8-1 like those of one length.  In one round: 0.76-0.93 on 0-8 K, 0.98-1.08 on prefixes of one length.
 constexpr int kGangMaxUnits = 256;   // units per XCD
 constexpr int kGangMinTiles = 48;    // key tiles per gang below which one pass per unit is kept
-inline int prefill_gangs(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t group,
+constexpr int kGangLongMean = 6144;  // mean keys of a request from which gangs pay beyond one round
+inline int prefill_gangs(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_kv, int64_t group,
                          int64_t max_len_extend, int64_t window, int block_rows, int key_splits,
                          int64_t forced_splits, bool whatever_the_size = false) {
   if (forced_splits > 0 || key_splits > 1 || window > 0 || batch <= 0 || batch > kRankedBatch) return 0;
@@ -223,6 +249,7 @@ inline int prefill_gangs(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t 
   const int64_t gangs = kUnitsPerXcd / n_qblk;
   if (whatever_the_size) return (int)gangs;
   if (n_pairs / 8 < gangs) return 0;  // fewer units than gangs: key splits are the tool
+  if (n_pairs / 8 > gangs && (total_kv < kGangLongMean * batch || 4 * total_q < 3 * batch * max_len_extend)) return 0;
   const int64_t tiles_per_xcd = prefill_tiles_bound(batch, total_kv) * n_kv / 8;
   if (tiles_per_xcd < gangs * kGangMinTiles) return 0;
   return (int)gangs;

@@ -473,3 +473,29 @@ def test_tile_route_ragged_shares_many_requests(gpu, head_dim, q_len):
                             kv_lens=[n + q_len for n in lens], extend_lens=[q_len] * len(lens),
                             pool_factor=1.1, store_new=True)
         _check(wl, gpu, f"tile route, {len(lens)} requests, d={head_dim} q_len={q_len} first={lens[0]}")
+
+
+@pytest.mark.parametrize("head_dim,n_q,n_kv,kv,ext,window", [
+    (128, 16, 8, [152 + 1000], [152], 0),               # splits of 2-3 tiles
+    (128, 16, 8, [152 + 4000], [152], 0),               # more splits than a merge asks for together
+    (128, 16, 8, [400 + 5000], [400], 1024),            # the window's keys are what is split
+    (128, 8, 1, [600, 90 + 33, 3000], [600, 90, 200], 0),  # requests of few tiles: empty splits
+    (256, 24, 4, [152 + 1000], [152], 0),
+    (256, 16, 2, [200, 64 + 40, 6500], [100, 64, 150], 0),
+])
+def test_short_splits(gpu, head_dim, n_q, n_kv, kv, ext, window):
+    """Small launches split by the rule alone, against the oracle and against one pass over the keys."""
+    from mini_sglang_amd_kernel import _lib
+
+    need = _lib.load().msgl_paged_prefill_workspace_bytes(len(kv), sum(ext), sum(kv), n_q, n_kv, head_dim, max(ext))
+    assert need >= 4 * sum(ext) * n_q * (head_dim + 1) * 4  # four splits or more
+    wl = build_workload("t", "prefill", seed=780 + sum(ext), n_q=n_q, n_kv=n_kv, head_dim=head_dim, kv_lens=kv, extend_lens=ext,
+                        pool_factor=1.2, store_new=True, sliding_window_size=window)
+    _check(wl, gpu, f"short splits head_dim={head_dim} heads={n_q}/{n_kv} kv={kv} W={window}")
+    got, _ = run_gpu(wl, gpu)
+    _lib.set_tuning(_lib.TUNE_PREFILL_KEY_SPLITS, 1)
+    try:
+        one_pass, _ = run_gpu(wl, gpu)
+    finally:
+        _lib.set_tuning(_lib.TUNE_PREFILL_KEY_SPLITS, 0)
+    assert_close_bf16(got, one_pass.float(), "short splits vs one pass", max_tol=8e-3, mean_tol=4e-4)
