@@ -12,7 +12,8 @@
 // the state, so the serial part of a chunk is five products.
 //
 // Token after token a request costs 0.33 us per token whatever the chip has free; here a chunk of 64 costs
-// 4.4 us.  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32: 1353 -> 287 us; one of 1024: 298 -> 78.
+// 4.3 us, or 3.2 us in pairs of waves (below).  Requests of 992, 1581, 4005 and 1601 tokens at hk 16, hv 32:
+// 1353 -> 217 us (283 without pairs); one of 2000: 147 -> 109.
 //
 // Work: one workgroup per (request, value head, half of its 128 rows).  Waves 0-3 ("state" waves, 16
 // rows each, S^T in 32 accumulator registers) run the serial part of chunk j; waves 4-7 ("chunk" waves,
@@ -23,15 +24,27 @@
 //      2     R = beta (V - G X), U = T R           A, the decay ratios of P, the diagonal blocks of T of chunk j + 1
 //      3     Y = G Z + P U, S = G_64 S + K^T U     P, the blocks of T below the diagonal, V of chunk j + 1;
 //                                                  decay products of chunk j + 2
-// What bounds it: a chunk takes 10.6 K cycles (slots of 3.3, 2.9 and 4.4 K), in which a SIMD has 5.3 K cycles of
+// What bounds it: a chunk takes 10.4 K cycles (slots of 3.4, 2.6 and 4.3 K), in which a SIMD has 5.3 K cycles of
 // matrix instructions and as many of vector instructions in two chains that wait for their own results, and a
 // wave that has the SIMD for itself still pays about 5 cycles per instruction of any kind.  The last wave of a slot is
-// a chunk wave in all three, 0.6 K, 0.4 K and 0.5 K cycles behind the slowest state wave.  Hence: fp32 values
+// a chunk wave in slots 1 and 3, some 0.4 K cycles behind the slowest state wave.  Hence: fp32 values
 // are split by the matrix pipe (see Split: 16 instructions instead of 44), Z and Y are made transposed (4 stores
-// of 8 bytes a chunk instead of 16 of 2), V comes by transposing LDS reads, and the chunk waves share the blocks
-// out evenly (12.5 -> 10.7 K).  T and P of all chunks in a launch of their own, in parallel, measured the same
-// for the longest request of a launch and less for many short ones: their 20 KB per chunk and head cost 40 us
-// of writing for the requests above, and LDS and issue time in the serial part.
+// of 8 bytes a chunk instead of 16 of 2), V comes by transposing LDS reads, the chunk waves share the blocks
+// out evenly (12.5 -> 10.7 K), and what a block needs from LDS is read whether it is used or not (no branches, so the
+// reads of several blocks go out together: 10.6 -> 10.4 K).  T and P of all chunks in a launch of their own, in
+// parallel, measured the same for the longest request of a launch and less for many short ones: their 20 KB per chunk
+// and head cost 40 us of writing for the requests above, and LDS and issue time in the serial part.
+//
+// Pairs: the longest request's chain ends a launch when the others have left their compute units, and a launch of few
+// requests never fills the chip.  Such requests go on four workgroups a value head, of 32 rows: waves 0-1 are state
+// waves, and waves 2-3 ("output" waves) take what the next chunk does not wait for, Z and Y, from the S and U that
+// their state wave leaves in LDS, and P:
+//     slot   state waves, chunk j          output waves                  chunk waves
+//      1     X, R                           Z, two blocks of P to LDS      T of chunk j, K and Q of chunk j + 1 to LDS
+//      2     U, two blocks of A of j + 1    P of chunk j + 1               A, the diagonal blocks of T of chunk j + 1
+//      3     S                              Y, three blocks of P to LDS    the other blocks of T of chunk j + 1, V of j + 2
+// A chunk takes 7.7 K cycles (slots of 2.5, 2.4 and 2.7 K, every role 2.0-2.6 K of each).  It is 1.5 times the work of
+// the chip for a chunk, so a launch that fills the compute units evenly has no pairs (see in_pairs()).
 //
 // Precision: fp32 throughout, as in the token kernel.  q, k, v are bf16 and enter the bf16 matrix
 // instructions as they are; fp32 operands (S, R, U, T, P) are split into three bf16 parts of 8
@@ -53,6 +66,8 @@
 // stored in that order; for S^T the transposing LDS reads of K (4 tokens x 16 dims) pick their dims so
 // that result tile 2 s + h holds dims 32 s + 8 g + 4 h + i, which makes the pair (2 s, 2 s + 1) of a lane
 // 8 consecutive dims, the natural order of K and Q.
+#include <algorithm>
+
 #include "gdn_params.h"
 #include "prefill_tile_common.h"
 
@@ -61,6 +76,7 @@ namespace {
 
 constexpr int kChunk = 64;        // tokens per chunk
 constexpr int kRowsPerWg = 64;    // dv rows of a workgroup
+constexpr int kRowsPaired = 32;   // where output waves take half of the state waves' work
 constexpr int kRanked = 512;      // requests ranked by length (one per thread)
 
 // T and P as operands: fragment f of row block m and contraction step c (32 columns), those that are not
@@ -68,9 +84,10 @@ constexpr int kRanked = 512;      // requests ranked by length (one per thread)
 constexpr int kFragments = 6;
 __device__ constexpr int fragment(int m, int c) { return c == 0 ? m : m + 2; }
 
+template <bool PAIRED>
 struct ChunkLds {
   uint16_t k[2][kChunk][kDK], q[2][kChunk][kDK];  // 16-byte pieces of a row in swizzled order (see piece())
-  uint16_t v[kChunk][kRowsPerWg];
+  uint16_t v[PAIRED ? 2 : 1][kChunk][PAIRED ? kRowsPaired : kRowsPerWg];
   u32x4_t t[3][kFragments][64], p[3][kFragments][64];  // T and P in three bf16 parts
   float a[kChunk][68];            // A of the chunk being prepared (blocks on and below the diagonal)
   float diag[4][16][20];          // inverses of the diagonal blocks of I + A
@@ -81,7 +98,10 @@ struct ChunkLds {
   float g[kChunk], pre[kChunk], suf[kChunk], quad_pre[kChunk], block[4], quad[16];
   float total[3];                 // G_64, chunks j .. j + 2 (last: the arrays above are read 16 bytes at a time)
   int request;
-  alignas(16) float p_largest[4 * 64];  // per lane of the chunk waves: largest() of P's diagonal blocks, all chunks
+  alignas(16) float p_largest[4 * 64];  // per lane of the waves that make P: largest() of P's diagonal blocks, all chunks
+};
+struct PairedLds : ChunkLds<true> {
+  f32x4_t s[2][8][64], u[2][4][64];  // a state wave's S and U for its output wave, registers as they are
 };
 
 // Piece `c` of 16 bytes of row `row` lies at this place.  LDS serves 8 lanes of a 16-byte read and 16 of an
@@ -306,7 +326,94 @@ __device__ __forceinline__ void token_by_token(int start, int end, int slot, int
   for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
 }
 
-__device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int slot, int hv,
+// Decay ratios G_t / G_i of block (r, c), transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n).  Below the
+// diagonal: token t's block up to it, whole blocks, token i's block behind it; on the diagonal: token t's quad up to
+// it and the quads between, then token by token down the columns (1 above the diagonal).
+struct Decays {
+  f32x4_t col;
+  float row;
+  template <typename Lds>
+  __device__ __forceinline__ void load(const Lds& lds, int r, int c) {
+    const int x16 = lane_id() & 15, g = lane_id() >> 4;
+    row = r == c ? lds.quad_pre[16 * r + x16] : lds.pre[16 * r + x16];
+    col = *reinterpret_cast<const f32x4_t*>(r == c ? &lds.g[16 * r + 4 * g] : &lds.suf[16 * c + 4 * g]);
+  }
+  template <typename Lds>
+  __device__ __forceinline__ f32x4_t below(const Lds& lds, int r, int c) const {
+    const float b1 = lds.block[1], b2 = lds.block[2];
+    return row * (c < 1 && r > 1 ? b1 : 1.0f) * (c < 2 && r > 2 ? b2 : 1.0f) * col;
+  }
+  template <typename Lds>
+  __device__ __forceinline__ f32x4_t diagonal(const Lds& lds, int r) const {
+    const int x16 = lane_id() & 15, g = lane_id() >> 4;
+    const float q1 = lds.quad[4 * r + 1], q2 = lds.quad[4 * r + 2];
+    const float far = row * (g < 1 && x16 >= 8 ? q1 : 1.0f) * (g < 2 && x16 >= 12 ? q2 : 1.0f);
+    f32x4_t ratio;
+    ratio[3] = (x16 >> 2) > g ? far : 1.0f;
+#pragma unroll
+    for (int i = 2; i >= 0; --i) ratio[i] = ratio[i + 1] * (4 * g + i + 1 <= x16 ? col[i + 1] : 1.0f);
+    return ratio;
+  }
+};
+// <k, q> or <k, k> of a block, transposed likewise
+__device__ __forceinline__ f32x4_t block_dots(const bf16x8_t (&columns)[4], const bf16x8_t (&rows)[4]) {
+  f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < 4; ++n) d = mfma_16x16x32(columns[n], rows[n], d);
+  return d;
+}
+__device__ __forceinline__ void load_block_rows(const uint16_t (*m)[kDK], int r, bf16x8_t (&x)[4]) {
+  const int x16 = lane_id() & 15, g = lane_id() >> 4;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) x[d] = operand(&m[16 * r + x16][8 * piece(x16, 4 * d + g)]);
+}
+
+// Block (r, c) of A below the diagonal, to LDS; returns its ratios.
+template <typename Lds>
+struct BelowBlock {
+  bf16x8_t kc[4], kr[4];
+  Decays decays;
+  float beta;
+  __device__ __forceinline__ void load(const Lds& lds, int par, int tri, int r, int c) {
+    load_block_rows(lds.k[par], c, kc);
+    load_block_rows(lds.k[par], r, kr);
+    beta = lds.beta[tri][16 * r + (lane_id() & 15)];
+    decays.load(lds, r, c);
+  }
+  __device__ __forceinline__ f32x4_t store(Lds& lds, int r, int c, f32x4_t dots) const {
+    const f32x4_t ratio = decays.below(lds, r, c);
+    *reinterpret_cast<f32x4_t*>(&lds.a[16 * r + (lane_id() & 15)][16 * c + 4 * (lane_id() >> 4)]) = beta * ratio * dots;
+    return ratio;
+  }
+};
+
+// Rows of Y from its transpose: a lane has of token 16 m + x16 the state rows 4 g ..
+struct Outputs {
+  uint32_t step, lane_at;
+  int tokens;
+  char* base;
+  __device__ __forceinline__ Outputs(const GdnParams& p, int start, int end, int hv, int row)
+      : step((uint32_t)p.hv * kDV * 2u), lane_at((lane_id() & 15) * step + 8 * (lane_id() >> 4)), tokens(end - start),
+        base(reinterpret_cast<char*>(p.y + ((int64_t)start * p.hv + hv) * kDV + row)) {}
+  __device__ __forceinline__ void store(int chunk, const f32x4_t (&z)[4]) const {
+    char* to = base + (int64_t)chunk * kChunk * step;
+    const int left = tokens - chunk * kChunk;
+    auto one = [&](int m) {
+      *reinterpret_cast<u32x2_t*>(to + (lane_at + 16 * m * step)) = u32x2_t{pack_bf16x2(z[m][0], z[m][1]), pack_bf16x2(z[m][2], z[m][3])};
+    };
+    if (left >= kChunk) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) one(m);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (16 * m + (lane_id() & 15) < left) one(m);
+    }
+  }
+};
+
+template <bool PAIRED, typename Lds>
+__device__ __forceinline__ void state_waves(const GdnParams& p, Lds& lds, int start, int end, int slot, int hv,
                                             int row, int column) {
   const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
   const int n_chunks = (end - start + kChunk - 1) / kChunk;
@@ -315,9 +422,7 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
 #pragma unroll
   for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
 
-  // a lane's part of Y: of token 16 m + x16 the rows 4 g ..
-  const uint32_t y_step = (uint32_t)p.hv * kDV * 2u, y_lane = x16 * y_step + 8 * g;
-  char* ybase = reinterpret_cast<char*>(p.y + ((int64_t)start * p.hv + hv) * kDV + row);
+  const Outputs y(p, start, end, hv, row);
   const Picker pick;
   // places of K's and Q's pieces in LDS: as operands, row x16, and transposed, row `trow`, per 32 dims
   const int trow = 4 * g + (x16 >> 2);
@@ -334,11 +439,23 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       r.k[m] = operand(&lds.k[par][16 * m][0] + at[c]);
-      r.q[m] = operand(&lds.q[par][16 * m][0] + at[c]);
+      if constexpr (!PAIRED) r.q[m] = operand(&lds.q[par][16 * m][0] + at[c]);
     }
   };
+  auto hand_over = [&](f32x4_t (*to)[64], const f32x4_t* from, int n) {
+#pragma unroll
+    for (int i = 0; i < n; ++i) to[i][lane] = from[i];
+  };
+  if constexpr (PAIRED) hand_over(lds.s[column >> 4], s, 8);
   __builtin_amdgcn_s_setprio(1);  // before the chunk waves, but in slot 2, where those have the longer way
+  auto a_block = [&](int par, int tri) {  // (3, 2), and the other state wave (2, 1)
+    const int r = column ? 2 : 3, c = r - 1;
+    BelowBlock<Lds> x;
+    x.load(lds, par, tri, r, c);
+    x.store(lds, r, c, block_dots(x.kc, x.kr));
+  };
   slot_barrier();  // K, Q of chunk 0
+  if constexpr (PAIRED) a_block(0, 0);
   slot_barrier();  // A of chunk 0
   slot_barrier();  // what T of chunk 0 is made of
 
@@ -348,6 +465,7 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
   float most = 0.f;  // largest() of every U
   for (int j = 0, tri = 0; j < n_chunks; ++j, tri = tri == 2 ? 0 : tri + 1) {
     const int par = j & 1;
+    Triangle tp;
     // ---- slot 1 ----------------------------------------------------------------------------
     f32x4_t x[4], z[4];  // X, and Z transposed: a lane's four values are neighbours in a row of Y
 #pragma unroll
@@ -361,7 +479,7 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
           x[m] = product<false>(r.k[m], part, x[m]);
-          z[m] = product<true>(r.q[m], part, z[m]);
+          if constexpr (!PAIRED) z[m] = product<true>(r.q[m], part, z[m]);
         }
       };
       const Split now = sp;
@@ -371,33 +489,51 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
       step(now.hi);
       fence();
     }
-    slot_barrier();
-    // ---- slot 2 ----------------------------------------------------------------------------
-    Triangle tp;
-    load_triangle<0, 4>(lds.t, tp);
-    f32x4_t u[4];
-    {
+    Split rs0, rs1;
+    auto make_r = [&]() {
       f32x4_t r[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const f32x4_t bet = *reinterpret_cast<const f32x4_t*>(&lds.beta[tri][16 * m + 4 * g]);
         const f32x4_t gam = *reinterpret_cast<const f32x4_t*>(&lds.gamma[tri][16 * m + 4 * g]);
-        const u32x2_t v = lds_read_tr16(reinterpret_cast<const unsigned char*>(&lds.v[16 * m + trow][column + 4 * (x16 & 3)]));
+        const u32x2_t v = lds_read_tr16(reinterpret_cast<const unsigned char*>(&lds.v[PAIRED ? par : 0][16 * m + trow][column + 4 * (x16 & 3)]));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           r[m][i] = (bf16_bits_to_f32(i & 1 ? v[i >> 1] >> 16 : v[i >> 1] & 0xffffu) - gam[i] * x[m][i]) * bet[i];
-        u[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
-      load_triangle<4, 6>(lds.t, tp);
-      const Split rs0 = split(pick, r[0], r[1]);
-      const Split rs1 = split(pick, r[2], r[3]);
-      triangle_first<false>(tp, rs0, u);
-      triangle_second<false>(tp, rs1, u);
-    }
+      if constexpr (!PAIRED) load_triangle<4, 6>(lds.t, tp);
+      rs0 = split(pick, r[0], r[1]);
+      rs1 = split(pick, r[2], r[3]);
+    };
+    if constexpr (PAIRED) make_r();
+    slot_barrier();
+    // ---- slot 2 ----------------------------------------------------------------------------
+    if constexpr (PAIRED) a_block(par ^ 1, tri == 2 ? 0 : tri + 1);  // of chunk j + 1 (of no use behind the last one)
+    load_triangle<0, PAIRED ? 6 : 4>(lds.t, tp);
+    if constexpr (!PAIRED) make_r();
+    f32x4_t u[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) z[m] *= lds.gamma[tri][16 * m + x16];
-    fence();
-    load_triangle<0, 4>(lds.p, tp);
+    for (int m = 0; m < 4; ++m) u[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    triangle_first<false>(tp, rs0, u);
+    triangle_second<false>(tp, rs1, u);
+    f32x4_t tail[4];
+    Split ut0, ut1;
+    auto take_tail = [&]() {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) tail[m] = *reinterpret_cast<const f32x4_t*>(&lds.tail[tri][16 * m + 4 * g]);
+    };
+    auto weigh = [&]() {
+      ut0 = split(pick, u[0] * tail[0], u[1] * tail[1]);
+      ut1 = split(pick, u[2] * tail[2], u[3] * tail[3]);
+    };
+    if constexpr (PAIRED) {
+      hand_over(lds.u[column >> 4], u, 4);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) z[m] *= lds.gamma[tri][16 * m + x16];
+      fence();
+      load_triangle<0, 4>(lds.p, tp);
+    }
     slot_barrier();
     // ---- slot 3 ----------------------------------------------------------------------------
     const uint16_t* k = &lds.k[par][0][0];
@@ -412,25 +548,25 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
       }
     };
     bf16x8_t ka[2][4];
-    f32x4_t tail[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) tail[m] = *reinterpret_cast<const f32x4_t*>(&lds.tail[tri][16 * m + 4 * g]);
+    take_tail();
     const float total = lds.total[tri];
-    load_triangle<4, 6>(lds.p, tp);
+    if constexpr (!PAIRED) load_triangle<4, 6>(lds.p, tp);
     load_kt(0, ka[0]);
     load_kt(1, ka[1]);
-    const Split us0 = split(pick, u[0], u[1]);
-    const Split us1 = split(pick, u[2], u[3]);
-    fence();
-    triangle_first<true>(tp, us0, z);
-    const Split ut0 = split(pick, u[0] * tail[0], u[1] * tail[1]);
-    const Split ut1 = split(pick, u[2] * tail[2], u[3] * tail[3]);
+    Split us1;
+    if constexpr (!PAIRED) {
+      const Split us0 = split(pick, u[0], u[1]);
+      us1 = split(pick, u[2], u[3]);
+      fence();
+      triangle_first<true>(tp, us0, z);
+    }
+    weigh();
 #pragma unroll
     for (int c = 0; c < 8; ++c) s[c] *= total;
 #pragma unroll
     for (int m = 0; m < 4; ++m) most = largest(u[m], most);
     fence();
-    triangle_second<true>(tp, us1, z);
+    if constexpr (!PAIRED) triangle_second<true>(tp, us1, z);
     auto steps = [&](int n, const Split& b) {
       auto step = [&](bf16x8_t part) {
 #pragma unroll
@@ -447,26 +583,16 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, ChunkLds& lds, i
     fence();
     load_kt(3, ka[1]);
     steps(2, ut0);
-    char* to = ybase + (int64_t)j * kChunk * y_step;
-    const int left = end - start - j * kChunk;
-    auto store = [&](int m) {
-      *reinterpret_cast<u32x2_t*>(to + (y_lane + 16 * m * y_step)) = u32x2_t{pack_bf16x2(z[m][0], z[m][1]), pack_bf16x2(z[m][2], z[m][3])};
-    };
-    if (left >= kChunk) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) store(m);
-    } else {
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-        if (16 * m + x16 < left) store(m);
-    }
+    if constexpr (!PAIRED) y.store(j, z);
     fence();
     load_rows(par ^ 1, 0, rows[0]);  // of chunk j + 1 (of no use behind the last chunk)
     steps(3, ut1);
     sp = split(pick, s[0], s[1]);
+    if constexpr (PAIRED) hand_over(lds.s[column >> 4], s, 8);
     slot_barrier();
   }
-  most = largest(*reinterpret_cast<const f32x4_t*>(&lds.p_largest[4 * lane]), most);
+  if constexpr (PAIRED) slot_barrier();  // the output waves' stores are done
+  most = largest(*reinterpret_cast<const f32x4_t*>(&lds.p_largest[4 * (PAIRED ? lane & 31 : lane)]), most);
   if (__builtin_expect(!__all(splits(most)), 0)) {
     wait_all_vm();  // the stores of Y: the same places are written again
     token_by_token(start, end, slot, hv, row);
@@ -508,10 +634,11 @@ __device__ __forceinline__ f32x4_t mfma_f32_block(f32x4_t a, f32x4_t b, f32x4_t 
 // Blocks (R, C) of T below the diagonal from those of A and the inverses on the diagonal:
 // T_RC = -T_RR X_R, X_R = sum over C <= k < R of A_Rk T_kC.  A block is made as the operand of the rows below it
 // and transposed, four neighbours of a row to a lane, for LDS (T_RC^T = -X_R^T T_RR^T).  Operands of that:
+template <typename Lds>
 struct Inverse {
-  const ChunkLds& lds;
+  const Lds& lds;
   int x16, g;
-  __device__ __forceinline__ explicit Inverse(const ChunkLds& l) : lds(l), x16(lane_id() & 15), g(lane_id() >> 4) {}
+  __device__ __forceinline__ explicit Inverse(const Lds& l) : lds(l), x16(lane_id() & 15), g(lane_id() >> 4) {}
   __device__ __forceinline__ f32x4_t a(int r, int k) const { return *reinterpret_cast<const f32x4_t*>(&lds.a[16 * r + x16][16 * k + 4 * g]); }
   __device__ __forceinline__ f32x4_t minus_diag(int r) const { return -*reinterpret_cast<const f32x4_t*>(&lds.diag[r][x16][4 * g]); }
   __device__ __forceinline__ f32x4_t diag_plain(int r) const {
@@ -522,7 +649,8 @@ struct Inverse {
   }
 };
 
-__device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, int start, int end, int hv,
+template <bool PAIRED, typename Lds>
+__device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int start, int end, int hv,
                                             int wg_row, int w) {
   const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
   const Picker pick;
@@ -535,16 +663,17 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
   const char* gbase = reinterpret_cast<const char*>(p.g + (int64_t)start * p.hv + hv);
   const char* bbase = reinterpret_cast<const char*>(p.beta + (int64_t)start * p.hv + hv);
   const uint32_t k_step = (uint32_t)p.k_stride0 * 2u, q_step = (uint32_t)p.q_stride0 * 2u, g_step = (uint32_t)p.hv * 2u;
-  // V of the workgroup's rows, 8 tokens a load, straight to LDS; rows past the request's end: the last row
+  // V of the workgroup's rows, 8 tokens a load (16 of half as many rows), straight to LDS; rows past the request's end: the last row
   // (beta is zero there)
   const char* vbase = reinterpret_cast<const char*>(p.v + (int64_t)start * p.v_stride0 + hv * kDV + wg_row);
-  const uint32_t v_step = (uint32_t)p.v_stride0 * 2u, v_lds = (uint32_t)(uintptr_t)MSGL_LDS_PTR(uint16_t, &lds.v[16 * w][0]);
-  auto fetch_v = [&](int first) {
+  const uint32_t v_step = (uint32_t)p.v_stride0 * 2u, v_lds = (uint32_t)(uintptr_t)MSGL_LDS_PTR(uint16_t, &lds.v[0][16 * w][0]);
+  auto fetch_v = [&](int first, int par = 0) {
     const char* base = vbase + (int64_t)(first - start) * v_step;
+    constexpr int kLanes = PAIRED ? 4 : 8;  // a token
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
-      lds_direct_b128(__builtin_amdgcn_readfirstlane(v_lds + 1024 * n), base,
-                      min((uint32_t)(16 * w + 8 * n + (lane >> 3)), (uint32_t)(end - 1 - first)) * v_step + 16 * (lane & 7));
+    for (int n = 0; n < kLanes / 4; ++n)
+      lds_direct_b128(__builtin_amdgcn_readfirstlane(v_lds + 1024 * n + par * (uint32_t)sizeof(lds.v[0])), base,
+                      min((uint32_t)(16 * w + 8 * n + lane / kLanes), (uint32_t)(end - 1 - first)) * v_step + 16 * (lane % kLanes));
   };
   u32x4_t kr[4], qr[4];
   uint32_t graw, braw;
@@ -607,63 +736,27 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
     if (lane == 0) lds.total[tri] = b0 * b1 * b2 * b3;
   };
   // The ten blocks (r, c) of A and P on and below the diagonal: every wave its diagonal block and one
-  // more, waves 1 and 2 two.  Results are transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n), so that a
+  // more, waves 1 and 2 two (PAIRED: the state waves have those).  Results are transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n), so that a
   // lane's four values are neighbours in a row of A and of P.
-  const int n_blocks = w == 0 || w == 3 ? 2 : 3;
+  const int n_blocks = PAIRED || w == 0 || w == 3 ? 2 : 3;
   auto block_row = [&](int n) { return n == 0 ? w : n == 1 ? (w == 0 ? 3 : w) : (w == 2 ? 2 : 3); };
   auto block_col = [&](int n) { return n == 0 ? w : n == 1 ? (w == 3 ? 1 : 0) : (w == 1 ? 2 : 1); };
-  f32x4_t pp[3];  // the ratios of P of these blocks, then P
+  f32x4_t pp0, pp1, pp2;  // the ratios of P of these blocks, then P
   float most = 0.f;  // largest() of P's diagonal block, every chunk
   f32x4_t inv;    // the inverse of the diagonal block: row x16, columns 4 g ..
   auto products = [&](int par, int tri) {
-    struct Block {
-      bf16x8_t kc[4], kr[4];
-      f32x4_t col;
-      float row, beta;
-    };
-    auto load = [&](int r, int c, Block& x) {
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        x.kc[d] = operand(&lds.k[par][16 * c + x16][8 * piece(x16, 4 * d + g)]);
-        x.kr[d] = operand(&lds.k[par][16 * r + x16][8 * piece(x16, 4 * d + g)]);
-      }
-      x.beta = lds.beta[tri][16 * r + x16];
-      x.row = r == c ? lds.quad_pre[16 * r + x16] : lds.pre[16 * r + x16];
-      x.col = *reinterpret_cast<const f32x4_t*>(r == c ? &lds.g[16 * r + 4 * g] : &lds.suf[16 * c + 4 * g]);
-    };
-    auto dots = [&](const Block& x) {
-      f32x4_t kk = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int d = 0; d < 4; ++d) kk = mfma_16x16x32(x.kc[d], x.kr[d], kk);
-      return kk;
-    };
-    // G_t / G_i of a block below the diagonal: token t's block up to it, whole blocks, token i's block behind it
-    auto below_block = [&](int n, int r, int c, const Block& x, const f32x4_t& kk) {
-      float row = x.row;
-      if (c < 1 && r > 1) row *= lds.block[1];
-      if (c < 2 && r > 2) row *= lds.block[2];
-      const f32x4_t ratio = row * x.col;
-      pp[n] = ratio;
-      *reinterpret_cast<f32x4_t*>(&lds.a[16 * r + x16][16 * c + 4 * g]) = x.beta * ratio * kk;
-    };
-    Block b0, b1, b2;
+    BelowBlock<Lds> b0, b1, b2;
     const int r1 = block_row(1), c1 = block_col(1), r2 = block_row(2), c2 = block_col(2);
-    load(w, w, b0);
-    load(r1, c1, b1);
-    const f32x4_t kk0 = dots(b0);
+    b0.load(lds, par, tri, w, w);
+    b1.load(lds, par, tri, r1, c1);
+    const f32x4_t kk0 = block_dots(b0.kc, b0.kr);
     {
-      // on the diagonal: token t's quad up to it and the quads between, then token by token down the columns
-      float far = b0.row;
-      if (g < 1 && x16 >= 8) far *= lds.quad[4 * w + 1];
-      if (g < 2 && x16 >= 12) far *= lds.quad[4 * w + 2];
-      f32x4_t ratio, a;
-      ratio[3] = (x16 >> 2) > g ? far : 1.0f;
-#pragma unroll
-      for (int i = 2; i >= 0; --i) ratio[i] = ratio[i + 1] * (4 * g + i + 1 <= x16 ? b0.col[i + 1] : 1.0f);
+      const f32x4_t ratio = b0.decays.diagonal(lds, w);
+      f32x4_t a;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         a[i] = 4 * g + i < x16 ? b0.beta * ratio[i] * kk0[i] : 0.f;
-        pp[0][i] = 4 * g + i <= x16 ? ratio[i] : 0.f;
+        if constexpr (!PAIRED) pp0[i] = 4 * g + i <= x16 ? ratio[i] : 0.f;
       }
       *reinterpret_cast<f32x4_t*>(&lds.a[16 * w + x16][16 * w + 4 * g]) = a;
     }
@@ -676,83 +769,86 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n) inv[n] = x16 == 4 * g + n ? 1.0f : 0.0f;
+    // (no two branches of a lambda end in stores to different captures: those become one store to a chosen address,
+    // and the captures go to scratch memory)
     if (n_blocks > 2) {
-      load(r2, c2, b2);
-      const f32x4_t kk1 = dots(b1), kk2 = dots(b2);
+      b2.load(lds, par, tri, r2, c2);
+      const f32x4_t kk1 = block_dots(b1.kc, b1.kr), kk2 = block_dots(b2.kc, b2.kr);
       eliminate<0>(arow, inv);
-      below_block(1, r1, c1, b1, kk1);
-      below_block(2, r2, c2, b2, kk2);
+      pp2 = b2.store(lds, r2, c2, kk2);
+      pp1 = b1.store(lds, r1, c1, kk1);
     } else {
-      const f32x4_t kk1 = dots(b1);
+      const f32x4_t kk1 = block_dots(b1.kc, b1.kr);
       eliminate<0>(arow, inv);
-      below_block(1, r1, c1, b1, kk1);
+      pp1 = b1.store(lds, r1, c1, kk1);
     }
     *reinterpret_cast<f32x4_t*>(&lds.diag[w][x16][4 * g]) = inv;
   };
   auto finish_p = [&](int par) {  // P = ratios times <k, q>
-#pragma unroll
-    for (int n = 0; n < 3; ++n) {
-      if (n >= n_blocks) break;
-      f32x4_t qk = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-        qk = mfma_16x16x32(operand(&lds.k[par][16 * block_col(n) + x16][8 * piece(x16, 4 * d + g)]),
-                           operand(&lds.q[par][16 * block_row(n) + x16][8 * piece(x16, 4 * d + g)]), qk);
-      pp[n] *= qk;
-    }
-    most = largest(pp[0], most);
+    auto times_dots = [&](int n, f32x4_t& x) {
+      bf16x8_t k[4], q[4];
+      load_block_rows(lds.k[par], block_col(n), k);
+      load_block_rows(lds.q[par], block_row(n), q);
+      x *= block_dots(k, q);
+    };
+    times_dots(0, pp0);
+    times_dots(1, pp1);
+    if (n_blocks > 2) times_dots(2, pp2);
+    most = largest(pp0, most);
   };
   // Blocks of T below the diagonal, two waves with the first column: (1, 0) and (2, 0); (2, 1) and (3, 1); (3, 2);
   // (3, 0).  Everything a chain needs from LDS is asked for before it starts.
-  f32x4_t below[2];
-  auto inverse = [&]() {
-    const Inverse of(lds);
+  struct Below {
+    f32x4_t first, second;
+  } below;
+  auto inverse = [&]() -> Below {
+    const Inverse<Lds> of(lds);
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     if (w == 2) {
       const f32x4_t a32 = of.a(3, 2), t2 = of.diag_plain(2), d3 = of.minus_diag(3);
-      below[0] = mfma_f32_block(mfma_f32_block(a32, t2, zero), d3, zero);
-    } else if (w == 1) {
+      return {mfma_f32_block(mfma_f32_block(a32, t2, zero), d3, zero), zero};
+    }
+    if (w == 1) {
       const f32x4_t a21 = of.a(2, 1), a31 = of.a(3, 1), a32 = of.a(3, 2), t1 = of.diag_plain(1), d2 = of.minus_diag(2), d3 = of.minus_diag(3);
       const f32x4_t x2 = mfma_f32_block(a21, t1, zero);
       f32x4_t x3 = mfma_f32_block(a31, t1, zero);
       const f32x4_t t21 = mfma_f32_block(d2, x2, zero);
-      below[0] = mfma_f32_block(x2, d2, zero);
+      const f32x4_t first = mfma_f32_block(x2, d2, zero);
       x3 = mfma_f32_block(a32, t21, x3);
-      below[1] = mfma_f32_block(x3, d3, zero);
-    } else {
-      const f32x4_t a10 = of.a(1, 0), a20 = of.a(2, 0), a21 = of.a(2, 1), t0 = of.diag_plain(0), d1 = of.minus_diag(1), d2 = of.minus_diag(2);
-      if (w == 0) {
-        const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
-        f32x4_t x2 = mfma_f32_block(a20, t0, zero);
-        const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
-        below[0] = mfma_f32_block(x1, d1, zero);
-        x2 = mfma_f32_block(a21, t10, x2);
-        below[1] = mfma_f32_block(x2, d2, zero);
-      } else {
-        const f32x4_t a30 = of.a(3, 0), a31 = of.a(3, 1), a32 = of.a(3, 2), d3 = of.minus_diag(3);
-        const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
-        f32x4_t x2 = mfma_f32_block(a20, t0, zero), x3 = mfma_f32_block(a30, t0, zero);
-        const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
-        x2 = mfma_f32_block(a21, t10, x2);
-        x3 = mfma_f32_block(a31, t10, x3);
-        const f32x4_t t20 = mfma_f32_block(d2, x2, zero);
-        x3 = mfma_f32_block(a32, t20, x3);
-        below[0] = mfma_f32_block(x3, d3, zero);
-      }
+      return {first, mfma_f32_block(x3, d3, zero)};
     }
+    const f32x4_t a10 = of.a(1, 0), a20 = of.a(2, 0), a21 = of.a(2, 1), t0 = of.diag_plain(0), d1 = of.minus_diag(1), d2 = of.minus_diag(2);
+    if (w == 0) {
+      const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
+      f32x4_t x2 = mfma_f32_block(a20, t0, zero);
+      const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
+      const f32x4_t first = mfma_f32_block(x1, d1, zero);
+      x2 = mfma_f32_block(a21, t10, x2);
+      return {first, mfma_f32_block(x2, d2, zero)};
+    }
+    const f32x4_t a30 = of.a(3, 0), a31 = of.a(3, 1), a32 = of.a(3, 2), d3 = of.minus_diag(3);
+    const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
+    f32x4_t x2 = mfma_f32_block(a20, t0, zero), x3 = mfma_f32_block(a30, t0, zero);
+    const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
+    x2 = mfma_f32_block(a21, t10, x2);
+    x3 = mfma_f32_block(a31, t10, x3);
+    const f32x4_t t20 = mfma_f32_block(d2, x2, zero);
+    x3 = mfma_f32_block(a32, t20, x3);
+    if constexpr (PAIRED) return {x3, d3};  // this chain is the longest of slot 3: the last product comes in slot 1
+    else return {mfma_f32_block(x3, d3, zero), zero};
   };
   auto store_t = [&]() {
+    f32x4_t first = below.first;
+    if (PAIRED && w == 3) first = mfma_f32_block(first, below.second, f32x4_t{0.f, 0.f, 0.f, 0.f});
     split_store(pick, inv, lds.t, w, w);
     const int r = w == 0 ? 1 : w == 1 ? 2 : 3, c = w == 1 ? 1 : w == 2 ? 2 : 0;
-    split_store(pick, below[0], lds.t, r, c);
-    if (w < 2) split_store(pick, below[1], lds.t, r + 1, c);
+    split_store(pick, first, lds.t, r, c);
+    if (w < 2) split_store(pick, below.second, lds.t, r + 1, c);
   };
   auto store_p = [&]() {
-#pragma unroll
-    for (int n = 0; n < 3; ++n) {
-      if (n >= n_blocks) break;
-      split_store(pick, pp[n], lds.p, block_row(n), block_col(n));
-    }
+    split_store(pick, pp0, lds.p, block_row(0), block_col(0));
+    split_store(pick, pp1, lds.p, block_row(1), block_col(1));
+    if (n_blocks > 2) split_store(pick, pp2, lds.p, block_row(2), block_col(2));
   };
 
   fetch(start);
@@ -763,17 +859,21 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
   if (n_chunks > 1) fetch(start + kChunk);
   products(0, 0);
   slot_barrier();
-  finish_p(0);
-  inverse();
+  if constexpr (!PAIRED) finish_p(0);
+  below = inverse();
   if (w == 2 && n_chunks > 1) decays(start + kChunk, 1);
+  if constexpr (PAIRED) {
+    wait_all_vm();  // V of chunk 0 is in LDS
+    if (n_chunks > 1) fetch_v(start + kChunk, 1);
+  }
   slot_barrier();
   int tri = 1;  // of chunk j + 1, modulo 3
   for (int j = 0; j < n_chunks; ++j) {
     const int next = start + (j + 1) * kChunk, par = (j + 1) & 1;
     const bool more = j + 1 < n_chunks, two = j + 2 < n_chunks;
     store_t();
-    store_p();
-    wait_all_vm();  // V of chunk j is in LDS
+    if constexpr (!PAIRED) store_p();
+    wait_all_vm();  // V of chunk j (PAIRED: j + 1) is in LDS
     if (more) stage(next, par);
     if (two) fetch(next + kChunk);
     slot_barrier();
@@ -782,27 +882,143 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, ChunkLds& lds, i
     __builtin_amdgcn_s_setprio(0);
     slot_barrier();
     tri = tri == 2 ? 0 : tri + 1;
+    if (PAIRED && two) fetch_v(next + kChunk, j & 1);
     if (more) {
-      fetch_v(next);
-      finish_p(par);
-      inverse();
+      if constexpr (!PAIRED) fetch_v(next);
+      if constexpr (!PAIRED) finish_p(par);
+      below = inverse();
     }
     if (w == 2 && two) decays(next + kChunk, tri);
-    if (!more) lds.p_largest[64 * w + lane] = most;
+    if (!PAIRED && !more) lds.p_largest[64 * w + lane] = most;
     slot_barrier();
   }
+  if constexpr (PAIRED) slot_barrier();
 }
 
-// Workgroup -> (request, value head, half): the workgroups that read the same K and Q rows (the value
-// heads of a key head, both halves) get ids of one residue modulo 8, so one L2 serves them; requests go
-// longest first where there are more workgroups than compute units.
-__global__ __launch_bounds__(512) void gdn_chunk_kernel(GdnParams p, int ranked) {
-  __shared__ __attribute__((aligned(16))) ChunkLds lds;
+// The half of a state wave's work that the next chunk does not wait for, and P: slot 1 of a chunk P to LDS and
+// Z = Q S^T, slot 2 P of the next chunk, slot 3 Y = G Z + P U.  S and U come from the state wave, one slot behind it.
+template <int w>
+__device__ __forceinline__ void output_waves(const GdnParams& p, PairedLds& lds, int start, int end, int hv, int row) {
+  const int lane = lane_id(), x16 = lane & 15, g = lane >> 4;
+  const int n_chunks = (end - start + kChunk - 1) / kChunk;
+  const Outputs y(p, start, end, hv, row);
+  const Picker pick;
+  // the blocks of P: wave 0 has (0, 0), (1, 1), (1, 0), (2, 0) and (2, 1), wave 1 (2, 2), (3, 3), (3, 0), (3, 1) and (3, 2)
+  constexpr int block_row[5] = {2 * w, 2 * w + 1, w ? 3 : 1, w ? 3 : 2, w ? 3 : 2};
+  constexpr int block_col[5] = {2 * w, 2 * w + 1, 0, w ? 1 : 0, w ? 2 : 1};
+  constexpr int kColumns = w ? 4 : 2, kFirstRow = w ? 2 : 0, kRows = w ? 2 : 3;  // of K, of Q
+  f32x4_t pp[5];
+  float most = 0.f;  // largest() of P's diagonal blocks, every chunk
+  auto make_p = [&](int par) {
+    bf16x8_t k[kColumns][4], q[kRows][4];
+#pragma unroll
+    for (int c = 0; c < kColumns; ++c) load_block_rows(lds.k[par], c, k[c]);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) load_block_rows(lds.q[par], kFirstRow + r, q[r]);
+#pragma unroll
+    for (int n = 0; n < 5; ++n) {
+      const int r = block_row[n], c = block_col[n];
+      Decays decays;
+      decays.load(lds, r, c);
+      f32x4_t ratio;
+      if (n < 2) {
+        ratio = decays.diagonal(lds, r);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ratio[i] = 4 * g + i <= x16 ? ratio[i] : 0.f;
+      } else {
+        ratio = decays.below(lds, r, c);
+      }
+      pp[n] = ratio * block_dots(k[c], q[r - kFirstRow]);
+      if (n < 2) most = largest(pp[n], most);
+    }
+  };
+  auto store_p = [&](int from, int to) {
+#pragma unroll
+    for (int n = 0; n < 5; ++n)
+      if (n >= from && n < to) split_store(pick, pp[n], lds.p, block_row[n], block_col[n]);
+  };
+  uint32_t at[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) at[c] = x16 * kDK + 8 * piece(x16, 4 * c + g);
+  slot_barrier();
+  make_p(0);
+  slot_barrier();
+  store_p(0, 3);
+  slot_barrier();
+  for (int j = 0, tri = 0; j < n_chunks; ++j, tri = tri == 2 ? 0 : tri + 1) {
+    const int par = j & 1;
+    f32x4_t z[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) z[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      bf16x8_t q[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) q[m] = operand(&lds.q[par][16 * m][0] + at[c]);
+      const Split sp = split(pick, lds.s[w][2 * c][lane], lds.s[w][2 * c + 1][lane]);
+      auto step = [&](bf16x8_t part) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) z[m] = product<true>(q[m], part, z[m]);
+      };
+      step(sp.lo);
+      step(sp.mid);
+      step(sp.hi);
+    }
+    store_p(3, 5);
+    slot_barrier();
+    Triangle tp;
+    load_triangle<0, 6>(lds.p, tp);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) z[m] *= lds.gamma[tri][16 * m + x16];
+    if (j + 1 < n_chunks) make_p(par ^ 1);
+    slot_barrier();
+    const Split us0 = split(pick, lds.u[w][0][lane], lds.u[w][1][lane]);
+    const Split us1 = split(pick, lds.u[w][2][lane], lds.u[w][3][lane]);
+    triangle_first<true>(tp, us0, z);
+    triangle_second<true>(tp, us1, z);
+    y.store(j, z);
+    store_p(0, 3);  // of the next chunk (of no use behind the last one)
+    slot_barrier();
+  }
+  lds.p_largest[64 * w + lane] = most;
+  wait_all_vm();  // the state waves may have to write the same places again
+  slot_barrier();
+}
+
+// Requests in pairs: the `n` longest, each on four workgroups a value head instead of two and so with two of the
+// `slots` that a request without takes one of.  As many as leave a slot for every request; and beyond that down to the
+// i-th longest, if the rest (chunks on the slots that are left, and what the last one of them may stick out) ends
+// before it: 3/4 of the time that it takes without.
+__device__ __forceinline__ bool in_pairs(int i, int chunks, int rest, int shortest, int batch, int slots) {
+  const int left = slots - 2 * (i + 1);
+  return i < slots - batch || (left > 0 && 4 * (rest + (left - 1) * shortest) <= 3 * left * chunks);
+}
+// How many there are at most.  Where these do not all fit beside the others, workgroups of places that stay empty wait
+// for a compute unit at the end of the launch: 1.3 us, which launches of short requests are spared.
+constexpr int kPairsMeanTokens = 768;
+inline int most_in_pairs(const GdnParams& p, int64_t cus) {
+  const int64_t slots = cus / (p.hv * (kDV / kRowsPerWg));
+  const int64_t long_ones = p.tokens >= (int64_t)kPairsMeanTokens * p.batch ? (slots - 1) / 2 : 0;
+  return p.batch > 64 ? 0 : (int)std::min<int64_t>(p.batch, std::max<int64_t>({slots - p.batch, long_ones, 0}));
+}
+
+// Workgroup -> (place, value head, half or quarter of its rows): the workgroups that read the same K and Q rows (the
+// value heads of a key head, their halves) get ids of one residue modulo 8, so one L2 serves them; a request in
+// pairs has two places.  Requests go longest first where there are more workgroups than compute units or some may go
+// in pairs.
+__global__ __launch_bounds__(512) void gdn_chunk_kernel(GdnParams p, int ranked, int places, int slots) {
+  __shared__ union {
+    ChunkLds<false> whole;
+    PairedLds paired;
+    struct {
+      int length[kRanked], request;
+    } order;
+  } lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int halves = kDV / kRowsPerWg;
   const int sharing = p.hv_per_hk * halves, hk_n = p.hv / p.hv_per_hk;
-  int group, member;  // group = (request, key head)
-  const int groups = p.batch * hk_n;
+  int group, member;  // group = (place, key head)
+  const int groups = places * hk_n;
   if (groups % 8 == 0) {
     const int seq = blockIdx.x >> 3;
     group = (seq / sharing) * 8 + (blockIdx.x & 7);
@@ -811,41 +1027,82 @@ __global__ __launch_bounds__(512) void gdn_chunk_kernel(GdnParams p, int ranked)
     group = blockIdx.x / sharing;
     member = blockIdx.x % sharing;
   }
-  int b = group / hk_n;
-  const int hv = (group - b * hk_n) * p.hv_per_hk + member / halves;
-  const int row = (member % halves) * kRowsPerWg;
-  if (ranked) {
-    int* lens = reinterpret_cast<int*>(&lds.k[0][0][0]);
-    const int tid = threadIdx.x;
-    int mine = 0;
-    if (tid < p.batch) lens[tid] = mine = p.qo_indptr[tid + 1] - p.qo_indptr[tid];
-    __syncthreads();
-    if (tid < p.batch) {
-      int rank = 0;
-      for (int o = 0; o < p.batch; ++o) rank += (lens[o] > mine || (lens[o] == mine && o < tid)) ? 1 : 0;
-      if (rank == b) lds.request = tid;
+  const int place = group / hk_n, half = member % halves;
+  const int hv = (group - place * hk_n) * p.hv_per_hk + member / halves;
+  int b = place, n_paired = 0;
+  int start, end;
+  if (p.batch <= 64 && (ranked || places > p.batch)) {  // every wave for itself, a request per lane
+    const int lane = lane_id(), at = min(lane, p.batch - 1);
+    const int from = p.qo_indptr[at], to = p.qo_indptr[at + 1];
+    const int length = lane < p.batch ? max(0, to - from) : -1;
+    int rank = 0, rest = 0, shortest = 0x7fffffff;
+    for (int o = 0; o < p.batch; ++o) {
+      const int other = __builtin_amdgcn_readlane(length, o), chunks = (other + kChunk - 1) / kChunk;
+      const bool before = other > length || (other == length && o < lane);
+      rank += before ? 1 : 0;
+      rest += before || o == lane ? 0 : chunks;
+      shortest = min(shortest, chunks);
     }
-    __syncthreads();
-    b = lds.request;
-    __syncthreads();
+    const bool pairs = lane < p.batch && rank < places - p.batch &&
+                       in_pairs(rank, (length + kChunk - 1) / kChunk, rest, shortest, p.batch, slots);
+    while (__ballot(pairs && rank >= n_paired)) ++n_paired;
+    const int wanted = place < 2 * n_paired ? place >> 1 : place - n_paired;
+    const uint64_t found = __ballot(lane < p.batch && rank == wanted);
+    if (!found) return;  // a place for a request in pairs that there is not: the whole workgroup
+    b = __builtin_ctzll(found);
+    start = __builtin_amdgcn_readlane(from, b);
+    end = __builtin_amdgcn_readlane(to, b);
+  } else {
+    if (ranked) {
+      const int tid = threadIdx.x;
+      int mine = 0;
+      if (tid < p.batch) lds.order.length[tid] = mine = p.qo_indptr[tid + 1] - p.qo_indptr[tid];
+      __syncthreads();
+      if (tid < p.batch) {
+        int rank = 0;
+        for (int o = 0; o < p.batch; ++o) rank += (lds.order.length[o] > mine || (lds.order.length[o] == mine && o < tid)) ? 1 : 0;
+        if (rank == b) lds.order.request = tid;
+      }
+      __syncthreads();
+      b = lds.order.request;
+      __syncthreads();
+    }
+    b = __builtin_amdgcn_readfirstlane(b);
+    start = p.qo_indptr[b];
+    end = p.qo_indptr[b + 1];
   }
-  b = __builtin_amdgcn_readfirstlane(b);
-  const int start = p.qo_indptr[b], end = min(p.qo_indptr[b + 1], p.tokens);
+  end = min(end, p.tokens);
   if (end <= start) return;  // the whole workgroup: the state stays as it is
+  const int slot = __builtin_amdgcn_readfirstlane(p.slot_ids[b]);
   // the blocks of T and P above the diagonal that are read are never written: zero from here on
-  for (int i = threadIdx.x; i < (int)(sizeof(lds.t) + sizeof(lds.p)) / 16; i += 512)
-    reinterpret_cast<u32x4_t*>(&lds.t[0][0][0])[i] = u32x4_t{0u, 0u, 0u, 0u};
-  if (wave < 4) state_waves(p, lds, start, end, __builtin_amdgcn_readfirstlane(p.slot_ids[b]), hv, row + 16 * wave, 16 * wave);
-  else chunk_waves(p, lds, start, end, hv, row, wave - 4);
+  auto clear = [](auto& t, auto& p) {
+    for (int i = threadIdx.x; i < (int)(sizeof(t) + sizeof(p)) / 16; i += 512)
+      reinterpret_cast<u32x4_t*>(&t[0][0][0])[i] = u32x4_t{0u, 0u, 0u, 0u};
+  };
+  if (place < 2 * n_paired) {
+    const int row = (place & 1) * kRowsPerWg + half * kRowsPaired;
+    clear(lds.paired.t, lds.paired.p);
+    if (wave < 2) state_waves<true>(p, lds.paired, start, end, slot, hv, row + 16 * wave, 16 * wave);
+    else if (wave == 2) output_waves<0>(p, lds.paired, start, end, hv, row);
+    else if (wave == 3) output_waves<1>(p, lds.paired, start, end, hv, row + 16);
+    else chunk_waves<true>(p, lds.paired, start, end, hv, row, wave == 6 ? 3 : wave == 7 ? 2 : wave - 4);
+  } else {
+    const int row = half * kRowsPerWg;
+    clear(lds.whole.t, lds.whole.p);
+    if (wave < 4) state_waves<false>(p, lds.whole, start, end, slot, hv, row + 16 * wave, 16 * wave);
+    else chunk_waves<false>(p, lds.whole, start, end, hv, row, wave - 4);
+  }
 }
 
 }  // namespace
 
 int launch_gdn_chunks(const GdnParams& p, hipStream_t stream) {
-  const int64_t blocks = (int64_t)p.batch * p.hv * (kDV / kRowsPerWg);
+  const int64_t cus = device_cus();
+  const int64_t places = p.batch + most_in_pairs(p, cus);
+  const int64_t blocks = places * p.hv * (kDV / kRowsPerWg);
   if (blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  const int ranked = p.batch > 1 && p.batch <= kRanked && blocks > device_cus();
-  hipLaunchKernelGGL(gdn_chunk_kernel, dim3((unsigned)blocks), dim3(512), 0, stream, p, ranked);
+  const int ranked = p.batch > 1 && p.batch <= kRanked && blocks > cus;
+  hipLaunchKernelGGL(gdn_chunk_kernel, dim3((unsigned)blocks), dim3(512), 0, stream, p, ranked, (int)places, (int)(cus / (p.hv * (kDV / kRowsPerWg))));
   return check_launch();
 }
 

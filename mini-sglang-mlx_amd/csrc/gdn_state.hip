@@ -160,16 +160,19 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 
 // Whether the chunk kernel (gdn_chunk.hip) is the faster one.  Its time for up to 64 tokens per request
 // does not depend on their number: 12.8 us for each round of workgroups (two per value head, one per
-// compute unit).  The token kernel's grows with the mean length, by 0.315 us per token while the requests
+// compute unit), or 9.2 us and 0.9 us per request of 32 heads where all requests go in pairs of waves (four
+// workgroups per value head, in one round).  The token kernel's grows with the mean length, by 0.315 us per token while the requests
 // run side by side and by 0.095 us per token and request of 32 heads beyond.  Both fitted to 1, 4, 16 and 64
-// requests of 8, 16, 32 and 64 tokens; they meet between 15 and 30 tokens.
+// requests of 8, 16, 32 and 64 tokens; they meet between 15 and 30 tokens (one request of 24 at 32 heads: 11.1 us token by token, 9.8 in a chunk; of 16:
+// 8.6 and 9.8).
 static bool prefer_chunks(const GdnArgs& a) {
   if (a.v_stride0 >= (1 << 24) || a.k_stride0 >= (1 << 24) || a.q_stride0 >= (1 << 24) || a.hv >= (1 << 17))
     return false;  // its offsets inside a chunk are 32 bits wide
   if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return false;  // loads of 16 bytes, stores of 8
   const double units = (double)(a.batch * a.hv) / 32, mean = (double)a.tokens / (double)a.batch;
   const double rounds = (double)((a.batch * a.hv * 2 + device_cus() - 1) / device_cus());
-  return 12.8 * rounds < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
+  const bool pairs = a.batch <= 64 && a.batch * a.hv * 4 <= device_cus();
+  return (pairs ? 9.2 + 0.9 * units : 12.8 * rounds) < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
 }
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 void gdn_set_rows(int v) { t_force_rows = (v == 1 || v == 2 || v == 4) ? v : 0; }
