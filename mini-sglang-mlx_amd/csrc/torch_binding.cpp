@@ -600,9 +600,9 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (total == 0 || batch <= 0 || slots == 0 || q.scalar_type() != at::kBFloat16 || !dev.is_cuda()) return none();
     const int64_t max_extend = integer(a[11]), window = integer(a[13]);
     const bool cross = truth(a[12]);
-    if (window < 0 || window > 0x7fffffff || max_extend > 0x7fffffff) return none();
-    const size_t bytes = msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross, static_cast<int32_t>(window));
-    if (bytes == 0) return none();
+    if (window < 0 || window > 0x7fffffff || max_extend <= 0 || max_extend > 0x7fffffff || (d != 128 && d != 256) || n_kv == 0 ||
+        n_q == 0 || n_q % n_kv != 0)
+      return none();
     if (const char* env = std::getenv("MSGL_DEBUG_CHECKS"); env && *env && std::strcmp(env, "0") != 0) return none();
     auto same = [&](const Tensor& x) { return x.scalar_type() == at::kBFloat16 && x.device() == dev; };
     auto ints_of = [&](const Tensor& x, int64_t n) {
@@ -626,11 +626,26 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       NoGil nogil;
       OnDevice on(dev);
       out = empty({total, n_q, d}, at::kBFloat16, dev);
-      const Tensor ws = scratch(bytes, dev);
-      rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), stride0(k), stride0(v), ints(loc), kc.data_ptr(),
-                            vc.data_ptr(), ints(qp), ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.data_ptr(), bytes, batch,
-                            total, ix.size(0), n_q, n_kv, d, slots, stride0(kc), stride0(vc), scale,
-                            static_cast<int32_t>(max_extend), cross ? 1 : 0, static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+      const int64_t ks0 = stride0(k), vs0 = stride0(v), kcs = stride0(kc), vcs = stride0(vc);
+      size_t bytes = msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross, static_cast<int32_t>(window));
+      if (bytes > 0) {
+        const Tensor ws = scratch(bytes, dev);
+        rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), ks0, vs0, ints(loc), kc.data_ptr(), vc.data_ptr(), ints(qp),
+                              ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.data_ptr(), bytes, batch, total, ix.size(0), n_q,
+                              n_kv, d, slots, kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
+                              static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+      } else {
+        rc = msgl_store_kv_cache(kc.data_ptr(), vc.data_ptr(), ints(loc), k.data_ptr(), v.data_ptr(), total, n_kv, d, slots, kcs,
+                                 vcs, ks0, vs0, 2, on.ptr());
+        if (rc == MSGL_OK) {
+          bytes = msgl_paged_prefill_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend);
+          const Tensor ws = scratch(bytes, dev);
+          rc = msgl_paged_prefill_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(qp), ints(ip), ints(ix), ints(pl),
+                                            out.data_ptr(), data_or_null(ws), bytes, batch, total, ix.size(0), n_q, n_kv, d, slots,
+                                            kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
+                                            static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+        }
+      }
     }
     check_rc(op, rc);
     return THPVariable_Wrap(std::move(out));
