@@ -234,13 +234,13 @@ MSGL_API int msgl_paged_prefill_attention(const void* q, const void* k_cache, co
 /*
  * A prefill call's store inside its attention launch -- AttnBackend.forward for prefill metadata
  * (mini_sglang_mlx/attention/backend.py:129-172): what msgl_store_kv_cache on (k, v, out_loc) and
- * msgl_paged_prefill_attention behind it do.  For short query blocks of small launches (speculative verify,
- * drafts): msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
+ * msgl_paged_prefill_attention behind it do.  For short query blocks (speculative verify,
+ * drafts) and small launches of up to some hundred tokens a request: msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
  * msgl_extend_step refuses them (MSGL_ERR_SHAPE).
  *   q, k, v, out_loc: total_q rows each, in the order of qo_indptr; leading strides of k and v free, q
  *   contiguous; bf16
- * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; the request then sees
- * the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
+ * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; with short query blocks
+ * the request then sees the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
  * request.  As with msgl_decode_step a slot of out_loc that is listed for another request may be read
  * before or after the row is there: such a batch takes the two calls.
  */

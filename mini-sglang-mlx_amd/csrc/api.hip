@@ -464,7 +464,8 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
   return std::max(split_need, tile_need);
 }
 
-int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void* v_cache,
+// `tokens`: rows that the launch stores first, where stores_in_tiles() holds; out_loc nullptr: none.
+static int prefill_attention(const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* qo_indptr, const int32_t* kv_indptr,
                                  const int32_t* kv_indices, const int32_t* prefix_lens, void* out,
                                  void* workspace, size_t workspace_bytes, int64_t batch,
@@ -472,7 +473,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
                                  int64_t num_kv_heads, int64_t head_dim, int64_t num_slots,
                                  int64_t k_cache_stride0, int64_t v_cache_stride0, float sm_scale,
                                  int32_t max_len_extend, int32_t is_cross_attention,
-                                 int32_t sliding_window_size, int32_t dtype, void* stream) {
+                                 int32_t sliding_window_size, int32_t dtype, const msgl::NewTokens& tokens, void* stream) {
   if (head_dim != 128 && head_dim != 256) return MSGL_ERR_HEAD_DIM;
   if (num_q_heads <= 0 || num_kv_heads <= 0) return MSGL_ERR_SHAPE;
   if (num_q_heads % num_kv_heads != 0) return MSGL_ERR_HEAD_RATIO;
@@ -555,7 +556,8 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   a.is_cross = is_cross_attention ? 1 : 0;
   a.window = sliding_window_size;
   a.key_splits = 1;
-  a.by_length = 1;
+  a.new_tokens = tokens;  // stored by the tile kernels alone (see stores_in_tiles())
+  a.by_length = tokens.out_loc == nullptr;
   a.ragged_tiles = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
   if (a.ragged_tiles > 0) {
     // ragged shares need room for their partials; without it the keys go in one pass
@@ -575,7 +577,7 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
   }
   a.gangs = 0;
   if (t_gangs > 0 && a.ragged_tiles == 0) a.key_splits = 1;  // forced for a test: gang ranges instead
-  if (a.ragged_tiles == 0 && a.key_splits == 1) {
+  if (a.ragged_tiles == 0 && a.key_splits == 1 && tokens.out_loc == nullptr) {
     const int gangs = gangs_for(batch, total_q, total_kv, num_kv_heads, group, max_len_extend, head_dim,
                                 sliding_window_size, a.key_splits);
     // so are gang ranges: without room for their slots every unit goes to one workgroup per query block
@@ -587,6 +589,21 @@ int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void*
     }
   }
   return head_dim == 256 ? msgl::launch_prefill_tile256(a, s) : msgl::launch_prefill_tile(a, s);
+}
+
+int msgl_paged_prefill_attention(const void* q, const void* k_cache, const void* v_cache,
+                                 const int32_t* qo_indptr, const int32_t* kv_indptr,
+                                 const int32_t* kv_indices, const int32_t* prefix_lens, void* out,
+                                 void* workspace, size_t workspace_bytes, int64_t batch,
+                                 int64_t total_q, int64_t total_kv, int64_t num_q_heads,
+                                 int64_t num_kv_heads, int64_t head_dim, int64_t num_slots,
+                                 int64_t k_cache_stride0, int64_t v_cache_stride0, float sm_scale,
+                                 int32_t max_len_extend, int32_t is_cross_attention,
+                                 int32_t sliding_window_size, int32_t dtype, void* stream) {
+  return prefill_attention(q, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, out, workspace, workspace_bytes,
+                           batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, num_slots, k_cache_stride0,
+                           v_cache_stride0, sm_scale, max_len_extend, is_cross_attention, sliding_window_size, dtype,
+                           msgl::NewTokens{}, stream);
 }
 
 // The plan of a prefill call whose store goes into its attention launch; share_len == 0: none
@@ -603,13 +620,40 @@ static msgl::SharePlan extend_step_plan(int64_t batch, int64_t total_q, int64_t 
   return shares_route(plan, window_share, batch, total_kv, keys, n_kv, group, max_len_extend, head_dim, window) ? plan : none;
 }
 
+// Whether a tile kernel of such a call stores the rows itself, every workgroup those of its request: in launches of one round,
+// of up to kRowsStored tokens a request (half as many at head_dim 256). us: one prompt of 30 tokens 11.8 -> 9.3, nine of 25-86
+// 16.8 -> 13.8, 20 of 20-40 on 200-300 23.0 -> 20.4, one of 163 14.3 -> 13.1; beyond the lines the stores in front of every
+// workgroup outweigh the launch: one of 250 on 2000 33.6 -> 35.0, of 250 on 1000 at 24 / 4 heads of 256 33.3 -> 36.8.
+constexpr int64_t kRowsStored = 192, kBytesStored = 16 << 20;
+static bool stores_in_tiles(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_q, int64_t n_kv, int64_t head_dim,
+                            int64_t max_len_extend, bool is_cross, int64_t window) {
+  if (batch <= 0 || total_q <= 0 || total_kv <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv != 0 || max_len_extend <= 0 ||
+      window < 0 || (head_dim != 128 && head_dim != 256) || max_len_extend * head_dim > kRowsStored * 128 || msgl::tile_variant() != 0 || t_gangs > 0)
+    return false;
+  const int64_t group = n_q / n_kv;
+  if (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) &&
+      !window_prefers_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim, window))
+    return false;
+  const int ragged = ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim);
+  if (ragged > 0) return msgl::prefill_ragged_units(batch, total_kv, ragged) * n_kv <= 2 * msgl::device_cus();
+  const int splits = msgl::prefill_key_splits(batch, total_q, total_kv, n_kv, group, max_len_extend, window, head_dim, t_key_splits);
+  const int64_t rows = msgl::prefill_block_rows(head_dim);
+  const int64_t blocks = batch * n_kv * splits * ((max_len_extend * group + rows - 1) / rows);
+  return blocks <= msgl::device_cus() && blocks * max_len_extend * head_dim * 4 <= kBytesStored;
+}
+
 size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv, int64_t num_q_heads,
                                         int64_t num_kv_heads, int64_t head_dim, int64_t max_len_extend,
                                         int32_t is_cross_attention, int32_t sliding_window_size) {
   const msgl::SharePlan plan = extend_step_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
                                                 is_cross_attention != 0, sliding_window_size);
-  if (plan.share_len == 0) return 0;
-  return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, num_q_heads / num_kv_heads * max_len_extend);
+  if (plan.share_len > 0)
+    return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, num_q_heads / num_kv_heads * max_len_extend);
+  if (!stores_in_tiles(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend, is_cross_attention != 0,
+                       sliding_window_size))
+    return 0;
+  return std::max<size_t>(16, msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim,
+                                                                 max_len_extend));
 }
 
 int msgl_extend_step(const void* q, const void* k, const void* v, int64_t k_stride0, int64_t v_stride0, const int32_t* out_loc,
@@ -628,7 +672,21 @@ int msgl_extend_step(const void* q, const void* k, const void* v, int64_t k_stri
   if (!aligned16(k) || !aligned16(v) || k_stride0 % 8 || v_stride0 % 8) return MSGL_ERR_ALIGNMENT;
   const msgl::SharePlan plan = extend_step_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
                                                 is_cross_attention != 0, sliding_window_size);
-  if (plan.share_len == 0) return MSGL_ERR_SHAPE;
+  msgl::NewTokens tokens{};
+  tokens.k = k;
+  tokens.v = v;
+  tokens.out_loc = out_loc;
+  tokens.k_stride0 = k_stride0;
+  tokens.v_stride0 = v_stride0;
+  if (plan.share_len == 0) {
+    const size_t need = msgl_extend_step_workspace_bytes(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
+                                                         is_cross_attention, sliding_window_size);
+    if (need == 0) return MSGL_ERR_SHAPE;
+    if (!workspace || !aligned16(workspace) || workspace_bytes < need) return MSGL_ERR_WORKSPACE;
+    return prefill_attention(q, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, out, workspace, workspace_bytes,
+                             batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, num_slots, k_cache_stride0,
+                             v_cache_stride0, sm_scale, max_len_extend, is_cross_attention, sliding_window_size, dtype, tokens, stream);
+  }
   const int64_t cols = num_q_heads / num_kv_heads * max_len_extend;
   if (!workspace || !aligned16(workspace) || workspace_bytes < msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, cols))
     return MSGL_ERR_WORKSPACE;
@@ -655,12 +713,6 @@ int msgl_extend_step(const void* q, const void* k, const void* v, int64_t k_stri
   a.q_cap = max_len_extend;
   a.is_cross = is_cross_attention ? 1 : 0;
   a.window = sliding_window_size;
-  msgl::NewTokens tokens{};
-  tokens.k = k;
-  tokens.v = v;
-  tokens.out_loc = out_loc;
-  tokens.k_stride0 = k_stride0;
-  tokens.v_stride0 = v_stride0;
   return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
 }
 

@@ -119,6 +119,7 @@ struct PrefillArgs {
   int32_t gangs;
   unsigned long long gang_nonce;
   int32_t by_length;  // query blocks may go in order of length (the fused kernel does not know that order)
+  NewTokens new_tokens;  // k, v, out_loc: rows that the launch stores (neither gangs nor by_length then)
 };
 int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream);     // head_dim 128
 // ---- paged_prefill_d256.hip ----------------------------------------------------------

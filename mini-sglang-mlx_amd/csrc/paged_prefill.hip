@@ -822,6 +822,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   int piece_a = 0, piece_b = 0x7fffff, unit_start = 0, unit_tiles = 0;  // gang ranges: tiles [a, b) of the unit
   bool piece_whole = true;
   LengthBlock by_length{};
+  RequestPlace place{};
   if (ganged) {
     if (piece > plan.last_unit) break;
     // the stages double as the staging area of the previous part's output: read out by now
@@ -850,9 +851,10 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   } else if (p.ragged_tiles > 0) {
     kvh = (int)(blockIdx.x % (unsigned)p.n_kv);
     const int u = (int)(blockIdx.x / (unsigned)p.n_kv);
-    const RaggedUnit ru = ragged_unit<NW * 64>(p, u, tid);
-    if (!ru.ok) return;
-    b = ru.request;
+    place = place_of<NW * 64>(p, u, tid);
+    if (!place.ok) return;
+    const RaggedUnit& ru = place.unit;
+    b = place.b;
     split = ru.share;
     qblk = 0;
     n_shares = ru.count;
@@ -870,7 +872,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     qblk = work.qblk;
     const int want_rank = pair / p.n_kv;
     kvh = pair - want_rank * p.n_kv;
-    b = request_of_rank<NW * 64>(p.kv_indptr, p.batch, want_rank, tid);
+    place = place_of<NW * 64>(p, want_rank, tid);
+    b = place.b;
   }
 
   // the request's geometry: gang ranges keep it in LDS, blocks in order of length have it in their list (a part or
@@ -905,12 +908,11 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     kn = by_length.kv_len;
     prefix = by_length.prefix;
   } else {
-    b = uniform(b);
-    q_start = p.qo_indptr[b];
-    q_len = min(p.qo_indptr[b + 1] - q_start, p.max_len_extend);
-    kv_start = p.kv_indptr[b];
-    kn = max(p.kv_indptr[b + 1] - kv_start, 0);
-    prefix = p.prefix_lens[b];
+    q_start = uniform(place.q_start);
+    q_len = min(uniform(place.q_len), p.max_len_extend);
+    kv_start = uniform(place.kv_start);
+    kn = uniform(place.kv_len);
+    prefix = uniform(place.prefix);
   }
   int rows_total = q_len * p.group;
   int row0 = qblk * kRows;
@@ -918,6 +920,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     if (ganged) continue;  // this request has no such query block
     return;
   }
+  if constexpr (ORDER == Order::kBatch)
+    if (p.out_loc != nullptr) store_request_rows<NW * 64, D>(p, q_start, uniform(place.q_len), kvh, tid);
 
   bool idle = __builtin_amdgcn_readfirstlane(row0 + w * 32 >= rows_total ? 1 : 0) != 0;
   if constexpr (!listed) {

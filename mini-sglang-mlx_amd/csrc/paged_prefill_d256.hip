@@ -86,12 +86,14 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   bool to_partial = p.n_ksplit > 1;  // leave a partial for the merge kernel, not the result
   int64_t part_at = 0;               // partial row of the block's row 0 (ragged shares)
   LengthBlock by_length{};
+  RequestPlace place{};
   if (p.ragged_tiles > 0) {
     kvh = (int)(blockIdx.x % (unsigned)p.n_kv);
     const int u = (int)(blockIdx.x / (unsigned)p.n_kv);
-    const RaggedUnit ru = ragged_unit<kNW * 64>(p, u, tid);
-    if (!ru.ok) return;
-    b = __builtin_amdgcn_readfirstlane(ru.request);
+    place = place_of<kNW * 64>(p, u, tid);
+    if (!place.ok) return;
+    const RaggedUnit& ru = place.unit;
+    b = place.b;
     split = ru.share;
     qblk = 0;
     n_shares = ru.count;
@@ -115,7 +117,8 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     qblk = work.qblk;
     const int want_rank = pair / p.n_kv;
     kvh = pair - want_rank * p.n_kv;
-    b = __builtin_amdgcn_readfirstlane(request_of_rank<kNW * 64>(p.kv_indptr, p.batch, want_rank, tid));
+    place = place_of<kNW * 64>(p, want_rank, tid);
+    b = place.b;
   }
 
   int q_start, q_len, kv_start, kn, prefix;
@@ -126,15 +129,16 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     kn = by_length.kv_len;
     prefix = by_length.prefix;
   } else {
-    q_start = __builtin_amdgcn_readfirstlane(p.qo_indptr[b]);
-    q_len = min(__builtin_amdgcn_readfirstlane(p.qo_indptr[b + 1]) - q_start, p.max_len_extend);
-    kv_start = __builtin_amdgcn_readfirstlane(p.kv_indptr[b]);
-    kn = max(__builtin_amdgcn_readfirstlane(p.kv_indptr[b + 1]) - kv_start, 0);
-    prefix = __builtin_amdgcn_readfirstlane(p.prefix_lens[b]);
+    q_start = __builtin_amdgcn_readfirstlane(place.q_start);
+    q_len = min(__builtin_amdgcn_readfirstlane(place.q_len), p.max_len_extend);
+    kv_start = __builtin_amdgcn_readfirstlane(place.kv_start);
+    kn = __builtin_amdgcn_readfirstlane(place.kv_len);
+    prefix = __builtin_amdgcn_readfirstlane(place.prefix);
   }
   const int rows_total = q_len * p.group;
   const int row0 = qblk * kRows;
   if (row0 >= rows_total) return;
+  if (p.out_loc != nullptr) store_request_rows<kNW * 64, kD>(p, q_start, __builtin_amdgcn_readfirstlane(place.q_len), kvh, tid);
 
   const int qi_lo = row0 / p.group;
   const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;

@@ -179,19 +179,12 @@ struct LengthOrder {
 };
 
 // ---- ragged shares: which (request, share) is unit `u`? ------------------------------------------
-// Visible key range of a request's only query block (rows 0 .. q_len * group - 1), the floor
-// rounded down to a tile: the kernels compute the same for their block.
-__device__ __forceinline__ void ragged_key_range(const PrefillParams& p, int b, int* k_lo, int* k_hi, int* q_len) {
-  const int ql = min(p.qo_indptr[b + 1] - p.qo_indptr[b], p.max_len_extend);
-  const int kn = max(p.kv_indptr[b + 1] - p.kv_indptr[b], 0);
-  const int prefix = p.prefix_lens[b];
-  int hi = p.is_cross ? kn : min(kn, prefix + ql);
-  int lo = (p.window > 0) ? max(0, prefix - p.window + 1) : 0;
-  lo &= ~(kBN - 1);
-  if (hi < lo) hi = lo;
-  *k_lo = lo;
-  *k_hi = hi;
-  *q_len = ql;
+// Shares of a request, from the visible keys of its only query block (rows 0 .. q_len * group - 1), the
+// floor rounded down to a tile: the kernels compute the same for their block.
+__device__ __forceinline__ int ragged_shares(const PrefillParams& p, int q_len, int kn, int prefix) {
+  const int hi = p.is_cross ? kn : min(kn, prefix + q_len);
+  const int lo = ((p.window > 0) ? max(0, prefix - p.window + 1) : 0) & ~(kBN - 1);
+  return q_len > 0 ? max(1, ((max(hi - lo, 0) + kBN - 1) / kBN + p.ragged_tiles - 1) / p.ragged_tiles) : 0;
 }
 struct RaggedUnit {
   int request, share, count, first;  // count = shares of the request, first = its first unit
@@ -209,10 +202,8 @@ __device__ __forceinline__ RaggedUnit ragged_unit(const PrefillParams& p, int u,
   const int wave = tid / kWave;
   if (tid == 0) found[0] = -1;
   for (int i = tid; i < p.batch; i += THREADS) {
-    int lo, hi, ql;
-    ragged_key_range(p, i, &lo, &hi, &ql);
-    const int tiles = (hi - lo + kBN - 1) / kBN;
-    count[i] = ql > 0 ? max(1, (tiles + p.ragged_tiles - 1) / p.ragged_tiles) : 0;
+    count[i] = ragged_shares(p, min(p.qo_indptr[i + 1] - p.qo_indptr[i], p.max_len_extend),
+                             max(p.kv_indptr[i + 1] - p.kv_indptr[i], 0), p.prefix_lens[i]);
   }
   __syncthreads();
   const int n_chunks = (p.batch + kWave - 1) / kWave;
@@ -425,6 +416,104 @@ __device__ __forceinline__ int request_of_rank(const int32_t* kv_indptr, int bat
   }
   __syncthreads();
   return found;
+}
+
+// A block's request where every one has a lane of the wave: all that a block wants to know of it comes in one memory
+// round trip, and every wave finds it by itself (a round trip, two barriers and some 0.5 us less at a block's beginning).
+struct RequestPlace {
+  int b, q_start, q_len, kv_start, kv_len, prefix;  // q_len: not capped
+  RaggedUnit unit;                                  // of a launch in ragged shares
+  bool ok;
+};
+// `at`: the wanted unit of ragged shares, or else the wanted rank by length
+__device__ __forceinline__ RequestPlace place_in_lanes(const PrefillParams& p, int at) {
+  const int lane = lane_id(), i = min(lane, p.batch - 1);
+  const int q_start = p.qo_indptr[i], q_end = p.qo_indptr[i + 1], kv_start = p.kv_indptr[i], kv_end = p.kv_indptr[i + 1];
+  const int prefix = p.prefix_lens[i], kv_len = max(kv_end - kv_start, 0);
+  RequestPlace r{};
+  unsigned long long hit;
+  int n = 0, first = 0;
+  if (p.ragged_tiles > 0) {
+    n = lane < p.batch ? ragged_shares(p, min(q_end - q_start, p.max_len_extend), kv_len, prefix) : 0;
+    first = wave_inclusive_scan(n) - n;
+    hit = __ballot(at >= first && at < first + n);
+  } else {
+    int rank = 0;
+    for (int o = 0; o < p.batch; ++o) {
+      const int other = __builtin_amdgcn_readlane(kv_end - kv_start, o);
+      rank += (other > kv_end - kv_start) || (other == kv_end - kv_start && o < lane);
+    }
+    hit = __ballot(lane < p.batch && rank == at);
+  }
+  if (hit == 0) return r;
+  const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+  r.b = src;
+  r.q_start = __builtin_amdgcn_readlane(q_start, src);
+  r.q_len = __builtin_amdgcn_readlane(q_end, src) - r.q_start;
+  r.kv_start = __builtin_amdgcn_readlane(kv_start, src);
+  r.kv_len = __builtin_amdgcn_readlane(kv_len, src);
+  r.prefix = __builtin_amdgcn_readlane(prefix, src);
+  r.unit.request = src;
+  r.unit.first = __builtin_amdgcn_readlane(first, src);
+  r.unit.share = at - r.unit.first;
+  r.unit.count = __builtin_amdgcn_readlane(n, src);
+  r.unit.ok = r.ok = true;
+  return r;
+}
+// The same of any number of requests.
+template <int THREADS>
+__device__ __forceinline__ RequestPlace place_of(const PrefillParams& p, int at, int tid) {
+  if (p.batch <= kWave) return place_in_lanes(p, at);
+  RequestPlace r{};
+  if (p.ragged_tiles > 0) {
+    r.unit = ragged_unit<THREADS>(p, at, tid);
+    if (!r.unit.ok) return r;
+    r.b = r.unit.request;
+  } else {
+    r.b = request_of_rank<THREADS>(p.kv_indptr, p.batch, at, tid);
+  }
+  r.b = __builtin_amdgcn_readfirstlane(r.b);
+  r.q_start = p.qo_indptr[r.b];
+  r.q_len = p.qo_indptr[r.b + 1] - r.q_start;
+  r.kv_start = p.kv_indptr[r.b];
+  r.kv_len = max(p.kv_indptr[r.b + 1] - r.kv_start, 0);
+  r.prefix = p.prefix_lens[r.b];
+  r.ok = true;
+  return r;
+}
+
+// A request's new rows of k and v of one kv head into the pool, by the whole workgroup, before it reads the pool: every
+// workgroup of a small launch does it for its own request (the same bytes, several times), which is less than the
+// launch that it saves.
+template <int THREADS, int D>
+__device__ __forceinline__ void store_request_rows(const PrefillParams& p, int q_start, int n, int kvh, int tid) {
+  constexpr int LANES = D / 8, ROWS = THREADS / LANES;  // of a row, side by side
+  const int col = kvh * D + 8 * (tid % LANES);
+  auto trips = [&](auto in_flight) {
+    constexpr int U = decltype(in_flight)::value;
+    for (int r0 = tid / LANES; r0 < n; r0 += ROWS * U) {
+      uint32_t slot[U];
+      u32x4_t k[U], v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t row = q_start + min(r0 + u * ROWS, n - 1);
+        slot[u] = (uint32_t)p.out_loc[row];
+        k[u] = ld_global_b128(p.new_k + row * p.new_k_stride0 + col);
+        v[u] = ld_global_b128(p.new_v + row * p.new_v_stride0 + col);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (r0 + u * ROWS >= n || slot[u] > p.max_slot) continue;  // a slot id outside the pool stores nothing
+        st_global_b128(const_cast<uint16_t*>(p.k_cache) + (int64_t)slot[u] * p.k_stride0 + col, k[u]);
+        st_global_b128(const_cast<uint16_t*>(p.v_cache) + (int64_t)slot[u] * p.v_stride0 + col, v[u]);
+      }
+    }
+  };
+  if (n <= ROWS) trips(std::integral_constant<int, 1>{});
+  else if (n <= 4 * ROWS) trips(std::integral_constant<int, 4>{});
+  else trips(std::integral_constant<int, 8>{});
+  wait_all_vm();
+  __syncthreads();
 }
 
 }  // namespace msgl

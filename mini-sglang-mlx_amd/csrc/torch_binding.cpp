@@ -586,7 +586,7 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 
 // ---- extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, sm_scale,
 //                  max_len_extend, is_cross_attention, sliding_window_size) -> out or None ---------------
-// As decode_step, for prefill metadata.
+// As decode_step, for prefill metadata; the two launches are made here too where one is not the way.
 PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 14, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "extend_step";

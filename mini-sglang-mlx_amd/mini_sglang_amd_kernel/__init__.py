@@ -281,10 +281,11 @@ def extend_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
                 kv_indptr: torch.Tensor, kv_indices: torch.Tensor, prefix_lens: torch.Tensor, *,
                 sm_scale: float, max_len_extend: int, is_cross_attention: bool = False,
                 sliding_window_size: int = 0) -> Optional[torch.Tensor]:
-    """``paged_prefill_attention`` with ``store_kv_cache`` of the queries' own rows of k and v inside: the
-    attention output, or ``None`` (nothing done) where the two calls are the way: longer query blocks,
-    large launches, forms that need a copy, arguments that they refuse, index validation on.  As with
-    ``decode_step`` a slot of ``out_loc`` must not be listed for another request.
+    """``store_kv_cache`` of the queries' own rows of k and v and ``paged_prefill_attention`` as one call: in one
+    launch where the query blocks are short or the launch is small, else as the two calls.  Returns the
+    attention output, or ``None`` (nothing done) where the two calls have to be made by themselves: forms
+    that need a copy, arguments that they refuse, index validation on.  As with ``decode_step`` a slot
+    of ``out_loc`` must not be listed for another request.
     """
     return _native.extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices,
                                prefix_lens, sm_scale, max_len_extend, is_cross_attention,

@@ -172,3 +172,28 @@ def test_extend_one_launch_is_two(gpu, tuning, cached, ext, n_q, n_kv, d, share,
         diff = (x - y).abs()
         assert e == 0 or (float(diff.max()) <= 2e-2 and float(diff.mean()) <= 1e-3), (float(diff.max()), float(diff.mean()))
         at += e
+
+
+# the same for longer query blocks, whose tile kernel stores the rows of its request: trips of 32 rows (16 at head_dim 256)
+# and of 4 and 8 times as many, requests beyond a wave's lanes, key splits and ragged shares, rows past the cap
+TILES = [
+    ([0, 0, 40], [31, 33, 0], 32, 8, 128, 0),
+    ([0, 500, 64], [127, 128, 32], 16, 8, 128, 0),
+    ([900], [192], 16, 8, 128, 0),
+    ([1000, 200], [90, 20], 16, 4, 128, 0),
+    ([100] * 70, [17 + i % 5 for i in range(70)], 8, 1, 128, 0),
+    ([100] * 64, [20] * 64, 8, 1, 128, 0),
+    ([0, 300], [250, 90], 32, 8, 128, 100),
+    ([0, 300, 20], [17, 96, 16], 24, 4, 256, 0),
+    ([79, 2000], [65, 15], 16, 2, 256, 0),
+    ([30] * 66, [9] * 66, 8, 1, 256, 0),
+]
+
+
+@pytest.mark.parametrize("cached,ext,n_q,n_kv,d,cap", TILES)
+@pytest.mark.parametrize("cross,window", [(False, 0), (True, 0), (False, 100)])
+@pytest.mark.parametrize("places", ["last", "mixed"])
+def test_extend_in_tiles_is_two(gpu, cached, ext, n_q, n_kv, d, cap, cross, window, places):
+    if places == "last" and not cross:  # (a full mask may be shared out otherwise)
+        assert _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(ext) + sum(cached), n_q, n_kv, d, cap or max(ext), 0, window) > 0
+    test_extend_one_launch_is_two(gpu, lambda *_: None, cached, ext, n_q, n_kv, d, 0, cap, cross, window, places)
