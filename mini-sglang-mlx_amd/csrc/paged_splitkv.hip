@@ -273,10 +273,10 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
   }
 }
 
-// One workgroup of NW waves per (request, query, q head): merge the partials of the segments
-// that share the request, by base-2 LSE.  Requests without visible keys get zeros; requests
+// One workgroup of four waves per (request, query, q head), for few rows cut into many segments: merge the partials
+// of the segments that share the request, by base-2 LSE.  Requests without visible keys get zeros; requests
 // that sat inside one segment were written by the attention kernel itself.
-// Up to kMergeSmall items (a request cut a few times: the usual case) one wave reads whole rows
+// Up to kMergeSmall items (a request cut a few times) one wave reads whole rows
 // and nothing crosses lanes.  Beyond that a partial row is taken as D / 8 chunks of 8 floats,
 // one chunk per lane, so a wave holds 64 / (D / 8) rows side by side and a workgroup
 // NG = NW * that many; each of these lane groups takes every NG-th item, one in the first trip
@@ -285,8 +285,10 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
 // round trips where a loop over its items needs a hundred.
 constexpr int kMergeUnroll = 3;
 constexpr int kMergeSmall = 8;
-template <int D, bool F16, int NW>
-__global__ __launch_bounds__(64 * NW) void splitkv_merge_kernel(SplitKvParams p) {
+constexpr int kMergeWaves = 4;
+template <int D, bool F16>
+__global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_kernel(SplitKvParams p) {
+  constexpr int NW = kMergeWaves;
   constexpr int LPI = D / 8;          // lanes per item
   constexpr int GPW = kWave / LPI;    // items side by side in a wave
   constexpr int NG = GPW * NW;        // ... and in the workgroup
@@ -432,25 +434,98 @@ __global__ __launch_bounds__(64 * NW) void splitkv_merge_kernel(SplitKvParams p)
     for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], off, kWave);
     wsum += __shfl_xor(wsum, off, kWave);
   }
-  if constexpr (NW > 1) {
-    __shared__ float fold[NW - 1][LPI][9];
-    if (wave > 0 && lane < LPI) {
+  __shared__ float fold[NW - 1][LPI][9];
+  if (wave > 0 && lane < LPI) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) fold[wave - 1][lane][e] = acc[e];
-      fold[wave - 1][lane][8] = wsum;
-    }
-    __syncthreads();
-    if (wave > 0) return;
-    if (lane < LPI) {
+    for (int e = 0; e < 8; ++e) fold[wave - 1][lane][e] = acc[e];
+    fold[wave - 1][lane][8] = wsum;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  if (lane < LPI) {
 #pragma unroll
-      for (int w = 0; w < NW - 1; ++w) {
+    for (int w = 0; w < NW - 1; ++w) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += fold[w][lane][e];
-        wsum += fold[w][lane][8];
-      }
+      for (int e = 0; e < 8; ++e) acc[e] += fold[w][lane][e];
+      wsum += fold[w][lane][8];
     }
   }
   if (lane >= LPI) return;
+  const float inv = (wsum > 0.f) ? 1.0f / wsum : 0.f;
+  u32x4_t w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = pack_16x2<F16>(acc[2 * e] * inv, acc[2 * e + 1] * inv);
+  st_global_b128(orow, w);
+}
+
+// The same for many rows: D / 8 lanes take a row (one q head of a query), a wave the rows of neighbouring heads, and
+// every lane the items by eight (four where there are no more), all their loads in flight together.  A workgroup of one
+// wave per row was bound by the launching of workgroups: us, 32 requests of 8 tokens at 32 heads 7.4 -> 6.4, 55 of 12
+// 11.1 -> 7.5, 13 of 5-16 at 16 heads 8.6 -> 6.0.
+template <int D, bool F16>
+__global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_rows_kernel(SplitKvParams p) {
+  constexpr int LPR = D / 8, RPW = kWave / LPR;
+  const int b = blockIdx.x / p.max_len_extend;
+  const int qi = blockIdx.x - b * p.max_len_extend;
+  const int lane = lane_id(), dl = lane % LPR;
+  const int hq = ((int)blockIdx.y * kMergeWaves + (int)(threadIdx.x >> 6)) * RPW + lane / LPR;
+  const int s_first = p.req_items[2 * b];
+  const int n_items = p.req_items[2 * b + 1];
+  const ReqInfo r = request_info(p, b);
+  if (qi >= r.q_len || hq >= p.n_q) return;
+  uint16_t* orow = p.out + ((int64_t)(r.q_start + qi) * p.n_q + hq) * D + dl * 8;
+  if (r.hi - r.lo == 0) {  // no visible key: nobody wrote req_items, the row is zero
+    st_global_b128(orow, u32x4_t{0u, 0u, 0u, 0u});
+    return;
+  }
+  if (n_items == 1) return;  // written by the attention kernel itself
+  const int kvh = hq / p.group;
+  const int col = qi * p.group + (hq - kvh * p.group);
+  const int64_t block0 = (int64_t)(s_first + b) * p.n_kv + kvh;  // item 0
+  float m = kNegInf, wsum = 0.f, acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  auto merge = [&](auto in_flight) {
+    constexpr int U = decltype(in_flight)::value;
+    for (int it0 = 0; it0 < n_items; it0 += U) {
+      float lse[U];
+      typename std::conditional<F16, f32x4_t[2], f16x8s_t[1]>::type v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // items past the last: that again, with weight 0
+        const int64_t block = block0 + (int64_t)min(it0 + u, n_items - 1) * p.n_kv;
+        const int64_t at = partial_offset(block, p.cols, col, dl * 8, D);
+        lse[u] = p.part_lse[block * p.cols + col];
+        if constexpr (F16) {
+          v[u][0] = *reinterpret_cast<const f32x4_t*>(p.part_o + at);
+          v[u][1] = *reinterpret_cast<const f32x4_t*>(p.part_o + at + 4);
+        } else {
+          v[u][0] = *reinterpret_cast<const f16x8s_t*>(reinterpret_cast<const _Float16*>(p.part_o) + at);
+        }
+        if (it0 + u >= n_items) lse[u] = kNegInf;
+      }
+      float m_new = m;
+#pragma unroll
+      for (int u = 0; u < U; ++u) m_new = fmaxf(m_new, lse[u]);
+      const float m_safe = m_new == kNegInf ? 0.f : m_new;
+      const float old = fast_exp2(m - m_safe);
+      m = m_new;
+      wsum *= old;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] *= old;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float w = fast_exp2(lse[u] - m_safe);  // 0 for an item that is not there
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (F16) acc[e] += w * v[u][e >> 2][e & 3];
+          else acc[e] += w * (float)v[u][0][e];
+        }
+        wsum += w;
+      }
+    }
+  };
+  if (n_items <= 4) merge(std::integral_constant<int, 4>{});
+  else merge(std::integral_constant<int, kMergeSmall>{});
   const float inv = (wsum > 0.f) ? 1.0f / wsum : 0.f;
   u32x4_t w;
 #pragma unroll
@@ -505,11 +580,13 @@ int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
   constexpr int kItemsPerTrip = kWave / (D / 8) * (1 + kMergeUnroll);
   const bool wide_merge = p.n_seg > kItemsPerTrip && (int64_t)mgrid.x * mgrid.y <= 1024;
   if (wide_merge) {
-    if (p.f16) hipLaunchKernelGGL((splitkv_merge_kernel<D, true, 4>), mgrid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((splitkv_merge_kernel<D, false, 4>), mgrid, dim3(256), 0, stream, p);
+    if (p.f16) hipLaunchKernelGGL((splitkv_merge_kernel<D, true>), mgrid, dim3(64 * kMergeWaves), 0, stream, p);
+    else hipLaunchKernelGGL((splitkv_merge_kernel<D, false>), mgrid, dim3(64 * kMergeWaves), 0, stream, p);
   } else {
-    if (p.f16) hipLaunchKernelGGL((splitkv_merge_kernel<D, true, 1>), mgrid, dim3(64), 0, stream, p);
-    else hipLaunchKernelGGL((splitkv_merge_kernel<D, false, 1>), mgrid, dim3(64), 0, stream, p);
+    constexpr unsigned kRows = kMergeWaves * (kWave / (D / 8));  // of a workgroup
+    const dim3 rows(mgrid.x, (mgrid.y + kRows - 1) / kRows);
+    if (p.f16) hipLaunchKernelGGL((splitkv_merge_rows_kernel<D, true>), rows, dim3(64 * kMergeWaves), 0, stream, p);
+    else hipLaunchKernelGGL((splitkv_merge_rows_kernel<D, false>), rows, dim3(64 * kMergeWaves), 0, stream, p);
   }
   return check_launch();
 }
