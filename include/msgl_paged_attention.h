@@ -163,8 +163,10 @@ MSGL_API int msgl_paged_decode_attention_noalloc(const void* q, const void* k_ca
  *   out_loc (batch): the slot of request b's row, which as a rule is the last one listed for it in
  *   kv_indices; the request then sees the row itself and not the pool.  Otherwise the row is in the
  *   pool before that is read for the request.  A slot outside the pool stores nothing.
- * The rows are stored by the launch that attends, so a slot of out_loc that is listed for another
- * request may be read before or after the row is there: such a step takes the two calls.
+ * The rows are stored by the launch that attends, and no request waits for another's.  The caller guarantees
+ * that no slot of out_loc is listed in kv_indices for another request, nor twice for its own (such a slot may
+ * be read before or after the row is there); for a step with such slots the caller makes the two calls.  The
+ * arrays are on the device, so nothing here can tell.
  */
 MSGL_API size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads,
                                                  int64_t num_kv_heads, int64_t head_dim,
@@ -241,8 +243,8 @@ MSGL_API int msgl_paged_prefill_attention(const void* q, const void* k_cache, co
  *   contiguous; bf16
  * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; with short query blocks
  * the request then sees the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
- * request.  As with msgl_decode_step a slot of out_loc that is listed for another request may be read
- * before or after the row is there: such a batch takes the two calls.
+ * request.  As with msgl_decode_step the caller guarantees that no slot of out_loc is listed for a request that
+ * its row does not belong to, nor twice for its own, and makes the two calls for a batch with such slots.
  */
 MSGL_API size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv,
                                                  int64_t num_q_heads, int64_t num_kv_heads,

@@ -585,10 +585,11 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 }
 
 // ---- extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, sm_scale,
-//                  max_len_extend, is_cross_attention, sliding_window_size) -> out or None ---------------
-// As decode_step, for prefill metadata; the two launches are made here too where one is not the way.
+//                  max_len_extend, is_cross_attention, sliding_window_size, own_slots) -> out or None ----
+// As decode_step, for prefill metadata; the two launches are made here too where one is not the way, and always
+// without own_slots.
 PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
-  return guarded(args, n_args, 14, [](PyObject* const* a) -> PyObject* {
+  return guarded(args, n_args, 15, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "extend_step";
     for (int i = 0; i < 10; ++i)
       if (!THPVariable_Check(a[i])) return none();
@@ -599,7 +600,7 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const c10::Device dev = q.device();
     if (total == 0 || batch <= 0 || slots == 0 || q.scalar_type() != at::kBFloat16 || !dev.is_cuda()) return none();
     const int64_t max_extend = integer(a[11]), window = integer(a[13]);
-    const bool cross = truth(a[12]);
+    const bool cross = truth(a[12]), own_slots = truth(a[14]);
     if (window < 0 || window > 0x7fffffff || max_extend <= 0 || max_extend > 0x7fffffff || (d != 128 && d != 256) || n_kv == 0 ||
         n_q == 0 || n_q % n_kv != 0)
       return none();
@@ -627,7 +628,8 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       OnDevice on(dev);
       out = empty({total, n_q, d}, at::kBFloat16, dev);
       const int64_t ks0 = stride0(k), vs0 = stride0(v), kcs = stride0(kc), vcs = stride0(vc);
-      size_t bytes = msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross, static_cast<int32_t>(window));
+      size_t bytes = !own_slots ? 0 : msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross,
+                                                                       static_cast<int32_t>(window));
       if (bytes > 0) {
         const Tensor ws = scratch(bytes, dev);
         rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), ks0, vs0, ints(loc), kc.data_ptr(), vc.data_ptr(), ints(qp),

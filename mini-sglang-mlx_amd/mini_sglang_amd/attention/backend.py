@@ -1,11 +1,13 @@
 """Attention backend of the path on torch-ROCm
 (reference: mini_sglang_mlx/attention/backend.py:15-307).
 
-``AttnBackend.forward`` stores the new K/V rows first and then attends through the slot
-lists, so the new tokens are read back from the pool exactly like cached ones
-(backend.py:139-141).  Metadata are int32 CSR arrays; ``kv_indices`` holds one pool slot
-per token.  The builders keep the reference's formulas and keyword overrides (virtual
-extend windows for speculative verify, backend.py:205-293).
+``AttnBackend.forward`` stores the new K/V rows and attends through the slot lists
+(backend.py:139-141): in one launch where the metadata say that the new slots are their
+requests' own (``own_slots``) and the step's sizes make that the better way, else the store
+first and then attention, which reads the new tokens back from the pool like cached ones.
+Metadata are int32 CSR arrays; ``kv_indices`` holds one pool slot per token.  The builders keep
+the reference's formulas and keyword overrides (virtual extend windows for speculative verify,
+backend.py:205-293).
 """
 from __future__ import annotations
 
@@ -39,6 +41,7 @@ class PrefillMetadata(BaseAttnMetadata):
     kv_indices: torch.Tensor  # (total_kv,) int32 pool slots
     prefix_lens: torch.Tensor  # (batch,) int32
     max_len_extend: int
+    own_slots: bool = False  # see AttnBackend.forward
 
     def get_last_indices(self, bs: int) -> torch.Tensor:
         return self.qo_indptr[1 : 1 + bs] - 1
@@ -52,6 +55,7 @@ class DecodeMetadata(BaseAttnMetadata):
     kv_indices: torch.Tensor  # (total_kv,) int32 pool slots
     num_kv_splits: torch.Tensor  # (batch,) int32
     max_kv_splits: int
+    own_slots: bool = False  # see AttnBackend.forward
 
     def get_last_indices(self, bs: int) -> torch.Tensor:
         return torch.arange(bs, dtype=torch.int32, device=self.kv_indptr.device)
@@ -79,6 +83,13 @@ class AttnBackend:
 
         The two flags select one of four masks on the prefill path (backend.py:112-127):
         causal, full, causal + window, bidirectional + window.  Decode rejects both.
+
+        ``batch.attn_metadata.own_slots`` says that no slot of ``batch.out_loc`` is listed in
+        ``kv_indices`` for a request that the row does not belong to, nor twice for its own.  The
+        rows may then be stored by the launch that attends: a request sees its own new rows, and
+        nobody waits for those of others.  Without it every row is in the pool before the
+        attention starts, and requests may share new slots in any way.  Metadata made by hand do
+        not claim it; of those the builders make see ``_slots_are_own``.
         """
         assert sliding_window_size >= 0, (
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
@@ -101,7 +112,7 @@ class AttnBackend:
         """``mini_sglang_amd_kernel.decode_step`` on the step's pool, where this package writes that
         itself; ``None``: the step takes its two calls."""
         metadata, cache = batch.attn_metadata, self.kvcache
-        if type(metadata) is not DecodeMetadata or type(cache) is not MHAKVCache:
+        if type(metadata) is not DecodeMetadata or not metadata.own_slots or type(cache) is not MHAKVCache:
             return None
         return _native.decode_step(q, k, v, q_weight, k_weight, positions, batch.out_loc,
                                    cache.k_cache(layer_id), cache.v_cache(layer_id),
@@ -110,14 +121,15 @@ class AttnBackend:
 
     def _extend_step(self, q, k, v, layer_id: int, batch, is_cross_attention: bool,
                      sliding_window_size: int) -> Optional[torch.Tensor]:
-        """The same for ``mini_sglang_amd_kernel.extend_step``."""
+        """The same for ``mini_sglang_amd_kernel.extend_step``, which makes the two launches too."""
         metadata, cache = batch.attn_metadata, self.kvcache
         if type(cache) is not MHAKVCache:
             return None
         return _native.extend_step(q, k, v, batch.out_loc, cache.k_cache(layer_id),
                                    cache.v_cache(layer_id), metadata.qo_indptr, metadata.kv_indptr,
                                    metadata.kv_indices, metadata.prefix_lens, self.sm_scale,
-                                   metadata.max_len_extend, is_cross_attention, sliding_window_size)
+                                   metadata.max_len_extend, is_cross_attention, sliding_window_size,
+                                   metadata.own_slots)
 
     def _attend(self, q, k_cache, v_cache, metadata, is_cross_attention: bool,
                 sliding_window_size: int) -> torch.Tensor:
@@ -144,7 +156,8 @@ class AttnBackend:
         """``forward`` for a Qwen3-style layer that hands over the raw projections: q/k RMSNorm,
         rotary embedding at ``batch.attn_metadata.positions`` and the KV-store run as one kernel
         (the reference does them as four array ops plus the store, models/qwen3.py:60-68 and
-        backend.py:139), then attention runs on the pool without storing again."""
+        backend.py:139), then attention runs on the pool without storing again; small decode steps
+        whose slots are their requests' own (``own_slots``, see ``forward``) do it all in one."""
         assert sliding_window_size >= 0, (
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
@@ -167,11 +180,13 @@ class AttnBackend:
         self.kvcache.store_kv(k, v, out_loc, layer_id)
 
     def prepare_metadata(self, batch) -> None:
-        reqs = batch.padded_reqs
+        """Metadata of ``batch.padded_reqs``; a batch with an attribute ``own_slots`` decides about
+        theirs (``None`` and no attribute: the builders do)."""
+        reqs, own_slots = batch.padded_reqs, getattr(batch, "own_slots", None)
         if batch.is_prefill:
-            batch.attn_metadata = self.build_prefill_metadata(reqs)
+            batch.attn_metadata = self.build_prefill_metadata(reqs, own_slots=own_slots)
         else:
-            batch.attn_metadata = self.build_decode_metadata(reqs)
+            batch.attn_metadata = self.build_decode_metadata(reqs, own_slots=own_slots)
 
     def _gather_indices(self, reqs, kv_lens: Sequence[int]) -> torch.Tensor:
         return torch.cat([self.page_table[reqs[i].table_idx, : kv_lens[i]]
@@ -186,8 +201,11 @@ class AttnBackend:
 
     def build_prefill_metadata(self, reqs: List, *, extend_lens: Optional[List[int]] = None,
                                kv_lens: Optional[List[int]] = None,
-                               positions: Optional[torch.Tensor] = None) -> PrefillMetadata:
+                               positions: Optional[torch.Tensor] = None,
+                               own_slots: Optional[bool] = None) -> PrefillMetadata:
         device = self.page_table.device
+        if own_slots is None:
+            own_slots = _slots_are_own(reqs)
         if extend_lens is None:
             extend_lens = [req.extend_len for req in reqs]
         if kv_lens is None:
@@ -197,7 +215,7 @@ class AttnBackend:
             return PrefillMetadata(
                 positions=m["positions"] if positions is None else positions,
                 qo_indptr=m["qo_indptr"], kv_indptr=m["kv_indptr"], kv_indices=m["kv_indices"],
-                prefix_lens=m["prefix_lens"], max_len_extend=max(extend_lens))
+                prefix_lens=m["prefix_lens"], max_len_extend=max(extend_lens), own_slots=own_slots)
         # slot table in host memory (host-side tests): the same arrays with torch ops
         cached_lens = [kv_lens[i] - extend_lens[i] for i in range(len(reqs))]
         if positions is None:
@@ -212,11 +230,15 @@ class AttnBackend:
             kv_indices=self._gather_indices(reqs, kv_lens),
             prefix_lens=torch.tensor(cached_lens, dtype=torch.int32, device=device),
             max_len_extend=max(extend_lens),
+            own_slots=own_slots,
         )
 
     def build_decode_metadata(self, reqs: List, *, kv_lens: Optional[List[int]] = None,
-                              positions: Optional[torch.Tensor] = None) -> DecodeMetadata:
+                              positions: Optional[torch.Tensor] = None,
+                              own_slots: Optional[bool] = None) -> DecodeMetadata:
         device = self.page_table.device
+        if own_slots is None:
+            own_slots = _slots_are_own(reqs)
         if kv_lens is None:
             kv_lens = [req.device_len for req in reqs]
         if device.type == "cuda":
@@ -231,7 +253,7 @@ class AttnBackend:
                     positions = torch.tensor(cached, dtype=torch.int32, device=device)
             return DecodeMetadata(positions=positions, kv_indptr=m["kv_indptr"],
                                   kv_indices=m["kv_indices"], num_kv_splits=m["num_kv_splits"],
-                                  max_kv_splits=MAX_KV_SPLITS)
+                                  max_kv_splits=MAX_KV_SPLITS, own_slots=own_slots)
         if positions is None:
             positions = torch.tensor([req.cached_len for req in reqs], dtype=torch.int32,
                                      device=device)
@@ -241,7 +263,17 @@ class AttnBackend:
             kv_indices=self._gather_indices(reqs, kv_lens),
             num_kv_splits=_compute_num_kv_splits(kv_lens, device),
             max_kv_splits=MAX_KV_SPLITS,
+            own_slots=own_slots,
         )
+
+
+def _slots_are_own(reqs: Sequence) -> bool:
+    """``own_slots`` of requests in the slot table, unless the caller says otherwise: the allocator
+    hands a new token's slot to one request, once, and a prefix is shared when it has been computed
+    (scheduler/cache.py:45-57), so it holds for distinct rows of the table, and not for a row that
+    comes twice.  A caller whose rows share slots of the step's own tokens says so
+    (``own_slots=False``)."""
+    return len({req.table_idx for req in reqs}) == len(reqs)
 
 
 def _build_indptr(lens: Sequence[int], device=None) -> torch.Tensor:

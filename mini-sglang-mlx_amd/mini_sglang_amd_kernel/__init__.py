@@ -269,8 +269,9 @@ def decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
     the way: large launches, forms that need a copy, arguments that they refuse, index
     validation on.
 
-    One new token per request, row ``b`` at slot ``out_loc[b]``.  A slot of ``out_loc`` must not be
-    listed for another request: the launch that reads it writes it.
+    One new token per request, row ``b`` at slot ``out_loc[b]``.  No slot of ``out_loc`` may be listed in
+    ``kv_indices`` for another request, nor twice for its own: the launch that reads it writes it.  A
+    step with such slots is the two calls.
     """
     return _native.decode_step(q, k, v, q_weight, k_weight, positions, out_loc, k_cache, v_cache,
                                kv_indptr, kv_indices, num_kv_splits, sm_scale, eps, rope_base)
@@ -280,16 +281,18 @@ def extend_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
                 k_cache: torch.Tensor, v_cache: torch.Tensor, qo_indptr: torch.Tensor,
                 kv_indptr: torch.Tensor, kv_indices: torch.Tensor, prefix_lens: torch.Tensor, *,
                 sm_scale: float, max_len_extend: int, is_cross_attention: bool = False,
-                sliding_window_size: int = 0) -> Optional[torch.Tensor]:
+                sliding_window_size: int = 0, own_slots: bool = True) -> Optional[torch.Tensor]:
     """``store_kv_cache`` of the queries' own rows of k and v and ``paged_prefill_attention`` as one call: in one
     launch where the query blocks are short or the launch is small, else as the two calls.  Returns the
     attention output, or ``None`` (nothing done) where the two calls have to be made by themselves: forms
-    that need a copy, arguments that they refuse, index validation on.  As with ``decode_step`` a slot
-    of ``out_loc`` must not be listed for another request.
+    that need a copy, arguments that they refuse, index validation on.
+
+    As with ``decode_step`` no slot of ``out_loc`` may be listed in ``kv_indices`` for a request that its row does not
+    belong to, nor twice for its own; ``own_slots=False`` is for such batches: the two launches, whatever the size.
     """
     return _native.extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices,
                                prefix_lens, sm_scale, max_len_extend, is_cross_attention,
-                               sliding_window_size)
+                               sliding_window_size, own_slots)
 
 
 def gdn_state_inplace(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
