@@ -240,7 +240,8 @@ MSGL_API int msgl_paged_prefill_attention(const void* q, const void* k_cache, co
  * drafts) and small launches of up to some hundred tokens a request: msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
  * msgl_extend_step refuses them (MSGL_ERR_SHAPE).
  *   q, k, v, out_loc: total_q rows each, in the order of qo_indptr; leading strides of k and v free, q
- *   contiguous; bf16
+ *   contiguous; bf16.  Rows in front of qo_indptr[0] and behind qo_indptr[batch] belong to no request: their k and v
+ *   are stored all the same
  * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; with short query blocks
  * the request then sees the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
  * request.  As with msgl_decode_step the caller guarantees that no slot of out_loc is listed for a request that

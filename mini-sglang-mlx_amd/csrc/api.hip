@@ -365,6 +365,7 @@ int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stri
   tokens.out_loc = out_loc;
   tokens.k_stride0 = k_stride0;
   tokens.v_stride0 = v_stride0;
+  tokens.rows = batch;
   tokens.eps = rms_norm_eps;
   tokens.rope_base = rope_base;
   const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
@@ -678,6 +679,7 @@ int msgl_extend_step(const void* q, const void* k, const void* v, int64_t k_stri
   tokens.out_loc = out_loc;
   tokens.k_stride0 = k_stride0;
   tokens.v_stride0 = v_stride0;
+  tokens.rows = total_q;
   if (plan.share_len == 0) {
     const size_t need = msgl_extend_step_workspace_bytes(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend,
                                                          is_cross_attention, sliding_window_size);

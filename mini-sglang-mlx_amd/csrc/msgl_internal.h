@@ -52,8 +52,11 @@ struct NewTokens {
   const int32_t* positions;
   const int32_t* out_loc;
   int64_t k_stride0, v_stride0;  // elements
+  int64_t rows;                  // of k and v
   float eps, rope_base;
 };
+// Workgroups that a prefill launch which stores its rows has for those of no request.
+constexpr int kRestBlocks = 8;
 // largest q_len * group the split-K kernel is instantiated for
 constexpr int kSplitKvMaxCols = 64;
 constexpr int kSplitKvMinSegment = 128;

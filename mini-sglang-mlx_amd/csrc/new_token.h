@@ -33,6 +33,7 @@ inline void fill_new_tokens(const NewTokens& n, SplitKvParams& p) {
   p.nt.v_pool = const_cast<uint16_t*>(p.v_cache);
   p.nt.k_stride0 = n.k_stride0;
   p.nt.v_stride0 = n.v_stride0;
+  p.nt.rows = (int32_t)n.rows;
   p.nt.eps = n.eps;
   p.nt.log2_base = n.q_weight ? log2f(n.rope_base) : 0.f;
 }

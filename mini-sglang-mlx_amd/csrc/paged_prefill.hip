@@ -736,6 +736,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   const ClockProbe clock_probe_(p.clock_probe);
 
   const int tid = threadIdx.x;
+  if constexpr (ORDER == Order::kBatch)
+    if (store_rows_of_no_request<NW * 64>(p, p.nt, p.n_kv * D, tid)) return;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int h = lane >> 5;
@@ -921,7 +923,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     return;
   }
   if constexpr (ORDER == Order::kBatch)
-    if (p.out_loc != nullptr) store_request_rows<NW * 64, D>(p, q_start, uniform(place.q_len), kvh, tid);
+    if (p.nt.out_loc != nullptr) store_request_rows<NW * 64, D>(p, q_start, uniform(place.q_len), kvh, tid);
 
   bool idle = __builtin_amdgcn_readfirstlane(row0 + w * 32 >= rows_total ? 1 : 0) != 0;
   if constexpr (!listed) {
@@ -1752,6 +1754,10 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
   }
   const int rc = make_prefill_params(args, p, n_blocks, wide);
   if (rc != MSGL_OK || n_blocks == 0) return rc;
+  if (p.nt.out_loc != nullptr) {
+    p.nt.blocks = (uint32_t)n_blocks;
+    n_blocks += kRestBlocks;
+  }
   const dim3 grid((unsigned)n_blocks);
   if (tile_variant() != 0) {
     if (wide) hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, true>), grid, dim3(512), 0, stream, p);

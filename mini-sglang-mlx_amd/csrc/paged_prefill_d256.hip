@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   const ClockProbe clock_probe_(p.clock_probe);
 
   const int tid = threadIdx.x;
+  if (store_rows_of_no_request<kNW * 64>(p, p.nt, p.n_kv * kD, tid)) return;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int h = lane >> 5;
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   const int rows_total = q_len * p.group;
   const int row0 = qblk * kRows;
   if (row0 >= rows_total) return;
-  if (p.out_loc != nullptr) store_request_rows<kNW * 64, kD>(p, q_start, __builtin_amdgcn_readfirstlane(place.q_len), kvh, tid);
+  if (p.nt.out_loc != nullptr) store_request_rows<kNW * 64, kD>(p, q_start, __builtin_amdgcn_readfirstlane(place.q_len), kvh, tid);
 
   const int qi_lo = row0 / p.group;
   const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;
@@ -553,6 +554,10 @@ int launch_prefill_tile256(const PrefillArgs& a, hipStream_t stream) {
   bool wide = false;
   const int rc = make_prefill_params(a, p, n_blocks, wide, kPrefillBlockRows256);
   if (rc != MSGL_OK || n_blocks == 0) return rc;
+  if (p.nt.out_loc != nullptr) {
+    p.nt.blocks = (uint32_t)n_blocks;
+    n_blocks += kRestBlocks;
+  }
   const dim3 grid((unsigned)n_blocks);
   if (wide) hipLaunchKernelGGL((prefill_tile256_kernel<true>), grid, dim3(kNW * 64), 0, stream, p);
   else hipLaunchKernelGGL((prefill_tile256_kernel<false>), grid, dim3(kNW * 64), 0, stream, p);

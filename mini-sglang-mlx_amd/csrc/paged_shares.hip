@@ -113,7 +113,11 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 
   ReqInfo r;
   int b, share, n_shares;
-  if (!find_share(p, sp.share_len, item, &r, &b, &share, &n_shares)) return;  // the whole workgroup
+  if (!find_share(p, sp.share_len, item, &r, &b, &share, &n_shares)) {  // the whole workgroup
+    // (behind the search, that the others do not wait for one more parameter: 0.2 us of 10)
+    if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(p, p.nt, p.n_kv * D, threadIdx.x);
+    return;
+  }
   const int ncols = r.q_len * p.group;
   if (ncols == 0) return;
   Columns<D, NCT> c;
@@ -448,7 +452,8 @@ size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv,
 int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& plan, hipStream_t stream) {
   const int64_t group = a.n_q / a.n_kv, cols = group * a.max_len_extend;
   const int64_t head_groups = a.n_kv / plan.heads_wg;
-  const int64_t blocks = plan.max_shares * head_groups;
+  const bool rows = n.k != nullptr && a.qo_indptr != nullptr;  // kStoreRows
+  const int64_t blocks = plan.max_shares * head_groups + (rows ? kRestBlocks : 0);
   if (blocks > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   ShareParams sp{};
   fill_splitkv_params(a, sp.s);
@@ -463,6 +468,7 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   sp.heads_wg = plan.heads_wg;
   sp.head_groups = (int32_t)head_groups;
   fill_new_tokens(n, sp.s);
+  sp.s.nt.blocks = (uint32_t)(plan.max_shares * head_groups);
   const int nct = nct_of(cols);
   if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
   if (nct == 1) return launch_shape<128, 1, 8>(sp, (unsigned)blocks, stream);

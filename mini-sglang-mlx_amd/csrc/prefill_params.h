@@ -48,11 +48,16 @@ struct PrefillParams {
   // this many rounds (see kMaxRounds)
   int32_t length_rounds;
   uint32_t group_magic, group_shift;  // row / group of a row below 2^31: see row_to_query()
-  // the queries' own rows of k and v, which the launch stores itself (see prefill_stores_rows()); out_loc nullptr:
+  // the queries' own rows of k and v, which the launch stores itself (see stores_in_tiles() in api.hip); out_loc nullptr:
   // they are in the pool
-  const uint16_t *new_k, *new_v;
-  const int32_t* out_loc;
-  int64_t new_k_stride0, new_v_stride0;
+  struct {
+    const uint16_t *k, *v;
+    const int32_t* out_loc;
+    uint16_t *k_pool, *v_pool;
+    int64_t k_stride0, v_stride0;
+    int32_t rows;     // of k and v
+    uint32_t blocks;  // workgroups in front of those of store_rows_of_no_request(), which a launch that stores has
+  } nt;
 };
 
 constexpr int kBN = 64;  // keys per tile
@@ -324,11 +329,15 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
   while ((1u << p.group_shift) < (uint32_t)p.group) ++p.group_shift;
   p.group_magic = (uint32_t)(((1ull << (31 + p.group_shift)) + p.group - 1) / p.group);
   p.clock_probe = clock_probe();
-  p.new_k = static_cast<const uint16_t*>(a.new_tokens.k);
-  p.new_v = static_cast<const uint16_t*>(a.new_tokens.v);
-  p.out_loc = a.new_tokens.out_loc;
-  p.new_k_stride0 = a.new_tokens.k_stride0;
-  p.new_v_stride0 = a.new_tokens.v_stride0;
+  p.nt.k = static_cast<const uint16_t*>(a.new_tokens.k);
+  p.nt.v = static_cast<const uint16_t*>(a.new_tokens.v);
+  p.nt.out_loc = a.new_tokens.out_loc;
+  p.nt.k_pool = const_cast<uint16_t*>(p.k_cache);
+  p.nt.v_pool = const_cast<uint16_t*>(p.v_cache);
+  p.nt.k_stride0 = a.new_tokens.k_stride0;
+  p.nt.v_stride0 = a.new_tokens.v_stride0;
+  p.nt.rows = (int32_t)a.new_tokens.rows;
+  p.nt.blocks = 0xffffffffu;
   if (a.ragged_tiles > 0 && n_qblk == 1) {
     const int64_t units = prefill_ragged_units(a.batch, a.total_kv, a.ragged_tiles);
     p.n_ksplit = 1;

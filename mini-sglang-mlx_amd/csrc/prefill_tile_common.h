@@ -482,6 +482,26 @@ __device__ __forceinline__ RequestPlace place_of(const PrefillParams& p, int at,
   return r;
 }
 
+// Rows of k and v in front of the first request's and behind the last's are stored by nobody's block: kRestBlocks
+// workgroups behind the others take them, all heads of a row at once, and as a rule end after one round trip.  (Spread
+// over the launch's own workgroups they cost the tile loop of head_dim 128 12 bytes of spills.)  `n`: what the launch's
+// parameters say about its new rows.  False: not one of those workgroups.
+template <int THREADS, typename P, typename N>
+__device__ __forceinline__ bool store_rows_of_no_request(const P& p, const N& n, int width, int tid) {
+  if (blockIdx.x < n.blocks) return false;
+  const int front = min(max(p.qo_indptr[0], 0), n.rows), end = min(max(p.qo_indptr[p.batch], front), n.rows);
+  for (int i = blockIdx.x - n.blocks; i < front + n.rows - end; i += kRestBlocks) {
+    const int64_t row = i < front ? i : i - front + end;
+    const uint32_t slot = (uint32_t)n.out_loc[row];
+    if (slot > p.max_slot) continue;  // a slot id outside the pool stores nothing
+    for (int e = 8 * tid; e < width; e += 8 * THREADS) {
+      st_global_b128(n.k_pool + (int64_t)slot * p.k_stride0 + e, ld_global_b128(n.k + row * n.k_stride0 + e));
+      st_global_b128(n.v_pool + (int64_t)slot * p.v_stride0 + e, ld_global_b128(n.v + row * n.v_stride0 + e));
+    }
+  }
+  return true;
+}
+
 // A request's new rows of k and v of one kv head into the pool, by the whole workgroup, before it reads the pool: every
 // workgroup of a small launch does it for its own request (the same bytes, several times), which is less than the
 // launch that it saves.
@@ -497,15 +517,15 @@ __device__ __forceinline__ void store_request_rows(const PrefillParams& p, int q
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t row = q_start + min(r0 + u * ROWS, n - 1);
-        slot[u] = (uint32_t)p.out_loc[row];
-        k[u] = ld_global_b128(p.new_k + row * p.new_k_stride0 + col);
-        v[u] = ld_global_b128(p.new_v + row * p.new_v_stride0 + col);
+        slot[u] = (uint32_t)p.nt.out_loc[row];
+        k[u] = ld_global_b128(p.nt.k + row * p.nt.k_stride0 + col);
+        v[u] = ld_global_b128(p.nt.v + row * p.nt.v_stride0 + col);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (r0 + u * ROWS >= n || slot[u] > p.max_slot) continue;  // a slot id outside the pool stores nothing
-        st_global_b128(const_cast<uint16_t*>(p.k_cache) + (int64_t)slot[u] * p.k_stride0 + col, k[u]);
-        st_global_b128(const_cast<uint16_t*>(p.v_cache) + (int64_t)slot[u] * p.v_stride0 + col, v[u]);
+        st_global_b128(p.nt.k_pool + (int64_t)slot[u] * p.k_stride0 + col, k[u]);
+        st_global_b128(p.nt.v_pool + (int64_t)slot[u] * p.v_stride0 + col, v[u]);
       }
     }
   };

@@ -38,6 +38,8 @@ struct SplitKvParams {
     const int32_t *positions, *out_loc;
     uint16_t *k_pool, *v_pool;
     int64_t k_stride0, v_stride0;
+    int32_t rows;     // of k and v
+    uint32_t blocks;  // workgroups in front of those of store_rows_of_no_request()
     float eps, log2_base;
   } nt;
 };

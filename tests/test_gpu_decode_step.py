@@ -197,3 +197,52 @@ def test_extend_in_tiles_is_two(gpu, cached, ext, n_q, n_kv, d, cap, cross, wind
     if places == "last" and not cross:  # (a full mask may be shared out otherwise)
         assert _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(ext) + sum(cached), n_q, n_kv, d, cap or max(ext), 0, window) > 0
     test_extend_one_launch_is_two(gpu, lambda *_: None, cached, ext, n_q, n_kv, d, 0, cap, cross, window, places)
+
+
+# rows that belong to no request, in front of the first and behind the last: cached, new tokens, heads, such rows, max_len_extend
+NOBODYS = [
+    ([90, 0, 300], [8, 8, 8], 32, 8, 128, (0, 40), 8),      # shares
+    ([5, 64, 0], [3, 0, 5], 16, 8, 128, (3, 1), 8),
+    ([40], [1], 16, 8, 128, (0, 2000), 1),                   # more of them than workgroups
+    ([7, 9], [0, 0], 16, 8, 128, (2, 6), 3),                 # no request has rows
+    ([40, 300], [5, 3], 16, 4, 256, (7, 70), 4),
+    ([0, 0, 40], [31, 33, 0], 32, 8, 128, (1, 63), 33),      # tiles
+    ([900], [192], 16, 8, 128, (0, 400), 192),
+    ([1000, 200], [90, 20], 16, 4, 128, (5, 0), 90),
+    ([7, 9], [0, 0], 32, 8, 128, (2, 300), 60),
+    ([2, 700], [0, 0], 32, 8, 128, (90, 300), 100),
+    ([100] * 70, [17 + i % 5 for i in range(70)], 8, 1, 128, (2, 90), 21),
+    ([0, 300, 20], [17, 96, 16], 24, 4, 256, (9, 33), 96),
+    ([0, 300, 20], [0, 0, 0], 24, 4, 256, (9, 33), 20),
+]
+
+
+@pytest.mark.parametrize("cached,ext,n_q,n_kv,d,nobodys,limit", NOBODYS)
+def test_rows_of_no_request_are_stored(gpu, cached, ext, n_q, n_kv, d, nobodys, limit):
+    kv = [c + e for c, e in zip(cached, ext)]
+    wl = build_workload("step", "prefill", seed=sum(kv), n_q=n_q, n_kv=n_kv, head_dim=d, kv_lens=kv, extend_lens=ext).to(gpu)
+    front, behind = nobodys
+    total = front + sum(ext) + behind
+    g = torch.Generator(device=gpu)
+    g.manual_seed(total)
+    q, k, v = (torch.randn((total, n, d), generator=g, device=gpu).bfloat16() for n in (n_q, n_kv, n_kv))
+    spare = wl.k_cache.shape[0]
+    kc, vc = (torch.cat([c, c.new_zeros((front + behind + 1, n_kv, d))]) for c in (wl.k_cache, wl.v_cache))
+    own = [wl.kv_indices[int(wl.kv_indptr[b]) + c:int(wl.kv_indptr[b + 1])] for b, c in enumerate(cached)]
+    rest = spare + torch.randperm(front + behind, generator=g, device=gpu).to(torch.int32)
+    if behind > 1:
+        rest[-1] = kc.shape[0] + 5  # outside the pool: nothing is stored
+    loc = torch.cat([rest[:front], *own, rest[front:]]).contiguous()
+    indptr = wl.qo_indptr + front
+    sizes = (len(ext), total, sum(kv), n_q, n_kv, d, limit, 0, 0)
+    assert _lib.load().msgl_extend_step_workspace_bytes(*sizes) > 0  # one launch
+    kc2, vc2 = kc.clone(), vc.clone()
+    print(f"rows of no request {cached[:4]} + {ext[:4]} {n_q}/{n_kv} d{d} {nobodys}", flush=True)
+    got = extend_step(q, k, v, loc, kc, vc, indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, sm_scale=wl.sm_scale, max_len_extend=limit)
+    store_kv_cache(kc2, vc2, loc, k, v)
+    want = paged_prefill_attention(q, kc2, vc2, indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, wl.sm_scale, limit)
+    for a, b in ((kc, kc2), (vc, vc2)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    at = torch.cat([torch.arange(min(e, limit)) + front + sum(ext[:b]) for b, e in enumerate(ext)])  # past the limit: not computed
+    diff = (got[at].float() - want[at].float()).abs()
+    assert sum(ext) == 0 or (float(diff.max()) <= 2e-2 and float(diff.mean()) <= 1e-3), (float(diff.max()), float(diff.mean()))
