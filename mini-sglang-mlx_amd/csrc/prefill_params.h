@@ -97,6 +97,11 @@ inline int64_t prefill_blocks_per_xcd(int64_t n_units, int64_t n_qblk) {
   return n_units / 8 * n_qblk + last_row;
 }
 
+// Query blocks with rows, of all requests and one kv head: a request's last block counts half.
+inline int64_t prefill_filled_blocks(int64_t batch, int64_t total_q, int64_t group, int block_rows) {
+  return (total_q * group + block_rows - 1) / block_rows + batch / 2;
+}
+
 // Number of key splits for a launch, from sizes the host knows (the per-request lengths stay on
 // the device: the average visible length stands for all of them).  The (request, kv head, split)
 // units are dealt round-robin to the 8 XCDs, a unit brings its query blocks, and an XCD runs its
@@ -123,7 +128,7 @@ inline int prefill_key_splits(int64_t batch, int64_t total_q, int64_t total_kv, 
   // Requests shorter than the longest leave some of the grid's blocks empty, which end at once.  In one pass the
   // others go in order of length (see prefill_by_length()) and fill the rounds; splits of them do not, and the XCD
   // that has the longest requests' counts: a fifth on top of the average.
-  const int64_t grid_blocks = batch * n_qblk, filled = (total_q * group + block_rows - 1) / block_rows + batch / 2;
+  const int64_t grid_blocks = batch * n_qblk, filled = prefill_filled_blocks(batch, total_q, group, block_rows);
   auto rounds = [&](int64_t k) {
     const int64_t grid = prefill_blocks_per_xcd(batch * n_kv * k, n_qblk);  // on the busiest XCD
     const int64_t uneven = (6 * grid * filled + 5 * grid_blocks - 1) / (5 * grid_blocks);
@@ -220,11 +225,17 @@ inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
 // rows and masks, in turn) beside 2.9 K a tile.  us, 32 / 8 heads unless said: prompts of 771-2710 tokens (11574 in
 // all) 249.8 -> 235.3, 30 x 100-300 on up to 500 cached 83.9 -> 74.9, 16 x 50-2000 at 64 / 8 heads 408 -> 370, three
 // of 1000-3000 under a window of 1024 166 -> 149.  A wave without rows computes all the same here (a loop of its own
-// costs 260 bytes of spills), and of few rounds the last ones are short: with 2 rounds (4 x 200-900) 33.1 -> 34.8,
-// with 3 (12 x 100-1000, 16 / 8 heads) 39.3 -> 40.9, with 4 (20 x 33-257 on 8 K, both sides) 281 -> 279: from 4 on.
-// The list of a workgroup's blocks is in LDS, hence the other limit; an XCD's workgroups work on one kv head (the
-// bases of the moves stay the same).
-constexpr int kMinRounds = 4, kMaxRounds = 64;
+// costs 260 bytes of spills), and of few rounds the last ones are short, so it pays from two rounds of blocks on.  Those
+// are blocks with rows: requests shorter than the longest leave most of the grid empty (one extend of 88 tokens beside 63
+// of 2, on 8 K keys: 4 rounds of the grid and 1.1 of blocks, 482 us and 601 with workgroups that stay; one of 4096 beside
+// fifteen of 16: 32 and 2.4, 153 and 131), so they are counted from all queries, a half for each
+// request's last block.  1050 launches of 1-64 even, ragged and very uneven extends, 4 and 8 kv heads, groups of 2-8, on
+// up to 8 K keys, staying against not, geometric means by such rounds: up to 1 1.10, 1-1.5 1.04, 1.5-2 0.985, 2-2.5
+// 0.963, 2.5-3 0.92, above 0.87-0.92; this line is 0.8 % from the better of the two on average, and 4 rounds of the
+// grid were 2.1 %.
+// The list of a workgroup's blocks is in LDS, hence the other limit (of the grid's rounds); an XCD's workgroups work on
+// one kv head (the bases of the moves stay the same).
+constexpr int kMinRounds = 2, kMaxRounds = 64;
 
 // Gang ranges, for launches with several query blocks per (request, kv head) (chunked extends on
 // long prefixes: their cost is the MFMA work, and it differs from unit to unit with the prefix).
@@ -390,7 +401,8 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     n_blocks = 8 * a.batch * p.length_heads * ((n_qblk + xcds - 1) / xcds);
     if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
     const int64_t rounds = (n_blocks + kComputeUnits - 1) / kComputeUnits;
-    if (block_rows == kPrefillBlockRows && p.length_heads == 1 && rounds >= kMinRounds && rounds <= kMaxRounds) {
+    const int64_t filled = 8 * prefill_filled_blocks(a.batch, a.total_q, p.group, block_rows);
+    if (block_rows == kPrefillBlockRows && p.length_heads == 1 && filled >= kMinRounds * kComputeUnits * xcds && rounds <= kMaxRounds) {
       p.length_rounds = (int32_t)rounds;
       n_blocks = kComputeUnits;
     }

@@ -52,6 +52,11 @@ STAY = [  # the last column: every third request's queries sit so far behind its
     (24, 8, _mixed(30, 520), [(i * 61) % 200 for i in range(30)], 64, True, True),
     (6, 2, _mixed(64, 400), [(i * 17) % 90 for i in range(64)], 0, False, False),
     (16, 1, _mixed(32, 500), [(i * 17) % 90 for i in range(32)], 0, False, False),
+    # about two rounds of blocks: of even extends, and of one long one beside short ones, whose grid has many more
+    (6, 2, _mixed(64, 700), [(i * 17) % 90 for i in range(64)], 0, False, False),
+    (16, 1, _mixed(32, 600), [(i * 17) % 90 for i in range(32)], 0, False, False),
+    (16, 4, [380] * 30, [(i * 61) % 500 for i in range(30)], 0, False, False),
+    (64, 8, [1700] + [16] * 14 + [0], [(i * 61) % 500 for i in range(16)], 0, False, False),
 ]
 
 
