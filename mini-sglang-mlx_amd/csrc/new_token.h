@@ -62,8 +62,6 @@ struct HeadLds {  // NORM: of one wave
 template <int D, bool NORM, bool F16>
 struct NewToken {
   static constexpr int E = D / 32, KS = D / 32, VH = D / 128;
-  // the rows of k and v are asked for in front of the first tile where they fit the registers beside it
-  static constexpr bool kRowsAhead = true;
   static constexpr int kEarly = 2;  // trips of four heads whose rows are asked for before the first tile
   using Half = typename HalfRow<E>::type;
   const SplitKvParams& sp;
@@ -105,7 +103,7 @@ struct NewToken {
       kwh = *reinterpret_cast<const Half*>(sp.nt.k_weight + D / 2 + off);
     }
     v = sp.nt.v + (int64_t)b * sp.nt.v_stride0 + kvh * D;
-    if (kRowsAhead && owner) rows();
+    if (owner) rows();  // in front of the first tile
   }
   __device__ __forceinline__ void rows() {
     const int g = lane_id() >> 4;
@@ -182,7 +180,6 @@ struct NewToken {
     __builtin_amdgcn_sched_barrier(0);
   }
   __device__ __forceinline__ void run() {
-    if (!kRowsAhead && owner) rows();
     if constexpr (NORM) normalise();
     if (!owner) return;
     const int g = lane_id() >> 4;
