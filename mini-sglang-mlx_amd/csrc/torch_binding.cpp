@@ -86,24 +86,50 @@ struct OnDevice {
   void* ptr() const { return stream.stream(); }
 };
 
-c10::Device require_device(const char* op, std::initializer_list<const Tensor*> ts) {
-  const c10::Device dev = (*ts.begin())->device();
-  if (!dev.is_cuda()) fail(op, "tensors must live on a ROCm GPU device (no CPU implementation exists)");
+// What is wrong with an operator's arguments, if anything.  An operator raises it; a step that is two operators in one
+// asks both (decode_step, extend_step), and leaves it to them to say so.
+struct Wrong {
+  const char *name = nullptr, *text = nullptr;  // the message: one behind the other
+  Wrong() = default;
+  Wrong(const char* t) : name(""), text(t) {}
+  Wrong(const char* n, const char* t) : name(n), text(t) {}
+  explicit operator bool() const { return text != nullptr; }
+};
+
+void require(const char* op, const Wrong& w) {
+  if (w) fail(op, std::string(w.name) + w.text);
+}
+
+Wrong device_of(std::initializer_list<const Tensor*> ts, c10::Device* dev) {
+  *dev = (*ts.begin())->device();
+  if (!dev->is_cuda()) return "tensors must live on a ROCm GPU device (no CPU implementation exists)";
   for (const Tensor* t : ts)
-    if (t->device() != dev) fail(op, "all tensors must be on the same device");
+    if (t->device() != *dev) return "all tensors must be on the same device";
+  return {};
+}
+
+c10::Device require_device(const char* op, std::initializer_list<const Tensor*> ts) {
+  c10::Device dev = c10::kCPU;
+  require(op, device_of(ts, &dev));
   return dev;
 }
 
+bool whole_rows(const Tensor& t) { return t.stride(2) == 1 && t.stride(1) == t.size(2); }  // of a 3D tensor
+// one row may report any leading stride
+int64_t row_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1) * t.size(2); }
+
+Wrong pool_form(const Tensor& pool, const char* name) {
+  return whole_rows(pool) ? Wrong() : Wrong(name, " must be contiguous in its (num_kv_heads, head_dim) dimensions");
+}
 int64_t pool_stride0(const char* op, const Tensor& pool, const char* name) {
-  if (pool.stride(2) != 1 || pool.stride(1) != pool.size(2))
-    fail(op, std::string(name) + " must be contiguous in its (num_kv_heads, head_dim) dimensions");
-  // a one-slot pool may report any leading stride
-  return pool.size(0) > 1 ? pool.stride(0) : pool.size(1) * pool.size(2);
+  require(op, pool_form(pool, name));
+  return row_stride(pool);
 }
 
-void require_int32(const char* op, const Tensor& t, const char* name) {
-  if (t.scalar_type() != at::kInt) fail(op, std::string(name) + " must be int32");
+Wrong int32_of(const Tensor& t, const char* name) {
+  return t.scalar_type() == at::kInt ? Wrong() : Wrong(name, " must be int32");
 }
+void require_int32(const char* op, const Tensor& t, const char* name) { require(op, int32_of(t, name)); }
 
 Tensor empty(c10::IntArrayRef size, at::ScalarType dtype, const c10::Device& dev) {
   return at::detail::empty_cuda(size, dtype, dev, std::nullopt);
@@ -164,77 +190,88 @@ PyObject* guarded(PyObject* const* args, Py_ssize_t n, Py_ssize_t want, F&& f) {
 PyObject* none() { Py_RETURN_NONE; }
 
 // ---- store_kv_cache(k_cache, v_cache, indices, k, v, validate) ----------------------------------
+Wrong store_args(const Tensor& kc, const Tensor& vc, const Tensor& idx, const Tensor& k, const Tensor& v, c10::Device* dev) {
+  if (kc.dim() != 3 || vc.dim() != 3) return "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)";
+  if (idx.dim() != 1) return "indices must be 1D";
+  if (k.dim() != 3 || v.dim() != 3) return "k and v must be 3D (length, num_kv_heads, head_dim)";
+  const auto dt = kc.scalar_type();
+  if (vc.scalar_type() != dt || k.scalar_type() != dt || v.scalar_type() != dt)
+    return "k_cache, v_cache, k, v must have the same dtype";
+  if (const Wrong w = int32_of(idx, "indices")) return w;
+  if (kc.size(2) % 4 != 0) return "head_dim must be a multiple of 4";
+  if (vc.sizes() != kc.sizes()) return "v_cache shape must match k_cache";
+  if (k.size(0) != idx.size(0) || k.size(1) != kc.size(1) || k.size(2) != kc.size(2) || v.sizes() != k.sizes())
+    return "k and v shape must be (length, num_kv_heads, head_dim)";
+  if (kc.element_size() != 2 && kc.element_size() != 4) return "unsupported dtype, must be float16, bfloat16 or float32";
+  return device_of({&kc, &vc, &idx, &k, &v}, dev);
+}
+
 PyObject* store_kv_cache(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 6, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "store_kv_cache";
     const Tensor &kc = tensor(a[0], "k_cache"), &vc = tensor(a[1], "v_cache"), &idx = tensor(a[2], "indices");
     const Tensor &k = tensor(a[3], "k"), &v = tensor(a[4], "v");
-    if (kc.dim() != 3 || vc.dim() != 3) fail(op, "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)");
-    if (idx.dim() != 1) fail(op, "indices must be 1D");
-    if (k.dim() != 3 || v.dim() != 3) fail(op, "k and v must be 3D (length, num_kv_heads, head_dim)");
-    const auto dt = kc.scalar_type();
-    if (vc.scalar_type() != dt || k.scalar_type() != dt || v.scalar_type() != dt)
-      fail(op, "k_cache, v_cache, k, v must have the same dtype");
-    require_int32(op, idx, "indices");
-    const int64_t pages = kc.size(0), heads = kc.size(1), d = kc.size(2), length = idx.size(0);
-    if (d % 4 != 0) fail(op, "head_dim must be a multiple of 4");
-    if (vc.sizes() != kc.sizes()) fail(op, "v_cache shape must match k_cache");
-    if (k.size(0) != length || k.size(1) != heads || k.size(2) != d || v.sizes() != k.sizes())
-      fail(op, "k and v shape must be (length, num_kv_heads, head_dim)");
-    const int64_t esz = kc.element_size();
-    if (esz != 2 && esz != 4) fail(op, "unsupported dtype, must be float16, bfloat16 or float32");
-    const c10::Device dev = require_device(op, {&kc, &vc, &idx, &k, &v});
+    c10::Device dev = c10::kCPU;
+    require(op, store_args(kc, vc, idx, k, v, &dev));
+    const int64_t pages = kc.size(0), heads = kc.size(1), d = kc.size(2), length = idx.size(0), esz = kc.element_size();
     if (length == 0) return none();
     debug_checks(a[5], op, {a[2], a[0]});
-    const int64_t row = heads * d, kcs = pool_stride0(op, kc, "k_cache"), vcs = pool_stride0(op, vc, "v_cache");
+    const int64_t kcs = pool_stride0(op, kc, "k_cache"), vcs = pool_stride0(op, vc, "v_cache");
     int rc;
     {
       NoGil nogil;
       OnDevice on(dev);
-      auto source = [d](const Tensor& t) { return t.stride(2) != 1 || t.stride(1) != d ? t.contiguous() : t; };
+      auto source = [](const Tensor& t) { return whole_rows(t) ? t : t.contiguous(); };
       const Tensor ks = source(k), vs = source(v), ix = idx.contiguous();
       rc = msgl_store_kv_cache(kc.data_ptr(), vc.data_ptr(), ints(ix), ks.data_ptr(), vs.data_ptr(), length, heads, d,
-                               pages, kcs, vcs, length > 1 ? ks.stride(0) : row, length > 1 ? vs.stride(0) : row,
-                               static_cast<int32_t>(esz), on.ptr());
+                               pages, kcs, vcs, row_stride(ks), row_stride(vs), static_cast<int32_t>(esz), on.ptr());
     }
     check_rc(op, rc);
     return none();
   });
 }
 
-int32_t attention_dtype(const char* op, const Tensor& q, const Tensor& kc, const Tensor& vc, bool half_ok) {
+Wrong attention_dtype(const Tensor& q, const Tensor& kc, const Tensor& vc, bool half_ok) {
   const auto dt = q.scalar_type();
-  if (dt != at::kBFloat16 && dt != at::kHalf) fail(op, "unsupported dtype, must be float16 or bfloat16");
-  if (kc.scalar_type() != dt || vc.scalar_type() != dt) fail(op, "q, k_cache and v_cache must have the same dtype");
+  if (dt != at::kBFloat16 && dt != at::kHalf) return "unsupported dtype, must be float16 or bfloat16";
+  if (kc.scalar_type() != dt || vc.scalar_type() != dt) return "q, k_cache and v_cache must have the same dtype";
   // float16 exists for decode only, as in the reference: its prefill kernel is instantiated for
   // bfloat16 alone (paged_prefill_attention.metal:646-647)
-  if (dt == at::kHalf && !half_ok) fail(op, "unsupported dtype, the prefill kernel is bfloat16 only");
-  return dt == at::kHalf ? MSGL_DTYPE_F16 : MSGL_DTYPE_BF16;
+  if (dt == at::kHalf && !half_ok) return "unsupported dtype, the prefill kernel is bfloat16 only";
+  return {};
 }
+int32_t dtype_code(const Tensor& q) { return q.scalar_type() == at::kHalf ? MSGL_DTYPE_F16 : MSGL_DTYPE_BF16; }
 
 // ---- paged_decode_attention(q, k_cache, v_cache, kv_indptr, kv_indices, num_kv_splits, sm_scale,
 //                             max_kv_splits, validate) -> out --------------------------------------
+Wrong decode_args(const Tensor& q, const Tensor& kc, const Tensor& vc, const Tensor& ip, const Tensor& ix, const Tensor& ns,
+                  c10::Device* dev) {
+  if (q.dim() != 3) return "q must be 3D (batch, num_q_heads, head_dim)";
+  if (kc.dim() != 3 || vc.dim() != 3) return "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)";
+  if (ip.dim() != 1 || ix.dim() != 1 || ns.dim() != 1) return "kv_indptr, kv_indices, num_kv_splits must be 1D";
+  const int64_t batch = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1);
+  if (d != 128 && d != 256) return "head_dim must be 128 or 256";
+  if (n_kv == 0 || n_q % n_kv != 0) return "num_q_heads must be a multiple of num_kv_heads";
+  if (n_q / n_kv > 16) return "only q_heads/kv_heads <= 16 is supported";
+  if (kc.size(2) != d || vc.size(2) != d) return "cache head_dim must match q head_dim";
+  if (vc.size(1) != n_kv) return "v_cache shape must match k_cache";
+  if (const Wrong w = attention_dtype(q, kc, vc, true)) return w;
+  if (const Wrong w = int32_of(ip, "kv_indptr")) return w;
+  if (const Wrong w = int32_of(ix, "kv_indices")) return w;
+  if (const Wrong w = int32_of(ns, "num_kv_splits")) return w;
+  if (ip.size(0) != batch + 1) return "kv_indptr must have batch + 1 entries";
+  if (ns.size(0) != batch) return "num_kv_splits must have batch entries";
+  return device_of({&q, &kc, &vc, &ip, &ix, &ns}, dev);
+}
+
 PyObject* paged_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 9, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "paged_decode_attention";
     const Tensor &q = tensor(a[0], "q"), &kc = tensor(a[1], "k_cache"), &vc = tensor(a[2], "v_cache");
     const Tensor &ip = tensor(a[3], "kv_indptr"), &ix = tensor(a[4], "kv_indices"), &ns = tensor(a[5], "num_kv_splits");
-    if (q.dim() != 3) fail(op, "q must be 3D (batch, num_q_heads, head_dim)");
-    if (kc.dim() != 3 || vc.dim() != 3) fail(op, "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)");
-    if (ip.dim() != 1 || ix.dim() != 1 || ns.dim() != 1) fail(op, "kv_indptr, kv_indices, num_kv_splits must be 1D");
+    c10::Device dev = c10::kCPU;
+    require(op, decode_args(q, kc, vc, ip, ix, ns, &dev));
     const int64_t batch = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1);
-    if (d != 128 && d != 256) fail(op, "head_dim must be 128 or 256");
-    if (n_kv == 0 || n_q % n_kv != 0) fail(op, "num_q_heads must be a multiple of num_kv_heads");
-    if (n_q / n_kv > 16) fail(op, "only q_heads/kv_heads <= 16 is supported");
-    if (kc.size(2) != d || vc.size(2) != d) fail(op, "cache head_dim must match q head_dim");
-    if (vc.size(1) != n_kv) fail(op, "v_cache shape must match k_cache");
-    const int32_t dtype = attention_dtype(op, q, kc, vc, true);
-    require_int32(op, ip, "kv_indptr");
-    require_int32(op, ix, "kv_indices");
-    require_int32(op, ns, "num_kv_splits");
-    if (ip.size(0) != batch + 1) fail(op, "kv_indptr must have batch + 1 entries");
-    if (ns.size(0) != batch) fail(op, "num_kv_splits must have batch entries");
-    const c10::Device dev = require_device(op, {&q, &kc, &vc, &ip, &ix, &ns});
     const float scale = static_cast<float>(real(a[6]));
     const int32_t max_splits = static_cast<int32_t>(integer(a[7]));
     if (batch > 0) debug_checks(a[8], op, {a[3], a[4], a[1]});
@@ -252,7 +289,7 @@ PyObject* paged_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n_
         const Tensor ws = scratch(bytes, dev);
         rc = msgl_paged_decode_attention(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(ipc), ints(ixc), ints(nsc),
                                          out.data_ptr(), data_or_null(ws), bytes, batch, total_kv, n_q, n_kv, d,
-                                         kc.size(0), kcs, vcs, scale, max_splits, dtype, on.ptr());
+                                         kc.size(0), kcs, vcs, scale, max_splits, dtype_code(q), on.ptr());
       }
     }
     check_rc(op, rc);
@@ -262,32 +299,40 @@ PyObject* paged_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n_
 
 // ---- paged_prefill_attention(q, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens,
 //        sm_scale, max_len_extend, is_cross_attention, sliding_window_size, validate) -> out -------
+Wrong prefill_args(const Tensor& q, const Tensor& kc, const Tensor& vc, const Tensor& qp, const Tensor& ip, const Tensor& ix,
+                   const Tensor& pl, PyObject* sliding_window_size, int64_t* window, c10::Device* dev) {
+  if (q.dim() != 3) return "q must be 3D (total_q_tokens, num_q_heads, head_dim)";
+  if (kc.dim() != 3 || vc.dim() != 3) return "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)";
+  if (qp.dim() != 1 || ip.dim() != 1 || ix.dim() != 1 || pl.dim() != 1)
+    return "qo_indptr, kv_indptr, kv_indices, prefix_lens must be 1D";
+  const int64_t n_q = q.size(1), d = q.size(2), n_kv = kc.size(1);
+  if (d != 128 && d != 256) return "head_dim must be 128 or 256";
+  if (n_kv == 0 || n_q % n_kv != 0) return "num_q_heads must be a multiple of num_kv_heads";
+  if (kc.size(2) != d || vc.size(2) != d) return "cache head_dim must match q head_dim";
+  *window = integer(sliding_window_size);
+  if (*window < 0) return "sliding_window_size must be >= 0";
+  const int64_t batch = qp.size(0) - 1;
+  if (batch <= 0) return "batch must be > 0";
+  if (vc.size(1) != n_kv) return "v_cache shape must match k_cache";
+  if (const Wrong w = attention_dtype(q, kc, vc, false)) return w;
+  if (const Wrong w = int32_of(qp, "qo_indptr")) return w;
+  if (const Wrong w = int32_of(ip, "kv_indptr")) return w;
+  if (const Wrong w = int32_of(ix, "kv_indices")) return w;
+  if (const Wrong w = int32_of(pl, "prefix_lens")) return w;
+  if (ip.size(0) != batch + 1 || pl.size(0) != batch) return "kv_indptr / prefix_lens length must match qo_indptr";
+  return device_of({&q, &kc, &vc, &qp, &ip, &ix, &pl}, dev);
+}
+
 PyObject* paged_prefill_attention(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 12, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "paged_prefill_attention";
     const Tensor &q = tensor(a[0], "q"), &kc = tensor(a[1], "k_cache"), &vc = tensor(a[2], "v_cache");
     const Tensor &qp = tensor(a[3], "qo_indptr"), &ip = tensor(a[4], "kv_indptr"), &ix = tensor(a[5], "kv_indices");
     const Tensor& pl = tensor(a[6], "prefix_lens");
-    if (q.dim() != 3) fail(op, "q must be 3D (total_q_tokens, num_q_heads, head_dim)");
-    if (kc.dim() != 3 || vc.dim() != 3) fail(op, "k_cache and v_cache must be 3D (num_pages, num_kv_heads, head_dim)");
-    if (qp.dim() != 1 || ip.dim() != 1 || ix.dim() != 1 || pl.dim() != 1)
-      fail(op, "qo_indptr, kv_indptr, kv_indices, prefix_lens must be 1D");
-    const int64_t total_q = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1);
-    if (d != 128 && d != 256) fail(op, "head_dim must be 128 or 256");
-    if (n_kv == 0 || n_q % n_kv != 0) fail(op, "num_q_heads must be a multiple of num_kv_heads");
-    if (kc.size(2) != d || vc.size(2) != d) fail(op, "cache head_dim must match q head_dim");
-    const int64_t window = integer(a[10]);
-    if (window < 0) fail(op, "sliding_window_size must be >= 0");
-    const int64_t batch = qp.size(0) - 1;
-    if (batch <= 0) fail(op, "batch must be > 0");
-    if (vc.size(1) != n_kv) fail(op, "v_cache shape must match k_cache");
-    const int32_t dtype = attention_dtype(op, q, kc, vc, false);
-    require_int32(op, qp, "qo_indptr");
-    require_int32(op, ip, "kv_indptr");
-    require_int32(op, ix, "kv_indices");
-    require_int32(op, pl, "prefix_lens");
-    if (ip.size(0) != batch + 1 || pl.size(0) != batch) fail(op, "kv_indptr / prefix_lens length must match qo_indptr");
-    const c10::Device dev = require_device(op, {&q, &kc, &vc, &qp, &ip, &ix, &pl});
+    int64_t window;
+    c10::Device dev = c10::kCPU;
+    require(op, prefill_args(q, kc, vc, qp, ip, ix, pl, a[10], &window, &dev));
+    const int64_t total_q = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1), batch = qp.size(0) - 1;
     const float scale = static_cast<float>(real(a[7]));
     const int64_t max_extend = integer(a[8]);
     const bool cross = truth(a[9]);
@@ -308,7 +353,7 @@ PyObject* paged_prefill_attention(PyObject*, PyObject* const* args, Py_ssize_t n
         rc = msgl_paged_prefill_attention(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(qpc), ints(ipc), ints(ixc),
                                           ints(plc), out.data_ptr(), data_or_null(ws), bytes, batch, total_q, total_kv,
                                           n_q, n_kv, d, kc.size(0), kcs, vcs, scale, static_cast<int32_t>(max_extend),
-                                          cross ? 1 : 0, static_cast<int32_t>(window), dtype, on.ptr());
+                                          cross ? 1 : 0, static_cast<int32_t>(window), dtype_code(q), on.ptr());
       }
     }
     check_rc(op, rc);
@@ -465,38 +510,49 @@ PyObject* build_metadata_from_host(PyObject*, PyObject* const* args, Py_ssize_t 
   });
 }
 
+Wrong heads_form(const Tensor& t, const char* name) {
+  if (t.dim() != 3) return {name, " must be 3D (tokens, heads, head_dim)"};
+  return whole_rows(t) ? Wrong() : Wrong(name, " must be contiguous in its (heads, head_dim) dimensions");
+}
 int64_t heads_stride0(const char* op, const Tensor& t, const char* name) {
-  if (t.dim() != 3) fail(op, std::string(name) + " must be 3D (tokens, heads, head_dim)");
-  if (t.stride(2) != 1 || t.stride(1) != t.size(2))
-    fail(op, std::string(name) + " must be contiguous in its (heads, head_dim) dimensions");
-  return t.size(0) > 1 ? t.stride(0) : t.size(1) * t.size(2);
+  require(op, heads_form(t, name));
+  return row_stride(t);
 }
 
 // ---- qk_norm_rope_store(q, k, v, q_weight, k_weight, positions, out_loc, k_cache, v_cache, eps,
 //                         rope_base, validate) -> rotated q -----------------------------------------
+Wrong norm_rope_args(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qw, const Tensor& kw, const Tensor& pos,
+                     const Tensor& loc, const Tensor& kc, const Tensor& vc, c10::Device* dev) {
+  if (const Wrong w = device_of({&q, &k, &v, &qw, &kw, &pos, &loc, &kc, &vc}, dev)) return w;
+  const std::pair<const Tensor*, const char*> typed[] = {{&q, "q"}, {&k, "k"}, {&v, "v"}, {&kc, "k_cache"},
+                                                         {&vc, "v_cache"}, {&qw, "q_weight"}, {&kw, "k_weight"}};
+  for (int i = 0; i < 3; ++i)
+    if (const Wrong w = heads_form(*typed[i].first, typed[i].second)) return w;
+  const int64_t tokens = q.size(0), d = q.size(2), n_kv = k.size(1);
+  if (d != 128 && d != 256) return "head_dim must be 128 or 256";
+  if (k.size(0) != tokens || k.size(2) != d || v.sizes() != k.sizes()) return "k and v shape must be (tokens, num_kv_heads, head_dim)";
+  if (kc.dim() != 3 || kc.size(1) != n_kv || kc.size(2) != d || vc.sizes() != kc.sizes())
+    return "k_cache and v_cache must be (num_pages, num_kv_heads, head_dim)";
+  for (const auto& [t, name] : typed)
+    if (t->scalar_type() != at::kBFloat16) return {name, " must be bfloat16"};
+  if (qw.dim() != 1 || qw.size(0) != d || kw.dim() != 1 || kw.size(0) != d) return "q_weight and k_weight must be (head_dim,)";
+  if (const Wrong w = int32_of(pos, "positions")) return w;
+  if (const Wrong w = int32_of(loc, "out_loc")) return w;
+  if (pos.dim() < 1 || loc.dim() < 1 || pos.size(0) != tokens || loc.size(0) != tokens)
+    return "positions and out_loc length must match q length";
+  return {};
+}
+
 PyObject* qk_norm_rope_store(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 12, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "qk_norm_rope_store";
     const Tensor &q = tensor(a[0], "q"), &k = tensor(a[1], "k"), &v = tensor(a[2], "v"), &qw = tensor(a[3], "q_weight");
     const Tensor &kw = tensor(a[4], "k_weight"), &pos = tensor(a[5], "positions"), &loc = tensor(a[6], "out_loc");
     const Tensor &kc = tensor(a[7], "k_cache"), &vc = tensor(a[8], "v_cache");
-    const c10::Device dev = require_device(op, {&q, &k, &v, &qw, &kw, &pos, &loc, &kc, &vc});
-    const int64_t qs = heads_stride0(op, q, "q"), ks = heads_stride0(op, k, "k"), vs = heads_stride0(op, v, "v");
+    c10::Device dev = c10::kCPU;
+    require(op, norm_rope_args(q, k, v, qw, kw, pos, loc, kc, vc, &dev));
+    const int64_t qs = row_stride(q), ks = row_stride(k), vs = row_stride(v);
     const int64_t tokens = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = k.size(1);
-    if (d != 128 && d != 256) fail(op, "head_dim must be 128 or 256");
-    if (k.size(0) != tokens || k.size(2) != d || v.sizes() != k.sizes())
-      fail(op, "k and v shape must be (tokens, num_kv_heads, head_dim)");
-    if (kc.dim() != 3 || kc.size(1) != n_kv || kc.size(2) != d || vc.sizes() != kc.sizes())
-      fail(op, "k_cache and v_cache must be (num_pages, num_kv_heads, head_dim)");
-    const std::pair<const Tensor*, const char*> typed[] = {{&q, "q"}, {&k, "k"}, {&v, "v"}, {&kc, "k_cache"},
-                                                           {&vc, "v_cache"}, {&qw, "q_weight"}, {&kw, "k_weight"}};
-    for (const auto& [t, name] : typed)
-      if (t->scalar_type() != at::kBFloat16) fail(op, std::string(name) + " must be bfloat16");
-    if (qw.dim() != 1 || qw.size(0) != d || kw.dim() != 1 || kw.size(0) != d) fail(op, "q_weight and k_weight must be (head_dim,)");
-    require_int32(op, pos, "positions");
-    require_int32(op, loc, "out_loc");
-    if (pos.dim() < 1 || loc.dim() < 1 || pos.size(0) != tokens || loc.size(0) != tokens)
-      fail(op, "positions and out_loc length must match q length");
     const float eps = static_cast<float>(real(a[9])), base = static_cast<float>(real(a[10]));
     debug_checks(a[11], op, {a[6], a[7]});
     const int64_t kcs = pool_stride0(op, kc, "k_cache"), vcs = pool_stride0(op, vc, "v_cache");
@@ -519,115 +575,92 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* args, Py_ssize_t n_args
 // ---- decode_step(q, k, v, q_weight | None, k_weight | None, positions | None, out_loc, k_cache, v_cache, kv_indptr,
 //                  kv_indices, num_kv_splits, sm_scale, eps, rope_base) -> out or None ------------------
 // Decode attention with the store (or norm, rotary embedding and store) inside, None where that is not the way: the
-// caller then makes the two calls, which check what is refused here and say why, and take every form.
+// caller then makes the two calls, which say what is wrong with their arguments, and take every form.
+//
+// What is refused here is what one of the two operators refuses (their own checks), what one of them would copy first,
+// and what the C ABI refuses before it launches anything (strides, alignment, constants).
+bool steps_are_checked() {  // index validation is the operators'
+  const char* env = std::getenv("MSGL_DEBUG_CHECKS");
+  return env && *env && std::strcmp(env, "0") != 0;
+}
+bool as_they_are(std::initializer_list<const Tensor*> rows, std::initializer_list<const Tensor*> indices) {
+  for (const Tensor* t : rows)
+    if (!whole_rows(*t)) return false;
+  for (const Tensor* t : indices)
+    if (t->dim() != 1 || !t->is_contiguous()) return false;
+  return true;
+}
+PyObject* step_result(const char* op, int rc, Tensor&& out) {
+  if (rc == MSGL_ERR_SHAPE || rc == MSGL_ERR_ALIGNMENT) return none();  // the two kinds that are left to the C ABI
+  check_rc(op, rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
 PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 15, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "decode_step";
     const bool norm = a[3] != Py_None;
     for (int i = 0; i < 12; ++i)
       if (!THPVariable_Check(a[i]) && (norm || i < 3 || i > 5)) return none();
-    if (const char* env = std::getenv("MSGL_DEBUG_CHECKS"); env && *env && std::strcmp(env, "0") != 0) return none();
+    if (steps_are_checked()) return none();
     auto t = [&](int i) -> const Tensor& { return THPVariable_Unpack(a[i]); };
     const Tensor &q = t(0), &k = t(1), &v = t(2), &loc = t(6), &kc = t(7), &vc = t(8), &ip = t(9), &ix = t(10), &ns = t(11);
-    if (q.dim() != 3 || k.dim() != 3 || kc.dim() != 3 || vc.dim() != 3) return none();
-    const int64_t batch = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = k.size(1), slots = kc.size(0);
-    const auto dt = q.scalar_type();
-    if (batch == 0 || slots == 0 || n_kv == 0 || n_q == 0 || (dt != at::kBFloat16 && (norm || dt != at::kHalf))) return none();
-    const c10::Device dev = q.device();
-    if (!dev.is_cuda()) return none();
-    auto same = [&](const Tensor& x) { return x.scalar_type() == dt && x.device() == dev; };
-    auto ints_of = [&](const Tensor& x, int64_t n) {
-      return x.dim() == 1 && x.size(0) == n && x.scalar_type() == at::kInt && x.device() == dev && x.is_contiguous();
-    };
-    auto rows = [&](const Tensor& x) {
-      return x.stride(2) == 1 && x.stride(1) == d && (batch == 1 || (x.stride(0) >= x.size(1) * d && x.stride(0) % 8 == 0)) &&
-             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-    };
-    auto pool = [&](const Tensor& x) {
-      return x.stride(2) == 1 && x.stride(1) == d && (slots == 1 || (x.stride(0) >= n_kv * d && x.stride(0) % 8 == 0)) &&
-             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-    };
-    const c10::IntArrayRef pool_size = kc.sizes();
-    if (!same(k) || !same(v) || !same(kc) || !same(vc) || k.size(0) != batch || k.size(2) != d || v.sizes() != k.sizes() ||
-        pool_size[1] != n_kv || pool_size[2] != d || vc.sizes() != pool_size || !rows(q) || !rows(k) || !rows(v) || !pool(kc) ||
-        !pool(vc) || !ints_of(loc, batch) || !ints_of(ip, batch + 1) || !ints_of(ix, ix.numel()) || !ints_of(ns, batch))
+    c10::Device dev = c10::kCPU, again = c10::kCPU;
+    if (decode_args(q, kc, vc, ip, ix, ns, &dev) || !as_they_are({&q, &kc, &vc}, {&ip, &ix, &ns})) return none();
+    if (norm ? bool(norm_rope_args(q, k, v, t(3), t(4), t(5), loc, kc, vc, &again)) : bool(store_args(kc, vc, loc, k, v, &again)))
       return none();
-    float eps = 0.f, base = 0.f;
-    if (norm) {
-      auto weight = [&](const Tensor& x) {
-        return same(x) && x.dim() == 1 && x.size(0) == d && x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-      };
-      if (!weight(t(3)) || !weight(t(4)) || !ints_of(t(5), batch)) return none();
-      eps = static_cast<float>(real(a[13]));
-      base = static_cast<float>(real(a[14]));
-      if (!(base > 1.0f) || !(eps >= 0.0f)) return none();
-    }
+    const int64_t batch = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1), slots = kc.size(0);
+    if (again != dev || loc.size(0) != batch || !as_they_are({&k, &v}, {&loc})) return none();
+    if (norm && !as_they_are({}, {&t(3), &t(4), &t(5)})) return none();
     const size_t bytes = msgl_decode_step_workspace_bytes(batch, ix.size(0), n_q, n_kv, d, norm ? 1 : 0);
     if (bytes == 0) return none();
     const float scale = static_cast<float>(real(a[12]));
-    auto stride0 = [](const Tensor& x) { return x.size(0) > 1 ? x.stride(0) : x.size(1) * x.size(2); };
+    const float eps = norm ? static_cast<float>(real(a[13])) : 0.f, base = norm ? static_cast<float>(real(a[14])) : 0.f;
     Tensor out;
     int rc;
     {
       NoGil nogil;
       OnDevice on(dev);
-      out = empty({batch, n_q, d}, dt, dev);
+      out = empty({batch, n_q, d}, q.scalar_type(), dev);
       const Tensor ws = scratch(bytes, dev);
-      rc = msgl_decode_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), stride0(q), stride0(k), stride0(v),
+      rc = msgl_decode_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), row_stride(q), row_stride(k), row_stride(v),
                             norm ? t(3).data_ptr() : nullptr, norm ? t(4).data_ptr() : nullptr, norm ? ints(t(5)) : nullptr,
                             ints(loc), kc.data_ptr(), vc.data_ptr(), ints(ip), ints(ix), out.data_ptr(), ws.data_ptr(), bytes,
-                            batch, ix.size(0), n_q, n_kv, d, slots, stride0(kc), stride0(vc), scale, eps, base,
-                            dt == at::kHalf ? MSGL_DTYPE_F16 : MSGL_DTYPE_BF16, on.ptr());
+                            batch, ix.size(0), n_q, n_kv, d, slots, row_stride(kc), row_stride(vc), scale, eps, base,
+                            dtype_code(q), on.ptr());
     }
-    check_rc(op, rc);
-    return THPVariable_Wrap(std::move(out));
+    return step_result(op, rc, std::move(out));
   });
 }
 
 // ---- extend_step(q, k, v, out_loc, k_cache, v_cache, qo_indptr, kv_indptr, kv_indices, prefix_lens, sm_scale,
 //                  max_len_extend, is_cross_attention, sliding_window_size, own_slots) -> out or None ----
 // As decode_step, for prefill metadata; the two launches are made here too where one is not the way, and always
-// without own_slots.
+// without own_slots.  (Where the second of them is refused, the rows are stored as the first call would have.)
 PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return guarded(args, n_args, 15, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "extend_step";
     for (int i = 0; i < 10; ++i)
       if (!THPVariable_Check(a[i])) return none();
+    if (steps_are_checked()) return none();
     auto t = [&](int i) -> const Tensor& { return THPVariable_Unpack(a[i]); };
     const Tensor &q = t(0), &k = t(1), &v = t(2), &loc = t(3), &kc = t(4), &vc = t(5), &qp = t(6), &ip = t(7), &ix = t(8), &pl = t(9);
-    if (q.dim() != 3 || k.dim() != 3 || kc.dim() != 3 || vc.dim() != 3 || qp.dim() != 1 || ix.dim() != 1) return none();
-    const int64_t total = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = k.size(1), slots = kc.size(0), batch = qp.size(0) - 1;
-    const c10::Device dev = q.device();
-    if (total == 0 || batch <= 0 || slots == 0 || q.scalar_type() != at::kBFloat16 || !dev.is_cuda()) return none();
-    const int64_t max_extend = integer(a[11]), window = integer(a[13]);
+    int64_t window = 0;
+    c10::Device dev = c10::kCPU, again = c10::kCPU;
+    if (prefill_args(q, kc, vc, qp, ip, ix, pl, a[13], &window, &dev) || store_args(kc, vc, loc, k, v, &again)) return none();
+    if (again != dev || !q.is_contiguous() || !as_they_are({&k, &v, &kc, &vc}, {&loc, &qp, &ip, &ix, &pl})) return none();
+    const int64_t total = q.size(0), n_q = q.size(1), d = q.size(2), n_kv = kc.size(1), slots = kc.size(0), batch = qp.size(0) - 1;
+    const int64_t max_extend = integer(a[11]);
     const bool cross = truth(a[12]), own_slots = truth(a[14]);
-    if (window < 0 || window > 0x7fffffff || max_extend <= 0 || max_extend > 0x7fffffff || (d != 128 && d != 256) || n_kv == 0 ||
-        n_q == 0 || n_q % n_kv != 0)
-      return none();
-    if (const char* env = std::getenv("MSGL_DEBUG_CHECKS"); env && *env && std::strcmp(env, "0") != 0) return none();
-    auto same = [&](const Tensor& x) { return x.scalar_type() == at::kBFloat16 && x.device() == dev; };
-    auto ints_of = [&](const Tensor& x, int64_t n) {
-      return x.dim() == 1 && x.size(0) == n && x.scalar_type() == at::kInt && x.device() == dev && x.is_contiguous();
-    };
-    auto rows = [&](const Tensor& x) {
-      return x.stride(2) == 1 && x.stride(1) == d && (x.size(0) == 1 || (x.stride(0) >= x.size(1) * d && x.stride(0) % 8 == 0)) &&
-             reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-    };
-    const c10::IntArrayRef pool_size = kc.sizes();
-    if (!same(k) || !same(v) || !same(kc) || !same(vc) || k.size(0) != total || k.size(2) != d || v.sizes() != k.sizes() ||
-        pool_size[1] != n_kv || pool_size[2] != d || vc.sizes() != pool_size || !q.is_contiguous() || !rows(q) || !rows(k) ||
-        !rows(v) || !rows(kc) || !rows(vc) || !ints_of(loc, total) || !ints_of(qp, batch + 1) || !ints_of(ip, batch + 1) ||
-        !ints_of(ix, ix.numel()) || !ints_of(pl, batch))
-      return none();
+    if (total == 0 || loc.size(0) != total || max_extend <= 0 || std::max(max_extend, window) > 0x7fffffff) return none();
     const float scale = static_cast<float>(real(a[10]));
-    auto stride0 = [](const Tensor& x) { return x.size(0) > 1 ? x.stride(0) : x.size(1) * x.size(2); };
     Tensor out;
     int rc;
     {
       NoGil nogil;
       OnDevice on(dev);
-      out = empty({total, n_q, d}, at::kBFloat16, dev);
-      const int64_t ks0 = stride0(k), vs0 = stride0(v), kcs = stride0(kc), vcs = stride0(vc);
+      out = empty({total, n_q, d}, q.scalar_type(), dev);
+      const int64_t ks0 = row_stride(k), vs0 = row_stride(v), kcs = row_stride(kc), vcs = row_stride(vc);
       size_t bytes = !own_slots ? 0 : msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross,
                                                                        static_cast<int32_t>(window));
       if (bytes > 0) {
@@ -635,22 +668,21 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), ks0, vs0, ints(loc), kc.data_ptr(), vc.data_ptr(), ints(qp),
                               ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.data_ptr(), bytes, batch, total, ix.size(0), n_q,
                               n_kv, d, slots, kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
-                              static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+                              static_cast<int32_t>(window), dtype_code(q), on.ptr());
       } else {
         rc = msgl_store_kv_cache(kc.data_ptr(), vc.data_ptr(), ints(loc), k.data_ptr(), v.data_ptr(), total, n_kv, d, slots, kcs,
-                                 vcs, ks0, vs0, 2, on.ptr());
+                                 vcs, ks0, vs0, static_cast<int32_t>(kc.element_size()), on.ptr());
         if (rc == MSGL_OK) {
           bytes = msgl_paged_prefill_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend);
           const Tensor ws = scratch(bytes, dev);
           rc = msgl_paged_prefill_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(qp), ints(ip), ints(ix), ints(pl),
                                             out.data_ptr(), data_or_null(ws), bytes, batch, total, ix.size(0), n_q, n_kv, d, slots,
                                             kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
-                                            static_cast<int32_t>(window), MSGL_DTYPE_BF16, on.ptr());
+                                            static_cast<int32_t>(window), dtype_code(q), on.ptr());
         }
       }
     }
-    check_rc(op, rc);
-    return THPVariable_Wrap(std::move(out));
+    return step_result(op, rc, std::move(out));
   });
 }
 

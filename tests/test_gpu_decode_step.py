@@ -246,3 +246,76 @@ def test_rows_of_no_request_are_stored(gpu, cached, ext, n_q, n_kv, d, nobodys, 
     at = torch.cat([torch.arange(min(e, limit)) + front + sum(ext[:b]) for b, e in enumerate(ext)])  # past the limit: not computed
     diff = (got[at].float() - want[at].float()).abs()
     assert sum(ext) == 0 or (float(diff.max()) <= 2e-2 and float(diff.mean()) <= 1e-3), (float(diff.max()), float(diff.mean()))
+
+
+def _turned(x):  # the same values, heads outermost
+    return x.transpose(0, 1).contiguous().transpose(0, 1)
+
+
+def _odd_rows(x):  # rows that start at odd multiples of 2 bytes
+    wide = x.new_zeros((x.shape[0], x.numel() // x.shape[0] + 1))
+    wide[:, 1:] = x.flatten(1)
+    return wide[:, 1:].view(x.shape)
+
+
+def _every_other(x):
+    return torch.stack([x, x], dim=1).flatten()[::2]
+
+
+# what one of the two operators refuses ...
+REFUSED = {
+    "q flat": dict(q=lambda x: x.flatten(1)), "k flat": dict(k=lambda x: x.flatten(1)), "k and v short": dict(k=lambda x: x[1:], v=lambda x: x[1:]),
+    "v of another type": dict(v=lambda x: x.half()), "q float": dict(q=lambda x: x.float()), "heads that do not divide": dict(q=lambda x: x[:, :-1]),
+    "slots int64": dict(loc=lambda x: x.long()), "one slot too few": dict(loc=lambda x: x[1:]), "one offset too few": dict(kv_indptr=lambda x: x[1:]),
+    "ids int64": dict(kv_indices=lambda x: x.long()), "v pool shorter": dict(vc=lambda x: x[:-1]), "k pool turned": dict(kc=_turned),
+    "slots in host memory": dict(loc=lambda x: x.cpu()),
+}
+# ... and what one of them copies, or the C ABI refuses
+FORMS = REFUSED | {
+    "q turned": dict(q=_turned), "k turned": dict(k=_turned), "q off by 2 bytes": dict(q=_odd_rows), "k off by 2 bytes": dict(k=_odd_rows),
+    "k repeated": dict(k=lambda x: x[:1].expand(x.shape)), "slots strided": dict(loc=_every_other), "offsets strided": dict(kv_indptr=_every_other),
+    "ids strided": dict(kv_indices=_every_other), "k pool off by 2 bytes": dict(kc=_odd_rows),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("kind", ["decode", "norm", "extend"])
+def test_forms_that_steps_leave_to_the_two_calls(gpu, kind, form):
+    """None, and nothing stored; what the two calls refuse they go on to say."""
+    ext = [3, 2] if kind == "extend" else [1, 1]
+    kv = [40, 70]
+    wl = build_workload("step", "prefill", seed=5, n_q=16, n_kv=8, head_dim=128, kv_lens=kv, extend_lens=ext).to(gpu)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(5)
+    rows = lambda n: torch.randn((sum(ext), n, 128), generator=g, device=gpu).bfloat16()  # noqa: E731
+    t = dict(q=rows(16), k=rows(8), v=rows(8), kc=wl.k_cache, vc=wl.v_cache, kv_indptr=wl.kv_indptr, kv_indices=wl.kv_indices,
+             loc=torch.cat([wl.kv_indices[int(wl.kv_indptr[b + 1]) - e:int(wl.kv_indptr[b + 1])] for b, e in enumerate(ext)]))
+    t |= {name: change(t[name]) for name, change in FORMS[form].items()}
+    kc, vc = t["kc"].clone(), t["vc"].clone()
+    w, pos = torch.ones(128, dtype=torch.bfloat16, device=gpu), torch.arange(2, dtype=torch.int32, device=gpu)
+    splits = torch.ones(2, dtype=torch.int32, device=gpu)
+
+    def one_launch():
+        pools = (t["loc"], t["kc"], t["vc"])
+        if kind == "extend":
+            return extend_step(t["q"], t["k"], t["v"], *pools, wl.qo_indptr, t["kv_indptr"], t["kv_indices"], wl.prefix_lens,
+                               sm_scale=0.1, max_len_extend=max(ext))
+        norm = dict(q_weight=w, k_weight=w, positions=pos, eps=1e-6, rope_base=1e6) if kind == "norm" else {}
+        return decode_step(t["q"], t["k"], t["v"], *pools, t["kv_indptr"], t["kv_indices"], splits, sm_scale=0.1, **norm)
+
+    def two_calls():
+        q = t["q"]
+        if kind == "norm":
+            q = qk_norm_rope_store(q, t["k"], t["v"], w, w, pos, t["loc"], kc, vc, eps=1e-6, rope_base=1e6)
+        else:
+            store_kv_cache(kc, vc, t["loc"], t["k"], t["v"])
+        if kind == "extend":
+            return paged_prefill_attention(q, kc, vc, wl.qo_indptr, t["kv_indptr"], t["kv_indices"], wl.prefix_lens, 0.1, max(ext))
+        return paged_decode_attention(q, kc, vc, t["kv_indptr"], t["kv_indices"], splits, 0.1, 32)
+
+    print(f"{kind}: {form}", flush=True)
+    assert one_launch() is None
+    assert torch.equal(t["kc"], kc) and torch.equal(t["vc"], vc)
+    if form in REFUSED:
+        with pytest.raises(RuntimeError):
+            two_calls()
