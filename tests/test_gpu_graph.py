@@ -8,7 +8,7 @@ import math
 import pytest
 import torch
 
-from mini_sglang_amd_kernel import (build_attention_metadata, paged_decode_attention,
+from mini_sglang_amd_kernel import (_lib, build_attention_metadata, decode_step, extend_step, paged_decode_attention,
                                     paged_prefill_attention, qk_norm_rope_store)
 
 pytestmark = pytest.mark.gpu
@@ -49,9 +49,43 @@ class _State:
         self.out.copy_(res)
 
 
+class _OneLaunch(_State):
+    """The same step with everything behind the metadata in one launch; ``norm`` off: the store alone."""
+
+    norm = True
+
+    def step(self):
+        self.kv_lens.add_(1)
+        meta = build_attention_metadata(self.page_table, self.table_rows, self.kv_lens,
+                                        total_kv=BATCH * MAX_SEQ)
+        out_loc = self.page_table[self.table_rows.long(), (self.kv_lens - 1).long()]
+        norm = dict(q_weight=self.qw, k_weight=self.kw, positions=meta["positions"], eps=EPS, rope_base=BASE) if self.norm else {}
+        res = decode_step(self.q, self.k, self.v, out_loc, self.k_cache, self.v_cache, meta["kv_indptr"], meta["kv_indices"],
+                          meta["num_kv_splits"], sm_scale=1.0 / math.sqrt(D), **norm)
+        assert res is not None
+        self.out.copy_(res)
+
+
+class _OneLaunchPlain(_OneLaunch):
+    norm = False
+
+
+@pytest.mark.parametrize("state,segments", [(_OneLaunch, False), (_OneLaunchPlain, False), (_OneLaunchPlain, True)])
+def test_decode_step_in_one_launch_replays_from_a_graph(gpu, tuning, state, segments):
+    """In shares, whose count words a replay finds as the launch before left them, and in segments."""
+    if segments:
+        tuning(_lib.TUNE_SHARES, -1)
+        tuning(_lib.TUNE_MIN_SEGMENT, 64)
+    _replay_decode_steps(gpu, state)
+
+
 def test_decode_step_replays_from_a_graph(gpu):
+    _replay_decode_steps(gpu, _State)
+
+
+def _replay_decode_steps(gpu, state):
     torch.cuda.set_device(gpu)
-    captured, eager = _State(gpu, 21), _State(gpu, 21)
+    captured, eager = state(gpu, 21), state(gpu, 21)
     g = torch.Generator().manual_seed(22)
     tokens = [[torch.randn(s, generator=g).to(torch.bfloat16) for s in
                ((BATCH, N_Q, D), (BATCH, N_KV, D), (BATCH, N_KV, D))] for _ in range(7)]
@@ -123,3 +157,43 @@ def test_extend_with_key_splits_replays_from_a_graph(gpu):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out.view(torch.int16), want.view(torch.int16)), f"extend {extend} replay {i}"
+
+
+@pytest.mark.parametrize("cached,ext", [([900, 40, 0, 2000], [6, 6, 6, 5]),   # shares
+                                        ([0, 300], [60, 33]),                  # the tile kernel stores them
+                                        ([3000, 100], [40, 40])])              # ... and leaves partials
+def test_extend_step_in_one_launch_replays_from_a_graph(gpu, cached, ext):
+    from mini_sglang_amd.workloads import build_workload
+
+    torch.cuda.set_device(gpu)
+    kv = [c + e for c, e in zip(cached, ext)]
+    w = build_workload("t", "prefill", seed=37, n_q=N_Q, n_kv=N_KV, head_dim=D, kv_lens=kv, extend_lens=ext).to(gpu)
+    loc = torch.cat([w.kv_indices[int(w.kv_indptr[b + 1]) - e:int(w.kv_indptr[b + 1])] for b, e in enumerate(ext)])
+    assert _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(kv), N_Q, N_KV, D, max(ext), 0, 0) > 0  # one launch
+    rows = lambda n, seed: torch.randn((sum(ext), n, D), generator=torch.Generator().manual_seed(seed)).to(gpu, torch.bfloat16)  # noqa: E731
+    q, k, v = rows(N_Q, 1), rows(N_KV, 2), rows(N_KV, 3)
+    pools = [(w.k_cache.clone(), w.v_cache.clone()) for _ in range(2)]
+
+    def run(kc, vc):
+        return extend_step(q, k, v, loc, kc, vc, w.qo_indptr, w.kv_indptr, w.kv_indices, w.prefix_lens, sm_scale=w.sm_scale,
+                           max_len_extend=max(ext))
+
+    want = run(*pools[0])
+    run(*pools[1])
+    torch.cuda.synchronize()
+    out = torch.zeros_like(want)
+    print(f"capturing an extend step {cached} + {ext}", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out.copy_(run(*pools[1]))
+    for i in range(4):
+        if i:  # new rows in the same buffers
+            for t, seed in ((q, 10 * i), (k, 10 * i + 1), (v, 10 * i + 2)):
+                t.copy_(rows(t.shape[1], seed))
+            want = run(*pools[0])
+            torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), f"replay {i}"
+        for a, b in zip(*pools):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"replay {i}"
