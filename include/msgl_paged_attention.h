@@ -8,6 +8,7 @@
  *   paged_decode_attention    GQA split-K decode over slots gathered through kv_indices
  *   paged_prefill_attention   extend attention (causal / full / window / bidirectional+window)
  *
+ * two calls that put a step's store inside its attention launch (msgl_decode_step, msgl_extend_step),
  * and the step's metadata build that feeds them (slot table -> CSR arrays), which the
  * reference does in Python (mini_sglang_mlx/attention/backend.py:205-307).
  *
