@@ -43,7 +43,7 @@
 //      1     X, R                           Z, two blocks of P to LDS      T of chunk j, K and Q of chunk j + 1 to LDS
 //      2     U, two blocks of A of j + 1    P of chunk j + 1               A, the diagonal blocks of T of chunk j + 1
 //      3     S                              Y, three blocks of P to LDS    the other blocks of T of chunk j + 1, V of j + 2
-// A chunk takes 7.7 K cycles (slots of 2.5, 2.4 and 2.7 K, every role 2.0-2.6 K of each).  It is 1.5 times the work of
+// A chunk takes 7.7 K cycles (slots of 2.5, 2.4 and 2.7 K, every role 1.9-2.6 K of each).  It is 1.5 times the work of
 // the chip for a chunk, so a launch that fills the compute units evenly has no pairs (see in_pairs()).
 //
 // Precision: fp32 throughout, as in the token kernel.  q, k, v are bf16 and enter the bf16 matrix

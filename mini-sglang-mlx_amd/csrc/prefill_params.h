@@ -221,8 +221,8 @@ inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
 // one's start: some 13 us outside the tile loop (finding the block, three dependent memory round trips, the epilogue)
 // with the compute unit idle.  Instead workgroup r of an XCD's 32 takes the blocks 32 i + r of the order above, or
 // 32 i + 31 - r in odd rounds i, as one stream of key tiles: the moves of a block's first tiles and its Q rows are
-// under way while the block before it is computed, and a change of blocks costs 6.5 K cycles (both wave groups'
-// rows and masks, in turn) beside 2.9 K a tile.  us, 32 / 8 heads unless said: prompts of 771-2710 tokens (11574 in
+// under way while the block before it is computed, and a block costs 8.4 K cycles (the change, in both wave groups
+// in turn, and the masks of its last tiles) beside 2.9 K a tile.  us, 32 / 8 heads unless said: prompts of 771-2710 tokens (11574 in
 // all) 249.8 -> 235.3, 30 x 100-300 on up to 500 cached 83.9 -> 74.9, 16 x 50-2000 at 64 / 8 heads 408 -> 370, three
 // of 1000-3000 under a window of 1024 166 -> 149.  A wave without rows computes all the same here (a loop of its own
 // costs 260 bytes of spills), and of few rounds the last ones are short, so it pays from two rounds of blocks on.  Those
@@ -230,8 +230,8 @@ inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
 // of 2, on 8 K keys: 4 rounds of the grid and 1.1 of blocks, 482 us and 601 with workgroups that stay; one of 4096 beside
 // fifteen of 16: 32 and 2.4, 153 and 131), so they are counted from all queries, a half for each
 // request's last block.  1050 launches of 1-64 even, ragged and very uneven extends, 4 and 8 kv heads, groups of 2-8, on
-// up to 8 K keys, staying against not, geometric means by such rounds: up to 1 1.10, 1-1.5 1.04, 1.5-2 0.985, 2-2.5
-// 0.963, 2.5-3 0.92, above 0.87-0.92; this line is 0.8 % from the better of the two on average, and 4 rounds of the
+// up to 8 K keys, staying against not, geometric means by such rounds: up to 1 1.11, 1-1.5 1.04, 1.5-2 0.99, 2-2.5
+// 0.96, 2.5-3 0.92, above 0.89; this line is 0.8 % from the better of the two on average, and four rounds of the
 // grid were 2.1 %.
 // The list of a workgroup's blocks is in LDS, hence the other limit (of the grid's rounds); an XCD's workgroups work on
 // one kv head (the bases of the moves stay the same).
