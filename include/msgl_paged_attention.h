@@ -356,6 +356,19 @@ MSGL_API int msgl_gdn_state_inplace(const void* q, const void* k, const void* v,
                            int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
                            int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
                            int64_t v_stride0, int32_t single_token_mode, void* stream);
+/*
+ * The same with scratch memory (16-byte aligned; NULL or too small: without), which requests of many
+ * tokens are faster with.  msgl_gdn_state_workspace_bytes: how much that is, 0 where it would not be used.
+ */
+MSGL_API size_t msgl_gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv,
+                                               int32_t single_token_mode);
+MSGL_API int msgl_gdn_state_inplace_in(const void* q, const void* k, const void* v, const void* g,
+                           const void* beta, void* state, const int32_t* slot_ids,
+                           const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
+                           int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
+                           int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
+                           int64_t v_stride0, int32_t single_token_mode, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /*
  * Tuning knobs, for benchmarking only (0 = built-in heuristic).  One set per HOST THREAD

@@ -840,12 +840,18 @@ int msgl_qk_norm_rope_store(const void* q, const void* k, const void* v, int64_t
   return msgl::launch_qk_norm_rope_store(a, static_cast<hipStream_t>(stream));
 }
 
-int msgl_gdn_state_inplace(const void* q, const void* k, const void* v, const void* g,
+size_t msgl_gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, int32_t single_token_mode) {
+  if (tokens <= 0 || batch <= 0 || hv <= 0) return 0;
+  return msgl::gdn_state_workspace_bytes(tokens, batch, hv, single_token_mode != 0);
+}
+
+int msgl_gdn_state_inplace_in(const void* q, const void* k, const void* v, const void* g,
                            const void* beta, void* state, const int32_t* slot_ids,
                            const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
                            int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
                            int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
-                           int64_t v_stride0, int32_t single_token_mode, void* stream) {
+                           int64_t v_stride0, int32_t single_token_mode, void* workspace,
+                              size_t workspace_bytes, void* stream) {
   if (dk != 128 || dv != 128) return MSGL_ERR_GDN_DIMS;  // gdn_state.cpp:80-83
   if (tokens < 0 || batch < 0 || hk <= 0 || hv <= 0 || num_slots < 0) return MSGL_ERR_SHAPE;
   if (hv % hk != 0) return MSGL_ERR_HEAD_RATIO;          // gdn_state.cpp:76-79
@@ -859,6 +865,7 @@ int msgl_gdn_state_inplace(const void* q, const void* k, const void* v, const vo
   if (!aligned16(q) || !aligned16(k) || !aligned16(state) || q_stride0 % 8 || k_stride0 % 8 ||
       state_stride0 % 4)
     return MSGL_ERR_ALIGNMENT;
+  if (workspace && !aligned16(workspace)) return MSGL_ERR_ALIGNMENT;
   msgl::GdnArgs a{};
   a.q = q;
   a.k = k;
@@ -878,7 +885,19 @@ int msgl_gdn_state_inplace(const void* q, const void* k, const void* v, const vo
   a.k_stride0 = k_stride0;
   a.v_stride0 = v_stride0;
   a.single_token_mode = single_token_mode;
+  a.workspace = workspace;
+  a.workspace_bytes = workspace_bytes;
   return msgl::launch_gdn_state(a, static_cast<hipStream_t>(stream));
+}
+
+int msgl_gdn_state_inplace(const void* q, const void* k, const void* v, const void* g,
+                           const void* beta, void* state, const int32_t* slot_ids,
+                           const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
+                           int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
+                           int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
+                           int64_t v_stride0, int32_t single_token_mode, void* stream) {
+  return msgl_gdn_state_inplace_in(q, k, v, g, beta, state, slot_ids, qo_indptr, y, tokens, batch, hk, hv, dk, dv, num_slots,
+                                   state_stride0, q_stride0, k_stride0, v_stride0, single_token_mode, nullptr, 0, stream);
 }
 
 }  // extern "C"

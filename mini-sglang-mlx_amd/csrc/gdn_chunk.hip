@@ -1,4 +1,5 @@
-// Gated delta rule over many tokens per request: chunks of 64 tokens on the matrix cores.
+// Gated delta rule over many tokens per request: chunks of 64 tokens on the matrix cores, in one launch.  (Requests of several
+// hundred tokens take two where there is memory for the systems below: gdn_long.hip.)
 //
 // The recurrence of gdn_state.hip (one state row dv of a head, tokens t = 1 .. 64 of a chunk, S the
 // state before the chunk, G_t the product of the decays g_1 .. g_t):
@@ -31,9 +32,7 @@
 // are split by the matrix pipe (see Split: 16 instructions instead of 44), Z and Y are made transposed (4 stores
 // of 8 bytes a chunk instead of 16 of 2), V comes by transposing LDS reads, the chunk waves share the blocks
 // out evenly (12.5 -> 10.7 K), and what a block needs from LDS is read whether it is used or not (no branches, so the
-// reads of several blocks go out together: 10.6 -> 10.4 K).  T and P of all chunks in a launch of their own, in
-// parallel, measured the same for the longest request of a launch and less for many short ones: their 20 KB per chunk
-// and head cost 40 us of writing for the requests above, and LDS and issue time in the serial part.
+// reads of several blocks go out together: 10.6 -> 10.4 K).
 //
 // Pairs: the longest request's chain ends a launch when the others have left their compute units, and a launch of few
 // requests never fills the chip.  Such requests go on four workgroups a value head, of 32 rows: waves 0-1 are state
@@ -66,23 +65,13 @@
 // stored in that order; for S^T the transposing LDS reads of K (4 tokens x 16 dims) pick their dims so
 // that result tile 2 s + h holds dims 32 s + 8 g + 4 h + i, which makes the pair (2 s, 2 s + 1) of a lane
 // 8 consecutive dims, the natural order of K and Q.
-#include <algorithm>
-
-#include "gdn_params.h"
-#include "prefill_tile_common.h"
+#include "gdn_chunk_tiles.h"
 
 namespace msgl {
 namespace {
 
-constexpr int kChunk = 64;        // tokens per chunk
 constexpr int kRowsPerWg = 64;    // dv rows of a workgroup
 constexpr int kRowsPaired = 32;   // where output waves take half of the state waves' work
-constexpr int kRanked = 512;      // requests ranked by length (one per thread)
-
-// T and P as operands: fragment f of row block m and contraction step c (32 columns), those that are not
-// zero; lane x16 + 16 g of a fragment holds row x16, columns 32 c + 4 g .. and 32 c + 16 + 4 g ..
-constexpr int kFragments = 6;
-__device__ constexpr int fragment(int m, int c) { return c == 0 ? m : m + 2; }
 
 template <bool PAIRED>
 struct ChunkLds {
@@ -91,6 +80,8 @@ struct ChunkLds {
   u32x4_t t[3][kFragments][64], p[3][kFragments][64];  // T and P in three bf16 parts
   float a[kChunk][68];            // A of the chunk being prepared (blocks on and below the diagonal)
   float diag[4][16][20];          // inverses of the diagonal blocks of I + A
+  __device__ __forceinline__ const float* a_row(int r, int c, int row) const { return &a[16 * r + row][16 * c]; }
+  __device__ __forceinline__ const float* diagonal_row(int r, int row) const { return diag[r][row]; }
   // per token, chunks j .. j + 2: beta, G, and tail_i = G_64 / G_i
   float beta[3][kChunk], gamma[3][kChunk], tail[3][kChunk];
   // of the chunk being prepared: the decays; products over the block of 16 up to a token, behind it, and
@@ -102,314 +93,6 @@ struct ChunkLds {
 };
 struct PairedLds : ChunkLds<true> {
   f32x4_t s[2][8][64], u[2][4][64];  // a state wave's S and U for its output wave, registers as they are
-};
-
-// Piece `c` of 16 bytes of row `row` lies at this place.  LDS serves 8 lanes of a 16-byte read and 16 of an
-// 8-byte one at a time: the rows 0-7 and 8-15 of an operand at one column go to 8 different places modulo 8,
-// the 4 rows x 4 columns of a transposing read to 16 different ones.
-__device__ __forceinline__ int swizzle(int row) {
-  const int r0 = row & 1, r1 = (row >> 1) & 1, r2 = (row >> 2) & 1, r3 = (row >> 3) & 1;
-  return (r1 ^ r3) << 3 | r0 << 2 | r1 << 1 | r2;
-}
-__device__ __forceinline__ int piece(int row, int c) { return c ^ swizzle(row); }
-
-// Eight fp32 values as three operands of bf16 parts: x = hi + mid + lo, each the nearest to what is left, so
-// exact.  The matrix pipe takes the parts off: x - hi is x plus the product of a matrix that picks, negated,
-// the result tile's rows out of the 32 contraction rows, and hi as it stands (12 conversions and 4 matrix
-// instructions; by vector instructions 44, and their issue is what a wave waits for).
-struct Split {
-  bf16x8_t hi, mid, lo;
-};
-struct Picker {
-  bf16x8_t first, second;
-  __device__ __forceinline__ Picker() {  // row 4 a + i of the first tile: contraction row 8 a + i; second: 8 a + 4 + i
-    const int x16 = lane_id() & 15, g = lane_id() >> 4;
-    u32x4_t f = {0u, 0u, 0u, 0u};
-    const uint32_t minus_one = g == (x16 >> 2) ? 0xbf80u << (16 * (x16 & 1)) : 0u;
-    const uint32_t even = (x16 & 2) ? 0u : minus_one, odd = (x16 & 2) ? minus_one : 0u;
-    f[0] = even;
-    f[1] = odd;
-    first = as_bf16x8(f);
-    second = as_bf16x8(u32x4_t{0u, 0u, even, odd});
-  }
-};
-__device__ __forceinline__ bf16x8_t nearest(f32x4_t a, f32x4_t b) {
-  return bf16x8_t{(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3], (__bf16)b[0], (__bf16)b[1], (__bf16)b[2], (__bf16)b[3]};
-}
-__device__ __forceinline__ Split split(const Picker& pick, f32x4_t a, f32x4_t b) {
-  Split s;
-  s.hi = nearest(a, b);
-  a = mfma_16x16x32(pick.first, s.hi, a);
-  b = mfma_16x16x32(pick.second, s.hi, b);
-  s.mid = nearest(a, b);
-  a = mfma_16x16x32(pick.first, s.mid, a);
-  b = mfma_16x16x32(pick.second, s.mid, b);
-  s.lo = nearest(a, b);
-  return s;
-}
-
-// Four neighbouring values of a row of T or P, a lane's part of block (r, c), to LDS.
-__device__ __forceinline__ void split_store(const Picker& pick, f32x4_t x, u32x4_t (*m)[kFragments][64], int r, int c) {
-  auto half = [&](f32x4_t f) { return u32x2_t{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])}; };
-  auto rest = [&](f32x4_t f, u32x2_t part) {
-    return mfma_16x16x32(pick.first, as_bf16x8(u32x4_t{part[0], part[1], 0u, 0u}), f);
-  };
-  const u32x2_t hi = half(x);
-  const f32x4_t y = rest(x, hi);
-  const u32x2_t mid = half(y);
-  const u32x2_t lo = half(rest(y, mid));
-  u32x2_t* to = reinterpret_cast<u32x2_t*>(&m[0][fragment(r, c >> 1)][lane_id()]) + (c & 1);
-  constexpr int kPart = kFragments * 64 * 2;
-  to[0] = hi;
-  to[kPart] = mid;
-  to[2 * kPart] = lo;
-}
-
-// LDS traffic of every wave done, then the workgroup barrier; loads from memory stay in flight.
-__device__ __forceinline__ void slot_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-__device__ __forceinline__ bf16x8_t operand(const uint16_t* p) {
-  return as_bf16x8(*reinterpret_cast<const u32x4_t*>(p));
-}
-
-struct Triangle {
-  bf16x8_t hi[kFragments], mid[kFragments], lo[kFragments];
-};
-template <int FROM, int TO>
-__device__ __forceinline__ void load_triangle(const u32x4_t (*m)[kFragments][64], Triangle& t) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int f = FROM; f < TO; ++f) {
-    t.lo[f] = as_bf16x8(m[2][f][lane]);
-    t.mid[f] = as_bf16x8(m[1][f][lane]);
-    t.hi[f] = as_bf16x8(m[0][f][lane]);
-  }
-}
-// a b, or its transpose: operands of both kinds have the same layout
-template <bool TRANSPOSED>
-__device__ __forceinline__ f32x4_t product(bf16x8_t a, bf16x8_t b, f32x4_t acc) {
-  return TRANSPOSED ? mfma_16x16x32(b, a, acc) : mfma_16x16x32(a, b, acc);
-}
-// acc += M B for contraction step 0 of M, B split: the six products above 2^-24, smallest first, four rows
-// of blocks side by side.
-template <bool TRANSPOSED>
-__device__ __forceinline__ void triangle_first(const Triangle& t, const Split& b, f32x4_t (&acc)[4]) {
-  auto step = [&](const bf16x8_t (&part)[kFragments], const bf16x8_t& b0) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = product<TRANSPOSED>(part[fragment(m, 0)], b0, acc[m]);
-  };
-  step(t.lo, b.hi);
-  step(t.mid, b.mid);
-  step(t.hi, b.lo);
-  step(t.mid, b.hi);
-  step(t.hi, b.mid);
-  step(t.hi, b.hi);
-}
-// The same for step 1, which two rows of blocks reach: three products of each in a sum of their own.
-template <bool TRANSPOSED>
-__device__ __forceinline__ void triangle_second(const Triangle& t, const Split& b, f32x4_t (&acc)[4]) {
-  f32x4_t x2 = {0.f, 0.f, 0.f, 0.f}, x3 = x2;
-  auto step = [&](const bf16x8_t (&pa)[kFragments], const bf16x8_t& ba, const bf16x8_t (&pb)[kFragments], const bf16x8_t& bb) {
-    x2 = product<TRANSPOSED>(pa[fragment(2, 1)], ba, x2);
-    x3 = product<TRANSPOSED>(pa[fragment(3, 1)], ba, x3);
-    acc[2] = product<TRANSPOSED>(pb[fragment(2, 1)], bb, acc[2]);
-    acc[3] = product<TRANSPOSED>(pb[fragment(3, 1)], bb, acc[3]);
-  };
-  step(t.lo, b.hi, t.mid, b.hi);
-  step(t.mid, b.mid, t.hi, b.mid);
-  step(t.hi, b.lo, t.hi, b.hi);
-  acc[2] += x2;
-  acc[3] += x3;
-}
-
-__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
-
-// The larger of m and the magnitudes of x, NaN if there is one (two instructions).
-__device__ __forceinline__ float largest(f32x4_t x, float m) {
-  auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
-  m = larger(larger(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])), m);
-  return larger(larger(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])), m);
-}
-// Finite, and so is the nearest bf16.
-__device__ __forceinline__ bool splits(float largest) { return largest < 0x1p127f; }
-
-// A parameter of the launch (they are the kernel's first argument), read where it stands: what is only needed behind
-// the chunks would push others out of the scalar registers meanwhile (2 % of a launch's time).
-template <typename T>
-__device__ __forceinline__ T parameter(T GdnParams::* member) {
-  auto args = __builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(args));
-  return ((const GdnParams*)args)->*member;
-}
-// Address of a lane's part of state row `row + lane % 16`: its four pieces of 8 dims lie 32 apart.
-__device__ __forceinline__ float* state_row(int slot, int hv, int row) {
-  uint32_t lane = lane_id();
-  pin(lane);
-  return parameter(&GdnParams::state) + (int64_t)slot * parameter(&GdnParams::state_stride0) +
-         ((int64_t)hv * kDV + row + (lane & 15)) * kDK + 8 * (lane >> 4);
-}
-
-// A request token after token, as in gdn_state.hip, for a wave's 16 rows from `row` on.
-__device__ __forceinline__ void token_by_token(int start, int end, int slot, int hv, int row) {
-  GdnParams p;
-  p.y = parameter(&GdnParams::y);
-  p.q = parameter(&GdnParams::q);
-  p.k = parameter(&GdnParams::k);
-  p.v = parameter(&GdnParams::v);
-  p.g = parameter(&GdnParams::g);
-  p.beta = parameter(&GdnParams::beta);
-  p.q_stride0 = parameter(&GdnParams::q_stride0);
-  p.k_stride0 = parameter(&GdnParams::k_stride0);
-  p.v_stride0 = parameter(&GdnParams::v_stride0);
-  p.hv = parameter(&GdnParams::hv);
-  p.hv_per_hk = parameter(&GdnParams::hv_per_hk);
-  uint32_t lane = lane_id();
-  pin(lane);
-  const int g = lane >> 4, hk = hv / p.hv_per_hk;
-  float* const srow = state_row(slot, hv, row);
-  row += lane & 15;
-  f32x4_t s[8];  // s[2 c + h][i]: dim 32 c + 8 g + 4 h + i
-#pragma unroll
-  for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
-  struct TokenIn {
-    u32x4_t k[4], q[4];
-    uint32_t g, beta, v;
-  };
-  auto load = [&](int64_t t, TokenIn& in) {
-    const uint16_t* k = p.k + t * p.k_stride0 + hk * kDK + 8 * g;
-    const uint16_t* q = p.q + t * p.q_stride0 + hk * kDK + 8 * g;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      in.k[c] = ld_global_b128(k + 32 * c);
-      in.q[c] = ld_global_b128(q + 32 * c);
-    }
-    in.g = p.g[t * p.hv + hv];
-    in.beta = p.beta[t * p.hv + hv];
-    in.v = p.v[t * p.v_stride0 + hv * kDV + row];
-  };
-  auto four = [](u32x4_t raw, int h) {
-    return f32x4_t{bf16_bits_to_f32(raw[2 * h] & 0xffffu), bf16_bits_to_f32(raw[2 * h] >> 16),
-                   bf16_bits_to_f32(raw[2 * h + 1] & 0xffffu), bf16_bits_to_f32(raw[2 * h + 1] >> 16)};
-  };
-  TokenIn next;
-  load(start, next);
-  for (int t = start; t < end; ++t) {
-    const TokenIn in = next;
-    load(min(t + 1, end - 1), next);
-    const float decay = bf16_bits_to_f32(in.g);
-    float dot = 0.f, y = 0.f;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const f32x4_t k = four(in.k[c >> 1], c & 1);
-      s[c] *= decay;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(s[c][i], k[i], dot);
-    }
-    const float delta = (bf16_bits_to_f32(in.v) - sum_across<32>(sum_across<16>(dot))) * bf16_bits_to_f32(in.beta);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const f32x4_t k = four(in.k[c >> 1], c & 1), q = four(in.q[c >> 1], c & 1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s[c][i] = __builtin_fmaf(k[i], delta, s[c][i]);
-        y = __builtin_fmaf(s[c][i], q[i], y);
-      }
-    }
-    y = sum_across<32>(sum_across<16>(y));
-    if (g == 0) p.y[((int64_t)t * p.hv + hv) * kDV + row] = __builtin_bit_cast(uint16_t, (__bf16)y);
-  }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
-}
-
-// Decay ratios G_t / G_i of block (r, c), transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n).  Below the
-// diagonal: token t's block up to it, whole blocks, token i's block behind it; on the diagonal: token t's quad up to
-// it and the quads between, then token by token down the columns (1 above the diagonal).
-struct Decays {
-  f32x4_t col;
-  float row;
-  template <typename Lds>
-  __device__ __forceinline__ void load(const Lds& lds, int r, int c) {
-    const int x16 = lane_id() & 15, g = lane_id() >> 4;
-    row = r == c ? lds.quad_pre[16 * r + x16] : lds.pre[16 * r + x16];
-    col = *reinterpret_cast<const f32x4_t*>(r == c ? &lds.g[16 * r + 4 * g] : &lds.suf[16 * c + 4 * g]);
-  }
-  template <typename Lds>
-  __device__ __forceinline__ f32x4_t below(const Lds& lds, int r, int c) const {
-    const float b1 = lds.block[1], b2 = lds.block[2];
-    return row * (c < 1 && r > 1 ? b1 : 1.0f) * (c < 2 && r > 2 ? b2 : 1.0f) * col;
-  }
-  template <typename Lds>
-  __device__ __forceinline__ f32x4_t diagonal(const Lds& lds, int r) const {
-    const int x16 = lane_id() & 15, g = lane_id() >> 4;
-    const float q1 = lds.quad[4 * r + 1], q2 = lds.quad[4 * r + 2];
-    const float far = row * (g < 1 && x16 >= 8 ? q1 : 1.0f) * (g < 2 && x16 >= 12 ? q2 : 1.0f);
-    f32x4_t ratio;
-    ratio[3] = (x16 >> 2) > g ? far : 1.0f;
-#pragma unroll
-    for (int i = 2; i >= 0; --i) ratio[i] = ratio[i + 1] * (4 * g + i + 1 <= x16 ? col[i + 1] : 1.0f);
-    return ratio;
-  }
-};
-// <k, q> or <k, k> of a block, transposed likewise
-__device__ __forceinline__ f32x4_t block_dots(const bf16x8_t (&columns)[4], const bf16x8_t (&rows)[4]) {
-  f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int n = 0; n < 4; ++n) d = mfma_16x16x32(columns[n], rows[n], d);
-  return d;
-}
-__device__ __forceinline__ void load_block_rows(const uint16_t (*m)[kDK], int r, bf16x8_t (&x)[4]) {
-  const int x16 = lane_id() & 15, g = lane_id() >> 4;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) x[d] = operand(&m[16 * r + x16][8 * piece(x16, 4 * d + g)]);
-}
-
-// Block (r, c) of A below the diagonal, to LDS; returns its ratios.
-template <typename Lds>
-struct BelowBlock {
-  bf16x8_t kc[4], kr[4];
-  Decays decays;
-  float beta;
-  __device__ __forceinline__ void load(const Lds& lds, int par, int tri, int r, int c) {
-    load_block_rows(lds.k[par], c, kc);
-    load_block_rows(lds.k[par], r, kr);
-    beta = lds.beta[tri][16 * r + (lane_id() & 15)];
-    decays.load(lds, r, c);
-  }
-  __device__ __forceinline__ f32x4_t store(Lds& lds, int r, int c, f32x4_t dots) const {
-    const f32x4_t ratio = decays.below(lds, r, c);
-    *reinterpret_cast<f32x4_t*>(&lds.a[16 * r + (lane_id() & 15)][16 * c + 4 * (lane_id() >> 4)]) = beta * ratio * dots;
-    return ratio;
-  }
-};
-
-// Rows of Y from its transpose: a lane has of token 16 m + x16 the state rows 4 g ..
-struct Outputs {
-  uint32_t step, lane_at;
-  int tokens;
-  char* base;
-  __device__ __forceinline__ Outputs(const GdnParams& p, int start, int end, int hv, int row)
-      : step((uint32_t)p.hv * kDV * 2u), lane_at((lane_id() & 15) * step + 8 * (lane_id() >> 4)), tokens(end - start),
-        base(reinterpret_cast<char*>(p.y + ((int64_t)start * p.hv + hv) * kDV + row)) {}
-  __device__ __forceinline__ void store(int chunk, const f32x4_t (&z)[4]) const {
-    char* to = base + (int64_t)chunk * kChunk * step;
-    const int left = tokens - chunk * kChunk;
-    auto one = [&](int m) {
-      *reinterpret_cast<u32x2_t*>(to + (lane_at + 16 * m * step)) = u32x2_t{pack_bf16x2(z[m][0], z[m][1]), pack_bf16x2(z[m][2], z[m][3])};
-    };
-    if (left >= kChunk) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) one(m);
-    } else {
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-        if (16 * m + (lane_id() & 15) < left) one(m);
-    }
-  }
 };
 
 template <bool PAIRED, typename Lds>
@@ -450,8 +133,8 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, Lds& lds, int st
   __builtin_amdgcn_s_setprio(1);  // before the chunk waves, but in slot 2, where those have the longer way
   auto a_block = [&](int par, int tri) {  // (3, 2), and the other state wave (2, 1)
     const int r = column ? 2 : 3, c = r - 1;
-    BelowBlock<Lds> x;
-    x.load(lds, par, tri, r, c);
+    BelowBlock x;
+    x.load(lds, lds.k[par], lds.beta[tri], r, c);
     x.store(lds, r, c, block_dots(x.kc, x.kr));
   };
   slot_barrier();  // K, Q of chunk 0
@@ -603,52 +286,6 @@ __device__ __forceinline__ void state_waves(const GdnParams& p, Lds& lds, int st
   for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
 }
 
-// A value from another lane of the row of 16, 1 where there is none.  DPP control C: 0x110 + n the lane n below,
-// 0x100 + n the lane n above.
-template <int C>
-__device__ __forceinline__ float row_shift(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), C, 0xf, 0xf, false));
-}
-// Lane t of every row of 16 lanes, in all of them.
-template <int T>
-__device__ __forceinline__ float row_broadcast(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + T, 0xf, 0xf, true));
-}
-// Inverse of I + A for a 16 x 16 block: lane x16 holds row x16 of the strictly lower A and, of the inverse,
-// columns 4 g .. 4 g + 3 of that row.  Row T is final when its turn comes and is taken off the rows below it.
-template <int T>
-__device__ __forceinline__ void eliminate(const float (&a)[16], f32x4_t& inv) {
-#pragma unroll
-  for (int n = 0; n < 4; ++n) inv[n] = __builtin_fmaf(-a[T], row_broadcast<T>(inv[n]), inv[n]);
-  if constexpr (T < 14) eliminate<T + 1>(a, inv);
-}
-
-__device__ __forceinline__ f32x4_t mfma_f32_block(f32x4_t a, f32x4_t b, f32x4_t c) {
-  // 16x16x16 in four steps: step i contracts over 4 g + i, which a lane's four values of a row
-  // (A operand) and four result rows of a column (B operand) are
-#pragma unroll
-  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
-  return c;
-}
-
-// Blocks (R, C) of T below the diagonal from those of A and the inverses on the diagonal:
-// T_RC = -T_RR X_R, X_R = sum over C <= k < R of A_Rk T_kC.  A block is made as the operand of the rows below it
-// and transposed, four neighbours of a row to a lane, for LDS (T_RC^T = -X_R^T T_RR^T).  Operands of that:
-template <typename Lds>
-struct Inverse {
-  const Lds& lds;
-  int x16, g;
-  __device__ __forceinline__ explicit Inverse(const Lds& l) : lds(l), x16(lane_id() & 15), g(lane_id() >> 4) {}
-  __device__ __forceinline__ f32x4_t a(int r, int k) const { return *reinterpret_cast<const f32x4_t*>(&lds.a[16 * r + x16][16 * k + 4 * g]); }
-  __device__ __forceinline__ f32x4_t minus_diag(int r) const { return -*reinterpret_cast<const f32x4_t*>(&lds.diag[r][x16][4 * g]); }
-  __device__ __forceinline__ f32x4_t diag_plain(int r) const {
-    f32x4_t d;
-#pragma unroll
-    for (int n = 0; n < 4; ++n) d[n] = lds.diag[r][4 * g + n][x16];
-    return d;
-  }
-};
-
 template <bool PAIRED, typename Lds>
 __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int start, int end, int hv,
                                             int wg_row, int w) {
@@ -706,34 +343,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
   auto decays = [&](int first, int tri) {
     const bool in = first + lane < end;
     const float gv = in ? bf16_bits_to_f32(graw) : 1.0f, bv = in ? bf16_bits_to_f32(braw) : 0.0f;
-    // products over a row of 16 lanes, or over quads (every lane shifts, then takes what is in its quad)
-    const float before1 = row_shift<0x111>(gv);
-    float pre = gv * before1, suf = gv * row_shift<0x101>(gv), quad_pre = gv * ((x16 & 3) >= 1 ? before1 : 1.0f);
-    const float quad2 = row_shift<0x112>(quad_pre);
-    quad_pre *= (x16 & 3) >= 2 ? quad2 : 1.0f;
-    pre *= row_shift<0x112>(pre);
-    suf *= row_shift<0x102>(suf);
-    pre *= row_shift<0x114>(pre);
-    suf *= row_shift<0x104>(suf);
-    pre *= row_shift<0x118>(pre);
-    suf *= row_shift<0x108>(suf);
-    suf = row_shift<0x101>(suf);  // behind the token
-    auto lane_value = [](float f, int l) {
-      return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), l));
-    };
-    const float b0 = lane_value(pre, 15), b1 = lane_value(pre, 31), b2 = lane_value(pre, 47), b3 = lane_value(pre, 63);
-    const float before = g == 0 ? 1.0f : g == 1 ? b0 : g == 2 ? b0 * b1 : b0 * b1 * b2;
-    const float behind = g == 3 ? 1.0f : g == 2 ? b3 : g == 1 ? b2 * b3 : b1 * b2 * b3;
-    lds.beta[tri][lane] = bv;
-    lds.gamma[tri][lane] = before * pre;
-    lds.tail[tri][lane] = suf * behind;
-    lds.g[lane] = gv;
-    lds.pre[lane] = pre;
-    lds.suf[lane] = suf;
-    lds.quad_pre[lane] = quad_pre;
-    if (x16 == 15) lds.block[g] = pre;
-    if ((lane & 3) == 3) lds.quad[lane >> 2] = quad_pre;
-    if (lane == 0) lds.total[tri] = b0 * b1 * b2 * b3;
+    decay_products(lds, gv, bv, lds.beta[tri], lds.gamma[tri], lds.tail[tri], lds.total[tri]);
   };
   // The ten blocks (r, c) of A and P on and below the diagonal: every wave its diagonal block and one
   // more, waves 1 and 2 two (PAIRED: the state waves have those).  Results are transposed (lane: token t = 16 r + x16, tokens i = 16 c + 4 g + n), so that a
@@ -745,17 +355,17 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
   float most = 0.f;  // largest() of P's diagonal block, every chunk
   f32x4_t inv;    // the inverse of the diagonal block: row x16, columns 4 g ..
   auto products = [&](int par, int tri) {
-    BelowBlock<Lds> b0, b1, b2;
+    BelowBlock b0, b1, b2;
     const int r1 = block_row(1), c1 = block_col(1), r2 = block_row(2), c2 = block_col(2);
-    b0.load(lds, par, tri, w, w);
-    b1.load(lds, par, tri, r1, c1);
+    b0.load(lds, lds.k[par], lds.beta[tri], w, w);
+    b1.load(lds, lds.k[par], lds.beta[tri], r1, c1);
     const f32x4_t kk0 = block_dots(b0.kc, b0.kr);
     {
       const f32x4_t ratio = b0.decays.diagonal(lds, w);
       f32x4_t a;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        a[i] = 4 * g + i < x16 ? b0.beta * ratio[i] * kk0[i] : 0.f;
+        a[i] = 4 * g + i < x16 ? -b0.beta * ratio[i] * kk0[i] : 0.f;  // negated, as eliminate() takes it
         if constexpr (!PAIRED) pp0[i] = 4 * g + i <= x16 ? ratio[i] : 0.f;
       }
       *reinterpret_cast<f32x4_t*>(&lds.a[16 * w + x16][16 * w + 4 * g]) = a;
@@ -772,7 +382,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
     // (no two branches of a lambda end in stores to different captures: those become one store to a chosen address,
     // and the captures go to scratch memory)
     if (n_blocks > 2) {
-      b2.load(lds, par, tri, r2, c2);
+      b2.load(lds, lds.k[par], lds.beta[tri], r2, c2);
       const f32x4_t kk1 = block_dots(b1.kc, b1.kr), kk2 = block_dots(b2.kc, b2.kr);
       eliminate<0>(arow, inv);
       pp2 = b2.store(lds, r2, c2, kk2);
@@ -796,47 +406,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
     if (n_blocks > 2) times_dots(2, pp2);
     most = largest(pp0, most);
   };
-  // Blocks of T below the diagonal, two waves with the first column: (1, 0) and (2, 0); (2, 1) and (3, 1); (3, 2);
-  // (3, 0).  Everything a chain needs from LDS is asked for before it starts.
-  struct Below {
-    f32x4_t first, second;
-  } below;
-  auto inverse = [&]() -> Below {
-    const Inverse<Lds> of(lds);
-    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-    if (w == 2) {
-      const f32x4_t a32 = of.a(3, 2), t2 = of.diag_plain(2), d3 = of.minus_diag(3);
-      return {mfma_f32_block(mfma_f32_block(a32, t2, zero), d3, zero), zero};
-    }
-    if (w == 1) {
-      const f32x4_t a21 = of.a(2, 1), a31 = of.a(3, 1), a32 = of.a(3, 2), t1 = of.diag_plain(1), d2 = of.minus_diag(2), d3 = of.minus_diag(3);
-      const f32x4_t x2 = mfma_f32_block(a21, t1, zero);
-      f32x4_t x3 = mfma_f32_block(a31, t1, zero);
-      const f32x4_t t21 = mfma_f32_block(d2, x2, zero);
-      const f32x4_t first = mfma_f32_block(x2, d2, zero);
-      x3 = mfma_f32_block(a32, t21, x3);
-      return {first, mfma_f32_block(x3, d3, zero)};
-    }
-    const f32x4_t a10 = of.a(1, 0), a20 = of.a(2, 0), a21 = of.a(2, 1), t0 = of.diag_plain(0), d1 = of.minus_diag(1), d2 = of.minus_diag(2);
-    if (w == 0) {
-      const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
-      f32x4_t x2 = mfma_f32_block(a20, t0, zero);
-      const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
-      const f32x4_t first = mfma_f32_block(x1, d1, zero);
-      x2 = mfma_f32_block(a21, t10, x2);
-      return {first, mfma_f32_block(x2, d2, zero)};
-    }
-    const f32x4_t a30 = of.a(3, 0), a31 = of.a(3, 1), a32 = of.a(3, 2), d3 = of.minus_diag(3);
-    const f32x4_t x1 = mfma_f32_block(a10, t0, zero);
-    f32x4_t x2 = mfma_f32_block(a20, t0, zero), x3 = mfma_f32_block(a30, t0, zero);
-    const f32x4_t t10 = mfma_f32_block(d1, x1, zero);
-    x2 = mfma_f32_block(a21, t10, x2);
-    x3 = mfma_f32_block(a31, t10, x3);
-    const f32x4_t t20 = mfma_f32_block(d2, x2, zero);
-    x3 = mfma_f32_block(a32, t20, x3);
-    if constexpr (PAIRED) return {x3, d3};  // this chain is the longest of slot 3: the last product comes in slot 1
-    else return {mfma_f32_block(x3, d3, zero), zero};
-  };
+  Below below;
   auto store_t = [&]() {
     f32x4_t first = below.first;
     if (PAIRED && w == 3) first = mfma_f32_block(first, below.second, f32x4_t{0.f, 0.f, 0.f, 0.f});
@@ -860,7 +430,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
   products(0, 0);
   slot_barrier();
   if constexpr (!PAIRED) finish_p(0);
-  below = inverse();
+  below = blocks_below<PAIRED>(lds, w);
   if (w == 2 && n_chunks > 1) decays(start + kChunk, 1);
   if constexpr (PAIRED) {
     wait_all_vm();  // V of chunk 0 is in LDS
@@ -886,7 +456,7 @@ __device__ __forceinline__ void chunk_waves(const GdnParams& p, Lds& lds, int st
     if (more) {
       if constexpr (!PAIRED) fetch_v(next);
       if constexpr (!PAIRED) finish_p(par);
-      below = inverse();
+      below = blocks_below<PAIRED>(lds, w);
     }
     if (w == 2 && two) decays(next + kChunk, tri);
     if (!PAIRED && !more) lds.p_largest[64 * w + lane] = most;

@@ -174,6 +174,16 @@ static bool prefer_chunks(const GdnArgs& a) {
   const bool pairs = a.batch <= 64 && a.batch * a.hv * 4 <= device_cus();
   return (pairs ? 9.2 + 0.9 * units : 12.8 * rounds) < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
 }
+// Room for the systems of all chunks where making those in a launch of their own pays (gdn_long.hip), 0 elsewhere.  The second
+// launch costs 3 to 5 us and saves a tenth to a quarter of a long request's chain: one request of 256, 384, 512, 4000 tokens
+// 19.7 -> 20.8, 25.7 -> 25.1, 32.0 -> 29.7, 208 -> 162 us; two of 384, 512, 1000 27.3 -> 28.0, 33.4 -> 32.9, 59.0 -> 54.1; four of 512, 1000
+// 44.3 -> 45.5, 80.0 -> 77.4; eight of 200 to 1600 148 -> 139.  A request and 32 heads have 640 KiB for every 64 tokens; a launch that
+// would need more than 2 GiB goes without.
+size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token) {
+  if (single_token || batch <= 0 || tokens < (batch == 1 ? 384 : batch <= 3 ? 448 : 560) * batch) return 0;
+  const size_t bytes = gdn_long_workspace_bytes(tokens, batch, hv);
+  return bytes <= ((size_t)2 << 30) ? bytes : 0;
+}
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 void gdn_set_rows(int v) { t_force_rows = (v == 1 || v == 2 || v == 4) ? v : 0; }
 
@@ -199,7 +209,11 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   p.single_token = a.single_token_mode ? 1 : 0;
   const int64_t heads = a.batch * a.hv;
   if (heads <= 0) return MSGL_OK;
-  if (!p.single_token && t_force_rows == 0 && prefer_chunks(a)) return launch_gdn_chunks(p, stream);
+  if (!p.single_token && t_force_rows == 0 && prefer_chunks(a)) {
+    const size_t bytes = gdn_state_workspace_bytes(a.tokens, a.batch, a.hv, false);
+    if (bytes > 0 && a.workspace != nullptr && a.workspace_bytes >= bytes) return launch_gdn_long(p, a.workspace, stream);
+    return launch_gdn_chunks(p, stream);
+  }
   // more rows per lane group (more overlap inside a wave) once there are enough workgroups
   // to fill the chip without it
   const int64_t blocks_r1 = heads * (kDV / 16);

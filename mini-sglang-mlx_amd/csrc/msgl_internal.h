@@ -187,8 +187,11 @@ struct GdnArgs {
   int64_t tokens, batch, hk, hv;
   int64_t state_stride0, q_stride0, k_stride0, v_stride0;  // elements
   int32_t single_token_mode;
+  void* workspace;  // may be null: requests of many chunks then take the one launch
+  size_t workspace_bytes;
 };
 int launch_gdn_state(const GdnArgs& a, hipStream_t stream);
+size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token);
 // benchmarking switch: state rows per 16-lane group (1, 2, 4; 0 = chosen from the problem size)
 void gdn_set_rows(int v);
 

@@ -68,6 +68,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
          _i64, _i64, _i64, _i64, _i32, _vp]),
+    "msgl_gdn_state_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
+    "msgl_gdn_state_inplace_in": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+         _i64, _i64, _i64, _i64, _i32, _vp, _sz, _vp]),
     # include/msgl_state_pool.h (recurrent-state pool)
     "msgl_copy_state_slots": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _vp]),
     # include/msgl_radix_cache.h (host-side prefix cache)
