@@ -465,7 +465,32 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
   return std::max(split_need, tile_need);
 }
 
-// `tokens`: rows that the launch stores first, where stores_in_tiles() holds; out_loc nullptr: none.
+// Whether prompts with nothing cached go through the tile kernel whose workgroups stay, which takes their keys and values from
+// the new rows and stores those on the way (see kMinFreshRounds): as many keys as rows, in one pass over them, from one round of blocks on.
+static bool prompts_stored(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_q, int64_t n_kv, int64_t head_dim,
+                           int64_t max_len_extend, bool is_cross, int64_t window) {
+  if (batch <= 0 || total_q <= 0 || total_kv != total_q || total_q > msgl::kMaxFreshRows || n_q <= 0 || n_kv <= 0 || n_q % n_kv != 0 || max_len_extend <= 0 ||
+      window < 0 || head_dim != 128 || msgl::tile_variant() != 0 || t_gangs > 0)
+    return false;
+  const int64_t group = n_q / n_kv;
+  if (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) ||
+      ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim) > 0)
+    return false;
+  const int splits = msgl::prefill_key_splits(batch, total_q, total_kv, n_kv, group, max_len_extend, window, head_dim, t_key_splits);
+  if (splits > 1 || gangs_for(batch, total_q, total_kv, n_kv, group, max_len_extend, head_dim, window, splits) > 0) return false;
+  msgl::PrefillArgs a{};
+  a.batch = batch;
+  a.total_q = total_q;
+  a.total_kv = total_kv;
+  a.n_kv = n_kv;
+  a.max_len_extend = (int32_t)max_len_extend;
+  a.is_cross = is_cross ? 1 : 0;
+  a.by_length = 1;
+  const int64_t n_qblk = (max_len_extend * group + msgl::kPrefillBlockRows - 1) / msgl::kPrefillBlockRows;
+  return msgl::prefill_by_length(a, n_qblk, true) && msgl::prefill_stay_rounds(batch, total_q, n_kv, group, n_qblk, msgl::kMinFreshRounds) > 0;
+}
+
+// `tokens`: rows that the launch stores itself, where stores_in_tiles() or prompts_stored() holds; out_loc nullptr: none.
 static int prefill_attention(const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* qo_indptr, const int32_t* kv_indptr,
                                  const int32_t* kv_indices, const int32_t* prefix_lens, void* out,
@@ -558,7 +583,8 @@ static int prefill_attention(const void* q, const void* k_cache, const void* v_c
   a.window = sliding_window_size;
   a.key_splits = 1;
   a.new_tokens = tokens;  // stored by the tile kernels alone (see stores_in_tiles())
-  a.by_length = tokens.out_loc == nullptr;
+  a.by_length = tokens.out_loc == nullptr || prompts_stored(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim,
+                                                            max_len_extend, is_cross_attention != 0, sliding_window_size);
   a.ragged_tiles = ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim);
   if (a.ragged_tiles > 0) {
     // ragged shares need room for their partials; without it the keys go in one pass
@@ -651,7 +677,9 @@ size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t 
   if (plan.share_len > 0)
     return msgl::share_workspace_bytes(plan, batch, num_kv_heads, head_dim, num_q_heads / num_kv_heads * max_len_extend);
   if (!stores_in_tiles(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend, is_cross_attention != 0,
-                       sliding_window_size))
+                       sliding_window_size) &&
+      !prompts_stored(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, max_len_extend, is_cross_attention != 0,
+                      sliding_window_size))
     return 0;
   return std::max<size_t>(16, msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim,
                                                                  max_len_extend));

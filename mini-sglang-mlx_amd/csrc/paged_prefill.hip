@@ -725,8 +725,25 @@ struct BlockList {
   int count, blank;  // blocks; whether one has no keys
 };
 
-template <bool WIDE, Order ORDER>
+// 0, 1, 2 ...: where keys come from a launch's rows, what the list of their slots is elsewhere.  (Made in the loop instead, the numbers cost
+// a branch in every M phase: 217 -> 251 us.)
+struct RowNumbers {
+  int32_t number[kMaxFreshRows];
+  constexpr RowNumbers() : number() {
+    for (int i = 0; i < kMaxFreshRows; ++i) number[i] = i;
+  }
+};
+__device__ const RowNumbers kRowNumbers;
+
+// FRESH (with kStay): every request is a prompt with nothing cached, and its rows of k and v are stored here (see
+// prompts_stored() in api.hip).  The tiles come from those rows themselves, which are the keys in order, and a block's own
+// tokens go from their tile in LDS to the pool beside the softmax of that tile: a launch in front of this one would have read
+// and written them with nothing beside it.  Holds if every row's slot is the one that its request lists for its place, which each workgroup
+// sees for itself first; where one is not, the workgroup stores all rows of its requests and reads the pool.
+// (Gains nothing where a wait for the Q rows or the slots comes behind the stores: 227 -> 230 us, with none 217.)
+template <bool WIDE, Order ORDER, bool FRESH = false>
 __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) {
+  static_assert(!FRESH || ORDER == Order::kStay);
   constexpr int D = 128, NW = 8, UPW = kUnits / NW, KSTEPS = D / 16, DT = D / 32;
   constexpr int kRows = NW * 32;
   constexpr int OROW = D + 8;
@@ -736,7 +753,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   const ClockProbe clock_probe_(p.clock_probe);
 
   const int tid = threadIdx.x;
-  if constexpr (ORDER == Order::kBatch)
+  if constexpr (ORDER == Order::kBatch || FRESH)
     if (store_rows_of_no_request<NW * 64>(p, p.nt, p.n_kv * D, tid)) return;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -769,6 +786,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   // ---- order of length: the workgroup's blocks, found by its waves side by side -----------------
   constexpr bool listed = ORDER == Order::kStay;
   int n_listed = 0;
+  bool from_rows = false;
+  if constexpr (FRESH) from_rows = uniform(rows_are_the_keys<NW * 64>(p, tid) ? 1 : 0) != 0;
   if constexpr (listed) {
     if (tid == 0) list.count = list.blank = 0;
     const LengthOrder<kRows, true> order(p);
@@ -811,6 +830,16 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       n_listed = uniform(list.count);
     }
     if (n_listed == 0) return;
+    if (FRESH && !from_rows) {
+      for (int i = 0; i < n_listed; ++i) {
+        const int start = uniform(list.block[i].q_start);
+        if (i > 0 && uniform(list.block[i - 1].q_start) == start) continue;
+        int n = 0;  // all of the request's rows, also those that have no block
+        for (int o = 0; o < p.batch; ++o)
+          if (p.qo_indptr[o] == start) n = max(n, p.qo_indptr[o + 1] - start);
+        store_request_rows<NW * 64, D>(p, start, min(n, p.nt.rows - start), uniform(list.block[i].kvh), tid);
+      }
+    }
   }
   GangPlan plan{0, 0, 0, 0};
   if (ganged) plan = gang_plan<NW * 64>(p, gang_lds, gang_xcd, gang_id, gang_member, kRows, tid);
@@ -984,11 +1013,22 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
 
   // ---- moving tiles -------------------------------------------------------------------------
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSGL_LDS_PTR(unsigned char, smem);
-  const int32_t* idx_base = p.kv_indices + kv_start;
-  const unsigned char* k_src = reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * D);
-  const unsigned char* v_src = reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * D);
-  const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
-  const uint32_t v_row_bytes = (uint32_t)p.v_stride0 * 2u;
+  const bool rows = FRESH && from_rows;
+  const uint16_t *k_base = p.k_cache, *v_base = p.v_cache;
+  const int32_t* id_base = p.kv_indices;
+  uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u, v_row_bytes = (uint32_t)p.v_stride0 * 2u;
+  if constexpr (FRESH)
+    if (rows) {
+      k_base = p.nt.k;
+      v_base = p.nt.v;
+      k_row_bytes = (uint32_t)p.nt.k_stride0 * 2u;
+      v_row_bytes = (uint32_t)p.nt.v_stride0 * 2u;
+      id_base = kRowNumbers.number;  // the launch's keys are its rows in order
+      asm volatile("" : "+s"(k_base), "+s"(v_base), "+s"(k_row_bytes), "+s"(v_row_bytes), "+s"(id_base));  // (a branch, not a choice of addresses)
+    }
+  const int32_t* idx_base = id_base + kv_start;
+  const unsigned char* k_src = reinterpret_cast<const unsigned char*>(k_base + (int64_t)kvh * D);
+  const unsigned char* v_src = reinterpret_cast<const unsigned char*>(v_base + (int64_t)kvh * D);
   const uint32_t chunk_off = (uint32_t)(lane & 15) * 16u;
   const int unit_key = w * UPW + 16 * (lane >> 4);  // + i for unit i of this wave
   auto row_offset = [&](uint32_t slot_id, uint32_t row_bytes) -> OffT {
@@ -1012,7 +1052,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       return;
     }
     const ListedBlock& l = list.block[ahead.block + 1];
-    ahead = Cursor{p.kv_indices + uniform(l.kv_start), ahead.block + 1, 0, uniform(l.n_tiles), uniform(l.k_lo), uniform(l.kv_len) - 1};
+    ahead = Cursor{id_base + uniform(l.kv_start), ahead.block + 1, 0, uniform(l.n_tiles), uniform(l.k_lo), uniform(l.kv_len) - 1};
   };
   auto ring_fetch = [&](int t) {  // tile t of this block, or of the list
     int key = k_lo + t * kBN, last = kn - 1;
@@ -1061,8 +1101,15 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   };
   // end of M phase j: everything older than this phase's own ring fetch and moves has landed,
   // among it the ring entries of tile j+5, which the next M phase turns into addresses
+  // (`stored`: this wave's stores of its own rows left behind the moves waited for and have not to be done yet)
+  bool stored = false;
   auto end_of_sends = [&](int j) {
-    wait_vm_at_most<2 * UPW + 1>();
+    if (FRESH && stored) {
+      wait_vm_at_most<2 * UPW + 1 + 2 * UPW>();
+      stored = false;
+    } else {
+      wait_vm_at_most<2 * UPW + 1>();
+    }
     ring_read(j + 5, ids);
   };
   auto slot_barrier = [&]() {
@@ -1418,6 +1465,58 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       // scores of this one are done, a V phase and four slices ahead of their use.
       bf16x8_t oa[pp::kOperandBuffers][4];
       int t = -1, at_block = 0;
+      // FRESH: the block's own rows to the pool in the V phase of its last tile.  Those among its keys (as a rule all) are in this
+      // wave's units of that tile: its own moves have landed, and the next ones over them are its own too.
+      uint32_t own_slot[UPW];
+      auto own_range = [&](int* own, int* end) {
+        *own = uniform(row_to_query(p, row0 + p.group - 1));
+        *end = uniform(row_to_query(p, min(row0 + kRows, rows_total) + p.group - 1));
+      };
+      auto slot_of = [&](int token) { return (uint32_t)p.nt.out_loc[q_start + token]; };
+      auto ask_for_slots = [&]() {
+        if (!rows) return;
+        int own, end;
+        own_range(&own, &end);
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) own_slot[i] = slot_of(min(k_lo + (n_tiles - 1) * kBN + unit_key + i, end - 1));
+      };
+      auto store_own = [&](int t) {
+        if (!rows) return;
+        int own, end;
+        own_range(&own, &end);
+        auto store = [&](int token, uint32_t slot, u32x4_t k, u32x4_t v) {
+          if (token < own || token >= end) return;
+          st_global_b128(p.nt.k_pool + (int64_t)slot * p.k_stride0 + kvh * D + 8 * (lane & 15), k);
+          st_global_b128(p.nt.v_pool + (int64_t)slot * p.v_stride0 + kvh * D + 8 * (lane & 15), v);
+        };
+        const int base = k_lo + (n_tiles - 1) * kBN;
+#pragma unroll 1
+        for (int first = own & ~(kBN - 1); first < end; first += kBN) {  // those of other tiles
+          if (first == base) continue;
+#pragma unroll
+          for (int i = 0; i < UPW; ++i) {
+            const int token = first + unit_key + i, from = q_start + min(token, end - 1);
+            store(token, slot_of(min(token, end - 1)), ld_global_b128(p.nt.k + (int64_t)from * p.nt.k_stride0 + kvh * D + 8 * (lane & 15)),
+                  ld_global_b128(p.nt.v + (int64_t)from * p.nt.v_stride0 + kvh * D + 8 * (lane & 15)));
+          }
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) {  // always as many stores, that a later wait can count them
+          const int token = base + unit_key + i;
+          const uint64_t mine = __ballot(token >= own && token < end);
+          uint64_t all;
+          const u32x4_t k = *reinterpret_cast<const u32x4_t*>(smem + k_stage_of(t) + (w * UPW + i) * kKUnit + 16 * lane);
+          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(smem + v_stage_of(t) + (w * UPW + i) * kVUnit + 16 * lane);
+          asm volatile("s_mov_b64 %0, exec\n\ts_and_b64 exec, exec, %1\n\tglobal_store_dwordx4 %2, %3, off\n\t"
+                       "global_store_dwordx4 %4, %5, off\n\ts_mov_b64 exec, %0"
+                       : "=&s"(all)
+                       : "s"(mine), "v"(p.nt.k_pool + (int64_t)own_slot[i] * p.k_stride0 + kvh * D + 8 * (lane & 15)), "v"(k),
+                         "v"(p.nt.v_pool + (int64_t)own_slot[i] * p.v_stride0 + kvh * D + 8 * (lane & 15)), "v"(v)
+                       : "memory", "scc");
+        }
+        stored = true;
+      };
       int out_row = -1;  // row of the block before this one, still in the accumulators
       if (second) slot_barrier();
       for (;;) {
@@ -1444,10 +1543,16 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
           slot_barrier();
           m_phase(++t, oa, Yes{}, Yes{});  // with its barrier
         }
+        if constexpr (FRESH) ask_for_slots();
         next_rows();
         v_phase(j, t, oa);
         slot_barrier();
         m_phase(++t, oa, Yes{}, No{});
+        if constexpr (FRESH) {  // the Q rows and the slots are there, and nobody waits for them behind the stores
+#pragma unroll
+          for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(qreg[ks]));
+          store_own(t);
+        }
         out_row = row0 + w * 32 + c32 < rows_total ? q_row : -1;
         if (++at_block == n_listed) break;
         enter(at_block);
@@ -1764,6 +1869,8 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
     else hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, false>), grid, dim3(512), 0, stream, p);
   } else {
     auto* const kernel = p.gangs > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kGang> : prefill_pingpong_kernel<false, Order::kGang>)
+                         : p.length_rounds > 0 && p.nt.out_loc != nullptr
+                             ? (wide ? prefill_pingpong_kernel<true, Order::kStay, true> : prefill_pingpong_kernel<false, Order::kStay, true>)
                          : p.length_rounds > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kStay> : prefill_pingpong_kernel<false, Order::kStay>)
                          : p.length_heads > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kLength> : prefill_pingpong_kernel<false, Order::kLength>)
                                               : (wide ? prefill_pingpong_kernel<true, Order::kBatch> : prefill_pingpong_kernel<false, Order::kBatch>);

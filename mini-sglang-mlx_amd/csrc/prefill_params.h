@@ -206,15 +206,15 @@ inline size_t prefill_ragged_workspace_bytes(int64_t batch, int64_t total_kv, in
 // 6 prompts of 771-2710 tokens, 32 / 8 heads of 128: 262 -> 247 us.)  The blocks of a
 // request no longer run side by side on one XCD; what its L2 then misses, the memory-side cache has.
 //
-// The kernel's wave holds one request per lane: at most 64.  The kv heads have to go into the XCDs evenly.
+// `fresh`: see kMinFreshRounds.  The kernel's wave holds one request per lane: at most 64.  The kv heads have to go into the XCDs evenly.
 // A launch of fewer blocks than compute units has no order.  Whole prompts of one length in many blocks
 // each are even as they are, and gain more from a request's blocks side by side (5 x 1722 tokens, 32 / 8
 // heads: 166 us against 172; below 16 blocks a request the order is the better one or equal: 11 x 463
 // tokens, 16 / 8 heads, 4 blocks: 48.7 against 42.5).
-inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
+inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk, bool fresh = false) {
   const bool even_prompts = !a.is_cross && a.total_kv == a.total_q && a.total_q == a.batch * a.max_len_extend;
   return a.by_length && a.batch <= 64 && (a.n_kv == 1 || a.n_kv == 2 || a.n_kv == 4 || a.n_kv % 8 == 0) &&
-         a.batch * a.n_kv * n_qblk > kComputeUnits && !(even_prompts && n_qblk >= 16);
+         (fresh || (a.batch * a.n_kv * n_qblk > kComputeUnits && !(even_prompts && n_qblk >= 16)));
 }
 
 // Rounds of blocks that a workgroup may stay for.  A workgroup of the head_dim 128 kernel that ends pays for the next
@@ -236,6 +236,25 @@ inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk) {
 // The list of a workgroup's blocks is in LDS, hence the other limit (of the grid's rounds); an XCD's workgroups work on
 // one kv head (the bases of the moves stay the same).
 constexpr int kMinRounds = 2, kMaxRounds = 64;
+// Prompts with nothing cached, whose rows of k and v the launch takes its keys from and stores (prompts_stored() in api.hip), go this
+// way from one round of blocks on, those of one length too.  us, the store in front and the launch as it was then against
+// this, 32 / 8 heads: 1015, 900 and 800 tokens 45.8 -> 41.8, two of 1000 36.7 -> 35.5, three 49.6 -> 40.4, four 60.0 -> 46.4, five of
+// 1722 148 -> 129, 16 of 100-300 33.1 -> 26.5, 237-3333 (11574 in all) 227 -> 217, one of 3000 86.5 -> 84.5; 64 / 8: three of 1000 80.2 ->
+// 69.0; 2000 and 1500 under a window of 500 52.3 -> 45.0.  Below one round: one of 1015 31.8 -> 33.0, two of 500 22.7 -> 23.0.
+constexpr int kMinFreshRounds = 1;
+constexpr int kMaxFreshRows = 1 << 17;  // of k and v, in a launch that takes its keys from them
+// XCDs that share a kv head's blocks, as a logarithm
+inline int prefill_log2_xcds(int64_t n_kv) { return n_kv == 1 ? 3 : n_kv == 2 ? 2 : n_kv == 4 ? 1 : 0; }
+inline int64_t prefill_length_blocks(int64_t batch, int64_t n_kv, int64_t n_qblk) {
+  const int64_t heads = n_kv >= 8 ? n_kv / 8 : 1, xcds = 1 << prefill_log2_xcds(n_kv);
+  return 8 * batch * heads * ((n_qblk + xcds - 1) / xcds);
+}
+// Rounds of a head_dim 128 launch in order of length whose workgroups stay; 0: they don't.
+inline int prefill_stay_rounds(int64_t batch, int64_t total_q, int64_t n_kv, int64_t group, int64_t n_qblk, int min_rounds = kMinRounds) {
+  const int64_t rounds = (prefill_length_blocks(batch, n_kv, n_qblk) + kComputeUnits - 1) / kComputeUnits;
+  const int64_t filled = 8 * prefill_filled_blocks(batch, total_q, group, kPrefillBlockRows);
+  return n_kv <= 8 && filled >= ((int64_t)min_rounds * kComputeUnits << prefill_log2_xcds(n_kv)) && rounds <= kMaxRounds ? (int)rounds : 0;
+}
 
 // Gang ranges, for launches with several query blocks per (request, kv head) (chunked extends on
 // long prefixes: their cost is the MFMA work, and it differs from unit to unit with the prefix).
@@ -394,24 +413,24 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     p.gang_nonce = a.gang_nonce;
     n_blocks = kComputeUnits;  // one workgroup per compute unit, 32 per XCD
   }
-  if (p.gangs == 0 && p.n_ksplit == 1 && prefill_by_length(a, n_qblk)) {
+  if (p.gangs == 0 && p.n_ksplit == 1 && prefill_by_length(a, n_qblk, p.nt.out_loc != nullptr)) {
     p.length_heads = a.n_kv >= 8 ? (int32_t)(a.n_kv / 8) : 1;
-    p.length_log2_xcds = a.n_kv == 1 ? 3 : a.n_kv == 2 ? 2 : a.n_kv == 4 ? 1 : 0;
-    const int64_t xcds = 1 << p.length_log2_xcds;
-    n_blocks = 8 * a.batch * p.length_heads * ((n_qblk + xcds - 1) / xcds);
+    p.length_log2_xcds = prefill_log2_xcds(a.n_kv);
+    n_blocks = prefill_length_blocks(a.batch, a.n_kv, n_qblk);
     if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-    const int64_t rounds = (n_blocks + kComputeUnits - 1) / kComputeUnits;
-    const int64_t filled = 8 * prefill_filled_blocks(a.batch, a.total_q, p.group, block_rows);
-    if (block_rows == kPrefillBlockRows && p.length_heads == 1 && filled >= kMinRounds * kComputeUnits * xcds && rounds <= kMaxRounds) {
-      p.length_rounds = (int32_t)rounds;
-      n_blocks = kComputeUnits;
-    }
+    if (block_rows == kPrefillBlockRows) p.length_rounds = prefill_stay_rounds(a.batch, a.total_q, a.n_kv, p.group, n_qblk, p.nt.out_loc != nullptr ? kMinFreshRounds : kMinRounds);
+    if (p.length_rounds > 0) n_blocks = kComputeUnits;
   }
   // narrow offsets: slot * row_bytes fits 32 bits and both factors fit 24 bits (one
   // full-rate 24-bit multiply per row)
   wide = (uint64_t)a.num_slots * (uint64_t)a.k_stride0 * 2u >= (1ull << 32) ||
          (uint64_t)a.num_slots * (uint64_t)a.v_stride0 * 2u >= (1ull << 32) ||
          a.num_slots >= (1 << 24) || a.k_stride0 * 2 >= (1 << 24) || a.v_stride0 * 2 >= (1 << 24);
+  if (p.nt.out_loc != nullptr && p.length_rounds > 0) {  // so do the rows of k and v, which the launch reads too
+    const NewTokens& n = a.new_tokens;
+    wide |= (uint64_t)n.rows * (uint64_t)n.k_stride0 * 2u >= (1ull << 32) || (uint64_t)n.rows * (uint64_t)n.v_stride0 * 2u >= (1ull << 32) ||
+            n.rows >= (1 << 24) || n.k_stride0 * 2 >= (1 << 24) || n.v_stride0 * 2 >= (1 << 24);
+  }
   return MSGL_OK;
 }
 

@@ -1,0 +1,76 @@
+"""Prompts with nothing cached whose rows the attention launch stores itself: output and pool are, bit for bit, those of the store and
+the attention called one after the other.  Groups whose blocks' own tokens are a tile, part of one, or several; last blocks that are
+not full; windows and cross attention; rows that belong to no request; rows whose slots are not the ones listed."""
+import numpy as np
+import pytest
+import torch
+
+from mini_sglang_amd_kernel import _lib, extend_step, paged_prefill_attention, store_kv_cache
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _one_launch(ext, n_q, n_kv, cross, window):
+    """Whether the call goes in one launch at all (some workspace is wanted then)."""
+    return _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(ext), n_q, n_kv, D, max(ext), int(cross), window) > 0
+
+
+def _check(gpu, ext, heads, window=0, cross=False, change=None, front=0, strided=False, pad=0):
+    n_q, n_kv = heads
+    g = torch.Generator(device=gpu)
+    g.manual_seed(sum(ext) + n_q)
+    total = sum(ext)
+    slots = 2 * total + 5
+    ids = torch.randperm(slots, generator=g, device=gpu)[:total].to(torch.int32)
+    out_loc = ids.clone()
+    rand = lambda *s: torch.randn(s, generator=g, device=gpu).bfloat16()  # noqa: E731
+    q = rand(total, n_q, D)
+    kv = rand(total, 2 * n_kv, D) if strided else None
+    k, v = (kv[:, :n_kv], kv[:, n_kv:]) if strided else (rand(total, n_kv, D), rand(total, n_kv, D))
+    # (`pad`: heads between a slot's rows and the next slot's; with enough of them offsets have 64 bits)
+    pools = [torch.empty((slots, n_kv + pad, D), dtype=torch.bfloat16, device=gpu)[:, :n_kv].copy_(rand(slots, n_kv, D)) for _ in range(2)]
+    starts = np.cumsum([front] + list(ext[:-1]) + [ext[-1] - front])  # with rows in front of the first request, its last one is shorter
+    ip = torch.tensor(starts, dtype=torch.int32, device=gpu)
+    prefix = torch.zeros(len(ext), dtype=torch.int32, device=gpu)
+    if change == "slot":  # a key of a request is a row of the pool that no row goes to
+        ids[total // 2] = next(s for s in range(slots) if not bool((out_loc == s).any()))
+    elif change == "outside":  # a row that goes nowhere
+        out_loc[total // 3] = -1
+    assert _one_launch(ext, n_q, n_kv, cross, window)
+    print(f"fresh {ext[:6]} heads {heads} window {window} cross {cross} {change} front {front}", flush=True)
+    want_pools = [p.clone() for p in pools]
+    store_kv_cache(*want_pools, out_loc, k, v)
+    want = paged_prefill_attention(q, *want_pools, ip, ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
+                                   is_cross_attention=cross, sliding_window_size=window)
+    got = extend_step(q, k, v, out_loc, *pools, ip, ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
+                      is_cross_attention=cross, sliding_window_size=window)
+    torch.cuda.synchronize()
+    for a, b in zip(pools, want_pools):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    lo, hi = int(starts[0]), int(starts[-1])
+    assert torch.equal(got[lo:hi].view(torch.int16), want[lo:hi].view(torch.int16))
+
+
+@pytest.mark.parametrize("heads", [(8, 8), (16, 8), (24, 8), (32, 8), (64, 8), (32, 4), (16, 2), (8, 1)])
+@pytest.mark.parametrize("ext", [[1500, 1, 1399, 63, 1300, 64, 65, 700, 3301], [2100] * 4])
+def test_as_store_and_attention(gpu, heads, ext):
+    _check(gpu, ext, heads)
+
+
+@pytest.mark.parametrize("window,cross", [(1, False), (70, False), (1024, False), (0, True), (300, True)])
+@pytest.mark.parametrize("heads", [(16, 8), (32, 8)])
+def test_masks(gpu, heads, window, cross):
+    _check(gpu, [1700, 129, 1999, 901], heads, window, cross)
+
+
+@pytest.mark.parametrize("change", [None, "slot", "outside"])
+@pytest.mark.parametrize("front", [0, 7])
+def test_rows_that_are_not_the_keys(gpu, change, front):
+    _check(gpu, [1300, 900, 64, 1100], (32, 8), change=change, front=front, strided=change is None)
+
+
+def test_wide_pool(gpu):
+    _check(gpu, [1300, 900, 64, 1100], (32, 8), pad=2500)
+    _check(gpu, [1300, 900, 64, 1100], (32, 8), pad=2500, change="slot")
