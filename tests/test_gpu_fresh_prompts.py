@@ -74,3 +74,30 @@ def test_rows_that_are_not_the_keys(gpu, change, front):
 def test_wide_pool(gpu):
     _check(gpu, [1300, 900, 64, 1100], (32, 8), pad=2500)
     _check(gpu, [1300, 900, 64, 1100], (32, 8), pad=2500, change="slot")
+
+
+@pytest.mark.parametrize("batch,length,heads", [(4, 1030, (32, 8)), (3, 2049, (16, 8)), (1, 4100, (32, 4))])
+def test_prompts_of_one_length(gpu, batch, length, heads):
+    """Their blocks go in order of length as those of others do; against attention in fp32."""
+    n_q, n_kv = heads
+    g = torch.Generator(device=gpu)
+    g.manual_seed(length)
+    rand = lambda *s: torch.randn(s, generator=g, device=gpu).bfloat16()  # noqa: E731
+    total = batch * length
+    q, k, v = rand(total, n_q, D), rand(total, n_kv, D), rand(total, n_kv, D)
+    ids = torch.randperm(total + 3, generator=g, device=gpu)[:total].to(torch.int32)
+    pools = [torch.zeros((total + 3, n_kv, D), dtype=torch.bfloat16, device=gpu) for _ in range(2)]
+    for pool, rows in zip(pools, (k, v)):
+        pool[ids.long()] = rows
+    ip = torch.arange(0, total + 1, length, dtype=torch.int32, device=gpu)
+    print(f"prompts of one length {batch} x {length} {heads}", flush=True)
+    got = paged_prefill_attention(q, *pools, ip, ip, ids, torch.zeros(batch, dtype=torch.int32, device=gpu), sm_scale=D ** -0.5, max_len_extend=length)
+    mask = torch.full((length, length), float("-inf"), device=gpu).triu(1)
+    for b in range(batch):
+        rows = slice(b * length, (b + 1) * length)
+        for h in range(n_q):
+            at = h // (n_q // n_kv)
+            p = torch.softmax(q[rows, h].float() @ k[rows, at].float().t() * D ** -0.5 + mask, dim=-1)
+            want = p @ v[rows, at].float()
+            # weights and results are bf16: 2^-8 of a value below 5, twice
+            assert (got[rows, h].float() - want).abs().max() <= 2e-2
