@@ -424,23 +424,27 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
   return plan;
 }
 
-// Measured against the segment kernel and its merge on 140 random shapes (1-256 requests of 1-60 K
+// Measured against the segment kernel and its merge on 400 random shapes (1-256 requests of 1-60 K
 // keys, 1-16 queries, both head sizes; us, segments -> shares): 46 x 4-18 keys 42.1 -> 7.3, 64 x 20-200
 // 18.9 -> 11.3, 200 x 6-99 28.5 -> 18.0, 4 x 37-1023 15.7 -> 9.1, one of 2 K 13.5 -> 10.3, 24 x 127-4095
 // at head_dim 256 35.9 -> 28.1.  Short requests gain most (a segment pays 8 us for each request
-// boundary it crosses) and up to the largest launches; where requests are long the segments' fixed
-// costs are the same for any number of bytes, while a share's last workgroup has ever more partials
-// to read and the shares' lengths vary: one request of 12 K keys 16.6 -> 19.2, 12 of 3-8 K 59 -> 71.
-// The lines lie where the two meet.
+// boundary it crosses), and nothing any more where they fill the chip several times over (107 MiB 27.3 -> 24.1, 160 39.6 ->
+// 39.5, 371 81 -> 92).
+// The segments' fixed costs are the same for any number of bytes, while the shares' lengths vary and the longest
+// decides; the larger head's segments pay more for their partials, so their line lies further out.  By MiB of keys and
+// values: head_dim 128 39 18.7 -> 14.2 (2 requests), 66 21.2 -> 17.9 (12), 97 27.3 -> 22.4 (9), 142 32.3 -> 29.0 (13), 196
+// 38.4 -> 36.3 (7), 201 39.6 -> 41.2 (92), 247 45.5 -> 51.9, 414 85 -> 106; head_dim 256 72 32.4 -> 25.6 (9), 134 40.6 ->
+// 33.0 (31), 256 60.7 -> 54.6 (63), 357 81 -> 72 (13), 415 89.7 -> 86.0 (10), 485 and more about equal.
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch;
   if (mean <= 512) return mb <= 160;
-  // few units: most of the time is the last share's, which reads all the others of a wide head group
-  if (head_dim == 256 && batch * n_kv < 12) return false;
-  if (mean <= 4096) return mb <= (head_dim == 256 ? 128 : 56);
-  return mb <= (mean <= 8192 ? 36 : 20);
+  // Few units: at head_dim 256 most of the time is the last share's, which reads all the others of a wide head group (2
+  // requests of 10 K, 2 kv heads: 23.4 -> 31.2); at 128 a request's 16 shares leave most of the chip idle and get long
+  // (one request, 8 kv heads: 8.7 K keys 16.4 -> 15.2, 26.5 K 26.7 -> 28.1)
+  if (batch * n_kv < 12 && (head_dim == 256 || mean > 12288)) return false;
+  return mb <= (head_dim == 256 ? 448 : 208);
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {
