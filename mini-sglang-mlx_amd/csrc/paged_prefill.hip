@@ -1508,8 +1508,10 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
           uint64_t all;
           const u32x4_t k = *reinterpret_cast<const u32x4_t*>(smem + k_stage_of(t) + (w * UPW + i) * kKUnit + 16 * lane);
           const u32x4_t v = *reinterpret_cast<const u32x4_t*>(smem + v_stage_of(t) + (w * UPW + i) * kVUnit + 16 * lane);
+          // (the wait states at its end are those that a store wants before the vector unit writes its data's registers again:
+          // the compiler, which sees to them elsewhere, does not look into the statement)
           asm volatile("s_mov_b64 %0, exec\n\ts_and_b64 exec, exec, %1\n\tglobal_store_dwordx4 %2, %3, off\n\t"
-                       "global_store_dwordx4 %4, %5, off\n\ts_mov_b64 exec, %0"
+                       "global_store_dwordx4 %4, %5, off\n\ts_mov_b64 exec, %0\n\ts_nop 1"
                        : "=&s"(all)
                        : "s"(mine), "v"(p.nt.k_pool + (int64_t)own_slot[i] * p.k_stride0 + kvh * D + 8 * (lane & 15)), "v"(k),
                          "v"(p.nt.v_pool + (int64_t)own_slot[i] * p.v_stride0 + kvh * D + 8 * (lane & 15)), "v"(v)
