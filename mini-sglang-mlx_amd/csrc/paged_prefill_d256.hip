@@ -27,6 +27,9 @@
 // one wave of 32 rows per SIMD issued 400 instructions per 32 keys at 5 cycles each (2380 cycles), two of 16 rows
 // read K and V twice as often from LDS (2050).  4 requests of 512-1972 tokens on prefixes up to 8 K, 24 / 4
 // heads: 837 us with the first, 775 with the second, 717 so.
+// Beside its steps a block pays for its start: with Q by way of LDS, each row once, and no products for nothing in the
+// first step 8 K cycles less than before: 23 prompts of 129-1833 tokens, 16 / 4 heads, 434 -> 397 us, 60 of up to 400
+// 139 -> 125, 30 x 10-400 on up to 500 cached, 24 / 4, 150 -> 135, 9 x 700-2329 under a window of 300 196 -> 175.
 //
 // Algorithmic flops: 4 * D per visible (query, key) pair and q head (QK^T + PV).
 #include <type_traits>
@@ -159,23 +162,13 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // a half past the end reads clamped keys and is fully masked
   const int n_steps = (k_hi - k_lo + kStep - 1) / kStep;
 
-  // ---- this lane's row: Q operand, visibility bounds ------------------------------------
-  bf16x8_t qreg[kKSteps];
+  // ---- this lane's row: visibility bounds -----------------------------------------------
   int row_lo, row_hi;
   int w_lo_max, w_hi_min;
   {
     const int row = row0 + group_row + c32;
     const bool valid = row < rows_total;
-    const int qi = valid ? row / p.group : 0;
-    const int hh = valid ? row - qi * p.group : 0;
-    const int64_t off = ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * kD;
-#pragma unroll
-    for (int ks = 0; ks < kKSteps; ++ks) {
-      u32x4_t raw = {0u, 0u, 0u, 0u};
-      if (valid) raw = ld_global_b128(p.q + off + ks * 16 + h * 8);
-      qreg[ks] = as_bf16x8(raw);
-    }
-    const int qpos = prefix + qi;
+    const int qpos = prefix + (valid ? row_to_query(p, row) : 0);
     row_lo = (p.window > 0) ? qpos - p.window + 1 : 0;
     // k_hi - 1 only binds under a key split: the pipeline settles one step past its share
     row_hi = min(p.is_cross ? kn - 1 : min(qpos, kn - 1), k_hi - 1);
@@ -199,6 +192,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // ---- moving a stage: wave w owns units 2w, 2w+1; in a unit, lane l fetches 16-byte chunk
   // l % 32 of key (unit + 16 (l / 32)) ----------------------------------------------------
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSGL_LDS_PTR(unsigned char, smem);
+  kvh = __builtin_amdgcn_readfirstlane(kvh);
   const unsigned char* k_src = reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * kD);
   const unsigned char* v_src = reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * kD);
   const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
@@ -252,6 +246,23 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   const uint32_t v_lane = (uint32_t)(4 * h + ((lane & 15) >> 2)) * kVUnit + (uint32_t)f * 256u +
                           (uint32_t)((lane >> 4) & 1) * 32u + (uint32_t)(lane & 3) * 8u;
   const unsigned char* const k_smem = smem + k_lane;
+  // The block's Q rows, in front of its first V, in the V stages: 32 rows lie like 32 keys of K.  (Every wave its rows from
+  // memory into registers is 32 bytes each of 32 rows a load, and every row twice: 6 K cycles a block.)  Rows past the
+  // request's last: the last again, never stored.
+  auto move_q = [&] {
+    const int qi0 = __builtin_amdgcn_readfirstlane(row_to_query(p, row0)), at = __builtin_amdgcn_readfirstlane(q_start) + qi0;
+    const uint16_t* const base = p.q + ((int64_t)at * p.n_q + kvh * p.group) * kD;
+#pragma unroll
+    for (int j = 0; j < 2 * kGroups; ++j) {
+      const int unit = 2 * kGroups * w + j;
+      const int row = min(row0 + 32 * (unit >> 4) + (unit & 15) + 16 * h, rows_total - 1);
+      const int qi = row_to_query(p, row);
+      lds_direct_b128(lds0 + kVBase + (uint32_t)unit * kKUnit, base, (uint32_t)((qi - qi0) * p.n_q + row - qi * p.group) * (kD * 2u) + chunk_off);
+    }
+  };
+  auto q_operand = [&](int kstep) {
+    return as_bf16x8(*reinterpret_cast<const u32x4_t*>(k_smem + kVBase + (w % kGroups) * kKStage + kstep * 32));
+  };
   const unsigned char* const v_smem = smem + kVBase + v_lane;
 
   // ---- the pieces of one step -------------------------------------------------------------
@@ -323,24 +334,29 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // other wave's, whose P comes from LDS.  Between slices 5 and 6 a barrier: every wave has its copy of the other's
   // P of step i-1, and P of step i goes over it.  Scheduling barriers separate the slices: inside one
   // the compiler interleaves freely, across them nothing moves.
-  auto step = [&](int i, f32x16_t& cur, f32x16_t& nxt, bool mask_nxt, int nxt_base, const bf16x8_t (&p_prev)[2],
+  // Of a block's first step (FIRST) there is no P V.
+  bf16x8_t qreg[kKSteps];
+  auto step = [&](auto first, int i, f32x16_t& cur, f32x16_t& nxt, bool mask_nxt, int nxt_base, const bf16x8_t (&p_prev)[2],
                   bf16x8_t (&p_cur)[2], const uint32_t (&vs)[2][kUPW]) {
+    constexpr bool FIRST = decltype(first)::value;
     bf16x8_t kq[2][2], vq[2][2], p_other[2];
-    const int k_half = 2 * i + 2 + f, v_own = i == 0 ? f : 2 * i - 2 + f, v_other = i == 0 ? 1 - f : 2 * i - 1 - f;
+    const int k_half = 2 * i + 2 + f, v_own = 2 * i - 2 + f, v_other = 2 * i - 1 - f;
     auto request = [&](int s) {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         kq[s & 1][e] = k_operand(k_half, 2 * s + e);
-        vq[s & 1][e] = v_operand(s < 4 ? v_own : v_other, (s >> 1) & 1, 2 * (s & 1) + e);
+        if constexpr (!FIRST) vq[s & 1][e] = v_operand(s < 4 ? v_own : v_other, (s >> 1) & 1, 2 * (s & 1) + e);
       }
     };
     const float m_other = *other_max;
     request(0);
+    if constexpr (!FIRST) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) p_other[u] = as_bf16x8(other_p[64 * u]);
-    if (__any(alpha != 1.0f)) {  // rare: some row's lazy max moved in the previous step
+      for (int u = 0; u < 2; ++u) p_other[u] = as_bf16x8(other_p[64 * u]);
+      if (__any(alpha != 1.0f)) {  // rare: some row's lazy max moved in the previous step
 #pragma unroll
-      for (int dt = 0; dt < kDT; ++dt) oacc[dt] *= alpha;
+        for (int dt = 0; dt < kDT; ++dt) oacc[dt] *= alpha;
+      }
     }
     settle(m_other);
     float psum = 0.f;
@@ -364,8 +380,8 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         nxt = mfma_32x32x16(kq[s & 1][e], qreg[2 * s + e], (s == 0 && e == 0) ? zero16 : nxt);
-        const int dt = 2 * (s & 1) + e;
-        oacc[dt] = mfma_32x32x16(vq[s & 1][e], s < 4 ? p_prev[s >> 1] : p_other[(s >> 1) & 1], oacc[dt]);
+        [[maybe_unused]] const int dt = 2 * (s & 1) + e;
+        if constexpr (!FIRST) oacc[dt] = mfma_32x32x16(vq[s & 1][e], s < 4 ? p_prev[s >> 1] : p_other[(s >> 1) & 1], oacc[dt]);
       }
       if (s < 4) {
 #pragma unroll
@@ -407,14 +423,15 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     return general_scale || (base < w_lo_max) || (base + 31 > w_hi_min);
   };
   if (n_steps > 0) {
-    // ---- prologue: K of halves 0..3 and V of halves 0, 1 leave and are waited for.  K of half x lives in
-    // K stage x % 4, V of half x in V stage x % 4.
+    // ---- prologue: the Q rows and K of halves 0..3 leave and are waited for.  K of half x lives in K stage x % 4, V of
+    // half x in V stage x % 4.
     u32x2_t sl[2], first_slots[4];
 #pragma unroll
     for (int x = 0; x < 4; ++x) slot_load(k_lo + x * kHalf, first_slots[x]);
 #pragma unroll
     for (int x = 0; x < 2; ++x) slot_load(k_lo + (4 + x) * kHalf, sl[x]);  // for the K moves of step 0
-    // one round trip for all six (the Q rows requested above arrive with them)
+    move_q();
+    // one round trip for all six slot ids
     asm volatile("s_waitcnt vmcnt(0)"
                  : "+v"(first_slots[0]), "+v"(first_slots[1]), "+v"(first_slots[2]), "+v"(first_slots[3]),
                    "+v"(sl[0]), "+v"(sl[1])
@@ -426,28 +443,24 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       for (int n = 0; n < kUPW; ++n) {
         v_slot[x >> 1][x & 1][n] = first_slots[x][n];
         move_k(x, n, first_slots[x][n]);
-        if (x < 2) move_v(x, n, first_slots[x][n]);
       }
     }
     wait_all_vm();
-#pragma unroll
-    for (int u = 0; u < 2; ++u) my_p[64 * u] = u32x4_t{0u, 0u, 0u, 0u};  // P of "step -1"
     __syncthreads();
 
     f32x16_t sa = zero16, sb;
     bf16x8_t pa[2], pb[2];
 #pragma unroll
-    for (int kstep = 0; kstep < kKSteps; ++kstep) sa = mfma_32x32x16(k_operand(f, kstep), qreg[kstep], sa);
+    for (int kstep = 0; kstep < kKSteps; ++kstep) qreg[kstep] = q_operand(kstep);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) pb[u] = as_bf16x8(u32x4_t{0u, 0u, 0u, 0u});
+    for (int kstep = 0; kstep < kKSteps; ++kstep) sa = mfma_32x32x16(k_operand(f, kstep), qreg[kstep], sa);
     reach(sa, needs_mask(k_lo + f * kHalf), k_lo + f * kHalf);
-    // Step 0 refills K stages 0 and 1 (every later step refills stages whose readers passed the barrier at the
-    // end of the step before): no wave may start those moves while another still reads them.
+    // Step 0 refills K stages 0 and 1 and the V stages that hold Q (every later step refills stages whose readers passed the
+    // barrier at the end of the step before): no wave may start those moves while another still reads them.
     __syncthreads();
-    // Step i reads K of halves 2i+2, 2i+3 and V of halves 2i-2, 2i-1 (step 0: those of 0 and 1, which are in LDS
-    // already and come once more, times a P of zero); it fills the K stages of halves 2i, 2i+1 with 2i+4, 2i+5 and
-    // the V stages of halves 2i-4, 2i-3 with 2i, 2i+1, all in its first half, to be there at its end.
-    auto one_step = [&](int i, f32x16_t& cur, f32x16_t& nxt, const bf16x8_t (&p_prev)[2], bf16x8_t (&p_cur)[2],
+    // Step i reads K of halves 2i+2, 2i+3 and V of halves 2i-2, 2i-1; it fills the K stages of halves 2i, 2i+1 with
+    // 2i+4, 2i+5 and the V stages of halves 2i-4, 2i-3 with 2i, 2i+1, all in its first half, to be there at its end.
+    auto one_step = [&](auto first, int i, f32x16_t& cur, f32x16_t& nxt, const bf16x8_t (&p_prev)[2], bf16x8_t (&p_cur)[2],
                         uint32_t (&vs)[2][kUPW]) {
 #pragma unroll
       for (int x = 0; x < 2; ++x)
@@ -456,7 +469,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
 #pragma unroll
       for (int x = 0; x < 2; ++x) slot_load(k_lo + (2 * i + 6 + x) * kHalf, sl[x]);
       const int base = k_lo + (i + 1) * kStep + f * kHalf;
-      step(i, cur, nxt, needs_mask(base), base, p_prev, p_cur, vs);
+      step(first, i, cur, nxt, needs_mask(base), base, p_prev, p_cur, vs);
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
@@ -464,10 +477,11 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       asm volatile("s_waitcnt vmcnt(0)" : "+v"(sl[0]), "+v"(sl[1]) : : "memory");
       __syncthreads();
     };
-    for (int i = 0; i < n_steps; i += 2) {
-      one_step(i, sa, sb, pb, pa, v_slot[0]);
+    one_step(std::true_type{}, 0, sa, sb, pb, pa, v_slot[0]);
+    for (int i = 1; i < n_steps; i += 2) {
+      one_step(std::false_type{}, i, sb, sa, pa, pb, v_slot[1]);
       if (i + 1 == n_steps) break;
-      one_step(i + 1, sb, sa, pa, pb, v_slot[1]);
+      one_step(std::false_type{}, i + 1, sa, sb, pb, pa, v_slot[0]);
     }
     // the last step's P V is still owed
     if (__any(alpha != 1.0f)) {
