@@ -487,7 +487,8 @@ static bool prompts_stored(int64_t batch, int64_t total_q, int64_t total_kv, int
   a.is_cross = is_cross ? 1 : 0;
   a.by_length = 1;
   const int64_t n_qblk = (max_len_extend * group + msgl::kPrefillBlockRows - 1) / msgl::kPrefillBlockRows;
-  return msgl::prefill_by_length(a, n_qblk, true) && msgl::prefill_stay_rounds(batch, total_q, n_kv, group, n_qblk, msgl::kMinFreshRounds) > 0;
+  return msgl::prefill_by_length(a, n_qblk, true) && msgl::prefill_stay_rounds(batch, total_q, n_kv, group, n_qblk, msgl::kPrefillBlockRows,
+                                   2 * msgl::kMinFreshRounds) > 0;
 }
 
 // `tokens`: rows that the launch stores itself, where stores_in_tiles() or prompts_stored() holds; out_loc nullptr: none.

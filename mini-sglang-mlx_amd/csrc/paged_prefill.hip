@@ -715,16 +715,6 @@ __device__ __forceinline__ void mask_keys(f32x16_t (&s)[2], int bound) {
   quad(std::integral_constant<int, 7>{});
 }
 
-// A workgroup's blocks of a launch in order of length
-struct ListedBlock {
-  int kvh, qblk, q_start, q_len, kv_start, kv_len, prefix;
-  int k_lo, k_hi, n_tiles;  // keys that some row of the block sees, from a whole tile on
-};
-struct BlockList {
-  ListedBlock block[kMaxRounds];
-  int count, blank;  // blocks; whether one has no keys
-};
-
 // 0, 1, 2 ...: where keys come from a launch's rows, what the list of their slots is elsewhere.  (Made in the loop instead, the numbers cost
 // a branch in every M phase: 217 -> 251 us.)
 struct RowNumbers {
@@ -770,65 +760,17 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   const int gang_id = ganged ? (int)(blockIdx.x >> 3) / p.n_qblk : 0;
   const int gang_member = ganged ? (int)(blockIdx.x >> 3) % p.n_qblk : 0;
   // keys that some row of a block sees
-  auto visible = [&](int prefix, int kn, int row0, int rows_total, int* lo, int* hi) {
-    const int qi_lo = row0 / p.group;
-    const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;
-    *hi = p.is_cross ? kn : min(kn, prefix + qi_hi + 1);
-    *lo = (p.window > 0) ? max(0, prefix + qi_lo - p.window + 1) : 0;
-    *lo &= ~(kBN - 1);
-    if (*hi < *lo) *hi = *lo;
-  };
   auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
   auto row_of = [&](int start, int head, int row, int total) {  // rows past the request's last: its first, never stored
     const int qi = row < total ? row_to_query(p, row) : 0;
     return (start + qi) * p.n_q + head * p.group + (row < total ? row - qi * p.group : 0);
   };
-  // ---- order of length: the workgroup's blocks, found by its waves side by side -----------------
   constexpr bool listed = ORDER == Order::kStay;
   int n_listed = 0;
   bool from_rows = false;
   if constexpr (FRESH) from_rows = uniform(rows_are_the_keys<NW * 64>(p, tid) ? 1 : 0) != 0;
   if constexpr (listed) {
-    if (tid == 0) list.count = list.blank = 0;
-    const LengthOrder<kRows, true> order(p);
-    const int r = (int)(blockIdx.x >> 3), rounds = p.length_rounds;
-    __syncthreads();
-    for (int i = w; i < rounds; i += NW) {
-      constexpr int kPerXcd = kComputeUnits / 8;
-      const int seq = i * kPerXcd + ((i & 1) ? kPerXcd - 1 - r : r);
-      const LengthBlock x = order.find(seq);
-      if (!x.ok) break;
-      ListedBlock l{x.kvh, x.qblk, x.q_start, x.q_len, x.kv_start, x.kv_len, x.prefix, 0, 0, 0};
-      visible(l.prefix, l.kv_len, l.qblk * kRows, l.q_len * p.group, &l.k_lo, &l.k_hi);
-      l.n_tiles = (l.k_hi - l.k_lo + kBN - 1) / kBN;
-      if (lane == 0) {
-        list.block[i] = l;
-        atomicMax(&list.count, i + 1);
-        if (l.n_tiles == 0) list.blank = 1;
-      }
-    }
-    __syncthreads();
-    n_listed = uniform(list.count);
-    if (uniform(list.blank) != 0) {  // rows without keys are zero; the list goes on without their blocks
-      for (int i = 0; i < n_listed; ++i) {
-        const ListedBlock& l = list.block[i];
-        const int row = l.qblk * kRows + tid / 2, total = l.q_len * p.group;
-        if (l.n_tiles == 0 && row < total) {
-          uint16_t* dst = p.out + (int64_t)row_of(l.q_start, l.kvh, row, total) * D + 64 * (tid & 1);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) st_global_b128(dst + 8 * e, u32x4_t{0u, 0u, 0u, 0u});
-        }
-      }
-      __syncthreads();
-      if (tid == 0) {
-        int n = 0;
-        for (int i = 0; i < n_listed; ++i)
-          if (list.block[i].n_tiles > 0) list.block[n++] = list.block[i];
-        list.count = n;
-      }
-      __syncthreads();
-      n_listed = uniform(list.count);
-    }
+    n_listed = list_blocks<NW * 64, D, kRows, kBN>(p, list, tid);
     if (n_listed == 0) return;
     if (FRESH && !from_rows) {
       for (int i = 0; i < n_listed; ++i) {
@@ -956,7 +898,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
 
   bool idle = __builtin_amdgcn_readfirstlane(row0 + w * 32 >= rows_total ? 1 : 0) != 0;
   if constexpr (!listed) {
-    visible(prefix, kn, row0, rows_total, &k_lo, &k_hi);
+    block_keys<kRows, kBN>(p, prefix, kn, row0, rows_total, &k_lo, &k_hi);
     if (ganged) {  // tiles [piece_a, piece_b) of the unit, as far as this query block sees them
       k_lo = min(k_lo + piece_a * kBN, k_hi);
       k_hi = min(k_hi, piece_b * kBN);

@@ -30,6 +30,10 @@
 // Beside its steps a block pays for its start: with Q by way of LDS, each row once, and no products for nothing in the
 // first step 8 K cycles less than before: 23 prompts of 129-1833 tokens, 16 / 4 heads, 434 -> 397 us, 60 of up to 400
 // 139 -> 125, 30 x 10-400 on up to 500 cached, 24 / 4, 150 -> 135, 9 x 700-2329 under a window of 300 196 -> 175.
+// Where the workgroup stays (STAY, see kMinHalfRounds256) the next block's slot ids are under way while the last one's P V
+// is added, its K and Q while the result is stored, straight from the registers: 12 K cycles from step to step.  There
+// are no registers to go on from block to block as in the head_dim 128 kernel (256 in the steps, 22 of a lane's constants
+// spilled around them), nor for steps that leave the scores of a block's last step out (105 spilled in them).
 //
 // Algorithmic flops: 4 * D per visible (query, key) pair and q head (QK^T + PV).
 #include <type_traits>
@@ -61,7 +65,8 @@ constexpr int kStageTotal = kMaxBase + kNW * 256;         // 154624
 constexpr int kKSteps = kD / 16;              // k-steps of QK^T
 constexpr int kDT = kD / 2 / 32;              // 32-dim tiles of a wave's half of O^T
 
-template <bool WIDE>
+// STAY: the workgroup takes the blocks of its list (see kMaxRounds), one after the other.
+template <bool WIDE, bool STAY>
 __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams p) {
   constexpr int kRows = kPrefillBlockRows256;
   static_assert(kRows == kGroups * 32, "one 32-row tile per two waves");
@@ -70,10 +75,13 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   constexpr int SMEM_BYTES = kStageTotal > O_BYTES ? kStageTotal : O_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM_BYTES];
   using OffT = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+  __shared__ BlockList list;
   const ClockProbe clock_probe_(p.clock_probe);
 
   const int tid = threadIdx.x;
-  if (store_rows_of_no_request<kNW * 64>(p, p.nt, p.n_kv * kD, tid)) return;
+  if constexpr (!STAY)
+    if (store_rows_of_no_request<kNW * 64>(p, p.nt, p.n_kv * kD, tid)) return;
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int h = lane >> 5;
@@ -86,12 +94,17 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // run heaviest first, requests in order of decreasing kv length (each block ranks the requests
   // itself from kv_indptr)
   // With ragged shares: block -> (unit = (request, share), kv head), see prefill_ragged_tiles().
-  int b, kvh, split = 0, qblk, n_shares = 1;
+  int b, kvh, split = 0, qblk, n_shares = 1, n_listed = 1;
   bool to_partial = p.n_ksplit > 1;  // leave a partial for the merge kernel, not the result
   int64_t part_at = 0;               // partial row of the block's row 0 (ragged shares)
   LengthBlock by_length{};
   RequestPlace place{};
-  if (p.ragged_tiles > 0) {
+  if constexpr (STAY) {
+    n_listed = list_blocks<kNW * 64, kD, kRows, kHalf>(p, list, tid);
+    if (n_listed == 0) return;
+    kvh = uniform(list.block[0].kvh);  // of all the XCD's blocks
+    b = qblk = 0;                      // the list has them
+  } else if (p.ragged_tiles > 0) {
     kvh = (int)(blockIdx.x % (unsigned)p.n_kv);
     const int u = (int)(blockIdx.x / (unsigned)p.n_kv);
     place = place_of<kNW * 64>(p, u, tid);
@@ -125,48 +138,59 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     b = place.b;
   }
 
-  int q_start, q_len, kv_start, kn, prefix;
-  if (by_length.ok) {  // they came with the block
+  int q_start, q_len, kv_start, kn, prefix, k_lo, k_hi;
+  auto take_listed = [&](int i) {
+    const ListedBlock& l = list.block[i];
+    q_start = uniform(l.q_start);
+    q_len = uniform(l.q_len);
+    kv_start = uniform(l.kv_start);
+    kn = uniform(l.kv_len);
+    prefix = uniform(l.prefix);
+    qblk = uniform(l.qblk);
+    k_lo = uniform(l.k_lo);
+    k_hi = uniform(l.k_hi);
+  };
+  if constexpr (STAY) {
+    take_listed(0);
+  } else if (by_length.ok) {  // they came with the block
     q_start = by_length.q_start;
     q_len = by_length.q_len;
     kv_start = by_length.kv_start;
     kn = by_length.kv_len;
     prefix = by_length.prefix;
   } else {
-    q_start = __builtin_amdgcn_readfirstlane(place.q_start);
-    q_len = min(__builtin_amdgcn_readfirstlane(place.q_len), p.max_len_extend);
-    kv_start = __builtin_amdgcn_readfirstlane(place.kv_start);
-    kn = __builtin_amdgcn_readfirstlane(place.kv_len);
-    prefix = __builtin_amdgcn_readfirstlane(place.prefix);
+    q_start = uniform(place.q_start);
+    q_len = min(uniform(place.q_len), p.max_len_extend);
+    kv_start = uniform(place.kv_start);
+    kn = uniform(place.kv_len);
+    prefix = uniform(place.prefix);
   }
-  const int rows_total = q_len * p.group;
-  const int row0 = qblk * kRows;
-  if (row0 >= rows_total) return;
-  if (p.nt.out_loc != nullptr) store_request_rows<kNW * 64, kD>(p, q_start, __builtin_amdgcn_readfirstlane(place.q_len), kvh, tid);
-
-  const int qi_lo = row0 / p.group;
-  const int qi_hi = min(rows_total - 1, row0 + kRows - 1) / p.group;
-  int k_hi = p.is_cross ? kn : min(kn, prefix + qi_hi + 1);
-  int k_lo = (p.window > 0) ? max(0, prefix + qi_lo - p.window + 1) : 0;
-  k_lo &= ~(kHalf - 1);
-  if (k_hi < k_lo) k_hi = k_lo;
-  // key split `split` of n_ksplit: a whole number of steps each, the last takes the ragged end;
-  // shares past the end are empty (they still leave a "nothing seen" partial)
-  if (p.ragged_tiles > 0 || p.n_ksplit > 1) {
-    const int shares = p.ragged_tiles > 0 ? n_shares : p.n_ksplit;  // ragged: the request's own count
-    const int all_steps = (k_hi - k_lo + kStep - 1) / kStep;
-    const int share = (all_steps + shares - 1) / shares * kStep;
-    k_lo = min(k_lo + split * share, k_hi);
-    k_hi = min(k_hi, k_lo + share);
+  int rows_total = q_len * p.group;
+  int row0 = qblk * kRows;
+  if constexpr (!STAY) {
+    if (row0 >= rows_total) return;
+    if (p.nt.out_loc != nullptr) store_request_rows<kNW * 64, kD>(p, q_start, uniform(place.q_len), kvh, tid);
+    block_keys<kRows, kHalf>(p, prefix, kn, row0, rows_total, &k_lo, &k_hi);
+    // key split `split` of n_ksplit: a whole number of steps each, the last takes the ragged end;
+    // shares past the end are empty (they still leave a "nothing seen" partial)
+    if (p.ragged_tiles > 0 || p.n_ksplit > 1) {
+      const int shares = p.ragged_tiles > 0 ? n_shares : p.n_ksplit;  // ragged: the request's own count
+      const int all_steps = (k_hi - k_lo + kStep - 1) / kStep;
+      const int share = (all_steps + shares - 1) / shares * kStep;
+      k_lo = min(k_lo + split * share, k_hi);
+      k_hi = min(k_hi, k_lo + share);
+    }
   }
   // a half past the end reads clamped keys and is fully masked
-  const int n_steps = (k_hi - k_lo + kStep - 1) / kStep;
+  int n_steps = (k_hi - k_lo + kStep - 1) / kStep;
 
   // ---- this lane's row: visibility bounds -----------------------------------------------
   int row_lo, row_hi;
   int w_lo_max, w_hi_min;
-  {
-    const int row = row0 + group_row + c32;
+  auto row_bounds = [&] {
+    int lane_row = c32;  // anew, see move_q()
+    asm volatile("" : "+v"(lane_row));
+    const int row = row0 + group_row + lane_row;
     const bool valid = row < rows_total;
     const int qpos = prefix + (valid ? row_to_query(p, row) : 0);
     row_lo = (p.window > 0) ? qpos - p.window + 1 : 0;
@@ -178,21 +202,26 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       row_lo = 1;
       row_hi = 0;
     }
-  }
-  w_lo_max = wave_max(w_lo_max);
-  w_hi_min = wave_min(w_hi_min);
+    w_lo_max = wave_max(w_lo_max);
+    w_hi_min = wave_min(w_hi_min);
+  };
 
   f32x16_t oacc[kDT];
+  float m_run, l_run;
+  auto reset = [&] {
 #pragma unroll
-  for (int dt = 0; dt < kDT; ++dt)
+    for (int dt = 0; dt < kDT; ++dt)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
-  float m_run = kNegInf, l_run = 0.f;
+      for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+    m_run = kNegInf;
+    l_run = 0.f;
+  };
+  reset();
 
   // ---- moving a stage: wave w owns units 2w, 2w+1; in a unit, lane l fetches 16-byte chunk
   // l % 32 of key (unit + 16 (l / 32)) ----------------------------------------------------
   const uint32_t lds0 = (uint32_t)(uintptr_t)MSGL_LDS_PTR(unsigned char, smem);
-  kvh = __builtin_amdgcn_readfirstlane(kvh);
+  kvh = uniform(kvh);
   const unsigned char* k_src = reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * kD);
   const unsigned char* v_src = reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * kD);
   const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
@@ -204,7 +233,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // caller's next wait, which names the result registers, makes them valid.  One 8-byte
   // load when the half lies inside the request, element-wise clamped loads on its last,
   // partial half.
-  const int32_t* idx_ptr = p.kv_indices + kv_start;
+  const int32_t* idx_ptr;
   const int lane_key = w * kUPW + 16 * (lane >> 5);
   auto slot_load = [&](int base, u32x2_t& sl) {
     const int first = base + lane_key;
@@ -250,14 +279,18 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   // memory into registers is 32 bytes each of 32 rows a load, and every row twice: 6 K cycles a block.)  Rows past the
   // request's last: the last again, never stored.
   auto move_q = [&] {
-    const int qi0 = __builtin_amdgcn_readfirstlane(row_to_query(p, row0)), at = __builtin_amdgcn_readfirstlane(q_start) + qi0;
-    const uint16_t* const base = p.q + ((int64_t)at * p.n_q + kvh * p.group) * kD;
+    // the lane's and the wave's numbers are taken anew: what follows from them alone would else be kept through the
+    // steps, in registers that those need
+    int half_row = h, chunk = (int)chunk_off, wave = w;
+    asm volatile("" : "+v"(half_row), "+v"(chunk), "+s"(wave));
+    const int qi0 = row_to_query(p, row0);
+    const uint16_t* const base = p.q + ((int64_t)(q_start + qi0) * p.n_q + kvh * p.group) * kD;
 #pragma unroll
     for (int j = 0; j < 2 * kGroups; ++j) {
-      const int unit = 2 * kGroups * w + j;
-      const int row = min(row0 + 32 * (unit >> 4) + (unit & 15) + 16 * h, rows_total - 1);
+      const int unit = 2 * kGroups * wave + j;
+      const int row = min(row0 + 32 * (unit >> 4) + (unit & 15) + 16 * half_row, rows_total - 1);
       const int qi = row_to_query(p, row);
-      lds_direct_b128(lds0 + kVBase + (uint32_t)unit * kKUnit, base, (uint32_t)((qi - qi0) * p.n_q + row - qi * p.group) * (kD * 2u) + chunk_off);
+      lds_direct_b128(lds0 + kVBase + (uint32_t)unit * kKUnit, base, (uint32_t)((qi - qi0) * p.n_q + row - qi * p.group) * (kD * 2u) + chunk);
     }
   };
   auto q_operand = [&](int kstep) {
@@ -422,32 +455,41 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   auto needs_mask = [&](int base) {  // some row of this wave sees only part of keys base .. base+31
     return general_scale || (base < w_lo_max) || (base + 31 > w_hi_min);
   };
-  if (n_steps > 0) {
-    // ---- prologue: the Q rows and K of halves 0..3 leave and are waited for.  K of half x lives in K stage x % 4, V of
-    // half x in V stage x % 4.
-    u32x2_t sl[2], first_slots[4];
+  u32x2_t sl[2], first_slots[4];
+  auto request_slots = [&] {
+    idx_ptr = p.kv_indices + kv_start;
 #pragma unroll
     for (int x = 0; x < 4; ++x) slot_load(k_lo + x * kHalf, first_slots[x]);
 #pragma unroll
     for (int x = 0; x < 2; ++x) slot_load(k_lo + (4 + x) * kHalf, sl[x]);  // for the K moves of step 0
-    move_q();
-    // one round trip for all six slot ids
-    asm volatile("s_waitcnt vmcnt(0)"
+  };
+  auto move_first_k = [&] {
+    // one round trip for all six
+    wait_all_vm();
+    asm volatile(""
                  : "+v"(first_slots[0]), "+v"(first_slots[1]), "+v"(first_slots[2]), "+v"(first_slots[3]),
                    "+v"(sl[0]), "+v"(sl[1])
                  :
                  : "memory");
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < 4; ++x)
 #pragma unroll
       for (int n = 0; n < kUPW; ++n) {
         v_slot[x >> 1][x & 1][n] = first_slots[x][n];
         move_k(x, n, first_slots[x][n]);
       }
-    }
+  };
+  // ---- prologue: the Q rows and K of halves 0..3 leave and are waited for.  K of half x lives in K stage x % 4, V of
+  // half x in V stage x % 4.
+  row_bounds();
+  if (STAY || n_steps > 0) {
+    request_slots();
+    move_q();
+    move_first_k();
     wait_all_vm();
+  }
+  for (int at = 0; STAY || n_steps > 0; ++at) {
     __syncthreads();
-
     f32x16_t sa = zero16, sb;
     bf16x8_t pa[2], pb[2];
 #pragma unroll
@@ -483,6 +525,17 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       if (i + 1 == n_steps) break;
       one_step(std::false_type{}, i + 1, sa, sb, pb, pa, v_slot[0]);
     }
+    // What the block leaves behind while the next one begins
+    const int last_half = 2 * n_steps - 2, done_q = q_start, done_rows = rows_total, done_row0 = row0;
+    const bool more = STAY && at + 1 < n_listed;  // constant where it doesn't stay
+    if (more) {
+      take_listed(at + 1);
+      rows_total = q_len * p.group;
+      row0 = qblk * kRows;
+      n_steps = (k_hi - k_lo + kStep - 1) / kStep;
+      row_bounds();
+      request_slots();
+    }
     // the last step's P V is still owed
     if (__any(alpha != 1.0f)) {
 #pragma unroll
@@ -494,9 +547,64 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
       for (int u = 0; u < 2; ++u) {
         const bf16x8_t pw = as_bf16x8((x == f ? my_p : other_p)[64 * u]);
 #pragma unroll
-        for (int dt = 0; dt < kDT; ++dt) oacc[dt] = mfma_32x32x16(v_operand(2 * n_steps - 2 + x, u, dt), pw, oacc[dt]);
+        for (int dt = 0; dt < kDT; ++dt) oacc[dt] = mfma_32x32x16(v_operand(last_half + x, u, dt), pw, oacc[dt]);
       }
+    if constexpr (STAY) {
+      // Nobody reads the K stages any more, nor the maxima; the barrier frees the V stages.
+      const float own = sum_across<32>(l_run);
+      *my_max = own;
+      if (more) move_first_k();
+      __syncthreads();
+      if (more) move_q();
+      const float l = own + *other_max, inv = (l > 0.f) ? 1.0f / l : 0.f;
+      // Lane (row c32, h) holds 4 of 8 adjacent dims.  Exchanges between lanes l and l + 32 give it all 8 of every second
+      // group, exchanges between rows c and c + 16 then leave a store 64 bytes each of 16 rows (32 of 32 rows take 1 K cycles
+      // more).  Every wave makes every store, whether or not a lane has a row: the wait below counts on it.
+      int lane_row = c32, half = h;  // anew, see move_q()
+      asm volatile("" : "+v"(lane_row), "+v"(half));
+      uint16_t* dst[2];
+      unsigned long long has[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int row = done_row0 + group_row + 16 * x + (lane_row & 15);
+        has[x] = __ballot(row < done_rows);
+        const int qi = row_to_query(p, row);  // of a row past the last: an address, which nothing is stored at
+        dst[x] = p.out + ((int64_t)(done_q + qi) * p.n_q + kvh * p.group + row - qi * p.group) * kD + 128 * f + 16 * (lane_row >> 4) + 8 * half;
+      }
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) {
+        u32x4_t out[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          uint32_t d[4];
+#pragma unroll
+          for (int a = 0; a < 4; ++a) d[a] = pack_bf16x2(oacc[dt][4 * a + 2 * e] * inv, oacc[dt][4 * a + 2 * e + 1] * inv);
+          const auto ab = __builtin_amdgcn_permlane32_swap(d[0], d[1], false, false), cd = __builtin_amdgcn_permlane32_swap(d[2], d[3], false, false);
+          const auto lo = __builtin_amdgcn_permlane16_swap(ab[0], cd[0], false, false), hi = __builtin_amdgcn_permlane16_swap(ab[1], cd[1], false, false);
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            out[x][e] = lo[x];
+            out[x][2 + e] = hi[x];
+          }
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          unsigned long long saved;
+          // (wait states: the store still reads its data's registers, and the compiler does not look into the statement)
+          asm volatile("s_mov_b64 %0, exec\n\ts_and_b64 exec, exec, %1\n\tglobal_store_dwordx4 %2, %3, off offset:%4\n\ts_mov_b64 exec, %0\n\ts_nop 1"
+                       : "=&s"(saved)
+                       : "s"(has[x]), "v"(dst[x]), "v"(out[x]), "n"(64 * dt)
+                       : "memory", "scc");
+        }
+      }
+      if (!more) return;
+      reset();
+      alpha = 1.0f;
+      wait_vm_at_most<2 * kDT>();  // all but the stores
+    }
+    if constexpr (!STAY) break;
   }
+  if constexpr (STAY) return;
   // both halves of the row sum
   float l = l_run;
   l = sum_across<32>(l);
@@ -573,8 +681,9 @@ int launch_prefill_tile256(const PrefillArgs& a, hipStream_t stream) {
     n_blocks += kRestBlocks;
   }
   const dim3 grid((unsigned)n_blocks);
-  if (wide) hipLaunchKernelGGL((prefill_tile256_kernel<true>), grid, dim3(kNW * 64), 0, stream, p);
-  else hipLaunchKernelGGL((prefill_tile256_kernel<false>), grid, dim3(kNW * 64), 0, stream, p);
+  auto* const kernel = p.length_rounds > 0 ? (wide ? prefill_tile256_kernel<true, true> : prefill_tile256_kernel<false, true>)
+                                           : (wide ? prefill_tile256_kernel<true, false> : prefill_tile256_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kNW * 64), 0, stream, p);
   const int launched = check_launch();
   if (launched != MSGL_OK || (p.n_ksplit == 1 && p.ragged_tiles == 0)) return launched;
   return launch_prefill_merge(p, kD, stream);

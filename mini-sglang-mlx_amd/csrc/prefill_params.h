@@ -244,17 +244,24 @@ constexpr int kMinRounds = 2, kMaxRounds = 64;
 // 69.0; 2000 and 1500 under a window of 500 52.3 -> 45.0.  Below one round: one of 1015 31.8 -> 33.0, two of 500 22.7 -> 23.0.
 constexpr int kMinFreshRounds = 1;
 constexpr int kMaxFreshRows = 1 << 17;  // of k and v, in a launch that takes its keys from them
+// The head_dim 256 kernel takes the same list one block after the other (12 K cycles between them; a workgroup that ends
+// pays for the dispatch of the next and its search on top).  330 launches of 1-40 even, ragged and very uneven extends, 1-8 kv heads, groups of 2-16, on up to 8 K keys,
+// staying against not, geometric means by rounds of blocks with rows: 1-1.25 1.014, 1.25-1.5 0.987 (0.84-1.16), 1.5-2 0.956, 2-3
+// 0.964, 3-4 0.915, above 0.953.  us: 60 prompts of up to 400 tokens, 16 / 4 heads, 124 -> 107, 23 of 129-1833 397 -> 382, 30 x 10-400 on up to
+// 500 cached, 24 / 4, 131 -> 122, three of 1344-2949 under a window of 64, 32 / 4, 105 -> 95, four of 512-1972 on up to 8 K 736 -> 719.
+constexpr int kMinHalfRounds256 = 3;
 // XCDs that share a kv head's blocks, as a logarithm
 inline int prefill_log2_xcds(int64_t n_kv) { return n_kv == 1 ? 3 : n_kv == 2 ? 2 : n_kv == 4 ? 1 : 0; }
 inline int64_t prefill_length_blocks(int64_t batch, int64_t n_kv, int64_t n_qblk) {
   const int64_t heads = n_kv >= 8 ? n_kv / 8 : 1, xcds = 1 << prefill_log2_xcds(n_kv);
   return 8 * batch * heads * ((n_qblk + xcds - 1) / xcds);
 }
-// Rounds of a head_dim 128 launch in order of length whose workgroups stay; 0: they don't.
-inline int prefill_stay_rounds(int64_t batch, int64_t total_q, int64_t n_kv, int64_t group, int64_t n_qblk, int min_rounds = kMinRounds) {
+// Rounds of a launch in order of length whose workgroups stay; 0: they don't.
+inline int prefill_stay_rounds(int64_t batch, int64_t total_q, int64_t n_kv, int64_t group, int64_t n_qblk, int block_rows,
+                               int min_half_rounds) {
   const int64_t rounds = (prefill_length_blocks(batch, n_kv, n_qblk) + kComputeUnits - 1) / kComputeUnits;
-  const int64_t filled = 8 * prefill_filled_blocks(batch, total_q, group, kPrefillBlockRows);
-  return n_kv <= 8 && filled >= ((int64_t)min_rounds * kComputeUnits << prefill_log2_xcds(n_kv)) && rounds <= kMaxRounds ? (int)rounds : 0;
+  const int64_t filled = 8 * prefill_filled_blocks(batch, total_q, group, block_rows);
+  return n_kv <= 8 && 2 * filled >= ((int64_t)min_half_rounds * kComputeUnits << prefill_log2_xcds(n_kv)) && rounds <= kMaxRounds ? (int)rounds : 0;
 }
 
 // Gang ranges, for launches with several query blocks per (request, kv head) (chunked extends on
@@ -419,7 +426,8 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     p.length_log2_xcds = prefill_log2_xcds(a.n_kv);
     n_blocks = prefill_length_blocks(a.batch, a.n_kv, n_qblk);
     if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-    if (block_rows == kPrefillBlockRows) p.length_rounds = prefill_stay_rounds(a.batch, a.total_q, a.n_kv, p.group, n_qblk, p.nt.out_loc != nullptr ? kMinFreshRounds : kMinRounds);
+    const int half_rounds = block_rows != kPrefillBlockRows ? kMinHalfRounds256 : 2 * (p.nt.out_loc != nullptr ? kMinFreshRounds : kMinRounds);
+    p.length_rounds = prefill_stay_rounds(a.batch, a.total_q, a.n_kv, p.group, n_qblk, block_rows, half_rounds);
     if (p.length_rounds > 0) n_blocks = kComputeUnits;
   }
   // narrow offsets: slot * row_bytes fits 32 bits and both factors fit 24 bits (one

@@ -178,6 +178,79 @@ struct LengthOrder {
   }
 };
 
+// Keys that some row of a block sees: row0 its first row, `floor` the granularity of the first key.
+template <int ROWS, int FLOOR>
+__device__ __forceinline__ void block_keys(const PrefillParams& p, int prefix, int kn, int row0, int rows_total, int* lo, int* hi) {
+  const int qi_lo = row0 / p.group;
+  const int qi_hi = min(rows_total - 1, row0 + ROWS - 1) / p.group;
+  *hi = p.is_cross ? kn : min(kn, prefix + qi_hi + 1);
+  *lo = (p.window > 0) ? max(0, prefix + qi_lo - p.window + 1) : 0;
+  *lo &= ~(FLOOR - 1);
+  if (*hi < *lo) *hi = *lo;
+}
+
+// The blocks of a workgroup that stays (see kMaxRounds), found by its waves side by side.
+struct ListedBlock {
+  int kvh, qblk, q_start, q_len, kv_start, kv_len, prefix;
+  int k_lo, k_hi, n_tiles;  // keys that some row of the block sees, from a whole tile on
+};
+struct BlockList {
+  ListedBlock block[kMaxRounds];
+  int count, blank;  // blocks; whether one has no keys
+};
+// How many there are: those without keys are not among them, their rows are zero already.  All threads of the workgroup.
+template <int THREADS, int D, int ROWS, int TILE>
+__device__ __forceinline__ int list_blocks(const PrefillParams& p, BlockList& list, int tid) {
+  constexpr int NW = THREADS / kWave;
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
+  const int w = uniform(tid / kWave), lane = tid & (kWave - 1);
+  if (tid == 0) list.count = list.blank = 0;
+  const LengthOrder<ROWS, true> order(p);
+  const int r = (int)(blockIdx.x >> 3), rounds = p.length_rounds;
+  __syncthreads();
+  for (int i = w; i < rounds; i += NW) {
+    constexpr int kPerXcd = kComputeUnits / 8;
+    const int seq = i * kPerXcd + ((i & 1) ? kPerXcd - 1 - r : r);
+    const LengthBlock x = order.find(seq);
+    if (!x.ok) break;
+    ListedBlock l{x.kvh, x.qblk, x.q_start, x.q_len, x.kv_start, x.kv_len, x.prefix, 0, 0, 0};
+    block_keys<ROWS, TILE>(p, l.prefix, l.kv_len, l.qblk * ROWS, l.q_len * p.group, &l.k_lo, &l.k_hi);
+    l.n_tiles = (l.k_hi - l.k_lo + kBN - 1) / kBN;
+    if (lane == 0) {
+      list.block[i] = l;
+      atomicMax(&list.count, i + 1);
+      if (l.n_tiles == 0) list.blank = 1;
+    }
+  }
+  __syncthreads();
+  int n_listed = uniform(list.count);
+  if (uniform(list.blank) != 0) {  // rows without keys are zero; the list goes on without their blocks
+    constexpr int kPerRow = THREADS / ROWS;
+    static_assert(D / kPerRow == 64, "a thread writes 64 values of a row");
+    for (int i = 0; i < n_listed; ++i) {
+      const ListedBlock& l = list.block[i];
+      const int row = l.qblk * ROWS + tid / kPerRow, total = l.q_len * p.group;
+      if (l.n_tiles == 0 && row < total) {
+        const int qi = row_to_query(p, row);
+        const int at = (l.q_start + qi) * p.n_q + l.kvh * p.group + row - qi * p.group;
+        uint16_t* dst = p.out + (int64_t)at * D + 64 * (tid % kPerRow);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) st_global_b128(dst + 8 * e, u32x4_t{0u, 0u, 0u, 0u});
+      }
+    }
+    __syncthreads();
+    if (tid == 0) {
+      int n = 0;
+      for (int i = 0; i < n_listed; ++i)
+        if (list.block[i].n_tiles > 0) list.block[n++] = list.block[i];
+      list.count = n;
+    }
+    __syncthreads();
+    n_listed = uniform(list.count);
+  }
+  return n_listed;
+}
+
 // ---- ragged shares: which (request, share) is unit `u`? ------------------------------------------
 // Shares of a request, from the visible keys of its only query block (rows 0 .. q_len * group - 1), the
 // floor rounded down to a tile: the kernels compute the same for their block.
