@@ -12,7 +12,7 @@
 // gdn_serial_kernel: quarters by the chain of a state wave, 4.5 K cycles of which 2.6 K are matrix instructions; halves where many
 // requests fill the chip by the matrix pipe at the power limit (1.0 PFLOP/s of bf16 products, 1.75 GHz).
 //
-// Both against the one launch, us: one request of 4005 tokens 208 -> 162; of 992, 1581, 4005 and 1601 tokens 208 -> 184; 2000 among five
+// Both against the one launch, us: one request of 4005 tokens 208 -> 159; of 992, 1581, 4005 and 1601 tokens 209 -> 177; 2000 among five
 // short ones 146 -> 95; eight of 1000 158 -> 156.
 #include "gdn_chunk_tiles.h"
 
