@@ -175,12 +175,19 @@ static bool prefer_chunks(const GdnArgs& a) {
   return (pairs ? 9.2 + 0.9 * units : 12.8 * rounds) < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
 }
 // Room for the systems of all chunks where making those in a launch of their own pays (gdn_long.hip), 0 elsewhere.  The second
-// launch costs 3 to 5 us and saves a tenth to a quarter of a long request's chain: one request of 256, 384, 512, 4000 tokens
-// 19.7 -> 20.8, 25.7 -> 25.1, 32.0 -> 29.7, 208 -> 162 us; two of 384, 512, 1000 27.3 -> 28.0, 33.4 -> 32.9, 59.0 -> 54.1; four of 512, 1000
-// 44.3 -> 45.5, 80.0 -> 77.4; eight of 200 to 1600 148 -> 139.  A request and 32 heads have 640 KiB for every 64 tokens; a launch that
-// would need more than 2 GiB goes without.
+// launch costs 3 to 5 us and saves a tenth to a quarter of a long request's chain; where the requests' heads fill the chip it
+// also deals them out by their lengths, which the one launch does not.  680 launches at 32 heads, even, ragged and of one long request
+// beside short ones, time in two launches by that in one: one request of 256-320 tokens 1.00, 352-384 0.96; two and three, by
+// their mean, 320-384 even 1.01, ragged 0.97, 384-448 0.985 and 0.93; four, whose pairs of workgroups fill the chip in one round, even
+// 320-384 1.06, 384-448 1.01, 512-640 0.975, ragged 0.85-1.00; five to eight even 128-192 0.94-1.10, 192-256 0.91-1.05, 256-320 0.93, ragged
+// 0.96 and one long 0.68 in all of these; more 96-128 0.99 (up to 1.03), 128-192 0.97, 0.96 and 0.74.  The lines lie where even ones do not
+// lose either.  us: one of 4000 208 -> 159, eight of 200-1600 148 -> 139, 2060 among five of 100-260 150 -> 91.  A request and 32 heads
+// have 640 KiB for every 64 tokens; a launch that would need more than 2 GiB goes without.
 size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token) {
-  if (single_token || batch <= 0 || tokens < (batch == 1 ? 384 : batch <= 3 ? 448 : 560) * batch) return 0;
+  if (single_token || batch <= 0 || hv <= 0) return 0;
+  const int64_t heads = batch * hv, cus = device_cus();
+  const int64_t mean = 8 * heads <= cus ? 352 : 8 * heads <= 3 * cus ? 384 : 2 * heads <= cus ? 448 : heads <= cus ? 256 : 128;
+  if (tokens < mean * batch) return 0;
   const size_t bytes = gdn_long_workspace_bytes(tokens, batch, hv);
   return bytes <= ((size_t)2 << 30) ? bytes : 0;
 }
