@@ -224,13 +224,9 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   // more rows per lane group (more overlap inside a wave) once there are enough workgroups
   // to fill the chip without it
   const int64_t blocks_r1 = heads * (kDV / 16);
-  // Several tokens per request are bound by vector instructions as soon as waves share a SIMD, and then a load of k and q, made
-  // fp32 once, should serve several rows.  us with 1, 2 and 4 rows, requests of 8 tokens at 32 heads: one 5.7, 6.3, 7.9; two
-  // 7.3, 6.8, 8.3; four 12.0, 9.4, 9.4; eight 18.4, 14.6, 14.0; eight of 16 27.1, 21.2, 20.5; five of 8-27 21.2, 19.4, 22.4.
-  const int64_t from_2 = p.single_token ? 4 * 1024 : 512, from_4 = p.single_token ? 8 * 1024 : 2 * 1024;
   int r = 1;
-  if (blocks_r1 >= from_4) r = 4;
-  else if (blocks_r1 >= from_2) r = 2;
+  if (blocks_r1 >= 8 * 1024) r = 4;
+  else if (blocks_r1 >= 4 * 1024) r = 2;
   if (t_force_rows > 0) r = t_force_rows;
   const int64_t blocks = heads * (kDV / (16 * r));
   if (blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
