@@ -38,7 +38,8 @@ def _bits(t):
 @pytest.mark.parametrize("what", [None, "v", "k", "q", "state"])
 @pytest.mark.parametrize("lengths,hk,hv", [
     ([384], 16, 32), ([447], 4, 4), ([1025], 2, 6), ([500, 449], 16, 32), ([64, 1400, 1], 16, 32), ([2300, 1, 0, 640], 8, 32),
-    ([700, 33, 1500, 65, 1200, 300], 16, 48), ([560] * 9, 16, 32), ([600] * 64 + [0, 1400, 601], 1, 2)])
+    ([700, 33, 1500, 65, 1200, 300], 16, 48), ([560] * 9, 16, 32), ([128] * 9, 16, 32),
+    ([1, 1300, 60, 0, 90, 85], 16, 32), ([600] * 64 + [0, 1400, 601], 1, 2)])
 def test_two_launches_are_one(gpu, lengths, hk, hv, what):
     print(f"gdn long {lengths[:6]} hk {hk} hv {hv} {what}", flush=True)
     rng = np.random.default_rng(sum(lengths) + hv)
