@@ -431,20 +431,28 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
 // boundary it crosses), and nothing any more where they fill the chip several times over (107 MiB 27.3 -> 24.1, 160 39.6 ->
 // 39.5, 371 81 -> 92).
 // The segments' fixed costs are the same for any number of bytes, while the shares' lengths vary and the longest
-// decides; the larger head's segments pay more for their partials, so their line lies further out.  By MiB of keys and
-// values: head_dim 128 39 18.7 -> 14.2 (2 requests), 66 21.2 -> 17.9 (12), 97 27.3 -> 22.4 (9), 142 32.3 -> 29.0 (13), 196
-// 38.4 -> 36.3 (7), 201 39.6 -> 41.2 (92), 247 45.5 -> 51.9, 414 85 -> 106; head_dim 256 72 32.4 -> 25.6 (9), 134 40.6 ->
-// 33.0 (31), 256 60.7 -> 54.6 (63), 357 81 -> 72 (13), 415 89.7 -> 86.0 (10), 485 and more about equal.
+// decides.  So a launch beyond the first lines has to be one whose shares are short, and sure to go in one round, requests of
+// one length included.  By MiB of keys and values: head_dim 128 39 18.7 -> 14.2 (2 requests), 66 21.2 -> 17.9 (12), 97 27.3 -> 22.4 (9),
+// 142 32.3 -> 29.0 (13), 165 35.4 -> 31.7 (5), with longer shares 118 28.5 -> 29.6 (24), 175 35.8 -> 40.8 (22), 247 45.5 -> 51.9, with a
+// workgroup too many 81 21.8 -> 27.8 (33); head_dim 256 72 32.4 -> 25.6 (9), 134 40.6 -> 33.0 (31), 237 58.4 -> 66.8 (17).  One long request
+// among short ones gains as much (64, 15 requests, the longest 9.2 K, 20.5 -> 17.6; head_dim 256 155, 19, 24.7 K 44.5 -> 38.5), but
+// not where several heads go to a workgroup (177, 48, 14 K 36.0 -> 39.7), nor few requests with many columns, whose last shares
+// have most to put together (59, 2 requests, 40 columns 28.4 -> 35.1).
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
-  const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch;
+  const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
-  // Few units: at head_dim 256 most of the time is the last share's, which reads all the others of a wide head group (2
-  // requests of 10 K, 2 kv heads: 23.4 -> 31.2); at 128 a request's 16 shares leave most of the chip idle and get long
-  // (one request, 8 kv heads: 8.7 K keys 16.4 -> 15.2, 26.5 K 26.7 -> 28.1)
-  if (batch * n_kv < 12 && (head_dim == 256 || mean > 12288)) return false;
-  return mb <= (head_dim == 256 ? 448 : 208);
+  // few units: most of the time is the last share's, which reads all the others of a wide head group
+  if (head_dim == 256 && units < 12) return false;
+  if (mb <= (mean > 8192 ? 20 : mean > 4096 ? 36 : head_dim == 256 ? 128 : 56)) return true;
+  const int64_t len = plan.share_len, head_groups = n_kv / plan.heads_wg;
+  const double shares = (double)keys / (double)len + 0.5 * (double)batch + std::sqrt((double)batch / 3);  // see share_plan()
+  if (shares * (double)head_groups > device_cus() || batch * ((mean + len - 1) / len) * head_groups > device_cus()) return false;
+  if (head_dim == 256) return units >= 24 && len * plan.heads_wg <= 1024 && mb <= 256;
+  // (at 128 one request's 16 shares leave most of the chip idle and get long: 8.7 K keys 16.4 -> 15.2, 26.5 K 26.7 -> 28.1)
+  if (units < 32 && (cols > 16 || (units < 12 && mean > 12288))) return false;
+  return len * plan.heads_wg <= 1536 && mb <= (units > device_cus() ? 128 : 208);
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {

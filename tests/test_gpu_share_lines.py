@@ -18,7 +18,8 @@ LINES = [  # kv lengths, q heads, kv heads, head_dim
     ([4000, 9000, 1], 16, 4, 128),  # 12 units
     ([20001, 17], 16, 4, 128),      # 8 of them, of some length
     ([9000, 300, 7000], 16, 4, 256), ([9000, 300], 24, 4, 256),
-    ([32768, 65536, 40000, 50000, 41000], 16, 2, 256), ([32768, 65536, 40000, 50000, 41200], 16, 2, 256),  # 448 and 449
+    ([32768, 40000, 17, 5000, 30000, 23200], 16, 4, 256), ([32768, 40000, 17, 5000, 30000, 23400], 16, 4, 256),  # 255 and 256
+    ([9000] * 6, 16, 4, 256), ([9000] * 5 + [4000], 16, 4, 256)
 ]
 
 
