@@ -770,9 +770,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   bool from_rows = false;
   if constexpr (FRESH) from_rows = uniform(rows_are_the_keys<NW * 64>(p, tid) ? 1 : 0) != 0;
   if constexpr (listed) {
-    n_listed = list_blocks<NW * 64, D, kRows, kBN>(p, list, tid);
-    if (n_listed == 0) return;
-    if (FRESH && !from_rows) {
+    n_listed = list_blocks<NW * 64, kRows, kBN>(p, list, tid);
+    if (FRESH && !from_rows) {  // of every request that has a block here, also where that one sees no key
       for (int i = 0; i < n_listed; ++i) {
         const int start = uniform(list.block[i].q_start);
         if (i > 0 && uniform(list.block[i - 1].q_start) == start) continue;
@@ -782,6 +781,8 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
         store_request_rows<NW * 64, D>(p, start, min(n, p.nt.rows - start), uniform(list.block[i].kvh), tid);
       }
     }
+    n_listed = drop_blank_blocks<NW * 64, D, kRows>(p, list, n_listed, tid);
+    if (n_listed == 0) return;
   }
   GangPlan plan{0, 0, 0, 0};
   if (ganged) plan = gang_plan<NW * 64>(p, gang_lds, gang_xcd, gang_id, gang_member, kRows, tid);

@@ -100,7 +100,8 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
   LengthBlock by_length{};
   RequestPlace place{};
   if constexpr (STAY) {
-    n_listed = list_blocks<kNW * 64, kD, kRows, kHalf>(p, list, tid);
+    n_listed = list_blocks<kNW * 64, kRows, kHalf>(p, list, tid);
+    n_listed = drop_blank_blocks<kNW * 64, kD, kRows>(p, list, n_listed, tid);
     if (n_listed == 0) return;
     kvh = uniform(list.block[0].kvh);  // of all the XCD's blocks
     b = qblk = 0;                      // the list has them

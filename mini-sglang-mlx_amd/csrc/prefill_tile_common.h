@@ -198,12 +198,11 @@ struct BlockList {
   ListedBlock block[kMaxRounds];
   int count, blank;  // blocks; whether one has no keys
 };
-// How many there are: those without keys are not among them, their rows are zero already.  All threads of the workgroup.
-template <int THREADS, int D, int ROWS, int TILE>
+// How many there are, those without keys among them.  All threads of the workgroup.
+template <int THREADS, int ROWS, int TILE>
 __device__ __forceinline__ int list_blocks(const PrefillParams& p, BlockList& list, int tid) {
   constexpr int NW = THREADS / kWave;
-  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };  // the same in every lane: a scalar
-  const int w = uniform(tid / kWave), lane = tid & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid & (kWave - 1);
   if (tid == 0) list.count = list.blank = 0;
   const LengthOrder<ROWS, true> order(p);
   const int r = (int)(blockIdx.x >> 3), rounds = p.length_rounds;
@@ -223,8 +222,12 @@ __device__ __forceinline__ int list_blocks(const PrefillParams& p, BlockList& li
     }
   }
   __syncthreads();
-  int n_listed = uniform(list.count);
-  if (uniform(list.blank) != 0) {  // rows without keys are zero; the list goes on without their blocks
+  return __builtin_amdgcn_readfirstlane(list.count);
+}
+// The list of `n_listed` goes on without the blocks that have no keys: their rows are zero.  How many are left.
+template <int THREADS, int D, int ROWS>
+__device__ __forceinline__ int drop_blank_blocks(const PrefillParams& p, BlockList& list, int n_listed, int tid) {
+  if (__builtin_amdgcn_readfirstlane(list.blank) != 0) {
     constexpr int kPerRow = THREADS / ROWS;
     static_assert(D / kPerRow == 64, "a thread writes 64 values of a row");
     for (int i = 0; i < n_listed; ++i) {
@@ -246,7 +249,7 @@ __device__ __forceinline__ int list_blocks(const PrefillParams& p, BlockList& li
       list.count = n;
     }
     __syncthreads();
-    n_listed = uniform(list.count);
+    n_listed = __builtin_amdgcn_readfirstlane(list.count);
   }
   return n_listed;
 }

@@ -1,6 +1,6 @@
 """Prompts with nothing cached whose rows the attention launch stores itself: output and pool are, bit for bit, those of the store and
 the attention called one after the other.  Groups whose blocks' own tokens are a tile, part of one, or several; last blocks that are
-not full; windows and cross attention; rows that belong to no request; rows whose slots are not the ones listed."""
+not full; windows and cross attention; rows that belong to no request; rows whose slots are not the ones listed; requests that see no key."""
 import numpy as np
 import pytest
 import torch
@@ -17,7 +17,7 @@ def _one_launch(ext, n_q, n_kv, cross, window):
     return _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(ext), n_q, n_kv, D, max(ext), int(cross), window) > 0
 
 
-def _check(gpu, ext, heads, window=0, cross=False, change=None, front=0, strided=False, pad=0):
+def _check(gpu, ext, heads, window=0, cross=False, change=None, front=0, strided=False, pad=0, hidden=(), keyless=False):
     n_q, n_kv = heads
     g = torch.Generator(device=gpu)
     g.manual_seed(sum(ext) + n_q)
@@ -34,17 +34,25 @@ def _check(gpu, ext, heads, window=0, cross=False, change=None, front=0, strided
     starts = np.cumsum([front] + list(ext[:-1]) + [ext[-1] - front])  # with rows in front of the first request, its last one is shorter
     ip = torch.tensor(starts, dtype=torch.int32, device=gpu)
     prefix = torch.zeros(len(ext), dtype=torch.int32, device=gpu)
+    kv_ip = ip
+    for b in hidden:  # the window lies behind all of the request's keys
+        prefix[b] = 5000
+    if keyless:  # the first request lists no keys, the second as many more, which are in the pool
+        kv_ip = ip.clone()
+        kv_ip[1] = 0
+        prefix[1] = ext[0]
+        ids[:ext[0]] = torch.arange(slots, device=gpu, dtype=torch.int32)[~torch.isin(torch.arange(slots, device=gpu), out_loc.long())][:ext[0]]
     if change == "slot":  # a key of a request is a row of the pool that no row goes to
         ids[total // 2] = next(s for s in range(slots) if not bool((out_loc == s).any()))
     elif change == "outside":  # a row that goes nowhere
         out_loc[total // 3] = -1
     assert _one_launch(ext, n_q, n_kv, cross, window)
-    print(f"fresh {ext[:6]} heads {heads} window {window} cross {cross} {change} front {front}", flush=True)
+    print(f"fresh {ext[:6]} heads {heads} window {window} cross {cross} {change} front {front} hidden {hidden} {keyless}", flush=True)
     want_pools = [p.clone() for p in pools]
     store_kv_cache(*want_pools, out_loc, k, v)
-    want = paged_prefill_attention(q, *want_pools, ip, ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
+    want = paged_prefill_attention(q, *want_pools, ip, kv_ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
                                    is_cross_attention=cross, sliding_window_size=window)
-    got = extend_step(q, k, v, out_loc, *pools, ip, ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
+    got = extend_step(q, k, v, out_loc, *pools, ip, kv_ip, ids, prefix, sm_scale=D ** -0.5, max_len_extend=max(ext),
                       is_cross_attention=cross, sliding_window_size=window)
     torch.cuda.synchronize()
     for a, b in zip(pools, want_pools):
@@ -69,6 +77,18 @@ def test_masks(gpu, heads, window, cross):
 @pytest.mark.parametrize("front", [0, 7])
 def test_rows_that_are_not_the_keys(gpu, change, front):
     _check(gpu, [1300, 900, 64, 1100], (32, 8), change=change, front=front, strided=change is None)
+
+
+@pytest.mark.parametrize("heads", [(32, 8), (16, 2)])
+@pytest.mark.parametrize("hidden", [(0,), (1, 3), (0, 1, 2, 3)])
+def test_requests_whose_keys_the_window_hides(gpu, hidden, heads):
+    _check(gpu, [1300] * 4, heads, window=1024, hidden=hidden)
+    _check(gpu, [1700, 64, 1999, 901], heads, window=300, hidden=hidden)
+
+
+@pytest.mark.parametrize("heads", [(32, 8), (16, 2)])
+def test_request_without_keys(gpu, heads):
+    _check(gpu, [700, 1300, 900, 1500], heads, keyless=True)
 
 
 def test_wide_pool(gpu):
