@@ -730,11 +730,18 @@ PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args)
       y = empty({tokens, hv, dv}, at::kBFloat16, dev);
       const Tensor gc = g.contiguous(), bc = beta.contiguous(), sc = slots.contiguous();
       const Tensor ipc = single ? Tensor() : THPVariable_Unpack(a[7]).contiguous();
-      const size_t bytes = msgl_gdn_state_workspace_bytes(tokens, batch, hv, single ? 1 : 0);
-      const Tensor ws = bytes ? scratch(bytes, dev) : Tensor();
+      size_t bytes = msgl_gdn_state_workspace_bytes(tokens, batch, hv, single ? 1 : 0);
+      Tensor ws;
+      if (bytes > 0) {
+        try {
+          ws = scratch(bytes, dev);
+        } catch (const c10::OutOfMemoryError&) {  // it is an optimisation: the call goes without
+          bytes = 0;
+        }
+      }
       rc = msgl_gdn_state_inplace_in(q.data_ptr(), k.data_ptr(), v.data_ptr(), gc.data_ptr(), bc.data_ptr(), state.data_ptr(),
                                   ints(sc), single ? nullptr : ints(ipc), y.data_ptr(), tokens, batch, hk, hv, dk, dv,
-                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, bytes ? ws.data_ptr() : nullptr, bytes, on.ptr());
+                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, data_or_null(ws), bytes, on.ptr());
     }
     check_rc(op, rc);
     return THPVariable_Wrap(std::move(y));
