@@ -357,8 +357,9 @@ MSGL_API int msgl_gdn_state_inplace(const void* q, const void* k, const void* v,
                            int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
                            int64_t v_stride0, int32_t single_token_mode, void* stream);
 /*
- * The same with scratch memory (16-byte aligned; NULL or too small: without), which requests of many
- * tokens are faster with.  msgl_gdn_state_workspace_bytes: how much that is, 0 where it would not be used.
+ * The same with scratch memory (16-byte aligned; NULL or too small: without, same results), which requests of many
+ * tokens are faster with.  msgl_gdn_state_workspace_bytes: how much that is, 0 where it would not be used.  (Nor is it
+ * used where v is not 16-byte aligned, v_stride0 no multiple of 8, a stride of q, k or v 2^24 or more, or hv 2^17.)
  */
 MSGL_API size_t msgl_gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv,
                                                int32_t single_token_mode);

@@ -174,6 +174,7 @@ static bool prefer_chunks(const GdnArgs& a) {
   const bool pairs = a.batch <= 64 && a.batch * a.hv * 4 <= device_cus();
   return (pairs ? 9.2 + 0.9 * units : 12.8 * rounds) < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
 }
+static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 // Room for the systems of all chunks where making those in a launch of their own pays (gdn_long.hip), 0 elsewhere.  The second
 // launch costs 3 to 5 us and saves a tenth to a quarter of a long request's chain; where the requests' heads fill the chip it
 // also deals them out by their lengths, which the one launch does not.  680 launches at 32 heads, even, ragged and of one long request
@@ -184,14 +185,13 @@ static bool prefer_chunks(const GdnArgs& a) {
 // lose either.  us: one of 4000 208 -> 159, eight of 200-1600 148 -> 139, 2060 among five of 100-260 150 -> 91.  A request and 32 heads
 // have 640 KiB for every 64 tokens; a launch that would need more than 2 GiB goes without.
 size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token) {
-  if (single_token || batch <= 0 || hv <= 0) return 0;
+  if (single_token || batch <= 0 || hv <= 0 || t_force_rows > 0) return 0;
   const int64_t heads = batch * hv, cus = device_cus();
   const int64_t mean = 8 * heads <= cus ? 352 : 8 * heads <= 3 * cus ? 384 : 2 * heads <= cus ? 448 : heads <= cus ? 256 : 128;
   if (tokens < mean * batch) return 0;
   const size_t bytes = gdn_long_workspace_bytes(tokens, batch, hv);
   return bytes <= ((size_t)2 << 30) ? bytes : 0;
 }
-static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 void gdn_set_rows(int v) { t_force_rows = (v == 1 || v == 2 || v == 4) ? v : 0; }
 
 int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {

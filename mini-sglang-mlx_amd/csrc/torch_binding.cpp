@@ -730,7 +730,9 @@ PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args)
       y = empty({tokens, hv, dv}, at::kBFloat16, dev);
       const Tensor gc = g.contiguous(), bc = beta.contiguous(), sc = slots.contiguous();
       const Tensor ipc = single ? Tensor() : THPVariable_Unpack(a[7]).contiguous();
-      size_t bytes = msgl_gdn_state_workspace_bytes(tokens, batch, hv, single ? 1 : 0);
+      // the forms whose scratch memory would not be used (see the header)
+      const bool plain = reinterpret_cast<uintptr_t>(v.data_ptr()) % 16 == 0 && vs % 8 == 0 && std::max({qs, ks, vs}) < (1 << 24) && hv < (1 << 17);
+      size_t bytes = plain ? msgl_gdn_state_workspace_bytes(tokens, batch, hv, single ? 1 : 0) : 0;
       Tensor ws;
       if (bytes > 0) {
         try {

@@ -113,3 +113,19 @@ def test_without_room_for_the_systems(gpu):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(_bits(y2), _bits(y1)) and torch.equal(_bits(s2), _bits(s1))
+
+
+@pytest.mark.parametrize("pad,rows", [(4, 0), (0, 1)])
+def test_no_memory_where_it_is_not_used(gpu, tuning, pad, rows):
+    """Rows of v that the chunked form does not take, and the token kernel set by hand."""
+    from mini_sglang_amd_kernel import _lib
+
+    x = _operator_inputs(gpu, 1024, 4, 8, pad)
+    tuning(_lib.TUNE_GDN_ROWS, rows)
+    state = x[5].clone()
+    print(f"gdn no memory pad {pad} rows {rows}", flush=True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y = _operator(x, state)
+    assert torch.cuda.max_memory_allocated() - before < y.numel() * 2 + (1 << 16)
