@@ -465,12 +465,18 @@ size_t msgl_paged_prefill_workspace_bytes(int64_t batch, int64_t total_q, int64_
   return std::max(split_need, tile_need);
 }
 
+static bool stores_in_tiles(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_q, int64_t n_kv, int64_t head_dim,
+                            int64_t max_len_extend, bool is_cross, int64_t window);
+
 // Whether prompts with nothing cached go through the tile kernel whose workgroups stay, which takes their keys and values from
 // the new rows and stores those on the way (see kMinFreshRounds): as many keys as rows, in one pass over them, from one round of blocks on.
+// Not those whose only round stores_in_tiles() has (us, there and here: 8 of 126 tokens, 64 / 8 heads, 16.0 and 18.4, 16 of 64 15.0 and 18.6,
+// 16 of 127, 32 / 4, 16.3 and 18.1, 16 of 126, 32 / 8, 17.3 and 18.8).
 static bool prompts_stored(int64_t batch, int64_t total_q, int64_t total_kv, int64_t n_q, int64_t n_kv, int64_t head_dim,
                            int64_t max_len_extend, bool is_cross, int64_t window) {
   if (batch <= 0 || total_q <= 0 || total_kv != total_q || total_q > msgl::kMaxFreshRows || n_q <= 0 || n_kv <= 0 || n_q % n_kv != 0 || max_len_extend <= 0 ||
-      window < 0 || head_dim != 128 || msgl::tile_variant() != 0 || t_gangs > 0)
+      window < 0 || head_dim != 128 || msgl::tile_variant() != 0 || t_gangs > 0 ||
+      stores_in_tiles(batch, total_q, total_kv, n_q, n_kv, head_dim, max_len_extend, is_cross, window))
     return false;
   const int64_t group = n_q / n_kv;
   if (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) ||
