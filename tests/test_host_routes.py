@@ -58,3 +58,12 @@ def route(tmp_path_factory):
     ([126] * 32, (16, 1), TILES), ([510] * 8, (16, 8), STAY), ([900, 1015, 800], (32, 8), STAY), ([1015], (32, 8), NOT)])
 def test_prompts_of_one_round(route, ext, heads, want):
     assert route(ext, heads) == want
+
+
+@pytest.mark.parametrize("ext,heads,cross,want", [
+    ([267] * 22, (8, 8), False, NOT), ([310] * 23, (8, 8), False, NOT), ([511] * 16, (8, 8), False, STAY),       # 0.7, 0.87, 1.0 rounds of rows
+    ([457] + [22] * 57, (8, 8), False, NOT), ([267] + [13] * 57, (16, 8), False, NOT), ([389] + [19] * 49, (32, 4), False, NOT),
+    ([237, 3333, 1500, 2200, 1700, 2604], (32, 8), False, STAY), ([237, 3333, 1500, 2200, 1700, 2604], (32, 8), True, STAY),
+    ([285] * 36, (64, 8), True, NOT), ([285] * 36, (64, 8), False, STAY), ([1923, 400, 476], (32, 4), True, NOT)])
+def test_prompts_that_have_most_of_a_round_to_store(route, ext, heads, cross, want):
+    assert route(ext, heads, cross) == want
