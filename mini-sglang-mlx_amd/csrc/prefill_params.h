@@ -245,13 +245,23 @@ constexpr int kMinRounds = 2, kMaxRounds = 64;
 constexpr int kMinFreshRounds = 1;
 constexpr int kMaxFreshRows = 1 << 17;  // of k and v, in a launch that takes its keys from them
 // The head_dim 256 kernel takes the same list one block after the other (12 K cycles between them; a workgroup that ends
-// pays for the dispatch of the next and its search on top).  330 launches of 1-40 even, ragged and very uneven extends, 1-8 kv heads, groups of 2-16, on up to 8 K keys,
-// staying against not, geometric means by rounds of blocks with rows: 1-1.25 1.014, 1.25-1.5 0.987 (0.84-1.16), 1.5-2 0.956, 2-3
-// 0.964, 3-4 0.915, above 0.953.  us: 60 prompts of up to 400 tokens, 16 / 4 heads, 124 -> 107, 23 of 129-1833 397 -> 382, 30 x 10-400 on up to
-// 500 cached, 24 / 4, 131 -> 122, three of 1344-2949 under a window of 64, 32 / 4, 105 -> 95, four of 512-1972 on up to 8 K 736 -> 719.
+// pays for the dispatch of the next and its search on top), from 1.5 rounds of blocks on.  us: 60 prompts of up to 400 tokens, 16 / 4 heads,
+// 124 -> 107, 23 of 129-1833 397 -> 382, three of 1344-2949 under a window of 64, 32 / 4, 105 -> 95, four of 512-1972 on up to 8 K 736 -> 719.
+// The blocks are dealt out beforehand, by number and not by length, and those that share a request's keys drift apart: that has to do no harm.
+// It does none where lengths follow from the rows' places, causal prompts with nothing cached and windows that most requests exceed (173 launches of
+// 1-60 even, ragged and very uneven requests, staying against not, geometric mean, best and worst: 0.938, 0.76 and 1.10), nor where an average
+// request's blocks fill their XCDs by themselves (97 on up to 16 K cached: 0.981, 0.91 and 1.02).  Requests of fewer blocks on prefixes of any length
+// gain less on average, 0.993 of 359, and lose up to 1.42 where one is much longer than the others (42 requests of 87 tokens, 32 / 2 heads, one on
+// 1290 cached, 45.5 and 61.8 us) or small groups' blocks each wait for their own keys (32 of up to 1269 on 4057 each, 8 / 8, 1114 and 1465); so do
+// those whose rows see all keys, 0.978 of 80 and 1.25.
 constexpr int kMinHalfRounds256 = 3;
 // XCDs that share a kv head's blocks, as a logarithm
 inline int prefill_log2_xcds(int64_t n_kv) { return n_kv == 1 ? 3 : n_kv == 2 ? 2 : n_kv == 4 ? 1 : 0; }
+inline bool prefill_may_stay_256(const PrefillArgs& a, int64_t group) {
+  if (a.is_cross) return false;
+  if (a.total_kv == a.total_q || (a.window > 0 && a.total_kv >= a.batch * a.window)) return true;
+  return a.total_q * group >= a.batch * ((kComputeUnits / 8 * kPrefillBlockRows256) << prefill_log2_xcds(a.n_kv));
+}
 inline int64_t prefill_length_blocks(int64_t batch, int64_t n_kv, int64_t n_qblk) {
   const int64_t heads = n_kv >= 8 ? n_kv / 8 : 1, xcds = 1 << prefill_log2_xcds(n_kv);
   return 8 * batch * heads * ((n_qblk + xcds - 1) / xcds);
@@ -427,7 +437,8 @@ inline int make_prefill_params(const PrefillArgs& a, PrefillParams& p, int64_t& 
     n_blocks = prefill_length_blocks(a.batch, a.n_kv, n_qblk);
     if (n_blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
     const int half_rounds = block_rows != kPrefillBlockRows ? kMinHalfRounds256 : 2 * (p.nt.out_loc != nullptr ? kMinFreshRounds : kMinRounds);
-    p.length_rounds = prefill_stay_rounds(a.batch, a.total_q, a.n_kv, p.group, n_qblk, block_rows, half_rounds);
+    if (block_rows == kPrefillBlockRows || prefill_may_stay_256(a, p.group))
+      p.length_rounds = prefill_stay_rounds(a.batch, a.total_q, a.n_kv, p.group, n_qblk, block_rows, half_rounds);
     if (p.length_rounds > 0) n_blocks = kComputeUnits;
   }
   // narrow offsets: slot * row_bytes fits 32 bits and both factors fit 24 bits (one

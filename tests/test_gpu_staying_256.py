@@ -29,6 +29,11 @@ CASES = [  # q heads, kv heads, extends, cached, window, cross, every third requ
     (16, 4, [190] * 14 + [150], [(i * 61) % 500 for i in range(15)], 0, False, False),
     (16, 4, [220] * 14 + [150], [(i * 61) % 500 for i in range(15)], 0, False, False),
     (32, 8, [1300] + [16] * 14 + [0], [(i * 61) % 500 for i in range(16)], 0, False, False),
+    # prefixes: under a window that most requests exceed, and beside blocks that fill their XCDs
+    (24, 4, _mixed(64, 300), [(i * 131) % 700 for i in range(64)], 200, False, False),
+    (16, 1, _mixed(32, 300), [0] * 32, 0, False, False),
+    (10, 2, _mixed(64, 300), [64 + (i * 17) % 90 for i in range(64)], 64, False, False),
+    (32, 8, [1024, 1100], [300, 40], 0, False, False),
 ]
 
 

@@ -1,5 +1,6 @@
-"""Which launches of the head_dim 128 extend kernel go to workgroups that stay (csrc/prefill_params.h): by the blocks that have
-rows, not by the grid of requests that are all as long as the longest."""
+"""Which launches of the extend kernels go to workgroups that stay (csrc/prefill_params.h): by the blocks that have
+rows, not by the grid of requests that are all as long as the longest; at head_dim 256 only where their lengths follow from
+the rows' places, or every request's blocks fill their XCDs."""
 import os
 import subprocess
 
@@ -12,14 +13,16 @@ PROGRAM = r"""
 namespace msgl { long long* clock_probe() { return nullptr; } }
 int main() {
   msgl::PrefillArgs a{};
-  long long batch, total_q, total_kv, n_q, n_kv, longest;
-  while (std::scanf("%lld %lld %lld %lld %lld %lld", &batch, &total_q, &total_kv, &n_q, &n_kv, &longest) == 6) {
+  long long batch, total_q, total_kv, n_q, n_kv, longest, head_dim, window, cross;
+  while (std::scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld", &batch, &total_q, &total_kv, &n_q, &n_kv, &longest, &head_dim, &window,
+                    &cross) == 9) {
+    a.window = window; a.is_cross = (int)cross;
     a.batch = batch; a.total_q = total_q; a.total_kv = total_kv; a.n_q = n_q; a.n_kv = n_kv; a.max_len_extend = (int)longest;
-    a.head_dim = 128; a.num_slots = 1 << 20; a.k_stride0 = a.v_stride0 = n_kv * 128; a.key_splits = 1; a.by_length = 1;
+    a.head_dim = head_dim; a.num_slots = 1 << 20; a.k_stride0 = a.v_stride0 = n_kv * head_dim; a.key_splits = 1; a.by_length = 1;
     msgl::PrefillParams p;
     int64_t blocks = 0;
     bool wide = false;
-    const int rc = msgl::make_prefill_params(a, p, blocks, wide);
+    const int rc = msgl::make_prefill_params(a, p, blocks, wide, msgl::prefill_block_rows(head_dim));
     std::printf("%d %d %lld\n", rc, (int)p.length_rounds, (long long)blocks);
   }
 }
@@ -44,8 +47,8 @@ def rounds(tmp_path_factory):
                     "-isystem", "/opt/rocm/include", str(src), "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-o", str(exe)],
                    check=True)
 
-    def ask(ext, cached, n_q, n_kv):
-        line = f"{len(ext)} {sum(ext)} {sum(ext) + cached * len(ext)} {n_q} {n_kv} {max(ext)}\n"
+    def ask(ext, cached, n_q, n_kv, head_dim=128, window=0, cross=False):
+        line = f"{len(ext)} {sum(ext)} {sum(ext) + cached * len(ext)} {n_q} {n_kv} {max(ext)} {head_dim} {window} {int(cross)}\n"
         out = subprocess.run([str(exe)], input=line, check=True, capture_output=True, text=True).stdout.split()
         return [int(x) for x in out]
     return ask
@@ -58,3 +61,26 @@ def test_rounds_count_blocks_with_rows(rounds, ext, cached, n_q, n_kv, stay):
     if stay:  # one workgroup per compute unit, and room in its list for every block of the grid
         most = -(-max(ext) * (n_q // n_kv) // 256)
         assert blocks == 256 and n * 256 >= 8 * len(ext) * -(-most // (8 // n_kv))
+
+
+CASES_256 = [  # extends, tokens cached (mean), q heads, kv heads, window, all keys seen; whether the workgroups stay
+    ([400, 237, 100, 333] * 15, 0, 16, 4, 0, False, True),     # prompts: 4.2 rounds
+    ([190] * 14 + [150], 0, 16, 4, 0, False, False),           # 1.4 of them
+    ([220] * 14 + [150], 0, 16, 4, 0, False, True),            # 1.6
+    ([698] * 22, 500, 8, 8, 0, False, False),                  # 6 blocks a request in an XCD
+    ([87, 40, 30] * 14, 100, 32, 2, 0, False, False),
+    ([698] * 22, 500, 8, 8, 300, False, True),                 # a window that most exceed
+    ([698] * 22, 500, 8, 8, 2000, False, False),               # and one that they do not
+    ([2048] * 4, 4000, 16, 4, 0, False, True), ([2047] * 4, 4000, 16, 4, 0, False, False),  # 32 blocks a request in an XCD
+    ([2731] * 4, 4000, 24, 8, 0, False, True), ([1365] * 4, 4000, 24, 8, 0, False, False),
+    ([2048] * 4, 0, 16, 4, 0, True, False), ([2048] * 4, 0, 16, 4, 300, True, False), ([2048] * 4, 0, 16, 4, 300, False, True),
+]
+
+
+@pytest.mark.parametrize("ext,cached,n_q,n_kv,window,cross,stay", CASES_256)
+def test_rounds_of_head_dim_256(rounds, ext, cached, n_q, n_kv, window, cross, stay):
+    rc, n, blocks = rounds(ext, cached, n_q, n_kv, 256, window, cross)
+    assert rc == 0 and (n > 0) is stay
+    if stay:
+        xcds, most = 8 // min(n_kv, 8), -(-max(ext) * (n_q // n_kv) // 128)
+        assert blocks == 256 and n * 256 >= 8 * len(ext) * -(-most // xcds)
