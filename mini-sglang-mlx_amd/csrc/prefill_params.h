@@ -210,12 +210,15 @@ inline size_t prefill_ragged_workspace_bytes(int64_t batch, int64_t total_kv, in
 // A launch of fewer blocks than compute units has no order.  Whole prompts of one length in many blocks each are even as
 // they are, and at head_dim 256 gain more from a request's blocks side by side (us, side by side and in order, 24 / 4 heads: six of 1000
 // tokens 112.0 and 120.1, two of 2000 122.8 and 125.5; 16 / 4: eight of 1024 101.7 and 114.7).  At head_dim 128 the order lets workgroups stay
-// (below): 32 / 8 heads, four of 1000 55.4 and 46.5, eight of 1024 96.2 and 81.8, five of 1722 133.9 and 125.1, one of 8000 444 and 437, one of
-// 4000 121.8 and 122.9; 16 / 8, three of 2000 68.4 and 59.4.
+// (below): 32 / 8 heads, four of 1000 55.4 and 46.5, eight of 1024 96.2 and 81.8, five of 1722 133.9 and 125.1, one of 8000 444 and 437; 16 / 8,
+// three of 2000 68.4 and 59.4.  Below two rounds they do not stay, and one or two are better off side by side: 55 launches, in order by side by side:
+// those below 0.97-1.036 (two of 3963, 16 / 8 heads, 129.9 and 134.6, two of 1981, 32 / 4, 70.5 and 72.6, one of 4000, 32 / 8, 121.8 and 122.9),
+// three and more 0.87-0.98, from two rounds on 0.73-0.99.
 inline bool prefill_by_length(const PrefillArgs& a, int64_t n_qblk, bool fresh = false) {
   const bool even_prompts = !a.is_cross && a.total_kv == a.total_q && a.total_q == a.batch * a.max_len_extend;
+  const int64_t blocks = a.batch * a.n_kv * n_qblk;
   return a.by_length && a.batch <= 64 && (a.n_kv == 1 || a.n_kv == 2 || a.n_kv == 4 || a.n_kv % 8 == 0) &&
-         (fresh || (a.batch * a.n_kv * n_qblk > kComputeUnits && !(even_prompts && n_qblk >= 16 && a.head_dim == 256)));
+         (fresh || (blocks > kComputeUnits && !(even_prompts && n_qblk >= 16 && (a.head_dim == 256 || (a.batch <= 2 && blocks < 2 * kComputeUnits)))));
 }
 
 // Rounds of blocks that a workgroup may stay for.  A workgroup of the head_dim 128 kernel that ends pays for the next

@@ -23,7 +23,7 @@ int main() {
     int64_t blocks = 0;
     bool wide = false;
     const int rc = msgl::make_prefill_params(a, p, blocks, wide, msgl::prefill_block_rows(head_dim));
-    std::printf("%d %d %lld\n", rc, (int)p.length_rounds, (long long)blocks);
+    std::printf("%d %d %lld %d\n", rc, (int)p.length_rounds, (long long)blocks, (int)p.length_heads);
   }
 }
 """
@@ -47,10 +47,10 @@ def rounds(tmp_path_factory):
                     "-isystem", "/opt/rocm/include", str(src), "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-o", str(exe)],
                    check=True)
 
-    def ask(ext, cached, n_q, n_kv, head_dim=128, window=0, cross=False):
+    def ask(ext, cached, n_q, n_kv, head_dim=128, window=0, cross=False, order=False):
         line = f"{len(ext)} {sum(ext)} {sum(ext) + cached * len(ext)} {n_q} {n_kv} {max(ext)} {head_dim} {window} {int(cross)}\n"
         out = subprocess.run([str(exe)], input=line, check=True, capture_output=True, text=True).stdout.split()
-        return [int(x) for x in out]
+        return [int(x) for x in out][:None if order else 3]
     return ask
 
 
@@ -84,3 +84,11 @@ def test_rounds_of_head_dim_256(rounds, ext, cached, n_q, n_kv, window, cross, s
     if stay:
         xcds, most = 8 // min(n_kv, 8), -(-max(ext) * (n_q // n_kv) // 128)
         assert blocks == 256 and n * 256 >= 8 * len(ext) * -(-most // xcds)
+
+
+@pytest.mark.parametrize("batch,length,n_q,n_kv,ordered,stay", [  # at head_dim 128, 16 blocks of a request or more
+    (1, 4000, 32, 8, False, False), (2, 1981, 32, 4, False, False), (2, 3963, 16, 8, False, False), (2, 2176, 16, 2, False, False),
+    (1, 4100, 32, 8, True, True), (2, 2048, 32, 8, True, True), (3, 1365, 32, 8, True, True), (5, 1171, 16, 2, True, False), (2, 900, 32, 8, False, False)])
+def test_prompts_of_one_length(rounds, batch, length, n_q, n_kv, ordered, stay):
+    rc, n, blocks, heads = rounds([length] * batch, 0, n_q, n_kv, order=True)
+    assert rc == 0 and (heads > 0) is ordered and (n > 0) is stay
