@@ -90,3 +90,15 @@ def test_the_builtin_scratch_holds_every_size_whose_segments_fit_8_mib():
         beyond += segments <= 8 << 20
         assert segments > 8 << 20 or need <= scratch, (size, segments, need)
     assert beyond > 2
+
+
+@pytest.mark.parametrize("batch,heads,line", [  # the mean length from which the gated delta rule takes scratch memory
+    (1, 32, 352), (2, 32, 384), (3, 32, 384), (4, 32, 448), (5, 32, 256), (8, 32, 256), (9, 32, 128), (64, 32, 128),
+    (3, 4, 352), (4, 4, 432), (8, 4, 624), (10, 4, 704), (24, 4, 704), (5, 24, 496), (8, 16, 640), (32, 4, 768),
+    (16, 16, 256), (32, 8, 384), (64, 4, 512), (64, 8, 256), (40, 8, 128), (100, 8, 128)])
+def test_gated_delta_rule_from_a_mean_length_on(batch, heads, line):
+    from mini_sglang_amd_kernel import _lib
+
+    ask = _lib.load().msgl_gdn_state_workspace_bytes
+    assert ask(line * batch - 1, batch, heads, 0) == 0 and ask(line * batch, batch, heads, 0) > 0
+    assert ask(line * batch, batch, heads, 1) == 0
