@@ -182,10 +182,9 @@ static thread_local int t_force_rows = 0;  // benchmarking switch, one value per
 // their mean, 320-384 even 1.01, ragged 0.97, 384-448 0.985 and 0.93; four, whose pairs of workgroups fill the chip in one round, even
 // 320-384 1.06, 384-448 1.01, 512-640 0.975, ragged 0.85-1.00; five to eight even 128-192 0.94-1.10, 192-256 0.91-1.05, 256-320 0.93, ragged
 // 0.96 and one long 0.68 in all of these; more 96-128 0.99 (up to 1.03), 128-192 0.97, 0.96 and 0.74.  The lines lie where even ones do not
-// lose either.  Few heads a request bring more requests to as many workgroups: each of those finds its place among them first, 3 to 6 us for 32
-// to 64, and even ones that fill the chip in halves have little to gain (32 requests of 452 tokens, 4 heads, 43.6 in one launch and 49.6 in
-// two, 64 of 319 69 and 75, 10 of 440 at 4 heads 27 and 31), so the lines go up with them.  750 launches at 2-128 heads, two launches by one: those
-// beyond the lines 0.903 (geometric mean of 583, worst 1.01), those that the requests' number leaves behind 0.991 of 167.
+// lose either.  Few heads a request bring more requests to as many workgroups, and even ones then lose (us, in one launch and in two: 32 of
+// 452 tokens, 4 heads, 43.6 and 49.6, 64 of 319 69 and 75, 10 of 445 29.6 and 33.6), so the lines go up with the requests' number.  750 launches at
+// 2-128 heads, two launches by one: those beyond the lines 0.903 (geometric mean of 583, worst 1.01), those that this leaves behind 0.991 of 167.
 // us: one of 4000 208 -> 159, eight of 200-1600 148 -> 139, 2060 among five of 100-260 150 -> 91.  A request and 32 heads
 // have 640 KiB for every 64 tokens; a launch that would need more than 2 GiB goes without.
 size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token) {
