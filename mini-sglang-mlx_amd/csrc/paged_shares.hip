@@ -437,7 +437,10 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
 // workgroup too many 81 21.8 -> 27.8 (33); head_dim 256 72 32.4 -> 25.6 (9), 134 40.6 -> 33.0 (31), 237 58.4 -> 66.8 (17).  One long request
 // among short ones gains as much (64, 15 requests, the longest 9.2 K, 20.5 -> 17.6; head_dim 256 155, 19, 24.7 K 44.5 -> 38.5), but
 // not where several heads go to a workgroup (177, 48, 14 K 36.0 -> 39.7), nor few requests with many columns, whose last shares
-// have most to put together (59, 2 requests, 40 columns 28.4 -> 35.1).
+// have most to put together (59, 2 requests, 40 columns 28.4 -> 35.1, 62, 4 requests, 24 columns 25.9 -> 29.1), nor shares twice as long as
+// a request on average, most of which take a whole request (73, 26 requests, one of them 7.5 K, 22.3 -> 24.0, with keys from memory 41.1 -> 45.8).
+// 502 launches beyond the first lines with 1-48 columns, shares by segments: with keys in the last-level cache 0.883 (geometric mean; worst
+// 1.04), with keys from memory 0.957 (1.05); 18 that the last two conditions leave out 0.926 (1.13) and 0.986 (1.11).
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
@@ -451,7 +454,7 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
   if (shares * (double)head_groups > device_cus() || batch * ((mean + len - 1) / len) * head_groups > device_cus()) return false;
   if (head_dim == 256) return units >= 24 && len * plan.heads_wg <= 1024 && mb <= 256;
   // (at 128 one request's 16 shares leave most of the chip idle and get long: 8.7 K keys 16.4 -> 15.2, 26.5 K 26.7 -> 28.1)
-  if (units < 32 && (cols > 16 || (units < 12 && mean > 12288))) return false;
+  if ((units < 48 && cols > 16) || (units < 12 && mean > 12288) || len > 2 * mean) return false;
   return len * plan.heads_wg <= 1536 && mb <= (units > device_cus() ? 128 : 208);
 }
 

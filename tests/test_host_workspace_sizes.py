@@ -102,3 +102,16 @@ def test_gated_delta_rule_from_a_mean_length_on(batch, heads, line):
     ask = _lib.load().msgl_gdn_state_workspace_bytes
     assert ask(line * batch - 1, batch, heads, 0) == 0 and ask(line * batch, batch, heads, 0) > 0
     assert ask(line * batch, batch, heads, 1) == 0
+
+
+@pytest.mark.parametrize("batch,kv,heads,q,shares", [  # beyond the first lines of the shares (csrc/paged_shares.hip)
+    (26, 18746, (32, 8, 128), 1, False), (32, 18048, (64, 8, 128), 1, False), (28, 18060, (32, 8, 128), 1, False),  # shares of 1536 keys
+    (19, 28310, (16, 8, 128), 1, True), (39, 28509, (32, 8, 128), 1, True),
+    (4, 15904, (32, 8, 128), 6, False), (5, 26780, (32, 8, 128), 6, False), (6, 26780, (32, 8, 128), 6, True), (4, 15904, (32, 8, 128), 4, True)])
+def test_launches_that_go_in_shares(batch, kv, heads, q, shares):
+    from mini_sglang_amd_kernel import _lib
+
+    lib, (n_q, n_kv, d) = _lib.load(), heads
+    if q == 1:  # with norm and rotary embedding a decode step is one launch where it goes in shares
+        assert (lib.msgl_decode_step_workspace_bytes(batch, kv, n_q, n_kv, d, 1) > 0) is shares
+    assert (lib.msgl_extend_step_workspace_bytes(batch, q * batch, kv, n_q, n_kv, d, q, 0, 0) > 0) is shares
