@@ -12,7 +12,7 @@ from test_gpu_gdn_chunk import _inputs
 pytestmark = pytest.mark.gpu
 
 
-def _launch(x, lengths, hk, hv, state, workspace):
+def _launch(x, lengths, hk, hv, state, workspace, short=0):
     from mini_sglang_amd_kernel import _lib
 
     lib, total, batch = _lib.load(), sum(lengths), len(lengths)
@@ -21,6 +21,7 @@ def _launch(x, lengths, hk, hv, state, workspace):
     y = torch.full((total, hv, 128), 7.0, dtype=torch.bfloat16, device=state.device)
     need = lib.msgl_gdn_state_workspace_bytes(total, batch, hv, 0)
     assert need > 0
+    need -= short
     ws = torch.full((need,), 0xff, dtype=torch.uint8, device=state.device) if workspace else None  # NaN wherever it is not written
     rc = lib.msgl_gdn_state_inplace_in(*(x[n].data_ptr() for n in ("q", "k", "v", "g", "beta")), state.data_ptr(), ids.data_ptr(),
                                        ip.data_ptr(), y.data_ptr(), total, batch, hk, hv, 128, 128, state.shape[0], state.stride(0),
@@ -28,6 +29,9 @@ def _launch(x, lengths, hk, hv, state, workspace):
                                        need if workspace else 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     torch.cuda.synchronize()
+    # the first request has tokens: in two launches the record of its first chunk is there, and nothing where the room is too small
+    assert ws is None or bool((ws[:20480] == 0xff).all()) is (short > 0)
+    assert short == 0 or bool((ws == 0xff).all())
     return y, state
 
 
@@ -56,6 +60,8 @@ def test_two_launches_are_one(gpu, lengths, hk, hv, what):
     y2, s2 = _launch(x, lengths, hk, hv, start.clone(), True)
     assert torch.equal(_bits(y2), _bits(y1)) and torch.equal(_bits(s2), _bits(s1))
     assert what is not None or bool(y2.isfinite().all() and s2.isfinite().all())
+    y3, s3 = _launch(x, lengths, hk, hv, start.clone(), True, short=1)
+    assert torch.equal(_bits(y3), _bits(y1)) and torch.equal(_bits(s3), _bits(s1))
 
 
 @pytest.mark.parametrize("lengths", [[385], [130, 1300, 64]])

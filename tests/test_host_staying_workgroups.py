@@ -13,9 +13,15 @@ PROGRAM = r"""
 namespace msgl { long long* clock_probe() { return nullptr; } }
 int main() {
   msgl::PrefillArgs a{};
-  long long batch, total_q, total_kv, n_q, n_kv, longest, head_dim, window, cross;
-  while (std::scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld", &batch, &total_q, &total_kv, &n_q, &n_kv, &longest, &head_dim, &window,
-                    &cross) == 9) {
+  long long batch, total_q, total_kv, n_q, n_kv, longest, head_dim, window, cross, row_stride;
+  static const int32_t slot = 0;
+  while (std::scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld %lld", &batch, &total_q, &total_kv, &n_q, &n_kv, &longest, &head_dim, &window,
+                    &cross, &row_stride) == 10) {
+    a.new_tokens = msgl::NewTokens{};
+    if (row_stride > 0) {  // the launch stores its rows
+      a.new_tokens.out_loc = &slot; a.new_tokens.rows = total_q;
+      a.new_tokens.k_stride0 = n_kv * head_dim; a.new_tokens.v_stride0 = row_stride;
+    }
     a.window = window; a.is_cross = (int)cross;
     a.batch = batch; a.total_q = total_q; a.total_kv = total_kv; a.n_q = n_q; a.n_kv = n_kv; a.max_len_extend = (int)longest;
     a.head_dim = head_dim; a.num_slots = 1 << 20; a.k_stride0 = a.v_stride0 = n_kv * head_dim; a.key_splits = 1; a.by_length = 1;
@@ -23,7 +29,7 @@ int main() {
     int64_t blocks = 0;
     bool wide = false;
     const int rc = msgl::make_prefill_params(a, p, blocks, wide, msgl::prefill_block_rows(head_dim));
-    std::printf("%d %d %lld %d\n", rc, (int)p.length_rounds, (long long)blocks, (int)p.length_heads);
+    std::printf("%d %d %lld %d %d\n", rc, (int)p.length_rounds, (long long)blocks, (int)p.length_heads, (int)wide);
   }
 }
 """
@@ -47,8 +53,8 @@ def rounds(tmp_path_factory):
                     "-isystem", "/opt/rocm/include", str(src), "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-o", str(exe)],
                    check=True)
 
-    def ask(ext, cached, n_q, n_kv, head_dim=128, window=0, cross=False, order=False):
-        line = f"{len(ext)} {sum(ext)} {sum(ext) + cached * len(ext)} {n_q} {n_kv} {max(ext)} {head_dim} {window} {int(cross)}\n"
+    def ask(ext, cached, n_q, n_kv, head_dim=128, window=0, cross=False, order=False, row_stride=0):
+        line = f"{len(ext)} {sum(ext)} {sum(ext) + cached * len(ext)} {n_q} {n_kv} {max(ext)} {head_dim} {window} {int(cross)} {row_stride}\n"
         out = subprocess.run([str(exe)], input=line, check=True, capture_output=True, text=True).stdout.split()
         return [int(x) for x in out][:None if order else 3]
     return ask
@@ -90,5 +96,16 @@ def test_rounds_of_head_dim_256(rounds, ext, cached, n_q, n_kv, window, cross, s
     (1, 4000, 32, 8, False, False), (2, 1981, 32, 4, False, False), (2, 3963, 16, 8, False, False), (2, 2176, 16, 2, False, False),
     (1, 4100, 32, 8, True, True), (2, 2048, 32, 8, True, True), (3, 1365, 32, 8, True, True), (5, 1171, 16, 2, True, False), (2, 900, 32, 8, False, False)])
 def test_prompts_of_one_length(rounds, batch, length, n_q, n_kv, ordered, stay):
-    rc, n, blocks, heads = rounds([length] * batch, 0, n_q, n_kv, order=True)
+    rc, n, blocks, heads, _ = rounds([length] * batch, 0, n_q, n_kv, order=True)
     assert rc == 0 and (heads > 0) is ordered and (n > 0) is stay
+
+
+@pytest.mark.parametrize("ext,n_q,n_kv,row_stride,stay,wide", [  # prompts whose rows the launch stores
+    ([510] * 8, 16, 8, 0, False, False), ([510] * 8, 16, 8, 1024, True, False),      # one round of blocks, no more than compute units
+    ([1015], 32, 8, 1024, False, False),                                             # half a round
+    ([4000], 32, 8, 0, False, False), ([4000], 32, 8, 1024, True, False),            # one request of many blocks, below two rounds
+    ([4000], 32, 8, 536864, True, False), ([4000], 32, 8, 536872, True, True),       # offsets of v's rows around 4 GiB
+    ([4000], 32, 8, (1 << 23) - 8, True, True), ([1015], 32, 8, 1 << 23, False, False)])
+def test_prompts_whose_rows_are_stored(rounds, ext, n_q, n_kv, row_stride, stay, wide):
+    rc, n, blocks, heads, offsets = rounds(ext, 0, n_q, n_kv, order=True, row_stride=row_stride)
+    assert rc == 0 and (n > 0) is stay and (not stay or blocks == 256) and bool(offsets) is wide
