@@ -238,14 +238,16 @@ MSGL_API int msgl_paged_prefill_attention(const void* q, const void* k_cache, co
  * A prefill call's store inside its attention launch -- AttnBackend.forward for prefill metadata
  * (mini_sglang_mlx/attention/backend.py:129-172): what msgl_store_kv_cache on (k, v, out_loc) and
  * msgl_paged_prefill_attention behind it do.  For short query blocks (speculative verify,
- * drafts) and small launches of up to some hundred tokens a request: msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
+ * drafts), small launches of up to some hundred tokens a request, and at head_dim 128 prompts with nothing cached whose rows (up
+ * to 131072) fill most of a round of query blocks: msgl_extend_step_workspace_bytes is 0 for the sizes that take the two calls, and
  * msgl_extend_step refuses them (MSGL_ERR_SHAPE).
  *   q, k, v, out_loc: total_q rows each, in the order of qo_indptr; leading strides of k and v free, q
  *   contiguous; bf16.  Rows in front of qo_indptr[0] and behind qo_indptr[batch] belong to no request: their k and v
  *   are stored all the same
- * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; with short query blocks
- * the request then sees the rows themselves and not the pool.  Otherwise its rows are in the pool before it is read for that
- * request.  As with msgl_decode_step the caller guarantees that no slot of out_loc is listed for a request that
+ * As a rule a request's rows are its last keys and out_loc holds the slots listed for those; with short query blocks,
+ * and in prompts with nothing cached where this holds for all of the launch's rows, the request then sees the rows themselves and not
+ * the pool.  Otherwise its rows are in the pool before it is read for that request.  Every row is stored, also those of requests
+ * that see no key.  As with msgl_decode_step the caller guarantees that no slot of out_loc is listed for a request that
  * its row does not belong to, nor twice for its own, and makes the two calls for a batch with such slots.
  */
 MSGL_API size_t msgl_extend_step_workspace_bytes(int64_t batch, int64_t total_q, int64_t total_kv,

@@ -1,4 +1,4 @@
-// Pieces of the chunked gated delta rule that its kernels share (gdn_chunk.hip, gdn_systems.hip): operands in three bf16
+// Pieces of the chunked gated delta rule that its kernels share (gdn_chunk.hip, gdn_long.hip): operands in three bf16
 // parts, decay ratios, the inverse of a chunk's triangular system, the way through a request token after token.
 #pragma once
 #include <algorithm>

@@ -9,10 +9,11 @@
 // gdn_systems_kernel: one workgroup per chunk and value head; 17 us for 63 chunks of 32 heads, 29 us for 130 (before its 15 KiB of A
 // and inverses shared their place with K and T and three workgroups more fitted a compute unit: 21 and 37).  Bound by the
 // round trips to memory in front of its 5 K cycles of work (its request, K, the gates), then by its stores (3 TB/s).
-// gdn_serial_kernel: quarters by the chain of a state wave, 4.5 K cycles of which 2.6 K are matrix instructions; halves where many
-// requests fill the chip by the matrix pipe at the power limit (1.0 PFLOP/s of bf16 products, 1.75 GHz).
+// gdn_serial_kernel: quarters by the chain of a state wave, 4.5 K cycles of which 2.6 K are matrix instructions, at 2.3 GHz (the pipe is
+// busy for 22 % of the SIMD cycles with one request, 43 % with the four below); halves where many requests fill the chip by the
+// matrix pipe: 1.12-1.15 PFLOP/s of bf16 products at 2.1 GHz, where a large product reaches 1.24.
 //
-// Both against the one launch, us: one request of 4005 tokens 208 -> 159; of 992, 1581, 4005 and 1601 tokens 209 -> 177; 2000 among five
+// Both against the one launch, us: one request of 4005 tokens 208 -> 159; of 992, 1581, 4005 and 1601 tokens 232 -> 183; 2000 among five
 // short ones 146 -> 95; eight of 1000 158 -> 156.
 #include "gdn_chunk_tiles.h"
 

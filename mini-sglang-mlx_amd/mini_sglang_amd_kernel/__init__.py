@@ -283,7 +283,9 @@ def extend_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
                 sm_scale: float, max_len_extend: int, is_cross_attention: bool = False,
                 sliding_window_size: int = 0, own_slots: bool = True) -> Optional[torch.Tensor]:
     """``store_kv_cache`` of the queries' own rows of k and v and ``paged_prefill_attention`` as one call: in one
-    launch where the query blocks are short or the launch is small, else as the two calls.  Returns the
+    launch where the query blocks are short, the launch is small, or at head_dim 128 its requests are prompts with nothing
+    cached that fill the chip (keys and values are then taken from the new rows, which are stored on the way, where
+    their slots are the listed ones), else as the two calls.  Returns the
     attention output, or ``None`` (nothing done) where the two calls have to be made by themselves: forms
     that need a copy, arguments that they refuse, index validation on.
 
