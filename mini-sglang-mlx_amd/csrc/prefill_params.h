@@ -255,13 +255,15 @@ constexpr int kMaxFreshRows = 1 << 17;  // of k and v, in a launch that takes it
 // 1-60 even, ragged and very uneven requests, staying against not, geometric mean, best and worst: 0.938, 0.76 and 1.10), nor where an average
 // request's blocks fill their XCDs by themselves (97 on up to 16 K cached: 0.981, 0.91 and 1.02).  Requests of fewer blocks on prefixes of any length
 // gain less on average, 0.993 of 359, and lose up to 1.42 where one is much longer than the others (42 requests of 87 tokens, 32 / 2 heads, one on
-// 1290 cached, 45.5 and 61.8 us) or small groups' blocks each wait for their own keys (32 of up to 1269 on 4057 each, 8 / 8, 1114 and 1465); so do
-// those whose rows see all keys, 0.978 of 80 and 1.25.
+// 1290 cached, 45.5 and 61.8 us) or small groups' blocks each wait for their own keys (32 of up to 1269 on 4057 each, 8 / 8, 1114 and 1465).  So do
+// those whose rows see all keys (80, 0.978 and 1.25), but for prompts with nothing cached and no window that cuts, the longest no longer than
+// three on average: 171, 0.950, 0.80 and 1.04, others up to 1.27.
 constexpr int kMinHalfRounds256 = 3;
 // XCDs that share a kv head's blocks, as a logarithm
 inline int prefill_log2_xcds(int64_t n_kv) { return n_kv == 1 ? 3 : n_kv == 2 ? 2 : n_kv == 4 ? 1 : 0; }
 inline bool prefill_may_stay_256(const PrefillArgs& a, int64_t group) {
-  if (a.is_cross) return false;
+  if (a.is_cross)
+    return a.total_kv == a.total_q && (a.window == 0 || a.window >= a.max_len_extend) && 3 * a.total_q >= a.batch * a.max_len_extend;
   if (a.total_kv == a.total_q || (a.window > 0 && a.total_kv >= a.batch * a.window)) return true;
   return a.total_q * group >= a.batch * ((kComputeUnits / 8 * kPrefillBlockRows256) << prefill_log2_xcds(a.n_kv));
 }

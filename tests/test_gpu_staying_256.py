@@ -34,6 +34,7 @@ CASES = [  # q heads, kv heads, extends, cached, window, cross, every third requ
     (16, 1, _mixed(32, 300), [0] * 32, 0, False, False),
     (10, 2, _mixed(64, 300), [64 + (i * 17) % 90 for i in range(64)], 64, False, False),
     (32, 8, [1024, 1100], [300, 40], 0, False, False),
+    (16, 4, [200, 333, 128, 1] * 6, [0] * 24, 400, True, False),  # all keys seen
 ]
 
 

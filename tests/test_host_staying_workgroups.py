@@ -79,7 +79,8 @@ CASES_256 = [  # extends, tokens cached (mean), q heads, kv heads, window, all k
     ([698] * 22, 500, 8, 8, 2000, False, False),               # and one that they do not
     ([2048] * 4, 4000, 16, 4, 0, False, True), ([2047] * 4, 4000, 16, 4, 0, False, False),  # 32 blocks a request in an XCD
     ([2731] * 4, 4000, 24, 8, 0, False, True), ([1365] * 4, 4000, 24, 8, 0, False, False),
-    ([2048] * 4, 0, 16, 4, 0, True, False), ([2048] * 4, 0, 16, 4, 300, True, False), ([2048, 2000] * 2, 0, 16, 4, 300, False, True),
+    ([2048] * 4, 0, 16, 4, 0, True, True), ([2048] * 4, 0, 16, 4, 300, True, False), ([2048] * 4, 0, 16, 4, 2048, True, True),
+    ([2048] * 4, 10, 16, 4, 0, True, False), ([979] + [51] * 53, 0, 8, 8, 0, True, False), ([2048, 2000] * 2, 0, 16, 4, 300, False, True),
 ]
 
 
