@@ -172,6 +172,25 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
   return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
 }
 
+// A kernel's parameters come through the scalar cache, 64 bytes at a time, from memory that no cache of the compute unit has
+// seen: a wave that reads them where it needs them waits half a microsecond each time.  Called while the first load of a
+// kernel's own is under way, this has all the lines of the first BYTES asked for together.  (The registers are nobody's: only the lines are wanted.)
+template <int BYTES>
+__device__ __forceinline__ void fetch_parameters() {
+  static_assert(BYTES > 0 && BYTES <= 512, "eight lines");
+  const auto at = __builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int kLast = (BYTES - 4) & ~3;
+  constexpr auto line = [](int i) { return 64 * i < kLast ? 64 * i : kLast; };
+  uint32_t r0, r1, r2, r3, r4, r5, r6, r7;
+  asm volatile(
+      "s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
+      "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&s"(r0), "=&s"(r1), "=&s"(r2), "=&s"(r3), "=&s"(r4), "=&s"(r5), "=&s"(r6), "=&s"(r7)
+      : "s"(at), "n"(line(0)), "n"(line(1)), "n"(line(2)), "n"(line(3)), "n"(line(4)), "n"(line(5)), "n"(line(6)), "n"(line(7))
+      : "memory");
+}
+
 // Measurement aid: when `dst` is given, thread 0 of workgroup 0 leaves the shader cycles and the
 // 100 MHz wall ticks between its construction and its destruction (every way out of the kernel) in
 // dst[0], dst[1]: cycles / ticks x 0.1 is the shader clock in GHz while the kernel ran.  (Both
@@ -179,9 +198,11 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
 struct ClockProbe {
   long long* dst;
   long long c0, w0;
-  __device__ __forceinline__ explicit ClockProbe(long long* d)
-      : dst((d != nullptr && blockIdx.x == 0 && threadIdx.x == 0) ? d : nullptr), c0(0), w0(0) {
-    if (dst != nullptr) {
+  __device__ __forceinline__ explicit ClockProbe(long long* d) : dst(nullptr), c0(0), w0(0) {
+    if (blockIdx.x != 0) return;
+    asm volatile("");  // a branch of its own: the other workgroups do not wait for the parameter
+    if (d != nullptr && threadIdx.x == 0) {
+      dst = d;
       c0 = clock64();
       w0 = wall_clock64();
     }

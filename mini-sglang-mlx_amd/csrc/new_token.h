@@ -321,11 +321,11 @@ struct NewRows {
   bool listed;            // their slots are the ones listed
   uint32_t slot, id;      // lane i: slot of row i; slot id listed for its place
 
-  __device__ __forceinline__ NewRows(const SplitKvParams& params, const ReqInfo& req, Columns<D, NCT>& c, int b, int head)
+  __device__ __forceinline__ NewRows(const SplitKvParams& params, const ReqInfo& req, Columns<D, NCT>& c, int head)
       : p(params), r(req), columns(c), kvh(head), owner(false) {
     const int lane = lane_id();
-    q0 = p.qo_indptr[b];
-    n = p.qo_indptr[b + 1] - q0;
+    q0 = req.q_start;  // (a launch of shares covers the queries from the first on)
+    n = req.rows;
     last_keys = n > 0 && n <= kWave && r.prefix >= 0 && r.prefix + n == r.kv_len && r.hi > r.lo;
     end = last_keys ? max(min(r.hi, r.prefix), r.lo) : r.hi;
     slot = lane < n ? (uint32_t)p.nt.out_loc[q0 + lane] : 0u;

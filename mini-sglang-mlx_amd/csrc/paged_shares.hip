@@ -37,8 +37,41 @@ struct ShareParams {
   SplitKvParams s;
   unsigned long long* counts;  // [batch][head_groups]
   unsigned long long nonce;
-  int32_t share_len, share_waves, heads_wg, head_groups;
+  int32_t heads_wg, head_groups;
 };
+
+// What the way to a workgroup's share takes (see request_info()).  These are the kernel's first arguments, one by one, which
+// the launch leaves in scalar registers (-amdgpu-kernarg-preload-count, build.py).  Read where they were needed, the parameters were
+// some eight round trips of 0.2-0.5 us in a workgroup's 8 us, three of them in front of its first load; in registers, or fetched
+// together behind that load, with divisions that are multiplications: 28 layers of a step of 4 requests of 36-1022 tokens 269.7 ->
+// 246.2 us, 32 requests of 8 queries with a window of 1024 34.4 -> 33.5, 24 of 127-4095 tokens, 16 / 2 heads of 256, 27.1 -> 26.7.
+struct ShareStart {
+  const int32_t *kv_indptr, *qo_indptr, *prefix_lens;
+  int32_t batch, share_len, window, max_len_extend, q_cap, is_cross;
+  uint32_t len_magic, len_shift;  // x / share_len = high half of x * len_magic, >> len_shift
+  static constexpr int q_begin = 0;
+  __device__ __forceinline__ int shares_of(int keys) const {
+    return (int)(__umulhi((uint32_t)(keys + share_len - 1), len_magic) >> len_shift);
+  }
+};
+struct ShareShape {  // powers of two: waves on a head; head groups (kNoShift: they are none)
+  static constexpr uint32_t kNoShift = 255;
+  uint32_t bits;
+  __host__ __device__ ShareShape(uint32_t len_shift, uint32_t waves, uint32_t groups) : bits(len_shift | waves << 8 | groups << 16) {}
+  __host__ __device__ explicit ShareShape(uint32_t b) : bits(b) {}
+  __device__ __forceinline__ uint32_t len_shift() const { return bits & 0xffu; }
+  __device__ __forceinline__ uint32_t waves() const { return (bits >> 8) & 0xffu; }
+  __device__ __forceinline__ uint32_t groups() const { return bits >> 16; }
+};
+// ceil(a / b) of scalars, b > 0 and the result below 2^20 (the compiler's division is twice as long)
+__device__ __forceinline__ int ceil_div(int a, int b) {
+  int q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)b)));
+  const int rest = a - q * b;  // q is within one of a / b
+  if (rest > 0) ++q;
+  if (rest > b) ++q;
+  if (rest <= -b) --q;
+  return q;
+}
 
 __device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
   return (unsigned long long)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo);
@@ -51,19 +84,16 @@ __device__ __forceinline__ unsigned long long ld_agent(const unsigned long long*
 }
 
 // Share number `item` of the launch: its request, which of the request's shares it is, of how many.
-// All lanes must call; false past the last share.
-__device__ __forceinline__ bool find_share(const SplitKvParams& p, int share_len, int item, ReqInfo* r, int* b,
-                                           int* share, int* n_shares) {
+// All lanes must call; false past the last share.  The launch's other parameters are fetched while the first requests' lengths are.
+template <int PARAMETERS>
+__device__ __forceinline__ bool find_share(const ShareStart& p, int item, ReqInfo* r, int* b, int* share, int* n_shares) {
   const int lane = lane_id();
   int base = 0;
   for (int b0 = 0; b0 < p.batch; b0 += kWave) {
-    ReqInfo mine{};
-    int n = 0;
-    if (b0 + lane < p.batch) {
-      mine = request_info(p, b0 + lane);
-      // a request without visible keys has one empty share: its rows are zero
-      n = max((mine.hi - mine.lo + share_len - 1) / share_len, 1);
-    }
+    ReqInfo mine = request_info(p, min(b0 + lane, p.batch - 1));
+    if (b0 == 0) fetch_parameters<PARAMETERS>();
+    // a request without visible keys has one empty share: its rows are zero
+    const int n = b0 + lane < p.batch ? max(p.shares_of(mine.hi - mine.lo), 1) : 0;
     const int incl = wave_inclusive_scan(n);
     const int sum = __builtin_amdgcn_readlane(incl, kWave - 1);
     if (item < base + sum) {
@@ -77,6 +107,7 @@ __device__ __forceinline__ bool find_share(const SplitKvParams& p, int share_len
       r->prefix = __builtin_amdgcn_readlane(mine.prefix, src);
       r->lo = __builtin_amdgcn_readlane(mine.lo, src);
       r->hi = __builtin_amdgcn_readlane(mine.hi, src);
+      r->rows = __builtin_amdgcn_readlane(mine.rows, src);
       *b = b0 + src;
       *share = item - __builtin_amdgcn_readlane(first, src);
       *n_shares = __builtin_amdgcn_readlane(n, src);
@@ -93,8 +124,12 @@ struct Nothing {
 };
 
 template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
-__global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(ShareParams sp) {
+__global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
+    const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
+    int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams sp) {
   const SplitKvParams& p = sp.s;
+  const ShareShape shape(shape_bits);
+  const ShareStart start{kv_indptr, qo_indptr, prefix_lens, batch, share_len, window, max_len_extend, q_cap, is_cross, len_magic, shape.len_shift()};
   constexpr int VH = D / 128;
   constexpr int kCols = 16 * NCT;
   constexpr int kBlock = kCols * 8 + 8;  // floats of one block of 8 dims: [col][8], padded
@@ -105,16 +140,20 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   const int lane = lane_id();
   const int t16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int item = blockIdx.x / sp.head_groups;
-  const int hg = blockIdx.x - item * sp.head_groups;
-  const int sub = wave / sp.share_waves;  // which of the workgroup's kv heads
-  const int sw = wave - sub * sp.share_waves;
-  const int kvh = hg * sp.heads_wg + sub;
+  int item = blockIdx.x >> shape.groups(), hg = blockIdx.x & ((1u << shape.groups()) - 1);
+  if (shape.groups() == ShareShape::kNoShift) {
+    item = blockIdx.x / sp.head_groups;
+    hg = blockIdx.x - item * sp.head_groups;
+  }
+  const int share_waves = 1 << shape.waves();
+  const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
+  const int sw = wave & (share_waves - 1);
+  const int kvh = hg * (NW >> shape.waves()) + sub;
 
   ReqInfo r;
   int b, share, n_shares;
-  if (!find_share(p, sp.share_len, item, &r, &b, &share, &n_shares)) {  // the whole workgroup
-    // (behind the search, that the others do not wait for one more parameter: 0.2 us of 10)
+  constexpr int kParameters = 3 * 8 + 8 * 4 + sizeof(ShareParams);
+  if (!find_share<kParameters>(start, item, &r, &b, &share, &n_shares)) {  // the whole workgroup
     if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(p, p.nt, p.n_kv * D, threadIdx.x);
     return;
   }
@@ -122,20 +161,20 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   if (ncols == 0) return;
   Columns<D, NCT> c;
   // the keys that are walked: all, but for a prefill call's own new ones
-  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, b, kvh);
+  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, kvh);
   int hi = r.hi;
   if constexpr (NEW == kStoreRows) hi = new_rows.end;
   const int vis = hi - r.lo;
-  const int per = ((vis + n_shares - 1) / n_shares + 31) & ~31;
+  const int per = (ceil_div(vis, n_shares) + 31) & ~31;
   const int s_begin = min(r.lo + share * per, hi), s_end = min(s_begin + per, hi);
-  const int per_wave = ((per + sp.share_waves - 1) / sp.share_waves + 31) & ~31;
+  const int per_wave = (((per + share_waves - 1) >> shape.waves()) + 31) & ~31;
   const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
 
   unsigned long long* const cnt = sp.counts + (int64_t)b * sp.head_groups + hg;
   const unsigned long long fresh = sp.nonce << 16;
   // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
-  // for it: whoever finds the word not made yet makes it (below).
-  if (n_shares > 1 && share == 0 && threadIdx.x == 0) {
+  // for it: whoever finds the word not made yet makes it (below).  (The last wave, which has the fewest keys or none.)
+  if (n_shares > 1 && share == 0 && threadIdx.x == 64 * (NW - 1)) {
     unsigned long long seen = ld_agent(cnt);
     if ((seen >> 16) != sp.nonce)
       (void)__hip_atomic_compare_exchange_strong(cnt, &seen, fresh, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -148,7 +187,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     start_columns(p, r, kvh, 0, t_end, c);
     if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
   } else if constexpr (NEW == kStoreRows) {
-    new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == sp.share_waves - 1;
+    new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == share_waves - 1;
     start_columns(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
     new_rows.check();
     if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
@@ -201,7 +240,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   __syncthreads();
 
   constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column
-  const int threads = 64 * sp.share_waves;
+  const int threads = 64 * share_waves;
   const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols;
   // every wave's part of a quad is asked for before the first is used
   auto put_together = [&](auto waves) {
@@ -229,7 +268,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
       }
       acc *= (l > 0.f) ? 1.0f / l : 0.f;
       if (n_shares == 1) {
-        const int qi = col / p.group;
+        const int qi = query_of(p, col);
         uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4;
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(acc[0], acc[1]), pack_16x2<F16>(acc[2], acc[3])};
       } else {
@@ -242,9 +281,9 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
       }
     }
   };
-  if (sp.share_waves == NW) put_together(std::integral_constant<int, NW>{});
-  else if (sp.share_waves == NW / 2) put_together(std::integral_constant<int, NW / 2>{});
-  else if (sp.share_waves == NW / 4) put_together(std::integral_constant<int, NW / 4>{});
+  if (share_waves == NW) put_together(std::integral_constant<int, NW>{});
+  else if (share_waves == NW / 2) put_together(std::integral_constant<int, NW / 2>{});
+  else if (share_waves == NW / 4) put_together(std::integral_constant<int, NW / 4>{});
   else put_together(std::integral_constant<int, 1>{});
   if (n_shares == 1) return;
 
@@ -329,7 +368,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 #pragma unroll
       for (int i = 0; i < I; ++i) {
         if (it0 + i * threads >= quads) break;
-        const int col = (int)(row[i] - first), qi = col / p.group;
+        const int col = (int)(row[i] - first), qi = query_of(p, col);
         const f32x4_t o = acc[i] * ((l[i] > 0.f) ? 1.0f / l[i] : 0.f);
         uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4[i];
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(o[0], o[1]), pack_16x2<F16>(o[2], o[3])};
@@ -346,9 +385,15 @@ int nct_of(int64_t cols) { return (int)((cols + 15) / 16); }
 int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
 
 template <int D, int NCT, int NW>
-int launch_shape(const ShareParams& sp, unsigned blocks, hipStream_t stream) {
+int launch_shape(const ShareParams& sp, int share_len, unsigned blocks, hipStream_t stream) {
+  auto log2_of = [](uint32_t x) { return 31u - (uint32_t)__builtin_clz(x); };
+  // x / d for x < 2^31, d > 1: with 2^s the next power of two, m = ceil(2^(31 + s) / d), it is x m >> (31 + s)
+  const uint32_t d = (uint32_t)share_len, s = log2_of(d - 1) + 1;
+  const uint32_t magic = (uint32_t)(((1ull << (31 + s)) + d - 1) / d), groups = (uint32_t)sp.head_groups;
+  const ShareShape shape(s - 1, log2_of((uint32_t)NW / (uint32_t)sp.heads_wg), (groups & (groups - 1)) == 0 ? log2_of(groups) : ShareShape::kNoShift);
   auto launch = [&](auto narrow, auto wide) {
-    hipLaunchKernelGGL(sp.s.wide ? wide : narrow, dim3(blocks), dim3(64 * NW), 0, stream, sp);
+    hipLaunchKernelGGL(sp.s.wide ? wide : narrow, dim3(blocks), dim3(64 * NW), 0, stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
+                       sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
     return check_launch();
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
@@ -386,7 +431,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
   const int64_t slots = device_cus();  // a workgroup takes a CU
   int64_t heads = 1, len;
   if (t_force > 0) {
-    len = t_force & 0xfffff;
+    len = std::max<int64_t>(t_force & 0xfffff, 2);
     heads = t_force >> 20;
     if (heads < 1 || heads > nw || n_kv % heads != 0 || nw % heads != 0) heads = 1;
   } else {
@@ -478,17 +523,15 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   sp.s.part_o = reinterpret_cast<float*>(ws);
   sp.s.part_lse = sp.s.part_o + (size_t)plan.max_shares * (size_t)(a.n_kv * cols * a.head_dim);
   sp.nonce = next_launch_number();
-  sp.share_len = plan.share_len;
-  sp.share_waves = plan.share_waves;
   sp.heads_wg = plan.heads_wg;
   sp.head_groups = (int32_t)head_groups;
   fill_new_tokens(n, sp.s);
   sp.s.nt.blocks = (uint32_t)(plan.max_shares * head_groups);
   const int nct = nct_of(cols);
-  if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
-  if (nct == 1) return launch_shape<128, 1, 8>(sp, (unsigned)blocks, stream);
-  if (nct == 2) return launch_shape<128, 2, 4>(sp, (unsigned)blocks, stream);
-  return nct == 3 ? launch_shape<128, 3, 4>(sp, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
+  if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, plan.share_len, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
+  if (nct == 1) return launch_shape<128, 1, 8>(sp, plan.share_len, (unsigned)blocks, stream);
+  if (nct == 2) return launch_shape<128, 2, 4>(sp, plan.share_len, (unsigned)blocks, stream);
+  return nct == 3 ? launch_shape<128, 3, 4>(sp, plan.share_len, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
 }
 
 }  // namespace msgl

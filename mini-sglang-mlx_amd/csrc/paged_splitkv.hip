@@ -220,7 +220,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
       const int col = (ct0 + ct) * 16 + t16;
       if (col >= ncols) continue;
-      const int qi = col / p.group;
+      const int qi = query_of(p, col);
       const int hh = col - qi * p.group;
       if (whole) {
         uint16_t* orow = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + hh) * D;
@@ -730,6 +730,7 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   p.prefix_lens = a.prefix_lens;
   p.out = static_cast<uint16_t*>(a.out);
   p.group = (int32_t)(a.n_q / a.n_kv);
+  p.per_group = 65535u / (uint32_t)p.group + 1u;
   p.cols = p.group * a.max_len_extend;
   p.k_stride0 = a.k_stride0;
   p.v_stride0 = a.v_stride0;

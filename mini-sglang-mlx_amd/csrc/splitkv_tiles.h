@@ -31,6 +31,7 @@ struct SplitKvParams {
   int32_t is_cross, window;
   int32_t wide;  // pool byte offsets need 64 bits
   uint32_t max_slot;  // num_slots - 1: slot ids are clamped to it before they become addresses
+  uint32_t per_group;  // ceil(2^16 / group), see query_of()
   float scale_log2e;
   long long* clock_probe;  // measurement aid, see ClockProbe; nullptr: off
   struct {  // a decode step's new tokens (new_token.h); k == nullptr: none
@@ -53,21 +54,25 @@ struct ReqInfo {
   int32_t q_start, q_len;    // rows of q / out
   int32_t prefix;            // position of query 0
   int32_t lo, hi;            // keys [lo, hi) can be visible to some query of the request
+  int32_t rows;              // of q, those that this launch does not cover included
 };
 
-__device__ __forceinline__ ReqInfo request_info(const SplitKvParams& p, int b) {
+// P: SplitKvParams, or what of it this takes
+template <typename P>
+__device__ __forceinline__ ReqInfo request_info(const P& p, int b) {
   ReqInfo r;
   r.kv_start = p.kv_indptr[b];
   r.kv_len = p.kv_indptr[b + 1] - r.kv_start;
   if (r.kv_len < 0) r.kv_len = 0;
   if (p.qo_indptr == nullptr) {
     r.q_start = b;
-    r.q_len = 1;
+    r.q_len = r.rows = 1;
     r.prefix = r.kv_len - 1;
   } else {
     // this launch covers queries q_begin .. q_begin + max_len_extend - 1 of every request
     const int q0 = p.qo_indptr[b];
-    const int q_all = min(p.qo_indptr[b + 1] - q0, p.q_cap);
+    r.rows = p.qo_indptr[b + 1] - q0;
+    const int q_all = min(r.rows, p.q_cap);
     r.q_start = q0 + p.q_begin;
     r.q_len = max(min(q_all - p.q_begin, p.max_len_extend), 0);
     r.prefix = p.prefix_lens[b] + p.q_begin;
@@ -82,6 +87,9 @@ __device__ __forceinline__ ReqInfo request_info(const SplitKvParams& p, int b) {
   }
   return r;
 }
+
+// The query that a column belongs to, col / group: exact up to 64 columns and heads to a group (a division is 25 instructions).
+__device__ __forceinline__ int query_of(const SplitKvParams& p, int col) { return (int)((uint32_t)col * p.per_group >> 16); }
 
 template <int D>
 struct KvTile {
@@ -113,7 +121,7 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
   for (int ct = 0; ct < NCT; ++ct) {
     const int col = (ct0 + ct) * 16 + t16;
     const bool valid = col < ncols;
-    const int qi = valid ? col / p.group : 0;
+    const int qi = valid ? query_of(p, col) : 0;
     const int hh = valid ? col - qi * p.group : 0;
     const uint16_t* qrow =
         p.q + (int64_t)(r.q_start + qi) * p.q_stride0 + (kvh * p.group + hh) * D + g * 8;
