@@ -198,11 +198,9 @@ __device__ __forceinline__ void fetch_parameters() {
 struct ClockProbe {
   long long* dst;
   long long c0, w0;
-  __device__ __forceinline__ explicit ClockProbe(long long* d) : dst(nullptr), c0(0), w0(0) {
-    if (blockIdx.x != 0) return;
-    asm volatile("");  // a branch of its own: the other workgroups do not wait for the parameter
-    if (d != nullptr && threadIdx.x == 0) {
-      dst = d;
+  __device__ __forceinline__ explicit ClockProbe(long long* d)
+      : dst((d != nullptr && blockIdx.x == 0 && threadIdx.x == 0) ? d : nullptr), c0(0), w0(0) {
+    if (dst != nullptr) {
       c0 = clock64();
       w0 = wall_clock64();
     }

@@ -59,6 +59,20 @@ struct HeadLds {  // NORM: of one wave
   uint16_t row[17][D];  // the new key, the heads of the columns
   float cosines[D / 2], sines[D / 2];
 };
+// Where the new token of request b goes and, with NORM, its position: asked for, in vector registers until they are taken
+// (a value known to be the wave's would be waited for at once, to become a scalar).
+template <bool NORM>
+struct NewTokenIds {
+  int32_t slot_, position_ = 0;
+  __device__ __forceinline__ NewTokenIds(const SplitKvParams& p, int b) {
+    uint32_t at = (uint32_t)b;
+    pin(at);
+    slot_ = p.nt.out_loc[at];
+    if constexpr (NORM) position_ = p.nt.positions[at];
+  }
+  __device__ __forceinline__ uint32_t slot() const { return (uint32_t)__builtin_amdgcn_readfirstlane(slot_); }
+  __device__ __forceinline__ int position() const { return __builtin_amdgcn_readfirstlane(position_); }
+};
 template <int D, bool NORM, bool F16>
 struct NewToken {
   static constexpr int E = D / 32, KS = D / 32, VH = D / 128;
@@ -79,21 +93,21 @@ struct NewToken {
   u32x4_t krow[KS], vrow[VH][4];  // lane group g: dims 32 c + 8 g .. (as operand), hf 128 + 32 g + 8 i .. (as output)
   Half lo[kEarly], hi[kEarly], qwl, qwh, kwl, kwh;
 
-  __device__ __forceinline__ NewToken(const SplitKvParams& s, const ReqInfo& r, Columns<D, 1>& c, HeadLds<D>& l, int b, int head, bool own)
+  __device__ __forceinline__ NewToken(const SplitKvParams& s, const ReqInfo& r, Columns<D, 1>& c, HeadLds<D>& l, const NewTokenIds<NORM>& ids, int b,
+                                      int head, bool own)
       : sp(s), columns(c), lds(l), owner(own), kvh(head) {
     const int lane = lane_id();
-    // one round trip for all three, beside that of the first tile's slot ids
-    const int32_t *loc = sp.nt.out_loc + b, *last = r.kv_len > 0 ? sp.kv_indices + r.kv_start + r.kv_len - 1 : loc;
-    const int32_t* second = r.kv_len > 1 ? last - 1 : last;
-    slot = (uint32_t)*loc;
+    // one round trip for both, beside that of the first tile's slot ids
+    const int32_t* last = r.kv_len > 0 ? sp.kv_indices + r.kv_start + r.kv_len - 1 : sp.nt.out_loc + b;
     const uint32_t last_id = (uint32_t)*last;
-    before = *second;
+    before = *(r.kv_len > 1 ? last - 1 : last);
+    slot = ids.slot();
     elsewhere = (r.kv_len > 0) & (slot <= sp.max_slot) & (last_id != slot);
     seen = owner & (r.kv_len > 0) & (slot <= sp.max_slot) & (last_id == slot);
     q = sp.q + (int64_t)b * sp.q_stride0 + kvh * sp.group * D;
     k = sp.nt.k + (int64_t)b * sp.nt.k_stride0 + kvh * D;
     if constexpr (NORM) {
-      position = (float)sp.nt.positions[b];
+      position = (float)ids.position();
 #pragma unroll
       for (int i = 0; i < kEarly; ++i) head_of(i, lo[i], hi[i]);
       const int off = E * (lane & 15);
@@ -128,15 +142,21 @@ struct NewToken {
   // The wave's own writes to LDS before its reads: no barrier
   __device__ __forceinline__ static void own_writes() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+  // Sines and cosines of the position, which is there before the slot ids of the first tile are (at head_dim 128).
+  __device__ __forceinline__ void angles() {
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = lane_id(); i < D / 2; i += kWave) {
+        float sn, cs;
+        sincosf(rope_angle<D>(position, i, sp.nt.log2_base), &sn, &cs);
+        lds.cosines[i] = cs;
+        lds.sines[i] = sn;
+      }
+    }
+  }
   __device__ __forceinline__ void normalise() {
     const int lane = lane_id(), t16 = lane & 15, g = lane >> 4, off = E * t16;
-#pragma unroll
-    for (int i = lane; i < D / 2; i += kWave) {
-      float sn, cs;
-      sincosf(rope_angle<D>(position, i, sp.nt.log2_base), &sn, &cs);
-      lds.cosines[i] = cs;
-      lds.sines[i] = sn;
-    }
+    if constexpr (D != 128) angles();
     own_writes();
     float cs[E], sn[E];
 #pragma unroll

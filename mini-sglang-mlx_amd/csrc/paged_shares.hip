@@ -90,8 +90,12 @@ __device__ __forceinline__ bool find_share(const ShareStart& p, int item, ReqInf
   const int lane = lane_id();
   int base = 0;
   for (int b0 = 0; b0 < p.batch; b0 += kWave) {
-    ReqInfo mine = request_info(p, min(b0 + lane, p.batch - 1));
-    if (b0 == 0) fetch_parameters<PARAMETERS>();
+    const ReqInfo mine = request_info(p, min(b0 + lane, p.batch - 1), [&] {
+      if (b0 != 0) return;
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_parameters<PARAMETERS>();
+      __builtin_amdgcn_sched_barrier(0);
+    });
     // a request without visible keys has one empty share: its rows are zero
     const int n = b0 + lane < p.batch ? max(p.shares_of(mine.hi - mine.lo), 1) : 0;
     const int incl = wave_inclusive_scan(n);
@@ -136,7 +140,6 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   __shared__ __attribute__((aligned(16))) float part[NW][D / 8][kBlock];
   __shared__ float2 state[NW][kCols];  // (maximum, sum) of a wave's columns
   __shared__ int is_last;
-  const ClockProbe clock_probe_(p.clock_probe);
   const int lane = lane_id();
   const int t16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -157,6 +160,10 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(p, p.nt, p.n_kv * D, threadIdx.x);
     return;
   }
+  const ClockProbe clock_probe_(p.clock_probe);
+  // what the rest of the way begins with and only the request's number leads to
+  const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
+  __builtin_amdgcn_sched_barrier(0);
   const int ncols = r.q_len * p.group;
   if (ncols == 0) return;
   Columns<D, NCT> c;
@@ -170,6 +177,9 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   const int per_wave = (((per + share_waves - 1) >> shape.waves()) + 31) & ~31;
   const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
 
+  FirstIds ids{};
+  if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
+  __builtin_amdgcn_sched_barrier(0);
   unsigned long long* const cnt = sp.counts + (int64_t)b * sp.head_groups + hg;
   const unsigned long long fresh = sp.nonce << 16;
   // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
@@ -180,15 +190,12 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
       (void)__hip_atomic_compare_exchange_strong(cnt, &seen, fresh, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
   }
-
-  FirstIds ids{};
-  if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
   if constexpr (NEW == kStored) {
-    start_columns(p, r, kvh, 0, t_end, c);
+    start_columns<D, NCT, true, true>(p, r, kvh, 0, t_end, c);
     if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
   } else if constexpr (NEW == kStoreRows) {
     new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == share_waves - 1;
-    start_columns(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
+    start_columns<D, NCT, true, true>(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
     new_rows.check();
     if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
     else new_rows();
@@ -196,14 +203,15 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     static_assert(sizeof(HeadLds<D>) <= sizeof(part[0]), "a wave's heads have their place in its part of the partials");
     const int tail = r.kv_len - 1;
     const bool owner = r.kv_len > 0 ? t_begin <= tail && tail < t_end : share == 0 && sw == 0;
-    NewToken<D, NEW == kNormRopeStore, F16> token(p, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), b, kvh, owner);
+    NewToken<D, NEW == kNormRopeStore, F16> token(p, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), new_ids, b, kvh, owner);
+    if constexpr (D == 128) token.angles();
     int walk_end = t_end;
     if (token.seen) {
       walk_end = tail;
       end_ids(ids, t_begin, tail, token.before);
     }
     token.check();
-    start_columns<D, NCT, NEW != kNormRopeStore>(p, r, kvh, 0, walk_end, c);
+    start_columns<D, NCT, NEW != kNormRopeStore, true>(p, r, kvh, 0, walk_end, c);
     if constexpr (D == 256) {
       token();
       if (t_begin < walk_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, walk_end, ids, c, [] {});
@@ -239,9 +247,10 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   }
   __syncthreads();
 
-  constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column
+  constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column, the 16 bytes at 16 it of a share's rows
   const int threads = 64 * share_waves;
   const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols;
+  char* const rows_to = reinterpret_cast<char*>(p.part_o + row0 * D);
   // every wave's part of a quad is asked for before the first is used
   auto put_together = [&](auto waves) {
     constexpr int W = decltype(waves)::value;
@@ -272,7 +281,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
         uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4;
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(acc[0], acc[1]), pack_16x2<F16>(acc[2], acc[3])};
       } else {
-        unsigned long long* dst = reinterpret_cast<unsigned long long*>(p.part_o + (row0 + col) * D + d4);
+        unsigned long long* dst = reinterpret_cast<unsigned long long*>(rows_to + 16u * (uint32_t)it);
         st_agent(dst, pair_bits(acc[0], acc[1]));
         st_agent(dst + 1, pair_bits(acc[2], acc[3]));
         if (d4 == 0)
@@ -310,22 +319,23 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   if (!is_last) return;
   constexpr int I = NW == 4 ? 2 : 1;  // a thread's quads whose loads are in flight together
   const int64_t step = (int64_t)p.n_kv * p.cols;  // rows from one share to the next
-  const int64_t first = ((int64_t)(item - share) * p.n_kv + kvh) * p.cols;
+  const int64_t first = row0 - share * step;
+  const char* const rows_from = reinterpret_cast<const char*>(p.part_o + first * D);
+  const char* const lse_from = reinterpret_cast<const char*>(p.part_lse + first);
   const int quads = ncols * kQuads;
   // ... for as many shares as there are, by fours, or 16 (loads past the last one cost as much as the others:
-  // 16 for all of four shares 9.3 -> 9.8 us; 8 for more than 8 in turns 11.6 us against 11.2 at two of 3000 tokens)
+  // 16 for all of four shares 9.3 -> 9.8 us; 8 for more than 8 in turns 11.6 us against 11.2 at two of 3000 tokens).
+  // A share's rows are a scalar base, a thread's place in them is 32 bits: with 64-bit addresses to each load, issuing
+  // them took 1.5 K cycles, longer than they were under way.
   auto merge = [&](auto in_flight) {
     constexpr int U = decltype(in_flight)::value;
     for (int it0 = threadIdx.x - sub * threads; it0 < quads; it0 += I * threads) {
       float m[I], l[I];
       f32x4_t acc[I];
-      int64_t row[I];
-      int d4[I];
+      uint32_t at[I];
 #pragma unroll
       for (int i = 0; i < I; ++i) {
-        const int it = min(it0 + i * threads, quads - 1);  // past the end: the last quad again, not written
-        row[i] = first + it / kQuads;
-        d4[i] = (it % kQuads) * 4;
+        at[i] = (uint32_t)min(it0 + i * threads, quads - 1);  // past the end: the last quad again, not written
         m[i] = kNegInf;
         l[i] = 0.f;
         acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -334,16 +344,18 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
         float lse[I][U];
         unsigned long long lo[I][U], hi[I][U];
 #pragma unroll
-        for (int i = 0; i < I; ++i)
+        for (int u = 0; u < U; ++u) {  // shares past the last one: the last again, with weight 0
+          const int64_t rows = min(s0 + u, n_shares - 1) * step;
+          const char* const from = rows_from + rows * (D * 4);
+          const char* const lse_at = lse_from + rows * 4;
 #pragma unroll
-          for (int u = 0; u < U; ++u) {  // shares past the last one: the last again, with weight 0
-            const int64_t at = row[i] + min(s0 + u, n_shares - 1) * step;
-            const unsigned long long* src = reinterpret_cast<const unsigned long long*>(p.part_o + at * D + d4[i]);
-            lse[i][u] = __hip_atomic_load(p.part_lse + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lo[i][u] = ld_agent(src);
-            hi[i][u] = ld_agent(src + 1);
+          for (int i = 0; i < I; ++i) {
+            lse[i][u] = __hip_atomic_load(reinterpret_cast<const float*>(lse_at + 4u * (at[i] / kQuads)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lo[i][u] = ld_agent(reinterpret_cast<const unsigned long long*>(from + 16u * at[i]));
+            hi[i][u] = ld_agent(reinterpret_cast<const unsigned long long*>(from + 16u * at[i]) + 1);
             if (s0 + u >= n_shares) lse[i][u] = kNegInf;
           }
+        }
 #pragma unroll
         for (int i = 0; i < I; ++i) {
           float m_new = m[i];
@@ -368,9 +380,9 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 #pragma unroll
       for (int i = 0; i < I; ++i) {
         if (it0 + i * threads >= quads) break;
-        const int col = (int)(row[i] - first), qi = query_of(p, col);
+        const int col = (int)(at[i] / kQuads), qi = query_of(p, col);
         const f32x4_t o = acc[i] * ((l[i] > 0.f) ? 1.0f / l[i] : 0.f);
-        uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4[i];
+        uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + 4 * (at[i] % kQuads);
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(o[0], o[1]), pack_16x2<F16>(o[2], o[3])};
       }
     }

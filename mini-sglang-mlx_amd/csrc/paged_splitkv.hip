@@ -220,7 +220,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
       const int col = (ct0 + ct) * 16 + t16;
       if (col >= ncols) continue;
-      const int qi = query_of(p, col);
+      const int qi = col / p.group;
       const int hh = col - qi * p.group;
       if (whole) {
         uint16_t* orow = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + hh) * D;

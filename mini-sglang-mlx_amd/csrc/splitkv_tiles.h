@@ -57,7 +57,18 @@ struct ReqInfo {
   int32_t rows;              // of q, those that this launch does not cover included
 };
 
-// P: SplitKvParams, or what of it this takes
+// P: SplitKvParams, or what of it this takes.
+template <typename P>
+__device__ __forceinline__ void visible_range(const P& p, ReqInfo& r) {
+  // first query has the lowest window floor, last query the highest causal limit
+  r.lo = (p.window > 0) ? max(0, r.prefix - p.window + 1) : 0;
+  r.lo &= ~15;
+  r.hi = p.is_cross ? r.kv_len : min(r.kv_len, r.prefix + r.q_len);
+  if (r.q_len <= 0 || r.hi <= r.lo) {
+    r.lo = 0;
+    r.hi = 0;
+  }
+}
 template <typename P>
 __device__ __forceinline__ ReqInfo request_info(const P& p, int b) {
   ReqInfo r;
@@ -77,14 +88,25 @@ __device__ __forceinline__ ReqInfo request_info(const P& p, int b) {
     r.q_len = max(min(q_all - p.q_begin, p.max_len_extend), 0);
     r.prefix = p.prefix_lens[b] + p.q_begin;
   }
-  // first query has the lowest window floor, last query the highest causal limit
-  r.lo = (p.window > 0) ? max(0, r.prefix - p.window + 1) : 0;
-  r.lo &= ~15;
-  r.hi = p.is_cross ? r.kv_len : min(r.kv_len, r.prefix + r.q_len);
-  if (r.q_len <= 0 || r.hi <= r.lo) {
-    r.lo = 0;
-    r.hi = 0;
-  }
+  visible_range(p, r);
+  return r;
+}
+// The same with meanwhile() called once the loads are under way.  (A decode call loads its lengths again for what it has not:
+// a branch around those loads would be waited in front of.)
+template <typename P, typename Meanwhile>
+__device__ __forceinline__ ReqInfo request_info(const P& p, int b, Meanwhile&& meanwhile) {
+  ReqInfo r;
+  const bool decode = p.qo_indptr == nullptr;
+  const int32_t *qo_indptr = decode ? p.kv_indptr : p.qo_indptr, *prefix_lens = decode ? p.kv_indptr : p.prefix_lens;
+  r.kv_start = p.kv_indptr[b];
+  const int kv_end = p.kv_indptr[b + 1], q0 = qo_indptr[b], q_end = qo_indptr[b + 1], prefix = prefix_lens[b];
+  meanwhile();
+  r.kv_len = max(kv_end - r.kv_start, 0);
+  r.rows = decode ? 1 : q_end - q0;
+  r.q_start = decode ? b : q0 + p.q_begin;
+  r.q_len = decode ? 1 : max(min(min(r.rows, p.q_cap) - p.q_begin, p.max_len_extend), 0);
+  r.prefix = decode ? r.kv_len - 1 : prefix + p.q_begin;
+  visible_range(p, r);
   return r;
 }
 
@@ -109,8 +131,8 @@ struct Columns {
 };
 
 // Columns ct0 * 16 .. of kv head `kvh` of request `r`, for the keys before `t_end`.  LOAD_Q: the Q operand from memory
-// (else it is left to the caller).
-template <int D, int NCT, bool LOAD_Q = true>
+// (else it is left to the caller).  SMALL: the launch is one of shares (the long walks' kernels have no register to spare for query_of()).
+template <int D, int NCT, bool LOAD_Q = true, bool SMALL = false>
 __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqInfo& r, int kvh, int ct0,
                                               int t_end, Columns<D, NCT>& c_) {
   constexpr int KS = D / 32, VH = D / 128;
@@ -121,7 +143,7 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
   for (int ct = 0; ct < NCT; ++ct) {
     const int col = (ct0 + ct) * 16 + t16;
     const bool valid = col < ncols;
-    const int qi = valid ? query_of(p, col) : 0;
+    const int qi = !valid ? 0 : SMALL ? query_of(p, col) : col / p.group;
     const int hh = valid ? col - qi * p.group : 0;
     const uint16_t* qrow =
         p.q + (int64_t)(r.q_start + qi) * p.q_stride0 + (kvh * p.group + hh) * D + g * 8;
