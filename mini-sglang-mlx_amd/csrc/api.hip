@@ -293,22 +293,31 @@ int msgl_paged_decode_attention_noalloc(const void* q, const void* k_cache, cons
                           k_cache_stride0, v_cache_stride0, sm_scale, max_kv_splits, dtype, stream);
 }
 
-size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads, int64_t num_kv_heads,
-                                        int64_t head_dim, int32_t norm_rope) {
+// The workspace of a decode step in one launch, 0: it is not the way; `plan`: of its shares, share_len 0 where it goes in segments.
+static size_t decode_step_route(int64_t batch, int64_t total_kv, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
+                                bool norm_rope, msgl::SharePlan* plan) {
   if (batch <= 0 || total_kv < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
       num_q_heads / num_kv_heads > 16 || (head_dim != 128 && head_dim != 256))
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
-  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
-  if (!msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group)) {
+  *plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
+  if (!msgl::shares_preferred(*plan, batch, total_kv, num_kv_heads, head_dim, group)) {
     // norm and rotary embedding would be made anew by every segment of a request: 3.5 us of a launch of their own is
     // less on the launches that go in segments.  On large ones the store's launch hides behind the start of the next,
     // and its part of the segments is paid by the slowest of them; us, store in front against inside, by MiB of keys and
     // values: 22 23.3 and 20.9 (2 requests, 24 / 4 heads of 256), 113 24.2 and 22.4 (1), 183 38.2 and 37.0 (68); 281
     // 53.5 and 53.6 (16 requests), 366 81.2 and 83.4 (128), 625 126.8 and 127.8 (64); at head_dim 256 312 65.3 and 63.5 (16)
     if (norm_rope || (total_kv * num_kv_heads * head_dim * 4 >> 20) > (head_dim == 256 ? 384 : 192)) return 0;
+    plan->share_len = 0;
+    return msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, 1, segments(total_kv, num_kv_heads, head_dim, group));
   }
-  return msgl_paged_decode_workspace_bytes(batch, total_kv, num_q_heads, num_kv_heads, head_dim);
+  return msgl::share_workspace_bytes(*plan, batch, num_kv_heads, head_dim, group);
+}
+
+size_t msgl_decode_step_workspace_bytes(int64_t batch, int64_t total_kv, int64_t num_q_heads, int64_t num_kv_heads,
+                                        int64_t head_dim, int32_t norm_rope) {
+  msgl::SharePlan plan{};
+  return decode_step_route(batch, total_kv, num_q_heads, num_kv_heads, head_dim, norm_rope != 0, &plan);
 }
 
 int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stride0, int64_t k_stride0, int64_t v_stride0,
@@ -333,7 +342,8 @@ int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stri
   if (!aligned16(k) || !aligned16(v) || q_stride0 % 8 || k_stride0 % 8 || v_stride0 % 8 || !aligned16(q_weight) ||
       !aligned16(k_weight))
     return MSGL_ERR_ALIGNMENT;
-  const size_t need = msgl_decode_step_workspace_bytes(batch, total_kv, num_q_heads, num_kv_heads, head_dim, q_weight != nullptr);
+  msgl::SharePlan plan{};
+  const size_t need = decode_step_route(batch, total_kv, num_q_heads, num_kv_heads, head_dim, q_weight != nullptr, &plan);
   if (need == 0) return MSGL_ERR_SHAPE;
   if (!workspace || workspace_bytes < need || !aligned16(workspace)) return MSGL_ERR_WORKSPACE;
   msgl::SplitKvArgs a{};
@@ -368,9 +378,7 @@ int msgl_decode_step(const void* q, const void* k, const void* v, int64_t q_stri
   tokens.rows = batch;
   tokens.eps = rms_norm_eps;
   tokens.rope_base = rope_base;
-  const msgl::SharePlan plan = shares_for(batch, total_kv, 0, num_kv_heads, head_dim, group);
-  if (msgl::shares_preferred(plan, batch, total_kv, num_kv_heads, head_dim, group))
-    return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
+  if (plan.share_len > 0) return msgl::launch_shares(a, tokens, plan, static_cast<hipStream_t>(stream));
   a.n_seg = segments(total_kv, num_kv_heads, head_dim, group);
   a.min_seg = min_segment(head_dim);
   return msgl::launch_splitkv(a, tokens, static_cast<hipStream_t>(stream));

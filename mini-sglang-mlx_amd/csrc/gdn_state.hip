@@ -244,15 +244,10 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)blocks), block(256);
   // decode has one token per request: nothing to look ahead to
   if (p.single_token) {
-    if (r == 4) hipLaunchKernelGGL((gdn_state_kernel<4, 1>), grid, block, 0, stream, p);
-    else if (r == 2) hipLaunchKernelGGL((gdn_state_kernel<2, 1>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((gdn_state_kernel<1, 1>), grid, block, 0, stream, p);
+    return launch_kernel(r == 4 ? gdn_state_kernel<4, 1> : r == 2 ? gdn_state_kernel<2, 1> : gdn_state_kernel<1, 1>, grid, block, stream, p);
   } else {
-    if (r == 4) hipLaunchKernelGGL((gdn_state_kernel<4, 8>), grid, block, 0, stream, p);
-    else if (r == 2) hipLaunchKernelGGL((gdn_state_kernel<2, 8>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((gdn_state_kernel<1, 8>), grid, block, 0, stream, p);
+    return launch_kernel(r == 4 ? gdn_state_kernel<4, 8> : r == 2 ? gdn_state_kernel<2, 8> : gdn_state_kernel<1, 8>, grid, block, stream, p);
   }
-  return check_launch();
 }
 
 }  // namespace msgl

@@ -1772,17 +1772,10 @@ int launch_prefill_merge(const PrefillParams& p, int head_dim, hipStream_t strea
   const dim3 grid((unsigned)((rows + 7) / 8), (unsigned)p.batch);
   if (p.ragged_tiles > 0) {
     if (p.req_units == nullptr) return MSGL_OK;  // no request can have a second share
-    if (head_dim == 256) hipLaunchKernelGGL((prefill_ragged_merge_kernel<256>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((prefill_ragged_merge_kernel<128>), grid, dim3(256), 0, stream, p);
-    return check_launch();
+    return launch_kernel(head_dim == 256 ? prefill_ragged_merge_kernel<256> : prefill_ragged_merge_kernel<128>, grid, dim3(256), stream, p);
   }
-  if (head_dim == 256)
-    hipLaunchKernelGGL((prefill_merge_kernel<256>), grid, dim3(256), 0, stream, p.part_o, p.part_lse,
+  return launch_kernel(head_dim == 256 ? prefill_merge_kernel<256> : prefill_merge_kernel<128>, grid, dim3(256), stream, p.part_o, p.part_lse,
                        p.qo_indptr, p.out, p.part_rows, p.n_q, p.n_ksplit, p.max_len_extend);
-  else
-    hipLaunchKernelGGL((prefill_merge_kernel<128>), grid, dim3(256), 0, stream, p.part_o, p.part_lse,
-                       p.qo_indptr, p.out, p.part_rows, p.n_q, p.n_ksplit, p.max_len_extend);
-  return check_launch();
 }
 
 // benchmarking switch, one value per host thread (see msgl_set_tuning): 0 the ping-pong kernel,
@@ -1809,9 +1802,9 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
     n_blocks += kRestBlocks;
   }
   const dim3 grid((unsigned)n_blocks);
+  int launched;
   if (tile_variant() != 0) {
-    if (wide) hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, true>), grid, dim3(512), 0, stream, p);
-    else hipLaunchKernelGGL((prefill_tile_kernel<128, 1, 8, false>), grid, dim3(512), 0, stream, p);
+    launched = launch_kernel(wide ? prefill_tile_kernel<128, 1, 8, true> : prefill_tile_kernel<128, 1, 8, false>, grid, dim3(512), stream, p);
   } else {
     auto* const kernel = p.gangs > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kGang> : prefill_pingpong_kernel<false, Order::kGang>)
                          : p.length_rounds > 0 && p.nt.out_loc != nullptr
@@ -1819,9 +1812,8 @@ int launch_prefill_tile(const PrefillArgs& a, hipStream_t stream) {
                          : p.length_rounds > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kStay> : prefill_pingpong_kernel<false, Order::kStay>)
                          : p.length_heads > 0 ? (wide ? prefill_pingpong_kernel<true, Order::kLength> : prefill_pingpong_kernel<false, Order::kLength>)
                                               : (wide ? prefill_pingpong_kernel<true, Order::kBatch> : prefill_pingpong_kernel<false, Order::kBatch>);
-    hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, p);
+    launched = launch_kernel(kernel, grid, dim3(512), stream, p);
   }
-  const int launched = check_launch();
   if (launched != MSGL_OK || (p.n_ksplit == 1 && p.ragged_tiles == 0)) return launched;
   return launch_prefill_merge(p, 128, stream);
 }

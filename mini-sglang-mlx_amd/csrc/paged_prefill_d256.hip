@@ -684,8 +684,7 @@ int launch_prefill_tile256(const PrefillArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)n_blocks);
   auto* const kernel = p.length_rounds > 0 ? (wide ? prefill_tile256_kernel<true, true> : prefill_tile256_kernel<false, true>)
                                            : (wide ? prefill_tile256_kernel<true, false> : prefill_tile256_kernel<false, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(kNW * 64), 0, stream, p);
-  const int launched = check_launch();
+  const int launched = launch_kernel(kernel, grid, dim3(kNW * 64), stream, p);
   if (launched != MSGL_OK || (p.n_ksplit == 1 && p.ragged_tiles == 0)) return launched;
   return launch_prefill_merge(p, kD, stream);
 }

@@ -404,9 +404,8 @@ int launch_shape(const ShareParams& sp, int share_len, unsigned blocks, hipStrea
   const uint32_t magic = (uint32_t)(((1ull << (31 + s)) + d - 1) / d), groups = (uint32_t)sp.head_groups;
   const ShareShape shape(s - 1, log2_of((uint32_t)NW / (uint32_t)sp.heads_wg), (groups & (groups - 1)) == 0 ? log2_of(groups) : ShareShape::kNoShift);
   auto launch = [&](auto narrow, auto wide) {
-    hipLaunchKernelGGL(sp.s.wide ? wide : narrow, dim3(blocks), dim3(64 * NW), 0, stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
-                       sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
-    return check_launch();
+    return launch_kernel(sp.s.wide ? wide : narrow, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
+                         sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
     const int mode = sp.s.nt.k == nullptr || sp.s.qo_indptr != nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;

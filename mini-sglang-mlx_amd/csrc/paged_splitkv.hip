@@ -544,9 +544,9 @@ int heads_per_group(int64_t n_kv) {
 }
 
 template <int D, int NCT, int NW>
-void launch_attn(const SplitKvParams& p, hipStream_t stream) {
+int launch_attn(const SplitKvParams& p, hipStream_t stream) {
   auto launch = [&](auto narrow, auto wide) {
-    hipLaunchKernelGGL(p.wide ? wide : narrow, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), 0, stream, p);
+    return launch_kernel(p.wide ? wide : narrow, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), stream, p);
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
     if (p.nt.k != nullptr && p.f16)
@@ -556,23 +556,19 @@ void launch_attn(const SplitKvParams& p, hipStream_t stream) {
     if (p.f16)
       return launch(splitkv_attention_kernel<D, NCT, NW, false, true, kStored>, splitkv_attention_kernel<D, NCT, NW, true, true, kStored>);
   }
-  launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStored>, splitkv_attention_kernel<D, NCT, NW, true, false, kStored>);
+  return launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStored>, splitkv_attention_kernel<D, NCT, NW, true, false, kStored>);
 }
 
 template <int D, int NCT>
 int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
   if ((p.f16 || p.nt.k != nullptr) && NCT != 1) return MSGL_ERR_DTYPE;
-  switch (waves) {
-    case 1: launch_attn<D, NCT, 1>(p, stream); break;
-    case 2: launch_attn<D, NCT, 2>(p, stream); break;
-    case 4: launch_attn<D, NCT, 4>(p, stream); break;
-    case 8:
-      if constexpr (D == 128 && NCT == 1) launch_attn<D, NCT, 8>(p, stream);
-      else return MSGL_ERR_SHAPE;
-      break;
-    default: return MSGL_ERR_SHAPE;
+  int rc = MSGL_ERR_SHAPE;
+  if (waves == 1) rc = launch_attn<D, NCT, 1>(p, stream);
+  else if (waves == 2) rc = launch_attn<D, NCT, 2>(p, stream);
+  else if (waves == 4) rc = launch_attn<D, NCT, 4>(p, stream);
+  if constexpr (D == 128 && NCT == 1) {
+    if (waves == 8) rc = launch_attn<D, NCT, 8>(p, stream);
   }
-  int rc = check_launch();
   if (rc != MSGL_OK) return rc;
   const dim3 mgrid((unsigned)(p.batch * p.max_len_extend), (unsigned)p.n_q);
   // four waves per row when a request can be cut into more items than one wave takes in a trip
@@ -580,15 +576,11 @@ int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
   constexpr int kItemsPerTrip = kWave / (D / 8) * (1 + kMergeUnroll);
   const bool wide_merge = p.n_seg > kItemsPerTrip && (int64_t)mgrid.x * mgrid.y <= 1024;
   if (wide_merge) {
-    if (p.f16) hipLaunchKernelGGL((splitkv_merge_kernel<D, true>), mgrid, dim3(64 * kMergeWaves), 0, stream, p);
-    else hipLaunchKernelGGL((splitkv_merge_kernel<D, false>), mgrid, dim3(64 * kMergeWaves), 0, stream, p);
-  } else {
-    constexpr unsigned kRows = kMergeWaves * (kWave / (D / 8));  // of a workgroup
-    const dim3 rows(mgrid.x, (mgrid.y + kRows - 1) / kRows);
-    if (p.f16) hipLaunchKernelGGL((splitkv_merge_rows_kernel<D, true>), rows, dim3(64 * kMergeWaves), 0, stream, p);
-    else hipLaunchKernelGGL((splitkv_merge_rows_kernel<D, false>), rows, dim3(64 * kMergeWaves), 0, stream, p);
+    return launch_kernel(p.f16 ? splitkv_merge_kernel<D, true> : splitkv_merge_kernel<D, false>, mgrid, dim3(64 * kMergeWaves), stream, p);
   }
-  return check_launch();
+  constexpr unsigned kRows = kMergeWaves * (kWave / (D / 8));  // of a workgroup
+  const dim3 rows(mgrid.x, (mgrid.y + kRows - 1) / kRows);
+  return launch_kernel(p.f16 ? splitkv_merge_rows_kernel<D, true> : splitkv_merge_rows_kernel<D, false>, rows, dim3(64 * kMergeWaves), stream, p);
 }
 
 // How a shape's column tiles map onto waves: tiles per wave and waves per kv head.

@@ -40,9 +40,8 @@ int launch(char* kc, char* vc, const int32_t* idx, const char* k, const char* v,
   const int64_t total = length * chunks;
   const int64_t blocks = (total + 255) / 256;
   if (blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  hipLaunchKernelGGL(store_kv_cache_kernel<VecT>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     kc, vc, idx, k, v, length, (int32_t)chunks, num_slots, kcs, vcs, ks, vs);
-  return check_launch();
+  return launch_kernel(store_kv_cache_kernel<VecT>, dim3((unsigned)blocks), dim3(256), stream,
+                       kc, vc, idx, k, v, length, (int32_t)chunks, num_slots, kcs, vcs, ks, vs);
 }
 
 struct alignas(16) B16 { uint32_t w[4]; };

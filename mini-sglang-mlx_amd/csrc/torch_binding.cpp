@@ -15,6 +15,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -27,6 +28,7 @@
 #include <optional>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/msgl_paged_attention.h"
@@ -135,13 +137,26 @@ Tensor empty(c10::IntArrayRef size, at::ScalarType dtype, const c10::Device& dev
   return at::detail::empty_cuda(size, dtype, dev, std::nullopt);
 }
 
-// Scratch from torch's caching allocator, taken on the launch stream: safe to drop right after the
-// launch because the allocator reuses a block in stream order.
-Tensor scratch(size_t bytes, const c10::Device& dev) {
-  return bytes ? empty({static_cast<int64_t>(bytes)}, at::kByte, dev) : Tensor();
-}
+// Scratch from torch's caching allocator, taken on the launch stream (the device is current): safe to give back right after
+// the launch because the allocator reuses a block in stream order.  Memory alone: a tensor around it takes as long again (0.3 us).
+class Scratch {
+ public:
+  Scratch() = default;
+  Scratch(size_t bytes, const OnDevice& on) : at_(bytes ? c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, on.stream) : nullptr) {}
+  Scratch(Scratch&& o) noexcept : at_(std::exchange(o.at_, nullptr)) {}
+  Scratch& operator=(Scratch&& o) noexcept {
+    std::swap(at_, o.at_);
+    return *this;
+  }
+  ~Scratch() {
+    if (at_) c10::hip::HIPCachingAllocator::raw_delete(at_);
+  }
+  void* ptr() const { return at_; }
 
-void* data_or_null(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+ private:
+  void* at_ = nullptr;
+};
+
 const int32_t* ints(const Tensor& t) { return static_cast<const int32_t*>(t.data_ptr()); }
 
 // ---- opt-in index validation: mini_sglang_amd_kernel._run_checks, given at import ---------------
@@ -286,9 +301,9 @@ PyObject* paged_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n_
         const int64_t kcs = pool_stride0(op, kc, "k_cache"), vcs = pool_stride0(op, vc, "v_cache");
         const Tensor qc = q.contiguous(), ipc = ip.contiguous(), ixc = ix.contiguous(), nsc = ns.contiguous();
         const size_t bytes = msgl_paged_decode_workspace_bytes(batch, total_kv, n_q, n_kv, d);
-        const Tensor ws = scratch(bytes, dev);
+        const Scratch ws(bytes, on);
         rc = msgl_paged_decode_attention(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(ipc), ints(ixc), ints(nsc),
-                                         out.data_ptr(), data_or_null(ws), bytes, batch, total_kv, n_q, n_kv, d,
+                                         out.data_ptr(), ws.ptr(), bytes, batch, total_kv, n_q, n_kv, d,
                                          kc.size(0), kcs, vcs, scale, max_splits, dtype_code(q), on.ptr());
       }
     }
@@ -349,9 +364,9 @@ PyObject* paged_prefill_attention(PyObject*, PyObject* const* args, Py_ssize_t n
         const Tensor qc = q.contiguous(), qpc = qp.contiguous(), ipc = ip.contiguous(), ixc = ix.contiguous(),
                      plc = pl.contiguous();
         const size_t bytes = msgl_paged_prefill_workspace_bytes(batch, total_q, total_kv, n_q, n_kv, d, max_extend);
-        const Tensor ws = scratch(bytes, dev);
+        const Scratch ws(bytes, on);
         rc = msgl_paged_prefill_attention(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(qpc), ints(ipc), ints(ixc),
-                                          ints(plc), out.data_ptr(), data_or_null(ws), bytes, batch, total_q, total_kv,
+                                          ints(plc), out.data_ptr(), ws.ptr(), bytes, batch, total_q, total_kv,
                                           n_q, n_kv, d, kc.size(0), kcs, vcs, scale, static_cast<int32_t>(max_extend),
                                           cross ? 1 : 0, static_cast<int32_t>(window), dtype_code(q), on.ptr());
       }
@@ -622,10 +637,10 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       NoGil nogil;
       OnDevice on(dev);
       out = empty({batch, n_q, d}, q.scalar_type(), dev);
-      const Tensor ws = scratch(bytes, dev);
+      const Scratch ws(bytes, on);
       rc = msgl_decode_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), row_stride(q), row_stride(k), row_stride(v),
                             norm ? t(3).data_ptr() : nullptr, norm ? t(4).data_ptr() : nullptr, norm ? ints(t(5)) : nullptr,
-                            ints(loc), kc.data_ptr(), vc.data_ptr(), ints(ip), ints(ix), out.data_ptr(), ws.data_ptr(), bytes,
+                            ints(loc), kc.data_ptr(), vc.data_ptr(), ints(ip), ints(ix), out.data_ptr(), ws.ptr(), bytes,
                             batch, ix.size(0), n_q, n_kv, d, slots, row_stride(kc), row_stride(vc), scale, eps, base,
                             dtype_code(q), on.ptr());
     }
@@ -664,9 +679,9 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       size_t bytes = !own_slots ? 0 : msgl_extend_step_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend, cross,
                                                                        static_cast<int32_t>(window));
       if (bytes > 0) {
-        const Tensor ws = scratch(bytes, dev);
+        const Scratch ws(bytes, on);
         rc = msgl_extend_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), ks0, vs0, ints(loc), kc.data_ptr(), vc.data_ptr(), ints(qp),
-                              ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.data_ptr(), bytes, batch, total, ix.size(0), n_q,
+                              ints(ip), ints(ix), ints(pl), out.data_ptr(), ws.ptr(), bytes, batch, total, ix.size(0), n_q,
                               n_kv, d, slots, kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
                               static_cast<int32_t>(window), dtype_code(q), on.ptr());
       } else {
@@ -674,9 +689,9 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
                                  vcs, ks0, vs0, static_cast<int32_t>(kc.element_size()), on.ptr());
         if (rc == MSGL_OK) {
           bytes = msgl_paged_prefill_workspace_bytes(batch, total, ix.size(0), n_q, n_kv, d, max_extend);
-          const Tensor ws = scratch(bytes, dev);
+          const Scratch ws(bytes, on);
           rc = msgl_paged_prefill_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ints(qp), ints(ip), ints(ix), ints(pl),
-                                            out.data_ptr(), data_or_null(ws), bytes, batch, total, ix.size(0), n_q, n_kv, d, slots,
+                                            out.data_ptr(), ws.ptr(), bytes, batch, total, ix.size(0), n_q, n_kv, d, slots,
                                             kcs, vcs, scale, static_cast<int32_t>(max_extend), cross ? 1 : 0,
                                             static_cast<int32_t>(window), dtype_code(q), on.ptr());
         }
@@ -733,17 +748,17 @@ PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args)
       // the forms whose scratch memory would not be used (see the header)
       const bool plain = reinterpret_cast<uintptr_t>(v.data_ptr()) % 16 == 0 && vs % 8 == 0 && std::max({qs, ks, vs}) < (1 << 24) && hv < (1 << 17);
       size_t bytes = plain ? msgl_gdn_state_workspace_bytes(tokens, batch, hv, single ? 1 : 0) : 0;
-      Tensor ws;
+      Scratch ws;
       if (bytes > 0) {
         try {
-          ws = scratch(bytes, dev);
+          ws = Scratch(bytes, on);
         } catch (const c10::OutOfMemoryError&) {  // it is an optimisation: the call goes without
           bytes = 0;
         }
       }
       rc = msgl_gdn_state_inplace_in(q.data_ptr(), k.data_ptr(), v.data_ptr(), gc.data_ptr(), bc.data_ptr(), state.data_ptr(),
                                   ints(sc), single ? nullptr : ints(ipc), y.data_ptr(), tokens, batch, hk, hv, dk, dv,
-                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, data_or_null(ws), bytes, on.ptr());
+                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, ws.ptr(), bytes, on.ptr());
     }
     check_rc(op, rc);
     return THPVariable_Wrap(std::move(y));

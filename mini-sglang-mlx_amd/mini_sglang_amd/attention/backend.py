@@ -94,42 +94,30 @@ class AttnBackend:
         assert sliding_window_size >= 0, (
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
-        metadata = batch.attn_metadata
+        metadata, cache = batch.attn_metadata, self.kvcache
         out = None
-        if type(metadata) is PrefillMetadata:
-            out = self._extend_step(q, k, v, layer_id, batch, is_cross_attention, sliding_window_size)
-        elif not is_cross_attention and sliding_window_size == 0:
-            out = self._decode_step(q, k, v, layer_id, batch)
+        # one native call, where this package writes the pool itself (a call of Python's own beside it costs as much as
+        # all the checks in it); None: the step takes its two calls
+        if type(cache) is not MHAKVCache:
+            pass
+        elif type(metadata) is PrefillMetadata:
+            out = _native.extend_step(q, k, v, batch.out_loc, cache.k_cache(layer_id),
+                                      cache.v_cache(layer_id), metadata.qo_indptr, metadata.kv_indptr,
+                                      metadata.kv_indices, metadata.prefix_lens, self.sm_scale,
+                                      metadata.max_len_extend, is_cross_attention, sliding_window_size,
+                                      metadata.own_slots)
+        elif (type(metadata) is DecodeMetadata and metadata.own_slots and not is_cross_attention
+              and sliding_window_size == 0):
+            out = _native.decode_step(q, k, v, None, None, None, batch.out_loc,
+                                      cache.k_cache(layer_id), cache.v_cache(layer_id),
+                                      metadata.kv_indptr, metadata.kv_indices,
+                                      metadata.num_kv_splits, self.sm_scale, 0.0, 0.0)
         if out is not None:
             return out
         self.kvcache.store_kv(k, v, batch.out_loc, layer_id)
         k_cache = self.kvcache.k_cache(layer_id)
         v_cache = self.kvcache.v_cache(layer_id)
         return self._attend(q, k_cache, v_cache, metadata, is_cross_attention, sliding_window_size)
-
-    def _decode_step(self, q, k, v, layer_id: int, batch, q_weight=None, k_weight=None,
-                     positions=None, eps: float = 0.0, rope_base: float = 0.0) -> Optional[torch.Tensor]:
-        """``mini_sglang_amd_kernel.decode_step`` on the step's pool, where this package writes that
-        itself; ``None``: the step takes its two calls."""
-        metadata, cache = batch.attn_metadata, self.kvcache
-        if type(metadata) is not DecodeMetadata or not metadata.own_slots or type(cache) is not MHAKVCache:
-            return None
-        return _native.decode_step(q, k, v, q_weight, k_weight, positions, batch.out_loc,
-                                   cache.k_cache(layer_id), cache.v_cache(layer_id),
-                                   metadata.kv_indptr, metadata.kv_indices, metadata.num_kv_splits,
-                                   self.sm_scale, eps, rope_base)
-
-    def _extend_step(self, q, k, v, layer_id: int, batch, is_cross_attention: bool,
-                     sliding_window_size: int) -> Optional[torch.Tensor]:
-        """The same for ``mini_sglang_amd_kernel.extend_step``, which makes the two launches too."""
-        metadata, cache = batch.attn_metadata, self.kvcache
-        if type(cache) is not MHAKVCache:
-            return None
-        return _native.extend_step(q, k, v, batch.out_loc, cache.k_cache(layer_id),
-                                   cache.v_cache(layer_id), metadata.qo_indptr, metadata.kv_indptr,
-                                   metadata.kv_indices, metadata.prefix_lens, self.sm_scale,
-                                   metadata.max_len_extend, is_cross_attention, sliding_window_size,
-                                   metadata.own_slots)
 
     def _attend(self, q, k_cache, v_cache, metadata, is_cross_attention: bool,
                 sliding_window_size: int) -> torch.Tensor:
@@ -162,9 +150,14 @@ class AttnBackend:
             f"sliding_window_size must be >= 0, got {sliding_window_size}"
         )
         metadata = batch.attn_metadata
-        if not is_cross_attention and sliding_window_size == 0:
-            out = self._decode_step(q, k, v, layer_id, batch, q_norm_weight, k_norm_weight,
-                                    metadata.positions, rms_norm_eps, rope_base)
+        cache = self.kvcache
+        if (type(metadata) is DecodeMetadata and metadata.own_slots and type(cache) is MHAKVCache
+                and not is_cross_attention and sliding_window_size == 0):
+            out = _native.decode_step(q, k, v, q_norm_weight, k_norm_weight, metadata.positions,
+                                      batch.out_loc, cache.k_cache(layer_id),
+                                      cache.v_cache(layer_id), metadata.kv_indptr,
+                                      metadata.kv_indices, metadata.num_kv_splits, self.sm_scale,
+                                      rms_norm_eps, rope_base)
             if out is not None:
                 return out
         k_cache = self.kvcache.k_cache(layer_id)
