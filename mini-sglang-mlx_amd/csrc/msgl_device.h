@@ -138,6 +138,17 @@ __device__ __forceinline__ float row_sum16(float v) {
   v += dpp<0x140>(v);
   return v;
 }
+__device__ __forceinline__ float row_max16(float v) {
+  v = fmaxf(v, dpp<0xB1>(v));
+  v = fmaxf(v, dpp<0x4E>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  return fmaxf(v, dpp<0x140>(v));
+}
+// The value of lane N of a row of 16 lanes, in all of them
+template <int N>
+__device__ __forceinline__ float of_row_lane(float v) {
+  return dpp<0x150 + N>(v);
+}
 __device__ __forceinline__ int row_max16(int v) {
   v = max(v, dpp<0x128>(v));
   v = max(v, dpp<0x124>(v));

@@ -73,14 +73,29 @@ __device__ __forceinline__ int ceil_div(int a, int b) {
   return q;
 }
 
-__device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
-  return (unsigned long long)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo);
-}
 __device__ __forceinline__ void st_agent(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ unsigned long long ld_agent(const unsigned long long* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 16 bytes of the partials at agent scope.  (As two 8-byte accesses, the largest there are of atomics, each of them walks all
+// the lines that the wave's 16-byte pieces lie in: 24 loads of a thread took 1.5 K cycles to be issued, 48 of head_dim 256 3.8 K.)
+constexpr int kAgentScope = 16;  // sc1
+struct Partials {
+  __amdgpu_buffer_rsrc_t at;
+  __device__ __forceinline__ Partials(float* from, uint32_t bytes) : at(__builtin_amdgcn_make_buffer_rsrc(from, 0, bytes, 0x00020000)) {}
+  __device__ __forceinline__ f32x4_t load(uint32_t lane_at, uint32_t share_at) const {
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(at, (int)lane_at, (int)share_at, kAgentScope));
+  }
+  __device__ __forceinline__ void store(uint32_t lane_at, f32x4_t v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), at, (int)lane_at, 0, kAgentScope);
+  }
+};
+template <typename F, int... I>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
 }
 
 // Share number `item` of the launch: its request, which of the request's shares it is, of how many.
@@ -250,40 +265,30 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column, the 16 bytes at 16 it of a share's rows
   const int threads = 64 * share_waves;
   const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols;
-  char* const rows_to = reinterpret_cast<char*>(p.part_o + row0 * D);
-  // every wave's part of a quad is asked for before the first is used
+  const Partials own(p.part_o + row0 * D, (uint32_t)(ncols * D * 4));
+  // Every wave's part of a quad is asked for before the first is used.  The lanes of a row of 16 work on one column: lane w has
+  // wave w's maximum and sum, and its weight goes to the others by DPP.
   auto put_together = [&](auto waves) {
     constexpr int W = decltype(waves)::value;
     for (int it = threadIdx.x - sub * threads; it < ncols * kQuads; it += threads) {
       const int col = it / kQuads, d4 = (it - col * kQuads) * 4;
-      float2 ml[W];
+      float2 ml = state[sub * W + min(t16, W - 1)][col];
       f32x4_t o[W];
 #pragma unroll
-      for (int w = 0; w < W; ++w) {
-        ml[w] = state[sub * W + w][col];
-        o[w] = *reinterpret_cast<const f32x4_t*>(&part[sub * W + w][d4 >> 3][col * 8 + (d4 & 7)]);
-      }
-      float m = kNegInf;
-#pragma unroll
-      for (int w = 0; w < W; ++w) m = fmaxf(m, ml[w].x);
+      for (int w = 0; w < W; ++w) o[w] = *reinterpret_cast<const f32x4_t*>(&part[sub * W + w][d4 >> 3][col * 8 + (d4 & 7)]);
+      if (t16 >= W) ml = float2{kNegInf, 0.f};
+      const float m = row_max16(ml.x), m_safe = (m == kNegInf) ? 0.f : m;
+      const float e = fast_exp2(ml.x - m_safe);  // 0 for a wave without visible keys
+      const float l = row_sum16(e * ml.y);
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      float l = 0.f;
-      const float m_safe = (m == kNegInf) ? 0.f : m;
-#pragma unroll
-      for (int w = 0; w < W; ++w) {
-        const float e = fast_exp2(ml[w].x - m_safe);  // 0 for a wave without visible keys
-        acc += e * o[w];
-        l += e * ml[w].y;
-      }
+      each([&](auto w) { acc += of_row_lane<decltype(w)::value>(e) * o[decltype(w)::value]; }, std::make_integer_sequence<int, W>{});
       acc *= (l > 0.f) ? 1.0f / l : 0.f;
       if (n_shares == 1) {
         const int qi = query_of(p, col);
         uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4;
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(acc[0], acc[1]), pack_16x2<F16>(acc[2], acc[3])};
       } else {
-        unsigned long long* dst = reinterpret_cast<unsigned long long*>(rows_to + 16u * (uint32_t)it);
-        st_agent(dst, pair_bits(acc[0], acc[1]));
-        st_agent(dst + 1, pair_bits(acc[2], acc[3]));
+        own.store(16u * (uint32_t)it, acc);
         if (d4 == 0)
           __hip_atomic_store(p.part_lse + row0 + col, (l > 0.f) ? m + __log2f(l) : kNegInf, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
@@ -320,13 +325,13 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   constexpr int I = NW == 4 ? 2 : 1;  // a thread's quads whose loads are in flight together
   const int64_t step = (int64_t)p.n_kv * p.cols;  // rows from one share to the next
   const int64_t first = row0 - share * step;
-  const char* const rows_from = reinterpret_cast<const char*>(p.part_o + first * D);
-  const char* const lse_from = reinterpret_cast<const char*>(p.part_lse + first);
+  const uint32_t step_bytes = (uint32_t)step * (D * 4);  // (launch_shares() sees to it that a request's partials are below 2 GiB)
+  const Partials all(p.part_o + first * D, (uint32_t)n_shares * step_bytes);
+  const float* const lse_from = p.part_lse + first;
   const int quads = ncols * kQuads;
   // ... for as many shares as there are, by fours, or 16 (loads past the last one cost as much as the others:
   // 16 for all of four shares 9.3 -> 9.8 us; 8 for more than 8 in turns 11.6 us against 11.2 at two of 3000 tokens).
-  // A share's rows are a scalar base, a thread's place in them is 32 bits: with 64-bit addresses to each load, issuing
-  // them took 1.5 K cycles, longer than they were under way.
+  // As above, the lanes of a row of 16 have a share's log-sum-exp each.
   auto merge = [&](auto in_flight) {
     constexpr int U = decltype(in_flight)::value;
     for (int it0 = threadIdx.x - sub * threads; it0 < quads; it0 += I * threads) {
@@ -341,40 +346,26 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
         acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
       for (int s0 = 0; s0 < n_shares; s0 += U) {
-        float lse[I][U];
-        unsigned long long lo[I][U], hi[I][U];
+        const int mine = min(s0 + min(t16, U - 1), n_shares - 1);
+        float lse[I];
+        f32x4_t o[I][U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {  // shares past the last one: the last again, with weight 0
-          const int64_t rows = min(s0 + u, n_shares - 1) * step;
-          const char* const from = rows_from + rows * (D * 4);
-          const char* const lse_at = lse_from + rows * 4;
+        for (int i = 0; i < I; ++i) {
+          lse[i] = __hip_atomic_load(lse_from + mine * step + at[i] / kQuads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-          for (int i = 0; i < I; ++i) {
-            lse[i][u] = __hip_atomic_load(reinterpret_cast<const float*>(lse_at + 4u * (at[i] / kQuads)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lo[i][u] = ld_agent(reinterpret_cast<const unsigned long long*>(from + 16u * at[i]));
-            hi[i][u] = ld_agent(reinterpret_cast<const unsigned long long*>(from + 16u * at[i]) + 1);
-            if (s0 + u >= n_shares) lse[i][u] = kNegInf;
-          }
+          for (int u = 0; u < U; ++u)  // shares past the last one: the last again, with weight 0
+            o[i][u] = all.load(16u * at[i], (uint32_t)min(s0 + u, n_shares - 1) * step_bytes);
         }
 #pragma unroll
         for (int i = 0; i < I; ++i) {
-          float m_new = m[i];
-#pragma unroll
-          for (int u = 0; u < U; ++u) m_new = fmaxf(m_new, lse[i][u]);
+          if (t16 >= U || s0 + t16 >= n_shares) lse[i] = kNegInf;
+          const float m_new = fmaxf(m[i], row_max16(lse[i]));
           const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
-          const float old = fast_exp2(m[i] - m_safe);
+          const float old = fast_exp2(m[i] - m_safe), e = fast_exp2(lse[i] - m_safe);
           acc[i] *= old;
-          l[i] *= old;
+          l[i] = l[i] * old + row_sum16(e);
           m[i] = m_new;
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float e = fast_exp2(lse[i][u] - m_safe);
-            acc[i][0] += e * __builtin_bit_cast(float, (uint32_t)lo[i][u]);
-            acc[i][1] += e * __builtin_bit_cast(float, (uint32_t)(lo[i][u] >> 32));
-            acc[i][2] += e * __builtin_bit_cast(float, (uint32_t)hi[i][u]);
-            acc[i][3] += e * __builtin_bit_cast(float, (uint32_t)(hi[i][u] >> 32));
-            l[i] += e;
-          }
+          each([&](auto u) { acc[i] += of_row_lane<decltype(u)::value>(e) * o[i][decltype(u)::value]; }, std::make_integer_sequence<int, U>{});
         }
       }
 #pragma unroll
@@ -526,6 +517,8 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   const bool rows = n.k != nullptr && a.qo_indptr != nullptr;  // kStoreRows
   const int64_t blocks = plan.max_shares * head_groups + (rows ? kRestBlocks : 0);
   if (blocks > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
+  // one request's partials (the plans' are below 128 MiB)
+  if ((plan.max_shares - a.batch + 1) * a.n_kv * cols * a.head_dim * 4 > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   ShareParams sp{};
   fill_splitkv_params(a, sp.s);
   char* ws = static_cast<char*>(a.workspace);
