@@ -80,7 +80,6 @@ int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t ma
 bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv, int64_t keys, int64_t n_kv,
                    int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
-  if (head_dim == 256 && batch * n_kv < 12) return false;  // see shares_preferred()
   const int64_t blocks = batch * (n_kv / plan.heads_wg), cus = msgl::device_cus();
   if (blocks > cus && 3 * blocks < 2 * cus * ((blocks + cus - 1) / cus)) return false;
   return cols <= 32 || plan.heads_wg == 1;

@@ -425,6 +425,32 @@ thread_local int64_t t_force = 0;  // benchmarking switch, see shares_force()
 
 void shares_force(int64_t v) { t_force = v; }
 
+// head_dim 256, (request, kv head) pairs no more than compute units: length and line of their own.
+static bool wide_heads_alone(int64_t batch, int64_t n_kv, int64_t head_dim) { return head_dim == 256 && batch * n_kv <= device_cus(); }
+
+// Length of the shares there: of those (in steps of a third or a half from 128 on) that fit the chip in one round, requests of one
+// length included, the one that costs least: its keys, what a share costs the one that puts the request together, and a round trip
+// for every 16 of them, all in keys' worth of time.  Fitted to 4280 launches (decode and verify, 1-40 requests of 200-100 000 keys, four
+// head counts, every length that fits timed): within 1.0 % of the best length on average up to 8 columns, 1.4 % beyond; the length that head_dim 128
+// has, at most 16 shares to a request, from 256 on, and segments for fewer than 12 pairs: 16 and 11 %.
+static int64_t wide_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols) {
+  const double slots = (double)device_cus(), mean = (double)(keys / batch), spread = 0.43 * std::sqrt((double)batch);
+  int64_t len = 0;
+  double lowest = 0;
+  for (int64_t c = 128; c < (1 << 20); c = (c & (c - 1)) ? c / 3 * 4 : c / 2 * 3) {
+    const double of_one = std::max(std::ceil(mean / (double)c), 1.0);
+    const double shares = std::max({(double)batch, (double)keys / (double)c + 0.5 * (double)batch + spread, (double)batch * of_one});
+    if (shares * (double)n_kv > slots) continue;
+    const double cost = std::min((double)c, 1.5 * mean) + (of_one > 1 ? (cols > 8 ? 160 : 100) : 0) + 4 * of_one + 100 * (std::ceil(of_one / 16) - 1);
+    if (len == 0 || cost < lowest) {
+      len = c;
+      lowest = cost;
+    }
+    if ((double)c >= 2 * mean) break;
+  }
+  return len > 0 ? len : 1 << 20;
+}
+
 SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols) {
   SharePlan plan{};
   const int nct = nct_of(cols);
@@ -443,7 +469,8 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     // average request: the last of them reads the others' partials.  Rounding adds half a share per request
     // and scatters around that: with two standard deviations more, 9 requests of 102-713 keys, 64 / 8 heads, have 192 keys a share
     // and take 12.5 us, without it 128, a few workgroups more than compute units, and 16.6
-    len = nct == 3 ? 512 : (nw == 4 && heads == 1) ? 256 : 128;
+    const bool wide = wide_heads_alone(batch, n_kv, head_dim);
+    len = nct == 3 ? 512 : (nw == 4 && heads == 1 && !wide) ? 256 : 128;
     const int64_t spread = (int64_t)std::sqrt((double)batch / 3);
     auto fits = [&](int64_t c) {
       return std::max(batch, keys / c + batch / 2 + spread) * (n_kv / heads) <= slots && keys <= 16 * c * batch;
@@ -451,6 +478,8 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     if (each > 0) {  // one length for all: as many equal shares as fit
       const int64_t n = std::min<int64_t>(std::max<int64_t>(slots * heads / (batch * n_kv), 1), 16);
       len = std::max(len, ((each + n - 1) / n + 31) & ~(int64_t)31);
+    } else if (wide) {
+      len = wide_share_length(batch, keys, n_kv, cols);
     } else {
       while (!fits(len) && len < (1 << 19)) len = (len & (len - 1)) ? len / 3 * 4 : len / 2 * 3;
     }
@@ -493,8 +522,15 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
   if (t_force > 0) return true;
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
-  // few units: most of the time is the last share's, which reads all the others of a wide head group
-  if (head_dim == 256 && units < 12) return false;
+  if (wide_heads_alone(batch, n_kv, head_dim)) {
+    // Beyond some MiB the shares have to fill the chip: a launch takes as long as its longest share.  By MiB of keys and values
+    // and what part of a round of shares as long as the longest they are, shares by segments (geometric mean, worst): up to 64 0.65
+    // (1.10), 64-128 0.76 (0.99), 128-256 from 0.5 on 0.83 (1.05) and 1.03 below, 256-420 from 0.62 on 0.91 (1.07), 1.05 below,
+    // 512-724 from 0.75 on 0.95 (1.03), 0.97 (1.09) below, 1.04 below 0.62, 1024-1448 from 0.88 on 0.96 (0.98), 0.98 (1.07) below, 1.02 below
+    // 0.75.  The line goes along that.  (Two of 408-2260 keys, 24 / 4 heads, 21.8 -> 11.0 us; one of 51.8 K, 16 / 2, 51 -> 35.)
+    const double longest = std::min((double)plan.share_len, 1.75 * (double)mean);
+    return mb <= 1400 && (double)(keys * n_kv) >= (0.12 * std::log2((double)std::max<int64_t>(mb, 1)) - 0.39) * longest * (double)device_cus();
+  }
   if (mb <= (mean > 8192 ? 20 : mean > 4096 ? 36 : head_dim == 256 ? 128 : 56)) return true;
   const int64_t len = plan.share_len, head_groups = n_kv / plan.heads_wg;
   const double shares = (double)keys / (double)len + 0.5 * (double)batch + std::sqrt((double)batch / 3);  // see share_plan()

@@ -42,3 +42,15 @@ def test_short_query_blocks(gpu, tuning, n_q, n_kv, q_len, share, cross, window)
     tuning(_lib.TUNE_SHARES, share | 1 << 20 if share else 0)
     print(f"share cuts verify {n_q}/{n_kv} q{q_len} {mask} cut {share}", flush=True)
     _close(paged_prefill_attention(*args(g), **mask), want)
+
+
+@pytest.mark.parametrize("lens,n_q,n_kv", [([20001], 16, 2), ([1907, 812], 24, 4), ([129], 32, 2), ([7000, 1, 255, 4100], 16, 2), ([5200], 16, 4)])
+def test_few_wide_heads(gpu, lens, n_q, n_kv):
+    """As many shares to a request as fit the chip: up to 53 here, put together 16 at a time."""
+    wl = build_workload("wide heads", "decode", seed=len(lens), n_q=n_q, n_kv=n_kv, head_dim=256, kv_lens=lens)
+    want = oracle.paged_decode_attention(wl.q, wl.k_cache, wl.v_cache, wl.kv_indptr, wl.kv_indices, wl.num_kv_splits,
+                                         wl.sm_scale, wl.max_kv_splits, return_f32=True)[1]
+    g = wl.to(gpu)
+    print(f"wide heads {lens} {n_q}/{n_kv}", flush=True)
+    for _ in range(2):
+        _close(paged_decode_attention(g.q, g.k_cache, g.v_cache, g.kv_indptr, g.kv_indices, g.num_kv_splits, g.sm_scale, 32), want)

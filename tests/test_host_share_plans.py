@@ -1,0 +1,17 @@
+"""Which decode launches at head_dim 256 go in shares of their requests' keys: few (request, kv head) pairs, long requests, and the two
+lines beyond which they go in segments.  (With norm and rotary embedding a decode step is one launch where it goes in shares.)"""
+import pytest
+
+
+@pytest.mark.parametrize("batch,keys,n_q,n_kv,shares", [
+    (1, 51820, 16, 2, True), (2, 3814, 24, 4, True), (1, 1, 16, 2, True), (2, 45000, 24, 4, True),
+    (22, 22 * 4116, 16, 4, False),      # shares long enough for one round fill less than half of it
+    (22, 22 * 2900, 16, 4, True),
+    (4, 717500, 16, 2, False), (4, 716000, 16, 2, True),  # 1400 MiB of keys and values
+    (64, 64 * 300, 16, 4, True)])
+def test_head_dim_256(batch, keys, n_q, n_kv, shares):
+    from mini_sglang_amd_kernel import _lib
+
+    lib = _lib.load()
+    assert (lib.msgl_decode_step_workspace_bytes(batch, keys, n_q, n_kv, 256, 1) > 0) is shares
+    assert lib.msgl_decode_step_workspace_bytes(batch, keys, n_q, n_kv, 256, 1) <= lib.msgl_paged_decode_workspace_bytes(batch, keys, n_q, n_kv, 256)
