@@ -22,7 +22,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(LIB_DIR, "libmsgl_paged_attention.so")
 SOURCES = ["api.hip", "store_kv_cache.hip", "paged_splitkv.hip", "paged_shares.hip", "paged_prefill.hip", "paged_prefill_d256.hip",
            "build_metadata.hip", "qk_norm_rope_store.hip",
-           "gdn_state.hip", "gdn_chunk.hip", "gdn_long.hip", "radix_cache.hip", "state_slots.hip"]
+           "gdn_state.hip", "gdn_short.hip", "gdn_chunk.hip", "gdn_long.hip", "radix_cache.hip", "state_slots.hip"]
 
 NATIVE_SRC = os.path.join(CSRC, "torch_binding.cpp")
 NATIVE_PATH = os.path.join(HERE, "mini_sglang_amd_kernel", "_native.so")

@@ -24,6 +24,7 @@ struct GdnParams {
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __builtin_bit_cast(float, b << 16); }
 
+int launch_gdn_short(const GdnParams& p, hipStream_t stream);
 int launch_gdn_chunks(const GdnParams& p, hipStream_t stream);
 size_t gdn_long_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv);
 int launch_gdn_long(const GdnParams& p, void* workspace, hipStream_t stream);

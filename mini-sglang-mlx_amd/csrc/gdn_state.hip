@@ -15,9 +15,8 @@
 // the next kDepth tokens are always in flight.  Decode (one token) is
 // HBM-bound: 2 * dv * dk * 4 bytes of state per (request, hv head) read and written once.
 // Prefill is a serial chain per row (as in the reference); parallelism is batch * hv * dv rows.  It takes
-// requests of a few tokens here; longer ones go in chunks (gdn_chunk.hip, prefer_chunks() below).
+// requests of very few tokens here; longer ones go in chunks (gdn_short.hip, gdn_chunk.hip, route_of() below).
 #include <algorithm>
-#include <atomic>
 
 #include "gdn_params.h"
 
@@ -158,21 +157,25 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 
 }  // namespace
 
-// Whether the chunk kernel (gdn_chunk.hip) is the faster one.  Its time for up to 64 tokens per request
-// does not depend on their number: 12.8 us for each round of workgroups (two per value head, one per
-// compute unit), or 9.2 us and 0.9 us per request of 32 heads where all requests go in pairs of waves (four
-// workgroups per value head, in one round).  The token kernel's grows with the mean length, by 0.315 us per token while the requests
-// run side by side and by 0.095 us per token and request of 32 heads beyond.  Both fitted to 1, 4, 16 and 64
-// requests of 8, 16, 32 and 64 tokens; they meet between 15 and 30 tokens (one request of 24 at 32 heads: 11.1 us token by token, 9.8 in a chunk; of 16:
-// 8.6 and 9.8).
-static bool prefer_chunks(const GdnArgs& a) {
+// Which kernel takes a call with more than a token a request, by the mean length and units of 32 heads.  us, token by token / in chunks
+// of 16 (gdn_short.hip) / in chunks of 64 (gdn_chunk.hip, whose time for up to 64 tokens does not depend on their number):
+//     requests of 32 heads   1: 4 tokens 5.8 / 5.8 / 9.3, 16 8.6 / 5.8 / 9.5, 32 13.4 / 7.3 / 9.3, 64 23 / 9.7 / 9.5
+//                            4: 4 tokens 9.8 / 7.1 / 12.1, 16 17 / 7.5 / 12.3, 32 28 / 8.6 / 12.4, 64 47 / 12.2 / 12.7
+//                            8: 4 tokens 11 / 9.4 / 25, 16 21 / 10.5 / 25, 64 61 / 17 / 25.6, 256 - / 44 / 57
+//                           16: 4 tokens 20 / 16 / 51, 16 37 / 17 / 50, 64 110 / 27 / 51, 256 - / 72 / 103
+// Up to three tokens the token kernel is as fast (1.00-1.28 beyond 16 units, 1.03-1.14 up to 1, where this goes for up to 8 tokens).
+// What ends the chunks of 16 is not the even launch but one long request among short ones, whose chunks come one after the
+// other, 1.5-2 us for 16 tokens against 0.8-1.1 in the larger ones: beside four of 12 tokens one of 184 22.5 -> 29.9, beside eight
+// of 36 one of 578 53 -> 88.  Beyond 16 units the work of all is longer than such a chain.  345 launches of 1-48 requests, 8-64 heads, 2-3000
+// tokens, even, ragged and of one long request: those this sends to chunks of 16, by their time before, 0.66 (geometric mean, 0.30-1.10).
+enum class GdnRoute { kTokens, kShort, kChunks };
+static GdnRoute route_of(const GdnArgs& a) {
   if (a.v_stride0 >= (1 << 24) || a.k_stride0 >= (1 << 24) || a.q_stride0 >= (1 << 24) || a.hv >= (1 << 17))
-    return false;  // its offsets inside a chunk are 32 bits wide
-  if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return false;  // loads of 16 bytes, stores of 8
-  const double units = (double)(a.batch * a.hv) / 32, mean = (double)a.tokens / (double)a.batch;
-  const double rounds = (double)((a.batch * a.hv * 2 + device_cus() - 1) / device_cus());
-  const bool pairs = a.batch <= 64 && a.batch * a.hv * 4 <= device_cus();
-  return (pairs ? 9.2 + 0.9 * units : 12.8 * rounds) < 3.0 + 0.5 * units + mean * std::max(0.315, 0.13 + 0.095 * units);
+    return GdnRoute::kTokens;  // the others' offsets inside a chunk are 32 bits wide
+  if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return GdnRoute::kTokens;  // loads of 16 bytes, stores of 8
+  const int64_t heads = a.batch * a.hv;
+  const int64_t least = heads <= 32 ? 9 : heads <= 64 || heads > 512 ? 4 : 2, most = heads <= 512 ? 41 : 128;
+  return a.tokens < least * a.batch ? GdnRoute::kTokens : a.tokens < most * a.batch ? GdnRoute::kShort : GdnRoute::kChunks;
 }
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 // Room for the systems of all chunks where making those in a launch of their own pays (gdn_long.hip), 0 elsewhere.  The second
@@ -227,10 +230,14 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   p.single_token = a.single_token_mode ? 1 : 0;
   const int64_t heads = a.batch * a.hv;
   if (heads <= 0) return MSGL_OK;
-  if (!p.single_token && t_force_rows == 0 && prefer_chunks(a)) {
-    const size_t bytes = gdn_state_workspace_bytes(a.tokens, a.batch, a.hv, false);
-    if (bytes > 0 && a.workspace != nullptr && a.workspace_bytes >= bytes) return launch_gdn_long(p, a.workspace, stream);
-    return launch_gdn_chunks(p, stream);
+  if (!p.single_token && t_force_rows == 0) {
+    const GdnRoute route = route_of(a);
+    if (route == GdnRoute::kShort) return launch_gdn_short(p, stream);
+    if (route == GdnRoute::kChunks) {
+      const size_t bytes = gdn_state_workspace_bytes(a.tokens, a.batch, a.hv, false);
+      if (bytes > 0 && a.workspace != nullptr && a.workspace_bytes >= bytes) return launch_gdn_long(p, a.workspace, stream);
+      return launch_gdn_chunks(p, stream);
+    }
   }
   // more rows per lane group (more overlap inside a wave) once there are enough workgroups
   // to fill the chip without it
