@@ -24,7 +24,7 @@
 // that fetch and make the systems ahead: 1.1 us a chunk for one request, no change for four; S's parts of 64 dims side by side: 4 % faster for
 // one request, 10 % slower for sixteen (registers).
 //
-// Precision: fp32 throughout, the parts are exact (see cut()).  The state's error against 64 bits, rms: 1.0-1.7e-8 at states of 0.1
+// Precision: fp32 throughout, the parts are exact (see upper()).  The state's error against 64 bits, rms: 1.0-1.7e-8 at states of 0.1
 // (the token kernel 1.2-2.5e-8, chunks of 64 1.2-1.8e-8); the chunk's addition to S in a sum of its own, joined by one multiply-add, is 7-10 %
 // of that.  Infinities and NaN as in gdn_chunk.hip: a wave whose U or P is not finite goes through its request again.
 #include "gdn_chunk_tiles.h"
@@ -137,8 +137,8 @@ __device__ __forceinline__ void make_products(ShortSystem& to, const uint16_t* k
   to.p[lane] = pt;
 }
 
-// The upper halves of four values, and of eight; the parts of eight as in split(), but cut instead of rounded: three of 8
-// significant bits of one sign, exact as well (a permutation takes 5 cycles where a conversion takes 8).
+// The upper halves of four values, and of eight.  Parts as in split(), but cut instead of rounded: three of 8 significant bits and one
+// sign, exact as well (a permutation takes 5 cycles where a conversion takes 8).
 __device__ __forceinline__ u32x2_t upper(f32x4_t f) {
   const u32x4_t bits = __builtin_bit_cast(u32x4_t, f);
   return u32x2_t{__builtin_amdgcn_perm(bits[1], bits[0], 0x07060302u), __builtin_amdgcn_perm(bits[3], bits[2], 0x07060302u)};
@@ -147,18 +147,6 @@ __device__ __forceinline__ bf16x8_t upper(f32x4_t a, f32x4_t b) {
   const u32x2_t x = upper(a), y = upper(b);
   return as_bf16x8(u32x4_t{x[0], x[1], y[0], y[1]});
 }
-__device__ __forceinline__ Split cut(const Picker& pick, f32x4_t a, f32x4_t b) {
-  Split s;
-  s.hi = upper(a, b);
-  a = mfma_16x16x32(pick.first, s.hi, a);
-  b = mfma_16x16x32(pick.second, s.hi, b);
-  s.mid = upper(a, b);
-  a = mfma_16x16x32(pick.first, s.mid, a);
-  b = mfma_16x16x32(pick.second, s.mid, b);
-  s.lo = upper(a, b);
-  return s;
-}
-
 // WAVES: 8, a head's rows in one workgroup, or 4, half of them
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnParams p) {
@@ -235,18 +223,50 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
     }
     // X = K S^T, tokens on the rows, and Z = S Q^T, tokens on the columns
     const uint16_t *const k = &lds.k[par][of][0][0], *const q = &lds.q[par][of][0][0];
-    f32x4_t x = zero, z = zero;
+    // The parts of S come off for 64 dims at a time, the products with the first ones in a sum of their own, so that the matrix
+    // pipe has work while the next is taken off (32 dims at a time 2-6 % slower, 128 twice as slow for want of registers).
+    constexpr int kSide = 2;
+    f32x4_t x = zero, z = zero, x_rest = zero, z_rest = zero;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const bf16x8_t kc = operand(k + (place ^ 32 * c)), qc = operand(q + (place ^ 32 * c));
-      const Split sp = cut(pick, s[2 * c], s[2 * c + 1]);
-      x = mfma_16x16x32(kc, sp.lo, x);
-      z = mfma_16x16x32(sp.lo, qc, z);
-      x = mfma_16x16x32(kc, sp.mid, x);
-      z = mfma_16x16x32(sp.mid, qc, z);
-      x = mfma_16x16x32(kc, sp.hi, x);
-      z = mfma_16x16x32(sp.hi, qc, z);
+    for (int h = 0; h < 4; h += kSide) {
+      bf16x8_t kc[kSide], qc[kSide], part[kSide];
+      f32x4_t a[kSide], b[kSide];
+      auto take_off = [&] {
+#pragma unroll
+        for (int c = 0; c < kSide; ++c) {
+          a[c] = mfma_16x16x32(pick.first, part[c], a[c]);
+          b[c] = mfma_16x16x32(pick.second, part[c], b[c]);
+        }
+      };
+      auto products = [&](f32x4_t& to_x, f32x4_t& to_z) {
+#pragma unroll
+        for (int c = 0; c < kSide; ++c) {
+          to_x = mfma_16x16x32(kc[c], part[c], to_x);
+          to_z = mfma_16x16x32(part[c], qc[c], to_z);
+        }
+      };
+      auto next_part = [&] {
+#pragma unroll
+        for (int c = 0; c < kSide; ++c) part[c] = upper(a[c], b[c]);
+      };
+#pragma unroll
+      for (int c = 0; c < kSide; ++c) {
+        kc[c] = operand(k + (place ^ 32 * (h + c)));
+        qc[c] = operand(q + (place ^ 32 * (h + c)));
+        a[c] = s[2 * (h + c)];
+        b[c] = s[2 * (h + c) + 1];
+      }
+      next_part();
+      take_off();
+      fence(); products(x, z);
+      next_part();
+      take_off();
+      fence(); products(x_rest, z_rest);
+      next_part();
+      fence(); products(x_rest, z_rest);
     }
+    x += x_rest;
+    z += z_rest;
     if (of == 0) slot_barrier();
     const ShortSystem& sys = lds.systems[of];
     auto of_rows = [&](const float (&m)[kShortChunk]) { return *reinterpret_cast<const f32x4_t*>(&m[4 * g]); };
@@ -290,7 +310,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
 int launch_gdn_short(const GdnParams& p, hipStream_t stream) {
   const int64_t heads = (int64_t)p.batch * p.hv;
   if (2 * heads > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  const bool halves = heads <= device_cus() && (2 * heads <= device_cus() || p.tokens <= 24 * (int64_t)p.batch);
+  // Half a head to a workgroup while that leaves one to a compute unit, or two and there is one chunk (8 requests of 32 heads: 16 tokens
+  // 10.4 us and 10.8 by whole heads, 32 tokens 12.9 and 11.7).
+  const bool halves = 2 * heads <= device_cus() || (heads <= device_cus() && p.tokens <= kShortChunk * (int64_t)p.batch);
   return halves ? launch_kernel(gdn_short_kernel<4>, dim3((unsigned)(2 * heads)), dim3(256), stream, p)
                 : launch_kernel(gdn_short_kernel<8>, dim3((unsigned)heads), dim3(512), stream, p);
 }
