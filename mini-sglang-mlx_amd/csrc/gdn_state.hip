@@ -166,7 +166,9 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 // Up to three tokens the token kernel is as fast (1.00-1.28 beyond 16 units, 1.03-1.14 up to 1, where this goes for up to 8 tokens).
 // What ends the chunks of 16 is not the even launch but one long request among short ones, whose chunks come one after the
 // other, 1.4-2 us for 16 tokens against 0.8-1.1 in the larger ones: of 54 tokens on average and 8-12 units 1.21 of the time before, of
-// 146 1.59.  Beyond 16 units the work of all is longer than such a chain.  An even launch has its requests' bits whatever their
+// 146 1.59.  The more units, the longer the work of all beside such a chain; one of 16 (8) times the others' length, by their mean: 17 units
+// 56 tokens 1.15 (0.89), 94 1.55 (1.21), 24 units 65 1.07 (0.79), 81 1.26 (0.89), 32 units 59 0.88, 88 1.13 (0.75), 48 units 79 0.82; even ones
+// 0.4-0.6 throughout.  An even launch has its requests' bits whatever their
 // number, which is why up to 16 units have one line.  345 launches of 1-48 requests, 8-64 heads, 2-3000 tokens, even, ragged and of
 // one long request: those this sends to chunks of 16, by their time before, 0.66 (geometric mean, 0.30-1.10).
 enum class GdnRoute { kTokens, kShort, kChunks };
@@ -175,7 +177,7 @@ static GdnRoute route_of(const GdnArgs& a) {
     return GdnRoute::kTokens;  // the others' offsets inside a chunk are 32 bits wide
   if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return GdnRoute::kTokens;  // loads of 16 bytes, stores of 8
   const int64_t heads = a.batch * a.hv;
-  const int64_t least = heads <= 32 ? 9 : heads <= 64 || heads > 512 ? 4 : 2, most = heads <= 512 ? 49 : 128;
+  const int64_t least = heads <= 32 ? 9 : heads <= 64 || heads > 512 ? 4 : 2, most = heads <= 512 ? 49 : std::min<int64_t>(128, 12 + 3 * heads / 32);
   return a.tokens < least * a.batch ? GdnRoute::kTokens : a.tokens < most * a.batch ? GdnRoute::kShort : GdnRoute::kChunks;
 }
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
