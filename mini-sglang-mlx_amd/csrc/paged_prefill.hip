@@ -1629,7 +1629,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
   if (to_partial) {
     const int row = row0 + w * 32 + c32;
     if (row < rows_total) {
-      const int qi = row / p.group;
+      const int qi = row_to_query(p, row);
       const int hh = row - qi * p.group;
       const int64_t at = p.ragged_tiles > 0 ? part_at + row
                                             : (int64_t)split * p.part_rows + (int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh;
@@ -1667,7 +1667,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
     const int lrow = pass * ROWS_PER_PASS + (tid >> 4);
     const int row = row0 + lrow;
     if (row < rows_total) {
-      const int qi = row / p.group;
+      const int qi = row_to_query(p, row);
       const int hh = row - qi * p.group;
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(os + (lrow * OROW + c * 8) * 2);
       st_global_b128(p.out + ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * D + c * 8, v);

@@ -621,7 +621,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     // ---- key split: normalised fp32 partial and log-sum-exp (base 2) per row, from registers
     const int row = row0 + group_row + c32;
     if (row < rows_total) {
-      const int qi = row / p.group;
+      const int qi = row_to_query(p, row);
       const int hh = row - qi * p.group;
       const int64_t at = p.ragged_tiles > 0 ? part_at + row
                                             : (int64_t)split * p.part_rows + (int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh;
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_tile256_kernel(PrefillParams
     const int lrow = pass * ROWS_PER_PASS + (tid >> 5);
     const int row = row0 + lrow;
     if (row < rows_total) {
-      const int qi = row / p.group;
+      const int qi = row_to_query(p, row);
       const int hh = row - qi * p.group;
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(os + (lrow * OROW + c * 8) * 2);
       st_global_b128(p.out + ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * kD + c * 8, v);

@@ -60,7 +60,8 @@ __device__ __forceinline__ u32x2_t lds_read_tr16(const unsigned char* p) {
 }
 
 // row / group, a multiplication: with 2^shift the power of two that holds the group, magic = ceil(2^(31 + shift) / group)
-// has 32 bits and the quotient is exact for rows below 2^31 (a division is 35 instructions).
+// has 32 bits and the quotient is exact for rows below 2^31 (a division is 35 instructions; eight of them where a block's rows leave
+// were 1-2 % of a small launch: five prompts of 34-392 tokens 22.5 -> 22.0 us, 13 of 10-18 at head_dim 256 11.4 -> 11.0).
 __device__ __forceinline__ int row_to_query(const PrefillParams& p, int row) {
   return (int)(__umulhi((uint32_t)row << 1, p.group_magic) >> p.group_shift);
 }
