@@ -4,16 +4,16 @@
 //
 // In one launch every workgroup of a value head, two or four of them, makes the systems of all its chunks beside the serial part, and
 // its waves share SIMDs and LDS with those of the chain that the launch waits for: 7.7 K cycles a chunk.  Here a system is made once,
-// and the chain is short: 5.1 K cycles a chunk where a request has four workgroups a value head, 7.6 K with two.
+// and the chain is short: 5.2 K cycles a chunk where a request has four workgroups a value head, 7.6 K with two.
 //
 // gdn_systems_kernel: one workgroup per chunk and value head; 17 us for 63 chunks of 32 heads, 29 us for 130 (before its 15 KiB of A
 // and inverses shared their place with K and T and three workgroups more fitted a compute unit: 21 and 37).  Bound by the
 // round trips to memory in front of its 5 K cycles of work (its request, K, the gates), then by its stores (3 TB/s).
-// gdn_serial_kernel: quarters by the chain of a state wave, 4.8 K of the 5.1 K cycles, 2.6 K of them matrix instructions, at 2.3 GHz (the
-// pipe is busy for 24 % of the SIMD cycles with one request, 43 % with the four below); halves where many requests fill the chip by the
+// gdn_serial_kernel: quarters by the chain of a state wave, 4.7 K of the 5.2 K cycles, 2.6 K of them matrix instructions, at 2.3 GHz (the
+// pipe is busy for 23 % of the SIMD cycles with one request, 43 % with the four below); halves where many requests fill the chip by the
 // matrix pipe: 1.12-1.15 PFLOP/s of bf16 products at 2.1 GHz, where a large product reaches 1.24.
 //
-// Both against the one launch, us: one request of 4005 tokens 208 -> 151; of 992, 1581, 4005 and 1601 tokens 232 -> 183; 2000 among five
+// Both against the one launch, us: one request of 4005 tokens 208 -> 156; of 992, 1581, 4005 and 1601 tokens 232 -> 183; 2000 among five
 // short ones 146 -> 95; eight of 1000 158 -> 156.
 #include "gdn_chunk_tiles.h"
 
@@ -222,24 +222,16 @@ struct Fetch {
     load(to_gates + (chunk & 1) * (uint32_t)sizeof(Gates) + 1024 * n, records + (int64_t)chunk * record_step,
          (uint32_t)(sizeof(ChunkRecord) - sizeof(Gates)) + 1024 * n + 16 * lane_id());
   }
-  // By wave w of four: K (Q), 4 loads; V and gates, ROWS / 32 and one more of waves 2 and 3; everything but T
-  __device__ __forceinline__ void k_four_waves(int chunk, int w) const {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) k_rows(chunk, 4 * w + i);
-  }
-  __device__ __forceinline__ void q_four_waves(int chunk, int w) const {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q_rows(chunk, 4 * w + i);
-  }
-  __device__ __forceinline__ void v_gates_four_waves(int chunk, int w) const {
+  // Everything of a chunk but T, by wave w of four: 9 loads, gates in front of them
+  __device__ __forceinline__ void four_waves(int chunk, int w) const {
     if (w >= 2) gates(chunk, w - 2);
 #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      k_rows(chunk, 4 * w + i);
+      q_rows(chunk, 4 * w + i);
+    }
+#pragma unroll
     for (int i = 0; i < ROWS / 32; ++i) v_rows(chunk, (ROWS / 32) * w + i);
-  }
-  __device__ __forceinline__ void four_waves(int chunk, int w) const {
-    v_gates_four_waves(chunk, w);
-    k_four_waves(chunk, w);
-    q_four_waves(chunk, w);
   }
   __device__ __forceinline__ void t_four_waves(int chunk, int w) const {
 #pragma unroll
@@ -521,13 +513,12 @@ __device__ __forceinline__ void half_helpers(SerialLds<64>& lds, const Fetch<64>
 
 // Quarters: X, R, U and S of 16 rows.
 //              state waves                          output waves                  helpers
-//     part 1   X of tokens 0-31                     Y of chunk j - 1, begun       T to LDS, K of chunk j + 1 asked for
-//     part 2   X of 32-63, R, U                     the rest of it, half of Z     V of chunk j + 1 asked for, P
-//     part 3   S                                    the rest of Z                 P to LDS, Q and T of chunk j + 1 asked for
-// S and U go to the output waves through LDS.  What the other waves do in a part is cut to fit beside the state waves' 1.0 K, 2.1 K and
-// 1.7 K cycles: with all of Z in part 3, and K, Q and V asked for in part 1, those waves were the last there by 0.2-0.35 K, 5.4 K cycles
-// a chunk instead of 5.1 K (one of 4005 tokens 159 -> 151 us, one of 1000 49 -> 47).  K's operands of part 1 read in the part
-// before it gave nothing.
+//     part 1   X of tokens 0-31                     Y of chunk j - 1, begun       T to LDS, chunk j + 1 asked for
+//     part 2   X of 32-63, R, U                     the rest of it, half of Z     P
+//     part 3   S                                    the rest of Z                 P to LDS, T of chunk j + 1 asked for
+// S and U go to the output waves through LDS.  With all of Z in part 3 the output waves were the last there, by 0.2 K cycles of
+// 5.36 K (one of 4005 tokens 159 -> 156 us, the four above 180.0 -> 178.9).  K, V and Q asked for in a part each, which takes the helpers
+// out of the way in part 1: 155.5, but the four 182; K's operands of part 1 read in the part before it: no change.
 __device__ __forceinline__ void quarter_state(QuarterLds& lds, int start, int end, int slot, int hv, int row, int w) {
   const int lane = lane_id();
   const int n_chunks = (end - start + kChunk - 1) / kChunk;
@@ -709,22 +700,19 @@ __device__ __forceinline__ void quarter_helpers(QuarterLds& lds, const Fetch<32>
   slot_barrier();
   for (int j = 0; j < n_chunks; ++j) {
     const bool more = j + 1 < n_chunks;
-    wait_all_vm();  // T, and Q in front of it
 #pragma unroll
     for (int i = 0; i < 5; ++i)
       if (i < 4 || w < 2) (&lds.t[0][0][0][0])[64 * (4 * i + w) + lane_id()] = t[i];
-    if (more) fetch.k_four_waves(j + 1, w);
+    if (more) fetch.four_waves(j + 1, w);
     slot_barrier();
-    if (more) fetch.v_gates_four_waves(j + 1, w);
     const f32x4_t x = blocks.make(lds, j & 1, w);
     most = largest(x, most);
     slot_barrier();
     blocks.store(pick, x, lds.p, w);
     if (more) {
-      fetch.q_four_waves(j + 1, w);
       load_t(j + 1);
-      if (w < 2) wait_vm_at_most<9>();  // all but Q and T
-      else wait_vm_at_most<8>();
+      if (w < 2) wait_vm_at_most<5>();  // all but T
+      else wait_vm_at_most<4>();
     } else {
       lds.p_largest[64 * w + lane_id()] = most;
     }
@@ -733,7 +721,7 @@ __device__ __forceinline__ void quarter_helpers(QuarterLds& lds, const Fetch<32>
   slot_barrier();
 }
 
-// Time of a chunk in halves, in quarters (7.4 K and 5.1 K cycles).
+// Time of a chunk in halves, in quarters (7.6 K and 5.2 K cycles).
 constexpr int kCost[2] = {16, 11};
 
 // Which request a place works for and how that is spread, the longest first: every request begins in halves, two places, and the
