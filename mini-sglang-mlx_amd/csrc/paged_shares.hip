@@ -22,8 +22,8 @@
 //
 // A decode step's new tokens (NEW) are stored here, normalised and rotated before where the step asks for that
 //   (new_token.h), instead of by a launch in front.  Norm, rotary embedding, store and attention of 4 requests of
-//   36-1022 tokens, 16 / 8 heads: 3.5 + 8.9 us in two launches, 9.8 in one, and one launch's host time less (28 layers
-//   359 -> 281 us); store and attention of 24 requests of 127-4095, 16 / 2 heads of 256: 4.5 + 25.0 us, 26.0 in one.
+//   36-1022 tokens, 16 / 8 heads: 3.5 + 8.9 us in two launches, 9.8 in one (8.1 since), and one launch's host time less (28 layers
+//   359 -> 281 us, now 240); store and attention of 24 requests of 127-4095, 16 / 2 heads of 256: 4.5 + 25.0 us, 26.0 in one (25.6 since).
 #include <algorithm>
 #include <cmath>
 
