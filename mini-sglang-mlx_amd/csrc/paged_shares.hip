@@ -325,7 +325,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   constexpr int I = NW == 4 ? 2 : 1;  // a thread's quads whose loads are in flight together
   const int64_t step = (int64_t)p.n_kv * p.cols;  // rows from one share to the next
   const int64_t first = row0 - share * step;
-  const uint32_t step_bytes = (uint32_t)step * (D * 4);  // (launch_shares() sees to it that a request's partials are below 2 GiB)
+  const uint32_t step_bytes = (uint32_t)step * (D * 4);  // (share_plan() sees to it that a request's partials are below 2 GiB)
   const Partials all(p.part_o + first * D, (uint32_t)n_shares * step_bytes);
   const float* const lse_from = p.part_lse + first;
   const int quads = ncols * kQuads;
@@ -484,6 +484,12 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
       while (!fits(len) && len < (1 << 19)) len = (len & (len - 1)) ? len / 3 * 4 : len / 2 * 3;
     }
   }
+  // The kernel's offsets inside one request's partials have 32 bits, its count of shares 16.  The lengths above keep to that by far
+  // (128 MiB and some hundred shares), whatever the requests' number: under a window a request is one share, or a few.  One set
+  // by hand is raised to what does.
+  const int64_t visible = each > 0 ? each : keys, row_bytes = n_kv * cols * head_dim * 4;
+  const int64_t most_of_one = std::min<int64_t>(std::max<int64_t>(0x7fffffffLL / row_bytes, 1), 0xffff);
+  len = std::max(len, (visible + most_of_one - 1) / most_of_one);
   plan.share_len = (int32_t)len;
   plan.heads_wg = (int32_t)heads;
   plan.share_waves = nw / plan.heads_wg;
@@ -553,8 +559,6 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   const bool rows = n.k != nullptr && a.qo_indptr != nullptr;  // kStoreRows
   const int64_t blocks = plan.max_shares * head_groups + (rows ? kRestBlocks : 0);
   if (blocks > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  // one request's partials (the plans' are below 128 MiB)
-  if ((plan.max_shares - a.batch + 1) * a.n_kv * cols * a.head_dim * 4 > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   ShareParams sp{};
   fill_splitkv_params(a, sp.s);
   char* ws = static_cast<char*>(a.workspace);

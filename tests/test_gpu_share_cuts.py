@@ -54,3 +54,20 @@ def test_few_wide_heads(gpu, lens, n_q, n_kv):
     print(f"wide heads {lens} {n_q}/{n_kv}", flush=True)
     for _ in range(2):
         _close(paged_decode_attention(g.q, g.k_cache, g.v_cache, g.kv_indptr, g.kv_indices, g.num_kv_splits, g.sm_scale, 32), want)
+
+
+def test_a_window_of_very_many_requests(gpu):
+    """17000 requests, 8 queries each: partials of more than 2 GiB in all, one share to a request."""
+    few, times, q_len, window = 34, 500, 8, 200
+    kv = [240 + 3 * i for i in range(few)]
+    wl = build_workload("many windows", "prefill", seed=34, n_q=32, n_kv=8, kv_lens=kv, extend_lens=[q_len] * few, sliding_window_size=window)
+    want = oracle.paged_prefill_attention(wl.q, wl.k_cache, wl.v_cache, wl.qo_indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, wl.sm_scale,
+                                          q_len, sliding_window_size=window, return_f32=True)[1]
+    g = wl.to(gpu)
+    indptr = lambda n: torch.cat([torch.zeros(1, dtype=torch.int64), torch.tensor(n * times).cumsum(0)]).int().to(gpu)  # noqa: E731
+    print("share cuts: 17000 windows", flush=True)
+    got = paged_prefill_attention(g.q.repeat(times, 1, 1), g.k_cache, g.v_cache, indptr([q_len] * few), indptr(kv), g.kv_indices.repeat(times),
+                                  g.prefix_lens.repeat(times), g.sm_scale, q_len, sliding_window_size=window).view(times, *want.shape)
+    _close(got[0], want)
+    _close(got[-1], want)
+    assert bool((got == got[0]).all())  # every request its own bits, wherever it stands

@@ -115,3 +115,19 @@ def test_launches_that_go_in_shares(batch, kv, heads, q, shares):
     if q == 1:  # with norm and rotary embedding a decode step is one launch where it goes in shares
         assert (lib.msgl_decode_step_workspace_bytes(batch, kv, n_q, n_kv, d, 1) > 0) is shares
     assert (lib.msgl_extend_step_workspace_bytes(batch, q * batch, kv, n_q, n_kv, d, q, 0, 0) > 0) is shares
+
+
+@pytest.mark.parametrize("batch,heads,ext,kv,window", [  # partials of more than 2 GiB in all
+    (17000, (32, 8, 128), 8, 240, 200), (25000, (32, 8, 128), 8, 128, 64), (40000, (64, 8, 128), 2, 1100, 1024)])
+def test_windows_of_very_many_requests_are_taken(batch, heads, ext, kv, window):
+    assert _prefill(batch, heads, ext, kv * batch, window=window) == ERR_LAUNCH
+
+
+@pytest.mark.parametrize("length", [1, 2, 300])
+def test_any_share_length_set_by_hand_is_taken(tuning, length):
+    from mini_sglang_amd_kernel import _lib
+
+    tuning(_lib.TUNE_SHARES, length | 1 << 20)
+    for kv in (100, 10**5, 10**7, 10**9):
+        assert _decode(1, (64, 8, 128), kv) == ERR_LAUNCH, kv
+        assert _decode(3, (32, 2, 256), kv) == ERR_LAUNCH, kv
