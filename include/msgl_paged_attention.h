@@ -372,6 +372,18 @@ MSGL_API int msgl_gdn_state_inplace_in(const void* q, const void* k, const void*
                            int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
                            int64_t v_stride0, int32_t single_token_mode, void* workspace,
                            size_t workspace_bytes, void* stream);
+/*
+ * The same with `longest`, most tokens of a request, for a caller that has the lengths on the host (0: not known).  Requests
+ * of a few dozen tokens are faster with it where none of them is long.  It decides which kernel takes the call, nothing else: with
+ * any value the results are right, to the rounding of another order of the same fp32 sums.
+ */
+MSGL_API int msgl_gdn_state_inplace_longest(const void* q, const void* k, const void* v, const void* g,
+                           const void* beta, void* state, const int32_t* slot_ids,
+                           const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
+                           int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
+                           int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
+                           int64_t v_stride0, int32_t single_token_mode, int64_t longest,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Tuning knobs, for benchmarking only (0 = built-in heuristic).  One set per HOST THREAD

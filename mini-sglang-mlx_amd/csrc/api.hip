@@ -893,15 +893,15 @@ size_t msgl_gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv,
   return msgl::gdn_state_workspace_bytes(tokens, batch, hv, single_token_mode != 0);
 }
 
-int msgl_gdn_state_inplace_in(const void* q, const void* k, const void* v, const void* g,
+int msgl_gdn_state_inplace_longest(const void* q, const void* k, const void* v, const void* g,
                            const void* beta, void* state, const int32_t* slot_ids,
                            const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
                            int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
                            int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
-                           int64_t v_stride0, int32_t single_token_mode, void* workspace,
-                              size_t workspace_bytes, void* stream) {
+                           int64_t v_stride0, int32_t single_token_mode, int64_t longest,
+                           void* workspace, size_t workspace_bytes, void* stream) {
   if (dk != 128 || dv != 128) return MSGL_ERR_GDN_DIMS;  // gdn_state.cpp:80-83
-  if (tokens < 0 || batch < 0 || hk <= 0 || hv <= 0 || num_slots < 0) return MSGL_ERR_SHAPE;
+  if (tokens < 0 || batch < 0 || hk <= 0 || hv <= 0 || num_slots < 0 || longest < 0) return MSGL_ERR_SHAPE;
   if (hv % hk != 0) return MSGL_ERR_HEAD_RATIO;          // gdn_state.cpp:76-79
   if (single_token_mode && tokens != batch) return MSGL_ERR_SHAPE;  // :107-111
   if (state_stride0 < hv * dv * dk || q_stride0 < hk * dk || k_stride0 < hk * dk ||
@@ -933,9 +933,22 @@ int msgl_gdn_state_inplace_in(const void* q, const void* k, const void* v, const
   a.k_stride0 = k_stride0;
   a.v_stride0 = v_stride0;
   a.single_token_mode = single_token_mode;
+  a.longest = longest;
   a.workspace = workspace;
   a.workspace_bytes = workspace_bytes;
   return msgl::launch_gdn_state(a, static_cast<hipStream_t>(stream));
+}
+
+int msgl_gdn_state_inplace_in(const void* q, const void* k, const void* v, const void* g,
+                           const void* beta, void* state, const int32_t* slot_ids,
+                           const int32_t* qo_indptr, void* y, int64_t tokens, int64_t batch,
+                           int64_t hk, int64_t hv, int64_t dk, int64_t dv, int64_t num_slots,
+                           int64_t state_stride0, int64_t q_stride0, int64_t k_stride0,
+                           int64_t v_stride0, int32_t single_token_mode, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  return msgl_gdn_state_inplace_longest(q, k, v, g, beta, state, slot_ids, qo_indptr, y, tokens, batch, hk, hv, dk, dv, num_slots,
+                                        state_stride0, q_stride0, k_stride0, v_stride0, single_token_mode, 0, workspace,
+                                        workspace_bytes, stream);
 }
 
 int msgl_gdn_state_inplace(const void* q, const void* k, const void* v, const void* g,

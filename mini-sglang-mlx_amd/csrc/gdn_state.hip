@@ -15,10 +15,11 @@
 // the next kDepth tokens are always in flight.  Decode (one token) is
 // HBM-bound: 2 * dv * dk * 4 bytes of state per (request, hv head) read and written once.
 // Prefill is a serial chain per row (as in the reference); parallelism is batch * hv * dv rows.  It takes
-// requests of very few tokens here; longer ones go in chunks (gdn_short.hip, gdn_chunk.hip, route_of() below).
+// requests of very few tokens here; longer ones go in chunks (gdn_short.hip, gdn_chunk.hip; gdn_route.h).
 #include <algorithm>
 
 #include "gdn_params.h"
+#include "gdn_route.h"
 
 namespace msgl {
 namespace {
@@ -157,28 +158,11 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
 
 }  // namespace
 
-// Which kernel takes a call with more than a token a request, by the mean length and units of 32 heads.  us, token by token / in chunks
-// of 16 (gdn_short.hip) / in chunks of 64 (gdn_chunk.hip, whose time for up to 64 tokens does not depend on their number):
-//     requests of 32 heads   1: 4 tokens 5.8 / 5.8 / 9.3, 16 8.6 / 5.9 / 9.5, 32 13.4 / 7.1 / 9.3, 64 23 / 9.6 / 9.5
-//                            4: 4 tokens 9.8 / 7.1 / 12.1, 16 17 / 7.5 / 12.3, 32 28 / 8.6 / 12.4, 64 47 / 11.6 / 12.7
-//                            8: 4 tokens 11 / 9.4 / 25, 16 21 / 10.5 / 25, 48 47 / 13.6 / 25, 256 - / 41 / 57
-//                           16: 4 tokens 20 / 16 / 51, 16 37 / 16 / 50, 64 110 / 25 / 51, 256 - / 69 / 103
-// Up to three tokens the token kernel is as fast (1.00-1.28 beyond 16 units, 1.03-1.14 up to 1, where this goes for up to 8 tokens).
-// What ends the chunks of 16 is not the even launch but one long request among short ones, whose chunks come one after the
-// other, 1.4-2 us for 16 tokens against 0.8-1.1 in the larger ones: of 54 tokens on average and 8-12 units 1.21 of the time before, of
-// 146 1.59.  The more units, the longer the work of all beside such a chain; one of 16 (8) times the others' length, by their mean: 17 units
-// 56 tokens 1.15 (0.89), 94 1.55 (1.21), 24 units 65 1.07 (0.79), 81 1.26 (0.89), 32 units 59 0.88, 88 1.13 (0.75), 48 units 79 0.82; even ones
-// 0.4-0.6 throughout.  An even launch has its requests' bits whatever their
-// number, which is why up to 16 units have one line.  345 launches of 1-48 requests, 8-64 heads, 2-3000 tokens, even, ragged and of
-// one long request: those this sends to chunks of 16, by their time before, 0.66 (geometric mean, 0.30-1.10).
-enum class GdnRoute { kTokens, kShort, kChunks };
 static GdnRoute route_of(const GdnArgs& a) {
   if (a.v_stride0 >= (1 << 24) || a.k_stride0 >= (1 << 24) || a.q_stride0 >= (1 << 24) || a.hv >= (1 << 17))
     return GdnRoute::kTokens;  // the others' offsets inside a chunk are 32 bits wide
   if ((uintptr_t)a.v % 16 || a.v_stride0 % 8 || (uintptr_t)a.y % 8) return GdnRoute::kTokens;  // loads of 16 bytes, stores of 8
-  const int64_t heads = a.batch * a.hv;
-  const int64_t least = heads <= 32 ? 9 : heads <= 64 || heads > 512 ? 4 : 2, most = heads <= 512 ? 49 : std::min<int64_t>(128, 12 + 3 * heads / 32);
-  return a.tokens < least * a.batch ? GdnRoute::kTokens : a.tokens < most * a.batch ? GdnRoute::kShort : GdnRoute::kChunks;
+  return gdn_route(a.tokens, a.batch, a.hv, a.longest, device_cus());
 }
 static thread_local int t_force_rows = 0;  // benchmarking switch, one value per host thread
 // Room for the systems of all chunks where making those in a launch of their own pays (gdn_long.hip), 0 elsewhere.  The second

@@ -187,6 +187,7 @@ struct GdnArgs {
   int64_t tokens, batch, hk, hv;
   int64_t state_stride0, q_stride0, k_stride0, v_stride0;  // elements
   int32_t single_token_mode;
+  int64_t longest;  // most tokens of a request, 0: not known (the route is chosen by it, the results do not depend on it)
   void* workspace;  // may be null: requests of many chunks then take the one launch
   size_t workspace_bytes;
 };

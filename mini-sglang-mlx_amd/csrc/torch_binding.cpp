@@ -701,13 +701,14 @@ PyObject* extend_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   });
 }
 
-// ---- gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr, single_token_mode) -> y -------
+// ---- gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr, single_token_mode, longest) -> y -----
 PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
-  return guarded(args, n_args, 9, [](PyObject* const* a) -> PyObject* {
+  return guarded(args, n_args, 10, [](PyObject* const* a) -> PyObject* {
     static const char op[] = "gdn_state_inplace";
     const Tensor &q = tensor(a[0], "q"), &k = tensor(a[1], "k"), &v = tensor(a[2], "v"), &g = tensor(a[3], "g");
     const Tensor &beta = tensor(a[4], "beta"), &state = tensor(a[5], "state"), &slots = tensor(a[6], "slot_ids");
     const bool single = truth(a[8]);
+    const int64_t longest = a[9] == Py_None ? 0 : std::max<int64_t>(integer(a[9]), 0);
     if (q.dim() != 3 || k.dim() != 3) fail(op, "q and k must be 3D");
     if (v.dim() != 3) fail(op, "v must be 3D");
     if (g.dim() != 2 || beta.dim() != 2) fail(op, "g and beta must be 2D");
@@ -756,9 +757,9 @@ PyObject* gdn_state_inplace(PyObject*, PyObject* const* args, Py_ssize_t n_args)
           bytes = 0;
         }
       }
-      rc = msgl_gdn_state_inplace_in(q.data_ptr(), k.data_ptr(), v.data_ptr(), gc.data_ptr(), bc.data_ptr(), state.data_ptr(),
+      rc = msgl_gdn_state_inplace_longest(q.data_ptr(), k.data_ptr(), v.data_ptr(), gc.data_ptr(), bc.data_ptr(), state.data_ptr(),
                                   ints(sc), single ? nullptr : ints(ipc), y.data_ptr(), tokens, batch, hk, hv, dk, dv,
-                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, ws.ptr(), bytes, on.ptr());
+                                  state.size(0), ss, qs, ks, vs, single ? 1 : 0, longest, ws.ptr(), bytes, on.ptr());
     }
     check_rc(op, rc);
     return THPVariable_Wrap(std::move(y));

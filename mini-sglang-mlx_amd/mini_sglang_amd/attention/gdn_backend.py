@@ -37,8 +37,11 @@ class GDNBackend:
             batch.mamba_slot_ids = torch.tensor(slots, dtype=torch.int32, device=device)
         # one field for both phases: ragged token offsets in prefill, 0..batch in decode
         if batch.mamba_prefill_indptr is None:
-            lens = torch.tensor([0] + [req.extend_len for req in batch.reqs], dtype=torch.int64)
-            batch.mamba_prefill_indptr = torch.cumsum(lens, 0).to(torch.int32).to(device)
+            lens = [0] + [req.extend_len for req in batch.reqs]
+            batch.mamba_prefill_indptr = torch.cumsum(torch.tensor(lens, dtype=torch.int64), 0).to(torch.int32).to(device)
+            # the longest goes with the offsets it belongs to: batches of any class, and offsets
+            # that a caller puts there itself, need no field for it
+            batch.mamba_prefill_indptr.max_len_extend = max(lens)
 
     # ---- one layer's recurrence over the batch (gdn_backend.py:69-98) --------------------------
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
@@ -48,7 +51,8 @@ class GDNBackend:
         assert batch.mamba_prefill_indptr is not None
         return gdn_state_inplace(q, k, v, g, beta, self.mamba_pool.temporal_state(linear_layer_idx),
                                  batch.mamba_slot_ids, batch.mamba_prefill_indptr,
-                                 single_token_mode=batch.is_decode)
+                                 single_token_mode=batch.is_decode,
+                                 max_len_extend=getattr(batch.mamba_prefill_indptr, "max_len_extend", None))
 
     # ---- speculative verify (gdn_backend.py:100-135) ---------------------------------------------
     def forward_verify(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
@@ -61,7 +65,8 @@ class GDNBackend:
         batch.gdn_verify_captured[linear_layer_idx] = (q, k, v, g, beta)
         return gdn_state_inplace(q, k, v, g, beta, self.mamba_pool.temporal_state(linear_layer_idx),
                                  batch.mamba_scratch_slots, batch.mamba_verify_indptr,
-                                 single_token_mode=False)
+                                 single_token_mode=False,
+                                 max_len_extend=getattr(batch, "mamba_verify_width", None))
 
     def commit_verify(self, batch, num_accepted_host: List[int]) -> None:
         """Request ``i`` accepted ``j_i`` drafts: its main slot advances by the first ``j_i + 1``
@@ -94,7 +99,7 @@ class GDNBackend:
             gdn_state_inplace(q.index_select(0, idx), k.index_select(0, idx), v.index_select(0, idx),
                               g.index_select(0, idx), beta.index_select(0, idx),
                               self.mamba_pool.temporal_state(layer), main, indptr,
-                              single_token_mode=False)
+                              single_token_mode=False, max_len_extend=int(lengths.max()))
             conv = self.mamba_pool.conv_state(layer, 0)
             conv[main.long()] = self.mamba_pool.conv_window(layer, 0)[scratch, row]
         batch.gdn_verify_captured = None  # the verify inputs may be freed now

@@ -300,20 +300,24 @@ def extend_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_loc: torc
 def gdn_state_inplace(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
                       beta: torch.Tensor, state: torch.Tensor, slot_ids: torch.Tensor,
                       qo_indptr: torch.Tensor, single_token_mode: bool = False, *,
-                      stream=None) -> torch.Tensor:
+                      stream=None, max_len_extend: Optional[int] = None) -> torch.Tensor:
     """Gated delta-rule recurrence over each request's tokens with the fp32 state of slot
     ``slot_ids[b]`` updated in place; returns ``y`` ``(tokens, hv, dv)`` bf16.
 
     Drop-in for ``mini_sglang_mlx_kernel.gdn_state_inplace`` (bindings.cpp:56-65,
     gdn_state.cpp:87-135): same argument order, ``single_token_mode`` (decode: one token per
     request, ``qo_indptr`` ignored) and error texts (gdn_state.cpp:26-84, 107-126).
+
+    ``max_len_extend``, most tokens of a request, is for callers that have the lengths on the host:
+    requests of a few dozen tokens are faster with it where none of them is long.  It chooses the
+    kernel and nothing else; any value gives right results.
     """
     if stream is None:
         return _native.gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr,
-                                         single_token_mode)
+                                         single_token_mode, max_len_extend)
     with _on_stream(stream, q):
         return _native.gdn_state_inplace(q, k, v, g, beta, state, slot_ids, qo_indptr,
-                                         single_token_mode)
+                                         single_token_mode, max_len_extend)
 
 
 def fast_compare_key(a: torch.Tensor, b: torch.Tensor) -> int:

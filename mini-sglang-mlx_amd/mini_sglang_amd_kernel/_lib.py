@@ -73,6 +73,10 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
          _i64, _i64, _i64, _i64, _i32, _vp, _sz, _vp]),
+    "msgl_gdn_state_inplace_longest": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+         _i64, _i64, _i64, _i64, _i32, _i64, _vp, _sz, _vp]),
     # include/msgl_state_pool.h (recurrent-state pool)
     "msgl_copy_state_slots": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _vp]),
     # include/msgl_radix_cache.h (host-side prefix cache)

@@ -39,7 +39,8 @@ def _run(gpu, lengths, hk, hv, decay, seed, place=None):
     q, k, v = (t.unflatten(1, (-1, 128)) for t in proj.split([hk * 128, hk * 128, hv * 128], dim=1))
     state = torch.from_numpy(d["state"].copy()).to(gpu)
     print(f"gdn short {lengths[:6]} of {batch} hk {hk} hv {hv} {decay} {place}", flush=True)
-    y = gdn_state_inplace(q, k, v, to(d["g"]), to(d["beta"]), state, torch.from_numpy(slots).to(gpu), torch.from_numpy(indptr).to(gpu))
+    y = gdn_state_inplace(q, k, v, to(d["g"]), to(d["beta"]), state, torch.from_numpy(slots).to(gpu), torch.from_numpy(indptr).to(gpu),
+                         max_len_extend=max(lengths))
     torch.cuda.synchronize()
     return (y.float().cpu().numpy(), state.cpu().numpy()), want, d["state"], slots
 
@@ -63,7 +64,18 @@ def test_against_the_oracle(gpu, lengths, hk, hv, decay):
     ("v", (5, 1, 37), np.inf), ("v", (17, 1, 127), np.nan), ("k", (16, 0, 5), np.nan), ("k", (3, 0, 64), -np.inf), ("q", (11, 1, 99), np.inf),
     ("q", (15, 0, 0), np.nan), ("g", (9, 2), np.nan), ("g", (16, 3), np.inf), ("beta", (2, 3), np.inf), ("state", (1, 2, 17, 64), np.nan)])
 def test_values_that_are_not_finite_stay_in_their_place(gpu, lengths, hk, hv, name, at, value):
-    got, want, _, _ = _run(gpu, lengths, hk, hv, "some", hv, (name, at, value))
+    _same_places(*_run(gpu, lengths, hk, hv, "some", hv, (name, at, value))[:2])
+
+
+# beyond the first four chunks of a request of nine, and behind it
+@pytest.mark.parametrize("name,at,value", [
+    ("v", (64, 1, 37), np.inf), ("k", (100, 0, 5), np.nan), ("k", (129, 1, 64), -np.inf), ("q", (79, 1, 99), np.inf), ("g", (127, 2), np.nan),
+    ("beta", (65, 3), np.inf), ("v", (128, 0, 127), np.nan), ("v", (135, 0, 0), np.inf)])
+def test_values_that_are_not_finite_in_later_groups(gpu, name, at, value):
+    _same_places(*_run(gpu, [130, 10, 4, 6, 3, 2, 9, 1], 2, 4, "some", 11, (name, at, value))[:2])
+
+
+def _same_places(got, want):
     for a, b, atol, rtol in zip(got, want, (1e-5, 2e-6 * 4), (2.0 ** -8, 2e-6)):
         finite = np.isfinite(b)
         np.testing.assert_array_equal(np.isfinite(a), finite)
