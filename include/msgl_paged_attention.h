@@ -419,7 +419,8 @@ MSGL_API int msgl_gdn_state_inplace_longest(const void* q, const void* k, const 
  *   MSGL_TUNE_CLOCK_PROBE    measurement aid: the value is a device pointer to two int64 (0: none).
  *                            Workgroup 0 of every attention kernel launched by this thread then
  *                            leaves there the shader cycles and the 100 MHz wall ticks it lived
- *                            for: cycles / ticks x 0.1 = the shader clock in GHz under that kernel
+ *                            for (in the launch of shares, from where it has found its share):
+ *                            cycles / ticks x 0.1 = the shader clock in GHz under that kernel
  *   MSGL_TUNE_SHARES         decode and verify on one launch of per-request key shares instead of
  *                            equal segments and a merge: negative: never; 0: chosen from the sizes;
  *                            positive: always, with share_len | kv heads per workgroup << 20

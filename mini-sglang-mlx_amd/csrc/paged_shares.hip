@@ -175,6 +175,8 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(p, p.nt, p.n_kv * D, threadIdx.x);
     return;
   }
+  // From here on, not from the kernel's beginning as elsewhere: the search is not in the interval.  (Stamps at the beginning cost every
+  // launch 0.03 us, with a test of whether there is a probe 0.14.)
   const ClockProbe clock_probe_(p.clock_probe);
   // what the rest of the way begins with and only the request's number leads to
   const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
