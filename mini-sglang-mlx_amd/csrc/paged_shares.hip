@@ -158,10 +158,13 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   const int lane = lane_id();
   const int t16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int item = blockIdx.x >> shape.groups(), hg = blockIdx.x & ((1u << shape.groups()) - 1);
+  int item, hg;
   if (shape.groups() == ShareShape::kNoShift) {
     item = blockIdx.x / sp.head_groups;
     hg = blockIdx.x - item * sp.head_groups;
+  } else {
+    item = blockIdx.x >> shape.groups();
+    hg = blockIdx.x & ((1u << shape.groups()) - 1);
   }
   const int share_waves = 1 << shape.waves();
   const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
