@@ -49,9 +49,11 @@ class GDNBackend:
         """``y`` of shape ``(tokens, hv, dv)``; the state of every request's slot is advanced."""
         assert batch.mamba_slot_ids is not None
         assert batch.mamba_prefill_indptr is not None
-        return gdn_state_inplace(q, k, v, g, beta, self.mamba_pool.temporal_state(linear_layer_idx),
-                                 batch.mamba_slot_ids, batch.mamba_prefill_indptr,
-                                 single_token_mode=batch.is_decode,
+        state = self.mamba_pool.temporal_state(linear_layer_idx)
+        if batch.is_decode:
+            return gdn_state_inplace(q, k, v, g, beta, state, batch.mamba_slot_ids,
+                                     batch.mamba_prefill_indptr, True)
+        return gdn_state_inplace(q, k, v, g, beta, state, batch.mamba_slot_ids, batch.mamba_prefill_indptr,
                                  max_len_extend=getattr(batch.mamba_prefill_indptr, "max_len_extend", None))
 
     # ---- speculative verify (gdn_backend.py:100-135) ---------------------------------------------
