@@ -15,3 +15,21 @@ def test_head_dim_256(batch, keys, n_q, n_kv, shares):
     lib = _lib.load()
     assert (lib.msgl_decode_step_workspace_bytes(batch, keys, n_q, n_kv, 256, 1) > 0) is shares
     assert lib.msgl_decode_step_workspace_bytes(batch, keys, n_q, n_kv, 256, 1) <= lib.msgl_paged_decode_workspace_bytes(batch, keys, n_q, n_kv, 256)
+
+
+@pytest.mark.parametrize("batch,keys,n_q,n_kv,shares", [  # few pairs, one whole column tile: slower in shares between the two lines
+    (1, 1500, 16, 1, True), (1, 2000, 16, 1, False), (2, 2 * 8000, 16, 1, False), (3, 3 * 16000, 16, 1, False), (3, 3 * 16500, 16, 1, True),
+    (4, 4 * 8000, 16, 1, True), (1, 8000, 24, 2, False), (1, 3500, 24, 2, True), (1, 8000, 8, 1, True), (1, 8000, 64, 4, True)])
+def test_few_pairs_with_many_columns(batch, keys, n_q, n_kv, shares):
+    from mini_sglang_amd_kernel import _lib
+
+    assert (_lib.load().msgl_decode_step_workspace_bytes(batch, keys, n_q, n_kv, 256, 1) > 0) is shares
+
+
+@pytest.mark.parametrize("batch,heads,window,shares", [
+    (1, (8, 1), 256, True), (1, (8, 1), 1024, False), (3, (8, 1), 2048, False), (4, (8, 1), 1024, True), (1, (16, 4), 4096, True)])
+def test_windows_of_few_pairs(batch, heads, window, shares):
+    from mini_sglang_amd_kernel import _lib
+
+    lib, (n_q, n_kv) = _lib.load(), heads
+    assert (lib.msgl_extend_step_workspace_bytes(batch, 2 * batch, 30000 * batch, n_q, n_kv, 256, 2, 0, window) > 0) is shares
