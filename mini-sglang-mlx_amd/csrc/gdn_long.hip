@@ -13,7 +13,7 @@
 // pipe is busy for 23 % of the SIMD cycles with one request, 43 % with the four below); halves where many requests fill the chip by the
 // matrix pipe: 1.12-1.15 PFLOP/s of bf16 products at 2.1 GHz, where a large product reaches 1.24.
 //
-// Both against the one launch, us: one request of 4005 tokens 208 -> 156; of 992, 1581, 4005 and 1601 tokens 232 -> 183; 2000 among five
+// Both against the one launch, us: one request of 4005 tokens 208 -> 156; of 992, 1581, 4005 and 1601 tokens 232 -> 178; 2000 among five
 // short ones 146 -> 95; eight of 1000 158 -> 156.
 #include "gdn_chunk_tiles.h"
 
@@ -517,7 +517,7 @@ __device__ __forceinline__ void half_helpers(SerialLds<64>& lds, const Fetch<64>
 //     part 2   X of 32-63, R, U                     the rest of it, half of Z     P
 //     part 3   S                                    the rest of Z                 P to LDS, T of chunk j + 1 asked for
 // S and U go to the output waves through LDS.  With all of Z in part 3 the output waves were the last there, by 0.2 K cycles of
-// 5.36 K (one of 4005 tokens 159 -> 156 us, the four above 180.0 -> 178.9).  K, V and Q asked for in a part each, which takes the helpers
+// 5.36 K (one of 4005 tokens 159 -> 156 us, the four above 179.3 -> 177.5).  K, V and Q asked for in a part each, which takes the helpers
 // out of the way in part 1: 155.5, but the four 182; K's operands of part 1 read in the part before it: no change.
 __device__ __forceinline__ void quarter_state(QuarterLds& lds, int start, int end, int slot, int hv, int row, int w) {
   const int lane = lane_id();

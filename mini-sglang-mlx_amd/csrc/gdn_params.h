@@ -1,5 +1,6 @@
-// Launch parameters and small pieces shared by the two gated delta-rule kernels (gdn_state.hip: token
-// after token; gdn_chunk.hip: chunks of 64 tokens on the matrix cores).
+// Launch parameters and small pieces shared by the gated delta-rule kernels (gdn_state.hip: token after
+// token; gdn_short.hip and gdn_chunk.hip: chunks of 16 and of 64 tokens on the matrix cores; gdn_long.hip:
+// chunks of 64 in two launches).
 #pragma once
 #include "msgl_device.h"
 #include "msgl_internal.h"

@@ -23,10 +23,10 @@ inline bool gdn_chunks_before_tokens(int64_t tokens, int64_t batch, int64_t hv, 
 // `longest`: most tokens of a request, 0: not known.
 //
 // By the mean length and units of 32 heads, even launches, us, token by token / in chunks of 16 / in chunks of 64:
-//     1 unit: 4 tokens 5.8 / 5.8 / 9.3, 16 8.6 / 5.9 / 9.5, 32 13.4 / 7.1 / 9.3, 64 23 / 9.6 / 9.5
-//     4:      4 tokens 9.8 / 7.1 / 12.1, 16 17 / 7.5 / 12.3, 32 28 / 8.6 / 12.4, 64 47 / 11.6 / 12.7
-//     8:      4 tokens 11 / 9.4 / 25, 16 21 / 10.5 / 25, 48 47 / 13.6 / 25, 256 - / 41 / 57
-//     16:     4 tokens 20 / 16 / 51, 16 37 / 16 / 50, 64 110 / 25 / 51, 256 - / 69 / 103
+//     1 unit: 4 tokens 5.7 / 5.8 / 9.2, 16 8.3 / 6.0 / 9.2, 32 13.0 / 6.7 / 9.3, 64 23 / 8.9 / 9.2
+//     4:      4 tokens 9.8 / 7.1 / 12.1, 16 17 / 7.2 / 12.1, 32 27 / 8.2 / 12.1, 64 46 / 10.5 / 12.4
+//     8:      4 tokens 16 / 9.7 / 25, 16 28 / 10.6 / 25, 48 62 / 13.0 / 25, 256 - / 40 / 56
+//     16:     4 tokens 20 / 15 / 50, 16 38 / 15.5 / 50, 64 112 / 25 / 51, 256 - / 73 / 107
 // Up to three tokens the token kernel is as fast (1.00-1.28 beyond 16 units, 1.03-1.14 up to 1, where this goes for up to 8 tokens).
 //
 // Against token by token chunks of 16 are faster whatever the lengths (850 launches of 1-200 requests, 4-64 heads, even, ragged, of

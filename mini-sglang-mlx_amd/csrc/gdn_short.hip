@@ -12,17 +12,18 @@
 //     Y = G Z + P U                 4 fp32 products, transposed: a lane stores four rows of a token
 //     S = G S + K^T (tail U)        16 products: two parts of U side by side in the 32 columns of one, the third beside zeros
 // A workgroup takes a head, or half of one where that fills the chip better (launch_gdn_short()).  Chunks go in groups of four: each
-// of four waves fetches the rows of one and makes its system; the next group's rows are under way meanwhile.  K and Q come by
+// of four waves fetches the rows of one and makes its system; the next group's rows are asked for in a group's first chunk.  K and Q come by
 // LDS, four whole rows a load, once for all waves: as operands straight from memory, 16 rows a load, the address unit was the limit
 // (16 requests of 64 tokens 38 us, now 26).  74 KB of LDS and 128 registers let two workgroups of eight waves share a compute unit
 // (lane_here() keeps what only a group's start needs out of the registers: in it they were 16 too many, 5-15 % of the time).
 //
-// What bounds it: up to 16 tokens the state, read and written (16 requests of 32 heads 16.2 us, 4.1 TB/s, before 37); beyond, the
-// chain of a chunk, 1.3 us for one to four requests, and from eight on the pipes of a SIMD, 0.23 us a chunk and request, half
-// of it matrix instructions.  us, by requests of 32 heads and tokens, before and now: 1 x 16 8.6 and 6.4, 32 9.4 and 7.1; 4 x 16 12.1 and
-// 7.5; 8 x 16 29 and 11, 40 25.6 and 13.8; 16 x 40 51 and 22.5; 24 x 100 106 and 57; 48 x 8 57 and 44.  Four more waves
-// that fetch and make the systems ahead: 1.1 us a chunk for one request, no change for four; S's parts of 64 dims side by side: 4 % faster for
-// one request, 10 % slower for sixteen (registers).
+// What bounds it: up to 16 tokens the state, read and written (16 requests of 32 heads 15.5 us, 4.3 TB/s, token by token 37.5); beyond, the
+// chain of a chunk, 1.25 us for one request, 1.45 for four, and from eight on the issue of the waves of a SIMD, 0.2-0.3 us a chunk and request, the
+// matrix pipe busy for a quarter to 38 % of the cycles.  A chunk ends in a wait for all memory operations of its wave (behind V's loads, which
+// are under a condition, and the masked rows of Y the compiler does not know how many are under way): V's round trip is in every chunk,
+// that of the next group's K and Q in a group's first.  us, by requests of 32 heads and tokens, before and now: 1 x 16 8.3 and 6.0, 32 9.3
+// and 6.7; 4 x 16 12.1 and 7.2; 8 x 16 24.9 and 10.6, 40 24.9 and 12.9; 16 x 40 50.7 and 21.5; 24 x 80 105 and 44; 48 x 8 57 and 43.  Four more
+// waves that fetch and make the systems ahead: 1.1 us a chunk for one request, no change for four.
 //
 // Precision: fp32 throughout, the parts are exact (see upper()).  The state's error against 64 bits, rms: 1.0-1.7e-8 at states of 0.1
 // (the token kernel 1.2-2.5e-8, chunks of 64 1.2-1.8e-8); the chunk's addition to S in a sum of its own, joined by one multiply-add, is 7-10 %

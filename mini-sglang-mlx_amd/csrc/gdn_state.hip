@@ -175,7 +175,7 @@ static thread_local int t_force_rows = 0;  // benchmarking switch, one value per
 // lose either.  Few heads a request bring more requests to as many workgroups, and even ones then lose (us, in one launch and in two: 32 of
 // 452 tokens, 4 heads, 43.6 and 49.6, 64 of 319 69 and 75, 10 of 445 29.6 and 33.6), so the lines go up with the requests' number.  750 launches at
 // 2-128 heads, two launches by one: those beyond the lines 0.903 (geometric mean of 583, worst 1.01), those that this leaves behind 0.991 of 167.
-// us: one of 4000 208 -> 159, eight of 200-1600 148 -> 139, 2060 among five of 100-260 150 -> 91.  A request and 32 heads
+// us: one of 4000 208 -> 156, eight of 200-1600 148 -> 139, 2060 among five of 100-260 150 -> 91.  A request and 32 heads
 // have 640 KiB for every 64 tokens; a launch that would need more than 2 GiB goes without.
 size_t gdn_state_workspace_bytes(int64_t tokens, int64_t batch, int64_t hv, bool single_token) {
   if (single_token || batch <= 0 || hv <= 0 || t_force_rows > 0) return 0;
