@@ -80,7 +80,7 @@ int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t ma
 bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv, int64_t keys, int64_t n_kv,
                    int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
-  if (msgl::few_pairs_in_segments(batch * n_kv, keys / batch, head_dim, cols, true)) return false;
+  if (msgl::few_pairs_in_segments(batch, n_kv, keys / batch, head_dim, cols, true)) return false;
   const int64_t blocks = batch * (n_kv / plan.heads_wg), cus = msgl::device_cus();
   if (blocks > cus && 3 * blocks < 2 * cus * ((blocks + cus - 1) / cus)) return false;
   return cols <= 32 || plan.heads_wg == 1;
@@ -429,7 +429,7 @@ static bool shares_route(const msgl::SharePlan& plan, bool window_share, int64_t
                          int64_t n_kv, int64_t group, int64_t max_len_extend, int64_t head_dim, int64_t window) {
   if (plan.share_len == 0) return false;
   if (window_share) return true;
-  if (keys < total_kv && msgl::few_pairs_in_segments(batch * n_kv, keys / batch, head_dim, group * max_len_extend, true)) return false;
+  if (keys < total_kv && msgl::few_pairs_in_segments(batch, n_kv, keys / batch, head_dim, group * max_len_extend, true)) return false;
   return use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) &&
          !window_prefers_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim, window) &&
          msgl::shares_preferred(plan, batch, keys, n_kv, head_dim, group * max_len_extend);

@@ -89,7 +89,7 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv);
 // whether the launch is small enough for its shares to beat the segment kernel
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols);
 // whether segments are faster for so few (request, kv head) pairs of `mean` visible keys; windowed: all of them have as many
-bool few_pairs_in_segments(int64_t pairs, int64_t mean, int64_t head_dim, int64_t cols, bool windowed);
+bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t head_dim, int64_t cols, bool windowed);
 int device_cus();  // paged_splitkv.hip
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);
 int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& plan, hipStream_t stream);

@@ -511,14 +511,16 @@ SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
   return plan;
 }
 
-// head_dim 256, up to three pairs, more than half a column tile: the last share's part, the others' partials, is long, and nothing
+// head_dim 256, up to three pairs (six of one kv head), more than half a column tile: the last share's part, the others' partials, is long, and nothing
 // else is left to run meanwhile.  Shares by segments, 700 launches of 1-11 pairs, geometric mean (worst): whole tiles, up to three
 // pairs, decode and verify of 512-1024 keys 0.87 (0.99), 1024-2048 1.00 (1.16), to 16384 1.07 (1.24), beyond 0.85; with norm and rotary embedding,
 // which go in a launch of their own then, 0.84, 0.93, 1.05 (1.23), 1.00; windows of 256 0.80, 1024 1.04 (1.10), 4096 1.11 (1.15).  9-12 columns: to 4096
-// 0.85, to 16384 1.02 (1.12), beyond 0.92.  Four pairs and more 0.88 (1.16).
-bool few_pairs_in_segments(int64_t pairs, int64_t mean, int64_t head_dim, int64_t cols, bool windowed) {
-  if (t_force > 0 || head_dim != 256 || pairs > 3 || cols <= 8 || mean > 16384) return false;
-  return mean > (cols <= 12 ? 4096 : windowed ? 1024 : 1536);
+// 0.85, to 16384 1.02 (1.12), beyond 0.92.  Four pairs and more 0.88 (1.16); of one kv head four to six whole tiles of 1500-2500 keys
+// 1.00 (1.13), to 8000 1.06 (1.21), beyond 0.92, seven and eight to 8000 0.99.
+bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t head_dim, int64_t cols, bool windowed) {
+  if (t_force > 0 || head_dim != 256 || cols <= 8) return false;
+  if (batch * n_kv <= 3) return mean <= 16384 && mean > (cols <= 12 ? 4096 : windowed ? 1024 : 1536);
+  return n_kv == 1 && batch <= 6 && cols > 12 && mean > 2500 && mean <= 8000;
 }
 
 // Measured against the segment kernel and its merge on 400 random shapes (1-256 requests of 1-60 K
@@ -543,7 +545,7 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
   if (t_force > 0) return true;
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
-  if (few_pairs_in_segments(units, mean, head_dim, cols, false)) return false;
+  if (few_pairs_in_segments(batch, n_kv, mean, head_dim, cols, false)) return false;
   if (wide_heads_alone(batch, n_kv, head_dim)) {
     // Beyond some MiB the shares have to fill the chip: a launch takes as long as its longest share.  By MiB of keys and values
     // and what part of a round of shares as long as the longest they are, shares by segments (geometric mean, worst): up to 64 0.65

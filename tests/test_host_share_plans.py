@@ -19,7 +19,8 @@ def test_head_dim_256(batch, keys, n_q, n_kv, shares):
 
 @pytest.mark.parametrize("batch,keys,n_q,n_kv,shares", [  # few pairs, one whole column tile: slower in shares between the two lines
     (1, 1500, 16, 1, True), (1, 2000, 16, 1, False), (2, 2 * 8000, 16, 1, False), (3, 3 * 16000, 16, 1, False), (3, 3 * 16500, 16, 1, True),
-    (4, 4 * 8000, 16, 1, True), (1, 8000, 24, 2, False), (1, 3500, 24, 2, True), (1, 8000, 8, 1, True), (1, 8000, 64, 4, True)])
+    (4, 4 * 8000, 16, 1, False), (4, 4 * 8100, 16, 1, True), (6, 6 * 2600, 16, 1, False), (6, 6 * 2500, 16, 1, True), (7, 7 * 4000, 16, 1, True),
+    (2, 2 * 4000, 32, 2, True), (4, 4 * 4000, 12, 1, True), (1, 8000, 24, 2, False), (1, 3500, 24, 2, True), (1, 8000, 8, 1, True), (1, 8000, 64, 4, True)])
 def test_few_pairs_with_many_columns(batch, keys, n_q, n_kv, shares):
     from mini_sglang_amd_kernel import _lib
 
