@@ -424,6 +424,8 @@ MSGL_API int msgl_gdn_state_inplace_longest(const void* q, const void* k, const 
  *   MSGL_TUNE_SHARES         decode and verify on one launch of per-request key shares instead of
  *                            equal segments and a merge: negative: never; 0: chosen from the sizes;
  *                            positive: always, with share_len | kv heads per workgroup << 20
+ *   MSGL_TUNE_STREAM         from how many KiB of keys and values on decode and verify read them past the
+ *                            caches (0: default, negative: never); the results are the same bits
  */
 #define MSGL_TUNE_SEGMENTS 0
 #define MSGL_TUNE_MIN_SEGMENT 1
@@ -436,6 +438,7 @@ MSGL_API int msgl_gdn_state_inplace_longest(const void* q, const void* k, const 
 #define MSGL_TUNE_PREFILL_GANGS 8
 #define MSGL_TUNE_CLOCK_PROBE 9
 #define MSGL_TUNE_SHARES 10
+#define MSGL_TUNE_STREAM 11
 MSGL_API int msgl_set_tuning(int32_t knob, int64_t value);
 /* The value the calling thread last set for `knob` (0 if it never did): what its launches and
  * workspace queries use.  Makes the per-thread scope observable: a value set on another thread

@@ -17,7 +17,7 @@ thread_local int64_t t_tune[3] = {0, 0, 0};
 thread_local int64_t t_key_splits = 0;
 thread_local int64_t t_gangs = 0;  // negative: never use gang ranges
 thread_local long long* t_clock_probe = nullptr;
-constexpr int kTuneKnobs = 11;
+constexpr int kTuneKnobs = 12;
 thread_local int64_t t_last_set[kTuneKnobs] = {};  // what this thread last passed to msgl_set_tuning
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -59,11 +59,6 @@ msgl::SharePlan shares_for(int64_t batch, int64_t keys, int64_t each, int64_t n_
       t_last_set[MSGL_TUNE_SPLITKV_BOUNDARY] != 0)
     return msgl::SharePlan{};
   return msgl::share_plan(batch, keys, each, n_kv, head_dim, cols);
-}
-// The keys that the rows of a launch see, at most.
-int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t max_len_extend, bool is_cross) {
-  if (window <= 0 || is_cross) return total_kv;
-  return std::min(total_kv, batch * (window + max_len_extend + 15));  // a window starts at a multiple of 16
 }
 // Under a sliding window that most requests exceed every request shows about `window` keys: one workgroup per
 // (request, kv head) is balanced as it is, whatever the requests' lengths, and needs no second launch.  Up to three
@@ -167,6 +162,10 @@ int msgl_set_tuning(int32_t knob, int64_t value) {
   }
   if (knob == MSGL_TUNE_SHARES) {
     msgl::shares_force(value);
+    return MSGL_OK;
+  }
+  if (knob == MSGL_TUNE_STREAM) {
+    msgl::set_stream_kib(value);
     return MSGL_OK;
   }
   if (knob < 0 || knob > 2) return MSGL_ERR_SHAPE;
@@ -537,7 +536,7 @@ static int prefill_attention(const void* q, const void* k_cache, const void* v_c
   const int64_t group = num_q_heads / num_kv_heads;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t cols = group * max_len_extend;
-  const int64_t keys = visible_keys(batch, total_kv, sliding_window_size, max_len_extend, is_cross_attention != 0);
+  const int64_t keys = msgl::visible_keys(batch, total_kv, sliding_window_size, max_len_extend, is_cross_attention != 0);
   const msgl::SharePlan plan = shares_for(batch, keys, keys < total_kv ? keys / batch : 0, num_kv_heads, head_dim, cols);
   // without room for their partials a launch goes the way it goes without shares
   const bool share_room = plan.share_len > 0 && workspace && aligned16(workspace) &&
@@ -663,7 +662,7 @@ static msgl::SharePlan extend_step_plan(int64_t batch, int64_t total_q, int64_t 
       window < 0 || (head_dim != 128 && head_dim != 256))
     return none;
   const int64_t group = n_q / n_kv, cols = group * max_len_extend;
-  const int64_t keys = visible_keys(batch, total_kv, window, max_len_extend, is_cross);
+  const int64_t keys = msgl::visible_keys(batch, total_kv, window, max_len_extend, is_cross);
   const msgl::SharePlan plan = shares_for(batch, keys, keys < total_kv ? keys / batch : 0, n_kv, head_dim, cols);
   const bool window_share = window_shares(plan, batch, total_kv, keys, n_kv, head_dim, cols);
   return shares_route(plan, window_share, batch, total_kv, keys, n_kv, group, max_len_extend, head_dim, window) ? plan : none;

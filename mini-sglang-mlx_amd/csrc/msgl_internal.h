@@ -16,6 +16,12 @@ int launch_store_kv_cache(void* k_cache, void* v_cache, const int32_t* indices, 
                           int64_t k_cache_stride_bytes, int64_t v_cache_stride_bytes,
                           int64_t k_stride_bytes, int64_t v_stride_bytes, hipStream_t stream);
 
+// The keys that the rows of a launch see, at most.
+inline int64_t visible_keys(int64_t batch, int64_t total_kv, int64_t window, int64_t max_len_extend, bool is_cross) {
+  if (window <= 0 || is_cross) return total_kv;
+  return std::min(total_kv, batch * (window + max_len_extend + 15));  // a window starts at a multiple of 16
+}
+
 // ---- paged_splitkv.hip -------------------------------------------------------------
 // One description serves decode (qo_indptr == nullptr: one query per request, every key
 // visible) and the short-query route of prefill (speculative verify / draft proposal).
@@ -91,6 +97,16 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
 // whether segments are faster for so few (request, kv head) pairs of `mean` visible keys; windowed: all of them have as many
 bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t head_dim, int64_t cols, bool windowed);
 int device_cus();  // paged_splitkv.hip
+// Whether a launch that reads so many bytes, each of them once, reads them past the caches (ld_stream_b128): from where its data
+// are so much of the 256 MiB of the last level that a later pass does not find them there.  us by MiB, plain and past the caches:
+// decode 1253 222 -> 201, 4718 803 -> 723, verify 718 143 -> 126, window shares 129 33.0 -> 27.7.  5600 and 5700 launches of decode and verify at
+// head_dim 128 and 256, three sets of keys in turn, past the caches by plain (geometric mean): 16-24 MiB 1.006 and 1.011, 32-64 1.041 and
+// 1.020, 64-80 1.034 and 1.018, 80-96 0.999 and 1.003, 96-128 0.939 and 0.967, 128-1024 0.92 and 0.95.  With twelve sets, as the layers of a
+// model, they cross at 24 MiB (32-48 0.978, 48-96 0.956), so the line is not higher.
+constexpr int64_t kStreamKiB = 80 << 10;
+bool streams(int64_t bytes);  // paged_splitkv.hip
+// benchmarking switch: from how many KiB on (0: default, negative: never)
+void set_stream_kib(int64_t v);
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);
 int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& plan, hipStream_t stream);
 // benchmarking switch: 0 default, negative never, else share_len | heads_wg << 20

@@ -20,6 +20,8 @@ namespace msgl {
 // are normalised and rotated, k and v stored.
 // (kStoreRows: kStore for several new tokens per request, a prefill call's.)
 enum NewMode { kStored = 0, kStore = 1, kNormRopeStore = 2, kStoreRows = 3 };
+template <NewMode MODE>
+using New = std::integral_constant<int, MODE>;
 
 inline void fill_new_tokens(const NewTokens& n, SplitKvParams& p) {
   if (n.k == nullptr) return;

@@ -142,7 +142,7 @@ struct Nothing {
   __device__ __forceinline__ explicit Nothing(const Args&...) {}
 };
 
-template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
+template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW>
 __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
     const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
     int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams sp) {
@@ -212,12 +212,12 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   }
   if constexpr (NEW == kStored) {
     start_columns<D, NCT, true, true>(p, r, kvh, 0, t_end, c);
-    if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
+    if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
   } else if constexpr (NEW == kStoreRows) {
     new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == share_waves - 1;
     start_columns<D, NCT, true, true>(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
     new_rows.check();
-    if (t_begin < t_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
+    if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
     else new_rows();
   } else {
     static_assert(sizeof(HeadLds<D>) <= sizeof(part[0]), "a wave's heads have their place in its part of the partials");
@@ -234,9 +234,9 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     start_columns<D, NCT, NEW != kNormRopeStore, true>(p, r, kvh, 0, walk_end, c);
     if constexpr (D == 256) {
       token();
-      if (t_begin < walk_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, walk_end, ids, c, [] {});
+      if (t_begin < walk_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, walk_end, ids, c, [] {});
     } else {
-      if (t_begin < walk_end) attend_keys<D, NCT, WIDE, F16, true>(p, r, kvh, t_begin, walk_end, ids, c, token);
+      if (t_begin < walk_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, walk_end, ids, c, token);
       else if (owner) token();
     }
   }
@@ -399,29 +399,33 @@ int launch_shape(const ShareParams& sp, int share_len, unsigned blocks, hipStrea
   const uint32_t d = (uint32_t)share_len, s = log2_of(d - 1) + 1;
   const uint32_t magic = (uint32_t)(((1ull << (31 + s)) + d - 1) / d), groups = (uint32_t)sp.head_groups;
   const ShareShape shape(s - 1, log2_of((uint32_t)NW / (uint32_t)sp.heads_wg), (groups & (groups - 1)) == 0 ? log2_of(groups) : ShareShape::kNoShift);
-  auto launch = [&](auto narrow, auto wide) {
-    return launch_kernel(sp.s.wide ? wide : narrow, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
+  auto launch = [&](auto f16, auto mode_of) {
+    constexpr bool F16 = decltype(f16)::value;
+    constexpr int NEW = decltype(mode_of)::value;
+    const auto kernel = sp.s.walk == kStream ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW>
+                        : sp.s.walk == kWide ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW>
+                                             : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW>;
+    return launch_kernel(kernel, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
                          sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
     const int mode = sp.s.nt.k == nullptr || sp.s.qo_indptr != nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
     if (sp.s.f16) {
       if (mode == kStored && sp.s.nt.k == nullptr)
-        return launch(share_attention_kernel<D, NCT, NW, false, true, kStored>, share_attention_kernel<D, NCT, NW, true, true, kStored>);
+        return launch(std::true_type{}, New<kStored>{});
       if (mode == kStore)
-        return launch(share_attention_kernel<D, NCT, NW, false, true, kStore>, share_attention_kernel<D, NCT, NW, true, true, kStore>);
+        return launch(std::true_type{}, New<kStore>{});
       return MSGL_ERR_DTYPE;
     }
     if (mode == kStore)
-      return launch(share_attention_kernel<D, NCT, NW, false, false, kStore>, share_attention_kernel<D, NCT, NW, true, false, kStore>);
+      return launch(std::false_type{}, New<kStore>{});
     if (mode == kNormRopeStore)
-      return launch(share_attention_kernel<D, NCT, NW, false, false, kNormRopeStore>,
-                    share_attention_kernel<D, NCT, NW, true, false, kNormRopeStore>);
+      return launch(std::false_type{}, New<kNormRopeStore>{});
   }
   if (sp.s.f16) return MSGL_ERR_DTYPE;
   if (sp.s.nt.k != nullptr)  // a prefill call's
-    return launch(share_attention_kernel<D, NCT, NW, false, false, kStoreRows>, share_attention_kernel<D, NCT, NW, true, false, kStoreRows>);
-  return launch(share_attention_kernel<D, NCT, NW, false, false, kStored>, share_attention_kernel<D, NCT, NW, true, false, kStored>);
+    return launch(std::false_type{}, New<kStoreRows>{});
+  return launch(std::false_type{}, New<kStored>{});
 }
 
 thread_local int64_t t_force = 0;  // benchmarking switch, see shares_force()

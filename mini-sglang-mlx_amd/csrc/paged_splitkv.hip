@@ -145,10 +145,9 @@ __device__ __forceinline__ bool locate_segment(const SplitKvParams& p, int seg, 
 
 // NCT = tiles of 16 columns per wave, NW = waves per workgroup (launch bound only).  One
 // column tile at head dim 128 fits 256 VGPRs, so two such waves per SIMD can be resident.
-// WIDE: pool byte offsets need 64 bits (a pool of 4 GiB or more); otherwise a row's offset is
-// one 32-bit multiply instead of a 64-bit multiply-add per load.
+// WALK: how the pool's rows are read.  (With offsets of 32 bits a row's is one multiply instead of a 64-bit multiply-add per load.)
 // NEW: a decode step's rows are stored here (kStore), or are in the pool already (kStored).
-template <int D, int NCT, int NW, bool WIDE, bool F16, int NEW>
+template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW>
 __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void splitkv_attention_kernel(SplitKvParams p) {
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const ClockProbe clock_probe_(p.clock_probe);
@@ -201,13 +200,13 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     FirstIds ids = first_ids(p, r, t_begin, t_end);
     if constexpr (NEW == kStored) {
       start_columns(p, r, kvh, ct0, t_end, c_);
-      attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
+      attend_keys<D, NCT, WALK, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
     } else {
       LateToken<D, F16> token(p, r, rows[wave], cur_b, kvh, t_end == r.hi);
       const int walk_end = token.seen ? t_end - 1 : t_end;
       if (token.seen) end_ids(ids, t_begin, walk_end, token.before);
       start_columns(p, r, kvh, ct0, walk_end, c_);
-      if (t_begin < walk_end) attend_keys<D, NCT, WIDE, F16, false>(p, r, kvh, t_begin, walk_end, ids, c_, [] {});
+      if (t_begin < walk_end) attend_keys<D, NCT, WALK, F16, false>(p, r, kvh, t_begin, walk_end, ids, c_, [] {});
       token.finish(c_, kvh, t_begin < walk_end);
     }
 
@@ -545,18 +544,23 @@ int heads_per_group(int64_t n_kv) {
 
 template <int D, int NCT, int NW>
 int launch_attn(const SplitKvParams& p, hipStream_t stream) {
-  auto launch = [&](auto narrow, auto wide) {
-    return launch_kernel(p.wide ? wide : narrow, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), stream, p);
+  auto launch = [&](auto f16, auto mode) {
+    constexpr bool F16 = decltype(f16)::value;
+    constexpr int NEW = decltype(mode)::value;
+    const auto kernel = p.walk == kStream ? splitkv_attention_kernel<D, NCT, NW, kStream, F16, NEW>
+                        : p.walk == kWide ? splitkv_attention_kernel<D, NCT, NW, kWide, F16, NEW>
+                                          : splitkv_attention_kernel<D, NCT, NW, kNarrow, F16, NEW>;
+    return launch_kernel(kernel, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), stream, p);
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
     if (p.nt.k != nullptr && p.f16)
-      return launch(splitkv_attention_kernel<D, NCT, NW, false, true, kStore>, splitkv_attention_kernel<D, NCT, NW, true, true, kStore>);
+      return launch(std::true_type{}, New<kStore>{});
     if (p.nt.k != nullptr)
-      return launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStore>, splitkv_attention_kernel<D, NCT, NW, true, false, kStore>);
+      return launch(std::false_type{}, New<kStore>{});
     if (p.f16)
-      return launch(splitkv_attention_kernel<D, NCT, NW, false, true, kStored>, splitkv_attention_kernel<D, NCT, NW, true, true, kStored>);
+      return launch(std::true_type{}, New<kStored>{});
   }
-  return launch(splitkv_attention_kernel<D, NCT, NW, false, false, kStored>, splitkv_attention_kernel<D, NCT, NW, true, false, kStored>);
+  return launch(std::false_type{}, New<kStored>{});
 }
 
 template <int D, int NCT>
@@ -654,6 +658,10 @@ int device_cus() {
 
 void splitkv_set_max_waves(int v) { t_max_waves = v > 0 ? v : 4; }  // 0 restores the default
 
+static thread_local int64_t t_stream_kib = 0;
+void set_stream_kib(int64_t v) { t_stream_kib = v; }
+bool streams(int64_t bytes) { return t_stream_kib >= 0 && bytes >= (t_stream_kib > 0 ? t_stream_kib : kStreamKiB) << 10; }
+
 // benchmarking switch, one value per host thread: stream positions charged per request boundary
 // (0: chosen from the shape, below; negative: none)
 static thread_local int t_boundary = 0;
@@ -739,8 +747,10 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   p.window = a.window;
   p.scale_log2e = a.sm_scale * kLog2e;
   p.clock_probe = clock_probe();
-  p.wide = ((uint64_t)a.num_slots * (uint64_t)a.k_stride0 * 2u >= (1ull << 32) ||
-            (uint64_t)a.num_slots * (uint64_t)a.v_stride0 * 2u >= (1ull << 32)) ? 1 : 0;
+  const uint64_t pool_bytes = (uint64_t)a.num_slots * (uint64_t)std::max(a.k_stride0, a.v_stride0) * 2u;
+  const int64_t keys = visible_keys(a.batch, a.total_kv, a.window, a.max_len_extend, a.is_cross != 0);
+  const bool once = col_split(nct_for(p.cols), a.head_dim).col_waves == 1;
+  p.walk = once && streams(keys * a.n_kv * a.head_dim * 4) ? kStream : pool_bytes >= (1ull << 32) ? kWide : kNarrow;
 }
 
 int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream) {

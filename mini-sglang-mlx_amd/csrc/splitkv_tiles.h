@@ -7,6 +7,10 @@
 
 namespace msgl {
 
+// How the pool's rows are read: with offsets of 32 bits; of 64 (a pool of 4 GiB or more); past the caches (streams() in
+// paged_splitkv.hip), with offsets of 64 whatever the pool.
+enum Walk { kNarrow = 0, kWide = 1, kStream = 2 };
+
 struct SplitKvParams {
   const uint16_t* q;
   const uint16_t* k_cache;
@@ -29,7 +33,7 @@ struct SplitKvParams {
   int32_t q_begin, q_cap;  // first query of every request in this launch; cap on a request's queries
   int32_t f16;             // elements are IEEE half instead of bf16
   int32_t is_cross, window;
-  int32_t wide;  // pool byte offsets need 64 bits
+  int32_t walk;  // Walk
   uint32_t max_slot;  // num_slots - 1: slot ids are clamped to it before they become addresses
   uint32_t per_group;  // ceil(2^16 / group), see query_of()
   float scale_log2e;
@@ -190,6 +194,24 @@ __device__ __forceinline__ FirstIds first_ids(const SplitKvParams& p, const ReqI
   return FirstIds{{idx[min(at, last)], idx[min(at + 16, last)]}, {idx[min(at + 32, last)], idx[min(at + 48, last)]}};
 }
 
+// A tile whose K rows came by whole lines (attend_keys): of the 16 rows of a sub-tile, lanes of t16 < 8 have even pieces of 64 bytes, of
+// row t16 in slice 2 c and of row t16 + 8 in slice 2 c + 1, the others odd ones, of row t16 - 8 and of row t16.  Lane t16 gives
+// lane t16 +- 8 what is of its row.
+template <int D>
+__device__ __forceinline__ void lines_to_operands(KvTile<D>& t) {
+  constexpr int kRor8 = 0x128;  // DPP: from the lane 8 away in a row of 16; banks 0xc: written in its upper 8 lanes, 0x3 in the lower
+#pragma unroll
+  for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+    for (int c = 0; c < D / 32; c += 2)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int a = (int)t.k[sub][c][e], b = (int)t.k[sub][c + 1][e];
+        t.k[sub][c][e] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, kRor8, 0xf, 0xc, false);
+        t.k[sub][c + 1][e] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, kRor8, 0xf, 0x3, false);
+      }
+}
+
 // Keys tb .. tb + 31, in registers, for the columns in `c_`.
 template <int D, int NCT, bool F16>
 __device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTile<D>& t, int tb, Columns<D, NCT>& c_) {
@@ -276,25 +298,36 @@ __device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTil
 // Keys [t_begin, t_end) of request `r`, in order, for the columns in `c_`; `first`: its first_ids(), asked for before
 // the columns were made.
 // SHORT: ranges of one tile are common, end behind it (in a long walk the test costs more than it saves).
+// kStream: the loads past the caches take whole lines.  A row of V is 16 lanes' load as it is.  K's rows as operands are not, 64 bytes
+// of 16 rows a load: long walks load 128 bytes of 8 rows and exchange them (lines_to_operands); in shares, where a wave waits
+// for each of its few tiles, the exchange costs more than it gives and K is read the plain way.  us, plain / V past the caches / K too, as operands / by
+// lines: decode 1253 MiB 225 / 207 / 234 / 202, 4718 MiB 810 / 738 / 837 / 725, verify 143.5 / 134.3 / 146 / 126, shares at head_dim 256
+// 26.3 / 24.8 / 28.6 / 26.3, of a window 33.1 / 27.7 / 31.6 / 29.6.  A row that two waves read (col_split) is read the plain way: 64 columns 1.0-1.2x past the
+// caches, at head_dim 256 1.0-1.3x.
 // meanwhile(): called once the first tile has been asked for; may finish the columns' Q operand and put keys of its own
 // into their state.
-template <int D, int NCT, bool WIDE, bool F16, bool SHORT, typename Meanwhile>
+template <int D, int NCT, Walk WALK, bool F16, bool SHORT, typename Meanwhile>
 __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInfo& r, int kvh, int t_begin,
                                             int t_end, const FirstIds& first, Columns<D, NCT>& c_, Meanwhile&& meanwhile) {
   constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
+  constexpr bool LINES = WALK == kStream && !SHORT;
   const int lane = lane_id();
   const int t16 = lane & 15;
   const int g = lane >> 4;
   const unsigned char* kbase =
-      reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * D + g * 8);
+      reinterpret_cast<const unsigned char*>(p.k_cache + (int64_t)kvh * D + g * 8 + (LINES ? (t16 >> 3) * 32 : 0));
   const unsigned char* vbase =
       reinterpret_cast<const unsigned char*>(p.v_cache + (int64_t)kvh * D + t16 * 8);
   const uint32_t k_row_bytes = (uint32_t)p.k_stride0 * 2u;
   const uint32_t v_row_bytes = (uint32_t)p.v_stride0 * 2u;
   auto row_offset = [](int slot_id, uint32_t row_bytes) -> uint64_t {
-    if constexpr (WIDE) return (uint64_t)(uint32_t)slot_id * row_bytes;
+    if constexpr (WALK != kNarrow) return (uint64_t)(uint32_t)slot_id * row_bytes;
     else return (uint64_t)((uint32_t)slot_id * row_bytes);
+  };
+  auto load = [](const unsigned char* from) {
+    if constexpr (WALK == kStream) return ld_stream_b128(from);
+    else return ld_global_b128(from);
   };
   const int32_t* idx_base = p.kv_indices + r.kv_start;
   const int last_tok = t_end - 1;
@@ -306,9 +339,18 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
   };
   auto load_tile = [&](KvTile<D>& t, int s0, int s1) {
 #pragma unroll
-    for (int c = 0; c < KS; ++c) {
-      t.k[0][c] = ld_global_b128(kbase + row_offset(s0, k_row_bytes) + c * 64);
-      t.k[1][c] = ld_global_b128(kbase + row_offset(s1, k_row_bytes) + c * 64);
+    for (int sub = 0; sub < 2; ++sub) {
+      const int s = sub ? s1 : s0;
+      if constexpr (LINES) {  // of 8 rows 128 bytes each: rows t16 % 8 and t16 % 8 + 8
+        const unsigned char* row[2] = {kbase + row_offset(__builtin_amdgcn_update_dpp(s, s, 0x128, 0xf, 0xc, false), k_row_bytes),
+                                       kbase + row_offset(__builtin_amdgcn_update_dpp(s, s, 0x128, 0xf, 0x3, false), k_row_bytes)};
+#pragma unroll
+        for (int c = 0; c < KS; ++c) t.k[sub][c] = load(row[c & 1] + (c >> 1) * 128);
+      } else {
+        const unsigned char* row = kbase + row_offset(s, k_row_bytes);
+#pragma unroll
+        for (int c = 0; c < KS; ++c) t.k[sub][c] = ld_global_b128(row + c * 64);
+      }
     }
     // V rows of this lane group: tokens 4g+j (j<4) of sub-tile 0, then of sub-tile 1;
     // their slot ids sit in lanes 4g+j of the K index registers.
@@ -318,7 +360,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
       const int slot = __shfl(j < 4 ? s0 : s1, src, kWave);
       const unsigned char* vrow = vbase + row_offset(slot, v_row_bytes);
 #pragma unroll
-      for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = ld_global_b128(vrow + hf * 256);
+      for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = load(vrow + hf * 256);
     }
   };
 
@@ -337,10 +379,12 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     const int tok = t_begin + pr * 64;
     load_tile(tb_, i1a, i1b);
     load_idx(tok + 96, i1a, i1b);
+    if constexpr (LINES) lines_to_operands(ta);
     compute_tile<D, NCT, F16>(p, ta, tok, c_);
     if (SHORT && tok + 32 >= t_end) break;
     load_tile(ta, i0a, i0b);
     load_idx(tok + 128, i0a, i0b);
+    if constexpr (LINES) lines_to_operands(tb_);
     compute_tile<D, NCT, F16>(p, tb_, tok + 32, c_);
   }
 }

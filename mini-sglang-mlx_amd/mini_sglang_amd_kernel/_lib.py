@@ -114,6 +114,7 @@ TUNE_SPLITKV_BOUNDARY = 7
 TUNE_PREFILL_GANGS = 8
 TUNE_CLOCK_PROBE = 9
 TUNE_SHARES = 10
+TUNE_STREAM = 11
 
 _lib = None
 
