@@ -8,15 +8,18 @@
 //     y[t, hv, dv] = <S[hv][dv][:], q[t, hk]>                    hk = hv / (HV / HK)
 // q, k, v, g, beta, y are bf16; the state and all arithmetic are fp32.
 //
-// One state row (dk = 128 floats) lives in the registers of 16 lanes, 8 values each, for the
-// whole token loop: the two inner products are 8 lane-local FMAs and a 4-step rotate-and-add
+// One state row (dk = 128 floats) lives in the registers of 16 lanes, 8 values each (4 neighbours of each half, so that a
+// load or store of a wave is 256 bytes of 4 rows: two whole lines each), for the whole token loop: the two inner products are 8 lane-local FMAs and a 4-step rotate-and-add
 // inside the 16-lane DPP row (no LDS, no cross-row traffic).  A lane group carries R rows, so
 // one load of k and q serves R independent recurrences whose latencies overlap; the inputs of
 // the next kDepth tokens are always in flight.  Decode (one token) is
-// HBM-bound: 2 * dv * dk * 4 bytes of state per (request, hv head) read and written once.
+// HBM-bound: 2 * dv * dk * 4 bytes of state per (request, hv head) read and written once, past the caches where
+// launch_gdn_state() says so: 64 requests of 32 heads 53.2 -> 45.9 us, 5.85 TB/s (a large copy reaches 4.9; 8 neighbours to a lane, 16 bytes
+// of every 32 a load: plain 52.8, past the caches 53.7).
 // Prefill is a serial chain per row (as in the reference); parallelism is batch * hv * dv rows.  It takes
 // requests of very few tokens here; longer ones go in chunks (gdn_short.hip, gdn_chunk.hip; gdn_route.h).
 #include <algorithm>
+#include <type_traits>
 
 #include "gdn_params.h"
 #include "gdn_route.h"
@@ -50,7 +53,7 @@ __device__ __forceinline__ void unpack8(const u32x4_t raw, float (&f)[kPerLane])
 
 // R = dv rows per 16-lane group.  Workgroup = 256 threads = 16 groups = 16 R consecutive rows
 // of one (request, hv head).
-template <int R, int kDepth>
+template <int R, int kDepth, bool STREAM>
 __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
   constexpr int kRowsPerBlock = 16 * R;
   constexpr int kBlocksPerHead = kDV / kRowsPerBlock;
@@ -66,12 +69,15 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
   if (end <= start) return;  // nothing to do: the state stays as it is
 
   float* srow = p.state + (int64_t)p.slot_ids[b] * p.state_stride0 +
-                ((int64_t)hv * kDV + row0) * kDK + lane16 * kPerLane;
+                ((int64_t)hv * kDV + row0) * kDK + lane16 * 4;
+  auto load_state = [](const float* from) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(from));
+    else return *reinterpret_cast<const f32x4_t*>(from);
+  };
   float s[R][kPerLane];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(srow + r * kDK);
-    const f32x4_t c = *reinterpret_cast<const f32x4_t*>(srow + r * kDK + 4);
+    const f32x4_t a = load_state(srow + r * kDK), c = load_state(srow + r * kDK + kDK / 2);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       s[r][e] = a[e];
@@ -79,10 +85,14 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
     }
   }
 
+  auto lane_dims = [&](const uint16_t* row) {
+    const u32x2_t a = *reinterpret_cast<const u32x2_t*>(row + lane16 * 4), c = *reinterpret_cast<const u32x2_t*>(row + kDK / 2 + lane16 * 4);
+    return u32x4_t{a[0], a[1], c[0], c[1]};
+  };
   auto load_token = [&](int t, u32x4_t& kraw, u32x4_t& qraw, uint32_t& graw, uint32_t& braw,
                         uint32_t (&vraw)[R]) {
-    kraw = ld_global_b128(p.k + (int64_t)t * p.k_stride0 + hk * kDK + lane16 * kPerLane);
-    qraw = ld_global_b128(p.q + (int64_t)t * p.q_stride0 + hk * kDK + lane16 * kPerLane);
+    kraw = lane_dims(p.k + (int64_t)t * p.k_stride0 + hk * kDK);
+    qraw = lane_dims(p.q + (int64_t)t * p.q_stride0 + hk * kDK);
     graw = p.g[(int64_t)t * p.hv + hv];
     braw = p.beta[(int64_t)t * p.hv + hv];
 #pragma unroll
@@ -143,6 +153,10 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
     }
   }
 
+  auto store_state = [](float* to, f32x4_t x) {
+    if constexpr (STREAM) __builtin_nontemporal_store(x, reinterpret_cast<f32x4_t*>(to));
+    else *reinterpret_cast<f32x4_t*>(to) = x;
+  };
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     f32x4_t a, c;
@@ -151,8 +165,8 @@ __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
       a[e] = s[r][e];
       c[e] = s[r][4 + e];
     }
-    *reinterpret_cast<f32x4_t*>(srow + r * kDK) = a;
-    *reinterpret_cast<f32x4_t*>(srow + r * kDK + 4) = c;
+    store_state(srow + r * kDK, a);
+    store_state(srow + r * kDK + kDK / 2, c);
   }
 }
 
@@ -232,16 +246,29 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   int r = 1;
   if (blocks_r1 >= 8 * 1024) r = 4;
   else if (blocks_r1 >= 4 * 1024) r = 2;
+  // Decode: the state once in and once out, past the caches from 96 MiB on, and up to 24 MiB, what the L2 caches have room for beside
+  // the next pass's.  us, rows 1, 2, 4, plain / past the caches, three sets of states in turn: 14 MiB 7.6, 7.5, 7.4 / 8.0, 7.1, 6.3, 24 MiB 10.3, 9.5, 9.6 /
+  // 12.8, 10.5, 9.2, 28 MiB 11.6, 10.9, 10.8 / 14.6, 12.0, 12.0, 64 MiB 22.0, 21.4, 20.6 / 28.4, 24.4, 24.7 (in the last level from the pass before), 92 MiB 38.9, 32.2, 32.8 / 41.1, 33.7, 34.7, 104 MiB
+  // 43.9, 38.5, 39.2 / 46.2, 38.1, 38.9, 128 MiB 52.6, 48.9, 52.1 / 51.2, 45.9, 47.2, 512 MiB 210, 200, 210 / 206, 178, 190; up to 12 MiB 5.4 to 6.5 all.
+  // (With twelve sets 28 MiB 14.5, 13.6, 14.5 / 14.7, 12.4, 12.8, 64 MiB 28.9, 27.9, 29.0 / 28.5, 24.9, 25.3.)
+  const int64_t state_bytes = heads * kDV * kDK * (int64_t)sizeof(float);
+  const bool large = streams(state_bytes, 96 << 10);
+  const bool stream_state = p.single_token && (large || state_bytes <= (24 << 20));
+  if (p.single_token) r = large || heads <= 192 ? 2 : 4;
   if (t_force_rows > 0) r = t_force_rows;
   const int64_t blocks = heads * (kDV / (16 * r));
   if (blocks > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   const dim3 grid((unsigned)blocks), block(256);
   // decode has one token per request: nothing to look ahead to
-  if (p.single_token) {
-    return launch_kernel(r == 4 ? gdn_state_kernel<4, 1> : r == 2 ? gdn_state_kernel<2, 1> : gdn_state_kernel<1, 1>, grid, block, stream, p);
-  } else {
-    return launch_kernel(r == 4 ? gdn_state_kernel<4, 8> : r == 2 ? gdn_state_kernel<2, 8> : gdn_state_kernel<1, 8>, grid, block, stream, p);
-  }
+  auto launch = [&](auto depth, auto past) {
+    constexpr int N = decltype(depth)::value;
+    constexpr bool STREAM = decltype(past)::value;
+    return launch_kernel(r == 4 ? gdn_state_kernel<4, N, STREAM> : r == 2 ? gdn_state_kernel<2, N, STREAM> : gdn_state_kernel<1, N, STREAM>, grid,
+                         block, stream, p);
+  };
+  if (!p.single_token) return launch(std::integral_constant<int, 8>{}, std::false_type{});
+  if (stream_state) return launch(std::integral_constant<int, 1>{}, std::true_type{});
+  return launch(std::integral_constant<int, 1>{}, std::false_type{});
 }
 
 }  // namespace msgl

@@ -104,7 +104,7 @@ int device_cus();  // paged_splitkv.hip
 // 1.020, 64-80 1.034 and 1.018, 80-96 0.999 and 1.003, 96-128 0.939 and 0.967, 128-1024 0.92 and 0.95.  With twelve sets, as the layers of a
 // model, they cross at 24 MiB (32-48 0.978, 48-96 0.956), so the line is not higher.
 constexpr int64_t kStreamKiB = 80 << 10;
-bool streams(int64_t bytes);  // paged_splitkv.hip
+bool streams(int64_t bytes, int64_t from_kib = kStreamKiB);  // paged_splitkv.hip
 // benchmarking switch: from how many KiB on (0: default, negative: never)
 void set_stream_kib(int64_t v);
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols);

@@ -660,7 +660,7 @@ void splitkv_set_max_waves(int v) { t_max_waves = v > 0 ? v : 4; }  // 0 restore
 
 static thread_local int64_t t_stream_kib = 0;
 void set_stream_kib(int64_t v) { t_stream_kib = v; }
-bool streams(int64_t bytes) { return t_stream_kib >= 0 && bytes >= (t_stream_kib > 0 ? t_stream_kib : kStreamKiB) << 10; }
+bool streams(int64_t bytes, int64_t from_kib) { return t_stream_kib >= 0 && bytes >= (t_stream_kib > 0 ? t_stream_kib : from_kib) << 10; }
 
 // benchmarking switch, one value per host thread: stream positions charged per request boundary
 // (0: chosen from the shape, below; negative: none)
