@@ -1670,7 +1670,7 @@ __global__ __launch_bounds__(512) void prefill_pingpong_kernel(PrefillParams p) 
       const int qi = row_to_query(p, row);
       const int hh = row - qi * p.group;
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(os + (lrow * OROW + c * 8) * 2);
-      st_global_b128(p.out + ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * D + c * 8, v);
+      st_stream_b128(p.out + ((int64_t)(q_start + qi) * p.n_q + kvh * p.group + hh) * D + c * 8, v);
     }
   }
   }  // the next part of the gang's range (a launch without gang ranges leaves here)
