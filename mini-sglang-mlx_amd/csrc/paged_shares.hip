@@ -434,19 +434,21 @@ thread_local int64_t t_force = 0;  // benchmarking switch, see shares_force()
 
 void shares_force(int64_t v) { t_force = v; }
 
-// head_dim 256, (request, kv head) pairs no more than compute units: length and line of their own.
-static bool wide_heads_alone(int64_t batch, int64_t n_kv, int64_t head_dim) { return head_dim == 256 && batch * n_kv <= device_cus(); }
+// (request, kv head) pairs no more than compute units: length and line from measured costs.
+static bool heads_alone(int64_t batch, int64_t n_kv) { return batch * n_kv <= device_cus(); }
 
-// Length of the shares there: of those (in steps of a third or a half from 128 on) that fit the chip in one round, requests of one
+// Length of the shares there: of those (in steps of a third or a half from `least` on) that fit the chip in one round, requests of one
 // length included, the one that costs least: its keys, what a share costs the one that puts the request together, and a round trip
-// for every 16 of them, all in keys' worth of time.  Fitted to 4280 launches (decode and verify, 1-40 requests of 200-100 000 keys, four
-// head counts, every length that fits timed): within 1.0 % of the best length on average up to 8 columns, 1.4 % beyond; the length that head_dim 128
-// has, at most 16 shares to a request, from 256 on, and segments for fewer than 12 pairs: 16 and 11 %.
-static int64_t wide_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols) {
+// for every 16 of them, all in keys' worth of time.  Fitted to 4280 launches at head_dim 256 (decode and verify, 1-40 requests of 200-100 000
+// keys, four head counts, every length that fits timed): within 1.0 % of the best length on average up to 8 columns, 1.4 % beyond; the shortest that
+// fits with at most 16 shares to a request, from 256 on, and segments for fewer than 12 pairs: 16 and 11 %.
+// The same costs hold at head_dim 128: 12 700 launches of up to 25 pairs within 0.3-3 % of the best, where the shortest that fits with at most 16
+// shares to a request was 1-3 % from 12 pairs on, 3-44 % for 4 to 11 and up to 2x for fewer.
+static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols, int64_t least) {
   const double slots = (double)device_cus(), mean = (double)(keys / batch), spread = 0.43 * std::sqrt((double)batch);
   int64_t len = 0;
   double lowest = 0;
-  for (int64_t c = 128; c < (1 << 20); c = (c & (c - 1)) ? c / 3 * 4 : c / 2 * 3) {
+  for (int64_t c = least; c < (1 << 20); c = (c & (c - 1)) ? c / 3 * 4 : c / 2 * 3) {
     const double of_one = std::max(std::ceil(mean / (double)c), 1.0);
     const double shares = std::max({(double)batch, (double)keys / (double)c + 0.5 * (double)batch + spread, (double)batch * of_one});
     if (shares * (double)n_kv > slots) continue;
@@ -478,8 +480,8 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     // average request: the last of them reads the others' partials.  Rounding adds half a share per request
     // and scatters around that: with two standard deviations more, 9 requests of 102-713 keys, 64 / 8 heads, have 192 keys a share
     // and take 12.5 us, without it 128, a few workgroups more than compute units, and 16.6
-    const bool wide = wide_heads_alone(batch, n_kv, head_dim);
-    len = nct == 3 ? 512 : (nw == 4 && heads == 1 && !wide) ? 256 : 128;
+    const bool alone = heads_alone(batch, n_kv);
+    len = nct == 3 ? 512 : (nw == 4 && heads == 1 && !(head_dim == 256 && alone)) ? 256 : 128;
     const int64_t spread = (int64_t)std::sqrt((double)batch / 3);
     auto fits = [&](int64_t c) {
       return std::max(batch, keys / c + batch / 2 + spread) * (n_kv / heads) <= slots && keys <= 16 * c * batch;
@@ -487,8 +489,8 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     if (each > 0) {  // one length for all: as many equal shares as fit
       const int64_t n = std::min<int64_t>(std::max<int64_t>(slots * heads / (batch * n_kv), 1), 16);
       len = std::max(len, ((each + n - 1) / n + 31) & ~(int64_t)31);
-    } else if (wide) {
-      len = wide_share_length(batch, keys, n_kv, cols);
+    } else if (alone) {
+      len = cost_share_length(batch, keys, n_kv, cols, len);
     } else {
       while (!fits(len) && len < (1 << 19)) len = (len & (len - 1)) ? len / 3 * 4 : len / 2 * 3;
     }
@@ -527,46 +529,50 @@ bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t he
   return n_kv == 1 && batch <= 6 && cols > 12 && mean > 2500 && mean <= 8000;
 }
 
-// Measured against the segment kernel and its merge on 400 random shapes (1-256 requests of 1-60 K
-// keys, 1-16 queries, both head sizes; us, segments -> shares): 46 x 4-18 keys 42.1 -> 7.3, 64 x 20-200
-// 18.9 -> 11.3, 200 x 6-99 28.5 -> 18.0, 4 x 37-1023 15.7 -> 9.1, one of 2 K 13.5 -> 10.3, 24 x 127-4095
-// at head_dim 256 35.9 -> 28.1.  Short requests gain most (a segment pays 8 us for each request
-// boundary it crosses), and nothing any more where they fill the chip several times over (107 MiB 27.3 -> 24.1, 160 39.6 ->
-// 39.5, 371 81 -> 92).
-// The segments' fixed costs are the same for any number of bytes, while the shares' lengths vary and the longest
-// decides.  So a launch beyond the first lines has to be one whose shares are short, and sure to go in one round, requests of
-// one length included.  By MiB of keys and values: head_dim 128 39 18.7 -> 14.2 (2 requests), 66 21.2 -> 17.9 (12), 97 27.3 -> 22.4 (9),
-// 142 32.3 -> 29.0 (13), 165 35.4 -> 31.7 (5), with longer shares 118 28.5 -> 29.6 (24), 175 35.8 -> 40.8 (22), 247 45.5 -> 51.9, with a
-// workgroup too many 81 21.8 -> 27.8 (33); head_dim 256 72 32.4 -> 25.6 (9), 134 40.6 -> 33.0 (31), 237 58.4 -> 66.8 (17).  One long request
-// among short ones gains as much (64, 15 requests, the longest 9.2 K, 20.5 -> 17.6; head_dim 256 155, 19, 24.7 K 44.5 -> 38.5), but
-// not where several heads go to a workgroup (177, 48, 14 K 36.0 -> 39.7), nor few requests with many columns, whose last shares
-// have most to put together (59, 2 requests, 40 columns 28.4 -> 35.1, 62, 4 requests, 24 columns 25.9 -> 29.1), nor shares twice as long as
-// a request on average, most of which take a whole request (73, 26 requests, one of them 7.5 K, 22.3 -> 24.0, with keys from memory 41.1 -> 45.8).
-// 502 launches beyond the first lines with 1-48 columns, shares by segments: with keys in the last-level cache 0.883 (geometric mean; worst
-// 1.04), with keys from memory 0.957 (1.05); 18 that the last two conditions leave out 0.926 (1.13) and 0.986 (1.11).
+// Short requests gain most against segments (a segment pays 8 us for each request boundary it crosses, us: 46 x 4-18 keys 42.1 -> 7.3,
+// 64 x 20-200 18.9 -> 11.3, 4 x 37-1023 15.7 -> 9.1), and nothing any more where they fill the chip several times over.  The segments'
+// fixed costs are the same for any number of bytes, while the shares' lengths vary and the longest decides: a launch beyond some
+// MiB has to be one whose shares fill one round, requests of one length included.
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
   if (few_pairs_in_segments(batch, n_kv, mean, head_dim, cols, false)) return false;
-  if (wide_heads_alone(batch, n_kv, head_dim)) {
-    // Beyond some MiB the shares have to fill the chip: a launch takes as long as its longest share.  By MiB of keys and values
-    // and what part of a round of shares as long as the longest they are, shares by segments (geometric mean, worst): up to 64 0.65
-    // (1.10), 64-128 0.76 (0.99), 128-256 from 0.5 on 0.83 (1.05) and 1.03 below, 256-420 from 0.62 on 0.91 (1.07), 1.05 below,
-    // 512-724 from 0.75 on 0.95 (1.03), 0.97 (1.09) below, 1.04 below 0.62, 1024-1448 from 0.88 on 0.96 (0.98), 0.98 (1.07) below, 1.02 below
-    // 0.75.  The line goes along that.  (Two of 408-2260 keys, 24 / 4 heads, 21.8 -> 11.0 us; one of 51.8 K, 16 / 2, 51 -> 35.)
-    const double longest = std::min((double)plan.share_len, 1.75 * (double)mean);
-    return mb <= 1400 && (double)(keys * n_kv) >= (0.12 * std::log2((double)std::max<int64_t>(mb, 1)) - 0.39) * longest * (double)device_cus();
+  const int64_t len = plan.share_len;
+  if (heads_alone(batch, n_kv)) {
+    // What part of a round of shares as long as the longest they are, by MiB of keys and values; shares by segments (geometric mean,
+    // worst).  head_dim 256: up to 64 0.65 (1.10), 64-128 0.76 (0.99), 128-256 from 0.5 on 0.83 (1.05) and 1.03 below, 256-420 from
+    // 0.62 on 0.91 (1.07), 1.05 below, 512-724 from 0.75 on 0.95 (1.03), 0.97 (1.09) below, 1.04 below 0.62, 1024-1448 from 0.88 on 0.96
+    // (0.98), 0.98 (1.07) below, 1.02 below 0.75.  (Two of 408-2260 keys, 24 / 4 heads, 21.8 -> 11.0 us; one of 51.8 K, 16 / 2, 51 -> 35.)
+    // head_dim 128, 18 600 launches, three and eight sets of keys in turn, by pairs: 1-3 0.81, up to 128 MiB; 4-11 24-50 MiB 0.85 and 0.82, 50-190
+    // 0.80 and 0.82; 12-256 24-50 0.7, 50-128 0.77 and 0.8, 128-190 0.83 and 0.89, the worst tenth of them 1.0; beyond by that part of a round: 190-220
+    // from 0.74 on 0.88, 0.98-1.0 below, 220-256 0.88 and 0.99-1.05, 256-300 0.95 and 0.97-1.05, 300-440 from 0.8 on 0.95-0.98, 1.0-1.2 below.
+    // (us: one of 10 K keys, 48 / 6, 16.3 -> 15.5; two, 54 K in all, 42.1 -> 32.1; 13 of 1 K, 32 / 4, 16.6 -> 11.4.)  Few pairs with two or
+    // three tiles of columns leave much to put together to the last share of each: from 16 MiB on up to five pairs 0.98-1.07 and 1.1-1.2.
+    const bool wide = head_dim == 256;
+    if (!wide) {
+      if (cols > 16 && units < 6 && mb > 16) return false;
+      // Some launches from 56 MiB on, 0.75-0.85 of segments as well, stay there: what a step of theirs takes (a launch of its own for norm and
+      // rotary embedding, scratch memory) is what it has been.
+      if (mb > 56 && mb <= 128 && ((units < 48 && cols > 16) || len > 2 * mean)) return false;
+      if (mb > 56 && mb <= 80 && units < 12 && mean > 12288) return false;
+    }
+    const double of_round = (double)(keys * n_kv) / (std::min((double)len, 1.75 * (double)mean) * (double)device_cus());
+    if (wide) return mb <= 1400 && of_round >= 0.12 * std::log2((double)std::max<int64_t>(mb, 1)) - 0.39;
+    return mb <= 190 || (mb <= 400 && of_round >= 0.72 + (double)(mb - 190) / 2000);
   }
-  if (mb <= (mean > 8192 ? 20 : mean > 4096 ? 36 : head_dim == 256 ? 128 : 56)) return true;
-  const int64_t len = plan.share_len, head_groups = n_kv / plan.heads_wg;
-  const double shares = (double)keys / (double)len + 0.5 * (double)batch + std::sqrt((double)batch / 3);  // see share_plan()
-  if (shares * (double)head_groups > device_cus() || batch * ((mean + len - 1) / len) * head_groups > device_cus()) return false;
-  if (head_dim == 256) return units >= 24 && len * plan.heads_wg <= 1024 && mb <= 256;
-  // (at 128 one request's 16 shares leave most of the chip idle and get long: 8.7 K keys 16.4 -> 15.2, 26.5 K 26.7 -> 28.1)
-  if ((units < 48 && cols > 16) || (units < 12 && mean > 12288) || len > 2 * mean) return false;
-  return len * plan.heads_wg <= 1536 && mb <= (units > device_cus() ? 128 : 208);
+  // Several heads to a workgroup.
+  const int64_t head_groups = n_kv / plan.heads_wg;
+  const bool even_fit = batch * ((mean + len - 1) / len) * head_groups <= device_cus();  // requests of one length go in one round
+  if (head_dim == 256) {
+    if (mb <= 128) return true;
+    const double shares = (double)keys / (double)len + 0.5 * (double)batch + std::sqrt((double)batch / 3);  // see share_plan()
+    return even_fit && shares * (double)head_groups <= device_cus() && len * plan.heads_wg <= 1024 && mb <= 256;
+  }
+  // 4800 launches of more than 256 pairs, as above: where requests of one length go in one round 45-96 MiB 0.7, 96-128 0.74 and 0.85, 128-160 0.79
+  // and 0.89, 160-190 0.87 and 0.92, 190-220 0.95 and 0.99, 1.0 beyond; where they don't, up to 128 0.86 and 0.9 (worst 1.5), 0.94 and 1.0 beyond.
+  return mb <= (even_fit ? 190 : 128);
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {
