@@ -17,12 +17,12 @@
 // (16 requests of 64 tokens 38 us, now 26).  74 KB of LDS and 128 registers let two workgroups of eight waves share a compute unit
 // (lane_here() keeps what only a group's start needs out of the registers: in it they were 16 too many, 5-15 % of the time).
 //
-// What bounds it: up to 16 tokens the state, read and written (16 requests of 32 heads 15.5 us, 4.3 TB/s, token by token 37.5); beyond, the
+// What bounds it: up to 16 tokens the state, read and written (16 requests of 32 heads of 8 tokens 13.5 us, 5.0 TB/s); beyond, the
 // chain of a chunk, 1.25 us for one request, 1.45 for four, and from eight on the issue of the waves of a SIMD, 0.2-0.3 us a chunk and request, the
 // matrix pipe busy for a quarter to 38 % of the cycles.  A chunk ends in a wait for all memory operations of its wave (behind V's loads, which
 // are under a condition, and the masked rows of Y the compiler does not know how many are under way): V's round trip is in every chunk,
 // that of the next group's K and Q in a group's first.  us, by requests of 32 heads and tokens, before and now: 1 x 16 8.3 and 6.0, 32 9.3
-// and 6.7; 4 x 16 12.1 and 7.2; 8 x 16 24.9 and 10.6, 40 24.9 and 12.9; 16 x 40 50.7 and 21.5; 24 x 80 105 and 44; 48 x 8 57 and 43.  Four more
+// and 6.7; 4 x 16 12.1 and 7.2; 8 x 16 24.9 and 9.1, 40 24.9 and 12.5; 16 x 40 50.7 and 21.5; 24 x 80 105 and 44; 48 x 8 57 and 42.7.  Four more
 // waves that fetch and make the systems ahead: 1.1 us a chunk for one request, no change for four.
 //
 // Precision: fp32 throughout, the parts are exact (see upper()).  The state's error against 64 bits, rms: 1.0-1.7e-8 at states of 0.1
@@ -148,8 +148,30 @@ __device__ __forceinline__ bf16x8_t upper(f32x4_t a, f32x4_t b) {
   const u32x2_t x = upper(a), y = upper(b);
   return as_bf16x8(u32x4_t{x[0], x[1], y[0], y[1]});
 }
-// WAVES: 8, a head's rows in one workgroup, or 4, half of them
-template <int WAVES>
+// A wave's 16 state rows by whole lines, which can go past the caches: a load takes 128 bytes of 8 rows, s[2 c] of rows lane % 8, s[2 c + 1]
+// of the others, and of the line's pieces of 16 bytes the lanes below 8 of 16 the even ones.  Lanes 8 apart then give each other
+// what is of the other's row, and the same brings them back.
+__device__ __forceinline__ float* state_lines(int slot, int hv, int row) {
+  uint32_t lane = lane_id();
+  pin(lane);
+  return parameter(&GdnParams::state) + (int64_t)slot * parameter(&GdnParams::state_stride0) +
+         ((int64_t)hv * kDV + row + (lane & 7)) * kDK + 8 * (lane >> 4) + 4 * ((lane >> 3) & 1);
+}
+__device__ constexpr int line_at(int c) { return 32 * (c >> 1) + 8 * kDK * (c & 1); }
+__device__ __forceinline__ void exchange_lines(f32x4_t (&s)[8]) {
+  constexpr int kRor8 = 0x128;  // DPP: from the lane 8 away in a row of 16
+#pragma unroll
+  for (int c = 0; c < 8; c += 2)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float even = s[c][i], odd = s[c + 1][i];  // (a bit cast of an element itself takes the first one)
+      const int a = __builtin_bit_cast(int, even), b = __builtin_bit_cast(int, odd);
+      s[c][i] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(a, b, kRor8, 0xf, 0xc, false));
+      s[c + 1][i] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, a, kRor8, 0xf, 0x3, false));
+    }
+}
+// WAVES: 8, a head's rows in one workgroup, or 4, half of them; LINES: the state by whole lines, past the caches
+template <int WAVES, bool LINES>
 __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnParams p) {
   __shared__ __attribute__((aligned(16))) ShortLds lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -193,10 +215,17 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
     v_chunk += kShortChunk * (int64_t)v_step;
   };
   fetch_group(0);
-  float* const srow = state_row(slot, hv, row);
   f32x4_t s[8];  // s[2 c + h][i]: dim 32 c + 8 g + 4 h + i of row lane % 16
+  if constexpr (LINES) {
+    const float* const from = state_lines(slot, hv, row);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
+    for (int c = 0; c < 8; ++c) s[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(from + line_at(c)));
+    exchange_lines(s);
+  } else {
+    const float* const from = state_row(slot, hv, row);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(from + 32 * (c >> 1) + 4 * (c & 1));
+  }
   load_v(start);
   const Picker pick;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -302,8 +331,16 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
     token_by_token(start, end, slot, hv, row);
     return;
   }
+  if constexpr (LINES) {
+    float* const to = state_lines(slot, hv, row);
+    exchange_lines(s);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
+    for (int c = 0; c < 8; ++c) __builtin_nontemporal_store(s[c], reinterpret_cast<f32x4_t*>(to + line_at(c)));
+  } else {
+    float* const to = state_row(slot, hv, row);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(to + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
+  }
 }
 
 }  // namespace
@@ -314,8 +351,13 @@ int launch_gdn_short(const GdnParams& p, hipStream_t stream) {
   // Half a head to a workgroup while that leaves one to a compute unit, or two and there is one chunk (8 requests of 32 heads: 16 tokens
   // 10.4 us and 10.8 by whole heads, 32 tokens 12.9 and 11.7).
   const bool halves = 2 * heads <= device_cus() || (heads <= device_cus() && p.tokens <= kShortChunk * (int64_t)p.batch);
-  return halves ? launch_kernel(gdn_short_kernel<4>, dim3((unsigned)(2 * heads)), dim3(256), stream, p)
-                : launch_kernel(gdn_short_kernel<8>, dim3((unsigned)heads), dim3(512), stream, p);
+  // Whole lines past the caches from four requests of 32 heads on.  us, plain and that, by requests: of 4-16 tokens 4 7.0-7.3 and 6.9-7.1, 8 10.6-11.1
+  // and 8.9-9.1, 16 15.2-16.1 and 13.4-14.3, 24 23.6-24.5 and 22.5-23.1, 64 60.2-63.8 and 56.7-59.2; of 32 tokens 8 12.3 and 11.5, 48 56.9 and 49.9,
+  // 100 108 and 99; of 48 16 22.2 and 21.9, 64 83.2 and 79.5, but 24 30.9 and 31.8, 100 121 and 127.  One and two requests find their state in the caches
+  // when it is asked for again: 5.0-8.0 and 0.3-0.8 more.
+  if (heads < 128) return launch_kernel(gdn_short_kernel<4, false>, dim3((unsigned)(2 * heads)), dim3(256), stream, p);
+  return halves ? launch_kernel(gdn_short_kernel<4, true>, dim3((unsigned)(2 * heads)), dim3(256), stream, p)
+                : launch_kernel(gdn_short_kernel<8, true>, dim3((unsigned)heads), dim3(512), stream, p);
 }
 
 }  // namespace msgl
