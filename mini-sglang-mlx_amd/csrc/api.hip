@@ -58,7 +58,8 @@ msgl::SharePlan shares_for(int64_t batch, int64_t keys, int64_t each, int64_t n_
   if (t_tune[MSGL_TUNE_SEGMENTS] != 0 || t_tune[MSGL_TUNE_MIN_SEGMENT] != 0 || t_last_set[MSGL_TUNE_SPLITKV_WAVES] != 0 ||
       t_last_set[MSGL_TUNE_SPLITKV_BOUNDARY] != 0)
     return msgl::SharePlan{};
-  return msgl::share_plan(batch, keys, each, n_kv, head_dim, cols);
+  const msgl::SharePlan plan = msgl::share_plan(batch, keys, each, n_kv, head_dim, cols);
+  return plan.col_groups > 1 && t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0 ? msgl::SharePlan{} : plan;
 }
 // Under a sliding window that most requests exceed every request shows about `window` keys: one workgroup per
 // (request, kv head) is balanced as it is, whatever the requests' lengths, and needs no second launch.  Up to three
@@ -74,7 +75,7 @@ msgl::SharePlan shares_for(int64_t batch, int64_t keys, int64_t each, int64_t n_
 // of 4) 202 and 164, 571 and 513.
 bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv, int64_t keys, int64_t n_kv,
                    int64_t head_dim, int64_t cols) {
-  if (plan.share_len == 0 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
+  if (plan.share_len == 0 || plan.col_groups > 1 || keys >= total_kv || keys > 4096 * batch || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
   if (msgl::few_pairs_in_segments(batch, n_kv, keys / batch, head_dim, cols, true)) return false;
   const int64_t blocks = batch * (n_kv / plan.heads_wg), cus = msgl::device_cus();
   if (blocks > cus && 3 * blocks < 2 * cus * ((blocks + cus - 1) / cus)) return false;
@@ -84,7 +85,8 @@ bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv,
 // to three column tiles in one wave; 49-64 columns would run on two waves per kv head that each
 // read every K / V row, and the tile kernel with ragged key shares is as fast or faster on them),
 // at head_dim 256 16 (one column tile; more would be a wave per tile, each reading every row,
-// and the tile kernel with ragged shares is 10-65 % faster from 17 columns on).  Up to 64 columns
+// and the tile kernel with ragged shares is 10-65 % faster from 17 columns on).  Few keys go in shares beyond that, see
+// wide_round() in paged_shares.hip.  Up to 64 columns
 // the split-K kernel also takes what the tile kernels cannot give ragged shares to (very many
 // or many short requests): its segments are balanced whatever the lengths, and one long request
 // among many short ones would otherwise be one long workgroup per kv head.
@@ -427,6 +429,7 @@ static bool window_prefers_tiles(int64_t batch, int64_t total_kv, int64_t n_kv, 
 static bool shares_route(const msgl::SharePlan& plan, bool window_share, int64_t batch, int64_t total_kv, int64_t keys,
                          int64_t n_kv, int64_t group, int64_t max_len_extend, int64_t head_dim, int64_t window) {
   if (plan.share_len == 0) return false;
+  if (plan.col_groups > 1) return msgl::shares_preferred(plan, batch, keys, n_kv, head_dim, group * max_len_extend);
   if (window_share) return true;
   if (keys < total_kv && msgl::few_pairs_in_segments(batch, n_kv, keys / batch, head_dim, group * max_len_extend, true)) return false;
   return use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, n_kv) &&

@@ -341,10 +341,11 @@ struct NewRows {
   int end;                // of the keys that are walked
   bool last_keys, owner;  // the new tokens are the request's last keys; this wave takes them
   bool listed;            // their slots are the ones listed
+  bool stores;            // (of several workgroups on the request's columns one stores the listed)
   uint32_t slot, id;      // lane i: slot of row i; slot id listed for its place
 
-  __device__ __forceinline__ NewRows(const SplitKvParams& params, const ReqInfo& req, Columns<D, NCT>& c, int head)
-      : p(params), r(req), columns(c), kvh(head), owner(false) {
+  __device__ __forceinline__ NewRows(const SplitKvParams& params, const ReqInfo& req, Columns<D, NCT>& c, int head, bool stores_rows)
+      : p(params), r(req), columns(c), kvh(head), owner(false), stores(stores_rows) {
     const int lane = lane_id();
     q0 = req.q_start;  // (a launch of shares covers the queries from the first on)
     n = req.rows;
@@ -393,7 +394,7 @@ struct NewRows {
 #pragma unroll
         for (int hf = 0; hf < VH; ++hf) t.v[hf][j] = ld_global_b128(row + hf * 128 + t16 * 8);
       }
-      if (listed) {
+      if (listed && stores) {
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
           const int i = i0 + 16 * sub + t16;

@@ -10,7 +10,7 @@
 //   A request's visible keys are cut into ceil(keys / share_len) equal shares.  A workgroup takes one
 //   share of `heads_wg` adjacent kv heads; `share_waves` waves cut the share of each head into
 //   adjacent ranges, so a share is read with every load of its first tiles in flight at once.  The
-//   waves of a head meet in LDS.  The grid holds the largest number of shares the sizes allow; a
+//   waves of a head meet in LDS.  (Columns that a wave has no registers for go to several workgroups, see wide_round().)  The grid holds the largest number of shares the sizes allow; a
 //   workgroup finds its (request, share) with one wave-wide prefix sum over kv_indptr and takes the
 //   request's geometry from the same registers; a workgroup past the last share ends.
 //   A request with one share is written at once.  Otherwise the share's normalised fp32 partial and
@@ -35,7 +35,7 @@ namespace {
 
 struct ShareParams {
   SplitKvParams s;
-  unsigned long long* counts;  // [batch][head_groups]
+  unsigned long long* counts;  // [batch][head_groups][col_groups]
   unsigned long long nonce;
   int32_t heads_wg, head_groups;
 };
@@ -54,14 +54,16 @@ struct ShareStart {
     return (int)(__umulhi((uint32_t)(keys + share_len - 1), len_magic) >> len_shift);
   }
 };
-struct ShareShape {  // powers of two: waves on a head; head groups (kNoShift: they are none)
+struct ShareShape {  // powers of two: waves on a head; head groups (kNoShift: they are none).  Column groups
   static constexpr uint32_t kNoShift = 255;
   uint32_t bits;
-  __host__ __device__ ShareShape(uint32_t len_shift, uint32_t waves, uint32_t groups) : bits(len_shift | waves << 8 | groups << 16) {}
+  __host__ __device__ ShareShape(uint32_t len_shift, uint32_t waves, uint32_t groups, uint32_t col_groups)
+      : bits(len_shift | waves << 8 | groups << 16 | col_groups << 24) {}
   __host__ __device__ explicit ShareShape(uint32_t b) : bits(b) {}
   __device__ __forceinline__ uint32_t len_shift() const { return bits & 0xffu; }
   __device__ __forceinline__ uint32_t waves() const { return (bits >> 8) & 0xffu; }
-  __device__ __forceinline__ uint32_t groups() const { return bits >> 16; }
+  __device__ __forceinline__ uint32_t groups() const { return (bits >> 16) & 0xffu; }
+  __device__ __forceinline__ uint32_t col_groups() const { return bits >> 24; }
 };
 // ceil(a / b) of scalars, b > 0 and the result below 2^20 (the compiler's division is twice as long)
 __device__ __forceinline__ int ceil_div(int a, int b) {
@@ -142,7 +144,8 @@ struct Nothing {
   __device__ __forceinline__ explicit Nothing(const Args&...) {}
 };
 
-template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW>
+// WIDE: a request's columns go to several workgroups, kCols to each.
+template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW, bool WIDE>
 __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
     const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
     int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams sp) {
@@ -159,13 +162,20 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   const int t16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int item, hg;
-  if (shape.groups() == ShareShape::kNoShift) {
-    item = blockIdx.x / sp.head_groups;
-    hg = blockIdx.x - item * sp.head_groups;
-  } else {
-    item = blockIdx.x >> shape.groups();
-    hg = blockIdx.x & ((1u << shape.groups()) - 1);
+  uint32_t block = blockIdx.x, cg = 0;
+  if (WIDE) {  // the column groups of a share are on one XCD
+    const uint32_t seq = block >> 3, base = seq / shape.col_groups();
+    cg = seq - base * shape.col_groups();
+    block = base * 8 + (block & 7);
   }
+  if (shape.groups() == ShareShape::kNoShift) {
+    item = block / sp.head_groups;
+    hg = block - item * sp.head_groups;
+  } else {
+    item = block >> shape.groups();
+    hg = block & ((1u << shape.groups()) - 1);
+  }
+  const int col0 = WIDE ? (int)cg * kCols : 0;  // the first of this workgroup's columns
   const int share_waves = 1 << shape.waves();
   const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
   const int sw = wave & (share_waves - 1);
@@ -184,11 +194,11 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   // what the rest of the way begins with and only the request's number leads to
   const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
   __builtin_amdgcn_sched_barrier(0);
-  const int ncols = r.q_len * p.group;
-  if (ncols == 0) return;
+  const int ncols = WIDE ? min(r.q_len * p.group - col0, kCols) : r.q_len * p.group;
+  if (ncols <= 0) return;
   Columns<D, NCT> c;
   // the keys that are walked: all, but for a prefill call's own new ones
-  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, kvh);
+  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, kvh, col0 == 0);
   int hi = r.hi;
   if constexpr (NEW == kStoreRows) hi = new_rows.end;
   const int vis = hi - r.lo;
@@ -200,7 +210,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   FirstIds ids{};
   if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
   __builtin_amdgcn_sched_barrier(0);
-  unsigned long long* const cnt = sp.counts + (int64_t)b * sp.head_groups + hg;
+  unsigned long long* const cnt = sp.counts + ((int64_t)b * sp.head_groups + hg) * (WIDE ? shape.col_groups() : 1) + cg;
   const unsigned long long fresh = sp.nonce << 16;
   // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
   // for it: whoever finds the word not made yet makes it (below).  (The last wave, which has the fewest keys or none.)
@@ -211,11 +221,11 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
                                                  __HIP_MEMORY_SCOPE_AGENT);
   }
   if constexpr (NEW == kStored) {
-    start_columns<D, NCT, true, true>(p, r, kvh, 0, t_end, c);
+    start_columns<D, NCT, true, true>(p, r, kvh, col0 >> 4, t_end, c);
     if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
   } else if constexpr (NEW == kStoreRows) {
     new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == share_waves - 1;
-    start_columns<D, NCT, true, true>(p, r, kvh, 0, new_rows.owner ? r.hi : t_end, c);
+    start_columns<D, NCT, true, true>(p, r, kvh, col0 >> 4, new_rows.owner ? r.hi : t_end, c);
     new_rows.check();
     if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
     else new_rows();
@@ -269,7 +279,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 
   constexpr int kQuads = D / 4;  // a thread's unit of work: 4 dims of one column, the 16 bytes at 16 it of a share's rows
   const int threads = 64 * share_waves;
-  const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols;
+  const int64_t row0 = ((int64_t)item * p.n_kv + kvh) * p.cols + col0;
   const Partials own(p.part_o + row0 * D, (uint32_t)(ncols * D * 4));
   // Every wave's part of a quad is asked for before the first is used.  The lanes of a row of 16 work on one column: lane w has
   // wave w's maximum and sum, and its weight goes to the others by DPP.
@@ -289,8 +299,8 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
       each([&](auto w) { acc += of_row_lane<decltype(w)::value>(e) * o[decltype(w)::value]; }, std::make_integer_sequence<int, W>{});
       acc *= (l > 0.f) ? 1.0f / l : 0.f;
       if (n_shares == 1) {
-        const int qi = query_of(p, col);
-        uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + d4;
+        const int qi = query_of(p, col0 + col);
+        uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col0 + col - qi * p.group)) * D + d4;
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(acc[0], acc[1]), pack_16x2<F16>(acc[2], acc[3])};
       } else {
         own.store(16u * (uint32_t)it, acc);
@@ -376,7 +386,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 #pragma unroll
       for (int i = 0; i < I; ++i) {
         if (it0 + i * threads >= quads) break;
-        const int col = (int)(at[i] / kQuads), qi = query_of(p, col);
+        const int col = col0 + (int)(at[i] / kQuads), qi = query_of(p, col);
         const f32x4_t o = acc[i] * ((l[i] > 0.f) ? 1.0f / l[i] : 0.f);
         uint16_t* dst = p.out + ((int64_t)(r.q_start + qi) * p.n_q + kvh * p.group + (col - qi * p.group)) * D + 4 * (at[i] % kQuads);
         *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{pack_16x2<F16>(o[0], o[1]), pack_16x2<F16>(o[2], o[3])};
@@ -388,27 +398,37 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   else merge(std::integral_constant<int, 16>{});
 }
 
-int nct_of(int64_t cols) { return (int)((cols + 15) / 16); }
+// A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256).  0: too many, see wide_round()
+struct ColGroups {
+  int groups, tiles;
+};
+ColGroups col_groups_of(int64_t head_dim, int64_t cols) {
+  const int tiles = (int)((cols + 15) / 16);
+  if (head_dim == 128) return tiles < 1 || tiles > 4 ? ColGroups{0, 0} : tiles == 4 ? ColGroups{2, 2} : ColGroups{1, tiles};
+  return tiles < 1 || tiles > 10 ? ColGroups{0, 0} : ColGroups{tiles, 1};
+}
 // waves of a workgroup: two per SIMD where a wave fits 256 registers
 int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
 
-template <int D, int NCT, int NW>
-int launch_shape(const ShareParams& sp, int share_len, unsigned blocks, hipStream_t stream) {
+template <int D, int NCT, int NW, bool WIDE>
+int launch_shape(const ShareParams& sp, const SharePlan& plan, unsigned blocks, hipStream_t stream) {
+  const int share_len = plan.share_len;
   auto log2_of = [](uint32_t x) { return 31u - (uint32_t)__builtin_clz(x); };
   // x / d for x < 2^31, d > 1: with 2^s the next power of two, m = ceil(2^(31 + s) / d), it is x m >> (31 + s)
   const uint32_t d = (uint32_t)share_len, s = log2_of(d - 1) + 1;
   const uint32_t magic = (uint32_t)(((1ull << (31 + s)) + d - 1) / d), groups = (uint32_t)sp.head_groups;
-  const ShareShape shape(s - 1, log2_of((uint32_t)NW / (uint32_t)sp.heads_wg), (groups & (groups - 1)) == 0 ? log2_of(groups) : ShareShape::kNoShift);
+  const ShareShape shape(s - 1, log2_of((uint32_t)NW / (uint32_t)sp.heads_wg), (groups & (groups - 1)) == 0 ? log2_of(groups) : ShareShape::kNoShift,
+                         (uint32_t)plan.col_groups);
   auto launch = [&](auto f16, auto mode_of) {
     constexpr bool F16 = decltype(f16)::value;
     constexpr int NEW = decltype(mode_of)::value;
-    const auto kernel = sp.s.walk == kStream ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW>
-                        : sp.s.walk == kWide ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW>
-                                             : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW>;
+    const auto kernel = sp.s.walk == kStream ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW, WIDE>
+                        : sp.s.walk == kWide ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, WIDE>
+                                             : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, WIDE>;
     return launch_kernel(kernel, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
                          sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
   };
-  if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
+  if constexpr (NCT == 1 && !WIDE) {  // IEEE half and new tokens exist for decode only (one column tile)
     const int mode = sp.s.nt.k == nullptr || sp.s.qo_indptr != nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
     if (sp.s.f16) {
       if (mode == kStored && sp.s.nt.k == nullptr)
@@ -444,8 +464,8 @@ static bool heads_alone(int64_t batch, int64_t n_kv) { return batch * n_kv <= de
 // fits with at most 16 shares to a request, from 256 on, and segments for fewer than 12 pairs: 16 and 11 %.
 // The same costs hold at head_dim 128: 12 700 launches of up to 25 pairs within 0.3-3 % of the best, where the shortest that fits with at most 16
 // shares to a request was 1-3 % from 12 pairs on, 3-44 % for 4 to 11 and up to 2x for fewer.
-static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols, int64_t least) {
-  const double slots = (double)device_cus(), mean = (double)(keys / batch), spread = 0.43 * std::sqrt((double)batch);
+static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols, int64_t least, int64_t round) {
+  const double slots = (double)round, mean = (double)(keys / batch), spread = 0.43 * std::sqrt((double)batch);
   int64_t len = 0;
   double lowest = 0;
   for (int64_t c = least; c < (1 << 20); c = (c & (c - 1)) ? c / 3 * 4 : c / 2 * 3) {
@@ -462,12 +482,28 @@ static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int6
   return len > 0 ? len : 1 << 20;
 }
 
+// Columns in several workgroups, each of which reads all of a share's keys: for launches of one round and few keys, where the tile
+// kernels' way (a block of 256 rows mostly empty, 13 us outside its loop, a merge launch) is longer.  2500 launches of 2-16 tokens a request, requests of
+// up to 64 K keys with and without a window of 1024, this by that (geometric mean, worst of a bin).  head_dim 256, by keys times column groups for
+// each compute unit: up to 64 0.72 (0.91), 181 0.72 (0.88), 256 0.77 (1.02), 362 0.86 (1.2), 512 0.96 (1.5), 724 1.09 (1.6); nine and ten groups 0.81 (0.94) up
+// to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.  head_dim 128: 49-64 columns
+// up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96, two groups of three tiles, 0.98 (1.2), three groups 0.95 (1.35); up to 192 keys a request 0.9-1.1,
+// more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens, window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12;
+// two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
+constexpr int64_t kXcds = 8;
+static int64_t wide_keys(int64_t head_dim) { return head_dim == 256 ? 400 : 512; }  // for each compute unit
+static bool wide_round(int64_t batch, int64_t keys, int64_t n_kv, int64_t slots, int64_t head_dim) {
+  return head_dim == 256 ? batch * n_kv <= slots && keys > 128 * batch : 4 * batch * n_kv <= 3 * slots && keys > 192 * batch;
+}
+
 SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols) {
   SharePlan plan{};
-  const int nct = nct_of(cols);
-  if (t_force < 0 || batch < 1 || cols < 1 || nct > (head_dim == 128 ? 3 : 1)) return plan;
+  const auto [col_groups, nct] = col_groups_of(head_dim, cols);
+  if (t_force < 0 || batch < 1 || col_groups == 0) return plan;
+  // (share, head group)s of a round, a compute unit to a workgroup; the column groups of one are on one XCD
+  const int64_t slots = col_groups == 1 ? device_cus() : device_cus() / (kXcds * col_groups) * kXcds;
+  if (col_groups > 1 && t_force == 0 && !wide_round(batch, keys, n_kv, slots, head_dim)) return plan;
   const int nw = waves_of(head_dim, nct);
-  const int64_t slots = device_cus();  // a workgroup takes a CU
   int64_t heads = 1, len;
   if (t_force > 0) {
     len = std::max<int64_t>(t_force & 0xfffff, 2);
@@ -480,7 +516,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     // average request: the last of them reads the others' partials.  Rounding adds half a share per request
     // and scatters around that: with two standard deviations more, 9 requests of 102-713 keys, 64 / 8 heads, have 192 keys a share
     // and take 12.5 us, without it 128, a few workgroups more than compute units, and 16.6
-    const bool alone = heads_alone(batch, n_kv);
+    const bool alone = col_groups > 1 || heads_alone(batch, n_kv);
     len = nct == 3 ? 512 : (nw == 4 && heads == 1 && !(head_dim == 256 && alone)) ? 256 : 128;
     const int64_t spread = (int64_t)std::sqrt((double)batch / 3);
     auto fits = [&](int64_t c) {
@@ -490,7 +526,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
       const int64_t n = std::min<int64_t>(std::max<int64_t>(slots * heads / (batch * n_kv), 1), 16);
       len = std::max(len, ((each + n - 1) / n + 31) & ~(int64_t)31);
     } else if (alone) {
-      len = cost_share_length(batch, keys, n_kv, cols, len);
+      len = cost_share_length(batch, keys, n_kv, std::min<int64_t>(cols, 16 * nct), len, slots);
     } else {
       while (!fits(len) && len < (1 << 19)) len = (len & (len - 1)) ? len / 3 * 4 : len / 2 * 3;
     }
@@ -505,6 +541,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
   plan.heads_wg = (int32_t)heads;
   plan.share_waves = nw / plan.heads_wg;
   plan.max_shares = keys / plan.share_len + batch;
+  plan.col_groups = col_groups;
   return plan;
 }
 
@@ -512,7 +549,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
 // where those alone are more: with n = one_round / batch, at least 1, share_plan() makes them of keys / (n batch) keys
 // or more, so keys / share_len is at most n batch.
 SharePlan with_any_window(SharePlan plan, int64_t batch, int64_t n_kv) {
-  const int64_t one_round = device_cus() * plan.heads_wg / n_kv;
+  const int64_t one_round = device_cus() * plan.heads_wg / (n_kv * plan.col_groups);
   plan.max_shares = std::max(plan.max_shares, std::max(one_round, batch) + batch);
   return plan;
 }
@@ -536,6 +573,7 @@ bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t he
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
+  if (plan.col_groups > 1) return keys * n_kv * plan.col_groups <= wide_keys(head_dim) * device_cus();
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
   if (few_pairs_in_segments(batch, n_kv, mean, head_dim, cols, false)) return false;
@@ -576,7 +614,7 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {
-  const size_t counts = (size_t)(batch * (n_kv / plan.heads_wg)) * sizeof(unsigned long long);
+  const size_t counts = (size_t)(batch * (n_kv / plan.heads_wg) * plan.col_groups) * sizeof(unsigned long long);
   const size_t rows = (size_t)plan.max_shares * (size_t)(n_kv * cols);
   return ((counts + 255) / 256 + (rows * (size_t)(head_dim + 1) * sizeof(float) + 255) / 256) * 256;
 }
@@ -585,25 +623,27 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   const int64_t group = a.n_q / a.n_kv, cols = group * a.max_len_extend;
   const int64_t head_groups = a.n_kv / plan.heads_wg;
   const bool rows = n.k != nullptr && a.qo_indptr != nullptr;  // kStoreRows
-  const int64_t blocks = plan.max_shares * head_groups + (rows ? kRestBlocks : 0);
+  const int64_t of_keys = plan.col_groups == 1 ? plan.max_shares * head_groups : (plan.max_shares * head_groups + 7) / 8 * 8 * plan.col_groups;
+  const int64_t blocks = of_keys + (rows ? kRestBlocks : 0);
   if (blocks > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   ShareParams sp{};
   fill_splitkv_params(a, sp.s);
   char* ws = static_cast<char*>(a.workspace);
   sp.counts = reinterpret_cast<unsigned long long*>(ws);
-  ws += ((size_t)(a.batch * head_groups) * sizeof(unsigned long long) + 255) / 256 * 256;
+  ws += ((size_t)(a.batch * head_groups * plan.col_groups) * sizeof(unsigned long long) + 255) / 256 * 256;
   sp.s.part_o = reinterpret_cast<float*>(ws);
   sp.s.part_lse = sp.s.part_o + (size_t)plan.max_shares * (size_t)(a.n_kv * cols * a.head_dim);
   sp.nonce = next_launch_number();
   sp.heads_wg = plan.heads_wg;
   sp.head_groups = (int32_t)head_groups;
   fill_new_tokens(n, sp.s);
-  sp.s.nt.blocks = (uint32_t)(plan.max_shares * head_groups);
-  const int nct = nct_of(cols);
-  if (a.head_dim == 256) return nct == 1 ? launch_shape<256, 1, 4>(sp, plan.share_len, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
-  if (nct == 1) return launch_shape<128, 1, 8>(sp, plan.share_len, (unsigned)blocks, stream);
-  if (nct == 2) return launch_shape<128, 2, 4>(sp, plan.share_len, (unsigned)blocks, stream);
-  return nct == 3 ? launch_shape<128, 3, 4>(sp, plan.share_len, (unsigned)blocks, stream) : MSGL_ERR_SHAPE;
+  sp.s.nt.blocks = (uint32_t)of_keys;
+  const int nct = col_groups_of(a.head_dim, cols).tiles;
+  const unsigned grid = (unsigned)blocks;
+  if (a.head_dim == 256) return plan.col_groups > 1 ? launch_shape<256, 1, 4, true>(sp, plan, grid, stream) : launch_shape<256, 1, 4, false>(sp, plan, grid, stream);
+  if (plan.col_groups > 1) return launch_shape<128, 2, 4, true>(sp, plan, grid, stream);
+  if (nct == 1) return launch_shape<128, 1, 8, false>(sp, plan, grid, stream);
+  return nct == 2 ? launch_shape<128, 2, 4, false>(sp, plan, grid, stream) : launch_shape<128, 3, 4, false>(sp, plan, grid, stream);
 }
 
 }  // namespace msgl
