@@ -91,6 +91,13 @@ bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv,
 // or many short requests): its segments are balanced whatever the lengths, and one long request
 // among many short ones would otherwise be one long workgroup per kv head.
 int64_t smallq_base_cols(int64_t head_dim) { return head_dim == 128 ? 48 : 16; }
+// Two column tiles of 256 dims in one wave of the split-K kernel (17 to 32 columns), which reads every row once and balances its segments
+// whatever the lengths; beside the tile kernel, by MiB of keys and values (geometric mean, worst, of 150 launches): 64 1.25 (1.5), 128 1.15 (1.3), 181
+// 1.0 (1.16), 256 0.92 (1.05), 362 0.81 (1.02), 512 0.79, 1024 0.72, 2048 0.67.  (us: 12 of 531 K keys in all, 6 tokens, 16 / 4 heads, 565 -> 341; six of
+// 84 K, 8, 32 / 8, 193 -> 125.)  33 to 64 columns, two such waves a head, 1.0-1.1 up to 2 GiB.
+bool two_tiles_in_segments(int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
+  return head_dim == 256 && cols > 16 && cols <= 32 && keys * n_kv * head_dim * 4 >= (int64_t)256 << 20;
+}
 
 }  // namespace
 
@@ -408,7 +415,7 @@ static bool use_splitkv_route(int64_t group, int64_t max_len_extend, int64_t hea
   if (max_len_extend < 1 || cols > msgl::kSplitKvMaxCols) return false;
   const int64_t t = t_tune[MSGL_TUNE_SMALLQ_MAXCOLS];
   if (t != 0) return t > 0 && cols <= t;  // set by hand; negative: never
-  if (cols <= smallq_base_cols(head_dim)) return true;
+  if (cols <= smallq_base_cols(head_dim) || two_tiles_in_segments(total_kv, n_kv, head_dim, cols)) return true;
   return ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim) == 0;
 }
 // Under a sliding window that most requests exceed (mean kv length at least twice the window),
@@ -418,8 +425,12 @@ static bool use_splitkv_route(int64_t group, int64_t max_len_extend, int64_t hea
 // does this; MSGL_TUNE_SMALLQ_MAXCOLS set by hand is obeyed as it stands.
 static bool window_prefers_tiles(int64_t batch, int64_t total_kv, int64_t n_kv, int64_t group,
                                  int64_t max_len_extend, int64_t head_dim, int64_t window) {
-  if (window <= 0 || head_dim != 128 || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
+  if (window <= 0 || t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0) return false;
   if (group * max_len_extend <= 16) return false;
+  if (head_dim == 256)  // what two_tiles_in_segments() took for its size is less under the window
+    return two_tiles_in_segments(total_kv, n_kv, head_dim, group * max_len_extend) &&
+           !two_tiles_in_segments(msgl::visible_keys(batch, total_kv, window, max_len_extend, false), n_kv, head_dim, group * max_len_extend) &&
+           ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim) > 0;
   if (total_kv < 2 * batch * (window + max_len_extend)) return false;
   return ragged_tiles(batch, total_kv, n_kv, group, max_len_extend, head_dim) > 0;
 }
@@ -547,13 +558,20 @@ static int prefill_attention(const void* q, const void* k_cache, const void* v_c
   const bool window_share = share_room && window_shares(plan, batch, total_kv, keys, num_kv_heads, head_dim, cols);
   const bool shares = share_room && shares_route(plan, window_share, batch, total_kv, keys, num_kv_heads, group, max_len_extend,
                                                  head_dim, sliding_window_size);
-  const bool direct = shares || (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
-                                 !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
-                                                       sliding_window_size));
-  if (direct) {
-    const int32_t n_seg = segments(total_kv, num_kv_heads, head_dim, cols);
+  bool direct = shares || (use_splitkv_route(group, max_len_extend, head_dim, batch, total_kv, num_kv_heads) &&
+                           !window_prefers_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim,
+                                                 sliding_window_size));
+  const int32_t n_seg = direct ? segments(total_kv, num_kv_heads, head_dim, cols) : 0;
+  if (direct && !shares) {
     const size_t need = msgl::splitkv_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, max_len_extend, n_seg);
-    if (!shares && (!workspace || workspace_bytes < need || !aligned16(workspace))) return MSGL_ERR_WORKSPACE;
+    const bool room = workspace && workspace_bytes >= need && aligned16(workspace);
+    // the tile kernel, which does without, where only the size asks for segments
+    if (!room && (t_tune[MSGL_TUNE_SMALLQ_MAXCOLS] != 0 || !two_tiles_in_segments(total_kv, num_kv_heads, head_dim, cols) ||
+                  ragged_tiles(batch, total_kv, num_kv_heads, group, max_len_extend, head_dim) == 0))
+      return MSGL_ERR_WORKSPACE;
+    direct = room;
+  }
+  if (direct) {
     msgl::SplitKvArgs a{};
     a.q = q;
     a.k_cache = k_cache;

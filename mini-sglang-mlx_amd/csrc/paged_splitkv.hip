@@ -162,6 +162,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
   const int kvh = (blockIdx.x - seg * p.head_groups) * p.nwh + (wave - cw * p.nwh);
   int seg_len, total, cur_b, vs;
   __shared__ __attribute__((aligned(16))) NewRowsLds<D> rows[NW];
+  __shared__ u32x4_t q_rows[Columns<D, NCT>::kQInLds ? NW : 1][Columns<D, NCT>::kQInts];
   if (NEW != kStored && seg == 0) {  // requests without keys come up in no segment
     for (int b0 = 0; b0 < p.batch; b0 += kWave) {
       const int b = min(b0 + lane, p.batch - 1);
@@ -197,6 +198,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     const int ncols = r.q_len * p.group;
 
     Columns<D, NCT> c_;
+    if constexpr (Columns<D, NCT>::kQInLds) c_.q = MSGL_LDS_PTR(u32x4_t, &q_rows[wave][0]) + lane;
     FirstIds ids = first_ids(p, r, t_begin, t_end);
     if constexpr (NEW == kStored) {
       start_columns(p, r, kvh, ct0, t_end, c_);
@@ -589,10 +591,16 @@ int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
 
 // How a shape's column tiles map onto waves: tiles per wave and waves per kv head.
 struct ColSplit { int nct_wave; int col_waves; };
-ColSplit col_split(int nct, int64_t head_dim) {
-  // head dim 256: one tile per wave (two would spill); three tiles take four waves, the last
-  // of which finds no valid column (workgroups come in 1, 2, 4 or 8 waves)
-  if (head_dim != 128) return ColSplit{1, nct == 3 ? 4 : nct};
+ColSplit col_split(int nct, int64_t head_dim, int64_t keys, int64_t n_kv) {
+  // head dim 256: two tiles in one wave from 64 MiB of keys and values on, three and four in two; its loads run less far ahead than
+  // those of one tile (attend_keys), which shows on little work.  One tile a wave below; three take four waves, the last of
+  // which finds no valid column (workgroups come in 1, 2, 4 or 8 waves).  130-900 requests of 32-2048 keys, two tiles a wave by one, by MiB:
+  // two tiles in all 23 1.19, 45 1.06, 64 1.0, 91 0.95, 181 0.88, 512 0.80; three and four 16 1.06, 32 0.99, 64 0.88, 181 0.81, 512 0.73, 724 0.68.
+  if (head_dim != 128) {
+    const bool two = keys * n_kv * head_dim * 4 >= (int64_t)64 << 20;
+    if (nct <= 1 || !two) return ColSplit{1, nct == 3 ? 4 : nct};
+    return nct == 2 ? ColSplit{2, 1} : ColSplit{2, 2};
+  }
   // head dim 128: up to three tiles in one wave (487 VGPRs; 33-48 columns run 22-26 % faster
   // than on two waves per kv head, which read every K / V row twice); four tiles spill, and with
   // the Q operand parked in LDS to avoid that they are no faster than two waves of two
@@ -600,13 +608,15 @@ ColSplit col_split(int nct, int64_t head_dim) {
 }
 
 template <int D>
-int launch_d(const SplitKvParams& p, int nct, hipStream_t stream) {
-  const ColSplit cs = col_split(nct, D);
+int launch_d(const SplitKvParams& p, int nct, int64_t keys, hipStream_t stream) {
+  const ColSplit cs = col_split(nct, D, keys, p.n_kv);
   const int waves = p.nwh * cs.col_waves;
   if (cs.nct_wave == 1) return launch_dn<D, 1>(p, waves, stream);
   if constexpr (D == 128) {
     if (cs.nct_wave == 2) return launch_dn<D, 2>(p, waves, stream);
     if (cs.nct_wave == 3) return launch_dn<D, 3>(p, waves, stream);
+  } else {
+    if (cs.nct_wave == 2) return launch_dn<D, 2>(p, waves, stream);
   }
   return MSGL_ERR_SHAPE;
 }
@@ -683,9 +693,9 @@ static int boundary_tokens(int64_t n_wgs, int nwh, int64_t head_dim) {
 // kv heads per workgroup for this shape: up to 4, halved when a second wave per head is
 // needed for the columns (a workgroup of the wide variants holds at most 4 waves: they
 // need more than 256 VGPRs, one wave per SIMD)
-static int nwh_for(int64_t n_kv, int nct, int64_t head_dim) {
+static int nwh_for(int64_t n_kv, int nct, int64_t head_dim, int64_t keys) {
   int nwh = heads_per_group(n_kv);
-  const int col_waves = col_split(nct, head_dim).col_waves;
+  const int col_waves = col_split(nct, head_dim, keys, n_kv).col_waves;
   const int max_waves = (nct == 1 && head_dim == 128) ? 8 : 4;
   while (nwh * col_waves > max_waves && nwh > 1) nwh /= 2;
   return nwh;
@@ -694,8 +704,8 @@ static int nwh_for(int64_t n_kv, int nct, int64_t head_dim) {
 int splitkv_default_segments(int64_t total_kv, int64_t n_kv, int64_t head_dim, int64_t cols,
                              int32_t min_seg) {
   const int nct = nct_for(cols);
-  const int nwh = nwh_for(n_kv, nct, head_dim);
-  const int waves = nwh * col_split(nct, head_dim).col_waves;
+  const int nwh = nwh_for(n_kv, nct, head_dim, total_kv);
+  const int waves = nwh * col_split(nct, head_dim, total_kv, n_kv).col_waves;
   const int64_t head_groups = n_kv / nwh;
   // Workgroups for 13 of every 16 CUs, at most one per CU (small workgroups are doubled up until
   // a CU holds four waves): the memory system is saturated well before every CU streams, and
@@ -749,7 +759,7 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   p.clock_probe = clock_probe();
   const uint64_t pool_bytes = (uint64_t)a.num_slots * (uint64_t)std::max(a.k_stride0, a.v_stride0) * 2u;
   const int64_t keys = visible_keys(a.batch, a.total_kv, a.window, a.max_len_extend, a.is_cross != 0);
-  const bool once = col_split(nct_for(p.cols), a.head_dim).col_waves == 1;
+  const bool once = col_split(nct_for(p.cols), a.head_dim, a.total_kv, a.n_kv).col_waves == 1;
   p.walk = once && streams(keys * a.n_kv * a.head_dim * 4) ? kStream : pool_bytes >= (1ull << 32) ? kWide : kNarrow;
 }
 
@@ -760,7 +770,7 @@ int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream)
   if (a.batch * a.max_len_extend > 0x7fffffffLL || a.total_kv > 0x7fffffffLL) return MSGL_ERR_SHAPE;
   if (a.batch == 0) return MSGL_OK;
   const int nct = nct_for(cols);
-  const int nwh = nwh_for(a.n_kv, nct, a.head_dim);
+  const int nwh = nwh_for(a.n_kv, nct, a.head_dim, a.total_kv);
 
   SplitKvParams p{};
   fill_splitkv_params(a, p);
@@ -777,8 +787,8 @@ int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream)
   p.boundary = boundary_tokens((int64_t)a.n_seg * (a.n_kv / nwh), nwh, a.head_dim);
   p.min_seg = a.min_seg;
   if ((int64_t)p.n_seg * p.head_groups > 0x7fffffffLL) return MSGL_ERR_SHAPE;
-  if (a.head_dim == 128) return launch_d<128>(p, nct, stream);
-  if (a.head_dim == 256) return launch_d<256>(p, nct, stream);
+  if (a.head_dim == 128) return launch_d<128>(p, nct, a.total_kv, stream);
+  if (a.head_dim == 256) return launch_d<256>(p, nct, a.total_kv, stream);
   return MSGL_ERR_HEAD_DIM;
 }
 

@@ -127,7 +127,10 @@ struct KvTile {
 // may see, and the running softmax state with the unnormalised output O^T.
 template <int D, int NCT>
 struct Columns {
-  u32x4_t q[NCT][D / 32];
+  // Two tiles of 256 dims leave no registers for Q beside the keys in flight: it is in LDS, a lane's 16 bytes 64 lanes apart.
+  static constexpr bool kQInLds = D == 256 && NCT > 1;
+  static constexpr int kQInts = kQInLds ? NCT * (D / 32) * kWave : 1;  // of 16 bytes
+  typename std::conditional<kQInLds, __attribute__((address_space(3))) u32x4_t*, u32x4_t[NCT][D / 32]>::type q;
   int lo[NCT], hi[NCT];        // first and last visible key of this lane's column in each tile
   int all_lo, all_hi;          // a tile of keys is mask-free iff inside [all_lo, all_hi]
   float m[NCT], l[NCT];        // running maximum (base 2); this lane's part of the sum
@@ -155,7 +158,8 @@ __device__ __forceinline__ void start_columns(const SplitKvParams& p, const ReqI
     for (int c = 0; c < KS; ++c) {
       u32x4_t raw = {0u, 0u, 0u, 0u};
       if (LOAD_Q && valid) raw = ld_global_b128(qrow + c * 32);
-      c_.q[ct][c] = raw;
+      if constexpr (Columns<D, NCT>::kQInLds) c_.q[(ct * KS + c) * kWave] = raw;
+      else c_.q[ct][c] = raw;
     }
     const int qpos = r.prefix + qi;
     int lo = (p.window > 0) ? qpos - p.window + 1 : 0;
@@ -212,24 +216,59 @@ __device__ __forceinline__ void lines_to_operands(KvTile<D>& t) {
       }
 }
 
-// Keys tb .. tb + 31, in registers, for the columns in `c_`.
+// The scores of a tile where Q is in LDS: S^T[token][col] for the two 16-token sub-tiles.
 template <int D, int NCT, bool F16>
-__device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTile<D>& t, int tb, Columns<D, NCT>& c_) {
+__device__ __forceinline__ void scores_from_lds(const KvTile<D>& t, const Columns<D, NCT>& c_, f32x4_t (&s)[2][NCT]) {
+  constexpr int KS = D / 32;
+  auto load = [&](int c, u32x4_t (&q)[NCT]) {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) q[ct] = c_.q[(ct * KS + c) * kWave];
+  };
+  u32x4_t q[2][NCT];
+  load(0, q[0]);
+#pragma unroll
+  for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) s[sub][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < KS; ++c) {
+    if (c + 1 < KS) load(c + 1, q[(c + 1) & 1]);
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) s[sub][ct] = mfma_16x16x32_raw<F16>(t.k[sub][c], q[c & 1][ct], s[sub][ct]);
+    __builtin_amdgcn_sched_barrier(0);  // no more of Q in registers than the next step's
+  }
+}
+
+// Keys tb .. tb + 31, in registers, for the columns in `c_`.  scored(): called when K is no longer wanted (Q in LDS)
+struct NothingElse {
+  __device__ __forceinline__ void operator()() const {}
+};
+template <int D, int NCT, bool F16, typename Scored = NothingElse>
+__device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTile<D>& t, int tb, Columns<D, NCT>& c_, Scored&& scored = {}) {
+  constexpr bool kQInLds = Columns<D, NCT>::kQInLds;
   constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
   const int g = lane_id() >> 4;
   // S^T[token][col] for the two 16-token sub-tiles
   f32x4_t s[2][NCT];
+  if constexpr (kQInLds) {
+    scores_from_lds<D, NCT, F16>(t, c_, s);
+    scored();
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
 #pragma unroll
-  for (int sub = 0; sub < 2; ++sub)
+    for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+      for (int ct = 0; ct < NCT; ++ct) {
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < KS; ++c)
-        acc = mfma_16x16x32_raw<F16>(t.k[sub][c], c_.q[ct][c], acc);
-      s[sub][ct] = acc;
-    }
+        for (int c = 0; c < KS; ++c)
+          acc = mfma_16x16x32_raw<F16>(t.k[sub][c], c_.q[ct][c], acc);
+        s[sub][ct] = acc;
+      }
+  }
   const bool need_mask = (tb < c_.all_lo) || (tb + 31 > c_.all_hi);
   uint32_t pb[NCT][4];
 #pragma unroll
@@ -275,6 +314,7 @@ __device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTil
         for (int n = 0; n < 8; ++n) c_.o[ct][hf][n] *= alpha;
     }
   }
+  if constexpr (kQInLds) __builtin_amdgcn_sched_barrier(0);
   // O^T += V^T P^T.  MFMA n of half hf produces d = hf*128 + 8*row + n on row = l%16.
 #pragma unroll
   for (int hf = 0; hf < VH; ++hf)
@@ -292,6 +332,7 @@ __device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTil
         const u32x4_t pv = {pb[ct][0], pb[ct][1], pb[ct][2], pb[ct][3]};
         c_.o[ct][hf][n] = mfma_16x16x32_raw<F16>(vt, pv, c_.o[ct][hf][n]);
       }
+      if constexpr (kQInLds) __builtin_amdgcn_sched_barrier(0);  // (and no more transposed V than one product's)
     }
 }
 
@@ -337,7 +378,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     s0 = (int)min((uint32_t)idx_base[min(tb + t16, last_tok)], p.max_slot);
     s1 = (int)min((uint32_t)idx_base[min(tb + 16 + t16, last_tok)], p.max_slot);
   };
-  auto load_tile = [&](KvTile<D>& t, int s0, int s1) {
+  auto load_k = [&](KvTile<D>& t, int s0, int s1) {
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int s = sub ? s1 : s0;
@@ -352,6 +393,8 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
         for (int c = 0; c < KS; ++c) t.k[sub][c] = ld_global_b128(row + c * 64);
       }
     }
+  };
+  auto load_v = [&](KvTile<D>& t, int s0, int s1) {
     // V rows of this lane group: tokens 4g+j (j<4) of sub-tile 0, then of sub-tile 1;
     // their slot ids sit in lanes 4g+j of the K index registers.
 #pragma unroll
@@ -364,6 +407,33 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     }
   };
 
+  auto load_tile = [&](KvTile<D>& t, int s0, int s1) {
+    load_k(t, s0, s1);
+    load_v(t, s0, s1);
+  };
+
+  if constexpr (Columns<D, NCT>::kQInLds) {
+    // ---- one register tile: the next one's K comes in beside the softmax and the PV product, its V beside the next scores
+    // (and whatever comes meanwhile has a tile of its own: it comes first)
+    meanwhile();
+    __builtin_amdgcn_sched_barrier(0);
+    KvTile<D> t;
+    int i0 = (int)min((uint32_t)first.a[0], p.max_slot), i1 = (int)min((uint32_t)first.a[1], p.max_slot);
+    load_tile(t, i0, i1);
+    i0 = (int)min((uint32_t)first.b[0], p.max_slot);
+    i1 = (int)min((uint32_t)first.b[1], p.max_slot);
+    for (int tok = t_begin; tok < t_end; tok += 32) {
+      if constexpr (LINES) lines_to_operands(t);
+      const int v0 = i0, v1 = i1;
+      compute_tile<D, NCT, F16>(p, t, tok, c_, [&] {
+        load_k(t, v0, v1);
+        load_idx(tok + 64, i0, i1);
+      });
+      load_v(t, v0, v1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return;
+  }
   // ---- tile loop: two register tiles, slot ids fetched two tiles ahead.  Every load in
   // the loop body is unconditional (tokens past the range clamp to its last token and
   // are masked), so the number of loads in flight at each wait is a compile-time
