@@ -312,7 +312,7 @@ static size_t decode_step_route(int64_t batch, int64_t total_kv, int64_t num_q_h
   if (!msgl::shares_preferred(*plan, batch, total_kv, num_kv_heads, head_dim, group)) {
     // norm and rotary embedding would be made anew by every segment of a request: 3.5 us of a launch of their own is
     // less on the launches that go in segments.  On large ones the store's launch hides behind the start of the next,
-    // and its part of the segments is paid by the slowest of them; us, store in front against inside, by MiB of keys and
+    // and its part of the segments is paid by the slowest of them; us (all read through the caches), store in front against inside, by MiB of keys and
     // values: 22 23.3 and 20.9 (2 requests, 24 / 4 heads of 256), 113 24.2 and 22.4 (1), 183 38.2 and 37.0 (68); 281
     // 53.5 and 53.6 (16 requests), 366 81.2 and 83.4 (128), 625 126.8 and 127.8 (64); at head_dim 256 312 65.3 and 63.5 (16)
     if (norm_rope || (total_kv * num_kv_heads * head_dim * 4 >> 20) > (head_dim == 256 ? 384 : 192)) return 0;
