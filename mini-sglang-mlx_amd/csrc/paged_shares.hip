@@ -398,13 +398,14 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   else merge(std::integral_constant<int, 16>{});
 }
 
-// A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256).  0: too many, see wide_round()
+// A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256; of several workgroups two
+// and one).  0: too many, see wide_round()
 struct ColGroups {
   int groups, tiles;
 };
 ColGroups col_groups_of(int64_t head_dim, int64_t cols) {
   const int tiles = (int)((cols + 15) / 16);
-  if (head_dim == 128) return tiles < 1 || tiles > 4 ? ColGroups{0, 0} : tiles == 4 ? ColGroups{2, 2} : ColGroups{1, tiles};
+  if (head_dim == 128) return tiles < 1 || tiles > 8 ? ColGroups{0, 0} : tiles > 3 ? ColGroups{(tiles + 1) / 2, 2} : ColGroups{1, tiles};
   return tiles < 1 || tiles > 10 ? ColGroups{0, 0} : ColGroups{tiles, 1};
 }
 // waves of a workgroup: two per SIMD where a wave fits 256 registers
@@ -486,10 +487,10 @@ static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int6
 // kernels' way (a block of 256 rows mostly empty, 13 us outside its loop, a merge launch) is longer.  2500 launches of 2-16 tokens a request, requests of
 // up to 64 K keys with and without a window of 1024, this by that (geometric mean, worst of a bin).  head_dim 256, by keys times column groups for
 // each compute unit: up to 64 0.72 (0.91), 181 0.72 (0.88), 256 0.77 (1.02), 362 0.86 (1.2), 512 0.96 (1.5), 724 1.09 (1.6); nine and ten groups 0.81 (0.94) up
-// to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.  head_dim 128: 49-64 columns
-// up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96, two groups of three tiles, 0.98 (1.2), three groups 0.95 (1.35); up to 192 keys a request 0.9-1.1,
-// more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens, window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12;
-// two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
+// to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.  head_dim 128, by the same, in
+// groups of two tiles: 49-64 columns up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96 0.73 (1.04), 0.80 (0.97), 0.93 (1.11); 97-128 0.72 (0.98), 0.76
+// (0.96), 0.88 (1.1) (of three tiles 65-96 0.98 (1.2)); up to 192 keys a request 0.9-1.1, more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens,
+// window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12; two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
 constexpr int64_t kXcds = 8;
 static int64_t wide_keys(int64_t head_dim) { return head_dim == 256 ? 400 : 512; }  // for each compute unit
 static bool wide_round(int64_t batch, int64_t keys, int64_t n_kv, int64_t slots, int64_t head_dim) {
