@@ -88,6 +88,7 @@ struct SharePlan {
   int32_t heads_wg;     // adjacent kv heads of a workgroup
   int64_t max_shares;   // most shares these sizes can give
   int32_t col_groups;   // workgroups that a share's columns go to
+  int32_t col_tiles;    // most tiles of 16 columns of one
 };
 // for `keys` visible keys in all; each > 0: about so many in every request
 SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols);

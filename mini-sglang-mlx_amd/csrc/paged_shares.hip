@@ -398,16 +398,6 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   else merge(std::integral_constant<int, 16>{});
 }
 
-// A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256; of several workgroups two
-// and one).  0: too many, see wide_round()
-struct ColGroups {
-  int groups, tiles;
-};
-ColGroups col_groups_of(int64_t head_dim, int64_t cols) {
-  const int tiles = (int)((cols + 15) / 16);
-  if (head_dim == 128) return tiles < 1 || tiles > 8 ? ColGroups{0, 0} : tiles > 3 ? ColGroups{(tiles + 1) / 2, 2} : ColGroups{1, tiles};
-  return tiles < 1 || tiles > 10 ? ColGroups{0, 0} : ColGroups{tiles, 1};
-}
 // waves of a workgroup: two per SIMD where a wave fits 256 registers
 int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
 
@@ -488,7 +478,7 @@ static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int6
 // up to 64 K keys with and without a window of 1024, this by that (geometric mean, worst of a bin).  head_dim 256, by keys times column groups for
 // each compute unit: up to 64 0.72 (0.91), 181 0.72 (0.88), 256 0.77 (1.02), 362 0.86 (1.2), 512 0.96 (1.5), 724 1.09 (1.6); nine and ten groups 0.81 (0.94) up
 // to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.  head_dim 128, by the same, in
-// groups of two tiles: 49-64 columns up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96 0.73 (1.04), 0.80 (0.97), 0.93 (1.11); 97-128 0.72 (0.98), 0.76
+// groups of two tiles (see col_groups_of() for those of one): 49-64 columns up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96 0.73 (1.04), 0.80 (0.97), 0.93 (1.11); 97-128 0.72 (0.98), 0.76
 // (0.96), 0.88 (1.1) (of three tiles 65-96 0.98 (1.2)); up to 192 keys a request 0.9-1.1, more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens,
 // window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12; two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
 constexpr int64_t kXcds = 8;
@@ -497,13 +487,40 @@ static bool wide_round(int64_t batch, int64_t keys, int64_t n_kv, int64_t slots,
   return head_dim == 256 ? batch * n_kv <= slots && keys > 128 * batch : 4 * batch * n_kv <= 3 * slots && keys > 192 * batch;
 }
 
+// (share, head group)s of a round, a compute unit to a workgroup; the column groups of one are on one XCD
+static int64_t round_slots(int64_t col_groups) { return col_groups == 1 ? device_cus() : device_cus() / (kXcds * col_groups) * kXcds; }
+
+// A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256; of several
+// workgroups two and one).  0: too many.  At head_dim 128 a workgroup to each tile where those are few enough for a round: eight waves instead of four, half
+// or a third to put together.  600 launches of 17-48 columns, that by all tiles in one workgroup: two tiles 0.76-0.80 (0.91), beyond 256 keys for each
+// compute unit 0.85 (1.08); three 0.60 (0.73) and 0.70 (0.83), in two workgroups 0.78 (0.93).  49-128 columns, a tile to each by two: up to 128 0.77 (0.85), 256 0.80
+// (0.89), 512 0.89 (1.03).  (us: one of 953 keys, 6 tokens, 64 / 8 heads, 18.8 -> 9.2; four of 5, window 1024, 32 / 4, 17.3
+// -> 10.2; two of 722 keys in all, 10 tokens, 32 / 4, 12.8 -> 8.3.)
+struct ColGroups {
+  int groups, tiles;
+};
+static ColGroups col_groups_of(int64_t head_dim, int64_t cols, int64_t batch, int64_t keys, int64_t n_kv) {
+  const bool d256 = head_dim == 256;
+  const int tiles = (int)((cols + 15) / 16);
+  if (tiles < 1 || tiles > (d256 ? 10 : 8)) return ColGroups{0, 0};
+  const ColGroups together{1, tiles}, pairs{(tiles + 1) / 2, 2}, apart{tiles, 1};
+  if (tiles == 1) return together;
+  if (t_force > 0) return d256 ? apart : tiles <= 3 ? together : pairs;
+  auto in_round = [&](const ColGroups& c) { return wide_round(batch, keys, n_kv, round_slots(c.groups), head_dim); };
+  auto fits = [&](const ColGroups& c) { return in_round(c) && keys * n_kv * c.groups <= wide_keys(head_dim) * device_cus(); };
+  if (fits(apart)) return apart;
+  if (!d256 && tiles > 2 && fits(pairs)) return pairs;
+  if (!d256 && tiles <= 3) return together;
+  const ColGroups any = d256 ? apart : pairs;  // (too many keys, but a window, unknown where a workspace's size is asked for, may make them few)
+  return in_round(any) ? any : ColGroups{0, 0};
+}
+
 SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, int64_t head_dim, int64_t cols) {
   SharePlan plan{};
-  const auto [col_groups, nct] = col_groups_of(head_dim, cols);
-  if (t_force < 0 || batch < 1 || col_groups == 0) return plan;
-  // (share, head group)s of a round, a compute unit to a workgroup; the column groups of one are on one XCD
-  const int64_t slots = col_groups == 1 ? device_cus() : device_cus() / (kXcds * col_groups) * kXcds;
-  if (col_groups > 1 && t_force == 0 && !wide_round(batch, keys, n_kv, slots, head_dim)) return plan;
+  if (t_force < 0 || batch < 1) return plan;
+  const auto [col_groups, nct] = col_groups_of(head_dim, cols, batch, keys, n_kv);
+  if (col_groups == 0) return plan;
+  const int64_t slots = round_slots(col_groups);
   const int nw = waves_of(head_dim, nct);
   int64_t heads = 1, len;
   if (t_force > 0) {
@@ -543,6 +560,7 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
   plan.share_waves = nw / plan.heads_wg;
   plan.max_shares = keys / plan.share_len + batch;
   plan.col_groups = col_groups;
+  plan.col_tiles = nct;
   return plan;
 }
 
@@ -615,7 +633,8 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {
-  const size_t counts = (size_t)(batch * (n_kv / plan.heads_wg) * plan.col_groups) * sizeof(unsigned long long);
+  // (under a window a request's columns may go to more workgroups, as many as tiles)
+  const size_t counts = (size_t)(batch * (n_kv / plan.heads_wg) * ((cols + 15) / 16)) * sizeof(unsigned long long);
   const size_t rows = (size_t)plan.max_shares * (size_t)(n_kv * cols);
   return ((counts + 255) / 256 + (rows * (size_t)(head_dim + 1) * sizeof(float) + 255) / 256) * 256;
 }
@@ -639,10 +658,11 @@ int launch_shares(const SplitKvArgs& a, const NewTokens& n, const SharePlan& pla
   sp.head_groups = (int32_t)head_groups;
   fill_new_tokens(n, sp.s);
   sp.s.nt.blocks = (uint32_t)of_keys;
-  const int nct = col_groups_of(a.head_dim, cols).tiles;
+  const int nct = plan.col_tiles;
   const unsigned grid = (unsigned)blocks;
   if (a.head_dim == 256) return plan.col_groups > 1 ? launch_shape<256, 1, 4, true>(sp, plan, grid, stream) : launch_shape<256, 1, 4, false>(sp, plan, grid, stream);
-  if (plan.col_groups > 1) return launch_shape<128, 2, 4, true>(sp, plan, grid, stream);
+  if (plan.col_groups > 1)
+    return nct == 1 ? launch_shape<128, 1, 8, true>(sp, plan, grid, stream) : launch_shape<128, 2, 4, true>(sp, plan, grid, stream);
   if (nct == 1) return launch_shape<128, 1, 8, false>(sp, plan, grid, stream);
   return nct == 2 ? launch_shape<128, 2, 4, false>(sp, plan, grid, stream) : launch_shape<128, 3, 4, false>(sp, plan, grid, stream);
 }

@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 CASES = [  # n_q, n_kv, head_dim, kv lengths, query tokens, window
     (49, 1, 128, [700, 1900], [1, 1], 0), (32, 4, 128, [3000, 260, 900], [8, 3, 1], 0), (32, 8, 128, [1500, 800, 2200, 400], [16, 5, 13, 4], 1024),
     (64, 8, 128, [500, 700], [8, 7], 0), (64, 8, 128, [500, 1700], [9, 12], 0), (48, 6, 128, [2600, 130, 900], [16, 2, 9], 513),
+    (32, 8, 128, [2000, 700, 90], [8, 5, 2], 0), (64, 8, 128, [900, 400, 250], [5, 6, 1], 300), (34, 2, 128, [1500], [1], 0),
     (48, 6, 128, [2600], [7], 513), (24, 3, 128, [900, 0, 7], [7, 0, 7], 0),
     (17, 1, 256, [600], [1], 0), (8, 1, 256, [3000, 130, 700], [4, 3, 2], 0), (24, 4, 256, [420, 900], [6, 1], 129), (16, 4, 256, [4100, 300], [9, 12], 0),
     (32, 2, 256, [700, 640, 5], [10, 7, 5], 0), (16, 2, 256, [1000] * 6 + [9], [16] * 6 + [3], 200), (40, 2, 256, [2000, 300], [8, 2], 0),
@@ -37,6 +38,7 @@ def test_against_the_oracle(gpu, tuning, n_q, n_kv, d, kv, ext, window, cross, s
 
 STORES = [  # cached, new tokens, n_q, n_kv, head_dim
     ([700, 300, 900], [8, 3, 8], 32, 4, 128), ([400, 700], [16, 1], 32, 8, 128), ([900, 200, 0], [8, 7, 5], 64, 8, 128), ([900, 300, 250], [16, 3, 10], 64, 8, 128),
+    ([700, 300, 900], [8, 3, 5], 32, 8, 128), ([1900, 300], [5, 1], 64, 8, 128),
     ([600], [2], 24, 2, 256), ([900, 140], [5, 12], 16, 4, 256), ([800, 300, 700], [10, 0, 4], 32, 2, 256), ([500, 600], [33, 9], 8, 2, 256),
 ]
 
@@ -57,7 +59,8 @@ def test_one_launch_is_two(gpu, tuning, cached, ext, n_q, n_kv, d, cross, window
     (256, 64, 200, 8, 2, 6), (256, 65, 200, 8, 2, 6), (256, 32, 150, 8, 1, 14), (256, 33, 150, 8, 1, 14), (256, 1, 25600, 16, 2, 4), (256, 1, 25664, 16, 2, 4),
     (256, 2, 128, 16, 2, 4), (256, 2, 129, 16, 2, 4), (256, 2, 600, 32, 2, 10), (256, 2, 600, 32, 2, 11), (128, 12, 193, 32, 8, 16), (128, 13, 193, 32, 8, 16),
     (128, 1, 8192, 32, 8, 16), (128, 1, 8193, 32, 8, 16), (128, 2, 192, 64, 8, 7), (128, 2, 193, 64, 8, 7), (128, 2, 500, 64, 8, 8), (128, 2, 500, 64, 8, 9),
-    (128, 1, 4096, 64, 8, 16), (128, 1, 4097, 64, 8, 16), (128, 6, 500, 64, 8, 16), (128, 7, 500, 64, 8, 16), (128, 1, 500, 64, 8, 17)])
+    (128, 1, 4096, 64, 8, 16), (128, 1, 4097, 64, 8, 16), (128, 6, 500, 64, 8, 16), (128, 7, 500, 64, 8, 16), (128, 1, 500, 64, 8, 17),
+    (128, 12, 300, 32, 8, 8), (128, 13, 300, 32, 8, 8), (128, 1, 8192, 32, 8, 8), (128, 1, 8193, 32, 8, 8), (128, 7, 300, 64, 8, 6), (128, 8, 300, 64, 8, 6), (128, 9, 300, 64, 8, 6)])
 def test_the_lines(gpu, d, batch, keys, n_q, n_kv, q_len):
     wl = build_workload("lines", "prefill", seed=keys, n_q=n_q, n_kv=n_kv, head_dim=d, kv_lens=[keys] * batch, extend_lens=[q_len] * batch)
     args = lambda w: (w.q, w.k_cache, w.v_cache, w.qo_indptr, w.kv_indptr, w.kv_indices, w.prefix_lens, w.sm_scale, q_len)  # noqa: E731
