@@ -10,9 +10,9 @@
 //   A request's visible keys are cut into ceil(keys / share_len) equal shares.  A workgroup takes one
 //   share of `heads_wg` adjacent kv heads; `share_waves` waves cut the share of each head into
 //   adjacent ranges, so a share is read with every load of its first tiles in flight at once.  The
-//   waves of a head meet in LDS.  (Columns that a wave has no registers for go to several workgroups, see wide_round().)  The grid holds the largest number of shares the sizes allow; a
-//   workgroup finds its (request, share) with one wave-wide prefix sum over kv_indptr and takes the
-//   request's geometry from the same registers; a workgroup past the last share ends.
+//   waves of a head meet in LDS.  (The columns of small launches go to several workgroups, a tile or two to each: col_groups_of().)
+//   The grid holds the largest number of shares the sizes allow; a workgroup finds its (request, share) with one
+//   wave-wide prefix sum over kv_indptr and takes the request's geometry from the same registers; a workgroup past the last share ends.
 //   A request with one share is written at once.  Otherwise the share's normalised fp32 partial and
 //   its log-sum-exp go to the workspace, the workgroup counts itself in the request's count word, and
 //   the one that counts last reads the others and writes the result: nobody waits for anybody.
@@ -477,9 +477,10 @@ static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int6
 // kernels' way (a block of 256 rows mostly empty, 13 us outside its loop, a merge launch) is longer.  2500 launches of 2-16 tokens a request, requests of
 // up to 64 K keys with and without a window of 1024, this by that (geometric mean, worst of a bin).  head_dim 256, by keys times column groups for
 // each compute unit: up to 64 0.72 (0.91), 181 0.72 (0.88), 256 0.77 (1.02), 362 0.86 (1.2), 512 0.96 (1.5), 724 1.09 (1.6); nine and ten groups 0.81 (0.94) up
-// to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.  head_dim 128, by the same, in
-// groups of two tiles (see col_groups_of() for those of one): 49-64 columns up to 256 0.73 (0.88), 512 0.82 (0.92), 724 0.98; 65-96 0.73 (1.04), 0.80 (0.97), 0.93 (1.11); 97-128 0.72 (0.98), 0.76
-// (0.96), 0.88 (1.1) (of three tiles 65-96 0.98 (1.2)); up to 192 keys a request 0.9-1.1, more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens,
+// to 256, eleven and more 0.95 (1.06) and 1.2-1.7 beyond; up to 128 keys a request 0.95-1.05, more than a round of workgroups 1.1-2.
+// head_dim 128, by the same, in groups of two tiles (col_groups_of() has those of one): 49-64 columns up to 256 0.73 (0.88), 512 0.82 (0.92), 724
+// 0.98; 65-96 0.73 (1.04), 0.80 (0.97), 0.93 (1.11); 97-128 0.72 (0.98), 0.76 (0.96), 0.88 (1.1) (of three tiles 65-96 0.98 (1.2)); up to 192 keys a
+// request 0.9-1.1, more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens,
 // window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12; two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
 constexpr int64_t kXcds = 8;
 static int64_t wide_keys(int64_t head_dim) { return head_dim == 256 ? 400 : 512; }  // for each compute unit
@@ -493,8 +494,8 @@ static int64_t round_slots(int64_t col_groups) { return col_groups == 1 ? device
 // A request's columns by tiles of 16: workgroups on them, and the tiles of one (three fit a wave at head_dim 128, one at 256; of several
 // workgroups two and one).  0: too many.  At head_dim 128 a workgroup to each tile where those are few enough for a round: eight waves instead of four, half
 // or a third to put together.  600 launches of 17-48 columns, that by all tiles in one workgroup: two tiles 0.76-0.80 (0.91), beyond 256 keys for each
-// compute unit 0.85 (1.08); three 0.60 (0.73) and 0.70 (0.83), in two workgroups 0.78 (0.93).  49-128 columns, a tile to each by two: up to 128 0.77 (0.85), 256 0.80
-// (0.89), 512 0.89 (1.03).  (us: one of 953 keys, 6 tokens, 64 / 8 heads, 18.8 -> 9.2; four of 5, window 1024, 32 / 4, 17.3
+// compute unit 0.85 (1.08); three 0.60 (0.73) and 0.70 (0.83), in two workgroups 0.78 (0.93).  49-128 columns, a tile to each by two: up to
+// 128 0.77 (0.85), 256 0.80 (0.89), 512 0.89 (1.03).  (us: one of 953 keys, 6 tokens, 64 / 8 heads, 18.8 -> 9.2; four of 5, window 1024, 32 / 4, 17.3
 // -> 10.2; two of 722 keys in all, 10 tokens, 32 / 4, 12.8 -> 8.3.)
 struct ColGroups {
   int groups, tiles;
