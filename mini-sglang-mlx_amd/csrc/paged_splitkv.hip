@@ -12,12 +12,12 @@
 //   16 CUs, all resident at once, one round, no tail; the HBM system, not the CUs, is the limit).
 //   A workgroup owns one segment and `nwh` adjacent kv heads, one wave64 per head; all
 //   waves walk the same tokens, so the workgroup touches nwh*256-byte stretches of every
-//   slot row together.  A wave holds up to two tiles of 16 columns; shapes with more
-//   columns add a second wave per head (measured: a second wave re-reading the rows costs
+//   slot row together.  A wave holds up to three tiles of 16 columns (two at head_dim 256); shapes
+//   with more columns add a second wave per head (measured: a second wave re-reading the rows costs
 //   about as much as reading them from HBM, so columns stay in one wave when they fit).
 //   A segment may
 //   cross request boundaries: the wave finishes one request's share (writing bf16 output
-//   directly if it covered the whole request, otherwise a normalised fp32 partial + base-2
+//   directly if it covered the whole request, otherwise a normalised partial + base-2
 //   LSE) and continues with the next.  splitkv_merge_kernel combines the partials.
 //   The host never reads device metadata: every wave derives its segment from kv_indptr
 //   (and qo_indptr / prefix_lens) with a wave-wide prefix sum.
@@ -46,7 +46,7 @@
 namespace msgl {
 namespace {
 
-// Element type of the partials.  bf16 launches keep them as IEEE half: a normalised partial row is
+// Element type of the partials.  bf16 launches, but for fp32_partials(), keep them as IEEE half: a normalised partial row is
 // a weighted mean of V rows, every bf16 value of ordinary size is a half value exactly (a share
 // that holds all of a row's weight hands the V row on unchanged), and half's 11 significant bits
 // are 8 times finer than the bf16 result the merge rounds to.  Values are clamped to half's range,
@@ -54,7 +54,15 @@ namespace {
 // queries a request but 7 % of the time (their stores compete with everybody's reads); halved,
 // the verify shape gains 3 %.  (16-bit fixed point against the row's largest element is finer on
 // rows that average many keys and coarser on a row's small elements: a copied V row then is no
-// longer exact.)  IEEE-half launches, whose results are as fine as such a partial, keep fp32.
+// longer exact.)  IEEE-half launches, whose results are as fine as such a partial, keep fp32, and so do two column tiles of 256 dims in a
+// wave: large launches go that way for their size alone, instead of to the tile kernel, whose partials are fp32, and what a call gives for values of V
+// beyond half's range, very small or not finite does not change with its size.  us, half and fp32: 12 requests of 528 K keys in all, 6 tokens,
+// 16 / 4 heads, 344.6 and 348.3; six of 84 K, 8, 32 / 8, 124.2 and 126.8; 64 of 350 K, 4, 16 / 2, 146.5 and 158.4; 200 of 65 K, 8, 32 / 8, 139.0 and 148.1.
+// (Either, by a parameter of the launch: 40 spilled registers, 363, 138, 162 and 146.)
+template <int D, int NCT, bool F16>
+constexpr bool fp32_partials() {
+  return F16 || (D == 256 && NCT == 2);
+}
 typedef _Float16 f16x8s_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2s_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_half2_clamped(float lo, float hi) {
@@ -237,7 +245,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
           }
       } else {
         const int64_t block = (int64_t)(seg + cur_b) * p.n_kv + kvh;
-        if constexpr (F16) {
+        if constexpr (fp32_partials<D, NCT, F16>()) {
 #pragma unroll
           for (int hf = 0; hf < VH; ++hf)
 #pragma unroll
@@ -287,7 +295,7 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
 constexpr int kMergeUnroll = 3;
 constexpr int kMergeSmall = 8;
 constexpr int kMergeWaves = 4;
-template <int D, bool F16>
+template <int D, bool F16, bool F32>  // F32: the partials'
 __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_kernel(SplitKvParams p) {
   constexpr int NW = kMergeWaves;
   constexpr int LPI = D / 8;          // lanes per item
@@ -332,7 +340,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_kernel(SplitKv
       if (u < n_items) {
         ls[u] = p.part_lse[row0 + u * stride];
         const int64_t at = partial_offset(block0 + (int64_t)u * p.n_kv, p.cols, col, lane * PER, D);
-        if constexpr (F16) {
+        if constexpr (F32) {
           const float* src = p.part_o + at;
 #pragma unroll
           for (int e = 0; e < PER; ++e) v[u][e] = src[e];
@@ -384,7 +392,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_kernel(SplitKv
       if (it < n_items) {
         lse[u] = p.part_lse[row0 + it * stride];
         const int64_t at = partial_offset(block0 + (int64_t)it * p.n_kv, p.cols, col, dl * 8, D);
-        if constexpr (F16) {
+        if constexpr (F32) {
           const float* src = p.part_o + at;
           va[u][0] = *reinterpret_cast<const f32x4_t*>(src);
           va[u][1] = *reinterpret_cast<const f32x4_t*>(src + 4);
@@ -463,7 +471,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_kernel(SplitKv
 // every lane the items by eight (four where there are no more), all their loads in flight together.  A workgroup of one
 // wave per row was bound by the launching of workgroups: us, 32 requests of 8 tokens at 32 heads 7.4 -> 6.4, 55 of 12
 // 11.1 -> 7.5, 13 of 5-16 at 16 heads 8.6 -> 6.0.
-template <int D, bool F16>
+template <int D, bool F16, bool F32>  // F32: the partials'
 __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_rows_kernel(SplitKvParams p) {
   constexpr int LPR = D / 8, RPW = kWave / LPR;
   const int b = blockIdx.x / p.max_len_extend;
@@ -490,13 +498,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_rows_kernel(Sp
     constexpr int U = decltype(in_flight)::value;
     for (int it0 = 0; it0 < n_items; it0 += U) {
       float lse[U];
-      typename std::conditional<F16, f32x4_t[2], f16x8s_t[1]>::type v[U];
+      typename std::conditional<F32, f32x4_t[2], f16x8s_t[1]>::type v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {  // items past the last: that again, with weight 0
         const int64_t block = block0 + (int64_t)min(it0 + u, n_items - 1) * p.n_kv;
         const int64_t at = partial_offset(block, p.cols, col, dl * 8, D);
         lse[u] = p.part_lse[block * p.cols + col];
-        if constexpr (F16) {
+        if constexpr (F32) {
           v[u][0] = *reinterpret_cast<const f32x4_t*>(p.part_o + at);
           v[u][1] = *reinterpret_cast<const f32x4_t*>(p.part_o + at + 4);
         } else {
@@ -518,7 +526,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void splitkv_merge_rows_kernel(Sp
         const float w = fast_exp2(lse[u] - m_safe);  // 0 for an item that is not there
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          if constexpr (F16) acc[e] += w * v[u][e >> 2][e & 3];
+          if constexpr (F32) acc[e] += w * v[u][e >> 2][e & 3];
           else acc[e] += w * (float)v[u][0][e];
         }
         wsum += w;
@@ -581,12 +589,13 @@ int launch_dn(const SplitKvParams& p, int waves, hipStream_t stream) {
   // and the rows are few enough that the extra waves cost nothing
   constexpr int kItemsPerTrip = kWave / (D / 8) * (1 + kMergeUnroll);
   const bool wide_merge = p.n_seg > kItemsPerTrip && (int64_t)mgrid.x * mgrid.y <= 1024;
+  constexpr bool kF32 = fp32_partials<D, NCT, false>();
   if (wide_merge) {
-    return launch_kernel(p.f16 ? splitkv_merge_kernel<D, true> : splitkv_merge_kernel<D, false>, mgrid, dim3(64 * kMergeWaves), stream, p);
+    return launch_kernel(p.f16 ? splitkv_merge_kernel<D, true, true> : splitkv_merge_kernel<D, false, kF32>, mgrid, dim3(64 * kMergeWaves), stream, p);
   }
   constexpr unsigned kRows = kMergeWaves * (kWave / (D / 8));  // of a workgroup
   const dim3 rows(mgrid.x, (mgrid.y + kRows - 1) / kRows);
-  return launch_kernel(p.f16 ? splitkv_merge_rows_kernel<D, true> : splitkv_merge_rows_kernel<D, false>, rows, dim3(64 * kMergeWaves), stream, p);
+  return launch_kernel(p.f16 ? splitkv_merge_rows_kernel<D, true, true> : splitkv_merge_rows_kernel<D, false, kF32>, rows, dim3(64 * kMergeWaves), stream, p);
 }
 
 // How a shape's column tiles map onto waves: tiles per wave and waves per kv head.

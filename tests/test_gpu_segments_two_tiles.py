@@ -68,3 +68,33 @@ def test_large_launches(gpu, n_q, n_kv, kv, q_len, window, room):
                 weight = torch.softmax((q @ k.t().contiguous() * wl.sm_scale).masked_fill(~seen, float("-inf")), -1)
                 want[b * q_len:(b + 1) * q_len, h * group + e] = (weight @ v).cpu()
     assert_close_bf16(got.cpu(), want.float(), "large launches")
+
+
+# A call gives the same for values of V that IEEE half does not hold whatever its size: below the line the tile kernel takes it, above it segments do
+@pytest.mark.parametrize("kv", [[40000, 25000, 90], [40000, 26000, 90]])
+@pytest.mark.parametrize("scale", [1e5, 1e-6])
+def test_values_beyond_half(gpu, kv, scale):
+    n_q, n_kv, q_len = 16, 4, 6
+    wl = build_workload("range", "prefill", seed=len(kv), n_q=n_q, n_kv=n_kv, head_dim=256, kv_lens=kv, extend_lens=[q_len] * len(kv)).to(gpu)
+    assert (sum(kv) * n_kv * 1024 >= 256 << 20) == (kv[1] == 26000)
+    v = ((1 + 0.1 * wl.v_cache.float()) * scale).bfloat16()
+    not_finite = [(0, 1000, 1, 5, float("inf")), (1, 20000, 2, 250, float("-inf")), (1, 300, 0, 77, float("nan")), (0, 39000, 3, 128, float("nan"))]
+    for b, at, h, dim, value in not_finite:
+        v[int(wl.kv_indices[int(wl.kv_indptr[b]) + at]), h, dim] = value
+    got = paged_prefill_attention(wl.q, wl.k_cache, v, wl.qo_indptr, wl.kv_indptr, wl.kv_indices, wl.prefix_lens, wl.sm_scale, q_len).double().cpu()
+    group, want = n_q // n_kv, torch.empty(wl.q.shape, dtype=torch.float64)
+    for b, n in enumerate(kv):
+        rows = wl.kv_indices[int(wl.kv_indptr[b]):int(wl.kv_indptr[b]) + n].long()
+        seen = torch.arange(n, device=gpu)[None] <= torch.arange(n - q_len, n, device=gpu)[:, None]
+        for h in range(n_kv):
+            k, vals = wl.k_cache[rows, h].double(), v[rows, h].double()
+            for e in range(group):
+                q = wl.q[b * q_len:(b + 1) * q_len, h * group + e].double()
+                weight = torch.softmax((q @ k.t().contiguous() * wl.sm_scale).masked_fill(~seen, float("-inf")), -1)
+                want[b * q_len:(b + 1) * q_len, h * group + e] = (weight @ vals.nan_to_num(0, 0, 0)).cpu()
+        for _, at, h, dim, value in (x for x in not_finite if x[0] == b):
+            want[b * q_len:(b + 1) * q_len, h * group:(h + 1) * group, dim] = value
+    finite = want.isfinite()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    # values of one sign: weights rounded to bf16 and the result, 2^-9 each, and as much again for the exponentials
+    assert ((got - want).abs()[finite] <= 2.0 ** -7 * want.abs()[finite]).all()
