@@ -100,10 +100,10 @@ __device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// Share number `item` of the launch: its request, which of the request's shares it is, of how many.
-// All lanes must call; false past the last share.  The launch's other parameters are fetched while the first requests' lengths are.
+// Share number `item` of the launch: its request, which of the request's shares it is, of how many; a lane's `other`: one of the requests
+// around it.  All lanes must call; false past the last share.  The launch's other parameters are fetched while the first requests' lengths are.
 template <int PARAMETERS>
-__device__ __forceinline__ bool find_share(const ShareStart& p, int item, ReqInfo* r, int* b, int* share, int* n_shares) {
+__device__ __forceinline__ bool find_share(const ShareStart& p, int item, ReqInfo* r, int* b, int* share, int* n_shares, OtherKeys* other) {
   const int lane = lane_id();
   int base = 0;
   for (int b0 = 0; b0 < p.batch; b0 += kWave) {
@@ -132,6 +132,7 @@ __device__ __forceinline__ bool find_share(const ShareStart& p, int item, ReqInf
       *b = b0 + src;
       *share = item - __builtin_amdgcn_readlane(first, src);
       *n_shares = __builtin_amdgcn_readlane(n, src);
+      *other = OtherKeys{mine.kv_start, lane == src || b0 + lane >= p.batch ? 0 : mine.kv_len};
       return true;
     }
     base += sum;
@@ -144,87 +145,42 @@ struct Nothing {
   __device__ __forceinline__ explicit Nothing(const Args&...) {}
 };
 
-// WIDE: a request's columns go to several workgroups, kCols to each.
-template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW, bool WIDE>
-__global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
-    const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
-    int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams sp) {
-  const SplitKvParams& p = sp.s;
-  const ShareShape shape(shape_bits);
-  const ShareStart start{kv_indptr, qo_indptr, prefix_lens, batch, share_len, window, max_len_extend, q_cap, is_cross, len_magic, shape.len_shift()};
+template <int D, int NCT, int NW>
+struct ShareLds {
+  static constexpr int kCols = 16 * NCT;
+  static constexpr int kBlock = kCols * 8 + 8;  // floats of one block of 8 dims: [col][8], padded
+  __attribute__((aligned(16))) float part[NW][D / 8][kBlock];
+  float2 state[NW][kCols];  // (maximum, sum) of a wave's columns
+  int is_last;
+};
+// A wave's place: share `item` of the launch, number `share` of the `n_shares` of request b; its kv head, the number of that in the
+// workgroup and the wave's of the `share_waves` on it; its keys; the request's columns that the workgroup has.
+struct SharePlace {
+  int item, b, share, n_shares, kvh, sub, sw, share_waves, t_begin, t_end, col0, ncols;
+  unsigned long long* cnt;
+  unsigned long long fresh;
+};
+
+// From a share's first slot ids on.  (All of it: a branch around the walk alone costs the kernel 20-40 spilled registers.)
+template <int D, int NCT, int NW, int WALK, bool F16, int NEW, typename NewIds, typename Rows>
+__device__ __forceinline__ void attend_share(const ShareParams& sp, const SplitKvParams& p, ShareLds<D, NCT, NW>& lds, const SharePlace& place, const ReqInfo& r,
+                                             FirstIds& ids, Columns<D, NCT>& c, const NewIds& new_ids, Rows& new_rows) {
   constexpr int VH = D / 128;
-  constexpr int kCols = 16 * NCT;
-  constexpr int kBlock = kCols * 8 + 8;  // floats of one block of 8 dims: [col][8], padded
-  __shared__ __attribute__((aligned(16))) float part[NW][D / 8][kBlock];
-  __shared__ float2 state[NW][kCols];  // (maximum, sum) of a wave's columns
-  __shared__ int is_last;
+  auto& part = lds.part;
+  auto& state = lds.state;
+  auto& is_last = lds.is_last;
+  const int item = place.item, share = place.share, n_shares = place.n_shares, kvh = place.kvh, sub = place.sub, share_waves = place.share_waves;
+  const int t_begin = place.t_begin, t_end = place.t_end, col0 = place.col0, ncols = place.ncols;
+  unsigned long long* const cnt = place.cnt;
+  const unsigned long long fresh = place.fresh;
   const int lane = lane_id();
   const int t16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int item, hg;
-  uint32_t block = blockIdx.x, cg = 0;
-  if (WIDE) {  // the column groups of a share are on one XCD
-    const uint32_t seq = block >> 3, base = seq / shape.col_groups();
-    cg = seq - base * shape.col_groups();
-    block = base * 8 + (block & 7);
-  }
-  if (shape.groups() == ShareShape::kNoShift) {
-    item = block / sp.head_groups;
-    hg = block - item * sp.head_groups;
-  } else {
-    item = block >> shape.groups();
-    hg = block & ((1u << shape.groups()) - 1);
-  }
-  const int col0 = WIDE ? (int)cg * kCols : 0;  // the first of this workgroup's columns
-  const int share_waves = 1 << shape.waves();
-  const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
-  const int sw = wave & (share_waves - 1);
-  const int kvh = hg * (NW >> shape.waves()) + sub;
-
-  ReqInfo r;
-  int b, share, n_shares;
-  constexpr int kParameters = 3 * 8 + 8 * 4 + sizeof(ShareParams);
-  if (!find_share<kParameters>(start, item, &r, &b, &share, &n_shares)) {  // the whole workgroup
-    if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(p, p.nt, p.n_kv * D, threadIdx.x);
-    return;
-  }
-  // From here on, not from the kernel's beginning as elsewhere: the search is not in the interval.  (Stamps at the beginning cost every
-  // launch 0.03 us, with a test of whether there is a probe 0.14.)
-  const ClockProbe clock_probe_(p.clock_probe);
-  // what the rest of the way begins with and only the request's number leads to
-  const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
-  __builtin_amdgcn_sched_barrier(0);
-  const int ncols = WIDE ? min(r.q_len * p.group - col0, kCols) : r.q_len * p.group;
-  if (ncols <= 0) return;
-  Columns<D, NCT> c;
-  // the keys that are walked: all, but for a prefill call's own new ones
-  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, kvh, col0 == 0);
-  int hi = r.hi;
-  if constexpr (NEW == kStoreRows) hi = new_rows.end;
-  const int vis = hi - r.lo;
-  const int per = (ceil_div(vis, n_shares) + 31) & ~31;
-  const int s_begin = min(r.lo + share * per, hi), s_end = min(s_begin + per, hi);
-  const int per_wave = (((per + share_waves - 1) >> shape.waves()) + 31) & ~31;
-  const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
-
-  FirstIds ids{};
-  if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
-  __builtin_amdgcn_sched_barrier(0);
-  unsigned long long* const cnt = sp.counts + ((int64_t)b * sp.head_groups + hg) * (WIDE ? shape.col_groups() : 1) + cg;
-  const unsigned long long fresh = sp.nonce << 16;
-  // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
-  // for it: whoever finds the word not made yet makes it (below).  (The last wave, which has the fewest keys or none.)
-  if (n_shares > 1 && share == 0 && threadIdx.x == 64 * (NW - 1)) {
-    unsigned long long seen = ld_agent(cnt);
-    if ((seen >> 16) != sp.nonce)
-      (void)__hip_atomic_compare_exchange_strong(cnt, &seen, fresh, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-  }
   if constexpr (NEW == kStored) {
     start_columns<D, NCT, true, true>(p, r, kvh, col0 >> 4, t_end, c);
     if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, [] {});
   } else if constexpr (NEW == kStoreRows) {
-    new_rows.owner = new_rows.last_keys && share == n_shares - 1 && sw == share_waves - 1;
+    new_rows.owner = new_rows.last_keys && share == n_shares - 1 && place.sw == share_waves - 1;
     start_columns<D, NCT, true, true>(p, r, kvh, col0 >> 4, new_rows.owner ? r.hi : t_end, c);
     new_rows.check();
     if (t_begin < t_end) attend_keys<D, NCT, WALK, F16, true>(p, r, kvh, t_begin, t_end, ids, c, new_rows);
@@ -232,8 +188,8 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   } else {
     static_assert(sizeof(HeadLds<D>) <= sizeof(part[0]), "a wave's heads have their place in its part of the partials");
     const int tail = r.kv_len - 1;
-    const bool owner = r.kv_len > 0 ? t_begin <= tail && tail < t_end : share == 0 && sw == 0;
-    NewToken<D, NEW == kNormRopeStore, F16> token(p, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), new_ids, b, kvh, owner);
+    const bool owner = r.kv_len > 0 ? t_begin <= tail && tail < t_end : share == 0 && place.sw == 0;
+    NewToken<D, NEW == kNormRopeStore, F16> token(p, r, c, *reinterpret_cast<HeadLds<D>*>(&part[wave][0][0]), new_ids, place.b, kvh, owner);
     if constexpr (D == 128) token.angles();
     int walk_end = t_end;
     if (token.seen) {
@@ -398,6 +354,92 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   else merge(std::integral_constant<int, 16>{});
 }
 
+// WIDE: a request's columns go to several workgroups, kCols to each.
+template <int D, int NCT, int NW, int WALK, bool F16, int NEW, bool WIDE>
+__global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
+    const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
+    int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams params) {
+  const ShareShape shape(shape_bits);
+  const ShareStart start{kv_indptr, qo_indptr, prefix_lens, batch, share_len, window, max_len_extend, q_cap, is_cross, len_magic, shape.len_shift()};
+  constexpr int kCols = 16 * NCT;
+  __shared__ ShareLds<D, NCT, NW> lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int item, hg;
+  uint32_t block = blockIdx.x, cg = 0;
+  if (WIDE) {  // the column groups of a share are on one XCD
+    const uint32_t seq = block >> 3, base = seq / shape.col_groups();
+    cg = seq - base * shape.col_groups();
+    block = base * 8 + (block & 7);
+  }
+  if (shape.groups() == ShareShape::kNoShift) {
+    item = block / params.head_groups;
+    hg = block - item * params.head_groups;
+  } else {
+    item = block >> shape.groups();
+    hg = block & ((1u << shape.groups()) - 1);
+  }
+  const int col0 = WIDE ? (int)cg * kCols : 0;  // the first of this workgroup's columns
+  const int share_waves = 1 << shape.waves();
+  const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
+  const int sw = wave & (share_waves - 1);
+  const int kvh = hg * (NW >> shape.waves()) + sub;
+
+  ReqInfo r;
+  int b, share, n_shares;
+  OtherKeys other;
+  constexpr int kParameters = 3 * 8 + 8 * 4 + sizeof(ShareParams);
+  static_assert((3 * 8 + 8 * 4) % alignof(ShareParams) == 0, "where they are, see below");
+  if (!find_share<kParameters>(start, item, &r, &b, &share, &n_shares, &other)) {  // the whole workgroup
+    if constexpr (NEW == kStoreRows) (void)store_rows_of_no_request<64 * NW>(params.s, params.s.nt, params.s.n_kv * D, threadIdx.x);
+    return;
+  }
+  // The rest of the parameters are read from here on, from lines that find_share() had fetched: loads of theirs in front of the search
+  // would be waited for there (28 layers of four requests 240.3 -> 243.5 us).
+  auto args = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  const ShareParams& sp = *reinterpret_cast<const ShareParams*>((const char*)args + (kParameters - sizeof(ShareParams)));
+  const SplitKvParams& p = sp.s;
+  // From here on, not from the kernel's beginning as elsewhere: the search is not in the interval.  (Stamps at the beginning cost every
+  // launch 0.03 us, with a test of whether there is a probe 0.14.)
+  const ClockProbe clock_probe_(p.clock_probe);
+  // what the rest of the way begins with and only the request's number leads to
+  const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
+  __builtin_amdgcn_sched_barrier(0);
+  const int ncols = WIDE ? min(r.q_len * p.group - col0, kCols) : r.q_len * p.group;
+  if (ncols <= 0) return;
+  Columns<D, NCT> c;
+  // the keys that are walked: all, but for a prefill call's own new ones
+  typename std::conditional<NEW == kStoreRows, NewRows<D, NCT>, Nothing>::type new_rows(p, r, c, kvh, col0 == 0);
+  int hi = r.hi;
+  if constexpr (NEW == kStoreRows) hi = new_rows.end;
+  const int vis = hi - r.lo;
+  const int per = (ceil_div(vis, n_shares) + 31) & ~31;
+  const int s_begin = min(r.lo + share * per, hi), s_end = min(s_begin + per, hi);
+  const int per_wave = (((per + share_waves - 1) >> shape.waves()) + 31) & ~31;
+  const int t_begin = min(s_begin + sw * per_wave, s_end), t_end = min(t_begin + per_wave, s_end);
+
+  FirstIds ids{};
+  if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
+  const typename std::conditional<(WALK & kStream) != 0, OtherSlots, Nothing>::type other_slots(p, other, r, s_begin < s_end ? s_begin : -1);
+  __builtin_amdgcn_sched_barrier(0);
+  unsigned long long* const cnt = sp.counts + ((int64_t)b * sp.head_groups + hg) * (WIDE ? shape.col_groups() : 1) + cg;
+  const unsigned long long fresh = sp.nonce << 16;
+  // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
+  // for it: whoever finds the word not made yet makes it (below).  (The last wave, which has the fewest keys or none.)
+  if (n_shares > 1 && share == 0 && threadIdx.x == 64 * (NW - 1)) {
+    unsigned long long seen = ld_agent(cnt);
+    if ((seen >> 16) != sp.nonce)
+      (void)__hip_atomic_compare_exchange_strong(cnt, &seen, fresh, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const SharePlace place{item, b, share, n_shares, kvh, sub, sw, share_waves, t_begin, t_end, col0, ncols, cnt, fresh};
+  if constexpr (WALK & kStream) {
+    if (other_slots.shared())
+      return attend_share<D, NCT, NW, WALK & kWide, F16, NEW>(sp, p, lds, place, r, ids, c, new_ids, new_rows);
+  }
+  attend_share<D, NCT, NW, WALK, F16, NEW>(sp, p, lds, place, r, ids, c, new_ids, new_rows);
+}
+
 // waves of a workgroup: two per SIMD where a wave fits 256 registers
 int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
 
@@ -413,9 +455,10 @@ int launch_shape(const ShareParams& sp, const SharePlan& plan, unsigned blocks, 
   auto launch = [&](auto f16, auto mode_of) {
     constexpr bool F16 = decltype(f16)::value;
     constexpr int NEW = decltype(mode_of)::value;
-    const auto kernel = sp.s.walk == kStream ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW, WIDE>
-                        : sp.s.walk == kWide ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, WIDE>
-                                             : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, WIDE>;
+    const auto kernel = sp.s.walk == kStream             ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW, WIDE>
+                        : sp.s.walk == (kStream | kWide) ? share_attention_kernel<D, NCT, NW, kStream | kWide, F16, NEW, WIDE>
+                        : sp.s.walk == kWide             ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, WIDE>
+                                                         : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, WIDE>;
     return launch_kernel(kernel, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
                          sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
   };

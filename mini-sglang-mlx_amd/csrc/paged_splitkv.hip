@@ -151,40 +151,25 @@ __device__ __forceinline__ bool locate_segment(const SplitKvParams& p, int seg, 
   return false;
 }
 
-// NCT = tiles of 16 columns per wave, NW = waves per workgroup (launch bound only).  One
-// column tile at head dim 128 fits 256 VGPRs, so two such waves per SIMD can be resident.
-// WALK: how the pool's rows are read.  (With offsets of 32 bits a row's is one multiply instead of a 64-bit multiply-add per load.)
-// NEW: a decode step's rows are stored here (kStore), or are in the pool already (kStored).
-template <int D, int NCT, int NW, Walk WALK, bool F16, int NEW>
-__global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void splitkv_attention_kernel(SplitKvParams p) {
+template <int D, int NCT, int NW>
+struct SegmentLds {
+  __attribute__((aligned(16))) NewRowsLds<D> rows[NW];
+  u32x4_t q[Columns<D, NCT>::kQInLds ? NW : 1][Columns<D, NCT>::kQInts];
+};
+
+// A wave's keys from stream position `vpos` on, in request `cur_b`, whose first key is at position `vs`, to `seg_end`.  (A segment is read in
+// one way: chosen at every request, around the walk alone, 205 us instead of 201 for decode of 64 requests of 1-8 K.)
+template <int D, int NCT, int NW, int WALK, bool F16, int NEW>
+__device__ __forceinline__ void walk_segment(const SplitKvParams& p, SegmentLds<D, NCT, NW>& lds, int seg, int seg_len, int cur_b, int vs, int vpos,
+                                             int seg_end) {
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
-  const ClockProbe clock_probe_(p.clock_probe);
   const int lane = lane_id();
   const int t16 = lane & 15;
   const int g = lane >> 4;
-
-  const int seg = blockIdx.x / p.head_groups;
   const int wave = threadIdx.x >> 6;
   const int cw = wave / p.nwh;  // which share of the columns this wave owns
   const int ct0 = cw * NCT;     // first of its tiles of 16 columns
   const int kvh = (blockIdx.x - seg * p.head_groups) * p.nwh + (wave - cw * p.nwh);
-  int seg_len, total, cur_b, vs;
-  __shared__ __attribute__((aligned(16))) NewRowsLds<D> rows[NW];
-  __shared__ u32x4_t q_rows[Columns<D, NCT>::kQInLds ? NW : 1][Columns<D, NCT>::kQInts];
-  if (NEW != kStored && seg == 0) {  // requests without keys come up in no segment
-    for (int b0 = 0; b0 < p.batch; b0 += kWave) {
-      const int b = min(b0 + lane, p.batch - 1);
-      unsigned long long empty = __ballot(b0 + lane < p.batch && p.kv_indptr[b + 1] <= p.kv_indptr[b]);
-      for (; empty != 0; empty &= empty - 1)
-        store_new_rows<D>(p, __builtin_amdgcn_readfirstlane(b0 + __ffsll((long long)empty) - 1), kvh);
-    }
-  }
-  if (!locate_segment(p, seg, &seg_len, &total, &cur_b, &vs)) return;
-  cur_b = __builtin_amdgcn_readfirstlane(cur_b);
-  vs = __builtin_amdgcn_readfirstlane(vs);
-  int vpos = seg * seg_len;
-  const int seg_end = min(vpos + seg_len, total);
-
   while (vpos < seg_end && cur_b < p.batch) {
     const ReqInfo r = request_info(p, cur_b);
     const int vlen = r.hi - r.lo;
@@ -206,13 +191,13 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
     const int ncols = r.q_len * p.group;
 
     Columns<D, NCT> c_;
-    if constexpr (Columns<D, NCT>::kQInLds) c_.q = MSGL_LDS_PTR(u32x4_t, &q_rows[wave][0]) + lane;
+    if constexpr (Columns<D, NCT>::kQInLds) c_.q = MSGL_LDS_PTR(u32x4_t, &lds.q[wave][0]) + lane;
     FirstIds ids = first_ids(p, r, t_begin, t_end);
     if constexpr (NEW == kStored) {
       start_columns(p, r, kvh, ct0, t_end, c_);
       attend_keys<D, NCT, WALK, F16, false>(p, r, kvh, t_begin, t_end, ids, c_, [] {});
     } else {
-      LateToken<D, F16> token(p, r, rows[wave], cur_b, kvh, t_end == r.hi);
+      LateToken<D, F16> token(p, r, lds.rows[wave], cur_b, kvh, t_end == r.hi);
       const int walk_end = token.seen ? t_end - 1 : t_end;
       if (token.seen) end_ids(ids, t_begin, walk_end, token.before);
       start_columns(p, r, kvh, ct0, walk_end, c_);
@@ -280,6 +265,59 @@ __global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void spl
 
     vpos += t_end - t_begin;  // the request's end, or the segment's: the loop head sorts it out
   }
+}
+
+// Whether the segment [vpos, seg_end), which begins in request `b`, has keys that other requests have as well (OtherSlots): its first key, or
+// the first of the next request, if that begins in it.  All lanes must call.
+__device__ __forceinline__ bool shares_keys(const SplitKvParams& p, int b, int vs, int vpos, int seg_end) {
+  const int last = p.batch - 1, next_b = min(b + 1, last);
+  auto others = [&](int request) {
+    const int i = min((request & ~(kWave - 1)) + lane_id(), last);
+    const int start = p.kv_indptr[i], end = p.kv_indptr[i + 1];
+    return OtherKeys{start, i == request ? 0 : end - start};
+  };
+  const OtherKeys others_b = others(b), others_next = others(next_b);
+  __builtin_amdgcn_sched_barrier(0);
+  const ReqInfo r = request_info(p, b), next = request_info(p, next_b);
+  const int vlen = r.hi - r.lo;
+  const bool next_begins = b < last && vs + stream_length(p, vlen) < seg_end && next.hi > next.lo;
+  const OtherSlots first(p, others_b, r, vpos < vs + vlen ? r.lo + (vpos - vs) : -1), of_next(p, others_next, next, next_begins ? next.lo : -1);
+  return __ballot(first.same() || of_next.same()) != 0;
+}
+
+// NCT = tiles of 16 columns per wave, NW = waves per workgroup (launch bound only).  One
+// column tile at head dim 128 fits 256 VGPRs, so two such waves per SIMD can be resident.
+// WALK: how the pool's rows are read.  (With offsets of 32 bits a row's is one multiply instead of a 64-bit multiply-add per load.)
+// NEW: a decode step's rows are stored here (kStore), or are in the pool already (kStored).
+template <int D, int NCT, int NW, int WALK, bool F16, int NEW>
+__global__ __launch_bounds__(64 * NW, ((D == 128 && NCT == 1) ? 2 : 1)) void splitkv_attention_kernel(SplitKvParams p) {
+  const ClockProbe clock_probe_(p.clock_probe);
+  const int lane = lane_id();
+  const int seg = blockIdx.x / p.head_groups;
+  const int wave = threadIdx.x >> 6;
+  const int cw = wave / p.nwh;  // which share of the columns this wave owns
+  const int kvh = (blockIdx.x - seg * p.head_groups) * p.nwh + (wave - cw * p.nwh);
+  int seg_len, total, cur_b, vs;
+  __shared__ SegmentLds<D, NCT, NW> lds;
+  if (NEW != kStored && seg == 0) {  // requests without keys come up in no segment
+    for (int b0 = 0; b0 < p.batch; b0 += kWave) {
+      const int b = min(b0 + lane, p.batch - 1);
+      unsigned long long empty = __ballot(b0 + lane < p.batch && p.kv_indptr[b + 1] <= p.kv_indptr[b]);
+      for (; empty != 0; empty &= empty - 1)
+        store_new_rows<D>(p, __builtin_amdgcn_readfirstlane(b0 + __ffsll((long long)empty) - 1), kvh);
+    }
+  }
+  if (!locate_segment(p, seg, &seg_len, &total, &cur_b, &vs)) return;
+  cur_b = __builtin_amdgcn_readfirstlane(cur_b);
+  vs = __builtin_amdgcn_readfirstlane(vs);
+  int vpos = seg * seg_len;
+  const int seg_end = min(vpos + seg_len, total);
+
+  if constexpr (WALK & kStream) {
+    if (shares_keys(p, cur_b, vs, vpos, seg_end))
+      return walk_segment<D, NCT, NW, WALK & kWide, F16, NEW>(p, lds, seg, seg_len, cur_b, vs, vpos, seg_end);
+  }
+  walk_segment<D, NCT, NW, WALK, F16, NEW>(p, lds, seg, seg_len, cur_b, vs, vpos, seg_end);
 }
 
 // One workgroup of four waves per (request, query, q head), for few rows cut into many segments: merge the partials
@@ -557,9 +595,10 @@ int launch_attn(const SplitKvParams& p, hipStream_t stream) {
   auto launch = [&](auto f16, auto mode) {
     constexpr bool F16 = decltype(f16)::value;
     constexpr int NEW = decltype(mode)::value;
-    const auto kernel = p.walk == kStream ? splitkv_attention_kernel<D, NCT, NW, kStream, F16, NEW>
-                        : p.walk == kWide ? splitkv_attention_kernel<D, NCT, NW, kWide, F16, NEW>
-                                          : splitkv_attention_kernel<D, NCT, NW, kNarrow, F16, NEW>;
+    const auto kernel = p.walk == kStream             ? splitkv_attention_kernel<D, NCT, NW, kStream, F16, NEW>
+                        : p.walk == (kStream | kWide) ? splitkv_attention_kernel<D, NCT, NW, kStream | kWide, F16, NEW>
+                        : p.walk == kWide             ? splitkv_attention_kernel<D, NCT, NW, kWide, F16, NEW>
+                                                      : splitkv_attention_kernel<D, NCT, NW, kNarrow, F16, NEW>;
     return launch_kernel(kernel, dim3((unsigned)(p.n_seg * p.head_groups)), dim3(64 * NW), stream, p);
   };
   if constexpr (NCT == 1) {  // IEEE half and new tokens exist for decode only (one column tile)
@@ -769,7 +808,7 @@ void fill_splitkv_params(const SplitKvArgs& a, SplitKvParams& p) {
   const uint64_t pool_bytes = (uint64_t)a.num_slots * (uint64_t)std::max(a.k_stride0, a.v_stride0) * 2u;
   const int64_t keys = visible_keys(a.batch, a.total_kv, a.window, a.max_len_extend, a.is_cross != 0);
   const bool once = col_split(nct_for(p.cols), a.head_dim, a.total_kv, a.n_kv).col_waves == 1;
-  p.walk = once && streams(keys * a.n_kv * a.head_dim * 4) ? kStream : pool_bytes >= (1ull << 32) ? kWide : kNarrow;
+  p.walk = (once && streams(keys * a.n_kv * a.head_dim * 4) ? kStream : kNarrow) | (pool_bytes >= (1ull << 32) ? kWide : kNarrow);
 }
 
 int launch_splitkv(const SplitKvArgs& a, const NewTokens& n, hipStream_t stream) {

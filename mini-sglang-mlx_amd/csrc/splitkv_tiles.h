@@ -7,8 +7,8 @@
 
 namespace msgl {
 
-// How the pool's rows are read: with offsets of 32 bits; of 64 (a pool of 4 GiB or more); past the caches (streams() in
-// paged_splitkv.hip), with offsets of 64 whatever the pool.
+// How the pool's rows are read: with offsets of 32 bits, or kWide of 64 (a pool of 4 GiB or more); kStream: past the caches (streams() in
+// paged_splitkv.hip), but those of keys that another request has as well (OtherSlots).
 enum Walk { kNarrow = 0, kWide = 1, kStream = 2 };
 
 struct SplitKvParams {
@@ -198,6 +198,28 @@ __device__ __forceinline__ FirstIds first_ids(const SplitKvParams& p, const ReqI
   return FirstIds{{idx[min(at, last)], idx[min(at + 16, last)]}, {idx[min(at + 32, last)], idx[min(at + 48, last)]}};
 }
 
+// Requests with a common prefix have its keys in the same slots, and each finds in the caches what another has read.  Plain loads get
+// 9-10 TB/s then, loads past the caches the 7 they always get: decode of 64 requests of 256 keys behind 4096 in common, 32 / 8 heads, 117.7 us
+// and 165.0, of 128 of 512 behind 1024 96 and 118, verify of 32 x 8 of 512 behind 4096 78 and 94, shares of 5 of 1024 behind 16 K, 16 / 2 heads of
+// 256, 32.1 and 34.8.  So a segment or share whose first key another request has in the same slot is read plainly.  Of the requests the 64 around
+// its own are looked at, one to a lane.  With nothing in common decode of 64 requests of 1-8 K 200.3 -> 201.5, 24 of 127-4095, 16 / 2 heads of 256, 24.3 -> 24.5.
+struct OtherKeys {  // of one of those requests; those of the request itself as none
+  int start, len;
+};
+struct OtherSlots {
+  bool has;
+  int slot, own;
+  // `at`: a key of request `r`, -1: none
+  __device__ __forceinline__ OtherSlots(const SplitKvParams& p, const OtherKeys& other, const ReqInfo& r, int at) {
+    has = at >= 0 && at < other.len;
+    const int own_at = at >= 0 ? r.kv_start + at : 0;
+    slot = p.kv_indices[has ? other.start + at : own_at];
+    own = p.kv_indices[own_at];
+  }
+  __device__ __forceinline__ bool same() const { return has && slot == own; }
+  __device__ __forceinline__ bool shared() const { return __ballot(same()) != 0; }  // all lanes must call
+};
+
 // A tile whose K rows came by whole lines (attend_keys): of the 16 rows of a sub-tile, lanes of t16 < 8 have even pieces of 64 bytes, of
 // row t16 in slice 2 c and of row t16 + 8 in slice 2 c + 1, the others odd ones, of row t16 - 8 and of row t16.  Lane t16 gives
 // lane t16 +- 8 what is of its row.
@@ -347,12 +369,12 @@ __device__ __forceinline__ void compute_tile(const SplitKvParams& p, const KvTil
 // caches, at head_dim 256 1.0-1.3x.
 // meanwhile(): called once the first tile has been asked for; may finish the columns' Q operand and put keys of its own
 // into their state.
-template <int D, int NCT, Walk WALK, bool F16, bool SHORT, typename Meanwhile>
+template <int D, int NCT, int WALK, bool F16, bool SHORT, typename Meanwhile>
 __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInfo& r, int kvh, int t_begin,
                                             int t_end, const FirstIds& first, Columns<D, NCT>& c_, Meanwhile&& meanwhile) {
   constexpr int KS = D / 32;   // k-steps of the QK product
   constexpr int VH = D / 128;  // 128-wide halves of D in the PV product
-  constexpr bool LINES = WALK == kStream && !SHORT;
+  constexpr bool LINES = (WALK & kStream) && !SHORT;
   const int lane = lane_id();
   const int t16 = lane & 15;
   const int g = lane >> 4;
@@ -367,7 +389,7 @@ __device__ __forceinline__ void attend_keys(const SplitKvParams& p, const ReqInf
     else return (uint64_t)((uint32_t)slot_id * row_bytes);
   };
   auto load = [](const unsigned char* from) {
-    if constexpr (WALK == kStream) return ld_stream_b128(from);
+    if constexpr (WALK & kStream) return ld_stream_b128(from);
     else return ld_global_b128(from);
   };
   const int32_t* idx_base = p.kv_indices + r.kv_start;

@@ -103,3 +103,56 @@ def test_beyond_the_line(gpu, d):
     print(f"stream beyond the line d{d}", flush=True)
     diff = (paged_decode_attention(g.q, g.k_cache, g.v_cache, g.kv_indptr, g.kv_indices, g.num_kv_splits, g.sm_scale, 32).float().cpu() - want).abs()
     assert float(diff.max()) <= 2e-2 and float(diff.mean()) <= 2e-3  # as for the plain way
+
+
+def _common_prefix(gpu, batch, common, own, heads, d, ext, dtype=torch.bfloat16):
+    """Requests whose first `common` keys are in the same slots, and the rest in slots of their own."""
+    n_q, n_kv = heads
+    g = torch.Generator(device=gpu)
+    g.manual_seed(batch + common)
+    slots = torch.randperm(common + own * batch, generator=g, device=gpu).int()
+    idx = torch.cat([torch.cat([slots[:common], slots[common + b * own:common + (b + 1) * own]]) for b in range(batch)])
+    rand = lambda *s: torch.randn(s, generator=g, device=gpu).to(dtype)  # noqa: E731
+    kc, vc, q = rand(slots.numel(), n_kv, d), rand(slots.numel(), n_kv, d), rand(batch * ext, n_q, d)
+    indptr = torch.arange(batch + 1, dtype=torch.int32, device=gpu) * (common + own)
+    if ext == 1:
+        splits = torch.ones(batch, dtype=torch.int32, device=gpu)
+        return lambda: paged_decode_attention(q, kc, vc, indptr, idx, splits, d ** -0.5, 32)
+    qo = torch.arange(batch + 1, dtype=torch.int32, device=gpu) * ext
+    prefix = torch.full((batch,), common + own - ext, dtype=torch.int32, device=gpu)
+    return lambda: paged_prefill_attention(q, kc, vc, qo, indptr, idx, prefix, d ** -0.5, ext)
+
+
+# no keys of a request's own before the first tile, in the middle of one, and none but its own behind the first; more requests than lanes
+@pytest.mark.parametrize("batch,common,own", [(1, 100, 30), (2, 64, 40), (5, 1000, 33), (3, 1, 700), (70, 90, 17), (130, 40, 9)])
+@pytest.mark.parametrize("heads,d,ext", [((16, 8), 128, 1), ((32, 8), 128, 8), ((8, 1), 256, 1), ((16, 4), 256, 6)])
+@pytest.mark.parametrize("shares", [-1, 64 | 1 << 20])
+def test_common_prefixes(gpu, tuning, batch, common, own, heads, d, ext, shares):
+    tuning(_lib.TUNE_SHARES, shares)
+    if d == 256 and ext > 1 and shares < 0:
+        tuning(_lib.TUNE_SMALLQ_MAXCOLS, 64)
+    print(f"common prefix {batch} x {common} + {own} {heads} d{d} x {ext} shares {shares}", flush=True)
+    plain, stream = _both(tuning, _common_prefix(gpu, batch, common, own, heads, d, ext))
+    assert bool(plain.isfinite().all()) and _same(plain, stream)
+
+
+def test_common_prefixes_come_from_the_caches(gpu, tuning):
+    """What one request has read, the others find: 80 MiB in all, of which 64 requests read 1088.  (Past the caches 1.3-1.4 times the time.)"""
+    launch = _common_prefix(gpu, 64, 4096, 256, (32, 8), 128, 1)
+
+    def us():
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(20):
+            launch()
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) * 50
+
+    times = {-1: [], 0: []}
+    for _ in range(5):
+        for kib in times:
+            tuning(_lib.TUNE_STREAM, kib)
+            launch()
+            times[kib].append(us())
+    assert min(times[0]) <= 1.15 * min(times[-1]), times
