@@ -215,6 +215,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
     v_chunk += kShortChunk * (int64_t)v_step;
   };
   fetch_group(0);
+  float* srow = nullptr;  // (by whole lines it is found anew behind the chunks: kept it is two more spilled registers, and 3-8 % of the time)
   f32x4_t s[8];  // s[2 c + h][i]: dim 32 c + 8 g + 4 h + i of row lane % 16
   if constexpr (LINES) {
     const float* const from = state_lines(slot, hv, row);
@@ -222,9 +223,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
     for (int c = 0; c < 8; ++c) s[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(from + line_at(c)));
     exchange_lines(s);
   } else {
-    const float* const from = state_row(slot, hv, row);
+    srow = state_row(slot, hv, row);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(from + 32 * (c >> 1) + 4 * (c & 1));
+    for (int c = 0; c < 8; ++c) s[c] = *reinterpret_cast<const f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1));
   }
   load_v(start);
   const Picker pick;
@@ -337,9 +338,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 2) void gdn_short_kernel(GdnPar
 #pragma unroll
     for (int c = 0; c < 8; ++c) __builtin_nontemporal_store(s[c], reinterpret_cast<f32x4_t*>(to + line_at(c)));
   } else {
-    float* const to = state_row(slot, hv, row);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(to + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
+    for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4_t*>(srow + 32 * (c >> 1) + 4 * (c & 1)) = s[c];
   }
 }
 
