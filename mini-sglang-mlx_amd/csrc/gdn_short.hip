@@ -351,13 +351,17 @@ int launch_gdn_short(const GdnParams& p, hipStream_t stream) {
   // Half a head to a workgroup while that leaves one to a compute unit, or two and there is one chunk (8 requests of 32 heads: 16 tokens
   // 10.4 us and 10.8 by whole heads, 32 tokens 12.9 and 11.7).
   const bool halves = 2 * heads <= device_cus() || (heads <= device_cus() && p.tokens <= kShortChunk * (int64_t)p.batch);
-  // Whole lines past the caches from four requests of 32 heads on.  us, plain and that, by requests: of 4-16 tokens 4 7.0-7.3 and 6.9-7.1, 8 10.6-11.1
-  // and 8.9-9.1, 16 15.2-16.1 and 13.4-14.3, 24 23.6-24.5 and 22.5-23.1, 64 60.2-63.8 and 56.7-59.2; of 32 tokens 8 12.3 and 11.5, 48 56.9 and 49.9,
-  // 100 108 and 99; of 48 16 22.2 and 21.9, 64 83.2 and 79.5, but 24 30.9 and 31.8, 100 121 and 127.  One and two requests find their state in the caches
-  // when it is asked for again: 5.0-8.0 and 0.3-0.8 more.
-  if (heads < 128) return launch_kernel(gdn_short_kernel<4, false>, dim3((unsigned)(2 * heads)), dim3(256), stream, p);
-  return halves ? launch_kernel(gdn_short_kernel<4, true>, dim3((unsigned)(2 * heads)), dim3(256), stream, p)
-                : launch_kernel(gdn_short_kernel<8, true>, dim3((unsigned)heads), dim3(512), stream, p);
+  // Whole lines past the caches from four requests of 32 heads on in one chunk, from eight beyond, but for 20 to 39 requests of more than 32
+  // tokens: what the states of that many leave in the last level the next pass finds there, and the chunks' chain hides the rest.  That by
+  // plain, three sets of states in turn (twelve, as the layers of a model), by requests, of up to 16 tokens, 17-32 and 33-48: 4 0.98-1.01 (0.97),
+  // 1.04 (1.02), 1.06 (1.07); 6 0.94-0.97 (0.95), 0.99 (1.01), 1.01 (1.02); 8 0.88 (0.90), 0.95 (0.95), 0.97 (0.97); 16 0.87 (0.72), 0.95 (0.87),
+  // 0.97 (0.92); 24 0.93 (0.83), 1.01 (0.90), 1.06 (0.98); 32 0.93 (0.82), 1.00 (0.87), 1.08 (0.98); 40 0.97 (0.89), 0.98 (0.89), 1.00 (0.99);
+  // 64 0.96 (0.96), 0.93 (0.91), 0.97 (0.97); 100 0.95 (0.95), 0.93 (0.93), 0.93 (0.95).  One to three find their state in the caches.
+  const bool one_chunk = p.tokens <= kShortChunk * (int64_t)p.batch, long_chain = p.tokens > 32 * (int64_t)p.batch;
+  const bool lines = heads >= (one_chunk ? 128 : 256) && !(long_chain && heads >= 640 && heads < 1280);
+  if (halves)
+    return launch_kernel(lines ? gdn_short_kernel<4, true> : gdn_short_kernel<4, false>, dim3((unsigned)(2 * heads)), dim3(256), stream, p);
+  return launch_kernel(lines ? gdn_short_kernel<8, true> : gdn_short_kernel<8, false>, dim3((unsigned)heads), dim3(512), stream, p);
 }
 
 }  // namespace msgl

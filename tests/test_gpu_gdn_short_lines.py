@@ -1,5 +1,5 @@
-"""Requests in chunks of 16 tokens on both sides of the number of heads from which their state comes and goes by whole lines: half a head to
-a workgroup and a whole one, against the float64 oracle; a request that is not finite among them is gone through again."""
+"""Requests in chunks of 16 tokens on both sides of the numbers of heads and tokens between which their state comes and goes by whole lines:
+half a head to a workgroup and a whole one, against the float64 oracle; a request that is not finite among them is gone through again."""
 import numpy as np
 import pytest
 
@@ -8,7 +8,9 @@ from test_gpu_gdn_short import _run, _same_places
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("lengths,hk,hv", [([4] * 127, 1, 1), ([4] * 128, 1, 1), ([17, 4, 33, 9], 4, 32), ([16] * 8, 16, 32), ([17] + [16] * 8, 8, 32)])
+@pytest.mark.parametrize("lengths,hk,hv", [([4] * 127, 1, 1), ([4] * 128, 1, 1), ([17, 4, 33, 9], 4, 32), ([16] * 8, 16, 32), ([17] + [16] * 8, 8, 32),
+                                           ([17] * 7, 16, 32), ([17] * 8, 16, 32), ([33] * 19, 16, 32), ([33] * 20, 16, 32), ([32] * 20, 16, 32),
+                                           ([33] * 40, 16, 32)])
 def test_against_the_oracle(gpu, lengths, hk, hv):
     (y, state), (want_y, want_state), before, slots = _run(gpu, lengths, hk, hv, "some", len(lengths) + hv)
     # bounds as for the rest of the kernel: fp32 arithmetic in the state, y rounded to bf16 once
