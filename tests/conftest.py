@@ -1,4 +1,5 @@
 import os
+import re
 import sys
 
 import pytest
@@ -22,7 +23,13 @@ def gpu():
     return torch.device("cuda:0")
 
 
-_KNOBS = range(11)  # MSGL_TUNE_* of include/msgl_paged_attention.h
+def _knobs():
+    """The numbers of the MSGL_TUNE_* switches."""
+    with open(os.path.join(ROOT, "include", "msgl_paged_attention.h")) as header:
+        return [int(n) for n in re.findall(r"^#define MSGL_TUNE_\w+ (\d+)$", header.read(), re.M)]
+
+
+_KNOBS = _knobs()
 
 
 def _reset_knobs():

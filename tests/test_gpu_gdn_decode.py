@@ -9,12 +9,6 @@ from mini_sglang_amd_kernel import _lib, gdn_state_inplace
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True)
-def _knob_back():
-    yield
-    _lib.set_tuning(_lib.TUNE_STREAM, 0)
-
-
 @pytest.mark.parametrize("batch,hk,hv", [(1, 1, 1), (3, 2, 6), (6, 16, 32), (7, 16, 32), (12, 16, 32), (13, 16, 32), (47, 16, 32), (48, 16, 32), (96, 16, 16)])
 def test_all_ways_are_one(gpu, tuning, batch, hk, hv):
     g = torch.Generator(device=gpu)

@@ -11,12 +11,6 @@ from mini_sglang_amd_kernel import _lib, decode_step, paged_decode_attention, pa
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True)
-def _knob_back():
-    yield
-    _lib.set_tuning(_lib.TUNE_STREAM, 0)
-
-
 def _both(tuning, launch):
     out = []
     for kib in (-1, 1):

@@ -358,3 +358,22 @@ def test_tuning_knobs_are_per_host_thread():
     out = __import__("ctypes").c_int64(5)
     assert lib.msgl_get_tuning(99, __import__("ctypes").byref(out)) == -9
     assert lib.msgl_get_tuning(0, None) == -1
+
+
+def test_every_knob_goes_back_between_tests():
+    import conftest
+    from mini_sglang_amd_kernel import _lib
+
+    header = open(os.path.join(ROOT, "include", "msgl_paged_attention.h")).read()
+    knobs = [int(n) for n in re.findall(r"#define MSGL_TUNE_\w+ (\d+)", header)]
+    assert len(knobs) == 12 and sorted(knobs) == list(range(12))
+    try:
+        for knob in knobs:
+            _lib.set_tuning(knob, 1)
+        assert all(_lib.get_tuning(knob) == 1 for knob in knobs)
+    finally:
+        conftest._reset_knobs()
+        left = [knob for knob in knobs if _lib.get_tuning(knob) != 0]
+        for knob in left:
+            _lib.set_tuning(knob, 0)
+    assert left == []
