@@ -425,7 +425,8 @@ MSGL_API int msgl_gdn_state_inplace_longest(const void* q, const void* k, const 
  *                            equal segments and a merge: negative: never; 0: chosen from the sizes;
  *                            positive: always, with share_len | kv heads per workgroup << 20
  *   MSGL_TUNE_STREAM         from how many KiB of keys and values on decode and verify read them past the
- *                            caches (0: default, negative: never); the results are the same bits
+ *                            caches (0: default, negative: never), and of state on the gated delta rule with
+ *                            one token a request reads and writes it so; the results are the same bits
  */
 #define MSGL_TUNE_SEGMENTS 0
 #define MSGL_TUNE_MIN_SEGMENT 1

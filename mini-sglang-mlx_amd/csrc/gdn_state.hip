@@ -259,7 +259,7 @@ int launch_gdn_state(const GdnArgs& a, hipStream_t stream) {
   // (With twelve sets 28 MiB 14.5, 13.6, 14.5 / 14.7, 12.4, 12.8, 64 MiB 28.9, 27.9, 29.0 / 28.5, 24.9, 25.3.)
   const int64_t state_bytes = heads * kDV * kDK * (int64_t)sizeof(float);
   const bool large = streams(state_bytes, 96 << 10);
-  const bool stream_state = p.single_token && (large || state_bytes <= (24 << 20));
+  const bool stream_state = p.single_token && (large || (state_bytes <= (24 << 20) && streams(state_bytes, 0)));
   if (p.single_token) r = large || heads <= 192 ? 2 : 4;
   if (t_force_rows > 0) r = t_force_rows;
   const int64_t blocks = heads * (kDV / (16 * r));
