@@ -44,13 +44,18 @@ STORES = [  # cached, new tokens, n_q, n_kv, head_dim
 
 
 @pytest.mark.parametrize("cached,ext,n_q,n_kv,d", STORES)
-@pytest.mark.parametrize("cross,window", [(False, 0), (True, 0), (False, 100)])
+# share 0: the plan that such a call has, a workgroup to each tile of columns; else two tiles to one at head_dim 128
+@pytest.mark.parametrize("share,cross,window", [(0, False, 0), (0, True, 0), (0, False, 600)] +
+                         [(s, *m) for s in (64, 96) for m in ((False, 0), (True, 0), (False, 100))])
 @pytest.mark.parametrize("places", ["last", "mixed"])
-@pytest.mark.parametrize("share", [0, 64])
-def test_one_launch_is_two(gpu, tuning, cached, ext, n_q, n_kv, d, cross, window, places, share):
-    if places == "last" and not cross and window == 0:
-        assert _lib.load().msgl_extend_step_workspace_bytes(len(ext), sum(ext), sum(ext) + sum(cached), n_q, n_kv, d, max(ext), 0, 0) > 0
-    shares_only = lambda knob, value: tuning(knob, value) if knob == _lib.TUNE_SHARES else None  # noqa: E731
+def test_one_launch_is_two(gpu, tuning, cached, ext, n_q, n_kv, d, share, cross, window, places):
+    batch, keys, tiles = len(ext), sum(ext) + sum(cached), -(-max(ext) * n_q // n_kv // 16)
+    if share == 0:
+        if window:
+            keys = min(keys, batch * (window + max(ext) + 15))
+        assert keys > 192 * batch and keys * n_kv * tiles <= (400 if d == 256 else 512) * 256 and 4 * batch * n_kv <= 3 * (256 // (8 * tiles) * 8)
+        assert _lib.load().msgl_extend_step_workspace_bytes(batch, sum(ext), sum(ext) + sum(cached), n_q, n_kv, d, max(ext), int(cross), window) > 0
+    shares_only = lambda knob, value: tuning(knob, value) if share and knob == _lib.TUNE_SHARES else None  # noqa: E731
     _one_launch_is_two(gpu, shares_only, cached, ext, n_q, n_kv, d, share, 0, cross, window, places)
 
 
