@@ -498,20 +498,32 @@ static bool heads_alone(int64_t batch, int64_t n_kv) { return batch * n_kv <= de
 // fits with at most 16 shares to a request, from 256 on, and segments for fewer than 12 pairs: 16 and 11 %.
 // The same costs hold at head_dim 128: 12 700 launches of up to 25 pairs within 0.3-3 % of the best, where the shortest that fits with at most 16
 // shares to a request was 1-3 % from 12 pairs on, 3-44 % for 4 to 11 and up to 2x for fewer.
+// Every decode step makes it twice, 28 layers of a step that the host's side bounds: the search is without divisions and ends where a length's own
+// keys cost as much as the best.  A plan, eight kv heads of 128, by all lengths in floating point and by this, ns: one request of 2000 keys 52
+// and 26, four of 300 34 and 22, eight of 1000 42 and 23, two of 20 K 64 and 27; two kv heads of 256, 24 of 2000, 49 and 29.
 static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int64_t cols, int64_t least, int64_t round) {
-  const double slots = (double)round, mean = (double)(keys / batch), spread = 0.43 * std::sqrt((double)batch);
-  int64_t len = 0;
-  double lowest = 0;
-  for (int64_t c = least; c < (1 << 20); c = (c & (c - 1)) ? c / 3 * 4 : c / 2 * 3) {
-    const double of_one = std::max(std::ceil(mean / (double)c), 1.0);
-    const double shares = std::max({(double)batch, (double)keys / (double)c + 0.5 * (double)batch + spread, (double)batch * of_one});
-    if (shares * (double)n_kv > slots) continue;
-    const double cost = std::min((double)c, 1.5 * mean) + (of_one > 1 ? (cols > 8 ? 160 : 100) : 0) + 4 * of_one + 100 * (std::ceil(of_one / 16) - 1);
-    if (len == 0 || cost < lowest) {
-      len = c;
-      lowest = cost;
+  // in a round beside half a share a request for the rounding and two standard deviations of that
+  const double room = (double)round / (double)n_kv - 0.5 * (double)batch - 0.43 * std::sqrt((double)batch);
+  const int64_t mean = keys / batch, most = round / (batch * n_kv);  // keys, and shares that fit the round, of a request of that length
+  const int64_t put_together = cols > 8 ? 320 : 200;  // costs are in halves of a key
+  bool thirds = (least & (least - 1)) != 0;  // a length is 2^shift or 3 2^shift
+  int shift = 63 - __builtin_clzll((uint64_t)(thirds ? least / 3 : least));
+  int64_t len = 0, lowest = 0;
+  for (int64_t c = least; c < (1 << 20); c = (int64_t)(thirds ? 3 : 1) << shift) {
+    const uint64_t up = (uint64_t)(mean + c - 1) >> shift;
+    const int64_t of_one = std::max<int64_t>((int64_t)(thirds ? up / 3 : up), 1);
+    if (of_one <= most && (double)keys <= (double)c * room) {
+      const int64_t alone = std::min(2 * c, 3 * mean);
+      if (len != 0 && alone + 8 >= lowest) break;
+      const int64_t cost = alone + (of_one > 1 ? put_together : 0) + 8 * of_one + 200 * ((of_one + 15) / 16 - 1);
+      if (len == 0 || cost < lowest) {
+        len = c;
+        lowest = cost;
+      }
+      if (c >= 2 * mean) break;
     }
-    if ((double)c >= 2 * mean) break;
+    shift += thirds ? 2 : -1;
+    thirds = !thirds;
   }
   return len > 0 ? len : 1 << 20;
 }
@@ -580,16 +592,16 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
     // and take 12.5 us, without it 128, a few workgroups more than compute units, and 16.6
     const bool alone = col_groups > 1 || heads_alone(batch, n_kv);
     len = nct == 3 ? 512 : (nw == 4 && heads == 1 && !(head_dim == 256 && alone)) ? 256 : 128;
-    const int64_t spread = (int64_t)std::sqrt((double)batch / 3);
-    auto fits = [&](int64_t c) {
-      return std::max(batch, keys / c + batch / 2 + spread) * (n_kv / heads) <= slots && keys <= 16 * c * batch;
-    };
     if (each > 0) {  // one length for all: as many equal shares as fit
       const int64_t n = std::min<int64_t>(std::max<int64_t>(slots * heads / (batch * n_kv), 1), 16);
       len = std::max(len, ((each + n - 1) / n + 31) & ~(int64_t)31);
     } else if (alone) {
       len = cost_share_length(batch, keys, n_kv, std::min<int64_t>(cols, 16 * nct), len, slots);
     } else {
+      const int64_t spread = (int64_t)std::sqrt((double)batch / 3);
+      auto fits = [&](int64_t c) {
+        return std::max(batch, keys / c + batch / 2 + spread) * (n_kv / heads) <= slots && keys <= 16 * c * batch;
+      };
       while (!fits(len) && len < (1 << 19)) len = (len & (len - 1)) ? len / 3 * 4 : len / 2 * 3;
     }
   }
@@ -597,8 +609,10 @@ SharePlan share_plan(int64_t batch, int64_t keys, int64_t each, int64_t n_kv, in
   // (128 MiB and some hundred shares), whatever the requests' number: under a window a request is one share, or a few.  One set
   // by hand is raised to what does.
   const int64_t visible = each > 0 ? each : keys, row_bytes = n_kv * cols * head_dim * 4;
-  const int64_t most_of_one = std::min<int64_t>(std::max<int64_t>(0x7fffffffLL / row_bytes, 1), 0xffff);
-  len = std::max(len, (visible + most_of_one - 1) / most_of_one);
+  if (visible > 0xffff || visible * row_bytes > 0x7fffffffLL) {  // (else shares of one key would)
+    const int64_t most_of_one = std::min<int64_t>(std::max<int64_t>(0x7fffffffLL / row_bytes, 1), 0xffff);
+    len = std::max(len, (visible + most_of_one - 1) / most_of_one);
+  }
   plan.share_len = (int32_t)len;
   plan.heads_wg = (int32_t)heads;
   plan.share_waves = nw / plan.heads_wg;

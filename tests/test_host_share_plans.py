@@ -1,5 +1,8 @@
 """Which decode launches at head_dim 256 go in shares of their requests' keys: few (request, kv head) pairs, long requests, and the two
 lines beyond which they go in segments.  (With norm and rotary embedding a decode step is one launch where it goes in shares.)"""
+import math
+import random
+
 import pytest
 
 
@@ -34,3 +37,39 @@ def test_windows_of_few_pairs(batch, heads, window, shares):
 
     lib, (n_q, n_kv) = _lib.load(), heads
     assert (lib.msgl_extend_step_workspace_bytes(batch, 2 * batch, 30000 * batch, n_q, n_kv, 256, 2, 0, window) > 0) is shares
+
+
+def _least_cost_shares(batch, keys, n_kv, d, cols, cus=256):
+    """Most shares of a launch whose lengths cost least, by the costs as they are stated: all lengths, in floating point."""
+    mean, length, lowest = keys // batch, None, 0.0
+    c = 512 if cols > 32 else 256 if cols > 16 and d == 128 else 128
+    while c < 1 << 20:
+        of_one = max(math.ceil(mean / c), 1)
+        if max(batch, keys / c + 0.5 * batch + 0.43 * math.sqrt(batch), batch * of_one) * n_kv <= cus:
+            cost = min(c, 1.5 * mean) + ((160 if cols > 8 else 100) if of_one > 1 else 0) + 4 * of_one + 100 * (math.ceil(of_one / 16) - 1)
+            if length is None or cost < lowest:
+                length, lowest = c, cost
+            if c >= 2 * mean:
+                break
+        c = c // 3 * 4 if c & (c - 1) else c // 2 * 3
+    return keys // (length or 1 << 20) + batch
+
+
+def test_lengths_cost_least():
+    from mini_sglang_amd_kernel import _lib
+
+    rng, need = random.Random(3), _lib.load().msgl_decode_step_workspace_bytes
+    log = lambda lo, hi: int(lo * (hi / lo) ** rng.random())  # noqa: E731
+    seen = 0
+    for _ in range(20000):
+        d, n_kv, group = rng.choice((128, 256)), rng.choice((1, 2, 3, 4, 6, 8, 16)), rng.randint(1, 16)
+        batch = log(1, 256 // n_kv + 1)
+        keys = batch * log(1, 100000) + rng.randrange(batch)
+        size = need(batch, keys, n_kv * group, n_kv, d, 1)
+        if size == 0 or batch * n_kv > 256:
+            continue
+        up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+        rows = _least_cost_shares(batch, keys, n_kv, d, group) * n_kv * group
+        assert size == up(8 * batch * n_kv) + up(rows * (d + 1) * 4), (batch, keys, n_kv, group, d)
+        seen += 1
+    assert seen > 5000
