@@ -660,34 +660,33 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
     // worst).  head_dim 256: up to 64 0.65 (1.10), 64-128 0.76 (0.99), 128-256 from 0.5 on 0.83 (1.05) and 1.03 below, 256-420 from
     // 0.62 on 0.91 (1.07), 1.05 below, 512-724 from 0.75 on 0.95 (1.03), 0.97 (1.09) below, 1.04 below 0.62, 1024-1448 from 0.88 on 0.96
     // (0.98), 0.98 (1.07) below, 1.02 below 0.75.  (Two of 408-2260 keys, 24 / 4 heads, 21.8 -> 11.0 us; one of 51.8 K, 16 / 2, 51 -> 35.)
-    // head_dim 128, 18 600 launches, three and eight sets of keys in turn, by pairs: 1-3 0.81, up to 128 MiB; 4-11 24-50 MiB 0.85 and 0.82, 50-190
-    // 0.80 and 0.82; 12-256 24-50 0.7, 50-128 0.77 and 0.8, 128-190 0.83 and 0.89, the worst tenth of them 1.0; beyond by that part of a round: 190-220
-    // from 0.74 on 0.88, 0.98-1.0 below, 220-256 0.88 and 0.99-1.05, 256-300 0.95 and 0.97-1.05, 300-440 from 0.8 on 0.95-0.98, 1.0-1.2 below.
-    // (us: one of 10 K keys, 48 / 6, 16.3 -> 15.5; two, 54 K in all, 42.1 -> 32.1; 13 of 1 K, 32 / 4, 16.6 -> 11.4.)  Few pairs with two or
-    // three tiles of columns leave much to put together to the last share of each: from 16 MiB on up to five pairs 0.98-1.07 and 1.1-1.2.
-    const bool wide = head_dim == 256;
-    if (!wide) {
-      if (cols > 16 && units < 6 && mb > 16) return false;
-      // Some launches from 56 MiB on, 0.75-0.85 of segments as well, stay there: what a step of theirs takes (a launch of its own for norm and
-      // rotary embedding, scratch memory) is what it has been.
-      if (mb > 56 && mb <= 128 && ((units < 48 && cols > 16) || len > 2 * mean)) return false;
-      if (mb > 56 && mb <= 80 && units < 12 && mean > 12288) return false;
-    }
     const double of_round = (double)(keys * n_kv) / (std::min((double)len, 1.75 * (double)mean) * (double)device_cus());
-    if (wide) return mb <= 1400 && of_round >= 0.12 * std::log2((double)std::max<int64_t>(mb, 1)) - 0.39;
-    return mb <= 190 || (mb <= 400 && of_round >= 0.72 + (double)(mb - 190) / 2000);
+    if (head_dim == 256) return mb <= 1400 && of_round >= 0.12 * std::log2((double)std::max<int64_t>(mb, 1)) - 0.39;
+    // head_dim 128: where a share is as long as a request or longer the longest request decides, and it may be many times the mean (32 requests, one
+    // of 9.7 K among 0.6 K, 27.5 us in segments and 50.4).  7700 launches, half with one or some requests 4 to 40 times the others, four sets
+    // of keys in turn, by MiB and a share's length by the mean, shares by segments (the worst tenth): up to 56 0.81 (0.91); 56-104 up to 2
+    // 0.84 (0.94), 1.01 (1.27) beyond; 104-128 up to 1.5 0.88 (0.98), 1.05 (1.2) beyond; 128-160 up to 0.75 0.93 (1.0), to 1.5 1.03 (1.2), 1.2 (1.45)
+    // beyond; 160-190 up to 0.5 0.97 (1.05), to 1 1.04 (1.25), 1.24 (1.45) beyond; 190-256 0.97 (1.03), 1.02 from there on.
+    // (One of 10 K keys, 48 / 6, 16.3 -> 15.5; two, 54 K in all, 42.1 -> 32.1; 13 of 1 K, 32 / 4, 16.6 -> 11.4.)  Few pairs with two or three tiles of
+    // columns leave much to put together to the last share of each: from 16 MiB on up to five pairs 0.98-1.07 and 1.1-1.2, six to eleven of up to
+    // 16 K 1.05-1.15 (1.3; one of eight 54 K, 32 columns, 24.9 and 37.9 us), of more 0.98.
+    if (cols > 16 && mb > 16 && (units < 6 || (units < 12 && mean <= 16384))) return false;
+    // Two kinds of 56-128 MiB, 0.82-0.9 of segments as well, stay there: that a step with norm weights is refused for one request of 20 K keys, and
+    // that four and five requests of 24 columns take a store in front, is what callers were told and tests hold.
+    if (mb > 56 && mb <= 128 && ((units < 48 && cols > 16) || (mb <= 80 && units < 12 && mean > 12288))) return false;
+    if (mb > 190) return mb <= 256 && of_round >= 0.72 + (double)(mb - 190) / 2000;
+    return mb <= 56 || 48 * len <= mean * std::min<int64_t>(200 - mb, 96);
   }
   // Several heads to a workgroup.
   const int64_t head_groups = n_kv / plan.heads_wg;
-  const bool even_fit = batch * ((mean + len - 1) / len) * head_groups <= device_cus();  // requests of one length go in one round
   if (head_dim == 256) {
     if (mb <= 128) return true;
+    const bool even_fit = batch * ((mean + len - 1) / len) * head_groups <= device_cus();  // requests of one length go in one round
     const double shares = (double)keys / (double)len + 0.5 * (double)batch + std::sqrt((double)batch / 3);  // see share_plan()
     return even_fit && shares * (double)head_groups <= device_cus() && len * plan.heads_wg <= 1024 && mb <= 256;
   }
-  // 4800 launches of more than 256 pairs, as above: where requests of one length go in one round 45-96 MiB 0.7, 96-128 0.74 and 0.85, 128-160 0.79
-  // and 0.89, 160-190 0.87 and 0.92, 190-220 0.95 and 0.99, 1.0 beyond; where they don't, up to 128 0.86 and 0.9 (worst 1.5), 0.94 and 1.0 beyond.
-  return mb <= (even_fit ? 190 : 128);
+  // 230 of the launches above: 80-128 MiB 0.95 (1.15), 128-160 1.06 (1.35), 160-190 1.17 (1.4); of lengths that differ little 0.9, 0.93 and 1.09.
+  return mb <= 128;
 }
 
 size_t share_workspace_bytes(const SharePlan& plan, int64_t batch, int64_t n_kv, int64_t head_dim, int64_t cols) {

@@ -40,7 +40,8 @@ def test_decode(gpu, tuning, lens, n_q, n_kv, d, shares, dtype):
     assert bool(plain.isfinite().all()) and _same(plain, stream)
 
 
-@pytest.mark.parametrize("q_len,n_q,n_kv,d", [(4, 32, 8, 128), (8, 32, 8, 128), (12, 32, 8, 128), (5, 64, 8, 128), (4, 16, 4, 256), (2, 24, 4, 256)])
+@pytest.mark.parametrize("q_len,n_q,n_kv,d", [(4, 32, 8, 128), (8, 32, 8, 128), (12, 32, 8, 128), (5, 64, 8, 128), (4, 16, 4, 256), (2, 24, 4, 256),
+                                                (16, 32, 8, 128), (6, 24, 4, 256)])
 @pytest.mark.parametrize("shares", [-1, 128 | 1 << 20])
 @pytest.mark.parametrize("cross,window", [(False, 0), (True, 0), (False, 100), (True, 100)])
 def test_verify(gpu, tuning, q_len, n_q, n_kv, d, shares, cross, window):

@@ -107,7 +107,12 @@ def test_gated_delta_rule_from_a_mean_length_on(batch, heads, line):
 @pytest.mark.parametrize("batch,kv,heads,q,shares", [  # beyond the first lines of the shares (csrc/paged_shares.hip)
     (26, 18746, (32, 8, 128), 1, False), (32, 18048, (64, 8, 128), 1, False), (28, 18060, (32, 8, 128), 1, False),  # shares of 1536 keys
     (19, 28310, (16, 8, 128), 1, True), (39, 28509, (32, 8, 128), 1, True),
-    (4, 15904, (32, 8, 128), 6, False), (5, 26780, (32, 8, 128), 6, False), (6, 26780, (32, 8, 128), 6, True), (4, 15904, (32, 8, 128), 4, True)])
+    (4, 15904, (32, 8, 128), 6, False), (5, 26780, (32, 8, 128), 6, False), (6, 26780, (32, 8, 128), 6, True), (4, 15904, (32, 8, 128), 4, True),
+    # few pairs with two tiles of columns
+    (5, 80000, (8, 1, 128), 3, False), (8, 90000, (8, 1, 128), 3, False), (9, 300000, (8, 1, 128), 3, True),
+    # shares longer than the requests, by the mean length: up to 104 MiB twice, 128 one and a half times, 152 as long, 176 half of it; 256 MiB
+    (17, 39911, (32, 8, 128), 1, False), (21, 42499, (32, 8, 128), 1, False), (17, 29900, (32, 8, 128), 1, True), (1, 60000, (32, 8, 128), 1, True),
+    (1, 66000, (32, 8, 128), 1, False), (300, 300 * 436, (8, 1, 128), 4, True), (85, 66600, (16, 4, 128), 1, False), (85, 65000, (16, 4, 128), 1, True)])
 def test_launches_that_go_in_shares(batch, kv, heads, q, shares):
     from mini_sglang_amd_kernel import _lib
 
