@@ -455,8 +455,10 @@ int launch_shape(const ShareParams& sp, const SharePlan& plan, unsigned blocks, 
   auto launch = [&](auto f16, auto mode_of) {
     constexpr bool F16 = decltype(f16)::value;
     constexpr int NEW = decltype(mode_of)::value;
-    const auto kernel = sp.s.walk == kStream             ? share_attention_kernel<D, NCT, NW, kStream, F16, NEW, WIDE>
-                        : sp.s.walk == (kStream | kWide) ? share_attention_kernel<D, NCT, NW, kStream | kWide, F16, NEW, WIDE>
+    // (launches with column groups are small, 64 MiB at most, and stay in the caches)
+    constexpr int kPast = WIDE ? kNarrow : kStream;
+    const auto kernel = sp.s.walk == kStream             ? share_attention_kernel<D, NCT, NW, kPast, F16, NEW, WIDE>
+                        : sp.s.walk == (kStream | kWide) ? share_attention_kernel<D, NCT, NW, kPast | kWide, F16, NEW, WIDE>
                         : sp.s.walk == kWide             ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, WIDE>
                                                          : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, WIDE>;
     return launch_kernel(kernel, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
