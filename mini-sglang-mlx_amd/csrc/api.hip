@@ -86,15 +86,15 @@ bool window_shares(const msgl::SharePlan& plan, int64_t batch, int64_t total_kv,
 // read every K / V row, and the tile kernel with ragged key shares is as fast or faster on them),
 // at head_dim 256 16 (one column tile; more would be a wave per tile, each reading every row,
 // and the tile kernel with ragged shares is 10-65 % faster from 17 columns on).  Few keys go in shares beyond that, see
-// wide_round() in paged_shares.hip.  Up to 64 columns
+// groups_round() in paged_shares.hip.  Up to 64 columns
 // the split-K kernel also takes what the tile kernels cannot give ragged shares to (very many
 // or many short requests): its segments are balanced whatever the lengths, and one long request
 // among many short ones would otherwise be one long workgroup per kv head.
 int64_t smallq_base_cols(int64_t head_dim) { return head_dim == 128 ? 48 : 16; }
 // Two column tiles of 256 dims in one wave of the split-K kernel (17 to 32 columns), which reads every row once and balances its segments
 // whatever the lengths; beside the tile kernel, by MiB of keys and values (geometric mean, worst, of 150 launches): 64 1.25 (1.5), 128 1.15 (1.3), 181
-// 1.0 (1.16), 256 0.92 (1.05), 362 0.81 (1.02), 512 0.79, 1024 0.72, 2048 0.67.  (us: 12 of 531 K keys in all, 6 tokens, 16 / 4 heads, 565 -> 341; six of
-// 84 K, 8, 32 / 8, 193 -> 125.)  33 to 64 columns, two such waves a head, 1.0-1.1 up to 2 GiB.
+// 1.0 (1.16), 256 0.92 (1.05), 362 0.81 (1.02), 512 0.79, 1024 0.72, 2048 0.67.  (us: 12 of 531 K keys in all, 6 tokens, 16 / 4 heads, 565 -> 348; six of
+// 84 K, 8, 32 / 8, 193 -> 127.)  33 to 64 columns, two such waves a head, 1.0-1.1 up to 2 GiB.
 bool two_tiles_in_segments(int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   return head_dim == 256 && cols > 16 && cols <= 32 && keys * n_kv * head_dim * 4 >= (int64_t)256 << 20;
 }

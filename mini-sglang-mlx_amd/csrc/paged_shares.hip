@@ -354,8 +354,8 @@ __device__ __forceinline__ void attend_share(const ShareParams& sp, const SplitK
   else merge(std::integral_constant<int, 16>{});
 }
 
-// WIDE: a request's columns go to several workgroups, kCols to each.
-template <int D, int NCT, int NW, int WALK, bool F16, int NEW, bool WIDE>
+// GROUPS: a request's columns go to several workgroups, kCols to each.
+template <int D, int NCT, int NW, int WALK, bool F16, int NEW, bool GROUPS>
 __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share_attention_kernel(
     const int32_t* kv_indptr, const int32_t* qo_indptr, const int32_t* prefix_lens, int32_t batch, int32_t share_len, int32_t window,
     int32_t max_len_extend, int32_t q_cap, int32_t is_cross, uint32_t len_magic, uint32_t shape_bits, ShareParams params) {
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int item, hg;
   uint32_t block = blockIdx.x, cg = 0;
-  if (WIDE) {  // the column groups of a share are on one XCD
+  if (GROUPS) {  // the column groups of a share are on one XCD
     const uint32_t seq = block >> 3, base = seq / shape.col_groups();
     cg = seq - base * shape.col_groups();
     block = base * 8 + (block & 7);
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
     item = block >> shape.groups();
     hg = block & ((1u << shape.groups()) - 1);
   }
-  const int col0 = WIDE ? (int)cg * kCols : 0;  // the first of this workgroup's columns
+  const int col0 = GROUPS ? (int)cg * kCols : 0;  // the first of this workgroup's columns
   const int share_waves = 1 << shape.waves();
   const int sub = wave >> shape.waves();  // which of the workgroup's kv heads
   const int sw = wave & (share_waves - 1);
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   // what the rest of the way begins with and only the request's number leads to
   const typename std::conditional<NEW == kStore || NEW == kNormRopeStore, NewTokenIds<NEW == kNormRopeStore>, Nothing>::type new_ids(p, b);
   __builtin_amdgcn_sched_barrier(0);
-  const int ncols = WIDE ? min(r.q_len * p.group - col0, kCols) : r.q_len * p.group;
+  const int ncols = GROUPS ? min(r.q_len * p.group - col0, kCols) : r.q_len * p.group;
   if (ncols <= 0) return;
   Columns<D, NCT> c;
   // the keys that are walked: all, but for a prefill call's own new ones
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
   if (t_begin < t_end) ids = first_ids(p, r, t_begin, t_end);
   const typename std::conditional<(WALK & kStream) != 0, OtherSlots, Nothing>::type other_slots(p, other, r, s_begin < s_end ? s_begin : -1);
   __builtin_amdgcn_sched_barrier(0);
-  unsigned long long* const cnt = sp.counts + ((int64_t)b * sp.head_groups + hg) * (WIDE ? shape.col_groups() : 1) + cg;
+  unsigned long long* const cnt = sp.counts + ((int64_t)b * sp.head_groups + hg) * (GROUPS ? shape.col_groups() : 1) + cg;
   const unsigned long long fresh = sp.nonce << 16;
   // The first share makes the count word this launch's, long before anybody counts.  Nothing waits
   // for it: whoever finds the word not made yet makes it (below).  (The last wave, which has the fewest keys or none.)
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(64 * NW, (D == 128 && NCT == 1) ? 2 : 1) void share
 // waves of a workgroup: two per SIMD where a wave fits 256 registers
 int waves_of(int64_t head_dim, int nct) { return head_dim == 128 && nct == 1 ? 8 : 4; }
 
-template <int D, int NCT, int NW, bool WIDE>
+template <int D, int NCT, int NW, bool GROUPS>
 int launch_shape(const ShareParams& sp, const SharePlan& plan, unsigned blocks, hipStream_t stream) {
   const int share_len = plan.share_len;
   auto log2_of = [](uint32_t x) { return 31u - (uint32_t)__builtin_clz(x); };
@@ -456,15 +456,15 @@ int launch_shape(const ShareParams& sp, const SharePlan& plan, unsigned blocks, 
     constexpr bool F16 = decltype(f16)::value;
     constexpr int NEW = decltype(mode_of)::value;
     // (launches with column groups are small, 64 MiB at most, and stay in the caches)
-    constexpr int kPast = WIDE ? kNarrow : kStream;
-    const auto kernel = sp.s.walk == kStream             ? share_attention_kernel<D, NCT, NW, kPast, F16, NEW, WIDE>
-                        : sp.s.walk == (kStream | kWide) ? share_attention_kernel<D, NCT, NW, kPast | kWide, F16, NEW, WIDE>
-                        : sp.s.walk == kWide             ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, WIDE>
-                                                         : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, WIDE>;
+    constexpr int kPast = GROUPS ? kNarrow : kStream;
+    const auto kernel = sp.s.walk == kStream             ? share_attention_kernel<D, NCT, NW, kPast, F16, NEW, GROUPS>
+                        : sp.s.walk == (kStream | kWide) ? share_attention_kernel<D, NCT, NW, kPast | kWide, F16, NEW, GROUPS>
+                        : sp.s.walk == kWide             ? share_attention_kernel<D, NCT, NW, kWide, F16, NEW, GROUPS>
+                                                         : share_attention_kernel<D, NCT, NW, kNarrow, F16, NEW, GROUPS>;
     return launch_kernel(kernel, dim3(blocks), dim3(64 * NW), stream, sp.s.kv_indptr, sp.s.qo_indptr, sp.s.prefix_lens,
                          sp.s.batch, (int32_t)share_len, sp.s.window, sp.s.max_len_extend, sp.s.q_cap, sp.s.is_cross, magic, shape.bits, sp);
   };
-  if constexpr (NCT == 1 && !WIDE) {  // IEEE half and new tokens exist for decode only (one column tile)
+  if constexpr (NCT == 1 && !GROUPS) {  // IEEE half and new tokens exist for decode only (one column tile)
     const int mode = sp.s.nt.k == nullptr || sp.s.qo_indptr != nullptr ? kStored : sp.s.nt.q_weight == nullptr ? kStore : kNormRopeStore;
     if (sp.s.f16) {
       if (mode == kStored && sp.s.nt.k == nullptr)
@@ -540,8 +540,8 @@ static int64_t cost_share_length(int64_t batch, int64_t keys, int64_t n_kv, int6
 // request 0.9-1.1, more than three quarters of a round 1.0 (1.2).  (us: 16 of 5 tokens,
 // window 1024, 8 / 1 heads of 256, 34 -> 16; one of 1.7 K, 12 tokens, the same, 22 -> 12; two of 14 tokens, window 1024, 32 / 8 heads of 128, 25 -> 13.)
 constexpr int64_t kXcds = 8;
-static int64_t wide_keys(int64_t head_dim) { return head_dim == 256 ? 400 : 512; }  // for each compute unit
-static bool wide_round(int64_t batch, int64_t keys, int64_t n_kv, int64_t slots, int64_t head_dim) {
+static int64_t groups_keys(int64_t head_dim) { return head_dim == 256 ? 400 : 512; }  // for each compute unit
+static bool groups_round(int64_t batch, int64_t keys, int64_t n_kv, int64_t slots, int64_t head_dim) {
   return head_dim == 256 ? batch * n_kv <= slots && keys > 128 * batch : 4 * batch * n_kv <= 3 * slots && keys > 192 * batch;
 }
 
@@ -564,8 +564,8 @@ static ColGroups col_groups_of(int64_t head_dim, int64_t cols, int64_t batch, in
   const ColGroups together{1, tiles}, pairs{(tiles + 1) / 2, 2}, apart{tiles, 1};
   if (tiles == 1) return together;
   if (t_force > 0) return d256 ? apart : tiles <= 3 ? together : pairs;
-  auto in_round = [&](const ColGroups& c) { return wide_round(batch, keys, n_kv, round_slots(c.groups), head_dim); };
-  auto fits = [&](const ColGroups& c) { return in_round(c) && keys * n_kv * c.groups <= wide_keys(head_dim) * device_cus(); };
+  auto in_round = [&](const ColGroups& c) { return groups_round(batch, keys, n_kv, round_slots(c.groups), head_dim); };
+  auto fits = [&](const ColGroups& c) { return in_round(c) && keys * n_kv * c.groups <= groups_keys(head_dim) * device_cus(); };
   if (fits(apart)) return apart;
   if (!d256 && tiles > 2 && fits(pairs)) return pairs;
   if (!d256 && tiles <= 3) return together;
@@ -652,7 +652,7 @@ bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t he
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
-  if (plan.col_groups > 1) return keys * n_kv * plan.col_groups <= wide_keys(head_dim) * device_cus();
+  if (plan.col_groups > 1) return keys * n_kv * plan.col_groups <= groups_keys(head_dim) * device_cus();
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
   if (mean <= 512) return mb <= 160;
   if (few_pairs_in_segments(batch, n_kv, mean, head_dim, cols, false)) return false;
