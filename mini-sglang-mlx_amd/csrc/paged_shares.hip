@@ -652,8 +652,13 @@ bool few_pairs_in_segments(int64_t batch, int64_t n_kv, int64_t mean, int64_t he
 bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_t n_kv, int64_t head_dim, int64_t cols) {
   if (plan.share_len == 0) return false;
   if (t_force > 0) return true;
-  if (plan.col_groups > 1) return keys * n_kv * plan.col_groups <= groups_keys(head_dim) * device_cus();
   const int64_t mb = keys * n_kv * head_dim * 4 >> 20, mean = keys / batch, units = batch * n_kv;
+  if (plan.col_groups > 1) {
+    // (and at head_dim 256, where a share is longer than two requests, few keys again, as below: eight requests, one of 2.7 K among 0.1 K, 24.3 us in
+    // tiles and 40.3; 22 such launches 0.87 of tiles, worst 1.66, those from 200 keys for each compute unit on 1.1-1.66)
+    const int64_t read = keys * n_kv * plan.col_groups, cus = device_cus();
+    return read <= groups_keys(head_dim) * cus && (head_dim == 128 || plan.share_len <= 2 * mean || read <= 200 * cus);
+  }
   if (mean <= 512) return mb <= 160;
   if (few_pairs_in_segments(batch, n_kv, mean, head_dim, cols, false)) return false;
   const int64_t len = plan.share_len;
@@ -671,8 +676,8 @@ bool shares_preferred(const SharePlan& plan, int64_t batch, int64_t keys, int64_
     // beyond; 160-190 up to 0.5 0.97 (1.05), to 1 1.04 (1.25), 1.24 (1.45) beyond; 190-256 0.97 (1.03), 1.02 from there on.
     // (One of 10 K keys, 48 / 6, 16.3 -> 15.5; two, 54 K in all, 42.1 -> 32.1; 13 of 1 K, 32 / 4, 16.6 -> 11.4.)  Few pairs with two or three tiles of
     // columns leave much to put together to the last share of each: from 16 MiB on up to five pairs 0.98-1.07 and 1.1-1.2, six to eleven of up to
-    // 16 K 1.05-1.15 (1.3; one of eight 54 K, 32 columns, 24.9 and 37.9 us), of more 0.98.
-    if (cols > 16 && mb > 16 && (units < 6 || (units < 12 && mean <= 16384))) return false;
+    // 16 K 1.05-1.15 (1.3; one of eight 54 K, 32 columns, 24.9 and 37.9 us), of more 0.98, twelve to 15 of up to 8 K 1.07 (1.5), of more 0.93.
+    if (cols > 16 && mb > 16 && (units < 6 || (units < 12 && mean <= 16384) || (units < 16 && mean <= 8192))) return false;
     // Two kinds of 56-128 MiB, 0.82-0.9 of segments as well, stay there: that a step with norm weights is refused for one request of 20 K keys, and
     // that four and five requests of 24 columns take a store in front, is what callers were told and tests hold.
     if (mb > 56 && mb <= 128 && ((units < 48 && cols > 16) || (mb <= 80 && units < 12 && mean > 12288))) return false;
