@@ -740,9 +740,9 @@ def _probe_lib():
 
 
 def hbm_read_probe(gib: int = 4, reps: int = 5):
-    """A plain streaming read of `gib` GiB (16 bytes per lane and load, consecutive lanes on
-    consecutive addresses, far beyond the 256 MB Infinity Cache): the rate the memory system
-    gives a kernel that does nothing but read, beside the datasheet's 8 TB/s."""
+    """A streaming read of `gib` GiB (16 bytes per lane and load, consecutive lanes on
+    consecutive addresses, a grid-stride loop with the non-temporal hint, far beyond the 256 MB Infinity Cache): the rate
+    the memory system gives a kernel that does nothing but read, beside the datasheet's 8 TB/s."""
     import ctypes
 
     lib = _probe_lib()
@@ -783,6 +783,23 @@ def mfma_rate_probe():
         out[name + "_shader_ghz"] = ghz.value
         log(f"[mfma probe] {name}: {tf.value:.0f} TFLOP/s at {ghz.value:.2f} GHz")
     return out
+
+
+def ways_to_read_probe(sizes=(4096, 80)):
+    """4 GiB by waves that walk blocks of 16 KiB, plainly and with the non-temporal hint, from buffers of `sizes` MiB: from memory, and what
+    the caches give where the same blocks are read again (bench_probes.hip)."""
+    import ctypes
+
+    lib = _probe_lib()
+    lib.msgl_probe_ways_to_read.restype = ctypes.c_int
+    lib.msgl_probe_ways_to_read.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_double)]
+    rows, out = [], (ctypes.c_double * 2)()
+    for mib in sizes:
+        if lib.msgl_probe_ways_to_read(mib, 7, out) != 0:
+            return None
+        rows.append({"buffer_MiB": mib, "plain_TBps": out[0], "non_temporal_TBps": out[1]})
+        log(f"[ways to read] 4 GiB from {mib} MiB: plain {out[0]:.2f} TB/s, non-temporal {out[1]:.2f} TB/s")
+    return rows
 
 
 def issue_rate_probes():
@@ -945,6 +962,7 @@ def main():
         result["hbm_read_probe"] = hbm_read_probe()
     if args.issue_probes:
         result["issue_probes"] = issue_rate_probes()
+        result["ways_to_read"] = ways_to_read_probe()
     if not args.no_metadata:
         result["qk_norm_rope_store"] = run_norm_rope_store(dev, args.steps, args.warmup,
                                                            not args.no_cpu_baseline)

@@ -9,10 +9,11 @@
 // bf16 attention kernel on random data is measured against; the datasheet peak assumes the
 // boost clock.  A third run feeds the A operand of every instruction from LDS.
 //
-// (2) What a plain streaming read sustains: every lane reads 16 bytes per load, consecutive
+// (2) What a streaming read sustains: every lane reads 16 bytes per load, consecutive
 // lanes consecutive addresses, a grid-stride loop over a buffer far larger than the 256 MB
-// Infinity Cache, eight loads in flight per lane.  The HBM-bound attention kernels are read
-// beside this figure as well as beside the datasheet's 8 TB/s.
+// Infinity Cache, eight loads in flight per lane, with the non-temporal hint.  The HBM-bound attention
+// kernels are read beside this figure as well as beside the datasheet's 8 TB/s.  That loop is not
+// the fastest way to read: see (4).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -140,6 +141,35 @@ __global__ __launch_bounds__(256) void hbm_read_kernel(const u32x4_t* __restrict
   for (; i < n_vec; i += stride) acc ^= __builtin_nontemporal_load(src + i);
   const uint32_t x = acc[0] ^ acc[1] ^ acc[2] ^ acc[3];
   if (x == 0x9e3779b9u) sink[0] = x;  // never true for the fill pattern; keeps the loads alive
+}
+
+// (4) Ways to read: each wave walks blocks of 16 KiB, 16 loads of 1 KiB (whole 128-byte lines), in a scattered order over the buffer,
+// the next block's loads in flight beside the one in use, one workgroup of four waves per CU, plainly or with the non-temporal hint.  (As
+// an attention kernel walks its keys; the grid-stride loop of (2) has all waves side by side.)  `blocks` of the buffer are
+// read, over and over where that is less than the waves read in all: what comes from the caches then.
+template <bool NT>
+__global__ __launch_bounds__(256) void block_read_kernel(const u32x4_t* __restrict__ src, uint32_t blocks, uint32_t per_wave, uint32_t* sink) {
+  const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  u32x4_t acc = {0u, 0u, 0u, 0u}, v[2][16];
+  // (through a descriptor of the block: the compiler makes one set of registers of two sets of plain loads, and drains them each time)
+  auto load = [&](u32x4_t (&to)[16], uint32_t i) {
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)(wave * per_wave + i) * 40503u % blocks));  // below 2^18
+    const auto block = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4_t*>(src + (size_t)at * 1024), 0, 16384, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      to[k] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(block, (int)(lane * 16 + k * 1024), 0, NT ? 2 : 0));
+  };
+  load(v[0], 0);
+  for (uint32_t i = 0; i < per_wave; i += 2) {
+    load(v[1], min(i + 1, per_wave - 1));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc ^= v[0][k];
+    load(v[0], min(i + 2, per_wave - 1));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc ^= v[1][k];
+  }
+  const uint32_t x = acc[0] ^ acc[1] ^ acc[2] ^ acc[3];
+  if (x == 0x9e3779b9u) sink[0] = x;
 }
 
 // (3) Rates behind the kernels' schedules, in shader cycles counted by one workgroup per launch:
@@ -328,6 +358,49 @@ extern "C" __attribute__((visibility("default"))) int msgl_probe_hbm_read(size_t
   }
   *best_tbps = best;
   *mean_tbps = total_ms > 0.0 ? (double)bytes * reps / (total_ms * 1e-3) / 1e12 : 0.0;
+  (void)hipEventDestroy(t0);
+  (void)hipEventDestroy(t1);
+  (void)hipFree(buf);
+  (void)hipFree(sink);
+  return (int)e;
+}
+
+// (4): 4 GiB read from a buffer of `mib` MiB (16 to 4096), best of `reps`, in TB/s: [0] plainly, [1] with the hint.  Returns 0 or a hipError_t value.
+extern "C" __attribute__((visibility("default"))) int msgl_probe_ways_to_read(int mib, int reps, double* tbps) {
+  int dev = 0, cus = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return (int)e;
+  e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess) return (int)e;
+  if (mib < 16 || mib > 4096 || reps < 1 || cus < 1) return (int)hipErrorInvalidValue;
+  u32x4_t* buf = nullptr;
+  uint32_t* sink = nullptr;
+  e = hipMalloc(&buf, (size_t)mib << 20);
+  if (e != hipSuccess) return (int)e;
+  e = hipMalloc(&sink, 4);
+  if (e != hipSuccess) {
+    (void)hipFree(buf);
+    return (int)e;
+  }
+  (void)hipMemset(buf, 0x5a, (size_t)mib << 20);
+  const uint32_t blocks = (uint32_t)mib * 64, per_wave = (uint32_t)(4096 * 64 / (cus * 4)) & ~1u;
+  hipEvent_t t0, t1;
+  (void)hipEventCreate(&t0);
+  (void)hipEventCreate(&t1);
+  for (int nt = 0; nt < 2 && e == hipSuccess; ++nt) {
+    tbps[nt] = 0.0;
+    for (int r = 0; r <= reps; ++r) {
+      (void)hipEventRecord(t0, 0);
+      if (nt) hipLaunchKernelGGL(block_read_kernel<true>, dim3(cus), dim3(256), 0, 0, buf, blocks, per_wave, sink);
+      else hipLaunchKernelGGL(block_read_kernel<false>, dim3(cus), dim3(256), 0, 0, buf, blocks, per_wave, sink);
+      (void)hipEventRecord(t1, 0);
+      e = hipEventSynchronize(t1);
+      float ms = 0.f;
+      if (e != hipSuccess || hipEventElapsedTime(&ms, t0, t1) != hipSuccess) break;
+      const double rate = (double)per_wave * cus * 4 * 16384 / (ms * 1e-3) / 1e12;
+      if (r > 0 && rate > tbps[nt]) tbps[nt] = rate;
+    }
+  }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   (void)hipFree(buf);

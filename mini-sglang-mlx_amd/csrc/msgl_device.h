@@ -22,8 +22,8 @@ constexpr float kNegInf = -__builtin_inff();
 __device__ __forceinline__ u32x4_t ld_global_b128(const void* p) {
   return *reinterpret_cast<const u32x4_t*>(p);
 }
-// The same of what nobody reads again soon: the line leaves the caches first.  A wave's load of whole 128-byte lines this way, 1 KiB of
-// each: 4 GiB at 7.0 TB/s, plain loads 6.2; of halves of lines, whose other half another load asks for, 5.2-6.1.
+// The same of what nobody reads again soon: the line leaves the caches first.  A wave's loads of whole 128-byte lines this way, 16 KiB after
+// 16 KiB: 4 GiB at 6.7-7.0 TB/s, plain loads 5.9-6.1; of halves of lines, whose other half another load asks for, 5.2-6.1.  (From the caches 12 and 25.)
 __device__ __forceinline__ u32x4_t ld_stream_b128(const void* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)); }
 __device__ __forceinline__ void st_global_b128(void* p, u32x4_t v) {
   *reinterpret_cast<u32x4_t*>(p) = v;

@@ -114,7 +114,7 @@ __device__ __forceinline__ ReqInfo request_info(const P& p, int b, Meanwhile&& m
   return r;
 }
 
-// The query that a column belongs to, col / group: exact up to 64 columns and heads to a group (a division is 25 instructions).
+// The query that a column belongs to, col / group: exact while col (group - 1) < 2^16 (160 columns at most; a division is 25 instructions).
 __device__ __forceinline__ int query_of(const SplitKvParams& p, int col) { return (int)((uint32_t)col * p.per_group >> 16); }
 
 template <int D>
